@@ -1629,9 +1629,11 @@ void mlstm_scan(Tensor out, Tensor qkvg, Tensor gates, Tensor S, Tensor n, Tenso
   TORCH_CHECK(S.dim() == 4 && S.size(1) == H && S.size(2) == d && S.size(3) == dv &&
               n.numel() == S.size(0) * H * d && m.numel() == S.size(0) * H,
               "kgc.mlstm_scan: state S [slots, H, d, dv], n [slots, H, d], m [slots, H]");
+  Tensor ws = at::empty({kgc::mlstm_scan_ws((int)(P + D), (int)H, (int)d)}, gates.options());
   kgc::launch_mlstm_scan(dt_code(qkvg), out.data_ptr<float>(), qkvg.data_ptr(), qkvg.stride(0),
                          gates.data_ptr<float>(), S.data_ptr<float>(), n.data_ptr<float>(),
-                         m.data_ptr<float>(), i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"),
+                         m.data_ptr<float>(), ws.data_ptr<float>(),
+                         i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"),
                          i32_ptr(seq_lens, P, "seq_lens"), i32_ptr(ctx_lens, D, "ctx_lens"),
                          i32_ptr(slots, P + D, "state slots"), (int)P, (int)D, (int)Tp, (int)H,
                          (int)d, (int)dv, (int)S.size(0), stream());

@@ -338,10 +338,12 @@ void launch_window_prefill_mfma(int dtype, void* out, const void* q, const void*
                                 int dk, int dv, int krs, int vrs, int bs, int num_blocks, float scale, int window,
                                 int keep_first, const float* gate, WindowExtra ex, hipStream_t s);
 int mlstm_scan_max_dim();
+int64_t mlstm_scan_ws(int seqs, int H, int d);   // floats of workspace
 void launch_mlstm_scan(int dtype, float* out, const void* qkvg, int64_t stride,
-                       const float* gates, float* S, float* nst, float* mst, const int* qsl,
-                       const int* seq_lens, const int* ctx_lens, const int* slots, int P, int D,
-                       int Tp, int H, int d, int dv, int num_slots, hipStream_t s);
+                       const float* gates, float* S, float* nst, float* mst, float* ws,
+                       const int* qsl, const int* seq_lens, const int* ctx_lens,
+                       const int* slots, int P, int D, int Tp, int H, int d, int dv,
+                       int num_slots, hipStream_t s);
 
 // ---- scaled residual stream, token shift, minGRU, latent attention rows, sigmoid routing --
 // `dtype`: activation type of add / proj / zxg ...; `out_dtype`: DT_F32 or the same

@@ -33,7 +33,8 @@ template <typename T, int RMAX>
 __global__ __launch_bounds__(NT) void mlstm_scan_kernel(
     float* __restrict__ out, const T* __restrict__ qkvg, int64_t stride,
     const float* __restrict__ gates, float* __restrict__ S, float* __restrict__ nst,
-    float* __restrict__ mst, const int* __restrict__ qsl, const int* __restrict__ seq_lens,
+    float* __restrict__ mst, const float* __restrict__ n0, const float* __restrict__ m0,
+    const int* __restrict__ qsl, const int* __restrict__ seq_lens,
     const int* __restrict__ ctx_lens, const int* __restrict__ slots, int P, int Tp, int H,
     int d, int dv, int num_slots) {
   constexpr int NU = (4 * RMAX + 63) / 64;
@@ -69,6 +70,9 @@ __global__ __launch_bounds__(NT) void mlstm_scan_kernel(
   float* Ss = S + ((int64_t)slot * H + h) * d * dv;
   float* ns = nst + ((int64_t)slot * H + h) * d;
   float* ms = mst + (int64_t)slot * H + h;
+  // where n and m are read: the launcher's copy when several workgroups share them
+  const float* n_in = n0 ? n0 + ((int64_t)s * H + h) * d : ns;
+  const float* m_in = m0 ? m0 + (int64_t)s * H + h : ms;
   float Sr[RMAX], nr[NU];
   float m = 0.f;
   const bool fresh = pos0 == 0;
@@ -81,9 +85,9 @@ __global__ __launch_bounds__(NT) void mlstm_scan_kernel(
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     const int r = lane + 64 * u;
-    nr[u] = (!fresh && r < d) ? ns[r] : 0.f;
+    nr[u] = (!fresh && r < d) ? n_in[r] : 0.f;
   }
-  if (!fresh) m = *ms;
+  if (!fresh) m = *m_in;
   const float qscale = 1.f / sqrtf((float)d);
   const int koff = H * d, voff = 2 * H * d;
   float pqk[NQK], pv[NV], pg = 0.f;
@@ -192,20 +196,36 @@ __global__ __launch_bounds__(NT) void mlstm_scan_kernel(
   }
 }
 
+// n and m of the step's sequences, copied before the scan: the column workgroups of a head all
+// start from them, and the first one writes the slot while later ones may not have begun.
+__global__ __launch_bounds__(64) void mlstm_head_state_kernel(
+    float* __restrict__ n0, float* __restrict__ m0, const float* __restrict__ nst,
+    const float* __restrict__ mst, const int* __restrict__ slots, int H, int d, int num_slots) {
+  const int s = blockIdx.x, h = blockIdx.y, slot = slots[s];
+  if (slot < 0 || slot >= num_slots) return;
+  const int64_t from = (int64_t)slot * H + h, to = (int64_t)s * H + h;
+  for (int r = threadIdx.x; r < d; r += 64) n0[to * d + r] = nst[from * d + r];
+  if (threadIdx.x == 0) m0[to] = mst[from];
+}
+
 static size_t scan_lds(int rmax) {
   return sizeof(float) * (size_t)(TB * 2 * 4 * rmax + TB * 64 + TB * 2 + TB + TB * NW * 64);
 }
 
 template <typename T>
 void scan_dispatch(float* out, const T* qkvg, int64_t stride, const float* gates, float* S,
-                   float* nst, float* mst, const int* qsl, const int* seq_lens,
+                   float* nst, float* mst, float* ws, const int* qsl, const int* seq_lens,
                    const int* ctx_lens, const int* slots, int P, int D, int Tp, int H, int d,
                    int dv, int num_slots, hipStream_t s) {
   const dim3 grid(P + D, H, (dv + 63) / 64);
+  float* n0 = grid.z > 1 ? ws : nullptr;
+  float* m0 = n0 ? ws + (int64_t)(P + D) * H * d : nullptr;
+  if (n0)
+    mlstm_head_state_kernel<<<dim3(P + D, H), 64, 0, s>>>(n0, m0, nst, mst, slots, H, d, num_slots);
 #define KGC_SCAN(R)                                                                          \
   mlstm_scan_kernel<T, R><<<grid, NT, scan_lds(R), s>>>(out, qkvg, stride, gates, S, nst, mst, \
-                                                        qsl, seq_lens, ctx_lens, slots, P, Tp, \
-                                                        H, d, dv, num_slots)
+                                                        n0, m0, qsl, seq_lens, ctx_lens, slots, \
+                                                        P, Tp, H, d, dv, num_slots)
   if (d <= 64) KGC_SCAN(16);
   else if (d <= 128) KGC_SCAN(32);
   else if (d <= 256) KGC_SCAN(64);
@@ -216,20 +236,22 @@ void scan_dispatch(float* out, const T* qkvg, int64_t stride, const float* gates
 }  // namespace
 
 int mlstm_scan_max_dim() { return 512; }
+int64_t mlstm_scan_ws(int seqs, int H, int d) { return (int64_t)seqs * H * (d + 1); }
 
 void launch_mlstm_scan(int dtype, float* out, const void* qkvg, int64_t stride,
-                       const float* gates, float* S, float* nst, float* mst, const int* qsl,
-                       const int* seq_lens, const int* ctx_lens, const int* slots, int P, int D,
-                       int Tp, int H, int d, int dv, int num_slots, hipStream_t s) {
+                       const float* gates, float* S, float* nst, float* mst, float* ws,
+                       const int* qsl, const int* seq_lens, const int* ctx_lens,
+                       const int* slots, int P, int D, int Tp, int H, int d, int dv,
+                       int num_slots, hipStream_t s) {
   if (P + D <= 0) return;
   if (dtype == DT_BF16)
-    scan_dispatch<bf16>(out, (const bf16*)qkvg, stride, gates, S, nst, mst, qsl, seq_lens,
+    scan_dispatch<bf16>(out, (const bf16*)qkvg, stride, gates, S, nst, mst, ws, qsl, seq_lens,
                         ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s);
   else if (dtype == DT_F16)
-    scan_dispatch<f16>(out, (const f16*)qkvg, stride, gates, S, nst, mst, qsl, seq_lens,
+    scan_dispatch<f16>(out, (const f16*)qkvg, stride, gates, S, nst, mst, ws, qsl, seq_lens,
                        ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s);
   else
-    scan_dispatch<float>(out, (const float*)qkvg, stride, gates, S, nst, mst, qsl, seq_lens,
+    scan_dispatch<float>(out, (const float*)qkvg, stride, gates, S, nst, mst, ws, qsl, seq_lens,
                          ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s);
 }
 

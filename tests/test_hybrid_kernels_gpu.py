@@ -165,6 +165,23 @@ def test_mlstm_scan(gpu, dt, H, d, dv):
         torch.testing.assert_close(a.cpu(), b, rtol=2e-4, atol=2e-4)
 
 
+def test_mlstm_scan_many_workgroups(gpu):
+    """More workgroups than the chip holds at once: those of a head's later columns begin after
+    the first one has written n and m back, and still start from the incoming ones."""
+    torch.manual_seed(14)
+    B, H, d, dv = 192, 4, 64, 512
+    m = _meta([], [], [50] * B, torch.zeros(B, 1, dtype=torch.int32), torch.randperm(B).tolist())
+    st = (torch.randn(B, H, d, dv) * 0.3, torch.randn(B, H, d) * 0.3, torch.rand(B, H) * 2)
+    qkvg = torch.randn(B, 2 * H * d + 2 * H * dv)
+    gates = torch.cat([torch.randn(B, H) * 2, -torch.rand(B, H) * 2], dim=1)
+    st_g = tuple(x.to(gpu) for x in st)
+    want = ops.mlstm_scan(qkvg, gates, st, m, H, d, dv)
+    got = ops.mlstm_scan(qkvg.to(gpu), gates.to(gpu), st_g, _to(m, gpu), H, d, dv)
+    torch.testing.assert_close(got.cpu(), want, rtol=2e-4, atol=2e-4)
+    for a, b in zip(st_g, st):
+        torch.testing.assert_close(a.cpu(), b, rtol=2e-4, atol=2e-4)
+
+
 @pytest.mark.parametrize("path", ["fast", "simple"])
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,G,dk,dv,window,keep", [(4, 2, 96, 64, 70, 5), (4, 1, 128, 128, 150, 3),
