@@ -1608,6 +1608,16 @@ void qk_norm_store(Tensor q_out, Tensor qkv, Tensor positions, Tensor qw, std::o
                             bs, prow, nb, (float)eps, interleaved, stream());
 }
 
+// the workspace of a chunkwise scan that cuts its sequences into segments
+void chunk_workspace(kgc::ChunkWork& w, int64_t per_item, int64_t H, const Tensor& like, Tensor& state,
+                     Tensor& gate) {
+  if (w.seg <= 0) return;
+  state = at::empty({w.items * per_item}, like.options().dtype(at::kFloat));
+  gate = at::empty({w.items * H * 2}, like.options().dtype(at::kDouble));
+  w.state = state.data_ptr<float>();
+  w.gate = gate.data_ptr<double>();
+}
+
 void mlstm_scan(Tensor out, Tensor qkvg, Tensor gates, Tensor S, Tensor n, Tensor m,
                 std::optional<Tensor> qsl, std::optional<Tensor> seq_lens,
                 std::optional<Tensor> ctx_lens, Tensor slots, int64_t P, int64_t D, int64_t Tp,
@@ -1630,13 +1640,21 @@ void mlstm_scan(Tensor out, Tensor qkvg, Tensor gates, Tensor S, Tensor n, Tenso
               n.numel() == S.size(0) * H * d && m.numel() == S.size(0) * H,
               "kgc.mlstm_scan: state S [slots, H, d, dv], n [slots, H, d], m [slots, H]");
   Tensor ws = at::empty({kgc::mlstm_scan_ws((int)(P + D), (int)H, (int)d)}, gates.options());
+  kgc::ChunkWork cw;
+  const bool chunk = kgc::mlstm_chunk_ok(dt_code(qkvg), qkvg.stride(0), qkvg.data_ptr(), (int)P,
+                                         (int)Tp, (int)H, (int)d, (int)dv);
+  Tensor cs, cg;
+  if (chunk) {
+    cw = kgc::mlstm_chunk_plan(dt_code(qkvg), (int)P, (int)Tp, (int)H, (int)d, (int)dv);
+    chunk_workspace(cw, H * d * (dv + 1), H, gates, cs, cg);
+  }
   kgc::launch_mlstm_scan(dt_code(qkvg), out.data_ptr<float>(), qkvg.data_ptr(), qkvg.stride(0),
                          gates.data_ptr<float>(), S.data_ptr<float>(), n.data_ptr<float>(),
                          m.data_ptr<float>(), ws.data_ptr<float>(),
                          i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"),
                          i32_ptr(seq_lens, P, "seq_lens"), i32_ptr(ctx_lens, D, "ctx_lens"),
                          i32_ptr(slots, P + D, "state slots"), (int)P, (int)D, (int)Tp, (int)H,
-                         (int)d, (int)dv, (int)S.size(0), stream());
+                         (int)d, (int)dv, (int)S.size(0), chunk ? &cw : nullptr, stream());
 }
 
 // ---- scaled residual stream, token shift, minGRU, latent attention rows, sigmoid routing --

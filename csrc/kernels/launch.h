@@ -337,13 +337,27 @@ void launch_window_prefill_mfma(int dtype, void* out, const void* q, const void*
                                 const int* work_blk, int n_work, int blk_rows, int H, int G,
                                 int dk, int dv, int krs, int vrs, int bs, int num_blocks, float scale, int window,
                                 int keep_first, const float* gate, WindowExtra ex, hipStream_t s);
+// chunkwise recurrences of prompt rows (chunk_scan.hip): tokens per segment (0: sequences are
+// walked whole), an upper bound of the number of segments, and their workspace (seg > 0):
+// items * H * d * (dv + 1) floats and items * H * 2 doubles
+struct ChunkWork {
+  int seg = 0, items = 0;
+  float* state = nullptr;
+  double* gate = nullptr;
+};
+bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, int H, int d, int dv);
+ChunkWork mlstm_chunk_plan(int dtype, int P, int Tp, int H, int d, int dv);
+void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride, const float* gates,
+                        float* S, float* nst, float* mst, const float* n0, const float* m0,
+                        const int* qsl, const int* seq_lens, const int* slots, int P, int H, int d,
+                        int dv, int num_slots, const ChunkWork& work, hipStream_t s);
 int mlstm_scan_max_dim();
 int64_t mlstm_scan_ws(int seqs, int H, int d);   // floats of workspace
 void launch_mlstm_scan(int dtype, float* out, const void* qkvg, int64_t stride,
                        const float* gates, float* S, float* nst, float* mst, float* ws,
                        const int* qsl, const int* seq_lens, const int* ctx_lens,
                        const int* slots, int P, int D, int Tp, int H, int d, int dv,
-                       int num_slots, hipStream_t s);
+                       int num_slots, const ChunkWork* chunk, hipStream_t s);
 
 // ---- scaled residual stream, token shift, minGRU, latent attention rows, sigmoid routing --
 // `dtype`: activation type of add / proj / zxg ...; `out_dtype`: DT_F32 or the same

@@ -36,7 +36,7 @@ __global__ __launch_bounds__(NT) void mlstm_scan_kernel(
     float* __restrict__ mst, const float* __restrict__ n0, const float* __restrict__ m0,
     const int* __restrict__ qsl, const int* __restrict__ seq_lens,
     const int* __restrict__ ctx_lens, const int* __restrict__ slots, int P, int Tp, int H,
-    int d, int dv, int num_slots) {
+    int d, int dv, int num_slots, int s0) {
   constexpr int NU = (4 * RMAX + 63) / 64;
   constexpr int NQK = (TB * 2 * 4 * RMAX + NT - 1) / NT;   // staged q | k values per thread
   constexpr int NV = TB * 64 / NT;                          // staged v values per thread
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(NT) void mlstm_scan_kernel(
   float* gg = vv + TB * 64;               // [TB][2]: log input gate, log forget gate
   float* dens = gg + TB * 2;              // [TB]
   float* part = dens + TB;                // [TB][NW][64]
-  const int s = blockIdx.x, h = blockIdx.y;
+  const int s = blockIdx.x + s0, h = blockIdx.y;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int col = blockIdx.z * 64 + lane;
   const bool colok = col < dv;
@@ -214,18 +214,14 @@ static size_t scan_lds(int rmax) {
 
 template <typename T>
 void scan_dispatch(float* out, const T* qkvg, int64_t stride, const float* gates, float* S,
-                   float* nst, float* mst, float* ws, const int* qsl, const int* seq_lens,
-                   const int* ctx_lens, const int* slots, int P, int D, int Tp, int H, int d,
-                   int dv, int num_slots, hipStream_t s) {
-  const dim3 grid(P + D, H, (dv + 63) / 64);
-  float* n0 = grid.z > 1 ? ws : nullptr;
-  float* m0 = n0 ? ws + (int64_t)(P + D) * H * d : nullptr;
-  if (n0)
-    mlstm_head_state_kernel<<<dim3(P + D, H), 64, 0, s>>>(n0, m0, nst, mst, slots, H, d, num_slots);
+                   float* nst, float* mst, const float* n0, const float* m0, const int* qsl,
+                   const int* seq_lens, const int* ctx_lens, const int* slots, int P, int D, int Tp,
+                   int H, int d, int dv, int num_slots, int s0, hipStream_t s) {
+  const dim3 grid(P + D - s0, H, (dv + 63) / 64);
 #define KGC_SCAN(R)                                                                          \
   mlstm_scan_kernel<T, R><<<grid, NT, scan_lds(R), s>>>(out, qkvg, stride, gates, S, nst, mst, \
                                                         n0, m0, qsl, seq_lens, ctx_lens, slots, \
-                                                        P, Tp, H, d, dv, num_slots)
+                                                        P, Tp, H, d, dv, num_slots, s0)
   if (d <= 64) KGC_SCAN(16);
   else if (d <= 128) KGC_SCAN(32);
   else if (d <= 256) KGC_SCAN(64);
@@ -242,17 +238,26 @@ void launch_mlstm_scan(int dtype, float* out, const void* qkvg, int64_t stride,
                        const float* gates, float* S, float* nst, float* mst, float* ws,
                        const int* qsl, const int* seq_lens, const int* ctx_lens,
                        const int* slots, int P, int D, int Tp, int H, int d, int dv,
-                       int num_slots, hipStream_t s) {
+                       int num_slots, const ChunkWork* chunk, hipStream_t s) {
   if (P + D <= 0) return;
+  float* n0 = dv > 64 || chunk ? ws : nullptr;
+  float* m0 = n0 ? ws + (int64_t)(P + D) * H * d : nullptr;
+  if (n0)
+    mlstm_head_state_kernel<<<dim3(P + D, H), 64, 0, s>>>(n0, m0, nst, mst, slots, H, d, num_slots);
+  const int s0 = chunk ? P : 0;          // prompt rows go chunkwise, the rest token by token
+  if (chunk)
+    launch_mlstm_chunk(dtype, out, qkvg, stride, gates, S, nst, mst, n0, m0, qsl, seq_lens, slots, P,
+                       H, d, dv, num_slots, *chunk, s);
+  if (P + D <= s0) return;
   if (dtype == DT_BF16)
-    scan_dispatch<bf16>(out, (const bf16*)qkvg, stride, gates, S, nst, mst, ws, qsl, seq_lens,
-                        ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s);
+    scan_dispatch<bf16>(out, (const bf16*)qkvg, stride, gates, S, nst, mst, n0, m0, qsl, seq_lens,
+                        ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s0, s);
   else if (dtype == DT_F16)
-    scan_dispatch<f16>(out, (const f16*)qkvg, stride, gates, S, nst, mst, ws, qsl, seq_lens,
-                       ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s);
+    scan_dispatch<f16>(out, (const f16*)qkvg, stride, gates, S, nst, mst, n0, m0, qsl, seq_lens,
+                       ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s0, s);
   else
-    scan_dispatch<float>(out, (const float*)qkvg, stride, gates, S, nst, mst, ws, qsl, seq_lens,
-                         ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s);
+    scan_dispatch<float>(out, (const float*)qkvg, stride, gates, S, nst, mst, n0, m0, qsl, seq_lens,
+                         ctx_lens, slots, P, D, Tp, H, d, dv, num_slots, s0, s);
 }
 
 // ---- token shift and minGRU over per-sequence state vectors -----------------------------

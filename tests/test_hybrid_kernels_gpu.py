@@ -182,6 +182,80 @@ def test_mlstm_scan_many_workgroups(gpu):
         torch.testing.assert_close(a.cpu(), b, rtol=2e-4, atol=2e-4)
 
 
+def _mlstm64(qkvg, gates, st, m, H, d, dv):
+    """The recurrence in float64, and a bound of what fp32 rounding can do to each result: the
+    sums of absolute values behind numerator and denominator (the same recurrence over |k|,
+    |v|, |q|) in units of 2^-24."""
+    T, P = qkvg.shape[0], m.num_prefills
+    qsl = m.query_start_loc.tolist() if P else [0]
+    seqs = [(qsl[i], qsl[i + 1] - qsl[i], int(m.prefill_seq_lens[i]) - (qsl[i + 1] - qsl[i]))
+            for i in range(P)]
+    seqs += [(qsl[-1] + i, 1, int(c) - 1) for i, c in
+             enumerate(m.decode_ctx_lens.tolist() if m.num_decodes else [])]
+    out, unit = torch.zeros(T, H, dv).double(), torch.zeros(T, H, dv).double()
+    S, n, mm = (x.double().clone() for x in st)
+    SA, nA = S.abs(), n.abs()
+    for (a, ln, p0), slot in zip(seqs, m.state_slots.tolist()):
+        if slot < 0:
+            continue
+        if p0 == 0:
+            for x in (S, n, mm, SA, nA):
+                x[slot] = 0
+        for t in range(a, a + ln):
+            row = qkvg[t].double()
+            q, k = row[: H * d].view(H, d) * d ** -0.5, row[H * d: 2 * H * d].view(H, d)
+            v = row[2 * H * d: 2 * H * d + H * dv].view(H, dv)
+            ig, fg = gates[t, :H].double(), gates[t, H:].double()
+            mn = torch.maximum(fg + mm[slot], ig)
+            f, i = torch.exp(fg + mm[slot] - mn)[:, None], torch.exp(ig - mn)[:, None]
+            mm[slot] = mn
+            S[slot] = f[..., None] * S[slot] + (i * k)[..., None] * v[:, None]
+            SA[slot] = f[..., None] * SA[slot] + (i * k).abs()[..., None] * v.abs()[:, None]
+            n[slot], nA[slot] = f * n[slot] + i * k, f * nA[slot] + (i * k).abs()
+            den = torch.maximum((n[slot] * q).sum(-1).abs(), torch.exp(-mn))[:, None] + 1e-6
+            out[t] = (S[slot] * q[..., None]).sum(1) / den
+            unit[t] = ((SA[slot] * q.abs()[..., None]).sum(1) +
+                       out[t].abs() * (nA[slot] * q.abs()).sum(-1, keepdim=True)) / den
+    return out.view(T, -1), unit.view(T, -1) * 2.0 ** -24, (S, n, mm), (SA, nA, mm.abs() + 16)
+
+
+# (chunk lengths, tokens before them): around the chunk (32 / 64 tokens) and tile (16) edges, a
+# padding sequence, decode rows behind the chunks, and long chunks that are cut into segments
+CHUNKS = [([1, 15, 16, 17, 31, 33], [0, 5, 0, 40, 0, 0], [9, 1]), ([63, 64, 65, 129], [0, 7, 0, 0], []),
+          ([700], [0], []), ([33, 1300], [3, 11], [30])]
+
+
+def _chunk_step(lens, before, D_ctx):
+    n = len(lens) + len(D_ctx)
+    slots = list(range(n))[::-1]
+    if len(lens) > 2:
+        slots[2] = -1                       # a padding sequence
+    return _meta(lens, [a + b for a, b in zip(lens, before)], D_ctx, torch.zeros(n, 1, dtype=torch.int32),
+                 slots), sum(lens) + len(D_ctx), n
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,d,dv", [(2, 128, 40), (1, 128, 128), (1, 256, 144)])
+@pytest.mark.parametrize("lens,before,D_ctx", CHUNKS)
+def test_mlstm_scan_chunkwise(gpu, dt, H, d, dv, lens, before, D_ctx):
+    """Prompt rows on the chunkwise kernel against float64: within 16 units of fp32 rounding of
+    the absolute sums (a chain of n additions comes to about sqrt(n) / 2 of them, and its largest
+    terms are few)."""
+    torch.manual_seed(24)
+    m, T, n = _chunk_step(lens, before, D_ctx)
+    st = (torch.randn(n, H, d, dv) * 0.3, torch.randn(n, H, d) * 0.3, torch.rand(n, H) * 2)
+    qkvg = torch.randn(T, 2 * H * d + 2 * H * dv).to(dt)
+    lf = torch.nn.functional.logsigmoid(torch.randn(T, H) * 2 + 2)
+    lf[::29] = -40.0                        # gates that close
+    gates = torch.cat([torch.randn(T, H) * 3, lf], dim=1)
+    st_g = tuple(x.to(gpu) for x in st)
+    want, unit, st_w, st_u = _mlstm64(qkvg, gates, st, m, H, d, dv)
+    got = ops.mlstm_scan(qkvg.to(gpu), gates.to(gpu), st_g, _to(m, gpu), H, d, dv)
+    assert ((got.double().cpu() - want).abs() <= 16 * unit).all()
+    for a, b, u in zip(st_g, st_w, st_u):
+        assert ((a.double().cpu() - b).abs() <= 16 * 2.0 ** -24 * u).all()
+
+
 @pytest.mark.parametrize("path", ["fast", "simple"])
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,G,dk,dv,window,keep", [(4, 2, 96, 64, 70, 5), (4, 1, 128, 128, 150, 3),
