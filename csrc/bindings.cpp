@@ -1732,13 +1732,23 @@ void ssd_scan(Tensor out, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, T
   TORCH_CHECK(out.is_contiguous() && out.numel() == T * H * V, "kgc.ssd_scan: out [T, H V]");
   TORCH_CHECK(S.is_contiguous() && S.dim() == 4 && S.size(1) == H && S.size(2) == N &&
               S.size(3) == V, "kgc.ssd_scan: state [slots, H, N, V]");
+  const float *al = f32_opt(a_log, H, "a_log"), *db = f32_opt(dt_bias, H, "dt_bias"),
+              *ds = f32_opt(dskip, H, "dskip");
+  const int *ql = i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"), *sl = i32_ptr(seq_lens, P, "seq_lens"),
+            *cl = i32_ptr(ctx_lens, D, "ctx_lens"), *st = i32_ptr(slots, P + D, "state slots");
+  if (kgc::ssd_chunk_ok(xbc.data_ptr<float>(), (int)P, (int)Tp, (int)H, (int)V, (int)N, (int)G)) {
+    kgc::ChunkWork cw = kgc::ssd_chunk_plan((int)P, (int)Tp, (int)H, (int)V, (int)G);
+    Tensor cs, cg;
+    chunk_workspace(cw, H * N * V, H, xbc, cs, cg);
+    kgc::launch_ssd_chunk(dt_code(dt), out.data_ptr<float>(), xbc.data_ptr<float>(), dt.data_ptr(),
+                          dt.stride(0), al, db, ds, S.data_ptr<float>(), ql, sl, st, (int)P, (int)H,
+                          (int)V, (int)N, (int)G, (int)S.size(0), cw, stream());
+    st += P;                             // the decode rows are left
+    P = 0;
+  }
   kgc::launch_ssd_scan(dt_code(dt), out.data_ptr<float>(), xbc.data_ptr<float>(), dt.data_ptr(),
-                       dt.stride(0), f32_opt(a_log, H, "a_log"), f32_opt(dt_bias, H, "dt_bias"),
-                       f32_opt(dskip, H, "dskip"), S.data_ptr<float>(),
-                       i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"),
-                       i32_ptr(seq_lens, P, "seq_lens"), i32_ptr(ctx_lens, D, "ctx_lens"),
-                       i32_ptr(slots, P + D, "state slots"), (int)P, (int)D, (int)Tp, (int)H,
-                       (int)V, (int)N, (int)G, (int)S.size(0), stream());
+                       dt.stride(0), al, db, ds, S.data_ptr<float>(), ql, sl, cl, st, (int)P, (int)D,
+                       (int)Tp, (int)H, (int)V, (int)N, (int)G, (int)S.size(0), stream());
 }
 
 void gated_delta_scan(Tensor out, Tensor qkv, Tensor ba, Tensor a_log, Tensor dt_bias, Tensor S,

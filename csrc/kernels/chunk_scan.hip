@@ -39,29 +39,54 @@ namespace {
 
 constexpr int NT = 512, NW = NT / 64;
 
+// x = sum of NP bf16 parts, each the rounding of what the ones before it leave; two at a time, so
+// that one instruction rounds and packs a pair
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 template <int NP>
-__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[NP]) {
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t (&p)[NP]) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    float r = x[i];
-#pragma unroll
-    for (int j = 0; j < NP; ++j) {
-      const bf16 h = (bf16)r;
-      p[j][i] = h;
-      r -= (float)h;
+  for (int j = 0; j < NP; ++j) {
+    p[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), bf16x2_t));
+    if (j + 1 < NP) {
+      x0 -= __builtin_bit_cast(float, p[j] << 16);
+      x1 -= __builtin_bit_cast(float, p[j] & 0xffff0000u);
     }
   }
 }
-
-// c += a b over the products of parts i, j with i + j <= 2, the small ones first
-template <int NA, int NB>
-__device__ __forceinline__ f32x4 mm(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], f32x4 c) {
+template <int NP>
+__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[NP]) {
+  u32x4 o[NP];
 #pragma unroll
-  for (int s = 2; s >= 0; --s)
+  for (int i = 0; i < 4; ++i) {
+    uint32_t w[NP];
+    split2<NP>(x[2 * i], x[2 * i + 1], w);
+#pragma unroll
+    for (int j = 0; j < NP; ++j) o[j][i] = w[j];
+  }
+#pragma unroll
+  for (int j = 0; j < NP; ++j) p[j] = __builtin_bit_cast(bf16x8, o[j]);
+}
+
+// hi + lo += a b over the products of parts i, j with i + j <= 2.  SEP: the corrections have a sum
+// of their own; added to the main sum one by one, each would round it (SSD: 1.2e-7 from float64,
+// 0.8e-7 so).  One-part operands have but two corrections, and no registers left.
+template <bool SEP, int NA, int NB>
+__device__ __forceinline__ void mm(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], f32x4& hi, f32x4& lo) {
+  f32x4& l = SEP ? lo : hi;
+#pragma unroll
+  for (int s = 2; s >= 1; --s)
 #pragma unroll
     for (int i = 0; i <= s; ++i)
-      if (i < NA && s - i < NB) c = mfma16x16x32(a[i], b[s - i], c);
-  return c;
+      if (i < NA && s - i < NB) l = mfma16x16x32(a[i], b[s - i], l);
+  if constexpr (SEP) hi += mfma16x16x32(a[0], b[0], f32x4{0.f, 0.f, 0.f, 0.f});
+  else hi = mfma16x16x32(a[0], b[0], hi);
+}
+
+// e^x for x <= 0 held in double: the rounding of x to fp32 is put back
+__device__ __forceinline__ float exp_d(double x) {
+  x = x < -1e4 ? -1e4 : x;
+  const float f = (float)x, e = expf(f);
+  return __builtin_fmaf(e, (float)(x - (double)f), e);
 }
 
 template <typename E> struct PartsOf { static constexpr int n = 1; };
@@ -119,8 +144,9 @@ struct ChunkArgs {
   const void *q, *k, *v;            // element (row, group / head, column) at row * stride + h * d + c
   int64_t stride;                   // elements, of all three
   const float* gates;               // mLSTM: [T, 2 H] log input | log forget gate
-  const void* dt;                   // SSD: [T, H] step sizes before softplus
+  const void* dt;                   // SSD: [T, H] step sizes before softplus, of type dt_type
   int64_t dts;
+  int dt_type;
   const float *a_log, *dt_bias, *dskip;
   float *S, *n, *m;
   const float *n0, *m0;             // mLSTM: copies of n and m of the step's sequences
@@ -130,10 +156,6 @@ struct ChunkArgs {
   float* seg_state;                 // [items][H][d (dv + 1)]: S, n of a segment from zero
   double* seg_gate;                 // [items][H][2]: its log decay, its m
 };
-
-__device__ __forceinline__ float softplus_(float x) {      // as the token-serial scan
-  return x > 20.f ? x : log1pf(expf(x));
-}
 
 // Sequence and segment of work item `item` (every lane of every wave gets the same answer)
 struct SegItem { int seq, idx, count, first; };
@@ -165,12 +187,13 @@ __device__ __forceinline__ SegItem seg_item(int item, const int* qsl, int P, int
   return r;
 }
 
-// E: element type of q, k, v; G: element type of dt; MLSTM or SSD; D: padded rows of S; L: chunk;
+// E: element type of q, k, v; MLSTM or SSD; D: padded rows of S; L: chunk;
 // HPW: heads per workgroup.  MODE 0: whole sequences, 1: segments from zero (states only),
 // 2: segments from their predecessors' states.
-template <typename E, typename G, bool MLSTM, int D, int L, int HPW, int MODE>
+template <typename E, bool MLSTM, int D, int L, int HPW, int MODE>
 __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
   constexpr int NP = PartsOf<E>::n;
+  constexpr bool SEP = NP > 1;
   constexpr int DP = D + 8, LP = L + 8;      // padded LDS rows: 16-byte reads without bank conflicts
   constexpr int WPH = NW / HPW;              // waves (column tiles) per head
   constexpr int DT = D / 16, LT = L / 16, KD = D / 32, KL = L / 32;
@@ -265,11 +288,11 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
       asm volatile("" : "+s"(vj));
       if (MLSTM) {
         const double mn = fmax(b + m0, mj);
-        f = expf((float)(b + m0 - mn));
-        g = expf((float)(mj - mn));
+        f = exp_d(b + m0 - mn);
+        g = exp_d(mj - mn);
         m0 = mn;
       } else {
-        f = expf((float)b);
+        f = exp_d(b);
       }
 #pragma unroll
       for (int i = 0; i < DT; ++i)
@@ -288,6 +311,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
   const E* qb = reinterpret_cast<const E*>(a.q) + (int64_t)grp * D;
   const E* kb = reinterpret_cast<const E*>(a.k) + (int64_t)grp * D;
   const E* vb = reinterpret_cast<const E*>(a.v) + (int64_t)h * a.dv + colc;
+  const float skip = MLSTM ? 0.f : a.dskip[h];
   const float qscale = MLSTM ? 1.f / sqrtf((float)D) : 1.f;
   Raw8<E> rq[NU], rk[NU];
   uint32_t rkt[NUT][8];
@@ -325,13 +349,18 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
   // The gates of the chunk at c0, one token per lane, and their running sums (and maxima): wave
   // NW - 1 - hh does them for head hh one chunk ahead, while the scores keep the others busy.
   const int hg = NW - 1 - wave;              // < HPW: the head of this wave's gates
+  const double dt_bias = MLSTM || hg >= HPW ? 0.0 : a.dt_bias[h0 + hg];
+  const double exp_a = MLSTM || hg >= HPW ? 0.0 : exp((double)a.a_log[h0 + hg]);
   auto fetch_gates = [&](int c0) {
     const int64_t t = start + c0 + min(lane, min(L, len - c0) - 1);
     if (MLSTM) {
       gi = a.gates[t * 2 * a.H + h0 + hg];
       gf = a.gates[t * 2 * a.H + a.H + h0 + hg];
     } else {
-      gi = to_f(reinterpret_cast<const G*>(a.dt)[t * a.dts + h0 + hg]);
+      const int64_t at = t * a.dts + h0 + hg;
+      gi = a.dt_type == DT_F32 ? reinterpret_cast<const float*>(a.dt)[at]
+           : a.dt_type == DT_F16 ? (float)reinterpret_cast<const f16*>(a.dt)[at]
+                                 : (float)reinterpret_cast<const bf16*>(a.dt)[at];
     }
   };
   // registers -> LDS
@@ -406,13 +435,16 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
   };
   auto scan_gates = [&](int nl, int buf) {
     const bool ok = lane < nl;
-    if (!MLSTM) {                            // step size and log decay
-      gi = softplus_(gi + a.dt_bias[h0 + hg]);
-      gf = -expf(a.a_log[h0 + hg]) * gi;
-    }
-    if (!ok) gi = gf = 0.f;
     // a decay of e^-1e6 is zero; a finite floor keeps the differences of running sums defined
-    const double b = wave_scan<false>(gf < -1e6f ? -1e6 : (double)gf);
+    double f = gf;
+    if (!MLSTM) {                            // step size and log decay, in double: two of a wave's
+      const double z = (double)gi + dt_bias; // sixteen heads per token, and nobody waits for them
+      const double size = z > 40.0 ? z : log1p(exp(z));
+      gi = (float)size;
+      f = -exp_a * size;
+    }
+    if (!ok) f = gi = 0.f;
+    const double b = wave_scan<false>(f < -1e6 ? -1e6 : f);
     const double bL = lane63(b);
     const int at = (buf * HPW + hg) * L + lane;
     if (MLSTM) {
@@ -422,21 +454,21 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
         rt[at] = -M;
         cs[at] = c;
         pw[at] = qscale;
-        inter[at] = expf((float)(m0 - M)) * qscale;
-        wt[at] = expf((float)(c - ML));
+        inter[at] = exp_d(m0 - M) * qscale;
+        wt[at] = exp_d(c - ML);
         em[buf * L + lane] = expf((float)-(b + M));
       }
-      if (lane == 0) sa[buf * HPW + hg] = expf((float)(m0 - ML));
+      if (lane == 0) sa[buf * HPW + hg] = exp_d(m0 - ML);
       m0 = bL + ML;
     } else {
       if (lane < L) {
         rt[at] = b;
         cs[at] = -b;
         pw[at] = gi;
-        inter[at] = expf((float)b);
-        wt[at] = expf((float)(bL - b)) * gi;
+        inter[at] = exp_d(b);
+        wt[at] = exp_d(bL - b) * gi;
       }
-      if (lane == 0) sa[buf * HPW + hg] = expf((float)bL);
+      if (lane == 0) sa[buf * HPW + hg] = exp_d(bL);
     }
     btot += bL;
   };
@@ -466,6 +498,12 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
         const int s = j * 32 + lg * 8 + i;
         vr[j][i] = vc[min(s, nl - 1) * rs];
       }
+    float xr[LT][4];                         // SSD: x of this lane's outputs, for D x
+    if (!MLSTM && MODE != 1)
+#pragma unroll
+      for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) xr[ti][r] = (float)vc[min(ti * 16 + lg * 4 + r, nl - 1) * rs];
     if (hg < HPW && c0 + L < len) {
       scan_gates(min(L, len - c0 - L), buf ^ 1);
       if (c0 + 2 * L < len) fetch_gates(c0 + 2 * L);
@@ -477,7 +515,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
         int ti = 0;
         while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
         const int si = tile - ti * (ti + 1) / 2;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f}, low = acc;
 #pragma unroll
         for (int ks = 0; ks < KD; ++ks) {
           bf16x8 fa[NP], fb[NP];
@@ -486,9 +524,10 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
             fa[i] = *reinterpret_cast<const bf16x8*>(Ks + i * L * DP + (si * 16 + lr) * DP + ks * 32 + lg * 8);
             fb[i] = *reinterpret_cast<const bf16x8*>(Qs + i * L * DP + (ti * 16 + lr) * DP + ks * 32 + lg * 8);
           }
-          acc = mm<NP, NP>(fa, fb, acc);
+          mm<SEP, NP, NP>(fa, fb, acc, low);
           if (ks % 2 == 1) __builtin_amdgcn_sched_barrier(0);
         }
+        if constexpr (SEP) acc += low;
         const int t = ti * 16 + lr, s0 = si * 16 + lg * 4;
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh) {
@@ -497,9 +536,8 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int s = s0 + r;
-            p[r] = s <= t ? acc[r] * (expf((float)(r0 + csc[hh * L + s])) * pc[hh * L + s]) : 0.f;
+            p[r] = s <= t ? acc[r] * (exp_d(r0 + csc[hh * L + s]) * pc[hh * L + s]) : 0.f;
             sum += p[r];
-            if (!MLSTM && s == t) p[r] += a.dskip[h0 + hh];
           }
           if (MLSTM) {
             sum += __shfl_xor(sum, 16, 64);
@@ -507,18 +545,11 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
             if (lg == 0) psum[si * L + t] = sum;
           }
           bf16* row = Ps + (hh * 3 * L + t) * LP + s0;
-          union { bf16 h[4]; u32x2 u; } o[3];
+          uint32_t lo2[3], hi2[3];
+          split2<3>(p[0], p[1], lo2);
+          split2<3>(p[2], p[3], hi2);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float x = p[r];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-              o[i].h[r] = (bf16)x;
-              x -= (float)o[i].h[r];
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2*>(row + i * L * LP) = o[i].u;
+          for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2*>(row + i * L * LP) = u32x2{lo2[i], hi2[i]};
         }
       }
       if (MLSTM) {                           // n_0 . q_t: NT / L threads per row
@@ -538,10 +569,10 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
         if (sub == 0) nq[t] = x;
       }
     }
-    f32x4 o[LT];
+    f32x4 o[LT], ol[LT];
     if (MODE != 1) {                         // Q S_0 of this wave's columns
 #pragma unroll
-      for (int i = 0; i < LT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < LT; ++i) o[i] = ol[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KD; ++ks) {
         float x[8];
@@ -555,7 +586,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
 #pragma unroll
           for (int i = 0; i < NP; ++i)
             fa[i] = *reinterpret_cast<const bf16x8*>(Qs + i * L * DP + (ti * 16 + lr) * DP + ks * 32 + lg * 8);
-          o[ti] = mm<NP, 3>(fa, sp, o[ti]);
+          mm<SEP, NP, 3>(fa, sp, o[ti], ol[ti]);
         }
         __builtin_amdgcn_sched_barrier(0);   // bounds the operands in flight: registers
       }
@@ -584,7 +615,8 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
       for (int ti = 0; ti < LT; ++ti) {
         const f32x4 f = *reinterpret_cast<const f32x4*>(ic + hw * L + ti * 16 + lg * 4);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[ti][r] *= f[r];
+        for (int r = 0; r < 4; ++r) o[ti][r] = (SEP ? o[ti][r] + ol[ti][r] : o[ti][r]) * f[r];
+        ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
 #pragma unroll
       for (int j = 0; j < KL; ++j) {
@@ -604,7 +636,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
 #pragma unroll
           for (int i = 0; i < 3; ++i)
             fa[i] = *reinterpret_cast<const bf16x8*>(Ps + ((hw * 3 + i) * L + ti * 16 + lr) * LP + j * 32 + lg * 8);
-          o[ti] = mm<3, NP>(fa, vp, o[ti]);
+          mm<SEP, 3, NP>(fa, vp, o[ti], ol[ti]);
         }
       }
 #pragma unroll
@@ -615,33 +647,40 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
         for (int r = 0; r < 4; ++r) {
           const int t = ti * 16 + lg * 4 + r;
           if (t < nl && colok)
-            oc[t * ro] = o[ti][r] * f[r];
+            oc[t * ro] = MLSTM ? (SEP ? o[ti][r] + ol[ti][r] : o[ti][r]) * f[r]
+                               : __builtin_fmaf(skip, xr[ti][r], o[ti][r] + ol[ti][r]);
         }
       }
     }
     const float decay = sa[buf * HPW + hw];
-#pragma unroll
-    for (int i = 0; i < DT; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S[i][r] *= decay;
+    bf16x8 vp[KL][3];
 #pragma unroll
     for (int j = 0; j < KL; ++j) {
       float x[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        x[i] = (float)vr[j][i] * wc[hw * L + j * 32 + lg * 8 + i];
-      }
-      bf16x8 vp[3];
-      split8<3>(x, vp);
+      for (int i = 0; i < 8; ++i) x[i] = (float)vr[j][i] * wc[hw * L + j * 32 + lg * 8 + i];
+      split8<3>(x, vp[j]);
+    }
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
+    for (int dt = 0; dt < DT; ++dt) {
+      // three parts: the update's main product from zero, then one fused step; else it starts from
+      // the decayed state
+      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+      if (NP <= 2)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) hi[r] = S[dt][r] * decay;
+#pragma unroll
+      for (int j = 0; j < KL; ++j) {
         bf16x8 fa[NP];
 #pragma unroll
         for (int i = 0; i < NP; ++i)
           fa[i] = *reinterpret_cast<const bf16x8*>(KT + i * D * LP + (dt * 16 + lr) * LP + j * 32 + lg * 8);
-        S[dt] = mm<NP, 3>(fa, vp, S[dt]);
-        if (dt % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        mm<(NP > 2), NP, 3>(fa, vp[j], hi, lo);
       }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        S[dt][r] = NP > 2 ? __builtin_fmaf(S[dt][r], decay, hi[r] + lo[r]) : hi[r];
+      if (dt % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
     if (MLSTM) {                             // n <- decay n + sum_t w_t k_t: NT / D threads per row
       constexpr int TPD = NT / D;
@@ -701,27 +740,27 @@ constexpr size_t chunk_lds() {
          32 * HPW * L + 4 * (6 * HPW * L + 4 + 3 * L + L / 16 * L + D + NW * L);
 }
 
-template <typename E, typename G, bool MLSTM, int D, int L, int HPW, int MODE>
+template <typename E, bool MLSTM, int D, int L, int HPW, int MODE>
 void chunk_run(const ChunkArgs& a, int items, hipStream_t s) {
   const int nct = (a.dv + 16 * (NW / HPW) - 1) / (16 * (NW / HPW));
   constexpr size_t lds = chunk_lds<E, D, L, HPW>();
   static const bool big = [] {
     return hipFuncSetAttribute(
-               reinterpret_cast<const void*>(&chunk_scan_kernel<E, G, MLSTM, D, L, HPW, MODE>),
+               reinterpret_cast<const void*>(&chunk_scan_kernel<E, MLSTM, D, L, HPW, MODE>),
                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
   }();
   (void)big;
-  chunk_scan_kernel<E, G, MLSTM, D, L, HPW, MODE>
+  chunk_scan_kernel<E, MLSTM, D, L, HPW, MODE>
       <<<dim3(items, a.H / HPW * nct), NT, lds, s>>>(a);
 }
 
-template <typename E, typename G, bool MLSTM, int D, int L, int HPW>
+template <typename E, bool MLSTM, int D, int L, int HPW>
 void chunk_dispatch(const ChunkArgs& a, int items, hipStream_t s) {
   if (a.seg <= 0) {
-    chunk_run<E, G, MLSTM, D, L, HPW, 0>(a, a.P, s);
+    chunk_run<E, MLSTM, D, L, HPW, 0>(a, a.P, s);
   } else {
-    chunk_run<E, G, MLSTM, D, L, HPW, 1>(a, items, s);
-    chunk_run<E, G, MLSTM, D, L, HPW, 2>(a, items, s);
+    chunk_run<E, MLSTM, D, L, HPW, 1>(a, items, s);
+    chunk_run<E, MLSTM, D, L, HPW, 2>(a, items, s);
   }
 }
 
@@ -774,12 +813,48 @@ void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride,
   a.P = P; a.H = H; a.hpg = 1; a.dv = dv; a.num_slots = num_slots;
   a.seg = work.seg; a.seg_state = work.state; a.seg_gate = work.gate;
   if (dtype == DT_BF16) {
-    if (d <= 128) chunk_dispatch<bf16, float, true, 128, 64, 1>(a, work.items, s);
-    else chunk_dispatch<bf16, float, true, 256, 64, 1>(a, work.items, s);
+    if (d <= 128) chunk_dispatch<bf16, true, 128, 64, 1>(a, work.items, s);
+    else chunk_dispatch<bf16, true, 256, 64, 1>(a, work.items, s);
   } else {
-    if (d <= 128) chunk_dispatch<f16, float, true, 128, 32, 1>(a, work.items, s);
-    else chunk_dispatch<f16, float, true, 256, 32, 1>(a, work.items, s);
+    if (d <= 128) chunk_dispatch<f16, true, 128, 32, 1>(a, work.items, s);
+    else chunk_dispatch<f16, true, 256, 32, 1>(a, work.items, s);
   }
+}
+
+// Mamba-2: 128 state rows, fp32 x | B | C (three bf16 parts each), 32-token chunks; two heads of up
+// to 64 columns share a workgroup's B and C.  2 x 8192 tokens, 32 heads of 128 x 64: 4821 us token by
+// token (a chain of 8192 steps in 64 workgroups), 509 us in chunks and segments of 1024; from float64
+// 7.0e-8 (7.3e-8).  Half of that time is vector work, most of it the splits of S, B and C.
+bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G) {
+  return P > 0 && Tp >= 16 * P && N == 128 && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(xbc) & 15) == 0;
+}
+
+static int ssd_heads(int H, int V, int G) { return V <= 64 && (H / G) % 2 == 0 ? 2 : 1; }
+
+ChunkWork ssd_chunk_plan(int P, int Tp, int H, int V, int G) {
+  const int hpw = ssd_heads(H, V, G), cols = 16 * (NW / hpw);
+  return chunk_plan(P, Tp, H / hpw * ((V + cols - 1) / cols), 32);
+}
+
+void launch_ssd_chunk(int dtype, float* out, const float* xbc, const void* dt, int64_t dts,
+                      const float* a_log, const float* dt_bias, const float* dskip, float* S,
+                      const int* qsl, const int* seq_lens, const int* slots, int P, int H, int V,
+                      int N, int G, int num_slots, const ChunkWork& work, hipStream_t s) {
+  ChunkArgs a{};
+  a.out = out;
+  a.v = xbc;
+  a.k = xbc + (int64_t)H * V;
+  a.q = xbc + (int64_t)H * V + (int64_t)G * N;
+  a.stride = (int64_t)H * V + 2 * (int64_t)G * N;
+  a.dt = dt; a.dts = dts; a.dt_type = dtype;
+  a.a_log = a_log; a.dt_bias = dt_bias; a.dskip = dskip;
+  a.S = S;
+  a.qsl = qsl; a.seq_lens = seq_lens; a.slots = slots;
+  a.P = P; a.H = H; a.hpg = H / G; a.dv = V; a.num_slots = num_slots;
+  a.seg = work.seg; a.seg_state = work.state; a.seg_gate = work.gate;
+  if (ssd_heads(H, V, G) == 2) chunk_dispatch<float, false, 128, 32, 2>(a, work.items, s);
+  else chunk_dispatch<float, false, 128, 32, 1>(a, work.items, s);
 }
 
 }  // namespace kgc

@@ -351,6 +351,12 @@ void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride,
                         float* S, float* nst, float* mst, const float* n0, const float* m0,
                         const int* qsl, const int* seq_lens, const int* slots, int P, int H, int d,
                         int dv, int num_slots, const ChunkWork& work, hipStream_t s);
+bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G);
+ChunkWork ssd_chunk_plan(int P, int Tp, int H, int V, int G);
+void launch_ssd_chunk(int dtype, float* out, const float* xbc, const void* dt, int64_t dts,
+                      const float* a_log, const float* dt_bias, const float* dskip, float* S,
+                      const int* qsl, const int* seq_lens, const int* slots, int P, int H, int V,
+                      int N, int G, int num_slots, const ChunkWork& work, hipStream_t s);
 int mlstm_scan_max_dim();
 int64_t mlstm_scan_ws(int seqs, int H, int d);   // floats of workspace
 void launch_mlstm_scan(int dtype, float* out, const void* qkvg, int64_t stride,

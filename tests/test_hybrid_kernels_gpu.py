@@ -186,16 +186,11 @@ def _mlstm64(qkvg, gates, st, m, H, d, dv):
     """The recurrence in float64, and a bound of what fp32 rounding can do to each result: the
     sums of absolute values behind numerator and denominator (the same recurrence over |k|,
     |v|, |q|) in units of 2^-24."""
-    T, P = qkvg.shape[0], m.num_prefills
-    qsl = m.query_start_loc.tolist() if P else [0]
-    seqs = [(qsl[i], qsl[i + 1] - qsl[i], int(m.prefill_seq_lens[i]) - (qsl[i + 1] - qsl[i]))
-            for i in range(P)]
-    seqs += [(qsl[-1] + i, 1, int(c) - 1) for i, c in
-             enumerate(m.decode_ctx_lens.tolist() if m.num_decodes else [])]
+    T = qkvg.shape[0]
     out, unit = torch.zeros(T, H, dv).double(), torch.zeros(T, H, dv).double()
     S, n, mm = (x.double().clone() for x in st)
     SA, nA = S.abs(), n.abs()
-    for (a, ln, p0), slot in zip(seqs, m.state_slots.tolist()):
+    for (a, ln, p0), slot in zip(_step_rows(m), m.state_slots.tolist()):
         if slot < 0:
             continue
         if p0 == 0:
@@ -254,6 +249,69 @@ def test_mlstm_scan_chunkwise(gpu, dt, H, d, dv, lens, before, D_ctx):
     assert ((got.double().cpu() - want).abs() <= 16 * unit).all()
     for a, b, u in zip(st_g, st_w, st_u):
         assert ((a.double().cpu() - b).abs() <= 16 * 2.0 ** -24 * u).all()
+
+
+def _step_rows(m):
+    """(first row, rows, position of the first) of every step sequence."""
+    qsl = m.query_start_loc.tolist() if m.num_prefills else [0]
+    seqs = [(qsl[i], qsl[i + 1] - qsl[i], int(m.prefill_seq_lens[i]) - (qsl[i + 1] - qsl[i]))
+            for i in range(m.num_prefills)]
+    return seqs + [(qsl[-1] + i, 1, c - 1) for i, c in
+                   enumerate(m.decode_ctx_lens.tolist() if m.num_decodes else [])]
+
+
+def _matrix64(m, S, q, k, v, decay, beta=None):
+    """S_t = decay_t S + k u^T, o = S^T q in float64 (u = v, or beta (v - S^T k) of the decayed S)
+    with the sums of absolute values behind o and S in units of 2^-24: q, k [T, H, d], v [T, H, dv],
+    decay [T, H, 1 or d], S [slots, H, d, dv]."""
+    out, unit = torch.zeros_like(v), torch.zeros_like(v)
+    S = S.double().clone()
+    SA = S.abs()
+    for (a, ln, p0), slot in zip(_step_rows(m), m.state_slots.tolist()):
+        if slot < 0:
+            continue
+        if p0 == 0:
+            S[slot], SA[slot] = 0, 0
+        for t in range(a, a + ln):
+            x, xa = decay[t][..., None] * S[slot], decay[t][..., None] * SA[slot]
+            u, ua = v[t], v[t].abs()
+            if beta is not None:
+                u = beta[t][:, None] * (u - (x * k[t][..., None]).sum(1))
+                ua = beta[t][:, None] * (ua + (xa * k[t].abs()[..., None]).sum(1))
+            S[slot], SA[slot] = x + k[t][..., None] * u[:, None], xa + k[t].abs()[..., None] * ua[:, None]
+            out[t] = (S[slot] * q[t][..., None]).sum(1)
+            unit[t] = (SA[slot] * q[t].abs()[..., None]).sum(1)
+    return out.flatten(1), unit.flatten(1) * 2.0 ** -24, S, SA * 2.0 ** -24
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("H,G,V", [(2, 1, 64), (4, 2, 40), (3, 3, 144)])
+@pytest.mark.parametrize("lens,before,D_ctx", CHUNKS)
+def test_ssd_scan_chunkwise(gpu, dt, H, G, V, lens, before, D_ctx):
+    """Prompt rows on the chunkwise kernel against float64 (the bound: see the mLSTM's test); two
+    heads per workgroup, heads of odd widths and heads that do not pair up."""
+    torch.manual_seed(25)
+    N = 128
+    m, T, n = _chunk_step(lens, before, D_ctx)
+    S = torch.randn(n, H, N, V) * 0.3
+    xbc, dtv = torch.randn(T, H * V + 2 * G * N), torch.randn(T, H + 5).to(dt)[:, 5:]
+    a_log, dtb, skip = torch.rand(H) * 2, torch.randn(H) - 2, torch.randn(H)
+    a_log[0] = 12.0                         # decays that forget everything at every token
+    x, B, C = (y.double() for y in xbc.split([H * V, G * N, G * N], 1))
+    size = torch.nn.functional.softplus(dtv.double() + dtb.double())
+    each = lambda y: y.view(T, G, N).repeat_interleave(H // G, 1)   # noqa: E731
+    x = x.view(T, H, V)
+    want, unit, S_w, S_u = _matrix64(m, S, each(C), each(B) * size[..., None], x,
+                                     torch.exp(-torch.exp(a_log.double()) * size)[..., None])
+    live = torch.zeros(T, 1)
+    for (a, ln, _), slot in zip(_step_rows(m), m.state_slots.tolist()):
+        live[a: a + ln] = slot >= 0
+    add = (skip.double()[:, None] * x).flatten(1) * live
+    S_g = S.to(gpu)
+    got = ops.ssd_scan(xbc.to(gpu), dtv.to(gpu), a_log.to(gpu), dtb.to(gpu), skip.to(gpu), S_g, _to(m, gpu),
+                       H, V, N, G)
+    assert ((got.double().cpu() - want - add).abs() <= 16 * (unit + add.abs() * 2.0 ** -24)).all()
+    assert ((S_g.double().cpu() - S_w).abs() <= 16 * S_u).all()
 
 
 @pytest.mark.parametrize("path", ["fast", "simple"])
