@@ -1770,13 +1770,24 @@ void gated_delta_scan(Tensor out, Tensor qkv, Tensor ba, Tensor a_log, Tensor dt
   TORCH_CHECK(out.is_contiguous() && out.numel() == T * H * V, "kgc.gated_delta_scan: out [T, H V]");
   TORCH_CHECK(S.is_contiguous() && S.dim() == 4 && S.size(1) == H && S.size(2) == d &&
               S.size(3) == V, "kgc.gated_delta_scan: state [slots, H, d, V]");
+  const float *al = f32_opt(a_log, H, "a_log"), *db = f32_opt(dt_bias, H, "dt_bias");
+  const int *ql = i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"), *sl = i32_ptr(seq_lens, P, "seq_lens"),
+            *cl = i32_ptr(ctx_lens, D, "ctx_lens"), *st = i32_ptr(slots, P + D, "state slots");
+  if (kgc::delta_chunk_ok(qkv.data_ptr<float>(), (int)P, (int)Tp, (int)H, (int)G, (int)d, (int)V)) {
+    const kgc::DeltaWork w = kgc::delta_chunk_plan((int)P, (int)Tp, (int)H, (int)G, (int)V);
+    Tensor wp = at::empty({w.wp}, qkv.options().dtype(at::kBFloat16));
+    Tensor ws = at::empty({w.floats}, qkv.options());
+    kgc::launch_delta_chunk(dt_code(ba), out.data_ptr<float>(), qkv.data_ptr<float>(), ba.data_ptr(),
+                            ba.stride(0), al, db, S.data_ptr<float>(), ql, sl, st, (int)P, (int)Tp,
+                            (int)H, (int)G, (int)V, (int)S.size(0), w, wp.data_ptr(),
+                            ws.data_ptr<float>(), stream());
+    st += P;                             // the decode rows are left
+    P = 0;
+  }
   kgc::launch_gated_delta_scan(dt_code(ba), out.data_ptr<float>(), qkv.data_ptr<float>(),
-                               ba.data_ptr(), ba.stride(0), f32_opt(a_log, H, "a_log"),
-                               f32_opt(dt_bias, H, "dt_bias"), S.data_ptr<float>(),
-                               i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"),
-                               i32_ptr(seq_lens, P, "seq_lens"), i32_ptr(ctx_lens, D, "ctx_lens"),
-                               i32_ptr(slots, P + D, "state slots"), (int)P, (int)D, (int)Tp,
-                               (int)H, (int)G, (int)d, (int)V, (int)S.size(0), stream());
+                               ba.data_ptr(), ba.stride(0), al, db, S.data_ptr<float>(), ql, sl, cl,
+                               st, (int)P, (int)D, (int)Tp, (int)H, (int)G, (int)d, (int)V,
+                               (int)S.size(0), stream());
 }
 
 void gated_rms_norm(Tensor out, Tensor y, Tensor gate, Tensor w, int64_t groups, double eps,

@@ -1,0 +1,121 @@
+// Shared by the chunkwise recurrences (chunk_scan.hip, chunk_delta.hip): fp32 operands of the bf16
+// matrix cores as sums of bf16 parts, wave-wide running sums in double, and the mapping of work
+// items to pieces of ragged sequences.
+#pragma once
+#include "common.h"
+
+namespace kgc {
+
+// x = sum of NP bf16 parts, each the rounding of what the ones before it leave; two at a time, so
+// that one instruction rounds and packs a pair
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <int NP>
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t (&p)[NP]) {
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    p[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), bf16x2_t));
+    if (j + 1 < NP) {
+      x0 -= __builtin_bit_cast(float, p[j] << 16);
+      x1 -= __builtin_bit_cast(float, p[j] & 0xffff0000u);
+    }
+  }
+}
+template <int NP>
+__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[NP]) {
+  u32x4 o[NP];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t w[NP];
+    split2<NP>(x[2 * i], x[2 * i + 1], w);
+#pragma unroll
+    for (int j = 0; j < NP; ++j) o[j][i] = w[j];
+  }
+#pragma unroll
+  for (int j = 0; j < NP; ++j) p[j] = __builtin_bit_cast(bf16x8, o[j]);
+}
+
+// hi + lo += a b over the products of parts i, j with i + j <= 2.  SEP: the corrections have a sum
+// of their own; added to the main sum one by one, each would round it (SSD: 1.2e-7 from float64,
+// 0.8e-7 so).  One-part operands have but two corrections, and no registers left.
+template <bool SEP, int NA, int NB>
+__device__ __forceinline__ void mm(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], f32x4& hi, f32x4& lo) {
+  f32x4& l = SEP ? lo : hi;
+#pragma unroll
+  for (int s = 2; s >= 1; --s)
+#pragma unroll
+    for (int i = 0; i <= s; ++i)
+      if (i < NA && s - i < NB) l = mfma16x16x32(a[i], b[s - i], l);
+  if constexpr (SEP) hi += mfma16x16x32(a[0], b[0], f32x4{0.f, 0.f, 0.f, 0.f});
+  else hi = mfma16x16x32(a[0], b[0], hi);
+}
+
+// e^x for x <= 0 held in double: the reduction to 2^n 2^f is exact to fp32 however large x is, so
+// the error is that of the hardware's 2^f, |f| <= 1/2
+__device__ __forceinline__ float exp_d(double x) {
+  const double y = (x < -1e4 ? -1e4 : x) * 1.4426950408889634074, n = __builtin_rint(y);
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((float)(y - n)), (int)n);
+}
+
+// inclusive running sum (MAX: maximum) over the 64 lanes, by row shifts and row broadcasts
+template <int CTRL, int ROWS, bool MAX> __device__ __forceinline__ double scan_step(double x) {
+  const double none = MAX ? -INFINITY : 0.0;
+  const uint64_t o = __builtin_bit_cast(uint64_t, none), b = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_update_dpp((uint32_t)o, (uint32_t)b, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp((uint32_t)(o >> 32), (uint32_t)(b >> 32), CTRL, ROWS,
+                                                  0xf, false);
+  const double y = __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+  return MAX ? fmax(x, y) : x + y;
+}
+template <bool MAX> __device__ __forceinline__ double wave_scan(double x) {
+  x = scan_step<0x111, 0xf, MAX>(x);         // row_shr 1, 2, 4, 8
+  x = scan_step<0x112, 0xf, MAX>(x);
+  x = scan_step<0x114, 0xf, MAX>(x);
+  x = scan_step<0x118, 0xf, MAX>(x);
+  x = scan_step<0x142, 0xa, MAX>(x);         // row_bcast 15 into rows 1 and 3
+  return scan_step<0x143, 0xc, MAX>(x);      // row_bcast 31 into rows 2 and 3
+}
+__device__ __forceinline__ double lane63(double x) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, 63);
+  const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), 63);
+  return __builtin_bit_cast(double, hi << 32 | lo);
+}
+
+// Sequence and segment of work item `item` (every lane of every wave gets the same answer)
+struct SegItem { int seq, idx, count, first; };
+__device__ __forceinline__ SegItem seg_item(int item, const int* qsl, int P, int seg) {
+  SegItem r{-1, 0, 0, 0};
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int p0 = 0; p0 < P; p0 += 64) {
+    const int p = p0 + lane;
+    const int n = p < P ? max(1, (qsl[p + 1] - qsl[p] + seg - 1) / seg) : 0;
+    int inc = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += y;
+    }
+    const int total = __shfl(inc, 63, 64);
+    if (item < base + total) {
+      const unsigned long long hit = __ballot(base + inc > item);
+      const int l = __ffsll((unsigned long long)hit) - 1;
+      r.seq = p0 + l;
+      r.count = __shfl(n, l, 64);
+      r.first = base + __shfl(inc, l, 64) - r.count;
+      r.idx = item - r.first;
+      return r;
+    }
+    base += total;
+  }
+  return r;
+}
+
+// column c of a k index that MFMAs read permuted, so that accumulators are operands as they lie:
+// the 4-column pieces of every 32 go in the order 0 4 1 5 2 6 3 7
+__device__ __forceinline__ int mfma_perm(int c) {
+  const int p = (c >> 2) & 7;
+  return (c & ~31) | ((((p & 3) << 1) | (p >> 2)) << 2) | (c & 3);
+}
+
+}  // namespace kgc

@@ -1,0 +1,604 @@
+// Chunkwise gated delta rule of prompt rows on the matrix cores.  Per (sequence, head), with unit
+// keys k_t, a decay g_t and a write strength beta_t,
+//     u_t = beta_t (v_t - g_t S_(t-1)^T k_t),   S_t = g_t S_(t-1) + k_t u_t^T,   o_t = S_t^T q_t .
+// Over a chunk of L = 32 tokens, b_t the running sum of ln g, gamma_t = e^(b_t) and S_0 the state
+// before it, the u of the chunk solve a unit lower triangular system:
+//     (I + A) U = diag(beta) (V - diag(gamma) K S_0),   A_ts = beta_t e^(b_t - b_s) k_t . k_s  (s < t)
+//     O   = diag(gamma) Q S_0 + P U,                    P_ts = e^(b_t - b_s) q_t . k_s         (s <= t)
+//     S_L = gamma_L S_0 + sum_s e^(b_L - b_s) k_s u_s^T
+// W = (I + A)^-1 diag(beta) and P depend on no state: a first launch computes them for all chunks at
+// once (a lane per column of the triangular inverse), as bf16 parts in the order the walk's MFMAs
+// read them.  The walk then has no serial step finer than a chunk: a workgroup of 8 waves owns 128
+// value columns of a head, a wave 16 of them with their S in accumulators, and everything between
+// two stagings of k and q concerns one wave's columns only:
+//     R = V - gamma K S_0,  U = W R,  O = gamma Q S_0 + P U,  S = gamma_L S_0 + K^T U.
+// Accumulators are B operands as they lie (mfma_perm), so R, U and S never pass through LDS.
+//
+// Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each, six products of parts,
+// the corrections summed apart; exponents are differences of running sums kept in double.
+//
+// Few long sequences are cut into segments: a chunk walk is linear in its state, so a first pass
+// walks every segment from zero (with its values) and from the identity (without), a second chains
+// S <- M_j S + dS_j over the segments, and the third walks all segments from their own states.
+#include "chunk.h"
+#include "launch.h"
+
+namespace kgc {
+
+namespace {
+
+constexpr int L = 32, D = 128;               // tokens per chunk, key channels
+constexpr int NT = 512, NW = NT / 64;
+constexpr int DT = D / 16, LT = L / 16, KD = D / 32;
+constexpr int DP = D + 8, LP = L + 8;        // padded LDS rows
+constexpr int MAT = 3 * L * L;               // bf16 of one matrix of a chunk: three parts
+
+struct DeltaArgs {
+  float* out;                                // [T, H dv]
+  const float* qkv;                          // [T, 2 G D + H dv]
+  int64_t stride;
+  const void* ba;                            // [T, 2 H]: write strength | decay, before activation
+  int64_t bas;
+  int ba_type;
+  const float *a_log, *dt_bias;
+  float* S;
+  const int *qsl, *seq_lens, *slots;
+  int P, H, G, dv, num_slots;
+  // workspace
+  bf16* wp;                                  // [chunks][H][W, P][3][L][L], columns permuted
+  // per token of a chunk, zero past the sequence's end:
+  float* gam;                                // [chunks][H][L]: gamma_t
+  double* kw;                                // [chunks][H][L]: e^(b_L - b_t) times rk
+  float *rk, *rq;                            // [chunks][G][L]: what makes k and q unit (q: d^-1/2 too)
+  int seg;                                   // tokens per segment (0: sequences are not cut)
+  float* seg_state;                          // [items][H][D][dv + D]: dS | M of a segment
+  float* seg_in;                             // [items][H][D][dv]: the state a segment starts from
+};
+
+__device__ __forceinline__ float ld_ba(const DeltaArgs& a, int64_t at) {
+  return a.ba_type == DT_F32 ? reinterpret_cast<const float*>(a.ba)[at]
+         : a.ba_type == DT_F16 ? (float)reinterpret_cast<const f16*>(a.ba)[at]
+                               : (float)reinterpret_cast<const bf16*>(a.ba)[at];
+}
+
+// chunks of the sequences before `seq`
+__device__ __forceinline__ int chunks_before(int seq, const int* qsl) {
+  const int lane = threadIdx.x & 63;
+  int n = 0;
+  for (int p = lane; p < seq; p += 64) n += max(1, (qsl[p + 1] - qsl[p] + L - 1) / L);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+  return n;
+}
+
+// inclusive running sum within each half of the wave
+__device__ __forceinline__ double half_scan(double x) {
+  x = scan_step<0x111, 0xf, false>(x);
+  x = scan_step<0x112, 0xf, false>(x);
+  x = scan_step<0x114, 0xf, false>(x);
+  x = scan_step<0x118, 0xf, false>(x);
+  return scan_step<0x142, 0xa, false>(x);
+}
+
+// between writing and reading LDS within one wave: its LDS operations execute in order
+__device__ __forceinline__ void wave_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// ---- W, P, the gates and the norms of every chunk: one wave per (chunk, q / k group) -----------
+__global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
+  __shared__ float KK[L][L + 1], QK[L][L + 1];           // [t][s]: dots of unit vectors, s <= t
+  __shared__ __align__(16) float X[2][L][L + 4];  // P, A, then W of two heads at a time
+  __shared__ double bs[2][L];
+  __shared__ float be[2][L], rks[L];
+  const SegItem it = seg_item(blockIdx.x, a.qsl, a.P, L);
+  if (it.seq < 0) return;
+  const int g = blockIdx.y, lane = threadIdx.x, lr = lane & 15, lg = lane >> 4;
+  const int c0 = it.idx * L, len = a.qsl[it.seq + 1] - a.qsl[it.seq];
+  const int nl = min(L, len - c0);
+  const int slot = a.slots[it.seq];
+  if (nl <= 0 || slot < 0 || slot >= a.num_slots || a.seq_lens[it.seq] < len) return;
+  const int64_t t0 = a.qsl[it.seq] + c0;
+  const float* qb = a.qkv + t0 * a.stride + g * D;
+  const float* kb = qb + (int64_t)a.G * D;
+  const int rs = (int)a.stride, hpg = a.H / a.G;
+
+  const int hf = lane >> 5;                  // this lane: column (and token) s of head h0 + hf
+  int s = lane & 31;
+  const int64_t row = (t0 + min(s, nl - 1)) * a.bas;
+  auto head = [&](int h0) { return g * hpg + min(h0 + hf, hpg - 1); };
+  float gx = ld_ba(a, row + head(0)), gz = ld_ba(a, row + a.H + head(0));   // land during the dots
+  float gb = a.dt_bias[head(0)], ga = a.a_log[head(0)];
+
+  // dots: tiles (0, 0), (1, 0), (1, 1) as D[s][t]; the squares of the same elements give the norms
+  f32x4 dk[3], dkl[3], dq[3], dql[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) dk[i] = dkl[i] = dq[i] = dql[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  double n2[2][2] = {{0.0, 0.0}, {0.0, 0.0}};             // [k, q][tile]
+#pragma unroll
+  for (int j = 0; j < KD; ++j) {
+    bf16x8 f[2][2][3];
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int ti = 0; ti < LT; ++ti) {
+        const float* p = (w ? qb : kb) + min(ti * 16 + lr, nl - 1) * rs + j * 32 + lg * 8;
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(p), x1 = *reinterpret_cast<const f32x4*>(p + 4);
+        const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) n2[w][ti] = __builtin_fma((double)x[i], (double)x[i], n2[w][ti]);
+        split8<3>(x, f[w][ti]);
+      }
+#pragma unroll
+    for (int tile = 0; tile < 3; ++tile) {
+      const int ti = tile > 0, si = tile > 1;
+      mm<true, 3, 3>(f[0][si], f[0][ti], dk[tile], dkl[tile]);
+      mm<true, 3, 3>(f[0][si], f[1][ti], dq[tile], dql[tile]);
+    }
+  }
+  float rn[2][2];
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti) {
+      double n = n2[w][ti];
+      n += __shfl_xor(n, 16, 64);
+      n += __shfl_xor(n, 32, 64);
+      rn[w][ti] = (float)(1.0 / sqrt((n + 1e-6) * (w ? D : 1)));
+      const int t = ti * 16 + lr;
+      if (lg == 0) {
+        (w ? a.rq : a.rk)[((int64_t)blockIdx.x * a.G + g) * L + t] = t < nl ? rn[w][ti] : 0.f;
+        if (w == 0) rks[t] = rn[w][ti];
+      }
+    }
+#pragma unroll
+  for (int tile = 0; tile < 3; ++tile) {
+    const int ti = tile > 0, si = tile > 1, t = ti * 16 + lr;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int c = si * 16 + lg * 4 + r;
+      const float f = __shfl(rn[0][si], lg * 4 + r, 64);
+      KK[t][c] = (dk[tile][r] + dkl[tile][r]) * (f * rn[0][ti]);
+      QK[t][c] = (dq[tile][r] + dql[tile][r]) * (f * rn[1][ti]);
+    }
+  }
+  wave_lds();
+
+  for (int h0 = 0; h0 < hpg; h0 += 2) {
+    const bool on = h0 + hf < hpg;
+    const int h = head(h0);
+    const bool ok = s < nl;
+    const float x = gx;
+    const double z = (double)gz + (double)gb;
+    double f = -exp((double)ga) * (z > 40.0 ? z : log1p(exp(z)));
+    if (h0 + 2 < hpg) {
+      gx = ld_ba(a, row + head(h0 + 2));
+      gz = ld_ba(a, row + a.H + head(h0 + 2));
+      gb = a.dt_bias[head(h0 + 2)];
+      ga = a.a_log[head(h0 + 2)];
+    }
+    // a decay of e^-1e6 is zero; a finite floor keeps the differences of running sums defined
+    const double b = half_scan(!ok ? 0.0 : f < -1e6 ? -1e6 : f);
+    const uint64_t bb = __builtin_bit_cast(uint64_t, b);
+    const uint32_t bl = __shfl((int)(uint32_t)bb, 31 + 32 * hf, 64), bh = __shfl((int)(bb >> 32), 31 + 32 * hf, 64);
+    const double bL = __builtin_bit_cast(double, (uint64_t)bh << 32 | bl);
+    const float beta = ok ? 1.f / (1.f + expf(-x)) : 0.f;
+    bs[hf][s] = b;
+    be[hf][s] = beta;
+    if (on) {
+      a.gam[((int64_t)blockIdx.x * a.H + h) * L + s] = ok ? (float)exp(b) : 0.f;
+      a.kw[((int64_t)blockIdx.x * a.H + h) * L + s] = ok ? exp(bL - b) * rks[s] : 0.0;
+    }
+    wave_lds();
+    // a matrix in X as three parts, eight (permuted) columns per store
+    auto put = [&](int mat) {
+      for (int u = lane; u < 2 * L * 4; u += 64) {
+        const int oct = u & 3, t = (u >> 2) & 31, hh = u >> 7;
+        if (h0 + hh >= hpg) continue;
+        const float* src = X[hh][t] + oct * 4;                      // pieces oct and oct + 4 of the row
+        const f32x4 p0 = *reinterpret_cast<const f32x4*>(src), p1 = *reinterpret_cast<const f32x4*>(src + 16);
+        const float y[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
+        bf16x8 o[3];
+        split8<3>(y, o);
+        bf16* dst = a.wp + (((int64_t)blockIdx.x * a.H + g * hpg + h0 + hh) * 2 + mat) * MAT + t * L + oct * 8;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(dst + i * L * L) = o[i];
+      }
+      wave_lds();
+    };
+    asm volatile("" : "+v"(s));               // masks are made where they are used, not kept
+    float e[L];
+#pragma unroll
+    for (int t = 0; t < L; ++t) {
+      e[t] = t >= s ? exp_d(bs[hf][t] - b) : 0.f;
+      X[hf][t][s] = t >= s ? e[t] * QK[t][s] : 0.f;
+    }
+    wave_lds();
+    put(1);
+    asm volatile("" : "+v"(s));
+#pragma unroll
+    for (int t = 0; t < L; ++t) X[hf][t][s] = t > s ? be[hf][t] * e[t] * KK[t][s] : 0.f;
+    wave_lds();
+    asm volatile("" : "+v"(s));
+    // column s of (I + A)^-1, from the top; rows of A are read by all lanes of a half together
+    float T[L];
+#pragma unroll
+    for (int t = 0; t < L; ++t) {
+      float x[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < t; j += 4) {
+        const f32x4 r = *reinterpret_cast<const f32x4*>(&X[hf][t][j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (j + i < t) x[i] += r[i] * T[j + i];
+      }
+      T[t] = t == s ? 1.f : t < s ? 0.f : -((x[0] + x[1]) + (x[2] + x[3]));
+    }
+    wave_lds();
+#pragma unroll
+    for (int t = 0; t < L; ++t) X[hf][t][s] = T[t] * beta;
+    wave_lds();
+    put(0);
+  }
+}
+
+// ---- the walk.  MODE 0: whole sequences; 1: segments from zero and from the identity (states
+// only); 2: segments from seg_in -----------------------------------------------------------------
+template <int MODE>
+__global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
+  __shared__ __align__(16) bf16 Ks[3 * L * DP], Qs[MODE == 1 ? 8 : 3 * L * DP], KT[3 * D * LP];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  int seq = blockIdx.x, seg_idx = 0, item = 0, seg_count = 1;
+  if (MODE != 0) {
+    const SegItem it = seg_item(blockIdx.x, a.qsl, a.P, a.seg);
+    if (it.seq < 0) return;
+    seq = it.seq;
+    seg_idx = it.idx;
+    seg_count = it.count;
+    item = it.first + it.idx;
+    if (MODE == 1 && seg_idx + 1 == seg_count) return;
+  }
+  const int nct = (a.dv + 127) / 128 + (MODE == 1);       // MODE 1: the last block is the identity's
+  const int h = blockIdx.y / nct, ct = blockIdx.y - h * nct, g = h / (a.H / a.G);
+  const bool ident = MODE == 1 && ct + 1 == nct;
+  const int col = (ident ? 0 : ct * 128) + wave * 16 + lr;
+  const bool colok = ident || col < a.dv;
+  const int colc = colok ? col : a.dv - 1;                // columns off the edge: read the last
+  const int seq0 = a.qsl[seq];
+  int start = seq0, len = a.qsl[seq + 1] - start;
+  const int pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
+  const int64_t os = (int64_t)a.H * a.dv;
+  const int chunk0 = chunks_before(seq, a.qsl) + (MODE != 0 ? seg_idx * (a.seg / L) : 0);
+  if (MODE != 0) {
+    start += seg_idx * a.seg;
+    len = min(a.seg, len - seg_idx * a.seg);
+  }
+  if (len <= 0) return;
+  if (slot < 0 || slot >= a.num_slots || pos0 < 0) {      // padding: defined zeros
+    if (MODE != 1 && colok)
+      for (int t = lg; t < len; t += 4) a.out[(start + t) * os + (int64_t)h * a.dv + col] = 0.f;
+    return;
+  }
+  f32x4 S[DT];
+  float* Ss = a.S + ((int64_t)slot * a.H + h) * D * a.dv;
+  {
+    const float* from = MODE == 2 ? a.seg_in + ((int64_t)item * a.H + h) * D * a.dv : Ss;
+    const bool zero = MODE == 1 || (MODE == 0 && pos0 == 0);
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = i * 16 + 4 * lg + r;
+        S[i][r] = zero ? (ident && row == col ? 1.f : 0.f) : from[row * a.dv + colc];
+      }
+  }
+  const float* qb = a.qkv + g * D;
+  const float* kb = qb + (int64_t)a.G * D;
+  const float* vb = a.qkv + 2 * (int64_t)a.G * D + (int64_t)h * a.dv;
+  const int vo = ident ? 0 : colc;
+  int rs = (int)a.stride, ro = (int)os;
+
+  // Staging: a thread takes 8 columns of one row of q and k, and 8 tokens of one column of k, in
+  // both cases the pieces 4 a .. and 16 + 4 a .. of 32: adjacent in the permuted order, one store.
+  // Rows past the sequence's end read its last (their factors are zero).
+  f32x4 rqv[2], rkv[2], rt[2];
+  double kw[8];
+  float nk = 0.f, nq = 0.f;
+  const int ut = tid / 16, uc = (tid % 16 / 4) * 32 + (tid % 4) * 4, up_ = (tid % 16) * 8;
+  const int ta = tid / D * 4, tc = tid % D;
+  auto fetch = [&](int c0, int ci) {
+    const int nl = min(L, len - c0);
+    const float* kr = kb + (int64_t)(start + c0) * a.stride;
+    const float* qr = qb + (int64_t)(start + c0) * a.stride;
+    const int at = __mul24(min(ut, nl - 1), rs) + uc;
+    rkv[0] = *reinterpret_cast<const f32x4*>(kr + at);
+    rkv[1] = *reinterpret_cast<const f32x4*>(kr + at + 16);
+    nk = a.rk[((int64_t)ci * a.G + g) * L + ut];
+    if (MODE != 1) {
+      rqv[0] = *reinterpret_cast<const f32x4*>(qr + at);
+      rqv[1] = *reinterpret_cast<const f32x4*>(qr + at + 16);
+      nq = a.rq[((int64_t)ci * a.G + g) * L + ut];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      rt[i >> 2][i & 3] = kr[__mul24(min(ta + (i >> 2) * 16 + (i & 3), nl - 1), rs) + tc];
+    const double* w = a.kw + ((int64_t)ci * a.H + h) * L + ta;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) kw[i] = w[(i >> 2) * 16 + (i & 3)];
+  };
+  auto park = [&]() {
+#pragma unroll
+    for (int w = 0; w < (MODE == 1 ? 1 : 2); ++w) {
+      const f32x4* v = w ? rqv : rkv;
+      const float f = w ? nq : nk;
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = v[i >> 2][i & 3] * f;
+      bf16x8 p[3];
+      split8<3>(x, p);
+      bf16* base = (w ? Qs : Ks) + ut * DP + up_;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(base + i * L * DP) = p[i];
+    }
+    // k^T times the weight of its token in the update, tokens permuted: U is the B operand as it lies
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = (float)(rt[i >> 2][i & 3] * kw[i]);
+    bf16x8 p[3];
+    split8<3>(x, p);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(KT + (i * D + tc) * LP + ta * 2) = p[i];
+  };
+
+  fetch(0, chunk0);
+  for (int c0 = 0, ci = chunk0; c0 < len; c0 += L, ++ci) {
+    const int nl = min(L, len - c0);
+    asm volatile("" : "+s"(rs), "+s"(ro));   // row offsets are computed per chunk, not kept
+    park();
+    __syncthreads();
+    const int64_t t0 = start + c0;
+    // this lane's v and gammas (rows 4 lg + r of each tile), and its fragments of W and P
+    const float* vc = vb + t0 * a.stride;
+    const float* gc = a.gam + ((int64_t)ci * a.H + h) * L;
+    float v[LT][4];
+    f32x4 gm[LT];
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti) {
+      gm[ti] = *reinterpret_cast<const f32x4*>(gc + ti * 16 + lg * 4);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        v[ti][r] = vc[__mul24(min(ti * 16 + lg * 4 + r, nl - 1), rs) + vo];
+    }
+    const float gL = gc[nl - 1];
+    const bf16* wp = a.wp + ((int64_t)ci * a.H + h) * 2 * MAT + lr * L + lg * 8;
+    bf16x8 fw[LT][3], fp[LT][3];
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        fw[ti][i] = *reinterpret_cast<const bf16x8*>(wp + i * L * L + ti * 16 * L);
+
+    f32x4 r[LT], rl[LT], o[LT], ol[LT];
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti) r[ti] = rl[ti] = o[ti] = ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < KD; ++j) {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = S[2 * j + (i >> 2)][i & 3];
+      bf16x8 sp[3];
+      split8<3>(x, sp);
+#pragma unroll
+      for (int ti = 0; ti < LT; ++ti) {
+        bf16x8 fa[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          fa[i] = *reinterpret_cast<const bf16x8*>(Ks + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
+        mm<true, 3, 3>(fa, sp, r[ti], rl[ti]);
+        if (MODE != 1) {
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+            fa[i] = *reinterpret_cast<const bf16x8*>(Qs + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
+          mm<true, 3, 3>(fa, sp, o[ti], ol[ti]);
+        }
+      }
+    }
+    // P, then the next chunk (the last one again at the end: a branch here would make every later
+    // wait one for all loads), land while U is computed
+    if (MODE != 1)
+#pragma unroll
+      for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          fp[ti][i] = *reinterpret_cast<const bf16x8*>(wp + MAT + i * L * L + ti * 16 * L);
+    {
+      const bool more = c0 + L < len;
+      fetch(more ? c0 + L : c0, more ? ci + 1 : ci);
+    }
+    // R, U = W R (rows past the end: W is zero there)
+    bf16x8 up[3];
+    {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int ti = i >> 2, e = i & 3;
+        x[i] = __builtin_fmaf(-gm[ti][e], r[ti][e] + rl[ti][e], ident ? 0.f : v[ti][e]);
+      }
+      if (nl < L)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if ((i >> 2) * 16 + lg * 4 + (i & 3) >= nl) x[i] = 0.f;
+      bf16x8 rp[3];
+      split8<3>(x, rp);
+#pragma unroll
+      for (int ti = 0; ti < LT; ++ti) {
+        f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+        mm<true, 3, 3>(fw[ti], rp, hi, lo);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[ti * 4 + e] = hi[e] + lo[e];
+      }
+      split8<3>(x, up);
+    }
+    if (MODE != 1) {
+      float* oc = a.out + t0 * os + (int64_t)h * a.dv;
+#pragma unroll
+      for (int ti = 0; ti < LT; ++ti) {
+        f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+        mm<true, 3, 3>(fp[ti], up, hi, lo);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          o[ti][e] = __builtin_fmaf(gm[ti][e], o[ti][e] + ol[ti][e], hi[e] + lo[e]);
+      }
+      if (colok) {
+        const int at = lg * 4 * ro + col;
+#pragma unroll
+        for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (nl == L || ti * 16 + lg * 4 + e < nl) (oc + (ti * 16 + e) * ro)[at] = o[ti][e];
+      }
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      bf16x8 fa[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        fa[i] = *reinterpret_cast<const bf16x8*>(KT + (i * D + dt * 16 + lr) * LP + lg * 8);
+      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+      mm<true, 3, 3>(fa, up, hi, lo);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[dt][e] = __builtin_fmaf(S[dt][e], gL, hi[e] + lo[e]);
+    }
+    __syncthreads();
+  }
+
+  if (MODE == 1 || MODE == 0 || seg_idx + 1 == seg_count) {
+    // MODE 1: dS and M side by side
+    const int w = MODE == 1 ? a.dv + D : a.dv;
+    float* dst = MODE == 1 ? a.seg_state + ((int64_t)item * a.H + h) * D * w + (ident ? a.dv : 0) : Ss;
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (colok) dst[(i * 16 + 4 * lg + e) * w + col] = S[i][e];
+  }
+}
+
+// ---- S_in of every segment: S <- M_j S + dS_j, a wave per 16 columns of one (sequence, head) ----
+__global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
+  const int lane = threadIdx.x, lr = lane & 15, lg = lane >> 4;
+  const int seq = blockIdx.x, h = blockIdx.y, col = blockIdx.z * 16 + lr;
+  const bool colok = col < a.dv;
+  const int colc = colok ? col : a.dv - 1;
+  const int len = a.qsl[seq + 1] - a.qsl[seq], pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
+  if (len <= 0 || slot < 0 || slot >= a.num_slots || pos0 < 0) return;
+  int first = 0;                             // segments of the sequences before this one
+  for (int p = lane; p < seq; p += 64) first += max(1, (a.qsl[p + 1] - a.qsl[p] + a.seg - 1) / a.seg);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) first += __shfl_xor(first, o, 64);
+  const int count = (len + a.seg - 1) / a.seg, w = a.dv + D;
+  const float* Ss = a.S + ((int64_t)slot * a.H + h) * D * a.dv;
+  f32x4 S[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S[i][e] = pos0 == 0 ? 0.f : Ss[(i * 16 + 4 * lg + e) * a.dv + colc];
+  for (int j = 0; j < count; ++j) {
+    const int64_t ih = (int64_t)(first + j) * a.H + h;
+    float* dst = a.seg_in + ih * D * a.dv;
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (colok) dst[(i * 16 + 4 * lg + e) * a.dv + col] = S[i][e];
+    if (j + 1 == count) break;
+    const float* st = a.seg_state + ih * D * w;
+    bf16x8 sp[KD][3];
+#pragma unroll
+    for (int k = 0; k < KD; ++k) {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = S[2 * k + (i >> 2)][i & 3];
+      split8<3>(x, sp[k]);
+    }
+#pragma unroll
+    for (int i = 0; i < DT; ++i) {
+      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+#pragma unroll
+      for (int k = 0; k < KD; ++k) {         // row i * 16 + lr of M, columns in the permuted order
+        const float* m = st + (i * 16 + lr) * w + a.dv + k * 32 + lg * 4;
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = m[(e >> 2) * 16 + (e & 3)];
+        bf16x8 fa[3];
+        split8<3>(x, fa);
+        mm<true, 3, 3>(fa, sp[k], hi, lo);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[i][e] = hi[e] + lo[e] + st[(i * 16 + 4 * lg + e) * w + colc];
+    }
+  }
+}
+
+}  // namespace
+
+// Chunkwise for 128 key channels, from 24 rows per sequence on or a thousand in all (16 rows of one
+// sequence: 19 us token by token, 32 us here; 48 rows: 43 and 37 us; 64 x 20 rows: 101 and 69 us).
+// 16 x 1000 tokens of 16 heads with 128 x 128 states: 1328 us token by token, 288 us chunkwise (71 us
+// for W and P); 2 x 8192: 7.5 ms and 0.9 ms.  The walk issues 1000 vector instructions and 168 MFMAs
+// per wave and chunk, 13 k of its 15 k cycles.
+bool delta_chunk_ok(const float* qkv, int P, int Tp, int H, int G, int d, int V) {
+  return P > 0 && (Tp >= 24 * P || Tp >= 1024) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(qkv) & 15) == 0;
+}
+
+DeltaWork delta_chunk_plan(int P, int Tp, int H, int G, int V) {
+  DeltaWork w;
+  w.items = P;
+  const int chunks = Tp / L + P, wgs = H * ((V + 127) / 128);
+  w.wp = (int64_t)chunks * H * 2 * MAT;
+  w.floats = (int64_t)chunks * L * (3 * H + 2 * G);
+  const int want = (256 + wgs - 1) / wgs;    // items for one workgroup per CU
+  if (P * 3 > want) return w;
+  int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
+  seg = (seg + L - 1) / L * L;
+  if (seg < 8 * L) seg = 8 * L;
+  if (Tp / P < 3 * seg) return w;
+  w.seg = seg;
+  w.items = Tp / seg + P;
+  w.floats += (int64_t)w.items * H * D * (2 * (int64_t)V + D);
+  return w;
+}
+
+void launch_delta_chunk(int dtype, float* out, const float* qkv, const void* ba, int64_t bas,
+                        const float* a_log, const float* dt_bias, float* S, const int* qsl,
+                        const int* seq_lens, const int* slots, int P, int Tp, int H, int G, int V,
+                        int num_slots, const DeltaWork& work, void* wp, float* ws, hipStream_t s) {
+  DeltaArgs a{};
+  a.out = out; a.qkv = qkv; a.stride = 2 * (int64_t)G * D + (int64_t)H * V;
+  a.ba = ba; a.bas = bas; a.ba_type = dtype;
+  a.a_log = a_log; a.dt_bias = dt_bias; a.S = S;
+  a.qsl = qsl; a.seq_lens = seq_lens; a.slots = slots;
+  a.P = P; a.H = H; a.G = G; a.dv = V; a.num_slots = num_slots;
+  a.wp = (bf16*)wp;
+  const int64_t rows = (int64_t)(Tp / L + P) * L;
+  a.kw = reinterpret_cast<double*>(ws);
+  a.gam = ws + 2 * rows * H;
+  a.rk = a.gam + rows * H;
+  a.rq = a.rk + rows * G;
+  a.seg = work.seg;
+  a.seg_state = a.rq + rows * G;
+  a.seg_in = a.seg_state + (int64_t)work.items * H * D * (V + D);
+  delta_prep_kernel<<<dim3(Tp / L + P, G), 64, 0, s>>>(a);
+  const int nct = (V + 127) / 128;
+  if (work.seg <= 0) {
+    delta_walk_kernel<0><<<dim3(P, H * nct), NT, 0, s>>>(a);
+  } else {
+    delta_walk_kernel<1><<<dim3(work.items, H * (nct + 1)), NT, 0, s>>>(a);
+    delta_chain_kernel<<<dim3(P, H, (V + 15) / 16), 64, 0, s>>>(a);
+    delta_walk_kernel<2><<<dim3(work.items, H * nct), NT, 0, s>>>(a);
+  }
+}
+
+}  // namespace kgc

@@ -30,7 +30,7 @@
 // Few long sequences: the walk is serial, so a step of few workgroups is cut into segments.  A
 // first launch computes every segment's contribution from a zero state, the second starts each
 // segment from the sum of its predecessors' decayed contributions.
-#include "common.h"
+#include "chunk.h"
 #include "launch.h"
 
 namespace kgc {
@@ -38,56 +38,6 @@ namespace kgc {
 namespace {
 
 constexpr int NT = 512, NW = NT / 64;
-
-// x = sum of NP bf16 parts, each the rounding of what the ones before it leave; two at a time, so
-// that one instruction rounds and packs a pair
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-template <int NP>
-__device__ __forceinline__ void split2(float x0, float x1, uint32_t (&p)[NP]) {
-#pragma unroll
-  for (int j = 0; j < NP; ++j) {
-    p[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), bf16x2_t));
-    if (j + 1 < NP) {
-      x0 -= __builtin_bit_cast(float, p[j] << 16);
-      x1 -= __builtin_bit_cast(float, p[j] & 0xffff0000u);
-    }
-  }
-}
-template <int NP>
-__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[NP]) {
-  u32x4 o[NP];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t w[NP];
-    split2<NP>(x[2 * i], x[2 * i + 1], w);
-#pragma unroll
-    for (int j = 0; j < NP; ++j) o[j][i] = w[j];
-  }
-#pragma unroll
-  for (int j = 0; j < NP; ++j) p[j] = __builtin_bit_cast(bf16x8, o[j]);
-}
-
-// hi + lo += a b over the products of parts i, j with i + j <= 2.  SEP: the corrections have a sum
-// of their own; added to the main sum one by one, each would round it (SSD: 1.2e-7 from float64,
-// 0.8e-7 so).  One-part operands have but two corrections, and no registers left.
-template <bool SEP, int NA, int NB>
-__device__ __forceinline__ void mm(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], f32x4& hi, f32x4& lo) {
-  f32x4& l = SEP ? lo : hi;
-#pragma unroll
-  for (int s = 2; s >= 1; --s)
-#pragma unroll
-    for (int i = 0; i <= s; ++i)
-      if (i < NA && s - i < NB) l = mfma16x16x32(a[i], b[s - i], l);
-  if constexpr (SEP) hi += mfma16x16x32(a[0], b[0], f32x4{0.f, 0.f, 0.f, 0.f});
-  else hi = mfma16x16x32(a[0], b[0], hi);
-}
-
-// e^x for x <= 0 held in double: the rounding of x to fp32 is put back
-__device__ __forceinline__ float exp_d(double x) {
-  x = x < -1e4 ? -1e4 : x;
-  const float f = (float)x, e = expf(f);
-  return __builtin_fmaf(e, (float)(x - (double)f), e);
-}
 
 template <typename E> struct PartsOf { static constexpr int n = 1; };
 template <> struct PartsOf<f16> { static constexpr int n = 2; };
@@ -114,31 +64,6 @@ template <> struct Raw8<float> {
   __device__ __forceinline__ float get(int i) const { return i < 4 ? a[i] : b[i - 4]; }
 };
 
-// inclusive running sum (MAX: maximum) over the 64 lanes, by row shifts and row broadcasts
-template <int CTRL, int ROWS, bool MAX> __device__ __forceinline__ double scan_step(double x) {
-  const double none = MAX ? -INFINITY : 0.0;
-  const uint64_t o = __builtin_bit_cast(uint64_t, none), b = __builtin_bit_cast(uint64_t, x);
-  const uint32_t lo = __builtin_amdgcn_update_dpp((uint32_t)o, (uint32_t)b, CTRL, ROWS, 0xf, false);
-  const uint32_t hi = __builtin_amdgcn_update_dpp((uint32_t)(o >> 32), (uint32_t)(b >> 32), CTRL, ROWS,
-                                                  0xf, false);
-  const double y = __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
-  return MAX ? fmax(x, y) : x + y;
-}
-template <bool MAX> __device__ __forceinline__ double wave_scan(double x) {
-  x = scan_step<0x111, 0xf, MAX>(x);         // row_shr 1, 2, 4, 8
-  x = scan_step<0x112, 0xf, MAX>(x);
-  x = scan_step<0x114, 0xf, MAX>(x);
-  x = scan_step<0x118, 0xf, MAX>(x);
-  x = scan_step<0x142, 0xa, MAX>(x);         // row_bcast 15 into rows 1 and 3
-  return scan_step<0x143, 0xc, MAX>(x);      // row_bcast 31 into rows 2 and 3
-}
-__device__ __forceinline__ double lane63(double x) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, x);
-  const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, 63);
-  const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), 63);
-  return __builtin_bit_cast(double, hi << 32 | lo);
-}
-
 struct ChunkArgs {
   float* out;                       // [T, H dv]
   const void *q, *k, *v;            // element (row, group / head, column) at row * stride + h * d + c
@@ -156,36 +81,6 @@ struct ChunkArgs {
   float* seg_state;                 // [items][H][d (dv + 1)]: S, n of a segment from zero
   double* seg_gate;                 // [items][H][2]: its log decay, its m
 };
-
-// Sequence and segment of work item `item` (every lane of every wave gets the same answer)
-struct SegItem { int seq, idx, count, first; };
-__device__ __forceinline__ SegItem seg_item(int item, const int* qsl, int P, int seg) {
-  SegItem r{-1, 0, 0, 0};
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  for (int p0 = 0; p0 < P; p0 += 64) {
-    const int p = p0 + lane;
-    const int n = p < P ? max(1, (qsl[p + 1] - qsl[p] + seg - 1) / seg) : 0;
-    int inc = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += y;
-    }
-    const int total = __shfl(inc, 63, 64);
-    if (item < base + total) {
-      const unsigned long long hit = __ballot(base + inc > item);
-      const int l = __ffsll((unsigned long long)hit) - 1;
-      r.seq = p0 + l;
-      r.count = __shfl(n, l, 64);
-      r.first = base + __shfl(inc, l, 64) - r.count;
-      r.idx = item - r.first;
-      return r;
-    }
-    base += total;
-  }
-  return r;
-}
 
 // E: element type of q, k, v; MLSTM or SSD; D: padded rows of S; L: chunk;
 // HPW: heads per workgroup.  MODE 0: whole sequences, 1: segments from zero (states only),
@@ -270,11 +165,6 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
     if (MODE == 1) m0 = -INFINITY;
     else if (!fresh) m0 = a.m0[(int64_t)seq * a.H + h];
   }
-  // position of column c of q, k and n in the permuted order: 4-column pieces 0 4 1 5 2 6 3 7
-  auto perm = [](int c) {
-    const int p = (c >> 2) & 7;
-    return (c & ~31) | ((((p & 3) << 1) | (p >> 2)) << 2) | (c & 3);
-  };
   float nreg = 0.f;                          // mLSTM: n[tid] for tid < D
   if (MLSTM && tid < D && !zero) nreg = a.n0[((int64_t)seq * a.H + h) * D + tid];
   if (MODE == 2) {
@@ -304,7 +194,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
       if (MLSTM && tid < D) nreg = f * nreg + g * sp[sh + tid];
     }
   }
-  if (MLSTM && tid < D) ns[perm(tid)] = nreg;
+  if (MLSTM && tid < D) ns[mfma_perm(tid)] = nreg;
   for (int i = tid; i < HPW * 3 * L * LP / 8; i += NT)           // tiles above the diagonal stay zero
     reinterpret_cast<u32x4*>(Ps)[i] = u32x4{0, 0, 0, 0};
 
@@ -374,7 +264,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
           rq[j].zero();
           rk[j].zero();
         }
-        const int at0 = t * DP + perm(c), at1 = t * DP + perm(c + 4);
+        const int at0 = t * DP + mfma_perm(c), at1 = t * DP + mfma_perm(c + 4);
 #pragma unroll
         for (int w = 0; w < 2; ++w) {
           const Raw8<E>& x = w ? rk[j] : rq[j];
@@ -696,7 +586,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
         }
 #pragma unroll
       for (int o = 1; o < TPD; o <<= 1) x += __shfl_xor(x, o, 64);
-      if (sub == 0) ns[perm(c)] = sa[buf * HPW] * ns[perm(c)] + x;
+      if (sub == 0) ns[mfma_perm(c)] = sa[buf * HPW] * ns[mfma_perm(c)] + x;
     }
     __syncthreads();
   }
@@ -718,7 +608,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
     if (ct == 0) {
       if (MLSTM && tid < D) {
         float* nd = MODE == 1 ? dst + sh : a.n + ((int64_t)slot * a.H + h) * D;
-        nd[tid] = ns[perm(tid)];
+        nd[tid] = ns[mfma_perm(tid)];
       }
       if (hg < HPW && lane == 0) {
         const int64_t ih = (int64_t)(seg_first + seg_idx) * a.H + h0 + hg;
@@ -775,7 +665,7 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L) {
   // and the pieces are long enough to pay for computing every contribution twice
   const int want = (256 + wgs - 1) / wgs;
   if (P * 2 > want) return p;
-  int seg = (Tp + want - 1) / want;
+  int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
   seg = (seg + L - 1) / L * L;
   if (seg < 4 * L) seg = 4 * L;
   if (Tp / P < 2 * seg) return p;
@@ -785,7 +675,7 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L) {
 }
 
 // Chunkwise from 16 rows per sequence on, heads of 128 or 256 key channels in 16 bits (fp32 rows in
-// three parts do not fit LDS).  32 x 512 tokens, 4 heads of 256 x 512: 1957 us token by token, 233 us
+// three parts do not fit LDS).  32 x 512 tokens, 4 heads of 256 x 512: 1957 us token by token, 219 us
 // chunkwise, and nearer to float64 (3.5e-7 against 4.7e-7).
 bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, int H, int d, int dv) {
   return (dtype == DT_BF16 || dtype == DT_F16) && P > 0 && Tp >= 16 * P && (d == 128 || d == 256) &&
@@ -823,7 +713,7 @@ void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride,
 
 // Mamba-2: 128 state rows, fp32 x | B | C (three bf16 parts each), 32-token chunks; two heads of up
 // to 64 columns share a workgroup's B and C.  2 x 8192 tokens, 32 heads of 128 x 64: 4821 us token by
-// token (a chain of 8192 steps in 64 workgroups), 509 us in chunks and segments of 1024; from float64
+// token (a chain of 8192 steps in 64 workgroups), 353 us in chunks and segments of 1184; from float64
 // 7.0e-8 (7.3e-8).  Half of that time is vector work, most of it the splits of S, B and C.
 bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G) {
   return P > 0 && Tp >= 16 * P && N == 128 && V >= 16 && ((int64_t)H * V) % 4 == 0 &&

@@ -357,6 +357,18 @@ void launch_ssd_chunk(int dtype, float* out, const float* xbc, const void* dt, i
                       const float* a_log, const float* dt_bias, const float* dskip, float* S,
                       const int* qsl, const int* seq_lens, const int* slots, int P, int H, int V,
                       int N, int G, int num_slots, const ChunkWork& work, hipStream_t s);
+// gated delta rule of prompt rows (chunk_delta.hip): segments as above, bf16 values of `wp` and floats
+// of `ws`
+struct DeltaWork {
+  int seg = 0, items = 0;
+  int64_t wp = 0, floats = 0;
+};
+bool delta_chunk_ok(const float* qkv, int P, int Tp, int H, int G, int d, int V);
+DeltaWork delta_chunk_plan(int P, int Tp, int H, int G, int V);
+void launch_delta_chunk(int dtype, float* out, const float* qkv, const void* ba, int64_t bas,
+                        const float* a_log, const float* dt_bias, float* S, const int* qsl,
+                        const int* seq_lens, const int* slots, int P, int Tp, int H, int G, int V,
+                        int num_slots, const DeltaWork& work, void* wp, float* ws, hipStream_t s);
 int mlstm_scan_max_dim();
 int64_t mlstm_scan_ws(int seqs, int H, int d);   // floats of workspace
 void launch_mlstm_scan(int dtype, float* out, const void* qkvg, int64_t stride,

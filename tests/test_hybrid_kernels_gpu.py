@@ -314,6 +314,36 @@ def test_ssd_scan_chunkwise(gpu, dt, H, G, V, lens, before, D_ctx):
     assert ((S_g.double().cpu() - S_w).abs() <= 16 * S_u).all()
 
 
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("H,G,V", [(2, 1, 128), (3, 3, 40), (3, 1, 144)])
+@pytest.mark.parametrize("lens,before,D_ctx", CHUNKS)
+def test_gated_delta_scan_chunkwise(gpu, dt, H, G, V, lens, before, D_ctx):
+    """Prompt rows on the chunkwise kernel against float64: keys that are nearly parallel (the
+    triangular systems are then as large as they get), heads that share keys in twos, threes and
+    not at all.  The bound is that of the mLSTM's test, doubled for the value that is read before
+    the write."""
+    torch.manual_seed(26)
+    d = 128
+    m, T, n = _chunk_step(lens, before, D_ctx)
+    S = torch.randn(n, H, d, V) * 0.3
+    qkv = torch.randn(T, 2 * G * d + H * V)
+    qkv[:, G * d: 2 * G * d] += 2 * torch.randn(G * d)
+    ba = torch.randn(T, 2 * H + 5).to(dt)[:, 5:]
+    a_log, dtb = torch.rand(H) * 2, torch.randn(H) - 2
+    a_log[-1] = 12.0                        # decays that forget everything at every token
+    q, k, v = (y.double() for y in qkv.split([G * d, G * d, H * V], 1))
+    unit = lambda y: y * torch.rsqrt(y.pow(2).sum(-1, keepdim=True) + 1e-6)   # noqa: E731
+    each = lambda y: unit(y.view(T, G, d)).repeat_interleave(H // G, 1)   # noqa: E731
+    size = torch.nn.functional.softplus(ba[:, H:].double() + dtb.double())
+    want, bound, S_w, S_u = _matrix64(m, S, each(q) * d ** -0.5, each(k), v.view(T, H, V),
+                                      torch.exp(-torch.exp(a_log.double()) * size)[..., None],
+                                      torch.sigmoid(ba[:, :H].double()))
+    S_g = S.to(gpu)
+    got = ops.gated_delta_scan(qkv.to(gpu), ba.to(gpu), a_log.to(gpu), dtb.to(gpu), S_g, _to(m, gpu), H, G, d, V)
+    assert ((got.double().cpu() - want).abs() <= 32 * bound).all()
+    assert ((S_g.double().cpu() - S_w).abs() <= 32 * S_u).all()
+
+
 @pytest.mark.parametrize("path", ["fast", "simple"])
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,G,dk,dv,window,keep", [(4, 2, 96, 64, 70, 5), (4, 1, 128, 128, 150, 3),
