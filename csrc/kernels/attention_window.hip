@@ -23,8 +23,7 @@
 //   pool_kv           mean rows of the blocks that a step's tokens complete
 #include <algorithm>
 
-#include "common.h"
-#include "launch.h"
+#include "window.h"
 
 namespace kgc {
 
@@ -122,12 +121,6 @@ __global__ __launch_bounds__(256) void norm_kv_store_kernel(
   }
 }
 
-// first position that a query at `pos` sees
-__device__ __forceinline__ int first_visible(int pos, int window, bool chunked) {
-  if (window <= 0) return 0;
-  return chunked ? pos - pos % window : max(0, pos - window + 1);
-}
-
 // whole blocks of `pool` tokens that end before the window of a query at `pos`
 __device__ __forceinline__ int pooled_count(int pos, int window, int pool) {
   const int n = pos - window + 1;
@@ -187,19 +180,6 @@ __device__ __forceinline__ int turn_partner(int c, int dv, bool inter) {
 }
 
 constexpr int MAX_DV_PER_LANE = 16;    // dv <= 1024
-
-// scaled score -> cap * tanh(score / cap) when a cap is set
-__device__ __forceinline__ float cap_score(float s, float cap) {
-  return cap > 0.f ? cap * tanhf(s / cap) : s;
-}
-
-// sigmoid of the element-wise output gate at (row t, column c of the concatenated heads)
-template <typename T>
-__device__ __forceinline__ float elem_gate(const WindowExtra& ex, int64_t t, int c) {
-  if (ex.egate == nullptr) return 1.f;
-  const float g = to_f(static_cast<const T*>(ex.egate)[t * ex.egs + c]);
-  return 1.f / (1.f + expf(-g));
-}
 
 // grid (T, H), one wave.  LDS: q row [dk] fp32, p [64], value-row offsets [64], and with
 // rotated values the output row [dv].
@@ -1681,6 +1661,10 @@ void launch_window_prefill_mfma(int dtype, void* out, const void* q, const void*
                                 int dk, int dv, int krs, int vrs, int bs, int num_blocks, float scale, int window,
                                 int keep_first, const float* gate, WindowExtra ex, hipStream_t s) {
   if (n_work <= 0) return;
+  if (launch_window_prefill_gqa(dtype, out, q, k_cache, v_cache, qsl, seq_lens, pbt, bt_stride, work_seq,
+                                work_blk, n_work, blk_rows, H, G, dk, dv, krs, vrs, bs, num_blocks, scale,
+                                window, keep_first, gate, ex, s))
+    return;
   if (dtype == DT_BF16)
     prefill_dispatch<bf16>((bf16*)out, (const bf16*)q, (const bf16*)k_cache,
                            (const bf16*)v_cache, qsl, seq_lens, pbt, bt_stride, work_seq,

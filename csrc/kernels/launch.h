@@ -331,6 +331,13 @@ void launch_window_decode_mfma(int dtype, void* out, const void* q, const void* 
                                int vrs, int bs, int num_blocks, float scale, int window,
                                int keep_first, const float* gate, WindowExtra ex, hipStream_t s);
 bool window_prefill_mfma_ok(int dtype, int dk, int dv);
+// false: not its shape
+bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* kc, const void* vc,
+                               const int* qsl, const int* seq_lens, const int* pbt, int bt_stride,
+                               const int* work_seq, const int* work_blk, int n_work, int blk_rows, int H,
+                               int G, int dk, int dv, int krs, int vrs, int bs, int num_blocks, float scale,
+                               int window, int keep_first, const float* gate, const WindowExtra& ex,
+                               hipStream_t s);
 void launch_window_prefill_mfma(int dtype, void* out, const void* q, const void* k_cache,
                                 const void* v_cache, const int* qsl, const int* seq_lens,
                                 const int* pbt, int bt_stride, const int* work_seq,

@@ -1,0 +1,27 @@
+// Shared by the windowed attention kernels (attention_window.hip, window_prefill.hip).
+#pragma once
+#include "common.h"
+#include "launch.h"
+
+namespace kgc {
+
+// first position that a query at `pos` sees
+__device__ __forceinline__ int first_visible(int pos, int window, bool chunked) {
+  if (window <= 0) return 0;
+  return chunked ? pos - pos % window : max(0, pos - window + 1);
+}
+
+// scaled score -> cap * tanh(score / cap) when a cap is set
+__device__ __forceinline__ float cap_score(float s, float cap) {
+  return cap > 0.f ? cap * tanhf(s / cap) : s;
+}
+
+// sigmoid of the element-wise output gate at (row t, column c of the concatenated heads)
+template <typename T>
+__device__ __forceinline__ float elem_gate(const WindowExtra& ex, int64_t t, int c) {
+  if (ex.egate == nullptr) return 1.f;
+  const float g = to_f(static_cast<const T*>(ex.egate)[t * ex.egs + c]);
+  return 1.f / (1.f + expf(-g));
+}
+
+}  // namespace kgc

@@ -409,3 +409,37 @@ def test_window_attention_many_decode_rows(gpu, dt):
     got = ops.window_attention(q.to(gpu), kc.to(gpu), vc.to(gpu), pos.to(gpu), _to(m, gpu), 0.2,
                                window, keep, None)
     torch.testing.assert_close(got.cpu().float(), want.float(), **_tol(dt))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,latent,bs,kw", [
+    (8, 2, False, 8, dict(window=0, keep=0, softcap=20.0)), (4, 1, False, 16, dict(window=70, keep=5)),
+    (8, 1, False, 8, dict(window=64, keep=70)), (4, 1, False, 24, dict(window=48, keep=0, chunked=True, sink=0.4)),
+    (8, 1, True, 8, dict(window=100, keep=0)), (4, 1, True, 32, dict(window=0, keep=0))])
+def test_window_attention_shared_tiles(gpu, dt, H, G, latent, bs, kw):
+    """Prompt rows where four heads share a key/value head: row counts around the wave (32), block
+    (64) and work item (128) edges, contexts that start inside a page and a tile, rows with one
+    visible key, kept tokens in tiles of their own and inside the window, pages of no power of two;
+    latent rows hold keys and values.  One rounding of the result to 16 bits (and of the weights'
+    pairs: 2^-17 of sums of values around 1)."""
+    torch.manual_seed(31)
+    dk, dv = (256, 192) if latent else (128, 128)
+    P_q, old = [1, 31, 33, 64, 65, 129, 150], [0, 90, 7, 0, 130, 0, 63]
+    P_sl, T = [a + b for a, b in zip(P_q, old)], sum(P_q)
+    width = max(P_sl) // bs + 1
+    nb = len(P_q) * width + 1
+    tables = (torch.randperm(nb - 1) + 1).view(len(P_q), width).int()
+    kc = torch.randn(nb, G, bs, dk).to(dt)
+    vc = kc[..., :dv] if latent else torch.randn(nb, G, bs, dv).to(dt)
+    m = _meta(P_q, P_sl, [], tables)
+    pos = torch.cat([torch.arange(o, o + a) for a, o in zip(P_q, old)])
+    q = torch.randn(T, H, dk).to(dt)
+    gate, eg = torch.rand(T, H), torch.randn(T, H * dv + 8).to(dt)[:, 8:]
+    kw = dict(kw)
+    args = (0.08, kw.pop("window"), kw.pop("keep"), gate)
+    want = ops.window_attention(q, kc, vc, pos, m, *args, elem_gate=eg, out_scale=1.3, **kw)
+    kg = kc.to(gpu)
+    got = ops.window_attention(q.to(gpu), kg, kg[..., :dv] if latent else vc.to(gpu), pos.to(gpu), _to(m, gpu),
+                               0.08, args[1], args[2], gate.to(gpu), elem_gate=eg.to(gpu), out_scale=1.3, **kw)
+    ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
+    torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
