@@ -191,6 +191,86 @@ __global__ __launch_bounds__(NT) void gla_scan_kernel(
   }
 }
 
+// A step of decode rows only, one token each: thread (16 row groups, 16 lanes of 4 columns) with state
+// rows rg + 16 i, so a state row is read and written 256 bytes at a time and all of a lane's rows are in
+// flight while the decays are computed (the scan above reads 64 bytes of a row).  V a multiple of 4.
+// Bound by the state's bytes: 64 rows of 8 heads [128, 256], 134 MB, 42 us by the scan, 27 here (5 TB/s, the
+// rate of a large copy); 8 rows 11.5 -> 10.
+template <typename T, int RI>
+__global__ __launch_bounds__(NT) void gla_decode_kernel(
+    float* __restrict__ out, const T* __restrict__ proj, int64_t ps, const T* __restrict__ low,
+    int64_t ls, const float* __restrict__ a2, const float* __restrict__ a2b, float* __restrict__ S,
+    const int* __restrict__ ctx, const int* __restrict__ slots, int H, int d, int V, int R,
+    float inv_tau, int num_slots) {
+  __shared__ float kqa[3][16 * RI];
+  __shared__ __align__(16) float sums[NT / 64][64];
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, rg = threadIdx.x >> 4;
+  const int cl = (threadIdx.x & 15) * 4, col = blockIdx.z * 64 + cl;
+  const bool colok = col < V;
+  const int slot = slots[s], pos = ctx[s] - 1;
+  float* orow = out + (int64_t)s * H * V + h * V + col;
+  if (slot < 0 || slot >= num_slots || pos < 0) {
+    if (rg == 0 && colok) *reinterpret_cast<float4*>(orow) = make_float4(0.f, 0.f, 0.f, 0.f);
+    return;
+  }
+  float* Sp = S + ((int64_t)slot * H + h) * d * V + col;
+  float4 Sr[RI];
+#pragma unroll
+  for (int i = 0; i < RI; ++i) {
+    const int r = rg + 16 * i;
+    Sr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (pos != 0 && r < d && colok) Sr[i] = *reinterpret_cast<const float4*>(Sp + (int64_t)r * V);
+  }
+  const T* row = proj + (int64_t)s * ps;
+  float v[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = colok ? to_f(row[2 * H * d + h * V + col + c]) : 0.f;
+  if (threadIdx.x < 16 * RI) {
+    const int r = threadIdx.x;
+    float kv = 0.f, qv = 0.f, al = 0.f;
+    if (r < d) {
+      kv = to_f(row[H * d + h * d + r]);
+      qv = to_f(row[h * d + r]) * (1.f / sqrtf((float)d));
+      const float* ar = a2 + (int64_t)(h * d + r) * R;
+      const T* lw = low + (int64_t)s * ls;
+      float acc = 0.f;
+#pragma unroll 8
+      for (int j = 0; j < R; ++j) acc += ar[j] * to_f(lw[j]);
+      al = expf(logsigmoid_f(acc + a2b[h * d + r]) * inv_tau);
+    }
+    kqa[0][r] = kv;
+    kqa[1][r] = qv;
+    kqa[2][r] = al;
+  }
+  __syncthreads();
+  float y[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < RI; ++i) {
+    const int r = rg + 16 * i;
+    const float kv = kqa[0][r], qv = kqa[1][r], av = kqa[2][r];
+    Sr[i] = make_float4(av * Sr[i].x + kv * v[0], av * Sr[i].y + kv * v[1], av * Sr[i].z + kv * v[2],
+                        av * Sr[i].w + kv * v[3]);
+    if (r < d && colok) *reinterpret_cast<float4*>(Sp + (int64_t)r * V) = Sr[i];
+    y[0] += Sr[i].x * qv;
+    y[1] += Sr[i].y * qv;
+    y[2] += Sr[i].z * qv;
+    y[3] += Sr[i].w * qv;
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    y[c] += __shfl_xor(y[c], 16, 64);
+    y[c] += __shfl_xor(y[c], 32, 64);
+  }
+  if (lane < 16) *reinterpret_cast<float4*>(&sums[wave][cl]) = make_float4(y[0], y[1], y[2], y[3]);
+  __syncthreads();
+  if (rg != 0 || !colok) return;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    y[c] = (sums[0][cl + c] + sums[1][cl + c]) + (sums[2][cl + c] + sums[3][cl + c]);
+  *reinterpret_cast<float4*>(orow) = make_float4(y[0], y[1], y[2], y[3]);
+}
+
 // ---- selective scan -------------------------------------------------------------------------
 // x, dt [T, I] (contiguous), bc [T, 2 N] (row stride bcs) = B | C, z [T, I] (row stride zs),
 // out [T, I] (row stride os), all of type T; At fp32 [N, I] = the transpose of A; state S
@@ -325,6 +405,20 @@ void launch_gla_scan(int dtype, float* out, const void* proj, int64_t ps, const 
                      int Tp, int H, int d, int V, int R, float tau, int num_slots,
                      hipStream_t s) {
   if (P + D <= 0) return;
+  // decode rows that share a launch with prompts stay with the scan, beside which they cost nothing
+  if (P == 0 && V % 4 == 0 && reinterpret_cast<uintptr_t>(S) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+    const dim3 grid(D, H, (V + 63) / 64);
+#define KGC_GLA_D(RI)                                                                        \
+  KGC_DS_DISPATCH_T(dtype, gla_decode_kernel<T, RI><<<grid, NT, 0, s>>>(                     \
+      out, (const T*)proj, ps, (const T*)low, ls, a2, a2b, S, ctx_lens, slots, H, d, V, R,   \
+      1.f / tau, num_slots))
+    if (d <= 64) KGC_GLA_D(4);
+    else if (d <= 128) KGC_GLA_D(8);
+    else KGC_GLA_D(16);
+#undef KGC_GLA_D
+    return;
+  }
   bool narrow = scan_narrow(P + D, H, V);
   // the narrow form pads 16 row groups; it has to fit 64 KB of LDS with the decay bottleneck
   if (narrow && sizeof(float) * (size_t)(3 * TB * (pow2_at_least(d, 64) + 64) + TB * 16 + TB * R) >

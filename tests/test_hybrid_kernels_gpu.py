@@ -443,3 +443,35 @@ def test_window_attention_shared_tiles(gpu, dt, H, G, latent, bs, kw):
                                0.08, args[1], args[2], gate.to(gpu), elem_gate=eg.to(gpu), out_scale=1.3, **kw)
     ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
+
+
+def _gla_case(T, slots, H, d, V, R, dt, tau, dev, open_=3.0):
+    """Inputs of gla_scan and its terms for ``_matrix64``."""
+    proj = (torch.randn(T, 2 * H * d + H * V + R) * 0.7).to(dt)
+    a2, bias, S = torch.randn(H * d, R) * 0.3, torch.randn(H * d) + open_, torch.randn(slots, H, d, V)
+    z = proj[:, -R:].double() @ a2.double().T + bias.double()
+    decay = torch.exp(torch.nn.functional.logsigmoid(z) / tau).view(T, H, d)
+    q, k, v = proj[:, : 2 * H * d + H * V].double().split([H * d, H * d, H * V], 1)
+    terms = (S, q.view(T, H, d) * d ** -0.5, k.view(T, H, d), v.reshape(T, H, V), decay)
+    dp = proj.to(dev)
+    return terms, lambda st, m: ops.gla_scan(dp, dp[:, -R:], a2.to(dev), bias.to(dev), st, m, H, d, V, tau)
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("H,d,V,R", [(2, 12, 4, 1), (1, 64, 60, 5), (3, 65, 64, 16), (2, 128, 68, 16),
+                                     (1, 129, 256, 37), (1, 256, 132, 128)])
+def test_gla_decode_rows(gpu, dt, H, d, V, R):
+    """A step of decode rows only: state rows around the 16, 64, 128 row edges, columns around a
+    workgroup's 64, a fresh row and a padding row.  The decay's logarithm is a sum of R + 1 terms
+    (below 64 in all here) over tau."""
+    torch.manual_seed(5)
+    n, tau = 5, 4.0
+    terms, run = _gla_case(n, n, H, d, V, R, dt, tau, gpu)
+    m = _meta([], [], [7, 1, 300, 4, 2], torch.zeros(n, 1, dtype=torch.int32), slots=[3, 0, -1, 1, 4])
+    want, unit, S, SA = _matrix64(m, *terms)
+    st = terms[0].to(gpu)
+    got = run(st, _to(m, gpu))
+    rel = 16 + 64 / tau
+    assert ((got.cpu() - want).abs() <= (d + rel) * unit + 1e-30).all()
+    assert ((st.cpu() - S).abs() <= rel * SA).all()
+    assert (got.cpu()[2] == 0).all() and (st.cpu()[2] == terms[0][2]).all()
