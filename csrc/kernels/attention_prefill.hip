@@ -32,6 +32,38 @@ constexpr int PF_BN = 64;
 
 __device__ __forceinline__ int kswz(int k) { return (k & 3) | (((k >> 3) & 3) << 2); }
 
+// cos / sin of one row's dims as pf_load_q uses them, loaded ahead of the rotation
+template <int D> struct PfRot { float4 c[D / 64][4]; };   // per fragment pair: cos lo / hi, sin lo / hi
+template <int D>
+__device__ __forceinline__ void pf_issue_rot(const float* __restrict__ cs_row, int qd, PfRot<D>& r) {
+#pragma unroll
+  for (int s = 0; s < D / 64; ++s) {
+    const int col = 32 * s + 8 * qd;
+    r.c[s][0] = *reinterpret_cast<const float4*>(cs_row + col);
+    r.c[s][1] = *reinterpret_cast<const float4*>(cs_row + col + 4);
+    r.c[s][2] = *reinterpret_cast<const float4*>(cs_row + D / 2 + col);
+    r.c[s][3] = *reinterpret_cast<const float4*>(cs_row + D / 2 + col + 4);
+  }
+}
+template <typename T, int D>
+__device__ __forceinline__ void pf_rotate(const PfRot<D>& r, Pack8<T> (&t)[D / 32]) {
+  constexpr int KS = D / 32;
+#pragma unroll
+  for (int s = 0; s < KS / 2; ++s) {
+    const float cc[8] = {r.c[s][0].x, r.c[s][0].y, r.c[s][0].z, r.c[s][0].w,
+                         r.c[s][1].x, r.c[s][1].y, r.c[s][1].z, r.c[s][1].w};
+    const float sn[8] = {r.c[s][2].x, r.c[s][2].y, r.c[s][2].z, r.c[s][2].w,
+                         r.c[s][3].x, r.c[s][3].y, r.c[s][3].z, r.c[s][3].w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float ra, rb;
+      neox_rot(to_f(t[s].h[j]), to_f(t[s + KS / 2].h[j]), cc[j], sn[j], ra, rb);
+      t[s].h[j] = from_f<T>(ra);
+      t[s + KS / 2].h[j] = from_f<T>(rb);
+    }
+  }
+}
+
 // q fragments of one 16-row q-tile: lane (r16, qd) holds dims 32 s + 8 qd .. + 7 of its
 // row.  cos_sin != nullptr: the row is the unrotated q of the fused QKV projection and
 // gets NeoX RoPE at position pos here -- dims i and i + D/2 sit in fragments s and
@@ -47,79 +79,13 @@ __device__ __forceinline__ void pf_load_q(const T* qrow, const float* __restrict
 #pragma unroll
   for (int s = 0; s < KS; ++s) t[s].u = *reinterpret_cast<const u32x4*>(qrow + 32 * s + 8 * qd);
   if (cos_sin != nullptr) {
+    PfRot<D> r;
     // clamped: a bad sequence length gives wrong output, never a fault
-    const float* cs = cos_sin + (int64_t)min(pos, cs_rows - 1) * D;
-#pragma unroll
-    for (int s = 0; s < KS / 2; ++s) {
-      const int col = 32 * s + 8 * qd;
-      const float4 c0 = *reinterpret_cast<const float4*>(cs + col);
-      const float4 c1 = *reinterpret_cast<const float4*>(cs + col + 4);
-      const float4 s0 = *reinterpret_cast<const float4*>(cs + D / 2 + col);
-      const float4 s1 = *reinterpret_cast<const float4*>(cs + D / 2 + col + 4);
-      const float cc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-      const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float ra, rb;
-        neox_rot(to_f(t[s].h[j]), to_f(t[s + KS / 2].h[j]), cc[j], sn[j], ra, rb);
-        t[s].h[j] = from_f<T>(ra);
-        t[s + KS / 2].h[j] = from_f<T>(rb);
-      }
-    }
+    pf_issue_rot<D>(cos_sin + (int64_t)min(pos, cs_rows - 1) * D, qd, r);
+    pf_rotate<T, D>(r, t);
   }
 #pragma unroll
   for (int s = 0; s < KS; ++s) qf[s] = t[s].v;
-}
-
-// pf_load_q in two halves, so the loads can be issued early and the rotation done later:
-// the persistent walk issues the next item's q (and cos / sin) loads BEFORE the current
-// item's output stores -- on gfx9 stores count in vmcnt too, so loads issued after the
-// stores would wait for the stores' completion at their first use.
-template <typename T, int D>
-struct PfQRaw {
-  Pack8<T> t[D / 32];
-  float4 c[D / 64][4];       // per rotated fragment pair: cos lo / hi, sin lo / hi
-};
-// cs_row: the row's cos / sin (always a readable row -- the caller passes a dummy one
-// without RoPE -- so every register of r is written here and none stays live across the
-// caller's loop)
-template <typename T, int D>
-__device__ __forceinline__ void pf_issue_q(const T* qrow, const float* __restrict__ cs_row,
-                                           int qd, PfQRaw<T, D>& r) {
-  constexpr int KS = D / 32;
-#pragma unroll
-  for (int s = 0; s < KS; ++s) r.t[s].u = *reinterpret_cast<const u32x4*>(qrow + 32 * s + 8 * qd);
-#pragma unroll
-  for (int s = 0; s < KS / 2; ++s) {
-    const int col = 32 * s + 8 * qd;
-    r.c[s][0] = *reinterpret_cast<const float4*>(cs_row + col);
-    r.c[s][1] = *reinterpret_cast<const float4*>(cs_row + col + 4);
-    r.c[s][2] = *reinterpret_cast<const float4*>(cs_row + D / 2 + col);
-    r.c[s][3] = *reinterpret_cast<const float4*>(cs_row + D / 2 + col + 4);
-  }
-}
-template <typename T, int D>
-__device__ __forceinline__ void pf_finish_q(PfQRaw<T, D>& r, bool rope,
-                                            typename Vec8<T>::type (&qf)[D / 32]) {
-  constexpr int KS = D / 32;
-  if (rope) {
-#pragma unroll
-    for (int s = 0; s < KS / 2; ++s) {
-      const float cc[8] = {r.c[s][0].x, r.c[s][0].y, r.c[s][0].z, r.c[s][0].w,
-                           r.c[s][1].x, r.c[s][1].y, r.c[s][1].z, r.c[s][1].w};
-      const float sn[8] = {r.c[s][2].x, r.c[s][2].y, r.c[s][2].z, r.c[s][2].w,
-                           r.c[s][3].x, r.c[s][3].y, r.c[s][3].z, r.c[s][3].w};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float ra, rb;
-        neox_rot(to_f(r.t[s].h[j]), to_f(r.t[s + KS / 2].h[j]), cc[j], sn[j], ra, rb);
-        r.t[s].h[j] = from_f<T>(ra);
-        r.t[s + KS / 2].h[j] = from_f<T>(rb);
-      }
-    }
-  }
-#pragma unroll
-  for (int s = 0; s < KS; ++s) qf[s] = r.t[s].v;
 }
 
 // Lazy O rescale (log2 units): the running max m only moves when some row's tile max
@@ -383,14 +349,14 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
 }
 
 // GQA-shared variant (G = nq / nkv >= 4): one workgroup = GH q-heads of ONE kv head x
-// QB = 256 / GH queries, 8 waves of 32 query rows (wave w: head w % GH, rows
-// 32 * (w / GH) ..).  Every K/V tile staged into LDS feeds 256 query rows of four or
-// eight heads instead of 128 rows of one head: half the K/V staging per FLOP, and one
-// staging pass per kv head instead of one per q-head.  The 128-row work items of the
-// engine's work list split into 128 / QB sub-blocks (grid.z); the per-wave math is the
-// single-head kernel's.
+// QB = 128 / GH queries, 4 waves of 32 query rows (wave w: head w % GH, rows
+// 32 * (w / GH) ..), two workgroups per CU.  Every K/V tile staged into LDS feeds 128 query rows of
+// four heads instead of 128 rows of one head, and there is one staging pass per kv head instead of
+// one per q-head.  The 128-row work items of the engine's work list split into 128 / QB sub-blocks; the
+// blocks of an item run over the heads first (with 8 kv heads an XCD sees one of them).  The per-wave
+// math is the single-head kernel's.
 template <typename T, int D, bool KV8, int GH>
-__global__ __launch_bounds__(512, 1) void prefill_attn_gqa_kernel(
+__global__ __launch_bounds__(256, 2) void prefill_attn_gqa_kernel(
     const T* __restrict__ q, T* __restrict__ out, const void* __restrict__ kc_,
     const void* __restrict__ vc_, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ qsl, const int* __restrict__ seq_lens,
@@ -406,8 +372,8 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_kernel(
     if constexpr (KV8) return fp8x8_widen<T>(r);
     else return r;
   };
-  constexpr int NT_ = 512;
-  constexpr int QB = 256 / GH;               // queries per workgroup
+  constexpr int NT_ = 256;
+  constexpr int QB = 128 / GH;               // queries per workgroup
   static_assert(QB <= PF_BM && PF_BM % QB == 0, "sub-blocks of the 128-row work item");
   constexpr int NCH = D / 8, KS = D / 32, DT = D / 16;
   constexpr int KPT = PF_BN * NCH / NT_;
@@ -417,23 +383,23 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_kernel(
   extern __shared__ __attribute__((aligned(16))) char smem[];
   T* lds = reinterpret_cast<T*>(smem);
 
-  const int seq = work_seq[blockIdx.x], mb = work_mblk[blockIdx.x];
-  const int G = nq / nkv;
-  const int h = blockIdx.y / (G / GH);                 // kv head
-  const int hg0 = h * G + (blockIdx.y % (G / GH)) * GH; // first q-head of this workgroup
+  const int G = nq / nkv, Y = nkv * (G / GH), w = blockIdx.x / (Y * (PF_BM / QB));
+  const int y = blockIdx.x % Y, z = blockIdx.x / Y % (PF_BM / QB);
+  const int seq = work_seq[w], mb = work_mblk[w];
+  const int h = y / (G / GH);                          // kv head
+  const int hg0 = h * G + (y % (G / GH)) * GH;         // first q-head of this workgroup
   const int q0 = qsl[seq];
   const int qlen = qsl[seq + 1] - q0;
   int L_in = seq_lens[seq];
   KGC_DCHECK_RANGE(L_in, 0, (bt_stride << bs_log2) + 1, "prefill seq_len");
   const int L = min(L_in, bt_stride << bs_log2);
   const int ctx0 = L - qlen;
-  const int qbase = mb * PF_BM + blockIdx.z * QB;      // first query row of the workgroup
+  const int qbase = mb * PF_BM + z * QB;      // first query row of the workgroup
   if (qlen <= 0 || ctx0 < 0 || qbase >= qlen) return;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int hq = hg0 + wave % GH;
   const int wq0 = qbase + (wave / GH) * 32;            // first query row of this wave
   const int r16 = lane & 15, qd = lane >> 4;
-  const int* bt = block_tables + (int64_t)seq * bt_stride;
   const int bsm = (1 << bs_log2) - 1;
   const int64_t hs = (int64_t)D << bs_log2;
 
@@ -458,50 +424,60 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_kernel(
   // Block ids of a tile's chunks are fetched one tile AHEAD of its K/V loads: the
   // dependent block-table load would otherwise stall every tile's load issue for an
   // L2 round trip before the compute it is meant to overlap.
+  // A wave's 64 chunks of one load are 4 whole keys (of a page: pages hold a multiple of 8) or half of
+  // an 8-key group: block ids and the groups' places are scalar.
+  static_assert(D == 128 && PF_BN == 64, "rows per wave");
   R kreg[KPT], vreg[VPT];
   int kblk[KPT], vblk[VPT];
+  typedef const __attribute__((address_space(4))) int* TablePtr;
+  const TablePtr bt = (TablePtr)(block_tables + (int64_t)seq * bt_stride);
   auto fetch_bt = [&](int kt) {
+    auto id = [&](int key) {
+      const int i = min(key, L - 1) >> bs_log2;
+      KGC_DCHECK_RANGE(i, 0, bt_stride, "block-table column");
+      const int v = bt[i];
+      KGC_DCHECK_RANGE(v, 0, num_blocks, "block id");
+      return v;
+    };
+#pragma unroll
+    for (int u = 0; u < KPT; ++u) kblk[u] = id(kt * PF_BN + 4 * wave + (NT_ / 16) * u);
+#pragma unroll
+    for (int u = 0; u < VPT; ++u) vblk[u] = id(kt * PF_BN + 8 * ((wave >> 1) + (NT_ / 128) * u));
+  };
+  // (the lane index behind an opaque move: addresses that depend on it alone are not kept in
+  // registers over the tile loop, where there are none left)
+  auto opaque = [](int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+  };
+  auto load_tile = [&](int kt) {
+    const int lane = opaque(threadIdx.x & 63);
 #pragma unroll
     for (int u = 0; u < KPT; ++u) {
-      const int key = (threadIdx.x + NT_ * u) / NCH;
-      kblk[u] = kgc_bt(bt, min(kt * PF_BN + key, L - 1) >> bs_log2, bt_stride, num_blocks);
+      const C* page = kc + ((int64_t)kblk[u] * nkv + h) * hs;
+      const int ka = min(kt * PF_BN + 4 * wave + (NT_ / 16) * u + (lane >> 4), L - 1);
+      kreg[u] = *reinterpret_cast<const R*>(page + ((ka & bsm) * D + (lane & 15) * 8));
     }
 #pragma unroll
     for (int u = 0; u < VPT; ++u) {
-      const int c = (threadIdx.x + NT_ * u) / D;
-      vblk[u] = kgc_bt(bt, (min(kt * PF_BN + 8 * c, L - 1) & ~7) >> bs_log2, bt_stride, num_blocks);
-    }
-  };
-  auto load_tile = [&](int kt) {
-#pragma unroll
-    for (int u = 0; u < KPT; ++u) {
-      const int ci = threadIdx.x + NT_ * u;
-      const int key = ci / NCH, c = ci % NCH;
-      const int ka = min(kt * PF_BN + key, L - 1);
-      const C* src = kc + ((int64_t)kblk[u] * nkv + h) * hs + (int64_t)(ka & bsm) * D + c * 8;
-      kreg[u] = *reinterpret_cast<const R*>(src);
-    }
-#pragma unroll
-    for (int u = 0; u < VPT; ++u) {       // 8-key group c of dim d: contiguous in d
-      const int ci = threadIdx.x + NT_ * u;
-      const int c = ci / D, d = ci % D;
-      const int ka = min(kt * PF_BN + 8 * c, L - 1) & ~7;
-      const C* src = vc + ((int64_t)vblk[u] * nkv + h) * hs + ((ka & bsm) >> 3) * (D * 8) + d * 8;
-      vreg[u] = *reinterpret_cast<const R*>(src);
+      const int ka = min(kt * PF_BN + 8 * ((wave >> 1) + (NT_ / 128) * u), L - 1);
+      const C* group = vc + ((int64_t)vblk[u] * nkv + h) * hs + ((ka & bsm) >> 3) * (D * 8);
+      vreg[u] = *reinterpret_cast<const R*>(group + ((wave & 1) * 64 + lane) * 8);
     }
   };
   auto store_tile = [&](int buf) {
+    const int tid = opaque(threadIdx.x);
     T* K = lds + buf * 2 * TILE;
     T* V = K + TILE;
 #pragma unroll
     for (int u = 0; u < KPT; ++u) {
-      const int ci = threadIdx.x + NT_ * u;
+      const int ci = tid + NT_ * u;
       const int key = ci / NCH, c = ci % NCH;
       *reinterpret_cast<u32x4*>(K + key * D + ((c ^ (kswz(key) & (NCH - 1))) * 8)) = widen(kreg[u]);
     }
 #pragma unroll
     for (int u = 0; u < VPT; ++u) {
-      const int ci = threadIdx.x + NT_ * u;
+      const int ci = tid + NT_ * u;
       const int c = ci / D, d = ci % D;
       *reinterpret_cast<u32x4*>(V + d * PF_BN + ((c ^ ((d >> 1) & 7)) * 8)) = widen(vreg[u]);
     }
@@ -519,15 +495,13 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_kernel(
   fetch_bt(0);
   load_tile(0);
   load_q();
-  if (n_tiles > 1) fetch_bt(1);
+  fetch_bt(n_tiles > 1);
+  __builtin_amdgcn_s_waitcnt(0x0f70);        // vmcnt(0): q is there
   store_tile(0);
   __syncthreads();
   for (int kt = 0; kt < n_tiles; ++kt) {
     const int buf = kt & 1;
-    if (kt + 1 < n_tiles) {
-      load_tile(kt + 1);
-      fetch_bt(min(kt + 2, n_tiles - 1));   // unconditional: static vmcnt below
-    }
+    load_tile(min(kt + 1, n_tiles - 1));
     if (kt < wave_tiles) {
       const T* K = lds + buf * 2 * TILE;
       const T* V = K + TILE;
@@ -536,7 +510,8 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_kernel(
       else
         pf_wave_tile<T, D, false>(K, V, qf, o, m, l, qpos, kt * PF_BN, scale_log2, r16, qd);
     }
-    if (kt + 1 < n_tiles) store_tile(buf ^ 1);
+    fetch_bt(min(kt + 2, n_tiles - 1));
+    store_tile(buf ^ 1);
     __syncthreads();
   }
 #pragma unroll
@@ -567,7 +542,12 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_kernel(
 // bit-identical).  Why: at short prompts every workgroup of the one-shot grid paid its own
 // pipeline fill -- the work_seq -> qsl / seq_lens -> block table -> K / V chain of dependent
 // loads, the q load and the first LDS store, ~10 us -- against 1-8 tiles of ~2.5 us of
-// work each (32 x 512 causal: 8 workgroups per CU, 0.40 PF/s against 0.84 PF/s at 16K).
+// work each (32 x 512 causal, 32 heads: 202 us one-shot).  What an item still costs beside its tiles
+// are its q and output rows: q comes by DMA while the item before it computes, outputs leave as whole
+// 256-byte rows (191 -> 168 us; 64 x 256 151 -> 126, 2 x 8192 1447 -> 1389).  The 32 x 512 floor is
+// 80 us of tiles and 60 us of bytes, which all CUs reach at the same time.  Rotating the rows in LDS
+// with each cos / sin row read once, and a stream of tiles without any wait before an item's compute,
+// measured within 3 % of this and slower on long prompts (2 x 8192: 1540).
 template <typename T, int D, bool KV8, int GH>
 __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
     const T* __restrict__ q, T* __restrict__ out, const void* __restrict__ kc_,
@@ -660,27 +640,48 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
                       cos_sin, cs_rows, qpos[qt], qd, qf[qt]);
     }
   };
-  PfQRaw<T, D> qraw[2];
-  int qpos_n[2];
+  // The next item's q rows come into LDS by DMA while this item computes (as register loads they
+  // would need 32 VGPRs more; issued after the last tile, their 5 us stood in every item).  A wave's
+  // 32 rows of its head, 16-byte chunks permuted by the row; afterwards the place where its output
+  // rows meet, so that they are stored 256 bytes at a time.
+  static_assert(D == 128, "16 chunks per row");
+  T* rows = lds + 4 * TILE + wave * 32 * D;
+  // (the lane index behind an opaque move: addresses that depend on it alone are not kept in
+  // registers over the tile loop, where there are none left)
+  auto opaque = [](int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+  };
   auto issue_q = [&](const Item& I) {
+    const int ln = opaque(lane), rl = ln >> 4, cl = ln & 15;
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-      const int qi = I.qbase + wrow + qt * 16 + r16;
-      const int qc = min(qi, I.qlen - 1);
-      qpos_n[qt] = I.ctx0 + qc;
-      // without RoPE the (unused) cos / sin come from a fixed readable row: q's first
-      const float* csr = cos_sin != nullptr
-                             ? cos_sin + (int64_t)min(qpos_n[qt], cs_rows - 1) * D
-                             : reinterpret_cast<const float*>(q);
-      pf_issue_q<T, D>(q + (int64_t)(I.q0 + qc) * q_stride + (int64_t)(I.hg0 + whead) * D,
-                       csr, qd, qraw[qt]);
+    for (int i = 0; i < 8; ++i) {
+      const int row = 4 * i + rl, qc = min(I.qbase + wrow + row, I.qlen - 1);
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(
+              q + (int64_t)(I.q0 + qc) * q_stride + (int64_t)(I.hg0 + whead) * D + ((cl ^ (row & 15)) * 8)),
+          (__attribute__((address_space(3))) void*)(rows + 4 * i * D), 16, 0, 0);
     }
   };
-  auto finish_q = [&]() {
+  auto finish_q = [&](const Item& I) {
+    const int ln = opaque(lane), r16 = ln & 15, qd = ln >> 4;
+    PfRot<D> rot[2];
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
-      qpos[qt] = qpos_n[qt];
-      pf_finish_q<T, D>(qraw[qt], cos_sin != nullptr, qf[qt]);
+      qpos[qt] = I.ctx0 + min(I.qbase + wrow + qt * 16 + r16, I.qlen - 1);
+      if (cos_sin != nullptr)
+        pf_issue_rot<D>(cos_sin + (int64_t)min(qpos[qt], cs_rows - 1) * D, qd, rot[qt]);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the wave's own DMAs: no barrier
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      Pack8<T> t[KS];
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        t[s].u = *reinterpret_cast<const u32x4*>(rows + (qt * 16 + r16) * D + (((4 * s + qd) ^ r16) * 8));
+      if (cos_sin != nullptr) pf_rotate<T, D>(rot[qt], t);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) qf[qt][s] = t[s].v;
     }
   };
   R kreg[KPT], vreg[VPT];
@@ -776,6 +777,7 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
         }
         loaded = true;
       }
+      if (kt == 0 && has_next) issue_q(nxt);
       if (kt < wave_tiles) {
         const T* K = lds + buf * 2 * TILE;
         const T* V = K + TILE;
@@ -788,33 +790,36 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
       __syncthreads();
       buf ^= 1;
     }
-    // the next item's q loads go out before this item's output stores (see PfQRaw);
-    // unconditional (the current item's rows again at the end of the walk) so the raw
-    // registers are written every iteration and not kept live around the loop
-    issue_q(has_next ? nxt : cur);
+    const Item done = cur;
+    if (has_next) finish_q(nxt);
+    const int ln = opaque(lane), rl = ln >> 4, cl = ln & 15;
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
       float tot = l[qt];
       tot += __shfl_xor(tot, 16, 64);
       tot += __shfl_xor(tot, 32, 64);
       const float inv = v_scale / tot;
-      const int qi = wq0 + qt * 16 + r16;
-      if (qi < cur.qlen && qi < cur.qbase + QB) {
-        T* orow = out + ((int64_t)(cur.q0 + qi) * nq + cur.hg0 + whead) * D + 4 * qd;
 #pragma unroll
-        for (int t = 0; t < DT; ++t) {
-          Pack4<T> pk;
+      for (int t = 0; t < DT; ++t) {
+        Pack4<T> pk;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) pk.h[i] = from_f<T>(o[qt][t][i] * inv);
-          *reinterpret_cast<u32x2*>(orow + 16 * t) = pk.u;
-        }
+        for (int i = 0; i < 4; ++i) pk.h[i] = from_f<T>(o[qt][t][i] * inv);
+        *reinterpret_cast<u32x2*>(rows + (qt * 16 + cl) * D + (((2 * t + (rl >> 1)) ^ cl) * 8) +
+                                  4 * (rl & 1)) = pk.u;
       }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = 4 * i + rl, qi = done.qbase + wrow + row;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(rows + row * D + cl * 8);
+      if (qi < done.qlen)
+        *reinterpret_cast<u32x4*>(out + ((int64_t)(done.q0 + qi) * nq + done.hg0 + whead) * D +
+                                  ((cl ^ (row & 15)) * 8)) = v;
     }
     if (!has_next) break;
     // the next item's first tile is already staged in LDS buffer `buf`
     cur = nxt;
     it = nit;
-    finish_q();
   }
 }
 
@@ -824,10 +829,10 @@ static int prefill_gqa_enabled() {
   return e ? atoi(e) : 1;
 }
 
-// KGC_PREFILL_PERSIST=0: the one-shot GQA grid instead of the persistent walk (A/B, tests)
-static int prefill_persist_enabled() {
+// KGC_PREFILL_PERSIST=0: the one-shot GQA grid everywhere, =1: the persistent walk (A/B, tests)
+static int prefill_persist_mode() {
   const char* e = getenv("KGC_PREFILL_PERSIST");
-  return e ? atoi(e) : 1;
+  return e ? atoi(e) : -1;
 }
 
 template <typename T, int D, bool KV8, int GH>
@@ -836,25 +841,33 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
                                  const int* ws, const int* wm, int n_work, int nq, int nkv,
                                  int bs_log2, float scale_log2, float v_scale, int num_blocks,
                                  int64_t q_stride, const float* cos_sin, int cs_rows, hipStream_t s) {
-  const size_t lds = 2 * 2 * PF_BN * D * sizeof(T);
+  constexpr size_t lds = 2 * 2 * PF_BN * D * sizeof(T);
   const int G = nq / nkv;
-  const dim3 grid(n_work, nkv * (G / GH), PF_BM / (256 / GH));
-  const int64_t n_items = (int64_t)grid.x * grid.y * grid.z;
-  if (prefill_persist_enabled() && n_items < ((int64_t)1 << 30)) {
-    // one workgroup per CU (launch_bounds(512, 1), 64 KB of LDS), never more than items
-    static const int n_cu = [] {
-      int dev = 0, cu = 256;
-      if (hipGetDevice(&dev) == hipSuccess)
-        hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev);
-      return cu > 0 ? cu : 256;
-    }();
-    const int g = (int)std::min<int64_t>(n_items, n_cu);
-    prefill_attn_gqa_persist_kernel<T, D, KV8, GH><<<g, 512, lds, s>>>(
+  const int64_t n_items = (int64_t)n_work * nkv * (G / GH) * (PF_BM / (256 / GH));
+  static const int n_cu = [] {
+    int dev = 0, cu = 256;
+    if (hipGetDevice(&dev) == hipSuccess)
+      hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev);
+    return cu > 0 ? cu : 256;
+  }();
+  // The walk pays with more items than CUs (32 x 512 rows, 32 heads: 179 us against 202); with one item
+  // per CU or less, twice as many workgroups of half the rows do (8 x 100 rows after 3000: 115 against
+  // 137, 512 rows alone 28 against 31, 2000 after 2000 168 against 179).
+  const int mode = prefill_persist_mode();
+  const bool dma = reinterpret_cast<uintptr_t>(q) % 16 == 0 && q_stride % 8 == 0;    // 16-byte DMAs
+  if (dma && (mode < 0 ? n_items > n_cu : mode != 0) && n_items < ((int64_t)1 << 30)) {
+    // one workgroup per CU: launch_bounds(512, 1), 128 KB of LDS (K / V tiles, the waves' q / output rows)
+    constexpr size_t lds_q = lds + 256 * D * sizeof(T);
+    static const hipError_t big = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&prefill_attn_gqa_persist_kernel<T, D, KV8, GH>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_q);
+    (void)big;
+    prefill_attn_gqa_persist_kernel<T, D, KV8, GH><<<(int)std::min<int64_t>(n_items, n_cu), 512, lds_q, s>>>(
         (const T*)q, (T*)out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, nq, nkv, bs_log2,
         scale_log2, v_scale, num_blocks, q_stride, cos_sin, cs_rows, (int)n_items);
     return;
   }
-  prefill_attn_gqa_kernel<T, D, KV8, GH><<<grid, 512, lds, s>>>(
+  prefill_attn_gqa_kernel<T, D, KV8, 4><<<nkv * (G / 4) * (PF_BM / 32) * n_work, 256, lds, s>>>(
       (const T*)q, (T*)out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, nq, nkv, bs_log2,
       scale_log2, v_scale, num_blocks, q_stride, cos_sin, cs_rows);
 }
@@ -866,7 +879,7 @@ static void prefill_dispatch(const void* q, void* out, const void* kc, const voi
                              int bs_log2, float scale_log2, float v_scale, int num_blocks,
                              int64_t q_stride, const float* cos_sin, int cs_rows, hipStream_t s) {
   const int G = nkv > 0 ? nq / nkv : 1;
-  if (D == 128 && prefill_gqa_enabled() && nq % nkv == 0 && (G == 4 || G % 8 == 0)) {
+  if constexpr (D == 128) if (prefill_gqa_enabled() && nq % nkv == 0 && (G == 4 || G % 8 == 0)) {
     if (G == 4)
       prefill_gqa_dispatch<T, D, KV8, 4>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work,
                                          nq, nkv, bs_log2, scale_log2, v_scale, num_blocks,

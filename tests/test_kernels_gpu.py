@@ -509,6 +509,38 @@ def test_prefill_persistent_walk_bit_identical(gpu, monkeypatch, dt, nq, nkv, d,
     assert torch.equal(out, outs["0"])
 
 
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("nq,nkv", [(32, 8), (16, 1)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_prefill_walk_rotates_the_next_item(gpu, monkeypatch, dt, nq, nkv, fp8):
+    """The walk's q rows of later items come through LDS and are rotated there: more items than CUs
+    (groups of four and of eight heads), prompts of one row up to several tiles, strided q rows.
+    Bit for bit the one-shot kernels' rows, which load and rotate them in registers, under every
+    choice of kernel."""
+    torch.manual_seed(22)
+    bs, d = 16, 128
+    seq_lens = [200] * 36 + [1, 64, 65, 129, 300] * (3 if nkv == 8 else 12)
+    query_lens = [L - L // 3 if i % 5 == 0 else L for i, L in enumerate(seq_lens)]
+    kc, vc, bt = _fill_random_cache(len(seq_lens), seq_lens, nkv, bs, d, dt, gpu)
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    T = sum(query_lens)
+    N = (nq + 2 * nkv) * d
+    qkv = torch.randn(T, N + 64, dtype=dt, device=gpu)[:, :N]
+    qsl = torch.tensor([0] + query_lens, dtype=torch.int32).cumsum(0).int().to(gpu)
+    sl = torch.tensor(seq_lens, dtype=torch.int32, device=gpu)
+    cs = ref.rope_cos_sin_cache(d, 1024, 500000.0).to(gpu)
+    outs = []
+    for persist in ("0", "1", None):
+        if persist is None:
+            monkeypatch.delenv("KGC_PREFILL_PERSIST")
+        else:
+            monkeypatch.setenv("KGC_PREFILL_PERSIST", persist)
+        outs.append(ops.prefill_attention_rope(qkv, cs, kc, vc, bt, qsl, sl, d ** -0.5, nq, d))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 def test_prefill_matches_dense(gpu):
     """End-to-end: rope_kv_write -> prefill kernel == dense causal attention."""
     torch.manual_seed(5)
