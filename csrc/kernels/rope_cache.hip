@@ -13,7 +13,9 @@
 // quantised is the T-rounded one, exactly what a T cache would store.
 #include "common.h"
 #include "launch.h"
+#include <climits>
 #include <cstdlib>
+#include <type_traits>
 
 namespace kgc {
 
@@ -44,6 +46,15 @@ __device__ __forceinline__ u32x4 qkv8(const void* qkv, int64_t row_elem, int col
     }
     return o.u;
   }
+}
+
+// fp8 of 8 elements over a scale
+template <typename T>
+__device__ __forceinline__ u32x2 fp8_8(const Pack8<T>& v, float inv) {
+  float f[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) f[j] = to_f(v.h[j]) * inv;
+  return u32x2{fp8x4(f[0], f[1], f[2], f[3]), fp8x4(f[4], f[5], f[6], f[7])};
 }
 
 // KVO: k / v only (q_out unused): the prefill attention kernel rotates q itself as it
@@ -195,109 +206,150 @@ __global__ __launch_bounds__(ROPE_NT) void rope_kv_kernel(
   }
 }
 
-// Prefill K / V write (KVO, RoPE, no k-norm, T cache): one 256-thread workgroup per
-// 8-token group.  The per-token grid above gives a token 8 K threads in a 64-lane wave
-// and 128 V threads that each issue eight 2-byte stores; at a 16K-token chunk that kernel
-// took 137 us per layer for 134 MB of traffic.  Here a group whose 8 tokens fill one
-// 8-key group of the cache (consecutive slots, the first a multiple of 8 -- every group
-// of a sequence's aligned prefill) is written as:
-//   K: every (token, head, chunk pair) item rotated and stored as two 16-byte rows;
-//   V: thread (head, chunk) loads the chunk of all 8 tokens and writes the 8 x 8 block
-//      transposed, eight 16-byte stores (whole V^T rows of the group).
-// Other groups (sequence boundaries inside the group, padding slots) take 2-byte V stores.
+// Prefill K / V write (KVO, RoPE, no k-norm).  The per-token grid above gives a token 8 K threads
+// in a 64-lane wave and 128 V threads that each issue eight 2-byte stores; at a 16K-token chunk that
+// kernel took 137 us per layer for 134 MB of traffic.  Here a thread takes one of 2 nkv d / 8 units of
+// a group of 8 rows, no barrier:
+//   K: (head, chunk pair) of every other row: four pairs rotated, each stored as two chunks;
+//   V: (head, chunk) of the 8-key cache group that STARTS in the 8 rows (consecutive slots, the first
+//      a multiple of 8): the chunk of its 8 rows, wherever they lie, written as a transposed 8 x 8
+//      block.  Rows of the 8 that are in no such block (ends of a prompt, padding slots) take 2-byte
+//      (fp8: 1-byte) stores.
+// Blocks that follow the cache and not the rows are what ragged prompts need: with blocks of 8 rows
+// aligned to the step, every prompt behind one of odd length took the 2-byte stores (32 x 512 ragged
+// rows, 8 heads of 128, 134 MB: 75 us, 28 here, the rate of a large copy; fp8 cache, which had the
+// per-token kernel, 86 -> 22).
 constexpr int KVG_NT = 256;
-template <typename T>
+template <typename T, bool KV8>
 __global__ __launch_bounds__(KVG_NT) void kv_group_kernel(
     const T* __restrict__ qkv, int64_t qkv_stride, const int64_t* __restrict__ positions,
-    const float* __restrict__ cos_sin, T* __restrict__ k_cache, T* __restrict__ v_cache,
-    const int64_t* __restrict__ slot_mapping, int T_, int nq, int nkv, int d, int bs,
-    int num_blocks) {
-  const int t0 = blockIdx.x * 8, nt = min(8, T_ - t0);
-  const int tph = d >> 4, half = d >> 1, cpr = d >> 3;
-  __shared__ int64_t s_slot[8];
-  __shared__ int s_full;
-  if (threadIdx.x < 8) {
-    int64_t s = threadIdx.x < nt ? slot_mapping[t0 + threadIdx.x] : -1;
-    KGC_DCHECK_RANGE(s, -1, (int64_t)num_blocks * bs, "KV slot");
-    s_slot[threadIdx.x] = s;
+    const float* __restrict__ cos_sin, void* __restrict__ k_cache, void* __restrict__ v_cache,
+    const int64_t* __restrict__ slot_mapping, int T_, int nq, int nkv, int d, int bs, int bs_shift,
+    int num_blocks, float k_inv, float v_inv, int groups) {
+  typedef std::conditional_t<KV8, uint8_t, T> C;
+  C* kc = reinterpret_cast<C*>(k_cache);
+  C* vc = reinterpret_cast<C*>(v_cache);
+  const int tph = d >> 4, half = d >> 1, cpr = d >> 3, nv = nkv * cpr;
+  // whole waves per group (`groups` of them per workgroup): what follows is uniform in a wave
+  const int tpg = KVG_NT / groups;
+  const int t0 = (blockIdx.x * groups + threadIdx.x / tpg) * 8;
+  if (t0 >= T_) return;
+  // lane i: slot and position of row t0 - 7 + i; blocks that start at those rows
+  const int lane = threadIdx.x & 63, row = t0 - 7 + lane;
+  int slot = -1, pos = 0;
+  if (lane < 22 && row >= 0 && row < T_) {
+    const int64_t sl = slot_mapping[row];
+    KGC_DCHECK_RANGE(sl, -1, (int64_t)num_blocks * bs, "KV slot");
+    slot = sl < 0 ? -1 : (int)sl;
+    if (slot >= 0) pos = (int)positions[row];
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    bool full = nt == 8 && s_slot[0] >= 0 && (s_slot[0] & 7) == 0;
-    for (int k = 1; k < 8; ++k) full = full && s_slot[k] == s_slot[0] + k;
-    s_full = full;
-  }
-  // K: items (token k, head h, chunk pair c), two per thread with both loads in flight
-  const int nk_items = nt * nkv * tph;
-  for (int base = 0; base < nk_items; base += 2 * KVG_NT) {
-    Pack8<T> a[2], b[2];
-    int kk[2], hh[2], cc_[2];
+  const int up = __shfl_down(slot, 1, 64);
+  const uint32_t next = (uint32_t)__ballot(slot >= 0 && up == slot + 1 && lane < 21);
+  uint32_t start = (uint32_t)__ballot(slot >= 0 && (slot & 7) == 0) & next & (next >> 1);
+  start &= (next >> 2) & (next >> 3) & (next >> 4) & (next >> 5) & (next >> 6);
+  uint32_t in = start | start << 1;
+  in |= in << 2;
+  in |= in << 4;                               // rows of a whole block
+  const uint32_t own = start >> 7 & 255;       // at most one block starts in the 8 rows
+  const uint32_t single = (uint32_t)__ballot(slot >= 0) >> 7 & 255 & ~(in >> 7);
+  auto page_of = [&](int s, int& off) {
+    const int page = bs_shift >= 0 ? s >> bs_shift : s / bs;
+    off = s - page * bs;
+    return (int64_t)page;
+  };
+  for (int u = threadIdx.x % tpg; u < (2 * nv + 63 & ~63); u += tpg) {
+    const int k = max(min(u, 2 * nv - 1) - nv, 0), par = k / (nkv * tph), hc = k - par * (nkv * tph);
+    int sl[4], ps[4];                          // (by every lane: a wave can hold units of both kinds)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int it = min(base + u * KVG_NT + (int)threadIdx.x, nk_items - 1);
-      kk[u] = it / (nkv * tph);
-      hh[u] = (it / tph) % nkv;
-      cc_[u] = it % tph;
-      const T* src = qkv + (int64_t)(t0 + kk[u]) * qkv_stride + (int64_t)(nq + hh[u]) * d;
-      a[u].u = *reinterpret_cast<const u32x4*>(src + cc_[u] * 8);
-      b[u].u = *reinterpret_cast<const u32x4*>(src + half + cc_[u] * 8);
+    for (int i = 0; i < 4; ++i) {
+      sl[i] = __shfl(slot, 7 + par + 2 * i, 64);
+      ps[i] = __shfl(pos, 7 + par + 2 * i, 64);
     }
+    if (u >= nv) {                             // ---- K
+      const int h = hc / tph, c = hc - h * tph;
+      Pack8<T> a[4], b[4];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int it = base + u * KVG_NT + (int)threadIdx.x;
-      const int64_t slot = s_slot[kk[u]];
-      if (it >= nk_items || slot < 0) continue;
-      const float* cs = cos_sin + positions[t0 + kk[u]] * d;
-      const int c = cc_[u];
-      const float4 c0 = *reinterpret_cast<const float4*>(cs + c * 8);
-      const float4 c1 = *reinterpret_cast<const float4*>(cs + c * 8 + 4);
-      const float4 s0 = *reinterpret_cast<const float4*>(cs + half + c * 8);
-      const float4 s1 = *reinterpret_cast<const float4*>(cs + half + c * 8 + 4);
-      const float co[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-      const float si[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-      Pack8<T> oa, ob;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float ra, rb;
-        neox_rot(to_f(a[u].h[j]), to_f(b[u].h[j]), co[j], si[j], ra, rb);
-        oa.h[j] = from_f<T>(ra);
-        ob.h[j] = from_f<T>(rb);
+      for (int i = 0; i < 4; ++i) {
+        const int r = par + 2 * i;
+        const T* src = qkv + (int64_t)min(t0 + r, T_ - 1) * qkv_stride + (int64_t)(nq + h) * d + c * 8;
+        a[i].u = *reinterpret_cast<const u32x4*>(src);
+        b[i].u = *reinterpret_cast<const u32x4*>(src + half);
       }
-      T* dst = k_cache + (((slot / bs) * nkv + hh[u]) * bs + slot % bs) * (int64_t)d;
-      *reinterpret_cast<u32x4*>(dst + c * 8) = oa.u;
-      *reinterpret_cast<u32x4*>(dst + half + c * 8) = ob.u;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float* cs = cos_sin + (int64_t)ps[i] * d + c * 8;
+        const float4 c0 = *reinterpret_cast<const float4*>(cs), c1 = *reinterpret_cast<const float4*>(cs + 4);
+        const float4 s0 = *reinterpret_cast<const float4*>(cs + half);
+        const float4 s1 = *reinterpret_cast<const float4*>(cs + half + 4);
+        const float co[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        const float si[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+        Pack8<T> oa, ob;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float ra, rb;
+          neox_rot(to_f(a[i].h[j]), to_f(b[i].h[j]), co[j], si[j], ra, rb);
+          oa.h[j] = from_f<T>(ra);
+          ob.h[j] = from_f<T>(rb);
+        }
+        if (sl[i] < 0 || u >= 2 * nv) continue;
+        int off;
+        const int64_t page = page_of(sl[i], off);
+        C* dst = kc + ((page * nkv + h) * bs + off) * (int64_t)d + c * 8;
+        if constexpr (KV8) {
+          *reinterpret_cast<u32x2*>(dst) = fp8_8(oa, k_inv);
+          *reinterpret_cast<u32x2*>(dst + half) = fp8_8(ob, k_inv);
+        } else {
+          *reinterpret_cast<u32x4*>(dst) = oa.u;
+          *reinterpret_cast<u32x4*>(dst + half) = ob.u;
+        }
+      }
+      continue;
     }
-  }
-  // V: item (head h, chunk c) over the group's tokens
-  __syncthreads();
-  const bool full = s_full;
-  for (int iv = threadIdx.x; iv < nkv * cpr; iv += KVG_NT) {
-    const int h = iv / cpr, c = iv % cpr;
+    // ---- V
+    const int h = u / cpr, c = u - h * cpr;
     const T* src = qkv + (int64_t)t0 * qkv_stride + (int64_t)(nq + nkv + h) * d + c * 8;
-    if (full) {
+    auto block = [&](int s) {                  // this unit's 8 x 8 block of the group that holds slot s
+      int off;
+      const int64_t page = page_of(s, off);
+      return vc + (page * nkv + h) * (int64_t)bs * d + ((int64_t)(off >> 3) * d + c * 8) * 8 + (off & 7);
+    };
+    if (own != 0) {
+      const int f = __builtin_ctz(own);
       Pack8<T> vv[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) vv[k].u = *reinterpret_cast<const u32x4*>(src + k * qkv_stride);
-      const int64_t slot = s_slot[0];
-      const int off = (int)(slot % bs);
-      T* dst = v_cache + ((slot / bs) * nkv + h) * (int64_t)bs * d +
-               ((int64_t)(off >> 3) * d + c * 8) * 8;
+      for (int k = 0; k < 8; ++k) vv[k].u = *reinterpret_cast<const u32x4*>(src + (f + k) * qkv_stride);
+      C* dst = block(__builtin_amdgcn_readlane(slot, 7 + f));
+      if constexpr (KV8) {
+        u32x2 w[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        Pack8<T> o;
+        for (int k = 0; k < 8; ++k) w[k] = fp8_8(vv[k], v_inv);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) o.h[k] = vv[k].h[j];
-        *reinterpret_cast<u32x4*>(dst + j * 8) = o.u;
+        for (int j = 0; j < 8; ++j) {
+          u32x2 o = {0u, 0u};
+#pragma unroll
+          for (int k = 0; k < 8; ++k) o[k >> 2] |= (w[k][j >> 2] >> (8 * (j & 3)) & 255u) << (8 * (k & 3));
+          *reinterpret_cast<u32x2*>(dst + j * 8) = o;
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          Pack8<T> o;
+#pragma unroll
+          for (int k = 0; k < 8; ++k) o.h[k] = vv[k].h[j];
+          *reinterpret_cast<u32x4*>(dst + j * 8) = o.u;
+        }
       }
-    } else {
-      for (int k = 0; k < nt; ++k) {
-        const int64_t slot = s_slot[k];
-        if (slot < 0) continue;
-        Pack8<T> v;
-        v.u = *reinterpret_cast<const u32x4*>(src + k * qkv_stride);
-        const int off = (int)(slot % bs);
-        T* dst = v_cache + ((slot / bs) * nkv + h) * (int64_t)bs * d +
-                 ((int64_t)(off >> 3) * d + c * 8) * 8 + (off & 7);
+    }
+    for (uint32_t left = single; left != 0; left &= left - 1) {
+      const int k = __builtin_ctz(left);
+      Pack8<T> v;
+      v.u = *reinterpret_cast<const u32x4*>(src + k * qkv_stride);
+      C* dst = block(__builtin_amdgcn_readlane(slot, 7 + k));
+      if constexpr (KV8) {
+        const u32x2 w = fp8_8(v, v_inv);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dst[j * 8] = (uint8_t)(w[j >> 2] >> (8 * (j & 3)));
+      } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) dst[j * 8] = v.h[j];
       }
@@ -333,11 +385,14 @@ static void rope_dispatch(const void* qkv, int64_t qkv_stride, int S, int64_t ss
       qkv, qkv_stride, S, ss, pos, cs, (T*)q_out, kc, vc, slots, (const T*)qn,               \
       (const T*)kn, nq, nkv, d, bs, eps, k_inv, v_inv, num_blocks)
   const bool norm = qn != nullptr;
-  if constexpr (!KV8 && !SL) {
-    if (kvo && rope && !norm && rope_kvg() && (d & 15) == 0 && (bs & 7) == 0) {
-      kv_group_kernel<T><<<(T_ + 7) / 8, KVG_NT, 0, s>>>(
-          (const T*)qkv, qkv_stride, pos, cs, (T*)kc, (T*)vc, slots, T_, nq, nkv, d, bs,
-          num_blocks);
+  if constexpr (!SL) {
+    const int64_t slots_end = (int64_t)num_blocks * bs;
+    if (kvo && rope && !norm && rope_kvg() && (d & 15) == 0 && (bs & 7) == 0 && slots_end < INT_MAX) {
+      const int units = nkv * (d >> 2);      // of one 8-row group
+      const int groups = units <= 64 ? 4 : units <= 128 ? 2 : 1;
+      kv_group_kernel<T, KV8><<<(T_ + 8 * groups - 1) / (8 * groups), KVG_NT, 0, s>>>(
+          (const T*)qkv, qkv_stride, pos, cs, kc, vc, slots, T_, nq, nkv, d, bs,
+          (bs & (bs - 1)) == 0 ? __builtin_ctz(bs) : -1, num_blocks, k_inv, v_inv, groups);
       return;
     }
   }

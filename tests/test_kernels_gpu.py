@@ -510,6 +510,39 @@ def test_prefill_persistent_walk_bit_identical(gpu, monkeypatch, dt, nq, nkv, d,
 
 
 @pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("nkv,d,bs", [(8, 128, 32), (4, 128, 8), (1, 128, 16), (3, 64, 24), (12, 96, 16)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_kv_write_rope_ragged_groups(gpu, monkeypatch, dt, nkv, d, bs, fp8):
+    """The 8-row K / V writer where rows and 8-key cache groups do not line up: prompts of odd
+    lengths behind each other, chunks that start inside a group, padding rows, a last row group
+    that is not full, heads whose units share a wave.  The per-token kernel's bytes."""
+    torch.manual_seed(23)
+    lens, old = [1, 7, 8, 9, 40, 3, 64, 15, 1, 1, 90], [0, 3, 0, 5, 2, 0, 0, 7, 9, 10, 0]
+    nb = sum((a + b) // bs + 1 for a, b in zip(lens, old)) + 1
+    free, pos, slots = iter(torch.randperm(nb).tolist()), [], []
+    for a, b in zip(lens, old):
+        pages = [next(free) for _ in range((a + b) // bs + 1)]
+        for p in range(b, a + b):
+            pos.append(p)
+            slots.append(pages[p // bs] * bs + p % bs)
+    for i in (20, 21, 50, 100, len(slots) - 1):
+        slots[i] = -1
+    T, N = len(pos), (2 + 2 * nkv) * d
+    qkv = torch.randn(T, N + 8, dtype=dt, device=gpu)[:, :N]
+    i64 = lambda v: torch.tensor(v, dtype=torch.int64, device=gpu)   # noqa: E731
+    cs = ref.rope_cos_sin_cache(d, 256, 500000.0).to(gpu)
+    ct = torch.float8_e4m3fn if fp8 else dt
+    got = []
+    for kvg in ("0", "1"):
+        monkeypatch.setenv("KGC_ROPE_KVG", kvg)
+        kc = torch.zeros(nb, nkv, bs, d, device=gpu).to(ct)
+        vc = torch.zeros(nb, nkv, bs // 8, d, 8, device=gpu).to(ct)
+        ops.kv_write_rope(qkv, i64(pos), cs, kc, vc, i64(slots), 2, nkv, d)
+        got.append((kc.view(torch.uint8), vc.view(torch.uint8)))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(got[0][1].any())
+
+
+@pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("nq,nkv", [(32, 8), (16, 1)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_prefill_walk_rotates_the_next_item(gpu, monkeypatch, dt, nq, nkv, fp8):
