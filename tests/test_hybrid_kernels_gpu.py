@@ -475,3 +475,25 @@ def test_gla_decode_rows(gpu, dt, H, d, V, R):
     assert ((got.cpu() - want).abs() <= (d + rel) * unit + 1e-30).all()
     assert ((st.cpu() - S).abs() <= rel * SA).all()
     assert (got.cpu()[2] == 0).all() and (st.cpu()[2] == terms[0][2]).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,W,N", [(64, 128, 1), (65, 1024, 17), (79, 1152, 8), (1000, 2048, 16), (64, 2304, 33),
+                                      (100, 4096, 5), (8200, 256, 8)])
+def test_gate_proj_many_rows(gpu, dt, rows, W, N):
+    """Rows from the matrix-core kernel's least, around its blocks of 16 rows and 16 outputs, widths of
+    every register form, more blocks than workgroups; a row of NaN stays alone.  Sums of W fp32 terms
+    in parts: 2^-24 of the sum of absolute products, times the sums' depth (below 24)."""
+    torch.manual_seed(41)
+    h, w = torch.randn(rows, W).to(dt), (torch.randn(N, W) * 0.05).to(dt)
+    b = torch.randn(N)
+    h[3] = float("nan")
+    got = ops.gate_proj(h.to(gpu), w.to(gpu), b.to(gpu), ops.GATE_NONE).cpu()
+    assert got[3].isnan().all()
+    keep = torch.arange(rows) != 3
+    want = h[keep].double() @ w.double().T + b.double()
+    unit = (h[keep].double().abs() @ w.double().abs().T + b.double().abs()) * 2.0 ** -24
+    assert ((got[keep] - want).abs() <= 24 * unit).all()
+    got = ops.gate_proj(h.to(gpu), w.to(gpu), None, ops.GATE_CAP_TANH, ops.GATE_LOGSIG_CAP_TANH, N // 2, 15.0).cpu()
+    want = ref.gate_proj(h[keep], w, None, ops.GATE_CAP_TANH, ops.GATE_LOGSIG_CAP_TANH, N // 2, 15.0)
+    torch.testing.assert_close(got[keep], want, rtol=1e-4, atol=1e-4)
