@@ -10,8 +10,9 @@
 //   residual_sum_norm    x += up to three results, each plain or RMS-normed; h = RMSNorm(x) * w
 //   gate_mul, relu_sq, side_gate   element-wise epilogues between GEMMs
 // All arithmetic is fp32; T is the activation dtype of h / y (bf16, f16 or fp32).
-// One workgroup per row; a row is walked twice (sum of squares, then scale), the second
-// walk re-reading what the same thread wrote in the first.
+// One workgroup per row.  Rows of any width are walked twice (sum of squares, then scale), the second
+// walk re-reading what the same thread wrote in the first; where vectors fit, the row stays in
+// registers.
 #include "common.h"
 #include "launch.h"
 
@@ -83,6 +84,164 @@ __global__ __launch_bounds__(NT) void depth_mix_norm_kernel(
   for (int c = threadIdx.x; c < W; c += NT) o[c] = from_f<T>(xr[c] * rs[c / gw] * w[c]);
 }
 
+// ---- the same by vectors: thread t holds the V float4 at columns 4 (t + 256 k), x and what is added to
+// it are read once and the row stays in registers.  Groups of a multiple of 256 columns: a wave's
+// float4 of one k lie in one group, so its sums meet in a table behind one barrier, whatever the
+// number of groups.  Bound by bytes; 16384 rows of 2048, by elements -> by vectors (us): residual and
+// norm 80 -> 58 (8 groups 102 -> 58), depth average over 2 / 7 / 13 results 187 / 362 / 573 -> 118 /
+// 243 / 409 (4.6 TB/s; 32 rows, 13 results 15 -> 9), head norm and gate 82 -> 48, xIELU of 8192
+// columns 144 -> 99.
+template <typename T>
+__device__ __forceinline__ float4 ld4(const T* p) {
+  if constexpr (sizeof(T) == 4) return *reinterpret_cast<const float4*>(p);
+  else {
+    Pack4<T> v;
+    v.u = *reinterpret_cast<const u32x2*>(p);
+    return make_float4(to_f(v.h[0]), to_f(v.h[1]), to_f(v.h[2]), to_f(v.h[3]));
+  }
+}
+template <typename T>
+__device__ __forceinline__ void st4(T* p, float4 v) {
+  if constexpr (sizeof(T) == 4) *reinterpret_cast<float4*>(p) = v;
+  else {
+    Pack4<T> o;
+    o.h[0] = from_f<T>(v.x);
+    o.h[1] = from_f<T>(v.y);
+    o.h[2] = from_f<T>(v.z);
+    o.h[3] = from_f<T>(v.w);
+    *reinterpret_cast<u32x2*>(p) = o.u;
+  }
+}
+
+// out = x / rms(group of x) * w for the row held in xv (zeros past W)
+template <typename T, int V>
+__device__ __forceinline__ void group_norm_out(T* o, const float4 (&xv)[V], const float* __restrict__ w,
+                                               int W, int gw, float eps, float (&tab)[V * NT / 64]) {
+  const int wave = threadIdx.x >> 6;
+  float4 wv[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int c = 4 * (threadIdx.x + NT * k);
+    wv[k] = c < W ? ld4(w + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float ss = wave_sum((xv[k].x * xv[k].x + xv[k].y * xv[k].y) + (xv[k].z * xv[k].z + xv[k].w * xv[k].w));
+    if ((threadIdx.x & 63) == 0) tab[k * (NT / 64) + wave] = ss;
+  }
+  __syncthreads();
+  const int per = gw >> 8;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int c = 4 * (threadIdx.x + NT * k), g = (k * (NT / 64) + wave) / per;
+    if (c >= W) break;
+    float ss = 0.f;
+    for (int i = 0; i < per; ++i) ss += tab[g * per + i];
+    const float r = 1.f / sqrtf(ss / (float)gw + eps);
+    st4(o + c, make_float4(xv[k].x * r * wv[k].x, xv[k].y * r * wv[k].y, xv[k].z * r * wv[k].z,
+                           xv[k].w * r * wv[k].w));
+  }
+}
+
+template <typename T, int V>
+__global__ __launch_bounds__(NT) void residual_group_norm_vec_kernel(
+    T* __restrict__ out, float* __restrict__ x, const T* __restrict__ y,
+    const float* __restrict__ w, int W, int gw, float eps) {
+  __shared__ float tab[V * NT / 64];
+  const int64_t row = blockIdx.x;
+  float* xr = x + row * W;
+  float4 xv[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int c = 4 * (threadIdx.x + NT * k);
+    xv[k] = c < W ? ld4(xr + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if (y != nullptr) {
+    const T* yr = y + row * W;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      const int c = 4 * (threadIdx.x + NT * k);
+      if (c >= W) break;
+      const float4 a = ld4(yr + c);
+      xv[k] = make_float4(xv[k].x + a.x, xv[k].y + a.y, xv[k].z + a.z, xv[k].w + a.w);
+      st4(xr + c, xv[k]);
+    }
+  }
+  group_norm_out<T, V>(out + row * W, xv, w, W, gw, eps, tab);
+}
+
+template <typename T, int V>
+__global__ __launch_bounds__(NT) void depth_mix_norm_vec_kernel(
+    T* __restrict__ out, float* __restrict__ x, float* __restrict__ hist,
+    const T* __restrict__ y, const float* __restrict__ coef, const float* __restrict__ w,
+    int layer, int64_t hist_stride, int W, int gw, float eps) {
+  __shared__ float tab[V * NT / 64];
+  const int64_t row = blockIdx.x;
+  float* xr = x + row * W;
+  const T* yr = y + row * W;
+  float* hr = hist + row * W;
+  float4 r[V], acc[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int c = min(4 * (int)(threadIdx.x + NT * k), W - 4);
+    const float4 a = ld4(xr + c), b = ld4(yr + c);
+    r[k] = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+    acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+#pragma unroll 4
+  for (int j = 0; j <= layer; ++j) {
+    const float cj = coef[j];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      const int c = min(4 * (int)(threadIdx.x + NT * k), W - 4);
+      const float4 h = ld4(hr + (int64_t)j * hist_stride + c);
+      acc[k] = make_float4(acc[k].x + cj * h.x, acc[k].y + cj * h.y, acc[k].z + cj * h.z, acc[k].w + cj * h.w);
+    }
+  }
+  const float own = coef[layer + 1];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int c = 4 * (threadIdx.x + NT * k);
+    acc[k] = make_float4(acc[k].x + own * r[k].x, acc[k].y + own * r[k].y, acc[k].z + own * r[k].z,
+                         acc[k].w + own * r[k].w);
+    if (c < W) {
+      st4(hr + (int64_t)(layer + 1) * hist_stride + c, r[k]);
+      st4(xr + c, acc[k]);
+    } else {
+      acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  }
+  group_norm_out<T, V>(out + row * W, acc, w, W, gw, eps, tab);
+}
+
+// one wave per head vector of dv <= 256 V columns, four of them per workgroup
+template <typename T, int V>
+__global__ __launch_bounds__(NT) void head_norm_gate_vec_kernel(
+    T* __restrict__ out, const float* __restrict__ o, const T* __restrict__ g, int64_t g_stride,
+    const float* __restrict__ w, int64_t n, int H, int dv, float eps) {
+  const int64_t i = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+  if (i >= n) return;
+  const int64_t row = i / H;
+  const int h = (int)(i - row * H), lane = threadIdx.x & 63;
+  const T* gr = g + row * g_stride + h * dv;
+  float4 ov[V], gv[V], wv[V];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int c = 4 * (lane + 64 * k), cc = min(c, dv - 4);
+    ov[k] = ld4(o + i * dv + cc);
+    gv[k] = ld4(gr + cc);
+    wv[k] = ld4(w + h * dv + cc);
+    if (c < dv) ss += (ov[k].x * ov[k].x + ov[k].y * ov[k].y) + (ov[k].z * ov[k].z + ov[k].w * ov[k].w);
+  }
+  const float r = 1.f / sqrtf(wave_sum(ss) / (float)dv + eps);
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int c = 4 * (lane + 64 * k);
+    if (c >= dv) break;
+    auto f = [&](float a, float b, float z) { return a * r * b * (1.f / (1.f + expf(-z))); };
+    st4(out + i * dv + c, make_float4(f(ov[k].x, wv[k].x, gv[k].x), f(ov[k].y, wv[k].y, gv[k].y),
+                                      f(ov[k].z, wv[k].z, gv[k].z), f(ov[k].w, wv[k].w, gv[k].w)));
+  }
+}
+
 // grid (rows, H), 64 threads: o fp32 [rows, H * dv]; g [rows, g_stride] (column slice)
 template <typename T>
 __global__ __launch_bounds__(64) void head_norm_gate_kernel(
@@ -111,6 +270,32 @@ __global__ __launch_bounds__(NT) void xielu_kernel(T* __restrict__ out, const T*
     const float v = to_f(z[i]);
     const float r = v > 0.f ? a * v * v + 0.5f * v : b * (expm1f(v) - v) + 0.5f * v;
     out[i] = from_f<T>(r);
+  }
+}
+
+// eight 16-bit elements per thread and step.  exp(v) - 1 - v without cancellation: the series
+// v^2 (1/2 + v/6 + .. + v^6/40320) from -1/2 up, where its next term is 5e-8 of it, else 2^(v log2 e).
+template <typename T>
+__global__ __launch_bounds__(NT) void xielu_vec_kernel(T* __restrict__ out, const T* __restrict__ z,
+                                                       const float* __restrict__ ab, int64_t n8) {
+  const float a = ab[0], b = ab[1];
+  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n8; i += (int64_t)gridDim.x * NT) {
+    Pack8<T> v, o;
+    v.u = reinterpret_cast<const u32x4*>(z)[i];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float x = to_f(v.h[j]);
+      float p = 1.f / 40320.f;
+      p = p * x + 1.f / 5040.f;
+      p = p * x + 1.f / 720.f;
+      p = p * x + 1.f / 120.f;
+      p = p * x + 1.f / 24.f;
+      p = p * x + 1.f / 6.f;
+      p = p * x + 0.5f;
+      const float e = x > -0.5f ? x * x * p : (__builtin_amdgcn_exp2f(x * 1.44269504088896340736f) - 1.f) - x;
+      o.h[j] = from_f<T>(x > 0.f ? a * x * x + 0.5f * x : b * e + 0.5f * x);
+    }
+    reinterpret_cast<u32x4*>(out)[i] = o.u;
   }
 }
 
@@ -272,10 +457,28 @@ __global__ __launch_bounds__(NW * 64) void gate_proj_mfma_kernel(
   } while (0)
 
 static bool al16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+// rows that 256 threads hold as at most eight float4 each, in groups that waves do not straddle
+static bool row_vectors(int W, int gw) { return W <= 8 * 4 * NT && gw % 256 == 0; }
+#define KGC_ROW_V(W, GO)         \
+  do {                           \
+    if ((W) <= 4 * NT) GO(1);    \
+    else if ((W) <= 8 * NT) GO(2); \
+    else if ((W) <= 16 * NT) GO(4); \
+    else GO(8);                  \
+  } while (0)
 
 void launch_residual_group_norm(int dtype, void* out, float* x, const void* y, const float* w,
                                 int rows, int W, int groups, float eps, hipStream_t s) {
   if (rows <= 0) return;
+  const int gw = W / groups;
+  if (row_vectors(W, gw) && al16(out) && al16(x) && al16(y) && al16(w)) {
+#define KGC_RGN(V)                                                                          \
+  KGC_DISPATCH_T(dtype, residual_group_norm_vec_kernel<T, V><<<rows, NT, 0, s>>>(           \
+      (T*)out, x, (const T*)y, w, W, gw, eps))
+    KGC_ROW_V(W, KGC_RGN);
+#undef KGC_RGN
+    return;
+  }
   KGC_DISPATCH_T(dtype, residual_group_norm_kernel<T><<<rows, NT, 0, s>>>(
       (T*)out, x, (const T*)y, w, W, groups, eps));
 }
@@ -284,6 +487,15 @@ void launch_depth_mix_norm(int dtype, void* out, float* x, float* hist, const vo
                            const float* coef, const float* w, int layer, int64_t hist_stride,
                            int rows, int W, int groups, float eps, hipStream_t s) {
   if (rows <= 0) return;
+  const int gw = W / groups;
+  if (row_vectors(W, gw) && hist_stride % 4 == 0 && al16(out) && al16(x) && al16(y) && al16(w) && al16(hist)) {
+#define KGC_DMN(V)                                                                          \
+  KGC_DISPATCH_T(dtype, depth_mix_norm_vec_kernel<T, V><<<rows, NT, 0, s>>>(                \
+      (T*)out, x, hist, (const T*)y, coef, w, layer, hist_stride, W, gw, eps))
+    KGC_ROW_V(W, KGC_DMN);
+#undef KGC_DMN
+    return;
+  }
   KGC_DISPATCH_T(dtype, depth_mix_norm_kernel<T><<<rows, NT, 0, s>>>(
       (T*)out, x, hist, (const T*)y, coef, w, layer, hist_stride, W, groups, eps));
 }
@@ -291,6 +503,18 @@ void launch_depth_mix_norm(int dtype, void* out, float* x, float* hist, const vo
 void launch_head_norm_gate(int dtype, void* out, const float* o, const void* g, int64_t g_stride,
                            const float* w, int rows, int H, int dv, float eps, hipStream_t s) {
   if (rows <= 0) return;
+  if (dv % 4 == 0 && dv <= 1024 && g_stride % 4 == 0 && al16(out) && al16(o) && al16(w) &&
+      reinterpret_cast<uintptr_t>(g) % (dtype == DT_F32 ? 16 : 8) == 0) {
+    const int64_t n = (int64_t)rows * H;
+#define KGC_HNG(V)                                                                              \
+  KGC_DISPATCH_T(dtype, head_norm_gate_vec_kernel<T, V><<<(n + NT / 64 - 1) / (NT / 64), NT, 0, s>>>( \
+      (T*)out, o, (const T*)g, g_stride, w, n, H, dv, eps))
+    if (dv <= 256) KGC_HNG(1);
+    else if (dv <= 512) KGC_HNG(2);
+    else KGC_HNG(4);
+#undef KGC_HNG
+    return;
+  }
   KGC_DISPATCH_T(dtype, head_norm_gate_kernel<T><<<dim3(rows, H), 64, 0, s>>>(
       (T*)out, o, (const T*)g, g_stride, w, H, dv, eps));
 }
@@ -298,7 +522,13 @@ void launch_head_norm_gate(int dtype, void* out, const float* o, const void* g, 
 void launch_xielu(int dtype, void* out, const void* z, const float* ab, int64_t n,
                   hipStream_t s) {
   if (n <= 0) return;
-  const int grid = (int)std::min<int64_t>((n + NT - 1) / NT, 256 * 32);
+  const bool vec = dtype != DT_F32 && n % 8 == 0 && al16(out) && al16(z);
+  const int grid = (int)std::min<int64_t>(((vec ? n / 8 : n) + NT - 1) / NT, 256 * 32);
+  if (vec) {
+    if (dtype == DT_BF16) xielu_vec_kernel<bf16><<<grid, NT, 0, s>>>((bf16*)out, (const bf16*)z, ab, n / 8);
+    else xielu_vec_kernel<f16><<<grid, NT, 0, s>>>((f16*)out, (const f16*)z, ab, n / 8);
+    return;
+  }
   KGC_DISPATCH_T(dtype, xielu_kernel<T><<<grid, NT, 0, s>>>((T*)out, (const T*)z, ab, n));
 }
 

@@ -497,3 +497,49 @@ def test_gate_proj_many_rows(gpu, dt, rows, W, N):
     got = ops.gate_proj(h.to(gpu), w.to(gpu), None, ops.GATE_CAP_TANH, ops.GATE_LOGSIG_CAP_TANH, N // 2, 15.0).cpu()
     want = ref.gate_proj(h[keep], w, None, ops.GATE_CAP_TANH, ops.GATE_LOGSIG_CAP_TANH, N // 2, 15.0)
     torch.testing.assert_close(got[keep], want, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("rows,W,G", [(1, 256, 1), (3, 1280, 5), (2, 2048, 1), (5, 2560, 2), (2, 4096, 16), (3, 8192, 1)])
+def test_row_kernels_by_vectors(gpu, dt, rows, W, G):
+    """Rows held in registers: one to eight float4 per thread, threads without columns, groups of
+    one wave up to the whole row, head vectors of no multiple of 256, xIELU around the ends of its
+    series.  Against float64: sums of W squares and quotients (32 units of 2^-24), one rounding to
+    the activation type."""
+    torch.manual_seed(51)
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[dt] * 1.01 + 32 * 2.0 ** -24
+    x, y, w = torch.randn(rows, W) * 3, torch.randn(rows, W).to(dt), torch.rand(W) + 0.5
+
+    def close(got, want, unit=None):
+        err = (got.cpu().double() - want).abs()
+        assert (err <= ulp * (want.abs() if unit is None else unit) + 1e-7).all()
+
+    def norm(v, n):
+        v = v.view(rows, n, -1)
+        return (v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-5)).view(rows, W)
+    x1 = x.clone().to(gpu)
+    s = (x + y.float()).double()
+    got = ops.group_rms_norm(x1, w.to(gpu), G, 1e-5, dt, add=y.to(gpu))
+    close(got, norm(s, G) * w.double())
+    assert torch.equal(x1.cpu().double(), s)
+    hist, coef = torch.randn(6, rows + 1, W), torch.randn(6)
+    hg, x1 = hist.to(gpu), x.clone().to(gpu)
+    for layer in (0, 4):
+        h64, x0 = hg.cpu().double()[:, :rows], x1.cpu()
+        h64[layer + 1] = (x0 + y.float()).double()
+        terms = coef[: layer + 2].double()[:, None, None] * h64[: layer + 2]
+        got = ops.depth_mix_norm(x1, hg, layer, y.to(gpu), coef[: layer + 2].to(gpu), w.to(gpu), G, 1e-5, dt)
+        assert torch.equal(hg[layer + 1, :rows].cpu().double(), h64[layer + 1])
+        assert ((x1.cpu().double() - terms.sum(0)).abs() <= 8 * 2.0 ** -24 * terms.abs().sum(0)).all()
+        close(got, norm(x1.cpu().double(), G) * w.double())
+    for H, dv in ((1, W if W <= 1024 else 1024), (3, 68), (2, 516)):
+        o, big, nw = torch.randn(rows, H * dv), torch.randn(rows, H * dv + 16).to(dt), torch.rand(H * dv) + 0.5
+        v = o.double().view(rows, H, dv)
+        want = (v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-5)).view(rows, -1) * nw.double()
+        got = ops.head_norm_gate(o.to(gpu), big.to(gpu)[:, 8: 8 + H * dv], nw.to(gpu), H, 1e-5, dt)
+        close(got, want * torch.sigmoid(big[:, 8: 8 + H * dv].double()))
+    z = torch.cat([torch.randn(rows * W - 8) * 2, torch.tensor([-0.5, -0.5001, -0.4999, -1e-3, 0.0, 1e-3, -30.0, 9.0])]).to(dt)
+    z64 = z.double()
+    want = torch.where(z64 > 0, 0.7 * z64 * z64 + 0.5 * z64, 1.3 * (torch.expm1(z64) - z64) + 0.5 * z64)
+    unit = torch.where(z64 > 0, want, 1.3 * (torch.expm1(z64) - z64).abs() + 0.5 * z64.abs())
+    close(ops.xielu(z.to(gpu), torch.tensor([0.7, 1.3]).to(gpu)), want, unit)
