@@ -543,3 +543,26 @@ def test_row_kernels_by_vectors(gpu, dt, rows, W, G):
     want = torch.where(z64 > 0, 0.7 * z64 * z64 + 0.5 * z64, 1.3 * (torch.expm1(z64) - z64) + 0.5 * z64)
     unit = torch.where(z64 > 0, want, 1.3 * (torch.expm1(z64) - z64).abs() + 0.5 * z64.abs())
     close(ops.xielu(z.to(gpu), torch.tensor([0.7, 1.3]).to(gpu)), want, unit)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("T,H,G,dk,dv,rot", [(1, 4, 1, 64, 64, 64), (37, 6, 2, 40, 24, 16), (130, 16, 4, 128, 128, 64),
+                                             (9, 3, 3, 24, 8, 0), (65, 2, 1, 192, 128, 192)])
+def test_rope_kv_store_by_chunks(gpu, dt, interleaved, T, H, G, dk, dv, rot):
+    """16-byte chunks against single elements (which rows at an odd address take): the same bytes, with
+    padding slots, slots past the cache and positions outside the table."""
+    torch.manual_seed(61)
+    n, bs, nb = (H + G) * dk + G * dv, 8, T // 8 + 3
+    wide = torch.randn(T, n + 9, device=gpu).to(dt)
+    qkv = torch.empty(T, n + 8, device=gpu, dtype=dt)[:, :n]
+    qkv.copy_(wide[:, 1: n + 1])
+    table = torch.randn(50, rot, device=gpu) if rot else None
+    pos, slots = torch.randint(-2, 60, (T,), device=gpu), torch.randperm(nb * bs, device=gpu)[:T]
+    if T > 2:
+        slots[1], slots[2] = -1, nb * bs
+    got = []
+    for x in (wide[:, 1: n + 1], qkv):
+        kc, vc = (torch.zeros(nb, G, bs, d, device=gpu, dtype=dt) for d in (dk, dv))
+        got.append((ops.rope_kv_store(x, pos, table, kc, vc, slots, H, G, dk, dv, interleaved), kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(got[0][2].any())
