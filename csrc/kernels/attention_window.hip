@@ -25,6 +25,7 @@
 
 #include "window.h"
 #include <climits>
+#include <type_traits>
 
 namespace kgc {
 
@@ -691,10 +692,10 @@ __global__ __launch_bounds__(64 * NWV) void window_decode_kernel(
 //                   8 (m >> 2) + (m & 3), + 4 in the second tile),
 //   online softmax in fp32, statistics per head in the lane,
 //   O^T += V^T . P^T with P^T straight from the S^T accumulators as a pair of values (value +
-//                   remainder) and V^T through the wave's own piece of LDS; where the values are
-//                   columns of the key rows the key fragments are what is written there.
+//                   remainder) and V^T by transposing reads of the value rows in the wave's own
+//                   piece of LDS; where the values are columns of the key rows the key fragments
+//                   are what is written there.
 // The waves' states meet in LDS at the end, in wave order.
-constexpr int DM_VST = 40;             // elements per V^T row: 32 keys + 8
 
 template <typename T, int KS, int DT, int NWV>
 __global__ __launch_bounds__(64 * NWV) void window_decode_mfma_kernel(
@@ -704,7 +705,11 @@ __global__ __launch_bounds__(64 * NWV) void window_decode_mfma_kernel(
     float scale, int window, int keep_first, const float* __restrict__ gate, bool shared,
     WindowExtra ex) {
   typedef typename Vec8<T>::type V8;
-  constexpr int VBYTES = NWV * DT * 16 * DM_VST * 2, OBYTES = NWV * 16 * DT * 16 * 4;
+  constexpr bool DMA = NWV == 16;                      // 128 registers: values go to LDS by DMA
+  static_assert(!DMA || (KS == 4 && DT == 8), "16 chunks of 16 bytes per value row");
+  typedef std::conditional_t<DMA, int, int64_t> Row;   // (2^31 rows of 256 bytes are more than a GPU's memory)
+  constexpr int VST = DT * 16 + (DMA ? 0 : 8);         // elements of a value row in LDS
+  constexpr int VBYTES = NWV * 32 * VST * 2, OBYTES = NWV * 16 * DT * 16 * 4;
   __shared__ __attribute__((aligned(16))) char smem[VBYTES > OBYTES ? VBYTES : OBYTES];
   __shared__ float mm[NWV][16], ml[NWV][16];
   const int dd = blockIdx.x, g = blockIdx.y, qpg = H / G, hq0 = blockIdx.z * 16;
@@ -731,7 +736,7 @@ __global__ __launch_bounds__(64 * NWV) void window_decode_mfma_kernel(
   const int lo_w = first_visible(pos, window, ex.chunked), ns = min(keep_first, lo_w);
   const int total = ns + (pos - lo_w + 1), nch = (total + 31) >> 5;
   const int keyA = 8 * (r16 >> 2) + (r16 & 3);
-  T* vt = reinterpret_cast<T*>(smem) + wave * DT * 16 * DM_VST;
+  T* vt = reinterpret_cast<T*>(smem) + wave * 32 * VST;
   float m = wave == 0 ? ex.sink : -INFINITY;          // (the first wave always has keys)
   float l = qd == 0 && m > -INFINITY ? 1.f : 0.f;
   f32x4 o[DT];
@@ -739,26 +744,37 @@ __global__ __launch_bounds__(64 * NWV) void window_decode_mfma_kernel(
   for (int d = 0; d < DT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int ch = wave; ch < nch; ch += NWV) {
     Pack8<T> kf[2][KS];
-    int64_t row[2];
+    Row row[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int idx = min(32 * ch + keyA + 4 * j, total - 1);      // clamped: weight 0 below
       const int key = idx < ns ? idx : lo_w + (idx - ns);
       int b = bt[key / bs];
       if (b < 0 || b >= num_blocks) b = 0;
-      row[j] = (int64_t)(b * G + g) * bs + key % bs;
-      const T* kr = k_cache + row[j] * krs + 8 * qd;
+      row[j] = ((Row)b * G + g) * bs + key % bs;
+      const T* kr = k_cache + (int64_t)row[j] * krs + 8 * qd;
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         kf[j][s].u = u32x4{0u, 0u, 0u, 0u};
         if (32 * s + 8 * qd < dk) kf[j][s].u = *reinterpret_cast<const u32x4*>(kr + 32 * s);
       }
     }
-    Pack8<T> vf[2][DT / 2];
-    if (!shared) {
+    Pack8<T> vf[2][DMA ? 1 : DT / 2];
+    if constexpr (DMA) {
+      // rows 4 i .. of the chunk, 16-byte pieces permuted by the row; a row's place from the lane that
+      // has its key (the last chunk's rows were read: their products are in o)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = __shfl(row[i & 1], 4 * (i >> 1) + qd, 64);
+        const T* src = v_cache + (int64_t)r * vrs + ((r16 ^ ((4 * i + qd) & 15)) * 8);
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)(vt + 4 * i * VST), 16, 0, 0);
+      }
+    } else if (!shared) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const T* vr = v_cache + row[j] * vrs + 8 * qd;
+        const T* vr = v_cache + (int64_t)row[j] * vrs + 8 * qd;
 #pragma unroll
         for (int s = 0; s < DT / 2; ++s) {
           vf[j][s].u = u32x4{0u, 0u, 0u, 0u};
@@ -774,18 +790,18 @@ __global__ __launch_bounds__(64 * NWV) void window_decode_mfma_kernel(
       for (int s = 0; s < KS; ++s) a = mfma16x16x32(kf[j][s].v, qf[s], a);
       sc[j] = a;
     }
-    // V^T of the chunk, while the products are under way
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");    // (the last chunk's fragments were read)
-    __builtin_amdgcn_wave_barrier();
+    if constexpr (!DMA) {
+      // the chunk's value rows, while the products are under way
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");    // (the last chunk's fragments were read)
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int s = 0; s < DT / 2; ++s) {
-      if (32 * s + 8 * qd < dv) {
+      for (int s = 0; s < DT / 2; ++s) {
+        if (32 * s + 8 * qd < dv) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            vt[(32 * s + 8 * qd + e) * DM_VST + keyA + 4 * j] =
-                shared ? kf[j][s < KS ? s : 0].h[e] : vf[j][s].h[e];
+          for (int j = 0; j < 2; ++j)
+            *reinterpret_cast<u32x4*>(vt + (keyA + 4 * j) * VST + 32 * s + 8 * qd) =
+                shared ? kf[j][s < KS ? s : 0].u : vf[j][s].u;
+        }
       }
     }
     float tmax = -INFINITY;
@@ -814,13 +830,18 @@ __global__ __launch_bounds__(64 * NWV) void window_decode_mfma_kernel(
       pl.h[i] = from_f<T>(pa - to_f(ph.h[i]));
       pl.h[4 + i] = from_f<T>(pb - to_f(ph.h[4 + i]));
     }
+    if constexpr (DMA) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
       if (16 * d < dv) {
+        const int vrow = 8 * qd + (r16 >> 2);
+        const int c0 = DMA ? (((2 * d + ((r16 & 3) >> 1)) ^ (vrow & 15)) * 8 + 4 * (r16 & 1)) : 16 * d + 4 * (r16 & 3);
+        const int c1 = DMA ? c0 ^ 32 : c0;             // row + 4
+        const u32x2 v0 = ld_tr4(vt + vrow * VST + c0), v1 = ld_tr4(vt + (vrow + 4) * VST + c1);
         Pack8<T> fr;
-        fr.u = *reinterpret_cast<const u32x4*>(vt + (16 * d + r16) * DM_VST + 8 * qd);
+        fr.u = u32x4{v0[0], v0[1], v1[0], v1[1]};
         f32x4 a = o[d] * alpha;
         a = mfma16x16x32(fr.v, ph.v, a);
         o[d] = mfma16x16x32(fr.v, pl.v, a);
@@ -1674,7 +1695,8 @@ static void decode_mfma_dispatch(T* out, const T* q, const T* kc, const T* vc, c
                                  hipStream_t s) {
   const dim3 grid(D, G, (H / G + 15) / 16);
   const bool shared = kc == vc && krs == vrs && dv <= dk;
-  const bool small = (int64_t)grid.x * grid.y * grid.z >= 512;     // several workgroups per CU
+  const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
+  const bool small = wgs >= 512;                       // several workgroups per CU
 #define KGC_DM(K, D_, W)                                                                       \
   window_decode_mfma_kernel<T, K, D_, W><<<grid, 64 * W, 0, s>>>(                              \
       out, q, kc, vc, ctx_lens, dbt, bt_stride, Tp, H, G, dk, dv, krs, vrs, bs, num_blocks, scale, \
@@ -1683,7 +1705,11 @@ static void decode_mfma_dispatch(T* out, const T* q, const T* kc, const T* vc, c
   do {                                              \
     if (small) KGC_DM(K, D_, 4); else KGC_DM(K, D_, 8); \
   } while (0)
-  if (dk <= 128 && dv <= 128) KGC_DM2(4, 8);
+  // A wave's chunks follow one another, 3 us each; 16 waves halve them.  128/128, 4 key/value heads, 8
+  // (4) waves -> 16: 929 keys alone 21.4 -> 17.3 us, 4000 keys alone 70 -> 46, 32 x 2000 45 -> 31,
+  // 100 x 4000 181 -> 153; with workgroups for all CUs twice, 4 waves: 256 x 1000 114 against 102.
+  if (dk == 128 && dv == 128 && !shared && !small) KGC_DM(4, 8, 16);
+  else if (dk <= 128 && dv <= 128) KGC_DM2(4, 8);
   else if (dv <= 192) KGC_DM2(8, 12);
   else KGC_DM(8, 16, 4);
 #undef KGC_DM2

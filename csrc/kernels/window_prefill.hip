@@ -26,14 +26,6 @@ namespace {
 
 constexpr int BM = 64, BN = 64, HW = 4, NT = 512;     // rows, keys per tile, heads per workgroup
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-// column (lane & 15) of four rows: lanes 4 r .. 4 r + 3 of every 16 address row r, 4 elements each
-__device__ __forceinline__ u32x2 ld_tr4(const void* p) {
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                       (__attribute__((address_space(3))) s16x4*)p));
-}
-
 // two weights as value + remainder
 template <typename T>
 __device__ __forceinline__ void pair2(float a, float b, uint32_t& hi, uint32_t& lo) {

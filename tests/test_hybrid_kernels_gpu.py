@@ -566,3 +566,29 @@ def test_rope_kv_store_by_chunks(gpu, dt, interleaved, T, H, G, dk, dv, rot):
         kc, vc = (torch.zeros(nb, G, bs, d, device=gpu, dtype=dt) for d in (dk, dv))
         got.append((ops.rope_kv_store(x, pos, table, kc, vc, slots, H, G, dk, dv, interleaved), kc, vc))
     assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(got[0][2].any())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,rows", [(8, 2, 9), (16, 1, 40), (12, 4, 140)])
+@pytest.mark.parametrize("kw", [dict(window=0, keep=0), dict(window=300, keep=5), dict(window=128, keep=0, chunked=True, sink=0.3),
+                                dict(window=0, keep=0, softcap=15.0)])
+def test_window_decode_many_waves(gpu, dt, H, G, rows, kw):
+    """Decode rows of 128/128 heads on 16 waves (and, with 560 workgroups, on 4): one key, chunks
+    around 32 and the 16 x 32 of a round, several rounds, a padding row."""
+    torch.manual_seed(71)
+    lens = [1, 31, 32, 33, 511, 513, 1025, 700, 0] + [5 + 13 * i for i in range(rows - 9)]
+    bs, width = 16, 70
+    nb = 400
+    tables = torch.randint(0, nb, (rows, width), dtype=torch.int32)
+    kc, vc = torch.randn(nb, G, bs, 128).to(dt), torch.randn(nb, G, bs, 128).to(dt)
+    q, gate = torch.randn(rows, H, 128).to(dt), torch.rand(rows, H)
+    lens = [min(n, width * bs) for n in lens]
+    m = _meta([], [], lens, tables)
+    pos, kw = torch.tensor(lens) - 1, dict(kw)
+    args = (0.09, kw.pop("window"), kw.pop("keep"))
+    want = ops.window_attention(q, kc, vc, pos, m, *args, gate, **kw)
+    got = ops.window_attention(q.to(gpu), kc.to(gpu), vc.to(gpu), pos.to(gpu), _to(m, gpu), *args, gate.to(gpu), **kw)
+    assert (got[8] == 0).all()
+    ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
+    keep = torch.arange(rows) != 8
+    torch.testing.assert_close(got.cpu().float()[keep], want.float()[keep], rtol=1.01 * ulp, atol=2e-4)
