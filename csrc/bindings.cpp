@@ -1833,13 +1833,21 @@ void gla_scan(Tensor out, Tensor proj, Tensor low, Tensor a2, Tensor a2_bias, Te
               "kgc.gla_scan: out [T, H V]");
   TORCH_CHECK(S.is_contiguous() && S.dim() == 4 && S.size(1) == H && S.size(2) == d &&
               S.size(3) == V && S.device() == proj.device(), "kgc.gla_scan: state [slots, H, d, V]");
+  const float *a2p = f32_opt(a2, H * d * R, "a2"), *a2bp = f32_opt(a2_bias, H * d, "a2_bias");
+  const int *qp = i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"), *sp = i32_ptr(seq_lens, P, "seq_lens");
+  const int *cp = i32_ptr(ctx_lens, D, "ctx_lens"), *slot = i32_ptr(slots, P + D, "state slots");
+  const bool chunk = kgc::gla_chunk_ok((int)P, (int)Tp, (int)H, (int)d, (int)V, (int)R);
+  Tensor ws;
+  if (chunk) {
+    ws = at::empty({kgc::gla_chunk_ws((int)P, (int)Tp, (int)H)}, out.options());
+    kgc::launch_gla_chunk(dt_code(proj), out.data_ptr<float>(), proj.data_ptr(), proj.stride(0), low.data_ptr(),
+                          low.stride(0), a2p, a2bp, S.data_ptr<float>(), qp, sp, slot, (int)P, (int)Tp, (int)H,
+                          (int)V, (int)R, (float)tau, (int)S.size(0), ws.data_ptr<float>(), stream());
+  }
   kgc::launch_gla_scan(dt_code(proj), out.data_ptr<float>(), proj.data_ptr(), proj.stride(0),
-                       low.data_ptr(), low.stride(0), f32_opt(a2, H * d * R, "a2"),
-                       f32_opt(a2_bias, H * d, "a2_bias"), S.data_ptr<float>(),
-                       i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"),
-                       i32_ptr(seq_lens, P, "seq_lens"), i32_ptr(ctx_lens, D, "ctx_lens"),
-                       i32_ptr(slots, P + D, "state slots"), (int)P, (int)D, (int)Tp, (int)H,
-                       (int)d, (int)V, (int)R, (float)tau, (int)S.size(0), stream());
+                       low.data_ptr(), low.stride(0), a2p, a2bp, S.data_ptr<float>(), qp, sp, cp,
+                       chunk ? slot + P : slot, chunk ? 0 : (int)P, (int)D, (int)Tp, (int)H, (int)d,
+                       (int)V, (int)R, (float)tau, (int)S.size(0), stream());
 }
 
 void selective_scan(Tensor out, Tensor x, Tensor dt, Tensor bc, Tensor At, Tensor dt_bias,

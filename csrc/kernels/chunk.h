@@ -1,4 +1,4 @@
-// Shared by the chunkwise recurrences (chunk_scan.hip, chunk_delta.hip): fp32 operands of the bf16
+// Shared by the chunkwise recurrences (chunk_scan.hip, chunk_delta.hip, chunk_gla.hip): fp32 operands of the bf16
 // matrix cores as sums of bf16 parts, wave-wide running sums in double, and the mapping of work
 // items to pieces of ragged sequences.
 #pragma once
@@ -109,6 +109,17 @@ __device__ __forceinline__ SegItem seg_item(int item, const int* qsl, int P, int
     base += total;
   }
   return r;
+}
+
+// chunks of L tokens of the sequences before `seq`
+template <int L>
+__device__ __forceinline__ int chunks_before(int seq, const int* qsl) {
+  const int lane = threadIdx.x & 63;
+  int n = 0;
+  for (int p = lane; p < seq; p += 64) n += max(1, (qsl[p + 1] - qsl[p] + L - 1) / L);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+  return n;
 }
 
 // column c of a k index that MFMAs read permuted, so that accumulators are operands as they lie:

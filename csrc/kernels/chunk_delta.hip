@@ -61,16 +61,6 @@ __device__ __forceinline__ float ld_ba(const DeltaArgs& a, int64_t at) {
                                : (float)reinterpret_cast<const bf16*>(a.ba)[at];
 }
 
-// chunks of the sequences before `seq`
-__device__ __forceinline__ int chunks_before(int seq, const int* qsl) {
-  const int lane = threadIdx.x & 63;
-  int n = 0;
-  for (int p = lane; p < seq; p += 64) n += max(1, (qsl[p + 1] - qsl[p] + L - 1) / L);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
-  return n;
-}
-
 // inclusive running sum within each half of the wave
 __device__ __forceinline__ double half_scan(double x) {
   x = scan_step<0x111, 0xf, false>(x);
@@ -269,7 +259,7 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
   int start = seq0, len = a.qsl[seq + 1] - start;
   const int pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
   const int64_t os = (int64_t)a.H * a.dv;
-  const int chunk0 = chunks_before(seq, a.qsl) + (MODE != 0 ? seg_idx * (a.seg / L) : 0);
+  const int chunk0 = chunks_before<L>(seq, a.qsl) + (MODE != 0 ? seg_idx * (a.seg / L) : 0);
   if (MODE != 0) {
     start += seg_idx * a.seg;
     len = min(a.seg, len - seg_idx * a.seg);

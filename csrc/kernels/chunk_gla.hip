@@ -1,0 +1,329 @@
+// Chunkwise gated linear attention of prompt rows on the matrix cores.  Per (sequence, head), with a
+// decay alpha_t per key channel,
+//     S_t = diag(alpha_t) S_(t-1) + k_t v_t^T,   o_t = S_t^T q_t .
+// Over a chunk of L = 32 tokens, p_t the product of the chunk's decays up to t, r_s of those after s and
+// S_0 the state before it (products channel by channel):
+//     O   = (Q p) S_0 + A V,     A_ts = sum_c q_tc k_sc alpha_(s+1)c .. alpha_tc  (s <= t)
+//     S_L = diag(p_L) S_0 + (K r)^T V
+// Q p, K r, p_L and A depend on no state: a first launch computes them for all chunks at once, A by
+// running products from every s upwards (no quotient of products, so no decay is too small).  The walk
+// then has no serial step finer than a chunk: a workgroup of 8 waves owns 128 value columns of a head,
+// a wave 16 of them with their S in accumulators.
+//
+// Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each, six products of parts, the
+// corrections summed apart; products p and r are kept in double.
+//
+// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 1441 -> 429 us, 260 of them the first
+// launch (two vector operations per pair of tokens and channel, 140 MB written) and 196 the walk
+// (splitting S and reading those 140 MB); 2 x 8192 8214 -> 1502 (one walk per sequence, not cut into
+// segments).  From float64: 1.1e-6 -> 1.0e-6.
+#include "chunk.h"
+#include "launch.h"
+
+namespace kgc {
+
+namespace {
+
+constexpr int L = 32, D = 128;               // tokens per chunk, key channels
+constexpr int NT = 512;
+constexpr int DT = D / 16, LT = L / 16, KD = D / 32;
+constexpr int DP = D + 8, LP = L + 8;        // padded LDS rows
+constexpr int MAT = 3 * L * L;               // bf16 of one matrix of a chunk: three parts
+constexpr int RMAX = 128;                    // rank of the decay projection
+
+struct GlaArgs {
+  float* out;                                // [T, H dv]
+  const void *proj, *low;                    // q | k | v rows; decay bottleneck rows
+  int64_t ps, ls;
+  const float *a2, *a2b;                     // [H D, R], [H D]
+  float* S;
+  const int *qsl, *seq_lens, *slots;
+  int P, H, dv, R, num_slots;
+  float inv_tau;
+  // workspace, per chunk and head; rows past a sequence's end are zero
+  float *qp, *kr;                            // [L][D]
+  float* pl;                                 // [D]
+  bf16* am;                                  // [3][L][L], columns permuted
+};
+
+// q p, k r, p_L and A of every chunk: one workgroup per (chunk, head)
+template <typename T>
+__global__ __launch_bounds__(256) void gla_prep_kernel(const GlaArgs a) {
+  __shared__ __align__(16) float qs[L][D], ks[L][D], al[L][D];
+  __shared__ float lw[L][RMAX];
+  __shared__ double half[D];
+  __shared__ __align__(16) float X[L][L + 4];
+  const SegItem it = seg_item(blockIdx.x, a.qsl, a.P, L);
+  if (it.seq < 0) return;
+  const int h = blockIdx.y, tid = threadIdx.x;
+  const int c0 = it.idx * L, len = a.qsl[it.seq + 1] - a.qsl[it.seq], nl = min(L, len - c0);
+  const int slot = a.slots[it.seq];
+  if (nl <= 0 || slot < 0 || slot >= a.num_slots || a.seq_lens[it.seq] < len) return;
+  const int64_t t0 = a.qsl[it.seq] + c0, at = (int64_t)blockIdx.x * a.H + h;
+  const T* proj = reinterpret_cast<const T*>(a.proj) + t0 * a.ps;
+  const T* low = reinterpret_cast<const T*>(a.low) + t0 * a.ls;
+  for (int e = tid; e < nl * a.R; e += 256) {
+    const int t = e / a.R, j = e - t * a.R;
+    lw[t][j] = to_f(low[t * a.ls + j]);
+  }
+  const float scale = 1.f / sqrtf((float)D);
+  for (int e = tid; e < L * D; e += 256) {
+    const int t = e / D, c = e % D;
+    const T* row = proj + t * a.ps + h * D + c;
+    qs[t][c] = t < nl ? to_f(row[0]) * scale : 0.f;
+    ks[t][c] = t < nl ? to_f(row[(int64_t)a.H * D]) : 0.f;
+  }
+  __syncthreads();
+  // thread (channel, half of the tokens): decays, their products up to and after each token
+  const int c = tid % D, hf = tid / D, b = hf * (L / 2);
+  {
+    float acc[L / 2];
+#pragma unroll
+    for (int i = 0; i < L / 2; ++i) acc[i] = 0.f;
+    const float* ar = a.a2 + ((int64_t)h * D + c) * a.R;
+    for (int j = 0; j < a.R; ++j) {
+      const float w = ar[j];
+#pragma unroll
+      for (int i = 0; i < L / 2; ++i) acc[i] += w * lw[min(b + i, nl - 1)][j];
+    }
+    const float bias = a.a2b[h * D + c];
+    double p = 1.0;
+#pragma unroll
+    for (int i = 0; i < L / 2; ++i) {
+      const float x = acc[i] + bias;
+      acc[i] = b + i < nl ? expf((fminf(x, 0.f) - log1pf(expf(-fabsf(x)))) * a.inv_tau) : 1.f;
+      al[b + i][c] = acc[i];
+      p *= acc[i];
+    }
+    if (hf == 0) half[c] = p;
+    __syncthreads();
+    const double first = half[c];            // the first half's product
+    __syncthreads();
+    if (hf == 1) half[c] = p;
+    __syncthreads();
+    const double second = half[c];
+    float* qo = a.qp + at * L * D + c;
+    float* ko = a.kr + at * L * D + c;
+    p = hf ? first : 1.0;
+#pragma unroll
+    for (int i = 0; i < L / 2; ++i) {
+      p *= acc[i];
+      qo[(b + i) * D] = (float)(qs[b + i][c] * p);
+    }
+    double r = hf ? 1.0 : second;
+#pragma unroll
+    for (int i = L / 2 - 1; i >= 0; --i) {
+      ko[(b + i) * D] = (float)(ks[b + i][c] * r);
+      r *= acc[i];
+    }
+    if (hf == 0) a.pl[at * D + c] = (float)(first * second);
+  }
+  // A: thread (column s, 16 channels) carries k_s times the decays since s
+  {
+    const int s = tid >> 3, g = (tid & 7) * 16;
+    float w[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w[i] = ks[s][g + i];
+    for (int t = 0; t < L; ++t) {
+      float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; i += 4) {
+        const f32x4 d = *reinterpret_cast<const f32x4*>(&al[t][g + i]);
+        const f32x4 q = *reinterpret_cast<const f32x4*>(&qs[t][g + i]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          w[i + e] = t > s ? w[i + e] * d[e] : w[i + e];
+          (e & 1 ? a1 : a0) += w[i + e] * q[e];
+        }
+      }
+      float x = a0 + a1;
+      x += __shfl_xor(x, 1, 64);
+      x += __shfl_xor(x, 2, 64);
+      x += __shfl_xor(x, 4, 64);
+      if ((tid & 7) == 0) X[t][s] = t >= s ? x : 0.f;
+    }
+  }
+  __syncthreads();
+  if (tid < L * 4) {                         // eight (permuted) columns per store
+    const int t = tid >> 2, oct = tid & 3;
+    const f32x4 x0 = *reinterpret_cast<const f32x4*>(&X[t][oct * 4]);
+    const f32x4 x1 = *reinterpret_cast<const f32x4*>(&X[t][oct * 4 + 16]);
+    const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+    bf16x8 p[3];
+    split8<3>(x, p);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      *reinterpret_cast<bf16x8*>(a.am + at * MAT + i * L * L + t * L + oct * 8) = p[i];
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
+  __shared__ __align__(16) bf16 Qs[3 * L * DP], KT[3 * D * LP];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const int seq = blockIdx.x, nct = (a.dv + 127) / 128;
+  const int h = blockIdx.y / nct, ct = blockIdx.y - h * nct;
+  const int col = ct * 128 + wave * 16 + lr;
+  const bool colok = col < a.dv;
+  const int colc = colok ? col : a.dv - 1;                // columns off the edge: read the last
+  const int start = a.qsl[seq], len = a.qsl[seq + 1] - start;
+  const int pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
+  const int64_t os = (int64_t)a.H * a.dv;
+  if (len <= 0) return;
+  if (slot < 0 || slot >= a.num_slots || pos0 < 0) {      // padding: defined zeros
+    if (colok)
+      for (int t = lg; t < len; t += 4) a.out[(start + t) * os + (int64_t)h * a.dv + col] = 0.f;
+    return;
+  }
+  f32x4 S[DT];
+  float* Ss = a.S + ((int64_t)slot * a.H + h) * D * a.dv;
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[i][r] = pos0 == 0 ? 0.f : Ss[(i * 16 + 4 * lg + r) * a.dv + colc];
+  const T* vb = reinterpret_cast<const T*>(a.proj) + 2 * (int64_t)a.H * D + (int64_t)h * a.dv + colc;
+  // Staging: a thread takes 8 columns of one row of q p, and 8 tokens of one column of k r, in both
+  // cases the pieces 4 i .. and 16 + 4 i .. of 32: adjacent in the permuted order, one store.
+  f32x4 rq[2], rt[2];
+  const int ut = tid / 16, uc = (tid % 16 / 4) * 32 + (tid % 4) * 4, up_ = (tid % 16) * 8;
+  const int ta = tid / D * 4, tc = tid % D;
+  const int chunk0 = chunks_before<L>(seq, a.qsl);
+  auto fetch = [&](int ci) {
+    const int64_t at = ((int64_t)ci * a.H + h) * L * D;
+    rq[0] = *reinterpret_cast<const f32x4*>(a.qp + at + ut * D + uc);
+    rq[1] = *reinterpret_cast<const f32x4*>(a.qp + at + ut * D + uc + 16);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) rt[i >> 2][i & 3] = a.kr[at + (ta + (i >> 2) * 16 + (i & 3)) * D + tc];
+  };
+  auto park = [&]() {
+    float x[8];
+    bf16x8 p[3];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = rq[i >> 2][i & 3];
+    split8<3>(x, p);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(Qs + i * L * DP + ut * DP + up_) = p[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = rt[i >> 2][i & 3];
+    split8<3>(x, p);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(KT + (i * D + tc) * LP + ta * 2) = p[i];
+  };
+  fetch(chunk0);
+  for (int c0 = 0, ci = chunk0; c0 < len; c0 += L, ++ci) {
+    const int nl = min(L, len - c0);
+    park();
+    __syncthreads();
+    const int64_t t0 = start + c0, at = (int64_t)ci * a.H + h;
+    // this lane's v (tokens 4 lg + r of each tile), its fragments of A, the channels' decays
+    T v[LT][4];
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[ti][r] = vb[(t0 + min(ti * 16 + lg * 4 + r, nl - 1)) * a.ps];
+    bf16x8 fp[LT][3];
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        fp[ti][i] = *reinterpret_cast<const bf16x8*>(a.am + at * MAT + i * L * L + (ti * 16 + lr) * L + lg * 8);
+    f32x4 pl[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) pl[dt] = *reinterpret_cast<const f32x4*>(a.pl + at * D + dt * 16 + 4 * lg);
+    f32x4 o[LT], ol[LT];
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti) o[ti] = ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < KD; ++j) {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = S[2 * j + (i >> 2)][i & 3];
+      bf16x8 sp[3];
+      split8<3>(x, sp);
+#pragma unroll
+      for (int ti = 0; ti < LT; ++ti) {
+        bf16x8 fa[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          fa[i] = *reinterpret_cast<const bf16x8*>(Qs + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
+        mm<true, 3, 3>(fa, sp, o[ti], ol[ti]);
+      }
+    }
+    fetch(c0 + L < len ? ci + 1 : ci);       // (the last one again at the end: no branch)
+    bf16x8 vp[3];
+    {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {          // tokens past the end: k r and A are zero, v may not be finite
+        const int t = (i >> 2) * 16 + lg * 4 + (i & 3);
+        x[i] = t < nl ? to_f(v[i >> 2][i & 3]) : 0.f;
+      }
+      split8<3>(x, vp);
+    }
+    float* oc = a.out + t0 * os + (int64_t)h * a.dv + col;
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti) {
+      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+      mm<true, 3, 3>(fp[ti], vp, hi, lo);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = ti * 16 + lg * 4 + e;
+        if (colok && t < nl) oc[t * os] = (o[ti][e] + hi[e]) + (ol[ti][e] + lo[e]);
+      }
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      bf16x8 fa[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        fa[i] = *reinterpret_cast<const bf16x8*>(KT + (i * D + dt * 16 + lr) * LP + lg * 8);
+      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+      mm<true, 3, 3>(fa, vp, hi, lo);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[dt][e] = __builtin_fmaf(S[dt][e], pl[dt][e], hi[e] + lo[e]);
+    }
+    __syncthreads();
+  }
+  if (colok)
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Ss[(i * 16 + 4 * lg + r) * a.dv + col] = S[i][r];
+}
+
+template <typename T>
+void run(const GlaArgs& a, int chunks, hipStream_t s) {
+  gla_prep_kernel<T><<<dim3(chunks, a.H), 256, 0, s>>>(a);
+  gla_walk_kernel<T><<<dim3(a.P, a.H * ((a.dv + 127) / 128)), NT, 0, s>>>(a);
+}
+
+}  // namespace
+
+bool gla_chunk_ok(int P, int Tp, int H, int d, int V, int R) {
+  // chunks that are mostly full: 1 x 48 tokens 46 -> 35 us, 64 x 48 218 -> 120, 4 x 60 63 -> 42
+  return P > 0 && (Tp >= 24 * P || Tp >= 1024) && d == D && V >= 16 && R <= RMAX &&
+         (int64_t)H * ((V + 127) / 128) <= 65535;
+}
+// floats of workspace
+int64_t gla_chunk_ws(int P, int Tp, int H) {
+  return (int64_t)(Tp / L + P) * H * (2 * L * D + D + MAT / 2);
+}
+void launch_gla_chunk(int dtype, float* out, const void* proj, int64_t ps, const void* low, int64_t ls,
+                      const float* a2, const float* a2b, float* S, const int* qsl, const int* seq_lens,
+                      const int* slots, int P, int Tp, int H, int V, int R, float tau, int num_slots,
+                      float* ws, hipStream_t s) {
+  const int chunks = Tp / L + P;
+  GlaArgs a{};
+  a.out = out; a.proj = proj; a.low = low; a.ps = ps; a.ls = ls; a.a2 = a2; a.a2b = a2b; a.S = S;
+  a.qsl = qsl; a.seq_lens = seq_lens; a.slots = slots;
+  a.P = P; a.H = H; a.dv = V; a.R = R; a.num_slots = num_slots; a.inv_tau = 1.f / tau;
+  a.qp = ws;
+  a.kr = a.qp + (int64_t)chunks * H * L * D;
+  a.pl = a.kr + (int64_t)chunks * H * L * D;
+  a.am = reinterpret_cast<bf16*>(a.pl + (int64_t)chunks * H * D);
+  if (dtype == DT_BF16) run<bf16>(a, chunks, s);
+  else if (dtype == DT_F16) run<f16>(a, chunks, s);
+  else run<float>(a, chunks, s);
+}
+
+}  // namespace kgc

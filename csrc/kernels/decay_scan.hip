@@ -200,7 +200,7 @@ template <typename T, int RI>
 __global__ __launch_bounds__(NT) void gla_decode_kernel(
     float* __restrict__ out, const T* __restrict__ proj, int64_t ps, const T* __restrict__ low,
     int64_t ls, const float* __restrict__ a2, const float* __restrict__ a2b, float* __restrict__ S,
-    const int* __restrict__ ctx, const int* __restrict__ slots, int H, int d, int V, int R,
+    const int* __restrict__ ctx, const int* __restrict__ slots, int row0, int H, int d, int V, int R,
     float inv_tau, int num_slots) {
   __shared__ float kqa[3][16 * RI];
   __shared__ __align__(16) float sums[NT / 64][64];
@@ -209,7 +209,8 @@ __global__ __launch_bounds__(NT) void gla_decode_kernel(
   const int cl = (threadIdx.x & 15) * 4, col = blockIdx.z * 64 + cl;
   const bool colok = col < V;
   const int slot = slots[s], pos = ctx[s] - 1;
-  float* orow = out + (int64_t)s * H * V + h * V + col;
+  const int64_t t = row0 + s;
+  float* orow = out + t * H * V + h * V + col;
   if (slot < 0 || slot >= num_slots || pos < 0) {
     if (rg == 0 && colok) *reinterpret_cast<float4*>(orow) = make_float4(0.f, 0.f, 0.f, 0.f);
     return;
@@ -222,7 +223,7 @@ __global__ __launch_bounds__(NT) void gla_decode_kernel(
     Sr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (pos != 0 && r < d && colok) Sr[i] = *reinterpret_cast<const float4*>(Sp + (int64_t)r * V);
   }
-  const T* row = proj + (int64_t)s * ps;
+  const T* row = proj + t * ps;
   float v[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) v[c] = colok ? to_f(row[2 * H * d + h * V + col + c]) : 0.f;
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(NT) void gla_decode_kernel(
       kv = to_f(row[H * d + h * d + r]);
       qv = to_f(row[h * d + r]) * (1.f / sqrtf((float)d));
       const float* ar = a2 + (int64_t)(h * d + r) * R;
-      const T* lw = low + (int64_t)s * ls;
+      const T* lw = low + t * ls;
       float acc = 0.f;
 #pragma unroll 8
       for (int j = 0; j < R; ++j) acc += ar[j] * to_f(lw[j]);
@@ -406,13 +407,14 @@ void launch_gla_scan(int dtype, float* out, const void* proj, int64_t ps, const 
                      hipStream_t s) {
   if (P + D <= 0) return;
   // decode rows that share a launch with prompts stay with the scan, beside which they cost nothing
+  // (prompts that run chunkwise are not in this call)
   if (P == 0 && V % 4 == 0 && reinterpret_cast<uintptr_t>(S) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(out) % 16 == 0) {
     const dim3 grid(D, H, (V + 63) / 64);
 #define KGC_GLA_D(RI)                                                                        \
   KGC_DS_DISPATCH_T(dtype, gla_decode_kernel<T, RI><<<grid, NT, 0, s>>>(                     \
-      out, (const T*)proj, ps, (const T*)low, ls, a2, a2b, S, ctx_lens, slots, H, d, V, R,   \
-      1.f / tau, num_slots))
+      out, (const T*)proj, ps, (const T*)low, ls, a2, a2b, S, ctx_lens, slots, Tp, H, d, V,  \
+      R, 1.f / tau, num_slots))
     if (d <= 64) KGC_GLA_D(4);
     else if (d <= 128) KGC_GLA_D(8);
     else KGC_GLA_D(16);

@@ -592,3 +592,23 @@ def test_window_decode_many_waves(gpu, dt, H, G, rows, kw):
     ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
     keep = torch.arange(rows) != 8
     torch.testing.assert_close(got.cpu().float()[keep], want.float()[keep], rtol=1.01 * ulp, atol=2e-4)
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("H,V,R", [(2, 64, 5), (1, 144, 16), (3, 40, 1)])
+@pytest.mark.parametrize("lens,before,D_ctx", CHUNKS)
+def test_gla_scan_chunkwise(gpu, dt, H, V, R, lens, before, D_ctx):
+    """Prompt rows in chunks of 32 (and decode rows behind them): ends inside a chunk, continued and
+    fresh states, a padding sequence, value columns off a wave's 16 and a workgroup's 128; decays from
+    next to nothing to all but zero.  Products of up to 32 decays (R + 1 terms over tau each) and
+    sums of d + 32 terms, in units of 2^-24 of the sums of absolute values."""
+    torch.manual_seed(81)
+    d, tau = 128, 4.0
+    m, T, n = _chunk_step(lens, before, D_ctx)
+    for open_ in (3.0, -12.0):
+        terms, run = _gla_case(T, n, H, d, V, R, dt, tau, gpu, open_)
+        want, unit, S, SA = _matrix64(m, *terms)
+        st = terms[0].to(gpu)
+        got = run(st, _to(m, gpu))
+        assert ((got.cpu() - want).abs() <= (d + 64) * unit + 1e-30).all()
+        assert ((st.cpu() - S).abs() <= 128 * SA + 1e-30).all()
