@@ -433,9 +433,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_gqa_kernel(
   const TablePtr bt = (TablePtr)(block_tables + (int64_t)seq * bt_stride);
   auto fetch_bt = [&](int kt) {
     auto id = [&](int key) {
-      const int i = min(key, L - 1) >> bs_log2;
+      int i = min(key, L - 1) >> bs_log2;
       KGC_DCHECK_RANGE(i, 0, bt_stride, "block-table column");
-      const int v = bt[i];
+      int v = bt[i];
       KGC_DCHECK_RANGE(v, 0, num_blocks, "block id");
       return v;
     };

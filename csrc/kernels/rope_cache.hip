@@ -238,7 +238,7 @@ __global__ __launch_bounds__(KVG_NT) void kv_group_kernel(
   const int lane = threadIdx.x & 63, row = t0 - 7 + lane;
   int slot = -1, pos = 0;
   if (lane < 22 && row >= 0 && row < T_) {
-    const int64_t sl = slot_mapping[row];
+    int64_t sl = slot_mapping[row];
     KGC_DCHECK_RANGE(sl, -1, (int64_t)num_blocks * bs, "KV slot");
     slot = sl < 0 ? -1 : (int)sl;
     if (slot >= 0) pos = (int)positions[row];
