@@ -29,7 +29,9 @@
 //
 // Few long sequences: the walk is serial, so a step of few workgroups is cut into segments.  A
 // first launch computes every segment's contribution from a zero state, the second starts each
-// segment from the sum of its predecessors' decayed contributions.
+// segment from the sum of its predecessors' decayed contributions.  The second launch writes the slots,
+// so it takes the states they held from copies (as n and m): the first launch's workgroups of a
+// sequence's last segment, whose contribution nobody needs, put S in that segment's place.
 #include "chunk.h"
 #include "launch.h"
 
@@ -78,7 +80,8 @@ struct ChunkArgs {
   const int *qsl, *seq_lens, *slots;
   int P, H, hpg, dv, num_slots;  // hpg: heads per q / k group
   int seg;                          // tokens per segment, a multiple of the chunk (0: not cut)
-  float* seg_state;                 // [items][H][d (dv + 1)]: S, n of a segment from zero
+  // [items][H][d (dv + 1)]: S, n of a segment from zero; a cut sequence's last: S as the slot held it
+  float* seg_state;
   double* seg_gate;                 // [items][H][2]: its log decay, its m
 };
 
@@ -124,8 +127,8 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
     seg_idx = it.idx;
     seg_first = it.first;
     seg_count = it.count;
-    if (MODE == 1 && seg_idx + 1 == seg_count) return;
   }
+  const bool last_seg = MODE != 0 && seg_idx + 1 == seg_count;
   const int nct = (a.dv + 16 * WPH - 1) / (16 * WPH);
   const int hb = blockIdx.y / nct, ct = blockIdx.y - hb * nct;
   const int h0 = hb * HPW, hw = wave / WPH, h = h0 + hw, grp = h0 / a.hpg;
@@ -147,20 +150,31 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
     return;
   }
   const bool fresh = pos0 == 0;
+  if (MODE == 1 && last_seg && (fresh || seg_count == 1)) return;
 
   // ---- the state this walk starts from --------------------------------------------------
-  const int64_t sh = (int64_t)D * a.dv;
+  const int64_t sh = (int64_t)D * a.dv, item_floats = sh + (MLSTM ? D : 0);
   float* Ss = a.S + ((int64_t)slot * a.H + h) * sh;
+  float* copy = a.seg_state + ((int64_t)(seg_first + seg_count - 1) * a.H + h) * item_floats;
+  const float* from = MODE == 2 && seg_count > 1 ? copy : Ss;
   f32x4 S[DT];
   double m0 = 0.0;                           // mLSTM: running maximum (kept by the gates' wave)
-  const bool zero = MODE == 1 || fresh;
+  const bool zero = (MODE == 1 && !last_seg) || fresh;
 #pragma unroll
   for (int i = 0; i < DT; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = i * 16 + 4 * lg + r;
-      S[i][r] = zero ? 0.f : Ss[row * a.dv + colc];
+      S[i][r] = zero ? 0.f : from[row * a.dv + colc];
     }
+  if (MODE == 1 && last_seg) {
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (colok) copy[(i * 16 + 4 * lg + r) * a.dv + col] = S[i][r];
+    return;
+  }
   if (MLSTM) {
     if (MODE == 1) m0 = -INFINITY;
     else if (!fresh) m0 = a.m0[(int64_t)seq * a.H + h];
@@ -172,7 +186,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
     for (int j = 0; j < seg_idx; ++j) {
       const int64_t it = (int64_t)(seg_first + j) * a.H + h;
       const double b = a.seg_gate[2 * it], mj = a.seg_gate[2 * it + 1];
-      const float* sp = a.seg_state + it * (sh + (MLSTM ? D : 0));
+      const float* sp = a.seg_state + it * item_floats;
       float f, g = 1.f;
       int vj = a.dv;                          // opaque: see below
       asm volatile("" : "+s"(vj));
@@ -594,10 +608,10 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
   // ---- the state after the walk -----------------------------------------------------------
   int dw = a.dv;                             // opaque: addresses are not kept across the walk
   asm volatile("" : "+s"(dw));
-  const bool to_slot = MODE == 0 || (MODE == 2 && seg_idx + 1 == seg_count);
+  const bool to_slot = MODE == 0 || (MODE == 2 && last_seg);
   if (MODE == 1 || to_slot) {
     const int64_t it = (int64_t)(seg_first + seg_idx) * a.H + h;
-    float* dst = MODE == 1 ? a.seg_state + it * (sh + (MLSTM ? D : 0)) : Ss;
+    float* dst = MODE == 1 ? a.seg_state + it * item_floats : Ss;
 #pragma unroll
     for (int i = 0; i < DT; ++i)
 #pragma unroll

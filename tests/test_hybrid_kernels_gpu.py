@@ -314,6 +314,42 @@ def test_ssd_scan_chunkwise(gpu, dt, H, G, V, lens, before, D_ctx):
     assert ((S_g.double().cpu() - S_w).abs() <= 16 * S_u).all()
 
 
+@pytest.mark.parametrize("op,dt", [("mlstm", torch.bfloat16), ("mlstm", torch.float16), ("ssd", torch.bfloat16)])
+def test_scan_segments_start_from_the_incoming_state(gpu, op, dt):
+    """Continued prompts that are cut into segments, while products on another stream hold
+    workgroups back: a segment that starts after its sequence's last one has ended still walks
+    from the state the slot held before the call.  The bits of the same call alone, which the
+    tests above compare with float64; the last segments are short."""
+    torch.manual_seed(27)
+    m, T, n = _chunk_step([1025, 449], [700, 33], [5])
+    m = _to(m, gpu)
+    if op == "mlstm":
+        H, d, dv = 4, 128, 256
+        st = [torch.randn(n, H, d, dv), torch.randn(n, H, d), torch.rand(n, H) * 2]
+        x = torch.randn(T, 2 * H * d + 2 * H * dv).to(dt).to(gpu)
+        gates = torch.cat([torch.randn(T, H), torch.full((T, H), -1e-3)], dim=1).to(gpu)
+        run = lambda s: ops.mlstm_scan(x, gates, s, m, H, d, dv)   # noqa: E731
+    else:
+        H, V, N = 48, 64, 128
+        st = [torch.randn(n, H, N, V)]
+        x, dtv = torch.randn(T, H * V + 2 * N).to(gpu), torch.randn(T, H).to(dt).to(gpu)
+        par = [torch.full((H,), -6.0), torch.zeros(H), torch.randn(H)]
+        par = [y.to(gpu) for y in par]
+        run = lambda s: ops.ssd_scan(x, dtv, *par, s[0], m, H, V, N, 1)   # noqa: E731
+    alone = [y.to(gpu) for y in st]
+    want = run(alone)
+    a, side = torch.randn(4096, 4096, device=gpu, dtype=torch.bfloat16), torch.cuda.Stream()
+    for _ in range(8):
+        s = [y.to(gpu) for y in st]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            for _ in range(6):
+                torch.mm(a, a)
+        got = run(s)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and all(torch.equal(y, z) for y, z in zip(s, alone))
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,G,V", [(2, 1, 128), (3, 3, 40), (3, 1, 144)])
 @pytest.mark.parametrize("lens,before,D_ctx", CHUNKS)
