@@ -516,7 +516,7 @@ def test_gla_decode_rows(gpu, dt, H, d, V, R):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,W,N", [(64, 128, 1), (65, 1024, 17), (79, 1152, 8), (1000, 2048, 16), (64, 2304, 33),
                                       (100, 4096, 5), (8200, 256, 8)])
-def test_gate_proj_many_rows(gpu, dt, rows, W, N):
+def test_gate_proj_matrix_cores(gpu, dt, rows, W, N):
     """Rows from the matrix-core kernel's least, around its blocks of 16 rows and 16 outputs, widths of
     every register form, more blocks than workgroups; a row of NaN stays alone.  Sums of W fp32 terms
     in parts: 2^-24 of the sum of absolute products, times the sums' depth (below 24)."""
