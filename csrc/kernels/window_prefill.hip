@@ -19,6 +19,7 @@
 // alone are 110 us of the 229 at a large product's rate) and the softmax's vector work (80 us), which
 // overlap in part.  Not the loads: a ring of four tiles filled by LDS-DMA three tiles ahead took 249 us.
 #include "window.h"
+#include <type_traits>
 
 namespace kgc {
 
@@ -36,9 +37,25 @@ __device__ __forceinline__ void pair2(float a, float b, uint32_t& hi, uint32_t& 
   lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((F2{a - (float)h[0], b - (float)h[1]}), T2));
 }
 
+// tanh of |y| <= 5/8: y + y^3 p(y^2), p fitted to the least relative error, 4e-9 of tanh.  (1 - 2 / (1 +
+// e^(2 y)) has the error of a number near 1 where tanh is small: scores of deviation 2 under a cap of 30
+// are off by up to 5.6e-6, 1.5e-6 rms; by 1.2e-6, 1.3e-7 here; by 1.1e-6, 0.9e-7 with a correctly rounded
+// tanh.)
+__device__ __forceinline__ float tanh_near(float y) {
+  const float z = y * y;
+  float p = __builtin_fmaf(z, -0.00570531f, 0.02063936f);
+  p = __builtin_fmaf(z, p, -0.05373979f);
+  p = __builtin_fmaf(z, p, 0.13331443f);
+  p = __builtin_fmaf(z, p, -0.33333282f);
+  return __builtin_fmaf(y * z, p, y);
+}
+__device__ __forceinline__ float tanh_far(float y) {
+  return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(y * 2.88539008177792681f));
+}
+
 // KS: dk / 32; DT: dv / 16; NJ: 16-key tiles per softmax step (fewer: fewer registers); ALIAS: values
 // are the first dv columns of the key rows
-template <typename T, int KS, int DT, int NJ, bool ALIAS>
+template <typename T, int KS, int DT, int NJ, bool ALIAS, bool CAP>
 __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
     T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k_cache,
     const T* __restrict__ v_cache, const int* __restrict__ qsl, const int* __restrict__ seq_lens,
@@ -157,10 +174,8 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
     }
   };
 
-  const bool capped = ex.softcap > 0.f;
-  const float sl = capped ? scale * (2.f * LOG2E) / ex.softcap : scale * LOG2E;
-  const float cl = ex.softcap * LOG2E;
-  const float fl = capped ? 1.f : sl;                 // what is left to multiply (> 0: see the launcher)
+  const float sl = CAP ? scale / ex.softcap : scale * LOG2E;
+  const float fl = CAP ? ex.softcap * LOG2E : sl;  // what is left to multiply (> 0: see the launcher)
   pages(0);
   fetch(0);
   pages(min(1, ntile - 1));
@@ -203,12 +218,32 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         // (whole loops under each uniform test: a branch per element costs more than its work)
-        if (capped)                          // cap tanh(y) = cap (1 - 2 / (1 + e^(2 y)))
+        if constexpr (CAP) {                 // tanh(score / cap); scores beyond 5/8 of the cap are rare
+          float far = 0.f;
 #pragma unroll
           for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              s[c][j][i] = cl - 2.f * cl * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[c][j][i] * sl));
+            for (int i = 0; i < 4; ++i) {
+              s[c][j][i] *= sl;
+              far = fmaxf(far, fabsf(s[c][j][i]));
+            }
+          if (__any(far > 0.625f)) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const float y = s[c][j][i], near = tanh_near(y);
+                float t = tanh_far(y);
+                asm("" : "+v"(t));           // (no branch per element)
+                s[c][j][i] = fabsf(y) > 0.625f ? t : near;
+              }
+          } else {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) s[c][j][i] = tanh_near(s[c][j][i]);
+          }
+        }
         if (!full) {
           const int last = min(hi - 1, qpos[c]) - k0 - 4 * qd, low = row_lo[c] - k0 - 4 * qd,
                     kept = keep_first - k0 - 4 * qd;
@@ -317,27 +352,27 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   }
 }
 
-template <typename T, int KS, int DT, int NJ, bool ALIAS>
+template <typename T, int KS, int DT, int NJ, bool ALIAS, bool CAP>
 void run(T* out, const T* q, const T* kc, const T* vc, const int* qsl, const int* seq_lens, const int* pbt,
          int bt_stride, const int* work_seq, const int* work_blk, int n_work, int blk_rows, int H, int G,
          int krs, int vrs, int bs, int num_blocks, float scale, int window, int keep_first, const float* gate,
          const WindowExtra& ex, hipStream_t s) {
   constexpr size_t lds = sizeof(T) * 2 * BN * (KS * 32 + 8 + (ALIAS ? 0 : DT * 16 + 8));
   static const bool set = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&window_prefill_gqa_kernel<T, KS, DT, NJ, ALIAS>),
+      reinterpret_cast<const void*>(&window_prefill_gqa_kernel<T, KS, DT, NJ, ALIAS, CAP>),
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
   (void)set;
   const int shift = (bs & (bs - 1)) == 0 ? __builtin_ctz(bs) : -1;
-  window_prefill_gqa_kernel<T, KS, DT, NJ, ALIAS>
+  window_prefill_gqa_kernel<T, KS, DT, NJ, ALIAS, CAP>
       <<<dim3(H / HW, n_work * (blk_rows / BM)), NT, lds, s>>>(
           out, q, kc, vc, qsl, seq_lens, pbt, bt_stride, work_seq, work_blk, blk_rows, H, G, krs, vrs, bs,
           shift, num_blocks, scale, window, keep_first, gate, ex);
 }
 
-template <typename T, typename... A>
+template <typename T, bool CAP, typename... A>
 bool dispatch(int dk, int dv, bool alias, T* out, const T* q, const T* kc, const T* vc, A... a) {
-  if (dk == 128 && dv == 128 && !alias) run<T, 4, 8, 4, false>(out, q, kc, vc, a...);
-  else if (dk == 256 && dv == 192 && alias) run<T, 8, 12, 2, true>(out, q, kc, vc, a...);
+  if (dk == 128 && dv == 128 && !alias) run<T, 4, 8, 4, false, CAP>(out, q, kc, vc, a...);
+  else if (dk == 256 && dv == 192 && alias) run<T, 8, 12, 2, true, CAP>(out, q, kc, vc, a...);
   else return false;
   return true;
 }
@@ -351,7 +386,7 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
                                int window, int keep_first, const float* gate, const WindowExtra& ex,
                                hipStream_t s) {
   // Four heads on one staged tile pay at every length, against one head per workgroup (bf16, 16 heads
-  // on 4 key/value heads): window 1024 with 8 x 2048 rows 355 -> 199 us, causal and capped 577 -> 337,
+  // on 4 key/value heads): window 1024 with 8 x 2048 rows 355 -> 199 us, causal and capped 577 -> 291,
   // 48 rows after 3000 83 -> 68, 48 alone equal; latent rows (one key/value head), 32 x 512 rows
   // 380 -> 131 us, 4 x 2000 after 500 974 -> 390.  The maximum is taken before the scale, which has to be
   // positive for that.
@@ -359,14 +394,15 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
       blk_rows % BM != 0)
     return false;
   const bool alias = kc == vc && krs == vrs;
-  if (dtype == DT_BF16)
-    return dispatch<bf16>(dk, dv, alias, (bf16*)out, (const bf16*)q, (const bf16*)kc, (const bf16*)vc, qsl,
-                          seq_lens, pbt, bt_stride, work_seq, work_blk, n_work, blk_rows, H, G, krs, vrs, bs,
-                          num_blocks, scale, window, keep_first, gate, ex, s);
-  if (dtype == DT_F16)
-    return dispatch<f16>(dk, dv, alias, (f16*)out, (const f16*)q, (const f16*)kc, (const f16*)vc, qsl,
-                         seq_lens, pbt, bt_stride, work_seq, work_blk, n_work, blk_rows, H, G, krs, vrs, bs,
-                         num_blocks, scale, window, keep_first, gate, ex, s);
+  auto go = [&](auto cap, auto* o) {
+    typedef std::remove_pointer_t<decltype(o)> T;
+    return dispatch<T, decltype(cap)::value>(dk, dv, alias, o, (const T*)q, (const T*)kc, (const T*)vc, qsl, seq_lens,
+                                             pbt, bt_stride, work_seq, work_blk, n_work, blk_rows, H, G, krs, vrs,
+                                             bs, num_blocks, scale, window, keep_first, gate, ex, s);
+  };
+  const bool capped = ex.softcap > 0.f;
+  if (dtype == DT_BF16) return capped ? go(std::true_type(), (bf16*)out) : go(std::false_type(), (bf16*)out);
+  if (dtype == DT_F16) return capped ? go(std::true_type(), (f16*)out) : go(std::false_type(), (f16*)out);
   return false;
 }
 

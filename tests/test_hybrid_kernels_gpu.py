@@ -481,6 +481,31 @@ def test_window_attention_shared_tiles(gpu, dt, H, G, latent, bs, kw):
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("latent", [False, True])
+@pytest.mark.parametrize("cap", [1e6, 1.5])
+def test_window_attention_capped_scores(gpu, dt, latent, cap):
+    """Capped scores keep fp32's relative precision where the cap is far above them (a difference
+    of numbers near the cap would be off by 1e6 2^-24 and more, whole units of the weights'
+    exponents), and take both ends of tanh where it is not.  The bound is the shared tiles'."""
+    torch.manual_seed(32)
+    G, H, bs, (dk, dv) = 1, 4, 16, (256, 192) if latent else (128, 128)
+    lens = [130, 33]
+    width = 9
+    tables = (torch.randperm(2 * width) + 1).view(2, width).int()
+    kc = torch.randn(2 * width + 1, G, bs, dk).to(dt)
+    vc = kc[..., :dv] if latent else torch.randn(2 * width + 1, G, bs, dv).to(dt)
+    m, T = _meta(lens, lens, [], tables), sum(lens)
+    pos, q = torch.cat([torch.arange(n) for n in lens]), torch.randn(T, H, dk).to(dt)
+    args = (1.5 / dk ** 0.5, 0, 0, torch.ones(T, H))
+    want = ops.window_attention(q, kc, vc, pos, m, *args, softcap=cap)
+    kg = kc.to(gpu)
+    got = ops.window_attention(q.to(gpu), kg, kg[..., :dv] if latent else vc.to(gpu), pos.to(gpu), _to(m, gpu),
+                               *args[:3], args[3].to(gpu), softcap=cap)
+    ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
+    torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
+
+
 def _gla_case(T, slots, H, d, V, R, dt, tau, dev, open_=3.0):
     """Inputs of gla_scan and its terms for ``_matrix64``."""
     proj = (torch.randn(T, 2 * H * d + H * V + R) * 0.7).to(dt)
