@@ -7,7 +7,7 @@
 namespace kgc {
 
 // x = sum of NP bf16 parts, each the rounding of what the ones before it leave; two at a time, so
-// that one instruction rounds and packs a pair
+// that one instruction rounds and packs a pair (an infinity leaves NaN)
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 template <int NP>
 __device__ __forceinline__ void split2(float x0, float x1, uint32_t (&p)[NP]) {
@@ -79,6 +79,39 @@ __device__ __forceinline__ double lane63(double x) {
   const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, 63);
   const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), 63);
   return __builtin_bit_cast(double, hi << 32 | lo);
+}
+
+// The products over a chunk multiply a token's value by the masked zeros of the rows before it, which a
+// value that is not finite would reach.  v[i]: token tok(i) of the lane's column (one of the four lanes
+// that share lane & 15).  Such values become zero; returned is the column's first such token, from
+// which on its outputs and its state have to be made NaN (`none`: every value is finite).  A sum that
+// overflows only costs the closer look.
+template <int N, typename V, typename F>
+__device__ __forceinline__ int take_nonfinite(V (&v)[N], int none, F tok) {
+  float z = 0.f;
+  if constexpr (sizeof(V) == 2) {            // products with zeros, two at a time
+    typedef V V2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < N; i += 2) {
+      if constexpr (__is_same(V, f16)) z = __builtin_amdgcn_fdot2(V2{v[i], v[i + 1]}, V2{0, 0}, z, false);
+      else z = __builtin_amdgcn_fdot2_f32_bf16(V2{v[i], v[i + 1]}, V2{0, 0}, z, false);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) z += (float)v[i];
+  }
+  int first = none;
+  if (__any(!(fabsf(z) < INFINITY))) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (!(fabsf((float)v[i]) < INFINITY)) {
+        first = min(first, tok(i));
+        v[i] = (V)0.f;
+      }
+    first = min(first, __shfl_xor(first, 16, 64));
+    first = min(first, __shfl_xor(first, 32, 64));
+  }
+  return first;
 }
 
 // Sequence and segment of work item `item` (every lane of every wave gets the same answer)

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
     }
     wave_lds();
 #pragma unroll
-    for (int t = 0; t < L; ++t) X[hf][t][s] = T[t] * beta;
+    for (int t = 0; t < L; ++t) X[hf][t][s] = t < s ? 0.f : T[t] * beta;   // (beta may be NaN)
     wave_lds();
     put(0);
   }
@@ -408,6 +408,7 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
     }
     // R, U = W R (rows past the end: W is zero there)
     bf16x8 up[3];
+    int bad = L;                             // first token whose value is not finite
     {
       float x[8];
 #pragma unroll
@@ -428,8 +429,30 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[ti * 4 + e] = hi[e] + lo[e];
       }
+      // A row of R or W that is not finite reaches all rows of U, or all from its own on: the last one
+      // shows it.  Then U once more without such rows of R, and without what is not finite itself,
+      // before P carries it to the rows before it.
+      if (__any(!(fabsf(x[7]) < INFINITY))) {
+        auto tok = [&](int i) { return (i >> 2) * 16 + lg * 4 + (i & 3); };
+        float y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = (float)rp[0][i];
+        bad = take_nonfinite(y, L, tok);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (tok(i) >= bad) rp[0][i] = rp[1][i] = rp[2][i] = (bf16)0.f;
+#pragma unroll
+        for (int ti = 0; ti < LT; ++ti) {
+          f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+          mm<true, 3, 3>(fw[ti], rp, hi, lo);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[ti * 4 + e] = hi[e] + lo[e];
+        }
+        bad = min(bad, take_nonfinite(x, L, tok));
+      }
       split8<3>(x, up);
     }
+    const bool some_bad = __any(bad < L);
     if (MODE != 1) {
       float* oc = a.out + t0 * os + (int64_t)h * a.dv;
 #pragma unroll
@@ -439,6 +462,9 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           o[ti][e] = __builtin_fmaf(gm[ti][e], o[ti][e] + ol[ti][e], hi[e] + lo[e]);
+        if (some_bad)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[ti][e] = ti * 16 + lg * 4 + e >= bad ? NAN : o[ti][e];
       }
       if (colok) {
         const int at = lg * 4 * ro + col;
@@ -460,6 +486,11 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) S[dt][e] = __builtin_fmaf(S[dt][e], gL, hi[e] + lo[e]);
     }
+    if (some_bad)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[dt][e] = bad < L ? NAN : S[dt][e];
     __syncthreads();
   }
 

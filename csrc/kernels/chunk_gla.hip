@@ -251,20 +251,24 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
     }
     fetch(c0 + L < len ? ci + 1 : ci);       // (the last one again at the end: no branch)
     bf16x8 vp[3];
+    int bad;
     {
       float x[8];
+      auto tok = [&](int i) { return (i >> 2) * 16 + lg * 4 + (i & 3); };
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {          // tokens past the end: k r and A are zero, v may not be finite
-        const int t = (i >> 2) * 16 + lg * 4 + (i & 3);
-        x[i] = t < nl ? to_f(v[i >> 2][i & 3]) : 0.f;
-      }
+      for (int i = 0; i < 8; ++i) x[i] = tok(i) < nl ? to_f(v[i >> 2][i & 3]) : 0.f;
+      bad = take_nonfinite(x, L, tok);
       split8<3>(x, vp);
     }
+    const bool some_bad = __any(bad < L);
     float* oc = a.out + t0 * os + (int64_t)h * a.dv + col;
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti) {
       f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
       mm<true, 3, 3>(fp[ti], vp, hi, lo);
+      if (some_bad)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hi[e] = ti * 16 + lg * 4 + e >= bad ? NAN : hi[e];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int t = ti * 16 + lg * 4 + e;
@@ -282,6 +286,11 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) S[dt][e] = __builtin_fmaf(S[dt][e], pl[dt][e], hi[e] + lo[e]);
     }
+    if (some_bad)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[dt][e] = bad < L ? NAN : S[dt][e];
     __syncthreads();
   }
   if (colok)

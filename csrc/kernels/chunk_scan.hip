@@ -394,13 +394,13 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
     // this chunk's v (B operand: rows 8 lg .. of every 32, the lane's column), in flight while the
     // scores and Q S_0 are computed
     const E* vc = vb + (int64_t)(start + c0) * a.stride;
-    E vr[KL][8];
+    E vr[KL * 8];
 #pragma unroll
     for (int j = 0; j < KL; ++j)
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int s = j * 32 + lg * 8 + i;
-        vr[j][i] = vc[min(s, nl - 1) * rs];
+        vr[j * 8 + i] = vc[min(s, nl - 1) * rs];
       }
     float xr[LT][4];                         // SSD: x of this lane's outputs, for D x
     if (!MLSTM && MODE != 1)
@@ -499,13 +499,16 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
 
     // ---- the rest of this wave's columns --------------------------------------------------
     __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): v is here; what follows need not be
-    if (c0 + L < len) fetch(c0 + L);         // lands while P V and the update run
+    if (MODE == 1 && c0 + L < len) fetch(c0 + L);
     if (nl < L)
 #pragma unroll
       for (int j = 0; j < KL; ++j)
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-          if (j * 32 + lg * 8 + i >= nl) vr[j][i] = (E)0.f;
+          if (j * 32 + lg * 8 + i >= nl) vr[j * 8 + i] = (E)0.f;
+    const int bad = take_nonfinite(vr, L, [&](int i) { return (i >> 3) * 32 + lg * 8 + (i & 7); });
+    const bool some_bad = __any(bad < L);
+    if (MODE != 1 && c0 + L < len) fetch(c0 + L);      // lands while P V and the update run
     if (MODE != 1) {
       if (MLSTM && lane < L) {
         float dsum = nq[lane] * ic[lane];
@@ -527,11 +530,11 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
         bf16x8 vp[NP];
         if constexpr (NP == 1) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) vp[0][i] = vr[j][i];
+          for (int i = 0; i < 8; ++i) vp[0][i] = vr[j * 8 + i];
         } else {
           float x[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) x[i] = (float)vr[j][i];
+          for (int i = 0; i < 8; ++i) x[i] = (float)vr[j * 8 + i];
           split8<NP>(x, vp);
         }
 #pragma unroll
@@ -543,6 +546,11 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
           mm<SEP, 3, NP>(fa, vp, o[ti], ol[ti]);
         }
       }
+      if (some_bad)
+#pragma unroll
+        for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[ti][r] = ti * 16 + lg * 4 + r >= bad ? NAN : o[ti][r];
 #pragma unroll
       for (int ti = 0; ti < LT; ++ti) {
         f32x4 f = {1.f, 1.f, 1.f, 1.f};
@@ -562,7 +570,7 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
     for (int j = 0; j < KL; ++j) {
       float x[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = (float)vr[j][i] * wc[hw * L + j * 32 + lg * 8 + i];
+      for (int i = 0; i < 8; ++i) x[i] = (float)vr[j * 8 + i] * wc[hw * L + j * 32 + lg * 8 + i];
       split8<3>(x, vp[j]);
     }
 #pragma unroll
@@ -586,6 +594,11 @@ __global__ __launch_bounds__(NT) void chunk_scan_kernel(const ChunkArgs a) {
         S[dt][r] = NP > 2 ? __builtin_fmaf(S[dt][r], decay, hi[r] + lo[r]) : hi[r];
       if (dt % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
+    if (some_bad)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[dt][r] = bad < L ? NAN : S[dt][r];
     if (MLSTM) {                             // n <- decay n + sum_t w_t k_t: NT / D threads per row
       constexpr int TPD = NT / D;
       const int c = tid / TPD, sub = tid % TPD;

@@ -673,3 +673,64 @@ def test_gla_scan_chunkwise(gpu, dt, H, V, R, lens, before, D_ctx):
         got = run(st, _to(m, gpu))
         assert ((got.cpu() - want).abs() <= (d + 64) * unit + 1e-30).all()
         assert ((st.cpu() - S).abs() <= 128 * SA + 1e-30).all()
+
+
+@pytest.mark.parametrize("op,dt", [("mlstm", torch.bfloat16), ("mlstm", torch.float16), ("ssd", torch.bfloat16),
+                                   ("delta", torch.bfloat16), ("gla", torch.bfloat16), ("gla", torch.float32)])
+@pytest.mark.parametrize("where,val", [("v", float("nan")), ("v", float("-inf")), ("k", float("nan")), ("gate", float("nan"))])
+@pytest.mark.parametrize("bad", [(0, 20), (0, 44), (1, 0), (1, 333), (1, 698), (2, 32)])
+def test_chunkwise_scans_keep_what_is_not_finite_to_later_rows(gpu, op, dt, where, val, bad):
+    """One value, key channel or gate that is not finite, at tokens inside, at the ends of and alone
+    in a chunk and in a prompt cut into segments: the rows before it, other sequences, and for a
+    value the other columns have the bits of the call without it; it reaches every row from its own
+    on and the state, as token by token."""
+    torch.manual_seed(91)
+    lens = [45, 700, 33]
+    m, T, n = _chunk_step(lens, [3, 0, 7], [])
+    m.state_slots = torch.tensor([2, 0, 1], dtype=torch.int32)
+    mg, d, H, G = _to(m, gpu), 128, 2, 2 if op in ("mlstm", "gla") else 1
+    V = 144
+    a, b = torch.full((H,), -1.0).to(gpu), torch.zeros(H).to(gpu)
+    if op == "mlstm":
+        x, g = torch.randn(T, 2 * H * d + 2 * H * V).to(dt), torch.cat([torch.randn(T, H), -torch.rand(T, H)], dim=1)
+        st = [torch.randn(n, H, d, V), torch.randn(n, H, d), torch.rand(n, H)]
+        koff, voff = H * d, 2 * H * d
+        run = lambda x, g, s: ops.mlstm_scan(x, g, s, mg, H, d, V)   # noqa: E731
+    elif op == "ssd":
+        x, g, st, koff, voff = torch.randn(T, H * V + 2 * G * d), torch.randn(T, H).to(dt), [torch.randn(n, H, d, V)], H * V, 0
+        run = lambda x, g, s: ops.ssd_scan(x, g, a, b, b, s[0], mg, H, V, d, G)   # noqa: E731
+    elif op == "delta":
+        x, g, st = torch.randn(T, 2 * G * d + H * V), torch.randn(T, 2 * H).to(dt), [torch.randn(n, H, d, V)]
+        koff, voff = G * d, 2 * G * d
+        run = lambda x, g, s: ops.gated_delta_scan(x, g, a, b, s[0], mg, H, G, d, V)   # noqa: E731
+    else:
+        R = 3
+        x, g, st = torch.randn(T, 2 * H * d + H * V).to(dt), torch.randn(T, R).to(dt), [torch.randn(n, H, d, V)]
+        koff, voff, a2, ab = H * d, 2 * H * d, torch.randn(H * d, R).to(gpu), torch.ones(H * d).to(gpu)
+        run = lambda x, g, s: ops.gla_scan(x, g, a2, ab, s[0], mg, H, d, V, 4.0)   # noqa: E731
+
+    def both(x, g):
+        s = [y.to(gpu) for y in st]
+        return run(x.to(gpu), g.to(gpu), s).cpu().view(T, H, V), s[0].cpu()
+    want, S_w = both(x, g)
+    assert want.isfinite().all() and S_w.isfinite().all()
+    seq, tok = bad
+    t, end, h, c = sum(lens[:seq]) + tok, sum(lens[:seq + 1]), H - 1, 77
+    if where == "v":
+        x[t, voff + h * V + c] = val
+    elif where == "k":
+        x[t, koff + (h if G == H else 0) * d + 100] = val
+    else:
+        g[t, h if op != "gla" else 0] = val
+    got, S = both(x, g)
+    hit = torch.zeros(T, H, V, dtype=torch.bool)
+    heads = slice(h, h + 1) if where == "v" or (where == "k" and G == H) or (where == "gate" and op != "gla") else slice(0, H)
+    hit[t:end, heads, slice(c, c + 1) if where == "v" else slice(0, V)] = True
+    assert not got[hit].isfinite().any() and torch.equal(got[~hit], want[~hit])
+    hit = torch.zeros(n, H, d, V, dtype=torch.bool)
+    slot = int(m.state_slots[seq])
+    if where == "k" and op in ("mlstm", "ssd", "gla"):      # only the channel's row of the state
+        hit[slot, heads, 100] = True
+    else:
+        hit[slot, heads, :, slice(c, c + 1) if where == "v" else slice(0, V)] = True
+    assert not S[hit].isfinite().any() and torch.equal(S[~hit], S_w[~hit])
