@@ -20,6 +20,7 @@
 //   K   [64 keys][D]   chunk c of key k stored at c ^ f(k), f(k) = (k&3)|((k>>3)&3)<<2
 //   V^T [D][64 keys]   chunk c of dim d stored at c ^ ((d>>1)&7)
 #include "common.h"
+#include "device.h"
 #include "launch.h"
 #include <algorithm>
 #include <cstdlib>
@@ -844,25 +845,18 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
   constexpr size_t lds = 2 * 2 * PF_BN * D * sizeof(T);
   const int G = nq / nkv;
   const int64_t n_items = (int64_t)n_work * nkv * (G / GH) * (PF_BM / (256 / GH));
-  static const int n_cu = [] {
-    int dev = 0, cu = 256;
-    if (hipGetDevice(&dev) == hipSuccess)
-      hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev);
-    return cu > 0 ? cu : 256;
-  }();
+  const int n_cu = device_cus();
   // The walk pays with more items than CUs (32 x 512 rows, 32 heads: 179 us against 202); with one item
   // per CU or less, twice as many workgroups of half the rows do (8 x 100 rows after 3000: 115 against
   // 137, 512 rows alone 28 against 31, 2000 after 2000 168 against 179).
   const int mode = prefill_persist_mode();
   const bool dma = reinterpret_cast<uintptr_t>(q) % 16 == 0 && q_stride % 8 == 0;    // 16-byte DMAs
-  if (dma && (mode < 0 ? n_items > n_cu : mode != 0) && n_items < ((int64_t)1 << 30)) {
-    // one workgroup per CU: launch_bounds(512, 1), 128 KB of LDS (K / V tiles, the waves' q / output rows)
-    constexpr size_t lds_q = lds + 256 * D * sizeof(T);
-    static const hipError_t big = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&prefill_attn_gqa_persist_kernel<T, D, KV8, GH>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_q);
-    (void)big;
-    prefill_attn_gqa_persist_kernel<T, D, KV8, GH><<<(int)std::min<int64_t>(n_items, n_cu), 512, lds_q, s>>>(
+  // one workgroup per CU: launch_bounds(512, 1), 128 KB of LDS (K / V tiles, the waves' q / output rows)
+  constexpr size_t lds_q = lds + 256 * D * sizeof(T);
+  const auto walk = &prefill_attn_gqa_persist_kernel<T, D, KV8, GH>;
+  static OncePerDevice once;
+  if (dma && (mode < 0 ? n_items > n_cu : mode != 0) && n_items < ((int64_t)1 << 30) && allow_lds(once, walk, lds_q)) {
+    walk<<<(int)std::min<int64_t>(n_items, n_cu), 512, lds_q, s>>>(
         (const T*)q, (T*)out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, nq, nkv, bs_log2,
         scale_log2, v_scale, num_blocks, q_stride, cos_sin, cs_rows, (int)n_items);
     return;

@@ -21,6 +21,7 @@
 // walks every segment from zero (with its values) and from the identity (without), a second chains
 // S <- M_j S + dS_j over the segments, and the third walks all segments from their own states.
 #include "chunk.h"
+#include "device.h"
 #include "launch.h"
 
 namespace kgc {
@@ -580,7 +581,7 @@ DeltaWork delta_chunk_plan(int P, int Tp, int H, int G, int V) {
   const int chunks = Tp / L + P, wgs = H * ((V + 127) / 128);
   w.wp = (int64_t)chunks * H * 2 * MAT;
   w.floats = (int64_t)chunks * L * (3 * H + 2 * G);
-  const int want = (256 + wgs - 1) / wgs;    // items for one workgroup per CU
+  const int want = (device_cus() + wgs - 1) / wgs;      // items for one workgroup per CU
   if (P * 3 > want) return w;
   int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
   seg = (seg + L - 1) / L * L;

@@ -33,6 +33,7 @@
 // so it takes the states they held from copies (as n and m): the first launch's workgroups of a
 // sequence's last segment, whose contribution nobody needs, put S in that segment's place.
 #include "chunk.h"
+#include "device.h"
 #include "launch.h"
 
 namespace kgc {
@@ -658,17 +659,22 @@ constexpr size_t chunk_lds() {
 }
 
 template <typename E, bool MLSTM, int D, int L, int HPW, int MODE>
+bool chunk_allowed() {
+  static OncePerDevice once;
+  return allow_lds(once, &chunk_scan_kernel<E, MLSTM, D, L, HPW, MODE>, chunk_lds<E, D, L, HPW>());
+}
+// the current device takes all launches of the form
+template <typename E, bool MLSTM, int D, int L, int HPW>
+bool chunk_form_ok() {
+  return chunk_allowed<E, MLSTM, D, L, HPW, 0>() && chunk_allowed<E, MLSTM, D, L, HPW, 1>() &&
+         chunk_allowed<E, MLSTM, D, L, HPW, 2>();
+}
+
+template <typename E, bool MLSTM, int D, int L, int HPW, int MODE>
 void chunk_run(const ChunkArgs& a, int items, hipStream_t s) {
   const int nct = (a.dv + 16 * (NW / HPW) - 1) / (16 * (NW / HPW));
-  constexpr size_t lds = chunk_lds<E, D, L, HPW>();
-  static const bool big = [] {
-    return hipFuncSetAttribute(
-               reinterpret_cast<const void*>(&chunk_scan_kernel<E, MLSTM, D, L, HPW, MODE>),
-               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-  }();
-  (void)big;
   chunk_scan_kernel<E, MLSTM, D, L, HPW, MODE>
-      <<<dim3(items, a.H / HPW * nct), NT, lds, s>>>(a);
+      <<<dim3(items, a.H / HPW * nct), NT, chunk_lds<E, D, L, HPW>(), s>>>(a);
 }
 
 template <typename E, bool MLSTM, int D, int L, int HPW>
@@ -688,9 +694,9 @@ void chunk_dispatch(const ChunkArgs& a, int items, hipStream_t s) {
 static ChunkWork chunk_plan(int P, int Tp, int wgs, int L) {
   ChunkWork p;
   p.items = P;
-  // 256 CUs hold one of these workgroups each; cut only where a good part of them would idle
+  // a CU holds one of these workgroups; cut only where a good part of the CUs would idle
   // and the pieces are long enough to pay for computing every contribution twice
-  const int want = (256 + wgs - 1) / wgs;
+  const int want = (device_cus() + wgs - 1) / wgs;
   if (P * 2 > want) return p;
   int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
   seg = (seg + L - 1) / L * L;
@@ -705,8 +711,11 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L) {
 // three parts do not fit LDS).  32 x 512 tokens, 4 heads of 256 x 512: 1957 us token by token, 219 us
 // chunkwise, and nearer to float64 (3.5e-7 against 4.7e-7).
 bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, int H, int d, int dv) {
-  return (dtype == DT_BF16 || dtype == DT_F16) && P > 0 && Tp >= 16 * P && (d == 128 || d == 256) &&
-         stride % 8 == 0 && (reinterpret_cast<uintptr_t>(qkvg) & 15) == 0 && dv >= 16;
+  if (!((dtype == DT_BF16 || dtype == DT_F16) && P > 0 && Tp >= 16 * P && (d == 128 || d == 256) &&
+        stride % 8 == 0 && (reinterpret_cast<uintptr_t>(qkvg) & 15) == 0 && dv >= 16))
+    return false;
+  if (dtype == DT_BF16) return d == 128 ? chunk_form_ok<bf16, true, 128, 64, 1>() : chunk_form_ok<bf16, true, 256, 64, 1>();
+  return d == 128 ? chunk_form_ok<f16, true, 128, 32, 1>() : chunk_form_ok<f16, true, 256, 32, 1>();
 }
 
 ChunkWork mlstm_chunk_plan(int dtype, int P, int Tp, int H, int d, int dv) {
@@ -742,12 +751,13 @@ void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride,
 // to 64 columns share a workgroup's B and C.  2 x 8192 tokens, 32 heads of 128 x 64: 4821 us token by
 // token (a chain of 8192 steps in 64 workgroups), 353 us in chunks and segments of 1184; from float64
 // 7.0e-8 (7.3e-8).  Half of that time is vector work, most of it the splits of S, B and C.
+static int ssd_heads(int H, int V, int G) { return V <= 64 && (H / G) % 2 == 0 ? 2 : 1; }
+
 bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G) {
   return P > 0 && Tp >= 16 * P && N == 128 && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
-         (reinterpret_cast<uintptr_t>(xbc) & 15) == 0;
+         (reinterpret_cast<uintptr_t>(xbc) & 15) == 0 &&
+         (ssd_heads(H, V, G) == 2 ? chunk_form_ok<float, false, 128, 32, 2>() : chunk_form_ok<float, false, 128, 32, 1>());
 }
-
-static int ssd_heads(int H, int V, int G) { return V <= 64 && (H / G) % 2 == 0 ? 2 : 1; }
 
 ChunkWork ssd_chunk_plan(int P, int Tp, int H, int V, int G) {
   const int hpw = ssd_heads(H, V, G), cols = 16 * (NW / hpw);

@@ -18,6 +18,7 @@
 // What bounds it: the MFMAs (two thirds of them the pairs of P V; at 8 x 2048 rows, window 1024, they
 // alone are 110 us of the 229 at a large product's rate) and the softmax's vector work (80 us), which
 // overlap in part.  Not the loads: a ring of four tiles filled by LDS-DMA three tiles ahead took 249 us.
+#include "device.h"
 #include "window.h"
 #include <type_traits>
 
@@ -353,28 +354,26 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
 }
 
 template <typename T, int KS, int DT, int NJ, bool ALIAS, bool CAP>
-void run(T* out, const T* q, const T* kc, const T* vc, const int* qsl, const int* seq_lens, const int* pbt,
+bool run(T* out, const T* q, const T* kc, const T* vc, const int* qsl, const int* seq_lens, const int* pbt,
          int bt_stride, const int* work_seq, const int* work_blk, int n_work, int blk_rows, int H, int G,
          int krs, int vrs, int bs, int num_blocks, float scale, int window, int keep_first, const float* gate,
          const WindowExtra& ex, hipStream_t s) {
   constexpr size_t lds = sizeof(T) * 2 * BN * (KS * 32 + 8 + (ALIAS ? 0 : DT * 16 + 8));
-  static const bool set = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&window_prefill_gqa_kernel<T, KS, DT, NJ, ALIAS, CAP>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-  (void)set;
+  const auto kernel = &window_prefill_gqa_kernel<T, KS, DT, NJ, ALIAS, CAP>;
+  static OncePerDevice once;
+  if (!allow_lds(once, kernel, lds)) return false;
   const int shift = (bs & (bs - 1)) == 0 ? __builtin_ctz(bs) : -1;
-  window_prefill_gqa_kernel<T, KS, DT, NJ, ALIAS, CAP>
-      <<<dim3(H / HW, n_work * (blk_rows / BM)), NT, lds, s>>>(
-          out, q, kc, vc, qsl, seq_lens, pbt, bt_stride, work_seq, work_blk, blk_rows, H, G, krs, vrs, bs,
-          shift, num_blocks, scale, window, keep_first, gate, ex);
+  kernel<<<dim3(H / HW, n_work * (blk_rows / BM)), NT, lds, s>>>(
+      out, q, kc, vc, qsl, seq_lens, pbt, bt_stride, work_seq, work_blk, blk_rows, H, G, krs, vrs, bs, shift,
+      num_blocks, scale, window, keep_first, gate, ex);
+  return true;
 }
 
 template <typename T, bool CAP, typename... A>
 bool dispatch(int dk, int dv, bool alias, T* out, const T* q, const T* kc, const T* vc, A... a) {
-  if (dk == 128 && dv == 128 && !alias) run<T, 4, 8, 4, false, CAP>(out, q, kc, vc, a...);
-  else if (dk == 256 && dv == 192 && alias) run<T, 8, 12, 2, true, CAP>(out, q, kc, vc, a...);
-  else return false;
-  return true;
+  if (dk == 128 && dv == 128 && !alias) return run<T, 4, 8, 4, false, CAP>(out, q, kc, vc, a...);
+  if (dk == 256 && dv == 192 && alias) return run<T, 8, 12, 2, true, CAP>(out, q, kc, vc, a...);
+  return false;
 }
 
 }  // namespace
