@@ -21,6 +21,7 @@
 // walks every segment from zero (with its values) and from the identity (without), a second chains
 // S <- M_j S + dS_j over the segments, and the third walks all segments from their own states.
 #include "chunk.h"
+#include "chunk_rows.h"
 #include "device.h"
 #include "launch.h"
 
@@ -565,13 +566,12 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
 
 }  // namespace
 
-// Chunkwise for 128 key channels, from 24 rows per sequence on or a thousand in all (16 rows of one
-// sequence: 19 us token by token, 32 us here; 48 rows: 43 and 37 us; 64 x 20 rows: 101 and 69 us).
-// 16 x 1000 tokens of 16 heads with 128 x 128 states: 1328 us token by token, 288 us chunkwise (71 us
-// for W and P); 2 x 8192: 7.5 ms and 0.9 ms.  The walk issues 1000 vector instructions and 168 MFMAs
-// per wave and chunk, 13 k of its 15 k cycles.
+// Chunkwise for 128 key channels where the rows pay (chunk_rows.h; a chunk's workspace is 200 KB for 16
+// heads, which few rows per sequence would multiply, too).  16 x 1000 tokens of 16 heads with 128 x 128
+// states: 1328 us token by token, 292 us chunkwise (71 us for W and P); 2 x 8192: 7.5 ms and 0.9 ms.  The
+// walk issues 1000 vector instructions and 168 MFMAs per wave and chunk.
 bool delta_chunk_ok(const float* qkv, int P, int Tp, int H, int G, int d, int V) {
-  return P > 0 && (Tp >= 24 * P || Tp >= 1024) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
+  return chunk_rows_pay(P, Tp, 48) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(qkv) & 15) == 0;
 }
 

@@ -18,6 +18,7 @@
 // (splitting S and reading those 140 MB); 2 x 8192 8214 -> 1502 (one walk per sequence, not cut into
 // segments).  From float64: 1.1e-6 -> 1.0e-6.
 #include "chunk.h"
+#include "chunk_rows.h"
 #include "launch.h"
 
 namespace kgc {
@@ -309,8 +310,8 @@ void run(const GlaArgs& a, int chunks, hipStream_t s) {
 }  // namespace
 
 bool gla_chunk_ok(int P, int Tp, int H, int d, int V, int R) {
-  // chunks that are mostly full: 1 x 48 tokens 46 -> 35 us, 64 x 48 218 -> 120, 4 x 60 63 -> 42
-  return P > 0 && (Tp >= 24 * P || Tp >= 1024) && d == D && V >= 16 && R <= RMAX &&
+  // 1 x 48 tokens 46 -> 35 us, 64 x 48 218 -> 120, 4 x 60 63 -> 42; fewer rows: chunk_rows.h
+  return chunk_rows_pay(P, Tp, 32) && d == D && V >= 16 && R <= RMAX &&
          (int64_t)H * ((V + 127) / 128) <= 65535;
 }
 // floats of workspace

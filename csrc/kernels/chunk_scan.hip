@@ -747,14 +747,16 @@ void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride,
   }
 }
 
-// Mamba-2: 128 state rows, fp32 x | B | C (three bf16 parts each), 32-token chunks; two heads of up
-// to 64 columns share a workgroup's B and C.  2 x 8192 tokens, 32 heads of 128 x 64: 4821 us token by
-// token (a chain of 8192 steps in 64 workgroups), 353 us in chunks and segments of 1184; from float64
-// 7.0e-8 (7.3e-8).  Half of that time is vector work, most of it the splits of S, B and C.
+// heads per workgroup
 static int ssd_heads(int H, int V, int G) { return V <= 64 && (H / G) % 2 == 0 ? 2 : 1; }
 
+// Mamba-2: 128 state rows, fp32 x | B | C (three bf16 parts each), 32-token chunks; two heads of up
+// to 64 columns share a workgroup's B and C.  16 rows alone stay token by token (9.9 us against 10.3;
+// 4 x 18: 12.8 and 10.9).  2 x 8192 tokens, 32 heads of 128 x 64: 4821 us token by
+// token (a chain of 8192 steps in 64 workgroups), 353 us in chunks and segments of 1184; from float64
+// 7.0e-8 (7.3e-8).  Half of that time is vector work, most of it the splits of S, B and C.
 bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G) {
-  return P > 0 && Tp >= 16 * P && N == 128 && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
+  return P > 0 && Tp >= 16 * P && Tp >= 20 && N == 128 && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(xbc) & 15) == 0 &&
          (ssd_heads(H, V, G) == 2 ? chunk_form_ok<float, false, 128, 32, 2>() : chunk_form_ok<float, false, 128, 32, 1>());
 }

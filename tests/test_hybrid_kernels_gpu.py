@@ -215,9 +215,10 @@ def _mlstm64(qkvg, gates, st, m, H, d, dv):
 
 
 # (chunk lengths, tokens before them): around the chunk (32 / 64 tokens) and tile (16) edges, a
-# padding sequence, decode rows behind the chunks, and long chunks that are cut into segments
+# padding sequence, decode rows behind the chunks, long chunks that are cut into segments, and
+# one and two rows among longer chunks
 CHUNKS = [([1, 15, 16, 17, 31, 33], [0, 5, 0, 40, 0, 0], [9, 1]), ([63, 64, 65, 129], [0, 7, 0, 0], []),
-          ([700], [0], []), ([33, 1300], [3, 11], [30])]
+          ([700], [0], []), ([33, 1300], [3, 11], [30]), ([1, 96, 2, 90, 31, 5], [0, 3, 9, 0, 0, 1], [4])]
 
 
 def _chunk_step(lens, before, D_ctx):

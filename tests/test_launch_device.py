@@ -1,4 +1,5 @@
-"""csrc/kernels/device.h: what launches ask of and set on a device, compiled against a fake runtime."""
+"""Host rules of the kernels' launchers, compiled against a fake runtime: what they ask of and set on a
+device (csrc/kernels/device.h), and which prompt rows go chunkwise (csrc/kernels/chunk_rows.h)."""
 import os
 import subprocess
 
@@ -44,12 +45,43 @@ int main() {
 }
 """
 
+RULE = """
+#include <initializer_list>
+#include "chunk_rows.h"
+using kgc::chunk_rows_pay;
+#define CHECK(x) if (!(x)) return __LINE__
+int main() {
+  for (long alone : {32, 48}) {
+    CHECK(!chunk_rows_pay(0, 0, alone) && !chunk_rows_pay(1, 24, alone) && chunk_rows_pay(1, alone, alone));
+    for (long P = 1; P <= 1024; ++P) {
+      CHECK(!chunk_rows_pay(P, 8 * P, alone) && !chunk_rows_pay(P, P, alone) && chunk_rows_pay(P, 48 * P, alone));
+      for (long n = 1, was = 0; n <= 64; ++n) {    // longer rows never go back
+        const bool now = chunk_rows_pay(P, n * P, alone);
+        CHECK(now >= was);
+        was = now;
+      }
+    }
+    CHECK(chunk_rows_pay(128, 128 * 12, alone) && !chunk_rows_pay(32, 32 * 12, alone) && chunk_rows_pay(32, 512, alone));
+  }
+  return 0;
+}
+"""
 
-def test_devices_are_asked_one_by_one(tmp_path):
+
+def _run(tmp_path, program):
     os.mkdir(tmp_path / "hip")
     (tmp_path / "hip" / "hip_runtime.h").write_text(RUNTIME)
-    (tmp_path / "main.cpp").write_text(PROGRAM)
+    (tmp_path / "main.cpp").write_text(program)
     exe = str(tmp_path / "main")
     subprocess.run(["g++", "-std=c++17", "-I", str(tmp_path), "-I", os.path.join(ROOT, "csrc", "kernels"),
                     str(tmp_path / "main.cpp"), "-o", exe], check=True)
     assert subprocess.run([exe]).returncode == 0
+
+
+def test_devices_are_asked_one_by_one(tmp_path):
+    _run(tmp_path, PROGRAM)
+
+
+def test_short_rows_stay_token_by_token(tmp_path):
+    """Hundreds of chunks of one to eight rows used to go chunkwise from 1024 rows on."""
+    _run(tmp_path, RULE)
