@@ -219,13 +219,8 @@ class ModelRunner:
         torch.cuda.reset_peak_memory_stats()
         base = torch.cuda.memory_allocated()
         self.init_kv_cache(16)
-        seqs = []
-        remaining = self.token_budget
-        while remaining > 0:
-            q = min(remaining, self.max_model_len)
-            seqs.append(q)
-            remaining -= q
-        self._dummy_prefill(seqs)
+        for qlens in self._profile_steps():
+            self._dummy_prefill(qlens)
         torch.cuda.synchronize()
         peak = torch.cuda.max_memory_allocated() - base
         self.kv = None
@@ -238,6 +233,20 @@ class ModelRunner:
         budget = total * gpu_mem_util - used_now - peak - reserve_graphs - self.state_bytes()
         nb = int(budget // self.kv_bytes_per_block())
         return max(nb, 2)
+
+    def _profile_steps(self) -> list[list[int]]:
+        """Prompt steps with the largest activations: the token budget in prompts as long as
+        they get, and for recurrent layers in as many as there are slots, too -- the chunkwise
+        scans keep a workspace per started chunk of every sequence, from 12 rows of each on (24
+        in small steps; csrc/kernels/chunk_rows.h)."""
+        long, remaining = [], self.token_budget
+        while remaining > 0:
+            long.append(min(remaining, self.max_model_len))
+            remaining -= long[-1]
+        n = min(self.max_num_seqs, self.token_budget // (12 if self.token_budget >= 1024 else 24))
+        if not self.state_layout or n <= len(long):
+            return [long]
+        return [long, [min(self.token_budget // n, self.max_model_len)] * n]
 
     def release(self) -> None:
         """Drop the KV arena, decode graphs and workspaces (engine shutdown): a process

@@ -417,3 +417,20 @@ def test_step_plan_header_carries_the_tp_overlap_split():
     assert len(h) == N_HDR and h[-1] == 1
     q = StepPlan(*h, z, z, z)
     assert q.split == 1 and q.vp == 1 and q.T == 40
+
+
+def test_memory_profile_covers_many_short_prompts():
+    """The step that sizes the KV pool: the longest prompts, and for recurrent layers (whose
+    chunkwise scans keep a workspace per sequence and started chunk) as many prompts as there
+    are slots and go chunkwise; never more rows or sequences than a step can have."""
+    from types import SimpleNamespace
+
+    from kubernetes_gpu_cluster_amd.engine.model_runner import ModelRunner
+    steps = lambda budget, longest, seqs, layout: ModelRunner._profile_steps(SimpleNamespace(   # noqa: E731
+        token_budget=budget, max_model_len=longest, max_num_seqs=seqs, state_layout=layout))
+    assert steps(16384, 8192, 256, []) == [[8192, 8192]]
+    assert steps(16384, 8192, 256, [()]) == [[8192, 8192], [64] * 256]
+    assert steps(16384, 8192, 2048, [()])[1] == [12] * 1365
+    assert steps(512, 8192, 256, [()])[1] == [24] * 21
+    assert steps(5000, 2048, 256, [()])[0] == [2048, 2048, 904]
+    assert steps(4096, 100, 256, [()])[1] == [16] * 256 and steps(2048, 8192, 1, [()]) == [[2048]]
