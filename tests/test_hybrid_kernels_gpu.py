@@ -221,6 +221,13 @@ CHUNKS = [([1, 15, 16, 17, 31, 33], [0, 5, 0, 40, 0, 0], [9, 1]), ([63, 64, 65, 
           ([700], [0], []), ([33, 1300], [3, 11], [30]), ([1, 96, 2, 90, 31, 5], [0, 3, 9, 0, 0, 1], [4])]
 
 
+def _whole(got, want):
+    """All 24 bits of every operand reach the result: the norm of the difference within 5e-7 of the
+    result's, four times what three bf16 parts per operand show (an operand of two parts is off by
+    2.4e-6, which bounds on single elements let pass: its errors average out in their sums)."""
+    return float((got.double().cpu() - want).norm()) <= 5e-7 * float(want.norm())
+
+
 def _chunk_step(lens, before, D_ctx):
     n = len(lens) + len(D_ctx)
     slots = list(range(n))[::-1]
@@ -248,6 +255,7 @@ def test_mlstm_scan_chunkwise(gpu, dt, H, d, dv, lens, before, D_ctx):
     want, unit, st_w, st_u = _mlstm64(qkvg, gates, st, m, H, d, dv)
     got = ops.mlstm_scan(qkvg.to(gpu), gates.to(gpu), st_g, _to(m, gpu), H, d, dv)
     assert ((got.double().cpu() - want).abs() <= 16 * unit).all()
+    assert _whole(st_g[0], st_w[0])         # (outputs: the denominators' cancellation is in `unit`)
     for a, b, u in zip(st_g, st_w, st_u):
         assert ((a.double().cpu() - b).abs() <= 16 * 2.0 ** -24 * u).all()
 
@@ -313,6 +321,7 @@ def test_ssd_scan_chunkwise(gpu, dt, H, G, V, lens, before, D_ctx):
                        H, V, N, G)
     assert ((got.double().cpu() - want - add).abs() <= 16 * (unit + add.abs() * 2.0 ** -24)).all()
     assert ((S_g.double().cpu() - S_w).abs() <= 16 * S_u).all()
+    assert _whole(got, want + add) and _whole(S_g, S_w)
 
 
 @pytest.mark.parametrize("op,dt", [("mlstm", torch.bfloat16), ("mlstm", torch.float16), ("ssd", torch.bfloat16)])
@@ -379,6 +388,7 @@ def test_gated_delta_scan_chunkwise(gpu, dt, H, G, V, lens, before, D_ctx):
     got = ops.gated_delta_scan(qkv.to(gpu), ba.to(gpu), a_log.to(gpu), dtb.to(gpu), S_g, _to(m, gpu), H, G, d, V)
     assert ((got.double().cpu() - want).abs() <= 32 * bound).all()
     assert ((S_g.double().cpu() - S_w).abs() <= 32 * S_u).all()
+    assert _whole(got, want) and _whole(S_g, S_w)
 
 
 @pytest.mark.parametrize("path", ["fast", "simple"])
@@ -662,18 +672,20 @@ def test_window_decode_many_waves(gpu, dt, H, G, rows, kw):
 def test_gla_scan_chunkwise(gpu, dt, H, V, R, lens, before, D_ctx):
     """Prompt rows in chunks of 32 (and decode rows behind them): ends inside a chunk, continued and
     fresh states, a padding sequence, value columns off a wave's 16 and a workgroup's 128; decays from
-    next to nothing to all but zero.  Products of up to 32 decays (R + 1 terms over tau each) and
+    none at all to all but zero.  Products of up to 32 decays (R + 1 terms over tau each) and
     sums of d + 32 terms, in units of 2^-24 of the sums of absolute values."""
     torch.manual_seed(81)
     d, tau = 128, 4.0
     m, T, n = _chunk_step(lens, before, D_ctx)
-    for open_ in (3.0, -12.0):
+    for open_ in (3.0, -12.0, 100.0):
         terms, run = _gla_case(T, n, H, d, V, R, dt, tau, gpu, open_)
         want, unit, S, SA = _matrix64(m, *terms)
         st = terms[0].to(gpu)
         got = run(st, _to(m, gpu))
         assert ((got.cpu() - want).abs() <= (d + 64) * unit + 1e-30).all()
         assert ((st.cpu() - S).abs() <= 128 * SA + 1e-30).all()
+        if open_ == 100.0:                  # every decay is 1: no error of theirs
+            assert _whole(got, want) and _whole(st, S)
 
 
 @pytest.mark.parametrize("op,dt", [("mlstm", torch.bfloat16), ("mlstm", torch.float16), ("ssd", torch.bfloat16),
