@@ -572,7 +572,8 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
 // walk issues 1000 vector instructions and 168 MFMAs per wave and chunk.
 bool delta_chunk_ok(const float* qkv, int P, int Tp, int H, int G, int d, int V) {
   return chunk_rows_pay(P, Tp, 48) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
-         (reinterpret_cast<uintptr_t>(qkv) & 15) == 0;
+         (reinterpret_cast<uintptr_t>(qkv) & 15) == 0 &&
+         chunk_fits(2L * G * D + (long)H * V, (long)H * V, (long)H * ((V + 127) / 128 + 1));
 }
 
 DeltaWork delta_chunk_plan(int P, int Tp, int H, int G, int V) {

@@ -312,7 +312,7 @@ void run(const GlaArgs& a, int chunks, hipStream_t s) {
 bool gla_chunk_ok(int P, int Tp, int H, int d, int V, int R) {
   // 1 x 48 tokens 46 -> 35 us, 64 x 48 218 -> 120, 4 x 60 63 -> 42; fewer rows: chunk_rows.h
   return chunk_rows_pay(P, Tp, 32) && d == D && V >= 16 && R <= RMAX &&
-         (int64_t)H * ((V + 127) / 128) <= 65535;
+         chunk_fits(0, (long)H * V, (long)H * ((V + 127) / 128));   // (row offsets have 64 bits)
 }
 // floats of workspace
 int64_t gla_chunk_ws(int P, int Tp, int H) {

@@ -1,7 +1,15 @@
-// Host side: whether prompt rows are worth a chunkwise scan that prepares whole chunks of 32 tokens.
+// Host side: whether prompt rows are worth a chunkwise scan that prepares whole chunks of 32 tokens, and
+// whether it can address them.
 #pragma once
 
 namespace kgc {
+
+// The walks hold offsets inside a chunk (64 rows of `stride` elements, some as 24-bit products) and inside
+// a head's state (256 rows of at most `cols` columns, all heads' together) in 32 bits, and put `blocks`
+// workgroups on a grid's second axis.  Larger calls stay token by token, where offsets have 64 bits.
+inline bool chunk_fits(long stride, long cols, long blocks) {
+  return stride < (1 << 22) && cols < 1000000 && blocks <= 65535;
+}
 
 // P sequences of Tp rows together; `alone`: rows from which one sequence by itself pays.  Token by token
 // a step costs its longest sequence and, once the chip is full, its rows; chunkwise it costs its chunks,

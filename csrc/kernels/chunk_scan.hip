@@ -33,6 +33,7 @@
 // so it takes the states they held from copies (as n and m): the first launch's workgroups of a
 // sequence's last segment, whose contribution nobody needs, put S in that segment's place.
 #include "chunk.h"
+#include "chunk_rows.h"
 #include "device.h"
 #include "launch.h"
 
@@ -712,7 +713,8 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L) {
 // chunkwise, and nearer to float64 (3.5e-7 against 4.7e-7).
 bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, int H, int d, int dv) {
   if (!((dtype == DT_BF16 || dtype == DT_F16) && P > 0 && Tp >= 16 * P && (d == 128 || d == 256) &&
-        stride % 8 == 0 && (reinterpret_cast<uintptr_t>(qkvg) & 15) == 0 && dv >= 16))
+        stride % 8 == 0 && (reinterpret_cast<uintptr_t>(qkvg) & 15) == 0 && dv >= 16 &&
+        chunk_fits(stride, (long)H * dv, (long)H * ((dv + 127) / 128))))
     return false;
   if (dtype == DT_BF16) return d == 128 ? chunk_form_ok<bf16, true, 128, 64, 1>() : chunk_form_ok<bf16, true, 256, 64, 1>();
   return d == 128 ? chunk_form_ok<f16, true, 128, 32, 1>() : chunk_form_ok<f16, true, 256, 32, 1>();
@@ -758,6 +760,7 @@ static int ssd_heads(int H, int V, int G) { return V <= 64 && (H / G) % 2 == 0 ?
 bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G) {
   return P > 0 && Tp >= 16 * P && Tp >= 20 && N == 128 && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(xbc) & 15) == 0 &&
+         chunk_fits((long)H * V + 2L * G * N, (long)H * V, (long)H * ((V + 127) / 128)) &&
          (ssd_heads(H, V, G) == 2 ? chunk_form_ok<float, false, 128, 32, 2>() : chunk_form_ok<float, false, 128, 32, 1>());
 }
 

@@ -85,3 +85,24 @@ def test_devices_are_asked_one_by_one(tmp_path):
 def test_short_rows_stay_token_by_token(tmp_path):
     """Hundreds of chunks of one to eight rows used to go chunkwise from 1024 rows on."""
     _run(tmp_path, RULE)
+
+
+def test_chunk_offsets_fit_their_types(tmp_path):
+    """A row stride of 2^25 elements (a view of a wide buffer) overflowed the offset of the chunk's last
+    row, and so many heads the grid: both stay token by token."""
+    _run(tmp_path, """
+#include <cstdint>
+#include "chunk_rows.h"
+using kgc::chunk_fits;
+#define CHECK(x) if (!(x)) return __LINE__
+int main() {
+  CHECK(chunk_fits(2 * 65536 + 3 * 131072, 131072, 1024));                     // far beyond any model
+  CHECK(!chunk_fits(1L << 25, 2048, 16) && !chunk_fits(1L << 40, 2048, 16));
+  CHECK(!chunk_fits(4096, 2048, 65536) && !chunk_fits(4096, 1L << 23, 16));
+  for (long x = 1; x < (1L << 40); x += x / 3 + 1) {     // what is taken stays inside its type
+    if (chunk_fits(x, 16, 1)) CHECK(63 * x + 256 <= INT32_MAX && x < (1 << 23));
+    if (chunk_fits(16, x, 1)) CHECK(255 * x + x <= INT32_MAX && 63 * x <= INT32_MAX && (x + 15) / 16 <= 65535);
+  }
+  return 0;
+}
+""")
