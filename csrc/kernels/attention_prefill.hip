@@ -543,12 +543,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_gqa_kernel(
 // bit-identical).  Why: at short prompts every workgroup of the one-shot grid paid its own
 // pipeline fill -- the work_seq -> qsl / seq_lens -> block table -> K / V chain of dependent
 // loads, the q load and the first LDS store, ~10 us -- against 1-8 tiles of ~2.5 us of
-// work each (32 x 512 causal, 32 heads: 202 us one-shot).  What an item still costs beside its tiles
+// work each.  What an item still costs beside its tiles
 // are its q and output rows: q comes by DMA while the item before it computes, outputs leave as whole
-// 256-byte rows (191 -> 168 us; 64 x 256 151 -> 126, 2 x 8192 1447 -> 1389).  The 32 x 512 floor is
-// 80 us of tiles and 60 us of bytes, which all CUs reach at the same time.  Rotating the rows in LDS
+// 256-byte rows (32 x 512 181 -> 162 us, 64 x 256 146 -> 126, 2 x 8192 1309 -> 1276).  At 32 x 512 vector
+// instructions issue in 47 % of a SIMD's cycles, its matrix core works in 20 %; 300 MB of rows, 60 us at the
+// rate of a copy, are what all CUs ask for at the same time.  Rotating the rows in LDS
 // with each cos / sin row read once, and a stream of tiles without any wait before an item's compute,
-// measured within 3 % of this and slower on long prompts (2 x 8192: 1540).
+// measured within 3 % of this and a tenth slower on long prompts.
 template <typename T, int D, bool KV8, int GH>
 __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
     const T* __restrict__ q, T* __restrict__ out, const void* __restrict__ kc_,
@@ -846,9 +847,9 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
   const int G = nq / nkv;
   const int64_t n_items = (int64_t)n_work * nkv * (G / GH) * (PF_BM / (256 / GH));
   const int n_cu = device_cus();
-  // The walk pays with more items than CUs (32 x 512 rows, 32 heads: 179 us against 202); with one item
-  // per CU or less, twice as many workgroups of half the rows do (8 x 100 rows after 3000: 115 against
-  // 137, 512 rows alone 28 against 31, 2000 after 2000 168 against 179).
+  // The walk pays with more items than CUs (32 x 512 rows, 32 heads: 162 us against 185); with one item
+  // per CU or less, twice as many workgroups of half the rows do (8 x 100 rows after 3000: 119 against
+  // 128, 512 rows alone 26 against 28, 2000 after 2000 159 against 161).
   const int mode = prefill_persist_mode();
   const bool dma = reinterpret_cast<uintptr_t>(q) % 16 == 0 && q_stride % 8 == 0;    // 16-byte DMAs
   // one workgroup per CU: launch_bounds(512, 1), 128 KB of LDS (K / V tiles, the waves' q / output rows)

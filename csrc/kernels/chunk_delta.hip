@@ -1,4 +1,5 @@
-// Chunkwise gated delta rule of prompt rows on the matrix cores.  Per (sequence, head), with unit
+// Chunkwise gated delta rule (Yang, Kautz and Hatamizadeh, gated delta networks, 2024) of prompt rows on the
+// matrix cores.  Per (sequence, head), with unit
 // keys k_t, a decay g_t and a write strength beta_t,
 //     u_t = beta_t (v_t - g_t S_(t-1)^T k_t),   S_t = g_t S_(t-1) + k_t u_t^T,   o_t = S_t^T q_t .
 // Over a chunk of L = 32 tokens, b_t the running sum of ln g, gamma_t = e^(b_t) and S_0 the state
@@ -568,8 +569,8 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
 
 // Chunkwise for 128 key channels where the rows pay (chunk_rows.h; a chunk's workspace is 200 KB for 16
 // heads, which few rows per sequence would multiply, too).  16 x 1000 tokens of 16 heads with 128 x 128
-// states: 1328 us token by token, 292 us chunkwise (71 us for W and P); 2 x 8192: 7.5 ms and 0.9 ms.  The
-// walk issues 1000 vector instructions and 168 MFMAs per wave and chunk.
+// states: 1328 us token by token, 296 us chunkwise (70 us for W and P); 2 x 8192: 7.5 ms and 0.8 ms.  The
+// walk issues 1000 vector instructions and 168 MFMAs per wave and chunk: 50 % and 34 % of a SIMD's cycles.
 bool delta_chunk_ok(const float* qkv, int P, int Tp, int H, int G, int d, int V) {
   return chunk_rows_pay(P, Tp, 48) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(qkv) & 15) == 0 &&

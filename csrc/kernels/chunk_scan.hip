@@ -1,6 +1,6 @@
-// Chunkwise matrix-state recurrences of prompt rows on the matrix cores: the mLSTM and the
-// Mamba-2 (SSD) scan.  Both carry S [d, dv] per (sequence, head) and, with a log decay f_t and a
-// log input weight i_t per token (SSD: i_t = ln of the step size),
+// Chunkwise matrix-state recurrences of prompt rows on the matrix cores: the mLSTM (Beck et al., xLSTM, 2024)
+// and the Mamba-2 (SSD) scan (Dao and Gu, 2024).  Both carry S [d, dv] per (sequence, head) and, with a log
+// decay f_t and a log input weight i_t per token (SSD: i_t = ln of the step size),
 //     S_t = e^(f_t) S_(t-1) + e^(i_t) k_t v_t^T,      o_t = S_t^T q_t .
 // Over a chunk of L tokens with b_t the running sum of f and S_0 the state before it:
 //     o_t = e^(b_t) S_0^T q_t + sum_(s <= t) e^(b_t - b_s + i_s) (q_t . k_s) v_s
@@ -23,9 +23,10 @@
 // products of parts whose weight is at least 2^-16 are kept, and the sums are fp32.  bf16
 // inputs are one exact part, f16 inputs two.
 //
-// What bounds it (mLSTM, 4 heads with 256 x 512 states, 64-token chunks): the vector work of a
-// chunk, most of it splitting S, takes 15 k cycles on a SIMD, its MFMAs 8 k, and the rest of 34 k
-// is barriers and latency that two waves per SIMD do not cover; LDS (140 KB) allows no third.
+// What bounds it (mLSTM, 4 heads with 256 x 512 states, 64-token chunks): a wave issues 1550 vector
+// instructions per chunk, most of them splitting S, and 222 MFMAs; they fill 42 % and 24 % of a SIMD's
+// cycles (SSD's second walk: 59 % and 26 %).  The rest is barriers and latency that two waves per SIMD do not
+// cover; LDS (140 KB) allows no third.
 //
 // Few long sequences: the walk is serial, so a step of few workgroups is cut into segments.  A
 // first launch computes every segment's contribution from a zero state, the second starts each
@@ -709,8 +710,8 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L) {
 }
 
 // Chunkwise from 16 rows per sequence on, heads of 128 or 256 key channels in 16 bits (fp32 rows in
-// three parts do not fit LDS).  32 x 512 tokens, 4 heads of 256 x 512: 1957 us token by token, 219 us
-// chunkwise, and nearer to float64 (3.5e-7 against 4.7e-7).
+// three parts do not fit LDS).  32 x 512 tokens, 4 heads of 256 x 512: 1957 us token by token, 222 us
+// chunkwise, and nearer to float64 (3.5e-7 against 5.0e-7).
 bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, int H, int d, int dv) {
   if (!((dtype == DT_BF16 || dtype == DT_F16) && P > 0 && Tp >= 16 * P && (d == 128 || d == 256) &&
         stride % 8 == 0 && (reinterpret_cast<uintptr_t>(qkvg) & 15) == 0 && dv >= 16 &&
@@ -755,8 +756,8 @@ static int ssd_heads(int H, int V, int G) { return V <= 64 && (H / G) % 2 == 0 ?
 // Mamba-2: 128 state rows, fp32 x | B | C (three bf16 parts each), 32-token chunks; two heads of up
 // to 64 columns share a workgroup's B and C.  16 rows alone stay token by token (9.9 us against 10.3;
 // 4 x 18: 12.8 and 10.9).  2 x 8192 tokens, 32 heads of 128 x 64: 4821 us token by
-// token (a chain of 8192 steps in 64 workgroups), 353 us in chunks and segments of 1184; from float64
-// 7.0e-8 (7.3e-8).  Half of that time is vector work, most of it the splits of S, B and C.
+// token (a chain of 8192 steps in 64 workgroups), 359 us in chunks and segments of 1184 (130 the walk
+// from zero, 255 the second); from float64 7.0e-8 (7.3e-8).
 bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G) {
   return P > 0 && Tp >= 16 * P && Tp >= 20 && N == 128 && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(xbc) & 15) == 0 &&

@@ -9,7 +9,9 @@
 // seq_lens[i] - rows) followed by its decode rows (one row each, position ctx_lens - 1).  A
 // chunk that starts at position 0 starts from zero state; a slot < 0 is a padding row and
 // gives zeros.  Prefill chunks and decode rows run the same code, token by token, so a
-// position's result does not depend on how the prompt was cut.
+// position's result does not depend on how the prompt was cut.  (gla_scan's prompts of more
+// than a few rows go chunkwise, chunk_gla.hip: as near
+// to exact, rounded differently.)
 //
 // Layout: grid (step sequences, heads, column tiles), four waves.  The state of one head is
 // S [R, V] (gla: R key channels, V value columns; selective scan: R states, V channels, kept
@@ -194,8 +196,8 @@ __global__ __launch_bounds__(NT) void gla_scan_kernel(
 // A step of decode rows only, one token each: thread (16 row groups, 16 lanes of 4 columns) with state
 // rows rg + 16 i, so a state row is read and written 256 bytes at a time and all of a lane's rows are in
 // flight while the decays are computed (the scan above reads 64 bytes of a row).  V a multiple of 4.
-// Bound by the state's bytes: 64 rows of 8 heads [128, 256], 134 MB, 42 us by the scan, 27 here (5 TB/s, the
-// rate of a large copy); 8 rows 11.5 -> 10.
+// Bound by the state's bytes: 64 rows of 8 heads [128, 256], 134 MB, 42 us by the scan, 25 here (5.4 TB/s; a
+// large copy reaches 4.8); 8 rows 11.5 -> 10.
 template <typename T, int RI>
 __global__ __launch_bounds__(NT) void gla_decode_kernel(
     float* __restrict__ out, const T* __restrict__ proj, int64_t ps, const T* __restrict__ low,

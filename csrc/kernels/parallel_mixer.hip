@@ -10,7 +10,9 @@
 // seq_lens[i] - rows) followed by its decode rows (one row each, position ctx_lens - 1).  A
 // chunk that starts at position 0 starts from zero state; a slot < 0 is a padding row and
 // gives zeros.  Prefill chunks and decode rows run the same code, token by token, so a
-// position's result does not depend on how the prompt was cut.
+// position's result does not depend on how the prompt was cut.  (Prompts of more than a few
+// rows go chunkwise, chunk_scan.hip and chunk_delta.hip: as near
+// to exact, rounded differently.)
 //
 // Scan layout: grid (step sequences, heads, value-column tiles), four waves.  The state of
 // one head is S [R, V] (R: state size N or key size d; V: value columns).  A wave owns 16

@@ -6,7 +6,8 @@
 //     o_t = S'^T q / (max(|n'.q|, e^(-m')) + 1e-6),   q scaled by d^-1/2
 // A sequence chunk that starts at position 0 starts from zero state; any other chunk reads
 // the slot the previous step left.  Prefill chunks and decode rows are the same scan (a
-// decode row is a chunk of one token).
+// decode row is a chunk of one token); 16-bit prompts of 128 or 256 key channels go chunkwise
+// (chunk_scan.hip).
 //
 // grid (step sequences, heads, ceil(dv / 64)), 256 threads.  A workgroup owns 64 value
 // columns of one head's S: lane = column, wave w holds a contiguous quarter of the rows in
@@ -197,7 +198,9 @@ __global__ __launch_bounds__(NT) void mlstm_scan_kernel(
 }
 
 // n and m of the step's sequences, copied before the scan: the column workgroups of a head all
-// start from them, and the first one writes the slot while later ones may not have begun.
+// start from them, and the first one writes the slot while later ones may not have begun.  The launch costs a
+// decode step 2 us per layer (4 heads of 256 x 512, graph replay: 1 row 14.6 -> 16.9 us, 64 rows 71.7 -> 75.0,
+// 256 rows 290 -> 295).
 __global__ __launch_bounds__(64) void mlstm_head_state_kernel(
     float* __restrict__ n0, float* __restrict__ m0, const float* __restrict__ nst,
     const float* __restrict__ mst, const int* __restrict__ slots, int H, int d, int num_slots) {

@@ -12,12 +12,13 @@
 // weights keep ~16 bits).  V^T fragments come from the row-major tile by transposing LDS reads; where
 // the values are columns of the key rows (latent rows) they come from the key tile itself.
 //
-// The waves of a SIMD take turns between MFMAs (raised priority: 231 -> 229 us and, for short prompts,
-// 18 -> 16 us) and the softmax.
+// The waves of a SIMD take turns between MFMAs (raised priority: 1 % at long prompts, 18 -> 16 us for short
+// ones) and the softmax.
 //
-// What bounds it: the MFMAs (two thirds of them the pairs of P V; at 8 x 2048 rows, window 1024, they
-// alone are 110 us of the 229 at a large product's rate) and the softmax's vector work (80 us), which
-// overlap in part.  Not the loads: a ring of four tiles filled by LDS-DMA three tiles ahead took 249 us.
+// What bounds it: 8 x 2048 rows, window 1024, 198 us; the MFMAs (two thirds of them the pairs of P V) work in
+// 36 % of a SIMD's cycles and vector instructions, most of them the softmax's, issue in 50 %, overlapping in
+// part (capped and causal: 30 % and 73 %; latent rows: 29 % and 40 %).  Not the loads: a ring of four tiles
+// filled by LDS-DMA three tiles ahead took 249 us where this took 229.
 #include "device.h"
 #include "window.h"
 #include <type_traits>
@@ -385,9 +386,9 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
                                int window, int keep_first, const float* gate, const WindowExtra& ex,
                                hipStream_t s) {
   // Four heads on one staged tile pay at every length, against one head per workgroup (bf16, 16 heads
-  // on 4 key/value heads): window 1024 with 8 x 2048 rows 355 -> 199 us, causal and capped 577 -> 291,
+  // on 4 key/value heads): window 1024 with 8 x 2048 rows 355 -> 198 us, causal and capped 577 -> 290,
   // 48 rows after 3000 83 -> 68, 48 alone equal; latent rows (one key/value head), 32 x 512 rows
-  // 380 -> 131 us, 4 x 2000 after 500 974 -> 390.  The maximum is taken before the scale, which has to be
+  // 380 -> 129 us, 4 x 2000 after 500 974 -> 390.  The maximum is taken before the scale, which has to be
   // positive for that.
   if (n_work <= 0 || !(scale > 0.f) || H / G % HW != 0 || ex.pool > 0 || ex.vtab != nullptr ||
       blk_rows % BM != 0)

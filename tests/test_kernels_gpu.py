@@ -458,7 +458,7 @@ def test_prefill_lazy_rescale_growing_scores(gpu, monkeypatch, gqa, shape):
 @pytest.mark.parametrize("shape", ["short_many", "mixed_chunked", "one_item"])
 def test_prefill_persistent_walk_bit_identical(gpu, monkeypatch, dt, nq, nkv, d, shape):
     """K2's persistent GQA walk (one workgroup per CU over the work list, the K / V tile
-    stream running across items; KGC_PREFILL_PERSIST=1, the default) against the one-shot
+    stream running across items; KGC_PREFILL_PERSIST=1) against the one-shot
     GQA grid (=0): the same tiles in the same order per wave, so the outputs must agree bit
     for bit -- on many short prompts (more items than CUs, 1-8 tiles each), on mixed fresh
     prompts and chunked continuations (empty sub-blocks, single-tile items next to long
