@@ -1,12 +1,17 @@
 // Windowed attention of prompt rows where four query heads share a key/value head (attention_window.hip
 // has the other shapes, pooled blocks and rotated values).
 //
-// A workgroup of 8 waves owns 64 query rows of four heads of one key/value group: a wave has 32 rows
-// of one head, as two MFMA column groups, so every key and value fragment read from LDS serves two
-// products and every staged tile four heads.  Key tiles are 64 rows -- first the kept first tokens that
-// lie before the earliest window, then the span from that window to the last row -- copied as they lie
-// (16 bytes a lane, rows padded by 8 elements) into one of two LDS buffers while the other is computed
-// on; the page numbers are loaded a tile further ahead.  Per tile and wave, as in the one-head kernel:
+// A workgroup of 8 waves owns 64 query rows of four heads of one key/value group: a wave has 16 rows
+// of two heads, as two MFMA column groups, so every key and value fragment read from LDS serves two
+// products and every staged tile four heads.  Both groups see the same keys, and a wave leaves out the
+// tiles of which it sees none: under weights of zero a value that is not finite would become NaN, so it
+// reaches 16 rows (32 rows of one head per wave: equal times but for short prompts with an element gate, where
+// a block of few rows then has fewer sigmoids per SIMD, 8 x 100 rows 18 us against 22).
+//
+// Key tiles are 64 rows -- first the kept first tokens that lie before the earliest window, then the span
+// from that window to the last row -- copied as they lie (16 bytes a lane, rows padded by 8 elements) into
+// one of two LDS buffers while the other is computed on; the page numbers are loaded a tile further ahead.
+// Per tile and wave, as in the one-head kernel:
 //   S^T = K Q^T, visibility, online softmax in fp32 (base 2), O^T += V^T P^T
 // with P^T taken from the S^T accumulators as a pair of 16-bit values (value + remainder: the fp32
 // weights keep ~16 bits).  V^T fragments come from the row-major tile by transposing LDS reads; where
@@ -83,19 +88,19 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   if (r0 >= qlen || ctx0 < 0) return;
   const int rows = min(BM, qlen - r0);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, qd = lane >> 4;
-  const int h = blockIdx.x * HW + (wave & 3), g = blockIdx.x * HW / (H / G);
+  const int g = blockIdx.x * HW / (H / G);
+  // column group c's head: c is swapped from one row group to the next, so that the waves write (and read
+  // the gates of) all four heads at a time (1 %)
+  auto head = [&](int c) { return (int)blockIdx.x * HW + 2 * (wave & 1) + (c ^ (wave >> 1 & 1)); };
   const int* bt = pbt + (int64_t)seq * bt_stride;
-  const int wr = r0 + 32 * (wave >> 2);               // the wave's first row
+  const int wr = r0 + 16 * (wave >> 1);               // the wave's first row
+  const int myrow = wr + r16, qpos = ctx0 + myrow;
+  const bool rowok = myrow < qlen;
+  const int row_lo = first_visible(qpos, window, ex.chunked);
   V8 qf[2][KS];
-  int qpos[2], row_lo[2];
-  bool rowok[2];
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    const int row = wr + 16 * c + r16;
-    rowok[c] = row < qlen;
-    qpos[c] = ctx0 + row;
-    row_lo[c] = first_visible(qpos[c], window, ex.chunked);
-    const T* qrow = q + ((int64_t)(q0 + min(row, qlen - 1)) * H + h) * DK + 8 * qd;
+    const T* qrow = q + ((int64_t)(q0 + min(myrow, qlen - 1)) * H + head(c)) * DK + 8 * qd;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       Pack8<T> t;
@@ -116,7 +121,7 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   const int ns = window > 0 ? min(keep_first, lo_min) : 0;
   const int nsink = (ns + BN - 1) / BN, ntile = nsink + (p_max - lo_min + BN) / BN;
   // the wave's own span of visible keys (tiles outside it are staged but not computed)
-  const int wp_lo = ctx0 + wr, wp_hi = min(wp_lo + 31, p_max);
+  const int wp_lo = ctx0 + wr, wp_hi = min(wp_lo + 15, p_max);
   const int w_lo = first_visible(wp_lo, window, ex.chunked);
   const int w_lo_hi = first_visible(wp_hi, window, ex.chunked);
   const bool live = wr < r0 + rows;
@@ -215,7 +220,7 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
       __builtin_amdgcn_s_setprio(0);
       // keys that all are there, not after the wave's first row and inside the window of its last
       // are seen by every row: no test per element
-      const bool full = k1 <= hi && k1 - 1 <= wp_lo && k0 >= w_lo_hi && wp_lo + 31 == wp_hi;
+      const bool full = k1 <= hi && k1 - 1 <= wp_lo && k0 >= w_lo_hi && wp_lo + 15 == wp_hi;
       V8 ph[2][NJ / 2], pl[2][NJ / 2];
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
@@ -247,14 +252,14 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
           }
         }
         if (!full) {
-          const int last = min(hi - 1, qpos[c]) - k0 - 4 * qd, low = row_lo[c] - k0 - 4 * qd,
+          const int last = min(hi - 1, qpos) - k0 - 4 * qd, low = row_lo - k0 - 4 * qd,
                     kept = keep_first - k0 - 4 * qd;
 #pragma unroll
           for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               const int key = 16 * j + i;
-              const bool vis = (key <= last) & ((key >= low) | (key < kept)) & rowok[c];
+              const bool vis = (key <= last) & ((key >= low) | (key < kept)) & rowok;
               s[c][j][i] = vis ? s[c][j][i] : -INFINITY;
             }
         }
@@ -320,8 +325,9 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   for (int c = 0; c < 2; ++c) {
     float ls = l[c] + __shfl_xor(l[c], 16, 64);
     ls += __shfl_xor(ls, 32, 64);
-    if (!rowok[c] || !live) continue;
-    const int64_t t = q0 + wr + 16 * c + r16;
+    if (!rowok || !live) continue;
+    const int64_t t = q0 + myrow;
+    const int h = head(c);
     const float gt = (gate != nullptr ? gate[t * H + h] : 1.f) * ex.out_scale;
     const float inv = ls > 0.f ? gt / ls : 0.f;
     T* orow = out + t * ex.ors + h * DV + 4 * qd;

@@ -517,6 +517,49 @@ def test_window_attention_capped_scores(gpu, dt, latent, cap):
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("latent", [False, True])
+@pytest.mark.parametrize("ctx,bad,clean,kw", [
+    (10, 70, [(0, 48)], {}),                                         # only the last 16 of the 64 rows see its tile
+    (16, 20, [(48, 64)], dict(window=64, chunked=True)),             # a chunk before these rows'
+    (10, 20, [], {})])                                               # every group sees its tile
+def test_window_attention_values_not_finite(gpu, dt, latent, ctx, bad, clean, kw):
+    """A value that is not finite: rows whose 16 rows see nothing of its 64 keys keep the bits of the call
+    without it (as in the kernel of one head per workgroup), every row keeps its other columns, and rows that
+    see it do not hide it."""
+    torch.manual_seed(33)
+    H, bs, n, (dk, dv) = 4, 16, 64, (256, 192) if latent else (128, 128)
+    total = n + ctx
+    width = (total + bs - 1) // bs
+    tables = (torch.randperm(width) + 1).view(1, width).int()
+    m, q = _meta([n], [total], [], tables), torch.randn(n, H, dk).to(dt)
+    kc = torch.randn(width + 1, 1, bs, dk).to(dt)
+    kw = dict(kw)
+    window = kw.pop("window", 0)
+    row, col = (int(tables[0, bad // bs]), 0, bad % bs), 100
+
+    def run(vc):
+        vg = vc.to(gpu)
+        kg = vg if latent else kc.to(gpu)
+        return ops.window_attention(q.to(gpu), kg, vg[..., :dv], torch.arange(ctx, total).to(gpu), _to(m, gpu),
+                                    dk ** -0.5, window, 0, torch.ones(n, H).to(gpu), **kw).cpu().view(n, H, dv)
+    vc = kc if latent else torch.randn(width + 1, 1, bs, dv).to(dt)
+    want = run(vc)
+    vb = vc.clone()
+    vb[row][col] = float("inf")
+    got = run(vb)
+    pos = torch.arange(ctx, total)
+    sees = pos >= bad
+    if window:
+        sees &= pos // window == bad // window
+    assert sees.any() and not got[sees][..., col].isfinite().any()
+    if not latent:                           # (a latent row is the key, too)
+        keep = torch.arange(dv) != col
+        assert torch.equal(got[..., keep], want[..., keep])
+    for a, b in clean:
+        assert torch.equal(got[a:b], want[a:b])
+
+
 def _gla_case(T, slots, H, d, V, R, dt, tau, dev, open_=3.0):
     """Inputs of gla_scan and its terms for ``_matrix64``."""
     proj = (torch.randn(T, 2 * H * d + H * V + R) * 0.7).to(dt)
