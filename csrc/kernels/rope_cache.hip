@@ -218,7 +218,8 @@ __global__ __launch_bounds__(ROPE_NT) void rope_kv_kernel(
 // Blocks that follow the cache and not the rows are what ragged prompts need: with blocks of 8 rows
 // aligned to the step, every prompt behind one of odd length took the 2-byte stores (32 x 512 ragged
 // rows, 8 heads of 128, 134 MB: 75 us, 28 here, the rate of a large copy; fp8 cache, which had the
-// per-token kernel, 86 -> 22).
+// per-token kernel, 86 -> 22).  Up to 1000 rows that do lie with the groups take 4.7 us where blocks
+// of the step's rows took 4.0: a thread has four pairs or eight rows.
 constexpr int KVG_NT = 256;
 template <typename T, bool KV8>
 __global__ __launch_bounds__(KVG_NT) void kv_group_kernel(

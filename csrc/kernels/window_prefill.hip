@@ -391,11 +391,13 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
                                int G, int dk, int dv, int krs, int vrs, int bs, int num_blocks, float scale,
                                int window, int keep_first, const float* gate, const WindowExtra& ex,
                                hipStream_t s) {
-  // Four heads on one staged tile pay at every length, against one head per workgroup (bf16, 16 heads
-  // on 4 key/value heads): window 1024 with 8 x 2048 rows 355 -> 198 us, causal and capped 577 -> 290,
-  // 48 rows after 3000 83 -> 68, 48 alone equal; latent rows (one key/value head), 32 x 512 rows
-  // 380 -> 129 us, 4 x 2000 after 500 974 -> 390.  The maximum is taken before the scale, which has to be
-  // positive for that.
+  // Four heads on one staged tile against one head per workgroup (bf16, 16 heads on 4 key/value heads): window
+  // 1024 with 8 x 2048 rows 355 -> 198 us, causal and capped 577 -> 290, 48 rows after 3000 83 -> 68; latent rows
+  // (one key/value head), 32 x 512 rows 380 -> 129 us, 4 x 2000 after 500 974 -> 390.  Up to 16 prompts of 33 to
+  // 64 rows without context are slower, a wave having two heads of its one tile (8 x 64: 11.0 -> 11.8, capped
+  // 16.2 -> 17.7, latent 12.8 -> 15.8); with 300 tokens of context they are faster (34.8 -> 27.3, 52.6 -> 35.9,
+  // 47.4 -> 38.3), and the context is known on the device only.  The maximum is taken before
+  // the scale, which has to be positive for that.
   if (n_work <= 0 || !(scale > 0.f) || H / G % HW != 0 || ex.pool > 0 || ex.vtab != nullptr ||
       blk_rows % BM != 0)
     return false;
