@@ -168,15 +168,20 @@ static __device__ unsigned int kgc_dbg_err;
     (void)hipMemcpyToSymbol(HIP_SYMBOL(kgc_dbg_err), &z, sizeof(z));         \
     return v;                                                                \
   }
-#define KGC_DCHECK_RANGE(v, lo, hi, what)                                                     \
-  do {                                                                                        \
-    if ((long long)(v) < (long long)(lo) || (long long)(v) >= (long long)(hi)) {              \
-      if (atomicOr(&kgc_dbg_err, 1u) == 0u)                                                   \
-        printf("kgc debug check: %s = %lld not in [%lld, %lld) at %s:%d (wg %d,%d,%d t %d)\n", \
-               what, (long long)(v), (long long)(lo), (long long)(hi), __FILE__, __LINE__,   \
-               (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)threadIdx.x);         \
-      (v) = (lo);                                                                             \
-    }                                                                                         \
+// One out-of-line report per translation unit: printf's string handling inlined at every check of
+// every instance made the two attention files compile for six and ten minutes.
+static __device__ __attribute__((noinline)) void kgc_dbg_report(long long v, long long lo, long long hi,
+                                                                const char* what, const char* file, int line) {
+  if (atomicOr(&kgc_dbg_err, 1u) == 0u)
+    printf("kgc debug check: %s = %lld not in [%lld, %lld) at %s:%d (wg %d,%d,%d t %d)\n", what, v, lo, hi,
+           file, line, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)threadIdx.x);
+}
+#define KGC_DCHECK_RANGE(v, lo, hi, what)                                                             \
+  do {                                                                                                \
+    if ((long long)(v) < (long long)(lo) || (long long)(v) >= (long long)(hi)) {                      \
+      kgc_dbg_report((long long)(v), (long long)(lo), (long long)(hi), what, __FILE__, __LINE__);     \
+      (v) = (lo);                                                                                     \
+    }                                                                                                 \
   } while (0)
 #else
 #define KGC_DEBUG_TU(name) \
