@@ -1528,10 +1528,21 @@ void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
   }
   if (fast && aligned && D > 0 &&
       kgc::window_decode_mfma_ok(dt, (int)dk, (int)dv, (int)(H / G), ex)) {
-    kgc::launch_window_decode_mfma(dt, out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
-                                   v_cache.data_ptr(), cp, dp, (int)bts, (int)Tp, (int)D, (int)H,
-                                   (int)G, (int)dk, (int)dv, (int)krs, (int)vrs, bs, nb,
-                                   (float)scale, (int)window, (int)keep_first, gp, ex, stream());
+    const int Z = kgc::window_split_pieces((int)D, (int)H, (int)G, (int)dk, (int)dv, (int)bts, bs,
+                                             (int)window, (int)keep_first);
+    if (Z > 0) {
+      Tensor work = at::empty({kgc::window_split_floats((int)D, (int)H, (int)dv, Z)},
+                              q.options().dtype(at::kFloat));
+      kgc::launch_window_split(dt, out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                               cp, dp, (int)bts, (int)Tp, (int)D, (int)H, (int)G, (int)dk, (int)dv,
+                               (int)krs, (int)vrs, bs, nb, (float)scale, (int)window, (int)keep_first, gp,
+                               ex, Z, work.data_ptr<float>(), stream());
+    } else {
+      kgc::launch_window_decode_mfma(dt, out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
+                                     v_cache.data_ptr(), cp, dp, (int)bts, (int)Tp, (int)D, (int)H,
+                                     (int)G, (int)dk, (int)dv, (int)krs, (int)vrs, bs, nb,
+                                     (float)scale, (int)window, (int)keep_first, gp, ex, stream());
+    }
     rest &= ~2;
   } else if (decode_fast) {
     kgc::launch_window_decode(dt, out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),

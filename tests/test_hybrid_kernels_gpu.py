@@ -709,6 +709,35 @@ def test_window_decode_many_waves(gpu, dt, H, G, rows, kw):
     torch.testing.assert_close(got.cpu().float()[keep], want.float()[keep], rtol=1.01 * ulp, atol=2e-4)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,dk,dv,latent", [(16, 4, 128, 128, False), (6, 2, 72, 40, False), (40, 1, 256, 192, True),
+                                              (3, 1, 200, 248, False), (20, 1, 128, 64, True)])
+@pytest.mark.parametrize("lens,kw", [([2100], dict(window=0, keep=0)), ([0, 1, 33, 300, 2100, 511], dict(window=0, keep=0, softcap=5.0)),
+                                     ([2100, 40, 1024], dict(window=300, keep=5, sink=0.4)), ([2081, 2048, 2047], dict(window=1024, keep=0, chunked=True))])
+def test_window_decode_in_pieces(gpu, dt, H, G, dk, dv, latent, lens, kw):
+    """Steps of few rows, their keys over many workgroups: rows with fewer chunks than pieces, several chunks
+    per piece, one key, a padding row, a sink, values of their own and as columns of the keys."""
+    torch.manual_seed(73)
+    n, bs, width, nb = len(lens), 16, 132, 300
+    tables = torch.randint(0, nb, (n, width), dtype=torch.int32)
+    kc = torch.randn(nb, G, bs, dk).to(dt)
+    vc = kc[..., :dv] if latent else torch.randn(nb, G, bs, dv).to(dt)
+    q, gate = torch.randn(n, H, dk).to(dt), torch.rand(n, H)
+    eg = torch.randn(n, H * dv + 8).to(dt)
+    m = _meta([], [], lens, tables)
+    pos, kw = torch.tensor(lens) - 1, dict(kw)
+    args = (0.09, kw.pop("window"), kw.pop("keep"))
+    want = ops.window_attention(q, kc, vc, pos, m, *args, gate, elem_gate=eg[:, 8:], **kw).float()
+    kg = kc.to(gpu)
+    vg = kg[..., :dv] if latent else vc.to(gpu)
+    got = ops.window_attention(q.to(gpu), kg, vg, pos.to(gpu), _to(m, gpu), *args, gate.to(gpu),
+                               elem_gate=eg.to(gpu)[:, 8:], **kw).cpu().float()
+    live = torch.tensor(lens) > 0
+    assert (got[~live] == 0).all()
+    ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
+    torch.testing.assert_close(got[live], want[live], rtol=1.01 * ulp, atol=2e-4)
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,V,R", [(2, 64, 5), (1, 144, 16), (3, 40, 1)])
 @pytest.mark.parametrize("lens,before,D_ctx", CHUNKS)
