@@ -1748,12 +1748,20 @@ void ssd_scan(Tensor out, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, T
   const int *ql = i32_ptr(qsl, P ? P + 1 : 0, "query_start_loc"), *sl = i32_ptr(seq_lens, P, "seq_lens"),
             *cl = i32_ptr(ctx_lens, D, "ctx_lens"), *st = i32_ptr(slots, P + D, "state slots");
   if (kgc::ssd_chunk_ok(xbc.data_ptr<float>(), (int)P, (int)Tp, (int)H, (int)V, (int)N, (int)G)) {
-    kgc::ChunkWork cw = kgc::ssd_chunk_plan((int)P, (int)Tp, (int)H, (int)V, (int)G);
-    Tensor cs, cg;
-    chunk_workspace(cw, H * N * V, H, xbc, cs, cg);
-    kgc::launch_ssd_chunk(dt_code(dt), out.data_ptr<float>(), xbc.data_ptr<float>(), dt.data_ptr(),
-                          dt.stride(0), al, db, ds, S.data_ptr<float>(), ql, sl, st, (int)P, (int)H,
-                          (int)V, (int)N, (int)G, (int)S.size(0), cw, stream());
+    if (kgc::ssd_shared_ok((int)P, (int)Tp, (int)H, (int)V, (int)G)) {
+      const kgc::SsdWork cw = kgc::ssd_shared_plan((int)P, (int)Tp, (int)H, (int)V, (int)G);
+      Tensor ws = at::empty({cw.bytes}, xbc.options().dtype(at::kByte));
+      kgc::launch_ssd_shared(dt_code(dt), out.data_ptr<float>(), xbc.data_ptr<float>(), dt.data_ptr(),
+                             dt.stride(0), al, db, ds, S.data_ptr<float>(), ql, sl, st, (int)P, (int)Tp,
+                             (int)H, (int)V, (int)G, (int)S.size(0), cw, ws.data_ptr(), stream());
+    } else {
+      kgc::ChunkWork cw = kgc::ssd_chunk_plan((int)P, (int)Tp, (int)H, (int)V, (int)G);
+      Tensor cs, cg;
+      chunk_workspace(cw, H * N * V, H, xbc, cs, cg);
+      kgc::launch_ssd_chunk(dt_code(dt), out.data_ptr<float>(), xbc.data_ptr<float>(), dt.data_ptr(),
+                            dt.stride(0), al, db, ds, S.data_ptr<float>(), ql, sl, st, (int)P, (int)H,
+                            (int)V, (int)N, (int)G, (int)S.size(0), cw, stream());
+    }
     st += P;                             // the decode rows are left
     P = 0;
   }

@@ -372,6 +372,18 @@ void launch_ssd_chunk(int dtype, float* out, const float* xbc, const void* dt, i
                       const float* a_log, const float* dt_bias, const float* dskip, float* S,
                       const int* qsl, const int* seq_lens, const int* slots, int P, int H, int V,
                       int N, int G, int num_slots, const ChunkWork& work, hipStream_t s);
+// of the calls that ssd_chunk_ok takes, those whose heads share enough (chunk_ssd.hip): `bytes` of workspace,
+// where its parts begin
+struct SsdWork {
+  int seg = 0, items = 0;
+  int64_t bytes = 0, state_at = 0, gate_at = 0;
+};
+bool ssd_shared_ok(int P, int Tp, int H, int V, int G);
+SsdWork ssd_shared_plan(int P, int Tp, int H, int V, int G);
+void launch_ssd_shared(int dtype, float* out, const float* xbc, const void* dt, int64_t dts,
+                       const float* a_log, const float* dt_bias, const float* dskip, float* S,
+                       const int* qsl, const int* seq_lens, const int* slots, int P, int Tp, int H, int V,
+                       int G, int num_slots, const SsdWork& work, void* ws, hipStream_t s);
 // gated delta rule of prompt rows (chunk_delta.hip): segments as above, bf16 values of `wp` and floats
 // of `ws`
 struct DeltaWork {

@@ -324,6 +324,15 @@ def test_ssd_scan_chunkwise(gpu, dt, H, G, V, lens, before, D_ctx):
     assert _whole(got, want + add) and _whole(S_g, S_w)
 
 
+@pytest.mark.parametrize("H,G,V", [(4, 1, 64), (8, 2, 40), (4, 1, 144), (8, 1, 33), (4, 1, 131), (4, 1, 16)])
+@pytest.mark.parametrize("lens,before,D_ctx", [([400, 129, 250, 33, 31, 1, 96], [0, 7, 0, 0, 9, 0, 64], [5]),
+                                               ([1025, 449], [33, 0], []), ([1000, 28, 1500], [0, 7, 9], [2])])
+def test_ssd_scan_shared_images(gpu, H, G, V, lens, before, D_ctx):
+    """Prompt rows of heads that share B and C: whole sequences and segments that end inside a chunk, a
+    padding sequence, pairs of heads, one head over two workgroups, an odd number of columns."""
+    test_ssd_scan_chunkwise(gpu, torch.bfloat16, H, G, V, lens, before, D_ctx)
+
+
 @pytest.mark.parametrize("op,dt", [("mlstm", torch.bfloat16), ("mlstm", torch.float16), ("ssd", torch.bfloat16)])
 def test_scan_segments_start_from_the_incoming_state(gpu, op, dt):
     """Continued prompts that are cut into segments, while products on another stream hold
