@@ -49,6 +49,43 @@ __device__ __forceinline__ void mm(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB],
   else hi = mfma16x16x32(a[0], b[0], hi);
 }
 
+// Products of three parts each, N row tiles a times the columns of b: several sums side by side, since an MFMA
+// waits for the one whose sum it continues.  The corrections first, the main products on top of them.
+template <int N>
+__device__ __forceinline__ void mm3(const bf16x8 (&a)[N][3], const bf16x8 (&b)[3], f32x4 (&c)[N]) {
+  constexpr int PA[6] = {0, 1, 2, 0, 1, 0}, PB[6] = {2, 1, 0, 1, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+#pragma unroll
+    for (int i = 0; i < N; ++i) c[i] = mfma16x16x32(a[i][PA[k]], b[PB[k]], k ? c[i] : f32x4{0.f, 0.f, 0.f, 0.f});
+}
+// hi + lo += a b
+template <int N>
+__device__ __forceinline__ void mm3_add(const bf16x8 (&a)[N][3], const bf16x8 (&b)[3], f32x4 (&hi)[N], f32x4 (&lo)[N]) {
+  constexpr int PA[6] = {0, 1, 2, 0, 1, 0}, PB[6] = {2, 1, 0, 1, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      f32x4& c = k == 5 ? hi[i] : lo[i];
+      c = mfma16x16x32(a[i][PA[k]], b[PB[k]], c);
+    }
+}
+
+// Order of the instructions up to here from the last sched_barrier: N times one MFMA and V vector instructions, which
+// run beside it, an LDS read after every R-th and a memory instruction after every M-th (0: where they fall; in a
+// burst they would hold up the wave).  An MFMA of 16 x 16 x 32 takes 8 cycles of issue and 16 of the matrix core, a vector
+// instruction 4; two waves of a SIMD overlap them by chance only, half of the time.
+template <int N, int V, int R = 0, int M = 0> __device__ __forceinline__ void interleave() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+    if (R > 0 && i % R == R - 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    if (M > 0 && i % M == M - 1) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+  }
+}
+
 // e^x for x <= 0 held in double: the reduction to 2^n 2^f is exact to fp32 however large x is, so
 // the error is that of the hardware's 2^f, |f| <= 1/2
 __device__ __forceinline__ float exp_d(double x) {

@@ -79,6 +79,9 @@ __device__ __forceinline__ void wave_lds() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// place of a 16-byte unit of W or P, so that 16 lanes read 16 different bank groups
+__device__ __forceinline__ int wp_unit(int t, int u) { return t * (L / 8) + (u ^ ((t >> 2) & 3)); }
+
 // ---- W, P, the gates and the norms of every chunk: one wave per (chunk, q / k group) -----------
 __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
   __shared__ float KK[L][L + 1], QK[L][L + 1];           // [t][s]: dots of unit vectors, s <= t
@@ -194,7 +197,7 @@ __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
         const float y[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
         bf16x8 o[3];
         split8<3>(y, o);
-        bf16* dst = a.wp + (((int64_t)blockIdx.x * a.H + g * hpg + h0 + hh) * 2 + mat) * MAT + t * L + oct * 8;
+        bf16* dst = a.wp + (((int64_t)blockIdx.x * a.H + g * hpg + h0 + hh) * 2 + mat) * MAT + wp_unit(t, oct) * 8;
 #pragma unroll
         for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(dst + i * L * L) = o[i];
       }
@@ -241,7 +244,9 @@ __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
 template <int MODE>
 __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
   __shared__ __align__(16) bf16 Ks[3 * L * DP], Qs[MODE == 1 ? 8 : 3 * L * DP], KT[3 * D * LP];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  __shared__ __align__(16) bf16 Ws[MAT], Ps[MODE == 1 ? 8 : MAT];
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int seq = blockIdx.x, seg_idx = 0, item = 0, seg_count = 1;
   if (MODE != 0) {
     const SegItem it = seg_item(blockIdx.x, a.qsl, a.P, a.seg);
@@ -300,7 +305,7 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
   float nk = 0.f, nq = 0.f;
   const int ut = tid / 16, uc = (tid % 16 / 4) * 32 + (tid % 4) * 4, up_ = (tid % 16) * 8;
   const int ta = tid / D * 4, tc = tid % D;
-  auto fetch = [&](int c0, int ci) {
+  auto fetch_rows = [&](int c0, int ci) {
     const int nl = min(L, len - c0);
     const float* kr = kb + (int64_t)(start + c0) * a.stride;
     const float* qr = qb + (int64_t)(start + c0) * a.stride;
@@ -313,6 +318,10 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
       rqv[1] = *reinterpret_cast<const f32x4*>(qr + at + 16);
       nq = a.rq[((int64_t)ci * a.G + g) * L + ut];
     }
+  };
+  auto fetch_cols = [&](int c0, int ci) {
+    const int nl = min(L, len - c0);
+    const float* kr = kb + (int64_t)(start + c0) * a.stride;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       rt[i >> 2][i & 3] = kr[__mul24(min(ta + (i >> 2) * 16 + (i & 3), nl - 1), rs) + tc];
@@ -320,9 +329,9 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) kw[i] = w[(i >> 2) * 16 + (i & 3)];
   };
-  auto park = [&]() {
+  auto park_rows = [&](int w0, int w1) {
 #pragma unroll
-    for (int w = 0; w < (MODE == 1 ? 1 : 2); ++w) {
+    for (int w = w0; w < w1; ++w) {
       const f32x4* v = w ? rqv : rkv;
       const float f = w ? nq : nk;
       float x[8];
@@ -334,6 +343,8 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
 #pragma unroll
       for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(base + i * L * DP) = p[i];
     }
+  };
+  auto park_cols = [&]() {
     // k^T times the weight of its token in the update, tokens permuted: U is the B operand as it lies
     float x[8];
 #pragma unroll
@@ -343,72 +354,103 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(KT + (i * D + tc) * LP + ta * 2) = p[i];
   };
-
-  fetch(0, chunk0);
-  for (int c0 = 0, ci = chunk0; c0 < len; c0 += L, ++ci) {
+  auto split_s = [&](bf16x8 (&sp)[3], int j) {
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = S[2 * j + (i >> 2)][i & 3];
+    split8<3>(x, sp);
+  };
+  struct Own { float v[LT][4]; f32x4 gm[LT]; float gL; };
+  // this lane's v and gammas (rows 4 lg + r of each tile)
+  auto fetch_own = [&](Own& w, int c0, int ci) {
     const int nl = min(L, len - c0);
-    asm volatile("" : "+s"(rs), "+s"(ro));   // row offsets are computed per chunk, not kept
-    park();
-    __syncthreads();
-    const int64_t t0 = start + c0;
-    // this lane's v and gammas (rows 4 lg + r of each tile), and its fragments of W and P
-    const float* vc = vb + t0 * a.stride;
+    const float* vc = vb + (int64_t)(start + c0) * a.stride;
     const float* gc = a.gam + ((int64_t)ci * a.H + h) * L;
-    float v[LT][4];
-    f32x4 gm[LT];
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti) {
-      gm[ti] = *reinterpret_cast<const f32x4*>(gc + ti * 16 + lg * 4);
+      w.gm[ti] = *reinterpret_cast<const f32x4*>(gc + ti * 16 + lg * 4);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        v[ti][r] = vc[__mul24(min(ti * 16 + lg * 4 + r, nl - 1), rs) + vo];
+        w.v[ti][r] = vc[__mul24(min(ti * 16 + lg * 4 + r, nl - 1), rs) + vo];
     }
-    const float gL = gc[nl - 1];
-    const bf16* wp = a.wp + ((int64_t)ci * a.H + h) * 2 * MAT + lr * L + lg * 8;
-    bf16x8 fw[LT][3], fp[LT][3];
+    w.gL = gc[nl - 1];
+  };
+  // W or P of a chunk, to LDS as they lie
+  auto dma = [&](int ci, int mat, bf16* dst) {
+    if (wave < MAT * 2 / 1024)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(a.wp + (((int64_t)ci * a.H + h) * 2 + mat) * MAT + wave * 512 + lane * 8),
+          (__attribute__((address_space(3))) void*)(dst + wave * 512), 16, 0, 0);
+  };
+  auto load_wp = [&](const bf16* m, bf16x8 (&f)[LT][3]) {
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti)
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        fw[ti][i] = *reinterpret_cast<const bf16x8*>(wp + i * L * L + ti * 16 * L);
+        f[ti][i] = *reinterpret_cast<const bf16x8*>(m + i * L * L + wp_unit(ti * 16 + lr, lg) * 8);
+  };
+  auto arrived = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
+  // Staged rows are parked while the last chunk's update runs, columns beside the products with S: k^T is not
+  // read before the barrier between the two.  (After the last chunk the same again: a branch would end the
+  // regions in which vector instructions and MFMAs are interleaved.)
+  Own next;
+  dma(chunk0, 0, Ws);
+  fetch_rows(0, chunk0);
+  fetch_cols(0, chunk0);
+  fetch_own(next, 0, chunk0);
+  park_rows(0, MODE == 1 ? 1 : 2);
+  for (int c0 = 0, ci = chunk0; c0 < len; c0 += L, ++ci) {
+    const int nl = min(L, len - c0);
+    const int cn = c0 + L < len ? c0 + L : c0, cin = c0 + L < len ? ci + 1 : ci;
+    asm volatile("" : "+s"(rs), "+s"(ro));   // row offsets are computed per chunk, not kept
+    arrived();
+    __syncthreads();
+    const int64_t t0 = start + c0;
+    const Own own = next;
+    if (MODE != 1) dma(ci, 1, Ps);
     f32x4 r[LT], rl[LT], o[LT], ol[LT];
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti) r[ti] = rl[ti] = o[ti] = ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < KD; ++j) {
-      float x[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = S[2 * j + (i >> 2)][i & 3];
-      bf16x8 sp[3];
-      split8<3>(x, sp);
-#pragma unroll
-      for (int ti = 0; ti < LT; ++ti) {
-        bf16x8 fa[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-          fa[i] = *reinterpret_cast<const bf16x8*>(Ks + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
-        mm<true, 3, 3>(fa, sp, r[ti], rl[ti]);
-        if (MODE != 1) {
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-            fa[i] = *reinterpret_cast<const bf16x8*>(Qs + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
-          mm<true, 3, 3>(fa, sp, o[ti], ol[ti]);
-        }
-      }
-    }
-    // P, then the next chunk (the last one again at the end: a branch here would make every later
-    // wait one for all loads), land while U is computed
-    if (MODE != 1)
+    // products with S in steps of 32 of its rows, k's and q's in turn: the next step's operands are read, and the
+    // next parts of S made, beside the MFMAs
+    bf16x8 sp[2][3], f[2][LT][3];
+    auto load_rows = [&](bf16x8 (&x)[LT][3], const bf16* m, int j) {
 #pragma unroll
       for (int ti = 0; ti < LT; ++ti)
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-          fp[ti][i] = *reinterpret_cast<const bf16x8*>(wp + MAT + i * L * L + ti * 16 * L);
-    {
-      const bool more = c0 + L < len;
-      fetch(more ? c0 + L : c0, more ? ci + 1 : ci);
+          x[ti][i] = *reinterpret_cast<const bf16x8*>(m + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
+    };
+    load_rows(f[0], Ks, 0);
+    split_s(sp[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < KD; ++j) {
+      const int k = MODE != 1 ? 0 : j & 1;
+      if (MODE != 1) load_rows(f[1], Qs, j);
+      else if (j + 1 < KD) load_rows(f[k ^ 1], Ks, j + 1);
+      if (j + 1 < KD) split_s(sp[(j + 1) & 1], j + 1);
+      if (j == 0) fetch_rows(cn, cin);       // of the next chunk
+      if (j == 1) fetch_own(next, cn, cin);
+      mm3_add<LT>(f[k], sp[j & 1], r, rl);
+      if (j < 2) interleave<12, 4, 2, 1>();
+      else interleave<12, 4, 2>();
+      __builtin_amdgcn_sched_barrier(0);
+      if (MODE != 1) {
+        if (j + 1 < KD) load_rows(f[0], Ks, j + 1);
+        else load_wp(Ws, f[0]);
+        if (j == KD - 2) park_cols();
+        mm3_add<LT>(f[1], sp[j & 1], o, ol);
+        interleave<12, 4, 2>();
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
+    if (MODE == 1) {
+      load_wp(Ws, f[0]);
+      park_cols();
+    }
+    bf16x8 (&fw)[LT][3] = f[0];
     // R, U = W R (rows past the end: W is zero there)
     bf16x8 up[3];
     int bad = L;                             // first token whose value is not finite
@@ -417,7 +459,7 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int ti = i >> 2, e = i & 3;
-        x[i] = __builtin_fmaf(-gm[ti][e], r[ti][e] + rl[ti][e], ident ? 0.f : v[ti][e]);
+        x[i] = __builtin_fmaf(-own.gm[ti][e], r[ti][e] + rl[ti][e], ident ? 0.f : own.v[ti][e]);
       }
       if (nl < L)
 #pragma unroll
@@ -425,13 +467,10 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
           if ((i >> 2) * 16 + lg * 4 + (i & 3) >= nl) x[i] = 0.f;
       bf16x8 rp[3];
       split8<3>(x, rp);
+      f32x4 u[LT];
+      mm3<LT>(fw, rp, u);
 #pragma unroll
-      for (int ti = 0; ti < LT; ++ti) {
-        f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
-        mm<true, 3, 3>(fw[ti], rp, hi, lo);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[ti * 4 + e] = hi[e] + lo[e];
-      }
+      for (int i = 0; i < 8; ++i) x[i] = u[i >> 2][i & 3];
       // A row of R or W that is not finite reaches all rows of U, or all from its own on: the last one
       // shows it.  Then U once more without such rows of R, and without what is not finite itself,
       // before P carries it to the rows before it.
@@ -444,57 +483,90 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           if (tok(i) >= bad) rp[0][i] = rp[1][i] = rp[2][i] = (bf16)0.f;
+        mm3<LT>(fw, rp, u);
 #pragma unroll
-        for (int ti = 0; ti < LT; ++ti) {
-          f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
-          mm<true, 3, 3>(fw[ti], rp, hi, lo);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x[ti * 4 + e] = hi[e] + lo[e];
-        }
+        for (int i = 0; i < 8; ++i) x[i] = u[i >> 2][i & 3];
         bad = min(bad, take_nonfinite(x, L, tok));
       }
       split8<3>(x, up);
     }
-    const bool some_bad = __any(bad < L);
+    const bool some_bad = __builtin_amdgcn_readfirstlane(__any(bad < L));
+    arrived();
+    __syncthreads();                         // k, q and W were read, k^T and P are there
+    dma(cin, 0, Ws);
+    auto load_cols = [&](bf16x8 (&x)[LT][3], int dt) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          x[k][i] = *reinterpret_cast<const bf16x8*>(KT + (i * D + (dt + k) * 16 + lr) * LP + lg * 8);
+    };
+    auto update = [&](int dt) {
+      const int k = dt >> 1 & 1;
+      if (dt + 2 < DT) load_cols(f[k ^ 1], dt + 2);
+      f32x4 t[2];
+      mm3<2>(f[k], up, t);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[dt + i][e] = __builtin_fmaf(S[dt + i][e], own.gL, t[i][e]);
+    };
+    if (MODE != 1) load_wp(Ps, f[1]);
+    load_cols(f[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
     if (MODE != 1) {
-      float* oc = a.out + t0 * os + (int64_t)h * a.dv;
+      f32x4 pu[LT];
+      mm3<LT>(f[1], up, pu);
 #pragma unroll
-      for (int ti = 0; ti < LT; ++ti) {
-        f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
-        mm<true, 3, 3>(fp[ti], up, hi, lo);
+      for (int ti = 0; ti < LT; ++ti)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          o[ti][e] = __builtin_fmaf(gm[ti][e], o[ti][e] + ol[ti][e], hi[e] + lo[e]);
-        if (some_bad)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[ti][e] = ti * 16 + lg * 4 + e >= bad ? NAN : o[ti][e];
-      }
-      if (colok) {
-        const int at = lg * 4 * ro + col;
+        for (int e = 0; e < 4; ++e) o[ti][e] = __builtin_fmaf(own.gm[ti][e], o[ti][e] + ol[ti][e], pu[ti][e]);
+    }
+    fetch_cols(cn, cin);                     // of the next chunk
+    park_rows(0, 1);
+    update(0);
+    update(2);
+    interleave<MODE != 1 ? 36 : 24, 3, 3, 2>();
+    __builtin_amdgcn_sched_barrier(0);
+    if (MODE != 1) {
+      if (some_bad)
 #pragma unroll
         for (int ti = 0; ti < LT; ++ti)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (nl == L || ti * 16 + lg * 4 + e < nl) (oc + (ti * 16 + e) * ro)[at] = o[ti][e];
+          for (int e = 0; e < 4; ++e) {
+            asm volatile("" : "+v"(o[ti][e]));  // a branch, not selects in every chunk
+            if (ti * 16 + lg * 4 + e >= bad) o[ti][e] = NAN;
+          }
+      float* oc = a.out + t0 * os + (int64_t)h * a.dv;
+      const int at = lg * 4 * ro + col;
+      if (colok) {
+        if (nl == L) {
+#pragma unroll
+          for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) (oc + (ti * 16 + e) * ro)[at] = o[ti][e];
+        } else {
+#pragma unroll
+          for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (ti * 16 + lg * 4 + e < nl) (oc + (ti * 16 + e) * ro)[at] = o[ti][e];
+        }
       }
+      park_rows(1, 2);
     }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      bf16x8 fa[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        fa[i] = *reinterpret_cast<const bf16x8*>(KT + (i * D + dt * 16 + lr) * LP + lg * 8);
-      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
-      mm<true, 3, 3>(fa, up, hi, lo);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) S[dt][e] = __builtin_fmaf(S[dt][e], gL, hi[e] + lo[e]);
-    }
+    update(4);
+    update(6);
+    interleave<24, 4, 2>();
+    __builtin_amdgcn_sched_barrier(0);
     if (some_bad)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) S[dt][e] = bad < L ? NAN : S[dt][e];
-    __syncthreads();
+        for (int e = 0; e < 4; ++e) {
+          asm volatile("" : "+v"(S[dt][e]));
+          if (bad < L) S[dt][e] = NAN;
+        }
   }
 
   if (MODE == 1 || MODE == 0 || seg_idx + 1 == seg_count) {
@@ -569,8 +641,11 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
 
 // Chunkwise for 128 key channels where the rows pay (chunk_rows.h; a chunk's workspace is 200 KB for 16
 // heads, which few rows per sequence would multiply, too).  16 x 1000 tokens of 16 heads with 128 x 128
-// states: 1328 us token by token, 296 us chunkwise (70 us for W and P); 2 x 8192: 7.5 ms and 0.8 ms.  The
-// walk issues 1000 vector instructions and 168 MFMAs per wave and chunk: 50 % and 34 % of a SIMD's cycles.
+// states: 1328 us token by token, 261 us chunkwise (45 us for W and P); 2 x 8192: 7.5 ms and 0.73 ms.  Per wave and
+// chunk the walk issues 670 vector instructions and 168 MFMAs in 13700 cycles: 8100 of two waves' issue, 6100 of
+// the LDS that 95 reads of 1 KB per wave keep busy, the rest the barriers and the chain R -> U.  (Products, systems and
+// update each by itself, sums of two MFMAs added afterwards: 1000 vector instructions, 293 us in all; W and P read
+// by every wave from memory: 276.)
 bool delta_chunk_ok(const float* qkv, int P, int Tp, int H, int G, int d, int V) {
   return chunk_rows_pay(P, Tp, 48) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(qkv) & 15) == 0 &&

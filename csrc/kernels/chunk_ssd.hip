@@ -211,17 +211,6 @@ __device__ __forceinline__ void mm3_add(const bf16x8 (&a)[2][3], const bf16x8 (&
       }
 }
 
-// The order of a region's instructions: N times one MFMA, then V vector instructions, which run beside it, and
-// a memory instruction after every M-th (in a burst they would hold up the wave).
-template <int N, int V, int M> __device__ __forceinline__ void interleave() {
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
-    if (i % M == M - 1) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-  }
-}
-
 // 1024 bytes from each wave's 64 lanes to LDS
 __device__ __forceinline__ void dma16(const void* src, void* dst) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
@@ -467,7 +456,7 @@ __global__ __launch_bounds__(NT, 2) void ssd_walk_kernel(const SsdArgs a) {
         }
         mm3_add(fa[ks & 1], sp[ks & 1], o, ol);
         __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
-        interleave<24, 4, 8>();
+        interleave<24, 4, 0, 8>();
         __builtin_amdgcn_sched_barrier(0);
       }
       f32x4 px[LT][2];
@@ -483,7 +472,7 @@ __global__ __launch_bounds__(NT, 2) void ssd_walk_kernel(const SsdArgs a) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) o[ti][c][r] = __builtin_fmaf(o[ti][c][r] + ol[ti][c][r], fin[ti][r], px[ti][c][r]);
       __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-      interleave<24, 4, 8>();
+      interleave<24, 4, 0, 8>();
       __builtin_amdgcn_sched_barrier(0);
       arrived();
       __syncthreads();
@@ -545,9 +534,9 @@ __global__ __launch_bounds__(NT, 2) void ssd_walk_kernel(const SsdArgs a) {
       if (dt > 0) add(dt - 2);
       if (MODE != 1) {
         __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
-        if (dt == 4) interleave<24, 6, 4>();
-        else if (dt == 6) interleave<24, 4, 6>();
-        else interleave<24, 2, 3>();
+        if (dt == 4) interleave<24, 6, 0, 4>();
+        else if (dt == 6) interleave<24, 4, 0, 6>();
+        else interleave<24, 2, 0, 3>();
       }
       __builtin_amdgcn_sched_barrier(0);
     }
