@@ -501,6 +501,41 @@ def test_window_attention_shared_tiles(gpu, dt, H, G, latent, bs, kw):
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
 
 
+@pytest.mark.parametrize("latent", [False, True])
+@pytest.mark.parametrize("at", [0, 4, 8])
+@pytest.mark.parametrize("bs", [1, 7, 32])
+def test_window_attention_output_slices_and_pages(gpu, latent, at, bs):
+    """Prompt rows of shared tiles into column slices of a wider buffer (stores of 16 bytes where the rows
+    allow it, else of 8), pages of one token, of no power of two and of 32: the bits of the plain call on
+    the same keys in pages of 16."""
+    torch.manual_seed(37)
+    H, dk, dv, lens, old = 4, 256 if latent else 128, 192 if latent else 128, [70, 3, 130], [0, 40, 25]
+    T, q = sum(lens), torch.randn(203, H, dk).bfloat16().to(gpu)
+    keys = [torch.randn(a + b, dk).bfloat16().to(gpu) for a, b in zip(lens, old)]
+    vals = [k[:, :dv] if latent else torch.randn(k.shape[0], dv).bfloat16().to(gpu) for k in keys]
+    pos = torch.cat([torch.arange(o, o + a) for a, o in zip(lens, old)]).to(gpu)
+
+    def run(bs, out=None):
+        width = max(k.shape[0] for k in keys) // bs + 1
+        tables = (torch.randperm(3 * width, generator=torch.Generator().manual_seed(bs))).view(3, width)
+        kc = torch.zeros(3 * width, 1, bs, dk, device=gpu, dtype=torch.bfloat16)
+        vc = kc[..., :dv] if latent else torch.zeros(3 * width, 1, bs, dv, device=gpu, dtype=torch.bfloat16)
+        for t, k, v in zip(tables.to(gpu), keys, vals):
+            j = torch.arange(k.shape[0], device=gpu)
+            kc[t[j // bs], 0, j % bs] = k
+            if not latent:
+                vc[t[j // bs], 0, j % bs] = v
+        m = _to(_meta(lens, [a + b for a, b in zip(lens, old)], [], tables.int()), gpu)
+        return ops.window_attention(q, kc, vc, pos, m, 0.08, 50, 3, None, out=out)
+
+    buf = torch.full((T, H * dv + 16), 7.0, device=gpu, dtype=torch.bfloat16)
+    got = run(bs, buf[:, at: at + H * dv])
+    assert torch.equal(got, run(16))
+    rest = torch.ones(H * dv + 16, dtype=torch.bool, device=gpu)
+    rest[at: at + H * dv] = False
+    assert (buf[:, rest] == 7).all()
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("latent", [False, True])
 @pytest.mark.parametrize("cap", [1e6, 1.5])
