@@ -120,10 +120,10 @@ __device__ __forceinline__ double lane63(double x) {
 
 // The products over a chunk multiply a token's value by the masked zeros of the rows before it, which a
 // value that is not finite would reach.  v[i]: token tok(i) of the lane's column (one of the four lanes
-// that share lane & 15).  Such values become zero; returned is the column's first such token, from
+// that share lane & 15; PAIR: of the two that share lane & 31).  Such values become zero; returned is the column's first such token, from
 // which on its outputs and its state have to be made NaN (`none`: every value is finite).  A sum that
 // overflows only costs the closer look.
-template <int N, typename V, typename F>
+template <bool PAIR = false, int N, typename V, typename F>
 __device__ __forceinline__ int take_nonfinite(V (&v)[N], int none, F tok) {
   float z = 0.f;
   if constexpr (sizeof(V) == 2) {            // products with zeros, two at a time
@@ -145,8 +145,13 @@ __device__ __forceinline__ int take_nonfinite(V (&v)[N], int none, F tok) {
         first = min(first, tok(i));
         v[i] = (V)0.f;
       }
-    first = min(first, __shfl_xor(first, 16, 64));
-    first = min(first, __shfl_xor(first, 32, 64));
+    if (PAIR) {
+      const auto p = __builtin_amdgcn_permlane32_swap(first, first, false, false);
+      first = min((int)p[0], (int)p[1]);
+    } else {
+      first = min(first, __shfl_xor(first, 16, 64));
+      first = min(first, __shfl_xor(first, 32, 64));
+    }
   }
   return first;
 }

@@ -23,6 +23,8 @@
 // products of parts whose weight is at least 2^-16 are kept, and the sums are fp32.  bf16
 // inputs are one exact part, f16 inputs two.
 //
+// Most bf16 rows of the mLSTM and SSD heads that share B and C have kernels of their own (chunk_mlstm.hip, chunk_ssd.hip).
+//
 // What bounds it (mLSTM, 4 heads with 256 x 512 states, 64-token chunks): a wave issues 1550 vector
 // instructions per chunk, most of them splitting S, and 222 MFMAs; they fill 42 % and 24 % of a SIMD's
 // cycles (SSD's second walk: 59 % and 26 %).  The rest is barriers and latency that two waves per SIMD do not
@@ -692,8 +694,9 @@ void chunk_dispatch(const ChunkArgs& a, int items, hipStream_t s) {
 }  // namespace
 
 // Segment length for a step of P sequences and Tp tokens whose walk has `wgs` workgroups per
-// sequence (0: sequences are not cut) and the number of segments it can come to.
-static ChunkWork chunk_plan(int P, int Tp, int wgs, int L) {
+// sequence, `least` chunks of L at least (0: sequences are not cut, as those of less than `shortest` chunks on
+// average), and the number of segments it can come to.
+static ChunkWork chunk_plan(int P, int Tp, int wgs, int L, int least, int shortest) {
   ChunkWork p;
   p.items = P;
   // a CU holds one of these workgroups; cut only where a good part of the CUs would idle
@@ -702,8 +705,8 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L) {
   if (P * 2 > want) return p;
   int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
   seg = (seg + L - 1) / L * L;
-  if (seg < 4 * L) seg = 4 * L;
-  if (Tp / P < 2 * seg) return p;
+  if (seg < least * L) seg = least * L;
+  if (Tp / P < 2 * seg || Tp / P < shortest * L) return p;
   p.seg = seg;
   p.items = Tp / seg + P;
   return p;
@@ -721,14 +724,31 @@ bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, 
   return d == 128 ? chunk_form_ok<f16, true, 128, 32, 1>() : chunk_form_ok<f16, true, 256, 32, 1>();
 }
 
+// bf16 rows by DMA in steps of at least 1024 rows or with a sequence long enough to be cut.  This file's kernel -> chunk_mlstm.hip's,
+// us, 4 heads of 256 x 512:
+//   32 x 512, 24 x 700, 16 x 1000, 64 x 20   219 -> 136, 263 -> 147, 206 -> 185, 97 -> 75
+//   1 x 384, 512, 1000, 4000, 2 x 8192       72 -> 59, 74 -> 60, 84 -> 70, 122 -> 101, 318 -> 234
+//   16 x 64, 8 x 256, 4 x 300, 32 x 16       31.4 -> 31.0, 59.5 -> 58.7, 64.0 -> 64.6, 90.0 -> 89.8
+//   8 x 64, 4 x 64, 1 x 64, 1 x 256          23.9 -> 24.3, 22.4 -> 23.1, 20.5 -> 21.4, 52.7 -> 53.9
 ChunkWork mlstm_chunk_plan(int dtype, int P, int Tp, int H, int d, int dv) {
-  return chunk_plan(P, Tp, H * ((dv + 127) / 128), dtype == DT_BF16 ? 64 : 32);
+  if (mlstm_rows_ok(dtype, dv)) {
+    const int cols = mlstm_rows_columns();
+    ChunkWork p = chunk_plan(P, Tp, H * ((dv + cols - 1) / cols), 64, 2, 6);
+    p.rows = p.seg > 0 || Tp >= 1024;
+    if (p.rows) return p;
+  }
+  return chunk_plan(P, Tp, H * ((dv + 127) / 128), dtype == DT_BF16 ? 64 : 32, 4, 8);
 }
 
 void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride, const float* gates,
                         float* S, float* nst, float* mst, const float* n0, const float* m0,
                         const int* qsl, const int* seq_lens, const int* slots, int P, int H, int d,
                         int dv, int num_slots, const ChunkWork& work, hipStream_t s) {
+  if (work.rows) {
+    launch_mlstm_rows(out, qkvg, (const char*)qkvg + 2 * H * d, (const char*)qkvg + 4 * H * d, stride, gates, S, nst, mst,
+                      n0, m0, qsl, seq_lens, slots, P, H, d, dv, num_slots, work, s);
+    return;
+  }
   ChunkArgs a{};
   a.out = out;
   const size_t es = 2;
@@ -767,7 +787,7 @@ bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G) {
 
 ChunkWork ssd_chunk_plan(int P, int Tp, int H, int V, int G) {
   const int hpw = ssd_heads(H, V, G), cols = 16 * (NW / hpw);
-  return chunk_plan(P, Tp, H / hpw * ((V + cols - 1) / cols), 32);
+  return chunk_plan(P, Tp, H / hpw * ((V + cols - 1) / cols), 32, 4, 8);
 }
 
 void launch_ssd_chunk(int dtype, float* out, const float* xbc, const void* dt, int64_t dts,

@@ -357,6 +357,7 @@ void launch_window_prefill_mfma(int dtype, void* out, const void* q, const void*
 // items * H * d * (dv + 1) floats and items * H * 2 doubles
 struct ChunkWork {
   int seg = 0, items = 0;
+  bool rows = false;                         // mLSTM: mlstm_rows_ok's
   float* state = nullptr;
   double* gate = nullptr;
 };
@@ -366,6 +367,13 @@ void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride,
                         float* S, float* nst, float* mst, const float* n0, const float* m0,
                         const int* qsl, const int* seq_lens, const int* slots, int P, int H, int d,
                         int dv, int num_slots, const ChunkWork& work, hipStream_t s);
+// of the calls that mlstm_chunk_ok takes, those whose rows come by DMA (chunk_mlstm.hip)
+bool mlstm_rows_ok(int dtype, int dv);
+int mlstm_rows_columns();                    // value columns of a workgroup
+void launch_mlstm_rows(float* out, const void* q, const void* k, const void* v, int64_t stride, const float* gates,
+                       float* S, float* nst, float* mst, const float* n0, const float* m0, const int* qsl,
+                       const int* seq_lens, const int* slots, int P, int H, int d, int dv, int num_slots,
+                       const ChunkWork& work, hipStream_t s);
 bool ssd_chunk_ok(const float* xbc, int P, int Tp, int H, int V, int N, int G);
 ChunkWork ssd_chunk_plan(int P, int Tp, int H, int V, int G);
 void launch_ssd_chunk(int dtype, float* out, const float* xbc, const void* dt, int64_t dts,

@@ -260,6 +260,42 @@ def test_mlstm_scan_chunkwise(gpu, dt, H, d, dv, lens, before, D_ctx):
         assert ((a.double().cpu() - b).abs() <= 16 * 2.0 ** -24 * u).all()
 
 
+@pytest.mark.parametrize("H,d,dv", [(2, 128, 40), (1, 128, 264), (1, 256, 144), (1, 256, 272), (1, 128, 36)])
+@pytest.mark.parametrize("lens,before,D_ctx", [([1, 15, 16, 17, 63, 64, 65, 129, 660], [0, 5, 0, 40, 0, 0, 9, 0, 3], [9, 1]),
+                                               ([384], [7], []), ([1300, 33, 2], [0, 11, 0], [30])])
+def test_mlstm_scan_rows_by_dma(gpu, H, d, dv, lens, before, D_ctx):
+    """Many rows, and sequences that are cut: whole and ragged chunks, a padding sequence, one and two workgroups
+    per head, the last one's columns in part, segments of two chunks; values not in 16-byte units."""
+    test_mlstm_scan_chunkwise(gpu, torch.bfloat16, H, d, dv, lens, before, D_ctx)
+
+
+@pytest.mark.parametrize("lens,bad", [([45, 700, 400], (1, 333)), ([45, 700, 400], (0, 0)), ([45, 700, 400], (2, 399)),
+                                      ([700, 33], (0, 130)), ([700, 33], (0, 698))])
+def test_mlstm_scan_rows_by_dma_not_finite(gpu, lens, bad):
+    """A value that is not finite reaches its own column from its row on, and nothing else changes by a bit; whole
+    sequences (1145 rows) and segments."""
+    torch.manual_seed(92)
+    H, d, dv, (seq, tok), c = 2, 128, 272, bad, 261
+    m, T, n = _chunk_step(lens, [0, 7, 0][:len(lens)], [])
+    m.state_slots = torch.arange(n, dtype=torch.int32)
+    x, g = torch.randn(T, 2 * H * d + 2 * H * dv).to(torch.bfloat16), torch.cat([torch.randn(T, H), -torch.rand(T, H)], dim=1)
+    st = [torch.randn(n, H, d, dv), torch.randn(n, H, d), torch.rand(n, H)]
+
+    def run():
+        s = tuple(y.to(gpu) for y in st)
+        return ops.mlstm_scan(x.to(gpu), g.to(gpu), s, _to(m, gpu), H, d, dv).cpu().view(T, H, dv), s[0].cpu()
+    want, S_w = run()
+    assert want.isfinite().all() and S_w.isfinite().all()
+    t, end = sum(lens[:seq]) + tok, sum(lens[:seq + 1])
+    x[t, 2 * H * d + dv + c] = float("-inf")
+    got, S = run()
+    hit, hit_S = torch.zeros(T, H, dv, dtype=torch.bool), torch.zeros(n, H, d, dv, dtype=torch.bool)
+    hit[t:end, 1, c] = True
+    hit_S[seq, 1, :, c] = True
+    assert not got[hit].isfinite().any() and torch.equal(got[~hit], want[~hit])
+    assert not S[hit_S].isfinite().any() and torch.equal(S[~hit_S], S_w[~hit_S])
+
+
 def _step_rows(m):
     """(first row, rows, position of the first) of every step sequence."""
     qsl = m.query_start_loc.tolist() if m.num_prefills else [0]
