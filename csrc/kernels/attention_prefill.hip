@@ -33,6 +33,16 @@ constexpr int PF_BN = 64;
 
 __device__ __forceinline__ int kswz(int k) { return (k & 3) | (((k >> 3) & 3) << 2); }
 
+// over the four lanes that share lane & 15, without the LDS's latency (a shuffle's) in the chain
+__device__ __forceinline__ float max_rows(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  x = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  const uint32_t w = __builtin_bit_cast(uint32_t, x);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
 // cos / sin of one row's dims as pf_load_q uses them, loaded ahead of the rotation
 template <int D> struct PfRot { float4 c[D / 64][4]; };   // per fragment pair: cos lo / hi, sin lo / hi
 template <int D>
@@ -145,8 +155,7 @@ __device__ __forceinline__ void pf_wave_tile(const T* __restrict__ K, const T* _
 #pragma unroll
     for (int j = 1; j < 4; ++j)
       tmax = fmaxf(tmax, fmaxf(fmaxf(s[qt][j][0], s[qt][j][1]), fmaxf(s[qt][j][2], s[qt][j][3])));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    tmax = max_rows(tmax);
     tmax *= c;                              // -inf stays -inf (a fully masked row)
     if (__any(tmax > m[qt] + PF_RESCALE_THR)) {
       const float mn = fmaxf(m[qt], tmax);
@@ -575,8 +584,9 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
   constexpr int VPT = D * (PF_BN / 8) / NT_;
   constexpr int TILE = PF_BN * D;
   static_assert(KPT * NT_ == PF_BN * NCH && VPT * NT_ == D * (PF_BN / 8), "staging split");
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  T* lds = reinterpret_cast<T*>(smem);
+  // two objects: the compiler lets an LDS read follow every DMA into the object that it reads
+  __shared__ __attribute__((aligned(16))) T lds[4 * TILE];
+  __shared__ __attribute__((aligned(16))) T all_rows[256 * D];
 
   const int G = nq / nkv;
   const int Y = nkv * (G / GH);
@@ -647,7 +657,7 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
   // 32 rows of its head, 16-byte chunks permuted by the row; afterwards the place where its output
   // rows meet, so that they are stored 256 bytes at a time.
   static_assert(D == 128, "16 chunks per row");
-  T* rows = lds + 4 * TILE + wave * 32 * D;
+  T* rows = all_rows + wave * 32 * D;
   // (the lane index behind an opaque move: addresses that depend on it alone are not kept in
   // registers over the tile loop, where there are none left)
   auto opaque = [](int x) {
@@ -719,17 +729,18 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
     }
   };
   auto store_tile = [&](int buf) {
+    const int tid = opaque(threadIdx.x);
     T* K = lds + buf * 2 * TILE;
     T* V = K + TILE;
 #pragma unroll
     for (int u = 0; u < KPT; ++u) {
-      const int ci = threadIdx.x + NT_ * u;
+      const int ci = tid + NT_ * u;
       const int key = ci / NCH, c = ci % NCH;
       *reinterpret_cast<u32x4*>(K + key * D + ((c ^ (kswz(key) & (NCH - 1))) * 8)) = widen(kreg[u]);
     }
 #pragma unroll
     for (int u = 0; u < VPT; ++u) {
-      const int ci = threadIdx.x + NT_ * u;
+      const int ci = tid + NT_ * u;
       const int c = ci / D, d = ci % D;
       *reinterpret_cast<u32x4*>(V + d * PF_BN + ((c ^ ((d >> 1) & 7)) * 8)) = widen(vreg[u]);
     }
@@ -740,20 +751,17 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
   if (it * G_ >= n_items) return;                 // uniform: the whole workgroup leaves
   fetch_bt(cur.bt, cur.L, 0);
   load_tile(cur.L, cur.h, 0);
+  fetch_bt(cur.bt, cur.L, min(1, cur.n_tiles - 1));
   load_q(cur);
   store_tile(0);
   __syncthreads();
   int buf = 0;
-  bool kb_ready = false;     // kblk / vblk already hold the block ids of this item's tile 1
+  bool ids_ready = cur.n_tiles > 1;          // kblk / vblk already hold the block ids of this item's tile 1
   for (;;) {
     const int nit = next_valid(it + 1, nxt);
     const bool has_next = nit * G_ < n_items;
-    // the block ids of the tile loaded next: this item's tile 1, or the next item's tile 0
-    if (!kb_ready) {
-      if (cur.n_tiles > 1) fetch_bt(cur.bt, cur.L, 1);
-      else if (has_next) fetch_bt(nxt.bt, nxt.L, 0);
-    }
-    kb_ready = false;
+    // an item of one tile: the block ids of the next item's tile 0
+    if (!ids_ready && has_next) fetch_bt(nxt.bt, nxt.L, 0);
     const int wq0 = cur.qbase + wrow;
     const int wave_tiles = (cur.ctx0 + min(wq0 + 31, cur.qlen - 1)) / PF_BN + 1;
     f32x4 o[2][DT];
@@ -763,22 +771,16 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
       for (int t = 0; t < DT; ++t) o[qt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
     for (int kt = 0; kt < cur.n_tiles; ++kt) {
-      // the tile after this one in the stream (this item's kt + 1, else the next item's
-      // tile 0) is loaded while this one computes; then the block ids of the one after it
-      bool loaded = false;
-      if (kt + 1 < cur.n_tiles) {
-        load_tile(cur.L, cur.h, kt + 1);
-        if (kt + 2 < cur.n_tiles) fetch_bt(cur.bt, cur.L, kt + 2);
-        else if (has_next) fetch_bt(nxt.bt, nxt.L, 0);
-        loaded = true;
-      } else if (has_next) {
-        load_tile(nxt.L, nxt.h, 0);
-        if (nxt.n_tiles > 1) {
-          fetch_bt(nxt.bt, nxt.L, 1);
-          kb_ready = true;
-        }
-        loaded = true;
-      }
+      // The tile after this one in the stream (this item's kt + 1, else the next item's tile 0) is loaded
+      // while this one computes; then the block ids of the one after it.  Unconditional (at the end of the
+      // stream the last tile once more): ids that branches merge are copied, and the copy waits for
+      // everything loaded before them, the tile too (whole step, 32 x 512 195 us so and 189 without, 64 x 256
+      // 158 and 150).
+      const bool last = kt + 1 == cur.n_tiles, loaded = !last || has_next, to_next = last && has_next;
+      load_tile(to_next ? nxt.L : cur.L, to_next ? nxt.h : cur.h, to_next ? 0 : min(kt + 1, cur.n_tiles - 1));
+      const bool own = kt + 2 < cur.n_tiles || !has_next;
+      fetch_bt(own ? cur.bt : nxt.bt, own ? cur.L : nxt.L,
+               own ? min(kt + 2, cur.n_tiles - 1) : last ? min(1, nxt.n_tiles - 1) : 0);
       if (kt == 0 && has_next) issue_q(nxt);
       if (kt < wave_tiles) {
         const T* K = lds + buf * 2 * TILE;
@@ -788,8 +790,10 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
         else
           pf_wave_tile<T, D, false>(K, V, qf, o, m, l, qpos, kt * PF_BN, scale_log2, r16, qd);
       }
-      if (loaded) store_tile(buf ^ 1);
-      __syncthreads();
+      if (loaded) {
+        store_tile(buf ^ 1);
+        __syncthreads();
+      }
       buf ^= 1;
     }
     const Item done = cur;
@@ -820,6 +824,7 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
     }
     if (!has_next) break;
     // the next item's first tile is already staged in LDS buffer `buf`
+    ids_ready = nxt.n_tiles > 1;
     cur = nxt;
     it = nit;
   }
@@ -853,11 +858,9 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
   const int mode = prefill_persist_mode();
   const bool dma = reinterpret_cast<uintptr_t>(q) % 16 == 0 && q_stride % 8 == 0;    // 16-byte DMAs
   // one workgroup per CU: launch_bounds(512, 1), 128 KB of LDS (K / V tiles, the waves' q / output rows)
-  constexpr size_t lds_q = lds + 256 * D * sizeof(T);
   const auto walk = &prefill_attn_gqa_persist_kernel<T, D, KV8, GH>;
-  static OncePerDevice once;
-  if (dma && (mode < 0 ? n_items > n_cu : mode != 0) && n_items < ((int64_t)1 << 30) && allow_lds(once, walk, lds_q)) {
-    walk<<<(int)std::min<int64_t>(n_items, n_cu), 512, lds_q, s>>>(
+  if (dma && (mode < 0 ? n_items > n_cu : mode != 0) && n_items < ((int64_t)1 << 30)) {
+    walk<<<(int)std::min<int64_t>(n_items, n_cu), 512, 0, s>>>(
         (const T*)q, (T*)out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, nq, nkv, bs_log2,
         scale_log2, v_scale, num_blocks, q_stride, cos_sin, cs_rows, (int)n_items);
     return;
