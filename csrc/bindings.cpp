@@ -1858,7 +1858,7 @@ void gla_scan(Tensor out, Tensor proj, Tensor low, Tensor a2, Tensor a2_bias, Te
   const bool chunk = kgc::gla_chunk_ok((int)P, (int)Tp, (int)H, (int)d, (int)V, (int)R);
   Tensor ws;
   if (chunk) {
-    ws = at::empty({kgc::gla_chunk_ws((int)P, (int)Tp, (int)H)}, out.options());
+    ws = at::empty({kgc::gla_chunk_ws((int)P, (int)Tp, (int)H, (int)V)}, out.options());
     kgc::launch_gla_chunk(dt_code(proj), out.data_ptr<float>(), proj.data_ptr(), proj.stride(0), low.data_ptr(),
                           low.stride(0), a2p, a2bp, S.data_ptr<float>(), qp, sp, slot, (int)P, (int)Tp, (int)H,
                           (int)V, (int)R, (float)tau, (int)S.size(0), ws.data_ptr<float>(), stream());

@@ -13,12 +13,17 @@
 // Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each, six products of parts, the
 // corrections summed apart; products p and r are kept in double.
 //
-// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 1340 -> 437 us, 250 of them the first
-// launch (two vector operations per pair of tokens and channel; 148 MB written) and 190 the walk (splitting S
-// and reading those 148 MB); 2 x 8192 8140 -> 1590 (one walk per sequence, not cut into segments).  From
-// float64, relative norm: outputs 7.7e-7 -> 7.3e-7, states 1.07e-6 -> 1.03e-6.
+// Few long sequences are cut into segments: one walk makes every segment's contribution from a zero state, a
+// small launch puts the states together in which the segments start, and the second walk has them all.
+//
+// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 303 us, 110 of them the first
+// launch (its LDS let two workgroups share a CU, and scalar LDS reads and shuffles held those up: 250; 148 MB
+// written) and 190 the walk (splitting S and reading those 148 MB); 2 x 8192 472 (one walk per sequence: 1562),
+// 1 x 4000 140 (659); token by token 1340 and 8140.  From float64, relative norm: outputs 7.3e-7, states 1.04e-6.
+#include <type_traits>
 #include "chunk.h"
 #include "chunk_rows.h"
+#include "device.h"
 #include "launch.h"
 
 namespace kgc {
@@ -45,15 +50,29 @@ struct GlaArgs {
   float *qp, *kr;                            // [L][D]
   float* pl;                                 // [D]
   bf16* am;                                  // [3][L][L], columns permuted
+  int seg, items;                            // tokens per segment, a multiple of the chunk (0: not cut)
+  float* seg_state;                          // [items][H][D][dv]: contribution, then state a segment starts from
 };
+
+// sum over eight neighbouring lanes, without the LDS
+__device__ __forceinline__ float sum8(float x) {
+  auto other = [](float y, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  x += other(x, std::integral_constant<int, 0xb1>());     // lanes 1 0 3 2
+  x += other(x, std::integral_constant<int, 0x4e>());     // lanes 2 3 0 1
+  return x + other(x, std::integral_constant<int, 0x141>());   // the eight in reverse
+}
 
 // q p, k r, p_L and A of every chunk: one workgroup per (chunk, head)
 template <typename T>
 __global__ __launch_bounds__(256) void gla_prep_kernel(const GlaArgs a) {
+  // 49 KB, so that three workgroups share a CU: the bottleneck's rows lie where the decays come, A where k was
   __shared__ __align__(16) float qs[L][D], ks[L][D], al[L][D];
-  __shared__ float lw[L][RMAX];
   __shared__ double half[D];
-  __shared__ __align__(16) float X[L][L + 4];
+  static_assert(RMAX <= D && L + 4 <= D, "");
+  float (&lw)[L][D] = al;
+  float (*X)[L + 4] = reinterpret_cast<float (*)[L + 4]>(&ks[0][0]);
   const SegItem it = seg_item(blockIdx.x, a.qsl, a.P, L);
   if (it.seq < 0) return;
   const int h = blockIdx.y, tid = threadIdx.x;
@@ -68,7 +87,20 @@ __global__ __launch_bounds__(256) void gla_prep_kernel(const GlaArgs a) {
     lw[t][j] = to_f(low[t * a.ls + j]);
   }
   const float scale = 1.f / sqrtf((float)D);
-  for (int e = tid; e < L * D; e += 256) {
+  constexpr int V = 16 / sizeof(T);          // elements of 16 bytes
+  if (a.ps % V == 0 && reinterpret_cast<uintptr_t>(a.proj) % 16 == 0) {
+    typedef T TV __attribute__((ext_vector_type(V)));
+    for (int e = tid * V; e < L * D; e += 256 * V) {
+      const int t = e / D, c = e % D;
+      const T* row = proj + min(t, nl - 1) * a.ps + h * D + c;
+      const TV q = *reinterpret_cast<const TV*>(row), k = *reinterpret_cast<const TV*>(row + (int64_t)a.H * D);
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        qs[t][c + i] = t < nl ? to_f(q[i]) * scale : 0.f;
+        ks[t][c + i] = t < nl ? to_f(k[i]) : 0.f;
+      }
+    }
+  } else for (int e = tid; e < L * D; e += 256) {
     const int t = e / D, c = e % D;
     const T* row = proj + t * a.ps + h * D + c;
     qs[t][c] = t < nl ? to_f(row[0]) * scale : 0.f;
@@ -82,13 +114,27 @@ __global__ __launch_bounds__(256) void gla_prep_kernel(const GlaArgs a) {
 #pragma unroll
     for (int i = 0; i < L / 2; ++i) acc[i] = 0.f;
     const float* ar = a.a2 + ((int64_t)h * D + c) * a.R;
-    for (int j = 0; j < a.R; ++j) {
+    int j = 0;
+    if (a.R % 4 == 0)                        // four at a time: a quarter of the LDS reads
+      for (; j < a.R; j += 4) {
+        f32x4 w;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) w[n] = ar[j + n];
+#pragma unroll
+        for (int i = 0; i < L / 2; ++i) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(&lw[min(b + i, nl - 1)][j]);
+#pragma unroll
+          for (int n = 0; n < 4; ++n) acc[i] += w[n] * x[n];
+        }
+      }
+    for (; j < a.R; ++j) {
       const float w = ar[j];
 #pragma unroll
       for (int i = 0; i < L / 2; ++i) acc[i] += w * lw[min(b + i, nl - 1)][j];
     }
     const float bias = a.a2b[h * D + c];
     double p = 1.0;
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < L / 2; ++i) {
       const float x = acc[i] + bias;
@@ -119,28 +165,30 @@ __global__ __launch_bounds__(256) void gla_prep_kernel(const GlaArgs a) {
     }
     if (hf == 0) a.pl[at * D + c] = (float)(first * second);
   }
-  // A: thread (column s, 16 channels) carries k_s times the decays since s
+  // A: thread (column s, channels 32 i + 4 g ..) carries k_s times the decays since s; eight threads read 128
+  // bytes next to each other, and a wave begins at its first column
   {
-    const int s = tid >> 3, g = (tid & 7) * 16;
+    const int s = tid >> 3, g = (tid & 7) * 4;
     float w[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) w[i] = ks[s][g + i];
-    for (int t = 0; t < L; ++t) {
+    for (int i = 0; i < 16; ++i) w[i] = ks[s][(i >> 2) * 32 + g + (i & 3)];
+    const int s0 = __builtin_amdgcn_readfirstlane(s & ~7);
+    __syncthreads();
+    for (int t = 0; t < s0; ++t)
+      if ((tid & 7) == 0) X[t][s] = 0.f;
+    for (int t = s0; t < L; ++t) {
       float a0 = 0.f, a1 = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; i += 4) {
-        const f32x4 d = *reinterpret_cast<const f32x4*>(&al[t][g + i]);
-        const f32x4 q = *reinterpret_cast<const f32x4*>(&qs[t][g + i]);
+        const f32x4 d = *reinterpret_cast<const f32x4*>(&al[t][i * 8 + g]);
+        const f32x4 q = *reinterpret_cast<const f32x4*>(&qs[t][i * 8 + g]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           w[i + e] = t > s ? w[i + e] * d[e] : w[i + e];
           (e & 1 ? a1 : a0) += w[i + e] * q[e];
         }
       }
-      float x = a0 + a1;
-      x += __shfl_xor(x, 1, 64);
-      x += __shfl_xor(x, 2, 64);
-      x += __shfl_xor(x, 4, 64);
+      const float x = sum8(a0 + a1);
       if ((tid & 7) == 0) X[t][s] = t >= s ? x : 0.f;
     }
   }
@@ -158,52 +206,74 @@ __global__ __launch_bounds__(256) void gla_prep_kernel(const GlaArgs a) {
   }
 }
 
-template <typename T>
+// MODE 0: whole sequences; 1: segments from zero (states only); 2: segments from the states that they start in
+template <typename T, int MODE>
 __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
-  __shared__ __align__(16) bf16 Qs[3 * L * DP], KT[3 * D * LP];
+  __shared__ __align__(16) bf16 Qs[MODE == 1 ? 8 : 3 * L * DP], KT[3 * D * LP];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
-  const int seq = blockIdx.x, nct = (a.dv + 127) / 128;
+  const int nct = (a.dv + 127) / 128;
+  int seq = blockIdx.x, seg_idx = 0, seg_count = 1, item = 0;
+  if (MODE != 0) {
+    const SegItem it = seg_item(blockIdx.x, a.qsl, a.P, a.seg);
+    if (it.seq < 0) return;
+    seq = __builtin_amdgcn_readfirstlane(it.seq);
+    seg_idx = __builtin_amdgcn_readfirstlane(it.idx);
+    seg_count = __builtin_amdgcn_readfirstlane(it.count);
+    item = __builtin_amdgcn_readfirstlane(it.first) + seg_idx;
+    if (MODE == 1 && seg_idx + 1 == seg_count) return;
+  }
   const int h = blockIdx.y / nct, ct = blockIdx.y - h * nct;
   const int col = ct * 128 + wave * 16 + lr;
   const bool colok = col < a.dv;
   const int colc = colok ? col : a.dv - 1;                // columns off the edge: read the last
-  const int start = a.qsl[seq], len = a.qsl[seq + 1] - start;
+  int start = a.qsl[seq], len = a.qsl[seq + 1] - start;
   const int pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
   const int64_t os = (int64_t)a.H * a.dv;
+  if (MODE != 0) {
+    start += seg_idx * a.seg;
+    len = min(a.seg, len - seg_idx * a.seg);
+  }
   if (len <= 0) return;
   if (slot < 0 || slot >= a.num_slots || pos0 < 0) {      // padding: defined zeros
-    if (colok)
+    if (MODE != 1 && colok)
       for (int t = lg; t < len; t += 4) a.out[(start + t) * os + (int64_t)h * a.dv + col] = 0.f;
     return;
   }
   f32x4 S[DT];
   float* Ss = a.S + ((int64_t)slot * a.H + h) * D * a.dv;
+  float* mine = a.seg_state + ((int64_t)item * a.H + h) * D * a.dv;
+  const bool own = MODE == 2 && seg_count > 1, zero = MODE == 1 || (pos0 == 0 && !own);
+  const float* from = own ? mine : Ss;
 #pragma unroll
   for (int i = 0; i < DT; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[i][r] = pos0 == 0 ? 0.f : Ss[(i * 16 + 4 * lg + r) * a.dv + colc];
+    for (int r = 0; r < 4; ++r) S[i][r] = zero ? 0.f : from[(i * 16 + 4 * lg + r) * a.dv + colc];
   const T* vb = reinterpret_cast<const T*>(a.proj) + 2 * (int64_t)a.H * D + (int64_t)h * a.dv + colc;
   // Staging: a thread takes 8 columns of one row of q p, and 8 tokens of one column of k r, in both
   // cases the pieces 4 i .. and 16 + 4 i .. of 32: adjacent in the permuted order, one store.
   f32x4 rq[2], rt[2];
   const int ut = tid / 16, uc = (tid % 16 / 4) * 32 + (tid % 4) * 4, up_ = (tid % 16) * 8;
   const int ta = tid / D * 4, tc = tid % D;
-  const int chunk0 = chunks_before<L>(seq, a.qsl);
+  const int chunk0 = chunks_before<L>(seq, a.qsl) + (MODE != 0 ? seg_idx * (a.seg / L) : 0);
   auto fetch = [&](int ci) {
     const int64_t at = ((int64_t)ci * a.H + h) * L * D;
-    rq[0] = *reinterpret_cast<const f32x4*>(a.qp + at + ut * D + uc);
-    rq[1] = *reinterpret_cast<const f32x4*>(a.qp + at + ut * D + uc + 16);
+    if (MODE != 1) {
+      rq[0] = *reinterpret_cast<const f32x4*>(a.qp + at + ut * D + uc);
+      rq[1] = *reinterpret_cast<const f32x4*>(a.qp + at + ut * D + uc + 16);
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) rt[i >> 2][i & 3] = a.kr[at + (ta + (i >> 2) * 16 + (i & 3)) * D + tc];
   };
   auto park = [&]() {
     float x[8];
     bf16x8 p[3];
+    if (MODE != 1) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = rq[i >> 2][i & 3];
-    split8<3>(x, p);
+      for (int i = 0; i < 8; ++i) x[i] = rq[i >> 2][i & 3];
+      split8<3>(x, p);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(Qs + i * L * DP + ut * DP + up_) = p[i];
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(Qs + i * L * DP + ut * DP + up_) = p[i];
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = rt[i >> 2][i & 3];
     split8<3>(x, p);
@@ -223,6 +293,7 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[ti][r] = vb[(t0 + min(ti * 16 + lg * 4 + r, nl - 1)) * a.ps];
     bf16x8 fp[LT][3];
+    if (MODE != 1)
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti)
 #pragma unroll
@@ -234,6 +305,7 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
     f32x4 o[LT], ol[LT];
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti) o[ti] = ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (MODE != 1)
 #pragma unroll
     for (int j = 0; j < KD; ++j) {
       float x[8];
@@ -263,6 +335,7 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
     }
     const bool some_bad = __any(bad < L);
     float* oc = a.out + t0 * os + (int64_t)h * a.dv + col;
+    if (MODE != 1)
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti) {
       f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
@@ -294,17 +367,67 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
         for (int e = 0; e < 4; ++e) S[dt][e] = bad < L ? NAN : S[dt][e];
     __syncthreads();
   }
-  if (colok)
+  float* dst = MODE == 1 ? mine : Ss;
+  if (colok && (MODE != 2 || seg_idx + 1 == seg_count))
 #pragma unroll
     for (int i = 0; i < DT; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) Ss[(i * 16 + 4 * lg + r) * a.dv + col] = S[i][r];
+      for (int r = 0; r < 4; ++r) dst[(i * 16 + 4 * lg + r) * a.dv + col] = S[i][r];
+}
+
+// ---- the states in which segments start, in place of the contributions: one element per thread ------------
+__global__ __launch_bounds__(256) void gla_chain_kernel(const GlaArgs a) {
+  const int seq = blockIdx.z, h = blockIdx.y, lane = threadIdx.x & 63;
+  const int len = a.qsl[seq + 1] - a.qsl[seq], pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
+  if (len <= a.seg || slot < 0 || slot >= a.num_slots || pos0 < 0) return;
+  int first = 0;                             // segments of the sequences before this one
+  for (int p = lane; p < seq; p += 64) first += max(1, (a.qsl[p + 1] - a.qsl[p] + a.seg - 1) / a.seg);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) first += __shfl_xor(first, o, 64);
+  const int count = (len + a.seg - 1) / a.seg, per = a.seg / L, sh = D * a.dv;
+  const int chunk0 = chunks_before<L>(seq, a.qsl);
+  const int at = blockIdx.x * 256 + threadIdx.x;
+  if (at >= sh) return;
+  const int64_t step = (int64_t)a.H * sh;
+  const float* pl = a.pl + ((int64_t)chunk0 * a.H + h) * D + at / a.dv;
+  float* p = a.seg_state + ((int64_t)first * a.H + h) * sh + at;
+  float S = pos0 == 0 ? 0.f : a.S[((int64_t)slot * a.H + h) * sh + at];
+  for (int j = 0; j < count - 1; ++j) {
+    const float c = p[j * step];
+    double f = 1.0;                          // the segment's decay
+#pragma unroll 8
+    for (int k = 0; k < per; ++k) f *= pl[(int64_t)(j * per + k) * a.H * D];
+    p[j * step] = S;
+    S = __builtin_fmaf((float)f, S, c);
+  }
+  p[(count - 1) * step] = S;
 }
 
 template <typename T>
 void run(const GlaArgs& a, int chunks, hipStream_t s) {
   gla_prep_kernel<T><<<dim3(chunks, a.H), 256, 0, s>>>(a);
-  gla_walk_kernel<T><<<dim3(a.P, a.H * ((a.dv + 127) / 128)), NT, 0, s>>>(a);
+  const int y = a.H * ((a.dv + 127) / 128);
+  if (a.seg <= 0) {
+    gla_walk_kernel<T, 0><<<dim3(a.P, y), NT, 0, s>>>(a);
+  } else {
+    gla_walk_kernel<T, 1><<<dim3(a.items, y), NT, 0, s>>>(a);
+    gla_chain_kernel<<<dim3((D * a.dv + 255) / 256, a.H, a.P), 256, 0, s>>>(a);
+    gla_walk_kernel<T, 2><<<dim3(a.items, y), NT, 0, s>>>(a);
+  }
+}
+
+// Tokens per segment (0: not cut) and a bound of their number: few sequences leave CUs idle, one workgroup
+// on each, over the whole walk.
+int plan(int P, int Tp, int H, int V, int* items) {
+  *items = P;
+  const int wgs = H * ((V + 127) / 128), want = (device_cus() + wgs - 1) / wgs;
+  if (P * 2 > want) return 0;
+  int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
+  seg = (seg + L - 1) / L * L;
+  if (seg < 4 * L) seg = 4 * L;
+  if (Tp / P < 2 * seg) return 0;
+  *items = Tp / seg + P;
+  return seg;
 }
 
 }  // namespace
@@ -315,8 +438,10 @@ bool gla_chunk_ok(int P, int Tp, int H, int d, int V, int R) {
          chunk_fits(0, (long)H * V, (long)H * ((V + 127) / 128));   // (row offsets have 64 bits)
 }
 // floats of workspace
-int64_t gla_chunk_ws(int P, int Tp, int H) {
-  return (int64_t)(Tp / L + P) * H * (2 * L * D + D + MAT / 2);
+int64_t gla_chunk_ws(int P, int Tp, int H, int V) {
+  int items;
+  const int64_t states = plan(P, Tp, H, V, &items) > 0 ? (int64_t)items * H * D * V : 0;
+  return (int64_t)(Tp / L + P) * H * (2 * L * D + D + MAT / 2) + states;
 }
 void launch_gla_chunk(int dtype, float* out, const void* proj, int64_t ps, const void* low, int64_t ls,
                       const float* a2, const float* a2b, float* S, const int* qsl, const int* seq_lens,
@@ -331,6 +456,8 @@ void launch_gla_chunk(int dtype, float* out, const void* proj, int64_t ps, const
   a.kr = a.qp + (int64_t)chunks * H * L * D;
   a.pl = a.kr + (int64_t)chunks * H * L * D;
   a.am = reinterpret_cast<bf16*>(a.pl + (int64_t)chunks * H * D);
+  a.seg = plan(P, Tp, H, V, &a.items);
+  a.seg_state = ws + (int64_t)chunks * H * (2 * L * D + D + MAT / 2);
   if (dtype == DT_BF16) run<bf16>(a, chunks, s);
   else if (dtype == DT_F16) run<f16>(a, chunks, s);
   else run<float>(a, chunks, s);

@@ -487,7 +487,7 @@ int decay_scan_max_rows();
 int gla_scan_max_rank();
 // prompt rows chunkwise (chunk_gla.hip); ws: gla_chunk_ws floats, 16-byte aligned
 bool gla_chunk_ok(int P, int Tp, int H, int d, int V, int R);
-int64_t gla_chunk_ws(int P, int Tp, int H);
+int64_t gla_chunk_ws(int P, int Tp, int H, int V);
 void launch_gla_chunk(int dtype, float* out, const void* proj, int64_t ps, const void* low, int64_t ls,
                       const float* a2, const float* a2b, float* S, const int* qsl, const int* seq_lens,
                       const int* slots, int P, int Tp, int H, int V, int R, float tau, int num_slots,

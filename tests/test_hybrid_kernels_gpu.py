@@ -840,6 +840,22 @@ def test_gla_scan_chunkwise(gpu, dt, H, V, R, lens, before, D_ctx):
             assert _whole(got, want) and _whole(st, S)
 
 
+@pytest.mark.parametrize("dt,R", [(torch.bfloat16, 16), (torch.float16, 7), (torch.float32, 4)])
+def test_gla_scan_long_segments(gpu, dt, R):
+    """Segments of seven chunks, the last one short, beside a sequence that is not cut, on two workgroups per
+    head; ranks in and out of fours, rows in 16-byte units and not.  Decays near one: what the segments hand on
+    stays in the sums."""
+    torch.manual_seed(82)
+    H, d, V = 8, 128, 144
+    m, T, n = _chunk_step([3000, 40], [5, 0], [3])
+    terms, run = _gla_case(T, n, H, d, V, R, dt, 4.0, gpu, 8.0)
+    want, unit, S, SA = _matrix64(m, *terms)
+    st = terms[0].to(gpu)
+    got = run(st, _to(m, gpu))
+    assert ((got.cpu() - want).abs() <= (d + 64) * unit + 1e-30).all()
+    assert ((st.cpu() - S).abs() <= 128 * SA + 1e-30).all()
+
+
 @pytest.mark.parametrize("op,dt", [("mlstm", torch.bfloat16), ("mlstm", torch.float16), ("ssd", torch.bfloat16),
                                    ("delta", torch.bfloat16), ("gla", torch.bfloat16), ("gla", torch.float32)])
 @pytest.mark.parametrize("where,val", [("v", float("nan")), ("v", float("-inf")), ("k", float("nan")), ("gate", float("nan"))])
