@@ -25,6 +25,7 @@
 // 130 -> 113, capped and causal 288 -> 260.  (A ring of four tiles filled by LDS-DMA three tiles ahead: 249 us where
 // this took 229.)
 #include "device.h"
+#include "chunk.h"
 #include "window.h"
 #include <type_traits>
 
@@ -217,7 +218,39 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
       f32x16 s[NB];
       float mx = -INFINITY;
       __builtin_amdgcn_sched_barrier(0);
-      if (NB == 2) next();
+      if (NB == 2 && CAP) next();
+      if constexpr (NB == 2 && !CAP) {
+        // S^T, four products at a time and the operands of the next four on their way; beside the first ones the next
+        // tile's addresses and loads (operands read just in time: 8 x 2048 189.3 -> 187.5 us, 1 x 8192 130 -> 126)
+        V8 kf[2][4];
+        const T* krow = Kt + (st * NB * 32 + col) * KST + 8 * hh;
+        auto load_k = [&](int g) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            kf[g & 1][i] = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(krow + (g * 4 / KS) * 32 * KST + 16 * (g * 4 % KS + i)));
+        };
+        static_assert(KS % 4 == 0, "");
+        load_k(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < NB * KS / 4; ++g) {
+          const int b = g * 4 / KS;
+          if (g + 1 < NB * KS / 4) load_k(g + 1);
+          if (g == 0) next();
+          if (g * 4 % KS == 0)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[b][i] = 0.f;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[b] = mfma32x32x16(kf[g & 1][i], qf[g * 4 % KS + i], s[b]);
+          if (g == KS / 4 + 1)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[0][i]);
+          __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+          interleave<4, 8, 0, 1>();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else
 #pragma unroll
       for (int b = 0; b < NB; ++b) {         // S^T; beside a block's products the maximum of the one before it
         const T* krow = Kt + ((st * NB + b) * 32 + col) * KST + 8 * hh;
@@ -256,17 +289,6 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-      }
-      if (NB == 2 && !CAP) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-        for (int i = 0; i < NB * KS; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          if (i % 2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
       }
       // keys that all are there, not after the wave's first row and inside the window of its last
       // are seen by every row: no test per element
