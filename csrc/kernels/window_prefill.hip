@@ -345,16 +345,27 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
       __builtin_amdgcn_sched_barrier(0);
       // ---- O^T += V^T P^T, 16 keys at a time, the next ones' weights beside the products: lane (col, hh) holds
       // column 32 t + col of keys 4 hh .. and 8 + 4 hh ..
+      constexpr bool AHEAD = NB == 2 && !CAP;             // values one product ahead, where registers are left
+      V8 vf[2];
+      auto load_v = [&](int n) {             // 16 keys n / DT, columns n % DT
+        const T* vrow = Vt + ((st * NB * 32) + 16 * (n / DT) + 4 * hh + (r16 >> 2)) * VST + 16 * (col >> 4) + 4 * (r16 & 3) + 32 * (n % DT);
+        const u32x2 a = ld_tr4(vrow), b = ld_tr4(vrow + 8 * VST);
+        vf[n & 1] = __builtin_bit_cast(V8, (u32x4{a[0], a[1], b[0], b[1]}));
+      };
+      if (AHEAD) {
+        load_v(0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int j = 0; j < 2 * NB; ++j) {
-        const T* vrow = Vt + ((st * NB * 32) + 16 * j + 4 * hh + (r16 >> 2)) * VST + 16 * (col >> 4) + 4 * (r16 & 3);
         if (j + 1 < 2 * NB) weigh(j + 1);
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
-          const u32x2 a = ld_tr4(vrow + 32 * t), b = ld_tr4(vrow + 8 * VST + 32 * t);
-          const V8 fr = __builtin_bit_cast(V8, (u32x4{a[0], a[1], b[0], b[1]}));
-          o[t] = mfma32x32x16(fr, pl[j], o[t]);
-          o[t] = mfma32x32x16(fr, ph[j], o[t]);
+          const int n = j * DT + t;
+          if (!AHEAD) load_v(n);
+          else if (n + 1 < 2 * NB * DT) load_v(n + 1);
+          o[t] = mfma32x32x16(vf[n & 1], pl[j], o[t]);
+          o[t] = mfma32x32x16(vf[n & 1], ph[j], o[t]);
         }
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
