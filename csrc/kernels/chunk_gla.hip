@@ -16,10 +16,11 @@
 // Few long sequences are cut into segments: one walk makes every segment's contribution from a zero state, a
 // small launch puts the states together in which the segments start, and the second walk has them all.
 //
-// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 303 us, 110 of them the first
+// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 259 us, 110 of them the first
 // launch (its LDS let two workgroups share a CU, and scalar LDS reads and shuffles held those up: 250; 148 MB
-// written) and 190 the walk (splitting S and reading those 148 MB); 2 x 8192 472 (one walk per sequence: 1562),
-// 1 x 4000 140 (659); token by token 1340 and 8140.  From float64, relative norm: outputs 7.3e-7, states 1.04e-6.
+// written) and 145 the walk (splitting S beside the MFMAs, operands a step ahead: 190 without, and reading those
+// 148 MB); 2 x 8192 410 (one walk per sequence: 1562), 1 x 4000 127 (659); token by token 1340 and 8140.  From
+// float64, relative norm: outputs 7.3e-7, states 1.04e-6.
 #include <type_traits>
 #include "chunk.h"
 #include "chunk_rows.h"
@@ -299,27 +300,43 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
 #pragma unroll
       for (int i = 0; i < 3; ++i)
         fp[ti][i] = *reinterpret_cast<const bf16x8*>(a.am + at * MAT + i * L * L + (ti * 16 + lr) * L + lg * 8);
-    f32x4 pl[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) pl[dt] = *reinterpret_cast<const f32x4*>(a.pl + at * D + dt * 16 + 4 * lg);
     f32x4 o[LT], ol[LT];
+    bf16x8 fa[2][2][3];                      // two row tiles, a step ahead
+    if (MODE != 1) {
 #pragma unroll
-    for (int ti = 0; ti < LT; ++ti) o[ti] = ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (MODE != 1)
+      for (int ti = 0; ti < LT; ++ti) o[ti] = ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
+      bf16x8 sp[2][3];                       // parts of 32 rows of S, likewise
+      auto load_q = [&](int j) {
 #pragma unroll
-    for (int j = 0; j < KD; ++j) {
-      float x[8];
+        for (int ti = 0; ti < LT; ++ti)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = S[2 * j + (i >> 2)][i & 3];
-      bf16x8 sp[3];
-      split8<3>(x, sp);
+          for (int i = 0; i < 3; ++i)
+            fa[j & 1][ti][i] = *reinterpret_cast<const bf16x8*>(Qs + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
+      };
+      auto split_s = [&](int j) {
+        float x[8];
 #pragma unroll
-      for (int ti = 0; ti < LT; ++ti) {
-        bf16x8 fa[3];
+        for (int i = 0; i < 8; ++i) x[i] = S[2 * j + (i >> 2)][i & 3];
+        split8<3>(x, sp[j & 1]);
+      };
+      load_q(0);
+      split_s(0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-          fa[i] = *reinterpret_cast<const bf16x8*>(Qs + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
-        mm<true, 3, 3>(fa, sp, o[ti], ol[ti]);
+      for (int j = 0; j < KD; ++j) {
+        if (j + 1 < KD) {
+          load_q(j + 1);
+          split_s(j + 1);
+        }
+        f32x4 main[LT];                      // (rounded into its sum once per step)
+#pragma unroll
+        for (int ti = 0; ti < LT; ++ti) main[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
+        mm3_add(fa[j & 1], sp[j & 1], main, ol);
+#pragma unroll
+        for (int ti = 0; ti < LT; ++ti) o[ti] += main[ti];
+        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+        interleave<12, 4>();
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
     fetch(c0 + L < len ? ci + 1 : ci);       // (the last one again at the end: no branch)
@@ -349,17 +366,34 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
         if (colok && t < nl) oc[t * os] = (o[ti][e] + hi[e]) + (ol[ti][e] + lo[e]);
       }
     }
+    f32x4 u[2][2], lo[2][2], pl[2][2];       // products of two row tiles, their corrections and decays
+    auto load_k = [&](int q) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      bf16x8 fa[3];
+      for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
-        fa[i] = *reinterpret_cast<const bf16x8*>(KT + (i * D + dt * 16 + lr) * LP + lg * 8);
-      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
-      mm<true, 3, 3>(fa, vp, hi, lo);
+        for (int i = 0; i < 3; ++i)
+          fa[q & 1][t][i] = *reinterpret_cast<const bf16x8*>(KT + (i * D + (2 * q + t) * 16 + lr) * LP + lg * 8);
+        pl[q & 1][t] = *reinterpret_cast<const f32x4*>(a.pl + at * D + (2 * q + t) * 16 + 4 * lg);
+      }
+    };
+    auto add = [&](int q) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[dt][e] = __builtin_fmaf(S[dt][e], pl[dt][e], hi[e] + lo[e]);
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[2 * q + t][e] = __builtin_fmaf(S[2 * q + t][e], pl[q & 1][t][e], u[q & 1][t][e] + lo[q & 1][t][e]);
+    };
+    load_k(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < DT / 2; ++q) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) u[q & 1][t] = lo[q & 1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      mm3_add(fa[q & 1], vp, u[q & 1], lo[q & 1]);
+      if (q > 0) add(q - 1);
+      if (q + 1 < DT / 2) load_k(q + 1);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    add(DT / 2 - 1);
     if (some_bad)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
