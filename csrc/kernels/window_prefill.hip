@@ -21,8 +21,8 @@
 // of 16 x 16 x 32, the same work: four), so the next keys' weights, the maximum and the next tile's addresses stand
 // between them in the order given below.  8 x 2048 rows, window 1024: per tile and wave 48 MFMAs and 380 vector
 // instructions, 4000 cycles of two waves' issue of the 5800 that a tile takes; the rest is the barrier, and 3.5
-// rounds of workgroups that take 4.  196 us in MFMAs of 16 x 16 x 32, 184 so; 32 x 512 rows 92 -> 82, latent rows
-// 130 -> 113, capped and causal 288 -> 260.  (A ring of four tiles filled by LDS-DMA three tiles ahead: 249 us where
+// rounds of workgroups that take 4.  197 us in MFMAs of 16 x 16 x 32, 178 so; 32 x 512 rows 92 -> 77, latent rows
+// 130 -> 114, capped and causal 288 -> 254.  (A ring of four tiles filled by LDS-DMA three tiles ahead: 249 us where
 // this took 229.)
 #include "device.h"
 #include "chunk.h"
