@@ -1,6 +1,7 @@
 """HIP kernels of the hybrid decoders against their fp32 PyTorch references
 (``ops.reference``), op by op, in bf16 and fp32, on sizes that are not multiples of the
 wave (odd head sizes, several norm groups, chunks that continue a slot's state)."""
+import math
 import types
 
 import pytest
@@ -535,6 +536,46 @@ def test_window_attention_shared_tiles(gpu, dt, H, G, latent, bs, kw):
                                0.08, args[1], args[2], gate.to(gpu), elem_gate=eg.to(gpu), out_scale=1.3, **kw)
     ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
+
+
+def _rounded_once(got, want, unit, eps):
+    """got (16 bits) within half a unit in its last place of want (float64), and eps of ``unit`` for the arithmetic."""
+    bits, low = (7, -126) if got.dtype == torch.bfloat16 else (10, -14)
+    half = torch.exp2(torch.floor(torch.log2(want.abs().clamp_min(2.0 ** low))) - bits - 1)
+    return ((got.double().cpu() - want).abs() <= half + eps * unit).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("latent", [False, True])
+@pytest.mark.parametrize("lo,hi", [(6.0, 7.9), (8.5, 12.0)])
+def test_window_attention_later_maximum(gpu, dt, latent, lo, hi):
+    """Prompt rows that see one key of score 0 in their first tile, one of 2^lo to 2^hi times its weight in a later
+    one, and no others to speak of: sums that are not zero move to a new maximum, and the weight that decides
+    the result is exact (a pair of bf16 holds 17 bits of any other: 2^-18).  16 units of 2^-24 cover the
+    fp32 steps: sums, exponents of the first key (its share is at most 2^-6), division, gate, scale."""
+    torch.manual_seed(38)
+    H, dk, dv, n, rows, old, bs = 4, 256 if latent else 128, 192 if latent else 128, 8, 128, 130, 16
+    width = (rows + old) // bs + 1
+    tables = torch.randperm(n * width).view(n, width).int()
+    k, v = torch.zeros(n, width * bs, dk), torch.randn(n, width * bs, dv).to(dt)
+    k[..., -1] = -16.0
+    k[:, 0, -1], k[:, 100, -1] = 0.0, 1.0
+    if latent:
+        k[..., :dv] = v.float()
+    kc = torch.empty(n * width, 1, bs, dk, dtype=dt)
+    kc[tables.long(), 0] = k.to(dt).view(n, width, bs, dk)
+    vc = torch.empty(n * width, 1, bs, dv, dtype=dt)
+    vc[tables.long(), 0] = v.view(n, width, bs, dv)
+    q, scale = torch.zeros(n * rows, H, dk).to(dt), 0.5
+    q[..., -1] = ((lo + torch.rand(n * rows, H) * (hi - lo)) * math.log(2) / scale).to(dt)
+    w = torch.exp(scale * q[..., -1].double())[..., None]
+    v0, v1 = (v[:, j].double().repeat_interleave(rows, 0)[:, None] for j in (0, 100))
+    want, unit = (v0 + w * v1) / (1 + w), (v0.abs() + w * v1.abs()) / (1 + w)
+    m = _to(_meta([rows] * n, [rows + old] * n, [], tables), gpu)
+    pos = torch.arange(old, old + rows).repeat(n).to(gpu)
+    kg = kc.to(gpu)
+    got = ops.window_attention(q.to(gpu), kg, kg[..., :dv] if latent else vc.to(gpu), pos, m, scale, 0, 0)
+    assert _rounded_once(got.view(-1, H, dv), want, unit, 16 * 2.0 ** -24)
 
 
 @pytest.mark.parametrize("latent", [False, True])
