@@ -61,11 +61,6 @@ __device__ __forceinline__ float tanh_far(float y) {
   return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(y * 2.88539008177792681f));
 }
 
-// a 16-bit gate's: within 3e-7 of itself for |x| < 3, 2e-6 beyond (the result is rounded to 16 bits)
-__device__ __forceinline__ float sigmoid(float x) {
-  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.44269504088896340736f));
-}
-
 // KS: dk / 16; DT: dv / 32; NB: blocks of 32 keys per softmax step (fewer: fewer registers); ALIAS: values
 // are the first dv columns of the key rows
 template <typename T, int KS, int DT, int NB, bool ALIAS, bool CAP>
@@ -404,13 +399,13 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
 #pragma unroll
         for (int k = 0; k < 4; ++k) e[k].u = *reinterpret_cast<const u32x2*>(eg + 32 * d + 8 * k);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[d][i] *= sigmoid(to_f(e[i >> 2].h[i & 3]));
+        for (int i = 0; i < 16; ++i) o[d][i] *= gate_sigmoid(to_f(e[i >> 2].h[i & 3]));
       }
     } else {
 #pragma unroll
       for (int d = 0; d < DT; ++d)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[d][i] *= sigmoid(to_f(eg[32 * d + 8 * (i >> 2) + (i & 3)]));
+        for (int i = 0; i < 16; ++i) o[d][i] *= gate_sigmoid(to_f(eg[32 * d + 8 * (i >> 2) + (i & 3)]));
     }
   }
   // the halves of the wave trade columns: 16 bytes of a row per lane

@@ -578,6 +578,26 @@ def test_window_attention_later_maximum(gpu, dt, latent, lo, hi):
     assert _rounded_once(got.view(-1, H, dv), want, unit, 16 * 2.0 ** -24)
 
 
+@pytest.mark.parametrize("at", [8, 1])
+def test_window_attention_one_gate(gpu, at):
+    """Rows that see themselves only give their value times the gate's sigmoid: prompt and decode rows the same
+    bits, from gates that can be read four at a time and not.  fp32: an exponent rounded at |x| log2 e (60 units of
+    2^-24), the exponential's 2, a sum, a quotient and two products.  (f16: a product and its rounding can be one step.)"""
+    torch.manual_seed(39)
+    H, d, T, bs, dt, low = 4, 128, 2048, 16, torch.bfloat16, -60.0
+    v = torch.randn(T, d).to(dt)
+    kc, vc = torch.zeros(T // bs, 1, bs, d, dtype=dt), v.view(T // bs, 1, bs, d)
+    eg = (torch.rand(T, H * d + at) * (3 - low) + low).to(dt)
+    tables = torch.arange(T // bs).view(1, -1).int()
+    run = lambda m: ops.window_attention(   # noqa: E731
+        torch.zeros(T, H, d, device=gpu, dtype=dt), kc.to(gpu), vc.to(gpu), torch.arange(T, device=gpu), _to(m, gpu),
+        1.0, 1, 0, elem_gate=eg.to(gpu)[:, at:])
+    got = run(_meta([T], [T], [], tables))
+    assert torch.equal(got, run(_meta([], [], list(range(1, T + 1)), tables.expand(T, -1))))
+    want = v.double()[:, None] * torch.sigmoid(eg[:, at:].double()).view(T, H, d)
+    assert _rounded_once(got.view(T, H, d), want, want.abs(), (6 - low) * 2.0 ** -24)
+
+
 @pytest.mark.parametrize("latent", [False, True])
 @pytest.mark.parametrize("at", [0, 4, 8])
 @pytest.mark.parametrize("bs", [1, 7, 32])
