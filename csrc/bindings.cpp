@@ -1403,7 +1403,7 @@ void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
                       std::optional<Tensor> gate, bool fast, double softcap, double out_scale,
                       std::optional<Tensor> elem_gate, int64_t pool, int64_t block_size,
                       std::optional<Tensor> v_table, bool interleaved,
-                      std::optional<Tensor> slots, bool chunked, double sink) {
+                      std::optional<Tensor> slots, bool chunked, double sink, int64_t max_ctx) {
   check_gpu(q, "q");
   c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
   TORCH_CHECK(q.dim() == 3 && q.is_contiguous() && act_dtype(q), "kgc.window_attention: q [T, H, dk]");
@@ -1529,7 +1529,7 @@ void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
   if (fast && aligned && D > 0 &&
       kgc::window_decode_mfma_ok(dt, (int)dk, (int)dv, (int)(H / G), ex)) {
     const int Z = kgc::window_split_pieces((int)D, (int)H, (int)G, (int)dk, (int)dv, (int)bts, bs,
-                                             (int)window, (int)keep_first);
+                                           (int)window, (int)keep_first, max_ctx);
     if (Z > 0) {
       Tensor work = at::empty({kgc::window_split_floats((int)D, (int)H, (int)dv, Z)},
                               q.options().dtype(at::kFloat));
@@ -2689,7 +2689,7 @@ TORCH_LIBRARY(kgc, m) {
         "Tensor? seq_lens, Tensor? pbt, Tensor? ctx_lens, Tensor? dbt, Tensor? work_seq, Tensor? work_blk, "
         "int P, int D, int Tp, float scale, int window, int keep_first, Tensor? gate, bool fast, "
         "float softcap, float out_scale, Tensor? elem_gate, int pool, int block_size, "
-        "Tensor? v_table, bool interleaved, Tensor? slots, bool chunked, float sink) -> ()");
+        "Tensor? v_table, bool interleaved, Tensor? slots, bool chunked, float sink, int max_ctx=0) -> ()");
   m.def("mlstm_scan(Tensor(a!) out, Tensor qkvg, Tensor gates, Tensor(b!) S, Tensor(c!) n, Tensor(d!) m, "
         "Tensor? qsl, Tensor? seq_lens, Tensor? ctx_lens, Tensor slots, int P, int D, int Tp, int H, int d, "
         "int dv) -> ()");

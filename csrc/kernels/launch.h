@@ -330,8 +330,10 @@ void launch_window_decode_mfma(int dtype, void* out, const void* q, const void* 
                                int bt_stride, int Tp, int D, int H, int G, int dk, int dv, int krs,
                                int vrs, int bs, int num_blocks, float scale, int window,
                                int keep_first, const float* gate, WindowExtra ex, hipStream_t s);
-// decode rows of small steps: their keys in pieces (0: one workgroup per row and kv head is better)
-int window_split_pieces(int D, int H, int G, int dk, int dv, int bt_stride, int bs, int window, int keep_first);
+// decode rows of small steps: their keys in pieces (0: one workgroup per row and kv head is better); max_ctx: no
+// context is longer, 0 where that is not known
+int window_split_pieces(int D, int H, int G, int dk, int dv, int bt_stride, int bs, int window, int keep_first,
+                        int64_t max_ctx);
 int64_t window_split_floats(int D, int H, int dv, int Z);
 void launch_window_split(int dtype, void* out, const void* q, const void* k_cache, const void* v_cache,
                          const int* ctx_lens, const int* dbt, int bt_stride, int Tp, int D, int H, int G,

@@ -263,25 +263,33 @@ void split_dispatch(const SplitArgs& a, int D, hipStream_t s) {
 
 }  // namespace
 
-// Pieces per row, from what the tables can hold (contexts are on the device).  The second launch costs 1.5
-// us, so steps whose tables hold up to 4 chunks stay whole where a workgroup has 16 waves for them (128 / 128),
-// and so do steps with workgroups for a quarter of the CUs.  One workgroup per row and kv head -> pieces, us:
-//   128 / 128, 4 kv heads   1 x 64: 6.7 -> 8.3, 2 x 200: 9.5 -> 8.6, 1 x 1000: 17.4 -> 8.9, 1 x 8192: 84 -> 13.4
-//                           8 x 4000: 48 -> 21, 16 x 128: 8.1 -> 8.9, 16 x 1000: 19.9 -> 14.4, 24 x 200: 9.8 ->
-//                           10.0, 24 x 1000: 20.4 -> 19.3, 32 x 2000: 31 -> 33
-//   256 / 192 latent rows   1 x 128: 13.1 -> 8.5, 1 x 1000: 27.2 -> 9.7, 64 x 300: 17.5 -> 14.4, 64 x 1000:
-//                           29.3 -> 21.2, 128 x 500: 21.2 -> 22.0
-// A row whose table is long and whose context is not pays the second launch for nothing: 2 x 128 7.9 -> 8.5.
+// Pieces per row, from the longest context where the caller knows it, else from what the tables can hold (the contexts
+// are on the device).  The second launch costs 1.5 us and workgroups without keys some more, so steps of few
+// keys stay whole where a workgroup has 16 waves for them (128 / 128): up to 6 chunks of 32, 8 where that makes more
+// than 768 workgroups and 12 from 1600 on (the CUs hold 1024 and take the rest later).  So do steps with workgroups for a
+// quarter of the CUs.  One workgroup per row and kv head -> pieces, us:
+//   128 / 128, 4 kv heads, window 1024, 33 (32) pieces whatever the contexts
+//     1 x 64, 128, 200, 400, 1000      5.8 -> 7.4, 6.9 -> 7.6, 8.5 -> 7.7, 12.2 -> 7.9, 17.6 -> 7.8
+//     8 x 64, 160, 200, 256, 1000      5.8 -> 8.1, 7.6 -> 8.3, 8.4 -> 8.4, 9.1 -> 8.4, 17.4 -> 10.8
+//     16 x 64, 256, 320, 400, 1000     5.8 -> 10.9, 9.2 -> 11.2, 10.6 -> 11.5, 12.3 -> 11.6, 18.3 -> 13.4
+//   pieces for the longest context: 4 x 160, 256 7.5 -> 7.8, 9.1 -> 7.9; 16 x 200, 256, 320 8.5 -> 8.5, 9.2 -> 9.1, 10.5 -> 9.3
+//   long tables: 1 x 8192 84 -> 13.4, 8 x 4000 48 -> 21, 24 x 200 9.8 -> 10.0, 24 x 1000 20.4 -> 19.3, 32 x 2000 31 -> 33
+//   256 / 192 latent rows (8 waves, one chunk 4 us)   1 x 20, 128, 1000: 10.9 -> 7.8, 12.9 -> 8.1, 27.2 -> 9.7; 64 x 64,
+//                           300, 1000: 11.8 -> 12.2 (9.4 where the contexts are known), 17.5 -> 14.4, 29.3 -> 21.2; 128 x 500: 21.2 -> 22.0
 // Waves in all: 2048 (1024 of the wide form, whose registers leave one per SIMD); 16 x 4000 with 1024, 2048, 4096:
 // 42.0, 32.8, 33; 64 latent x 1000 with 1024, 2048: 21.2, 25.4.
-int window_split_pieces(int D, int H, int G, int dk, int dv, int bt_stride, int bs, int window, int keep_first) {
+int window_split_pieces(int D, int H, int G, int dk, int dv, int bt_stride, int bs, int window, int keep_first,
+                        int64_t max_ctx) {
   const bool wide = dk > 128 || dv > 128;
   const int64_t wgs = (int64_t)D * G * ((H / G + 15) / 16);
   int64_t keys = (int64_t)bt_stride * bs;
+  if (max_ctx > 0) keys = std::min(keys, max_ctx);
   if (window > 0) keys = std::min<int64_t>(keys, (int64_t)window + keep_first);
   const int64_t chunks = (keys + 31) / 32;
-  if (wgs > 64 || chunks < (wide ? 2 : 5)) return 0;
-  return (int)std::min<int64_t>(std::min<int64_t>(chunks, SPLIT_MAX), (wide ? 1024 : 2048) / wgs);
+  if (wgs > 64 || chunks <= 0) return 0;
+  const int64_t pieces = std::min<int64_t>(std::min<int64_t>(chunks, SPLIT_MAX), (wide ? 1024 : 2048) / wgs);
+  const int64_t all = wgs * pieces;
+  return wide || chunks > (all <= 768 ? 6 : all < 1600 ? 8 : 12) ? (int)pieces : 0;
 }
 
 int64_t window_split_floats(int D, int H, int dv, int Z) { return (int64_t)D * H * Z * (dv + 2); }

@@ -40,6 +40,11 @@ def graph_buckets(max_bs: int) -> list[int]:
     return sorted({x for x in b if x <= max_bs} | {max_bs})
 
 
+# Longest contexts for which decode graphs of few rows are captured once more: up to the first their windowed
+# attention is one launch, up to the second its pieces are few (csrc/kernels/window_split.hip has the times)
+SHORT_CTX = (192, 384)
+
+
 @dataclasses.dataclass
 class StepPlan:
     T: int                 # tokens
@@ -147,6 +152,8 @@ class ModelRunner:
         if hasattr(model, "prepare"):
             model.prepare(rope_len + 1, max_tokens, device)
         self.graphs: dict[int, tuple] = {}
+        # (bucket, bound) -> the graph of steps whose contexts are no longer (SHORT_CTX)
+        self.short_graphs: dict[tuple[int, int], tuple] = {}
         self.graph_pool = None
         self.sample_out = torch.zeros(max_num_seqs, dtype=torch.int64, device=device)
         self.processor = LogitsProcessor(max_num_seqs, mcfg.vocab_size, device)
@@ -252,6 +259,7 @@ class ModelRunner:
         """Drop the KV arena, decode graphs and workspaces (engine shutdown): a process
         that builds a second engine must get the memory back."""
         self.graphs = {}
+        self.short_graphs = {}
         self.graph_pool = None
         self.kv = None
         self.kv_caches = []
@@ -481,6 +489,7 @@ class ModelRunner:
         if D:
             m.decode_block_tables = d32[L.dbt:L.dbt + D * mb].view(D, mb)
             m.decode_ctx_lens = d32[L.ctx:L.ctx + D]
+            m.decode_max_ctx = max_ctx
             if self.cache_layout is None:
                 m.decode_workspace = self.workspace
                 nkv = self.model.local_kv_heads()
@@ -614,7 +623,7 @@ class ModelRunner:
             torch.index_select(self.last_tok, 0, self.d64[L.dslots:L.dslots + n],
                                out=self.d64[L.ids + plan.Tp:L.ids + plan.Tp + n])
         if graph:
-            g, logits = self.graphs[plan.B]
+            g, logits = self._graph_of(plan.B, plan.max_ctx)
             link = self.pp_link
             if link is not None:
                 link.pre_replay(plan.B)     # host link: this step's input rows (no-op: IPC)
@@ -671,6 +680,20 @@ class ModelRunner:
         else:
             self._last_lp = None
         return res
+
+    def _graph_of(self, B: int, max_ctx: int) -> tuple:
+        for bound in SHORT_CTX:
+            if max_ctx <= bound and (B, bound) in self.short_graphs:
+                return self.short_graphs[B, bound]
+        return self.graphs[B]
+
+    def _short_bounds(self, B: int) -> list[int]:
+        """Context bounds for which bucket B has graphs of their own.  The windowed decode kernels of up to 64
+        (row, kv head) pairs are chosen by the longest context, which a captured step does not know."""
+        heads = [g for g, _, _, pool in map(self._cache_entry, self.cache_layout or []) if not pool]
+        # (stages of a pipeline keep one graph per bucket: its hand-off has rows for one)
+        whole = self.model.first and self.model.last
+        return [b for b in SHORT_CTX if b < self.max_model_len] if whole and heads and B * min(heads) <= 64 else []
 
     def _plan_thresholds(self, plan: StepPlan) -> bool:
         """Does any sampled row of this step use top-k / top-p (host-side blobs)?"""
@@ -820,9 +843,9 @@ class ModelRunner:
         self.d32.copy_(self.h32)
         torch.cuda.synchronize()
         self.graph_pool = torch.cuda.graph_pool_handle()
-        for B in sorted(self.buckets, reverse=True):
+        for B, bound in [(B, b) for B in sorted(self.buckets, reverse=True) for b in (*self._short_bounds(B), 0)]:
             z = ops.decode_grid_z(B, nkv, self.max_model_len)
-            meta = self._meta(B, 0, 0, B, 0, self.max_model_len, z=z)
+            meta = self._meta(B, 0, 0, B, 0, bound or self.max_model_len, z=z)
 
             def step_body(B=B, meta=meta):
                 # PP stages: receive from the previous stage / send to the next one as
@@ -842,6 +865,9 @@ class ModelRunner:
             g = torch.cuda.CUDAGraph()
             with torch.cuda.graph(g, pool=self.graph_pool):
                 logits = step_body()
-            self.graphs[B] = (g, logits)
+            if bound:
+                self.short_graphs[B, bound] = (g, logits)
+            else:
+                self.graphs[B] = (g, logits)
         torch.cuda.synchronize()
         return time.time() - t0

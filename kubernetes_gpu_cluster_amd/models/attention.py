@@ -33,6 +33,7 @@ class AttnMetadata:
     # decode part
     decode_block_tables: Optional[torch.Tensor] = None    # [D, max_blocks] int32
     decode_ctx_lens: Optional[torch.Tensor] = None        # [D] int32
+    decode_max_ctx: int = 0                               # no decode context is longer (0: not known)
     decode_grid_z: int = 1
     decode_workspace: Optional[tuple] = None
     # prefill-only TP step split into two token halves for comm/compute overlap:

@@ -774,7 +774,8 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                           float(softcap), float(out_scale), elem_gate, int(pool),
                           int(block_size), v_table, interleaved,
                           meta.slot_mapping if pool > 0 else None, chunked,
-                          float("-inf") if sink is None else float(sink))
+                          float("-inf") if sink is None else float(sink),
+                          int(getattr(meta, "decode_max_ctx", 0)))
     return out
 
 

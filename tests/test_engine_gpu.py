@@ -453,6 +453,36 @@ def test_fp8_kv_engine_graphs(gpu):
         assert abs(top_a[0][1] - b.logprobs[0][2][0][1]) < 0.15
 
 
+def test_decode_graphs_by_longest_context(gpu):
+    """Windowed layers: a decode bucket has graphs for short contexts beside the one for all; steps that grow
+    past both bounds give the logits of the same steps run eagerly."""
+    from kubernetes_gpu_cluster_amd.engine.config import EngineConfig
+    from kubernetes_gpu_cluster_amd.engine.llm_engine import LLMEngine
+    from kubernetes_gpu_cluster_amd.engine.model_runner import SHORT_CTX
+    from kubernetes_gpu_cluster_amd.engine.replay import TraceReplayer
+    toks = torch.randint(3, 1000, (400,), generator=torch.Generator().manual_seed(5)).tolist()
+    out = []
+    for eager in (False, True):
+        eng = LLMEngine(EngineConfig(model="tiny-dilavik", random_init=True, seed=3, device="cuda", dtype="bfloat16",
+                                     max_model_len=512, max_num_seqs=2, max_num_batched_tokens=512,
+                                     num_gpu_blocks_override=40, cuda_graph_max_bs=2, enforce_eager=eager))
+        r = eng.executor.runner
+        if not eager:
+            assert sorted(r.short_graphs) == [(b, c) for b in (1, 2) for c in SHORT_CTX]
+            pick = [r._graph_of(1, c) for c in (1, 192, 193, 384, 385, 512)]
+            a, b = r.short_graphs[1, 192], r.short_graphs[1, 384]
+            assert [g is w for g, w in zip(pick, (a, a, b, b, r.graphs[1], r.graphs[1]))] == [True] * 6
+        rp = TraceReplayer(eng)
+        rows = [rp.step([{"id": "x", "tokens": toks[:185], "want": [184]}])]
+        rows += [rp.step([{"id": "x", "tokens": [t], "want": [0]}], ["x"] if i == 214 else None)
+                 for i, t in enumerate(toks[185:])]
+        assert r.stats["graph_steps"] == (0 if eager else 215)
+        out.append(torch.cat(rows).cpu())
+        eng.shutdown()
+    err = (out[0] - out[1]).norm(dim=1) / out[1].norm(dim=1)
+    assert float(err.max()) < 2e-2                 # (the two choose their GEMMs by themselves)
+
+
 def _rccl_capture_worker(port):
     import os
     import torch.distributed as dist

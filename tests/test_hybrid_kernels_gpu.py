@@ -879,6 +879,35 @@ def test_window_decode_in_pieces(gpu, dt, H, G, dk, dv, latent, lens, kw):
     torch.testing.assert_close(got[live], want[live], rtol=1.01 * ulp, atol=2e-4)
 
 
+@pytest.mark.parametrize("rows,longest,pieces,latent", [
+    (1, 192, 0, False), (1, 193, 7, False), (8, 256, 8, False), (12, 1000, 32, False), (16, 192, 0, False),
+    (16, 384, 12, False), (16, 0, 32, False), (17, 4000, 0, False), (3, 30, 1, True), (64, 70, 3, True)])
+def test_window_decode_pieces_follow_the_longest_context(gpu, rows, longest, pieces, latent):
+    """A step whose longest context is known is split by it, not by tables that hold 4096 keys: one launch and no
+    workspace up to six chunks (four key/value heads a row; latent rows always); the results are those of a table as long as the
+    contexts, whichever route they take."""
+    torch.manual_seed(74)
+    H, G, dk, d, bs, width, dt = (16, 1, 256, 192, 32, 128, torch.bfloat16) if latent else (16, 4, 128, 128, 32, 128, torch.bfloat16)
+    lens = [max(1, min(longest or 300, 4000) - 7 * i) for i in range(rows)]
+    tables = torch.randint(0, 200, (rows, width), dtype=torch.int32)
+    kc, vc = (torch.randn(200, G, bs, dk).to(dt).to(gpu) for _ in range(2))
+    vc = kc[..., :d] if latent else vc
+    q, pos = torch.randn(rows, H, dk).to(dt).to(gpu), (torch.tensor(lens) - 1).to(gpu)
+
+    def run(m, out):
+        m = _to(m, gpu)
+        count = lambda: torch.cuda.memory_stats()["requested_bytes.all.allocated"]   # noqa: E731
+        before = count()
+        ops.window_attention(q, kc, vc, pos, m, 0.09, 1024, 0, out=out)
+        return count() - before
+    m = _meta([], [], lens, tables)
+    m.decode_max_ctx = longest
+    got, want = torch.empty(rows, H * d, dtype=dt, device=gpu), torch.empty(rows, H * d, dtype=dt, device=gpu)
+    assert run(m, got) == rows * H * pieces * (d + 2) * 4
+    run(_meta([], [], lens, tables[:, : max(lens) // bs + 1].contiguous()), want)
+    torch.testing.assert_close(got.float(), want.float(), rtol=1.01 * 2.0 ** -7, atol=2e-4)
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,V,R", [(2, 64, 5), (1, 144, 16), (3, 40, 1)])
 @pytest.mark.parametrize("lens,before,D_ctx", CHUNKS)
