@@ -619,37 +619,67 @@ template <bool PAIRS> void walk(const SsdArgs& a, int grid, hipStream_t s) {
 // heads per workgroup
 int heads_per_wg(int H, int V, int G) { return V <= 64 && (H / G) % 2 == 0 ? 2 : 1; }
 
+// workgroups of a sequence's walk
+int walk_wgs(int H, int V, int G) { return H / heads_per_wg(H, V, G) * (heads_per_wg(H, V, G) == 2 ? 1 : (V + 127) / 128); }
+
 }  // namespace
 
-// Of the calls that ssd_chunk_ok takes: at least four heads to a group (a chunk's image, 52 KB per group, is
-// written and read once more), and more than short prompts, which save the second launch.  chunk_scan.hip -> this in us:
-//   32 heads of 128 x 64, 1, 4, 8 and 16 groups, 2 x 8192 tokens   356 -> 222, 358 -> 258, 366 -> 317, 368 -> 459
-//   16 heads of 128 x 128, 4 groups, 32 x 512                      206 -> 171
-//   one group: 32 x 512 199 -> 151, 64 x 48 82 -> 62, 1 x 4000 109 -> 87, 8 x 128 29.9 -> 28.4, 8 x 96 24.1 -> 24.5,
-//   1 x 64 15.9 -> 19.5
-bool ssd_shared_ok(int P, int Tp, int H, int V, int G) {
-  const int hpw = heads_per_wg(H, V, G), wpi = H / hpw * (hpw == 2 ? 1 : (V + 127) / 128);
-  return H / G >= 4 && G + (H + 7) / 8 <= 65535 && (Tp > 112 * P || (int64_t)P * wpi > device_cus());
-}
-
+// Segments for two workgroups per CU, of at least four chunks.  Sequences of two to three segments are cut only where
+// every workgroup then has a CU of its own: the second walk's start costs 13 us (32 heads of 128 x 64, one group, whole ->
+// cut: 1 x 256, 272, 340 42.0 -> 46.0, 45.8 -> 44.1, 53.0 -> 44.5; 4 x 300, 380 50.3 -> 52.8, 58.0 -> 52.3; 8 x 300 51 -> 67).
 SsdWork ssd_shared_plan(int P, int Tp, int H, int V, int G) {
   SsdWork w;
   w.items = P;
   const int64_t chunks = Tp / L + P;
   w.bytes = chunks * G * IMG + chunks * H * (int64_t)sizeof(TokenRec);
-  const int hpw = heads_per_wg(H, V, G), wpi = H / hpw * (hpw == 2 ? 1 : (V + 127) / 128);
-  const int want = (2 * device_cus() + wpi - 1) / wpi;    // items for two workgroups per CU
+  const int cus = device_cus(), wpi = walk_wgs(H, V, G), want = (2 * cus + wpi - 1) / wpi;   // items for two workgroups per CU
   if (P * 2 > want) return w;
   int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
   seg = (seg + L - 1) / L * L;
   if (seg < 4 * L) seg = 4 * L;
-  if (Tp / P < 3 * seg) return w;
+  const int rows = Tp / P;
+  const int64_t wgs = (int64_t)P * ((rows + seg - 1) / seg) * wpi;
+  if (rows < 3 * seg && (wgs > cus || rows <= 2 * seg + (2 * wgs > cus ? 2 * L : 0))) return w;
   w.seg = seg;
   w.items = Tp / seg + P;
   w.state_at = w.bytes;
   w.gate_at = w.state_at + 4 * (int64_t)w.items * H * D * V;
   w.bytes = w.gate_at + 8 * (int64_t)w.items * H;
   return w;
+}
+
+// Of the calls that ssd_chunk_ok takes: at least four heads to a group, and rows enough for the images (52 KB per chunk
+// and group, written and read once more) and the launch that makes them.  chunk_scan.hip, one workgroup per CU where
+// this has two -> this, in us, 128 x 64 and (V 128) 128 x 128 states; a sequence has 16 workgroups:
+//   workgroups for up to all CUs: from four chunks a sequence on, from six where there are many images or heads of 128
+//   columns; which of the two walks is cut into segments decides between 256 and 1000 rows
+//     32 heads, 1 group    1 x 96, 144, 256, 1000   21.1 -> 22.6, 32.4 -> 30.3, 45.2 -> 42.0, 58 -> 51; 16 x 500 98 -> 79
+//                          (not cut here) 4 x 300, 380 50.1 -> 50.3, 52.8 -> 58.0
+//     32 heads, 4 groups   1 x 128, 144, 256   26.7 -> 27.5, 32.5 -> 31.6, 45.2 -> 43.2; 4 x 128 27.8 -> 29.2; 16 x 500 99 -> 89
+//                          cut: 1 x 340, 1000 45.6 -> 45.8, 58 -> 52; 4 x 380 51 -> 54; 3 x 700 62 -> 66
+//     V 128, 2 groups      1 x 128, 144, 200   25.1 -> 26.8, 30.4 -> 30.7, 40.6 -> 38.6; cut: 1 x 340 43.7 -> 44.9, 3 x 700 61 -> 64
+//     V 128, 8 heads, 1 group   1 x 128, 200   24.9 -> 25.8, 40.5 -> 36.9; cut: 1 x 300, 500 42.5 -> 41.1, 45.9 -> 43.7; 4 x 300 44.9 -> 47.4
+//   for more: from a second chunk on, with few images also one that is full
+//     1 group   17 x 20, 33 20.9 -> 21.0, 26.1 -> 22.7; 20 x 20 21.5 -> 22.4; 33 x 20, 48 30.9 -> 28.9, 50 -> 38; 256 x 20 154 -> 137
+//     4 groups  24 x 20 21.7 -> 23.7, 48 x 20 32.1 -> 34.0, 17 x 33 26.5 -> 24.7, 64 x 60 66 -> 55; V 128 32 x 64 33.6 -> 34.7
+//   an image for less than four workgroups (32 heads, 8 groups): where half the CUs are idle, or the images stay in the caches
+//     4 x 160, 256 33.1 -> 34.9, 51 -> 45; 16 x 200, 500 47 -> 51, 99 -> 116; 20 x 40 32.7 -> 33.4, 30 x 100 56 -> 48; 64 x 33,
+//     64, 120 56 -> 46, 67 -> 63, 112 -> 115
+//   2 x 8192, 32 heads, 1, 4, 8 and 16 groups   356 -> 222, 358 -> 258, 366 -> 317, 368 -> 459
+bool ssd_shared_ok(int P, int Tp, int H, int V, int G) {
+  if (H / G < 4 || G + (H + 7) / 8 > 65535) return false;
+  const int wpi = walk_wgs(H, V, G), cus = device_cus();
+  const int64_t wgs = (int64_t)P * wpi;
+  const bool light = G <= 2 && V <= 64, whole = wpi >= 4 * G;     // few images; shared by four workgroups
+  const auto rows = [&](int n) { return Tp > n * (int64_t)P; };
+  if (wgs <= cus) {
+    if (!(whole || 2 * wgs <= cus) || !rows(light ? 112 : 160)) return false;
+    const int seg = ssd_shared_plan(P, Tp, H, V, G).seg;
+    if (seg == 0) return !rows(256) || ssd_chunk_plan(P, Tp, H, V, G).seg == 0;
+    return rows(999) || ((light || G == 1) && (P <= 2 || rows(3 * seg - 1)));
+  }
+  if (!whole) return rows(wgs > 2 * cus ? 24 : 80) && ((int64_t)Tp / L + P) * G * IMG <= 96 << 20;
+  return rows(V > 64 && G > 2 && wgs <= 2 * cus ? 64 : 24) || (G <= 2 && wgs > 2 * cus);
 }
 
 void launch_ssd_shared(int dtype, float* out, const float* xbc, const void* dt, int64_t dts,
@@ -675,8 +705,7 @@ void launch_ssd_shared(int dtype, float* out, const float* xbc, const void* dt, 
   a.seg_state = reinterpret_cast<float*>(w + work.state_at);
   a.seg_gate = reinterpret_cast<double*>(w + work.gate_at);
   ssd_prep_kernel<<<dim3(chunks, G + (H + 7) / 8), NT, 0, s>>>(a);
-  const int wpi = H / a.hpw * (a.hpw == 2 ? 1 : (V + 127) / 128);
-  const int grid = (work.items + 7) / 8 * 8 * wpi;
+  const int grid = (work.items + 7) / 8 * 8 * walk_wgs(H, V, G);
   if (V % 2 == 0) walk<true>(a, grid, s);
   else walk<false>(a, grid, s);
 }

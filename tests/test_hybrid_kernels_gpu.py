@@ -370,6 +370,31 @@ def test_ssd_scan_shared_images(gpu, H, G, V, lens, before, D_ctx):
     test_ssd_scan_chunkwise(gpu, torch.bfloat16, H, G, V, lens, before, D_ctx)
 
 
+@pytest.mark.parametrize("H,G,V", [(4, 1, 144), (4, 1, 131), (8, 1, 200), (8, 2, 33)])
+@pytest.mark.parametrize("lens,before,D_ctx", [([256, 250, 0, 33, 255, 256, 254], [0, 7, 0, 0, 9, 0, 64], [5]),
+                                               ([1500, 1001], [33, 0], []), ([300], [2], []), ([335, 290], [0, 70], [])])
+def test_ssd_scan_shared_images_long(gpu, H, G, V, lens, before, D_ctx):
+    """The same for heads of more than 64 columns, which take longer prompts there, and for prompts that are
+    cut into two segments and a rest."""
+    test_ssd_scan_chunkwise(gpu, torch.bfloat16, H, G, V, lens, before, D_ctx)
+
+
+@pytest.mark.parametrize("G,P,n,allocs", [(1, 1, 113, 1), (1, 20, 20, 0), (8, 20, 20, 0), (8, 256, 20, 0), (1, 33, 20, 1), (4, 17, 33, 1),
+                                          (8, 4, 128, 0), (8, 16, 500, 0), (8, 33, 100, 1), (1, 1, 300, 1), (8, 1, 300, 2),
+                                          (1, 4, 300, 2), (8, 1, 1000, 1)])
+def test_ssd_scan_routes(gpu, G, P, n, allocs):
+    """Steps that pay for images of their chunks and steps that do not (csrc/kernels/chunk_ssd.hip has the times), told
+    by their workspaces: none, one for the images and segments, two for segments alone."""
+    H, V, d = 32, 64, 128
+    m = _to(_meta([n] * P, [n] * P, [], torch.zeros(P, 1, dtype=torch.int32), list(range(P))), gpu)
+    x, g = torch.zeros(P * n, H * V + 2 * G * d, device=gpu), torch.zeros(P * n, H, device=gpu).bfloat16()
+    z, S = torch.zeros(H, device=gpu), torch.zeros(P, H, d, V, device=gpu)
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]   # noqa: E731
+    before = count()
+    ops.ssd_scan(x, g, z, z, z, S, m, H, V, d, G)
+    assert count() - before == 1 + allocs                # (and the outputs)
+
+
 @pytest.mark.parametrize("op,dt", [("mlstm", torch.bfloat16), ("mlstm", torch.float16), ("ssd", torch.bfloat16)])
 def test_scan_segments_start_from_the_incoming_state(gpu, op, dt):
     """Continued prompts that are cut into segments, while products on another stream hold
