@@ -603,24 +603,41 @@ def test_window_attention_later_maximum(gpu, dt, latent, lo, hi):
     assert _rounded_once(got.view(-1, H, dv), want, unit, 16 * 2.0 ** -24)
 
 
+@pytest.mark.parametrize("dt,low,mag", [(torch.bfloat16, -60.0, 1.0), (torch.float16, -10.0, 1024.0)])
+@pytest.mark.parametrize("decode", [False, True])
 @pytest.mark.parametrize("at", [8, 1])
-def test_window_attention_one_gate(gpu, at):
-    """Rows that see themselves only give their value times the gate's sigmoid: prompt and decode rows the same
-    bits, from gates that can be read four at a time and not.  fp32: an exponent rounded at |x| log2 e (60 units of
-    2^-24), the exponential's 2, a sum, a quotient and two products.  (f16: a product and its rounding can be one step.)"""
+def test_window_attention_one_gate(gpu, dt, low, mag, decode, at):
+    """Rows that see themselves only give their value times the gate's sigmoid, in prompt and decode rows, from gates
+    that can be read four at a time and not: 6 units of 2^-24 (the sigmoid's 3, three products) and one rounding
+    to 16 bits.  A gate per head spreads the results between 16-bit values."""
     torch.manual_seed(39)
-    H, d, T, bs, dt, low = 4, 128, 2048, 16, torch.bfloat16, -60.0
-    v = torch.randn(T, d).to(dt)
+    H, d, T, bs = 4, 128, 2048, 16
+    v = (torch.randn(T, d) * mag).to(dt)
     kc, vc = torch.zeros(T // bs, 1, bs, d, dtype=dt), v.view(T // bs, 1, bs, d)
-    eg = (torch.rand(T, H * d + at) * (3 - low) + low).to(dt)
+    eg, gate = (torch.rand(T, H * d + at) * (3 - low) + low).to(dt), torch.rand(T, H) + 0.5
     tables = torch.arange(T // bs).view(1, -1).int()
-    run = lambda m: ops.window_attention(   # noqa: E731
-        torch.zeros(T, H, d, device=gpu, dtype=dt), kc.to(gpu), vc.to(gpu), torch.arange(T, device=gpu), _to(m, gpu),
-        1.0, 1, 0, elem_gate=eg.to(gpu)[:, at:])
-    got = run(_meta([T], [T], [], tables))
-    assert torch.equal(got, run(_meta([], [], list(range(1, T + 1)), tables.expand(T, -1))))
-    want = v.double()[:, None] * torch.sigmoid(eg[:, at:].double()).view(T, H, d)
-    assert _rounded_once(got.view(T, H, d), want, want.abs(), (6 - low) * 2.0 ** -24)
+    m = _meta([], [], list(range(1, T + 1)), tables.expand(T, -1)) if decode else _meta([T], [T], [], tables)
+    got = ops.window_attention(torch.zeros(T, H, d, device=gpu, dtype=dt), kc.to(gpu), vc.to(gpu),
+                               torch.arange(T, device=gpu), _to(m, gpu), 1.0, 1, 0, gate.to(gpu),
+                               elem_gate=eg.to(gpu)[:, at:])
+    want = v.double()[:, None] * torch.sigmoid(eg[:, at:].double()).view(T, H, d) * gate.double()[..., None]
+    assert _rounded_once(got.view(T, H, d), want, want.abs(), 6 * 2.0 ** -24)
+
+
+def test_window_attention_gate_ends(gpu):
+    """Gates at the ends of the range: one, zero, the smallest sigmoids and NaN."""
+    x = torch.tensor([200.0, 88.0, 0.0, -87.5, -100.0, -103.0, -105.0, -3e38, float("inf"), float("-inf"), float("nan")])
+    H, d, T = 4, 128, 128
+    eg = x.bfloat16().repeat(T * H * d // len(x) + 1)[: T * H * d].view(T, H * d)
+    v = torch.full((T // 16, 1, 16, d), 2.0 ** 100).bfloat16().to(gpu)
+    m = _to(_meta([T], [T], [], torch.arange(T // 16).view(1, -1).int()), gpu)
+    got = ops.window_attention(torch.zeros(T, H, d, device=gpu).bfloat16(), torch.zeros_like(v), v,
+                               torch.arange(T, device=gpu), m, 1.0, 1, 0, elem_gate=eg.to(gpu)).cpu()
+    want = torch.sigmoid(eg.double()) * 2.0 ** 100
+    assert (got.isnan() == eg.isnan()).all()
+    # (below 2^-126 a sigmoid has 2^-149 as its unit)
+    ok = (got.double() - want).abs() <= want * 2.0 ** -8 * 1.001 + 2.0 ** -49
+    assert ok[~eg.isnan()].all()
 
 
 @pytest.mark.parametrize("latent", [False, True])
