@@ -724,20 +724,30 @@ bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, 
   return d == 128 ? chunk_form_ok<f16, true, 128, 32, 1>() : chunk_form_ok<f16, true, 256, 32, 1>();
 }
 
-// bf16 rows by DMA in steps of at least 1024 rows or with a sequence long enough to be cut.  This file's kernel -> chunk_mlstm.hip's,
-// us, 4 heads of 256 x 512:
-//   32 x 512, 24 x 700, 16 x 1000, 64 x 20   219 -> 136, 263 -> 147, 206 -> 185, 97 -> 75
-//   1 x 384, 512, 1000, 4000, 2 x 8192       72 -> 59, 74 -> 60, 84 -> 70, 122 -> 101, 318 -> 234
-//   16 x 64, 8 x 256, 4 x 300, 32 x 16       31.4 -> 31.0, 59.5 -> 58.7, 64.0 -> 64.6, 90.0 -> 89.8
-//   8 x 64, 4 x 64, 1 x 64, 1 x 256          23.9 -> 24.3, 22.4 -> 23.1, 20.5 -> 21.4, 52.7 -> 53.9
+// bf16 rows by DMA: heads of more than 128 columns, of which a workgroup there has twice as many, in sequences long enough
+// to be cut and in steps of at least 1024 rows; with 128 key channels, whose walks gain less, the latter only where this
+// file's do not all fit the CUs.  Heads of up to 128 columns leave half of its waves idle, which only shorter segments
+// than this file's outweigh.  This file's kernel -> chunk_mlstm.hip's, us:
+//   4 heads of 256 x 512   32 x 512, 24 x 700, 16 x 1000, 64 x 20   219 -> 136, 263 -> 147, 206 -> 185, 97 -> 75
+//                          1 x 384, 512, 1000, 4000, 2 x 8192       72 -> 59, 74 -> 60, 84 -> 70, 122 -> 101, 318 -> 234
+//                          16 x 64, 8 x 256, 4 x 300, 32 x 16       31.4 -> 31.0, 59.5 -> 58.7, 64.0 -> 64.6, 90.0 -> 89.8
+//                          8 x 64, 4 x 64, 1 x 64, 1 x 256          23.9 -> 24.3, 22.4 -> 23.1, 20.5 -> 21.4, 52.7 -> 53.9
+//   4 heads of 128 x 512   4 x 300, 8 x 200, 16 x 100, 300, 1000    39.5 -> 42.6, 34.0 -> 36.6, 23.2 -> 24.3, 42 -> 46, 114 -> 125
+//                          32 x 64, 200, 64 x 20                    26 -> 21, 64 -> 40, 46 -> 32
+//                          1 x 600, 5000, 8 x 600, 1500 (cut)       49 -> 41, 86 -> 74, 74 -> 64, 164 -> 116
+//   4 heads of 256 x 128   32 x 200, 256 x 30                       56.0 -> 55.1, 77.9 -> 79.6
+//                          1 x 600, 2 x 5000, 8 x 1500 (segments of 128, 192, 256)   71 -> 54, 114 -> 92, 91 -> 98
+//   16 of 128 x 128        32 x 64, 16 x 300; 1 x 1500, 2 x 1000, 4 x 800 (128, 192, 320)   28 -> 29, 44 -> 48; 58 -> 47, 56 -> 56, 56 -> 69
 ChunkWork mlstm_chunk_plan(int dtype, int P, int Tp, int H, int d, int dv) {
+  const int wpi = H * ((dv + 127) / 128);
   if (mlstm_rows_ok(dtype, dv)) {
     const int cols = mlstm_rows_columns();
     ChunkWork p = chunk_plan(P, Tp, H * ((dv + cols - 1) / cols), 64, 2, 6);
-    p.rows = p.seg > 0 || Tp >= 1024;
+    if (p.seg > 0) p.rows = dv > 128 || p.seg <= 192;
+    else p.rows = Tp >= 1024 && dv > 128 && (d > 128 || (int64_t)P * wpi > device_cus());
     if (p.rows) return p;
   }
-  return chunk_plan(P, Tp, H * ((dv + 127) / 128), dtype == DT_BF16 ? 64 : 32, 4, 8);
+  return chunk_plan(P, Tp, wpi, dtype == DT_BF16 ? 64 : 32, 4, 8);
 }
 
 void launch_mlstm_chunk(int dtype, float* out, const void* qkvg, int64_t stride, const float* gates,

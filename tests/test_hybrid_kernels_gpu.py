@@ -270,6 +270,26 @@ def test_mlstm_scan_rows_by_dma(gpu, H, d, dv, lens, before, D_ctx):
     test_mlstm_scan_chunkwise(gpu, torch.bfloat16, H, d, dv, lens, before, D_ctx)
 
 
+@pytest.mark.parametrize("H,d,dv", [(10, 128, 264), (15, 128, 144)])
+def test_mlstm_scan_rows_by_dma_many_heads(gpu, H, d, dv):
+    """Whole sequences with 128 key channels, which take heads enough to fill the CUs."""
+    test_mlstm_scan_chunkwise(gpu, torch.bfloat16, H, d, dv, [1, 15, 16, 17, 63, 64, 65, 129, 660], [0, 5, 0, 40, 0, 0, 9, 0, 3], [9, 1])
+
+
+@pytest.mark.parametrize("H,d,dv,P,n,own", [(4, 128, 512, 16, 300, False), (4, 128, 512, 32, 64, True), (4, 256, 512, 16, 100, True),
+                                            (2, 128, 128, 64, 40, False), (4, 256, 128, 1, 600, True), (4, 256, 128, 8, 1500, False)])
+def test_mlstm_scan_routes(gpu, H, d, dv, P, n, own):
+    """Steps whose rows come by DMA and steps that stay in the general walk (csrc/kernels/chunk_scan.hip has the times)."""
+    m = _to(_meta([n] * P, [n] * P, [], torch.zeros(P, 1, dtype=torch.int32), list(range(P))), gpu)
+    x, g = torch.zeros(P * n, 2 * H * (d + dv), device=gpu).bfloat16(), torch.zeros(P * n, 2 * H, device=gpu)
+    st = tuple(torch.zeros(P, H, *y, device=gpu) for y in ((d, dv), (d,), ()))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        ops.mlstm_scan(x, g, st, m, H, d, dv)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages()]
+    assert any("mlstm_walk_kernel" in k for k in names) == own and any("chunk_scan_kernel" in k for k in names) != own
+
+
 @pytest.mark.parametrize("lens,bad", [([45, 700, 400], (1, 333)), ([45, 700, 400], (0, 0)), ([45, 700, 400], (2, 399)),
                                       ([700, 33], (0, 130)), ([700, 33], (0, 698))])
 def test_mlstm_scan_rows_by_dma_not_finite(gpu, lens, bad):
