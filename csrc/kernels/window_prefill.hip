@@ -27,6 +27,7 @@
 #include "device.h"
 #include "chunk.h"
 #include "window.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace kgc {
@@ -471,6 +472,7 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
   if (n_work <= 0 || !(scale > 0.f) || H / G % HW != 0 || ex.pool > 0 || ex.vtab != nullptr ||
       blk_rows % BM != 0)
     return false;
+  if ((int64_t)G * bs * std::max(krs, vrs) >= (int64_t)1 << 32) return false;   // pages are 32-bit factors of the offsets
   const bool alias = kc == vc && krs == vrs;
   auto go = [&](auto cap, auto* o) {
     typedef std::remove_pointer_t<decltype(o)> T;

@@ -695,6 +695,22 @@ def test_window_attention_output_slices_and_pages(gpu, latent, at, bs):
     assert (buf[:, rest] == 7).all()
 
 
+def test_window_attention_largest_pages(gpu):
+    """Latent rows in pages of 2^24 tokens, 2^32 elements each: rows of the second page are not the first's."""
+    torch.manual_seed(40)
+    H, dk, dv, T, bs = 4, 256, 192, 70, 1 << 24
+    q, rows, pos = torch.randn(T, H, dk).bfloat16().to(gpu), torch.randn(T, dk).bfloat16().to(gpu), torch.arange(T, device=gpu)
+
+    def run(bs, table):
+        kc = torch.empty(2, 1, bs, dk, device=gpu, dtype=torch.bfloat16)
+        kc[0, 0, :T] = 3.0
+        kc[1, 0, :T] = rows
+        return ops.window_attention(q, kc, kc[..., :dv], pos, _to(_meta([T], [T], [], torch.tensor([[table]]).int()), gpu), 0.08, 0, 0)
+    got, want = run(bs, 1).float(), run(128, 1).float()
+    torch.cuda.empty_cache()
+    torch.testing.assert_close(got, want, rtol=1.01 * 2.0 ** -7, atol=2e-4)
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("latent", [False, True])
 @pytest.mark.parametrize("cap", [1e6, 1.5])
