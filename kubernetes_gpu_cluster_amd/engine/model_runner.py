@@ -245,15 +245,18 @@ class ModelRunner:
         """Prompt steps with the largest activations: the token budget in prompts as long as
         they get, and for recurrent layers in as many as there are slots, too -- the chunkwise
         scans keep a workspace per started chunk of every sequence, from 12 rows of each on (24
-        in small steps; csrc/kernels/chunk_rows.h)."""
+        in small steps; csrc/kernels/chunk_rows.h), and the Mamba-2 scan images of the chunks'
+        keys, from 16 rows of each on with few groups and 25 with many (csrc/kernels/chunk_ssd.hip)."""
         long, remaining = [], self.token_budget
         while remaining > 0:
             long.append(min(remaining, self.max_model_len))
             remaining -= long[-1]
-        n = min(self.max_num_seqs, self.token_budget // (12 if self.token_budget >= 1024 else 24))
-        if not self.state_layout or n <= len(long):
-            return [long]
-        return [long, [min(self.token_budget // n, self.max_model_len)] * n]
+        counts = [min(self.max_num_seqs, self.token_budget // rows)
+                  for rows in (12 if self.token_budget >= 1024 else 24, 16, 25)]
+        steps = [long] if not self.state_layout else [long] + [
+            [min(self.token_budget // n, self.max_model_len)] * n
+            for n in dict.fromkeys(counts) if n > len(long)]
+        return steps
 
     def release(self) -> None:
         """Drop the KV arena, decode graphs and workspaces (engine shutdown): a process

@@ -434,3 +434,16 @@ def test_memory_profile_covers_many_short_prompts():
     assert steps(512, 8192, 256, [()])[1] == [24] * 21
     assert steps(5000, 2048, 256, [()])[0] == [2048, 2048, 904]
     assert steps(4096, 100, 256, [()])[1] == [16] * 256 and steps(2048, 8192, 1, [()]) == [[2048]]
+
+
+def test_memory_profile_covers_images_of_chunks():
+    """Where slots are many, twelve rows of each are too few for the Mamba-2 scan's images of chunks: the steps with
+    the most started chunks among those that make them are profiled, too."""
+    from types import SimpleNamespace
+
+    from kubernetes_gpu_cluster_amd.engine.model_runner import ModelRunner
+    steps = lambda budget, seqs: ModelRunner._profile_steps(SimpleNamespace(   # noqa: E731
+        token_budget=budget, max_model_len=8192, max_num_seqs=seqs, state_layout=[()]))
+    assert steps(8192, 1024) == [[8192], [12] * 682, [16] * 512, [25] * 327]
+    assert steps(8192, 600) == [[8192], [13] * 600, [16] * 512, [25] * 327]
+    assert steps(8192, 400) == [[8192], [20] * 400, [25] * 327] and steps(8192, 300) == [[8192], [27] * 300]
