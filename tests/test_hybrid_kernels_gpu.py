@@ -291,10 +291,10 @@ def test_mlstm_scan_routes(gpu, H, d, dv, P, n, own):
 
 
 @pytest.mark.parametrize("lens,bad", [([45, 700, 400], (1, 333)), ([45, 700, 400], (0, 0)), ([45, 700, 400], (2, 399)),
-                                      ([700, 33], (0, 130)), ([700, 33], (0, 698))])
+                                      ([700, 33], (0, 130)), ([700, 33], (0, 698)), ([780, 33], (0, 130)), ([780, 33], (0, 778))])
 def test_mlstm_scan_rows_by_dma_not_finite(gpu, lens, bad):
     """A value that is not finite reaches its own column from its row on, and nothing else changes by a bit; whole
-    sequences (1145 rows) and segments."""
+    sequences (1145 rows) and segments (780 and 33; 700 and 33 stay in the general walk)."""
     torch.manual_seed(92)
     H, d, dv, (seq, tok), c = 2, 128, 272, bad, 261
     m, T, n = _chunk_step(lens, [0, 7, 0][:len(lens)], [])
@@ -903,12 +903,13 @@ def test_rope_kv_store_by_chunks(gpu, dt, interleaved, T, H, G, dk, dv, rot):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("H,G,rows", [(8, 2, 9), (16, 1, 40), (12, 4, 140)])
+@pytest.mark.parametrize("H,G,rows", [(8, 2, 9), (16, 1, 40), (12, 4, 140), (16, 4, 17), (16, 4, 100)])
 @pytest.mark.parametrize("kw", [dict(window=0, keep=0), dict(window=300, keep=5), dict(window=128, keep=0, chunked=True, sink=0.3),
                                 dict(window=0, keep=0, softcap=15.0)])
 def test_window_decode_many_waves(gpu, dt, H, G, rows, kw):
-    """Decode rows of 128/128 heads on 16 waves (and, with 560 workgroups, on 4): one key, chunks
-    around 32 and the 16 x 32 of a round, several rounds, a padding row."""
+    """Decode rows of 128/128 heads on 16 waves (68 and 400 workgroups, and windows of 128 keys), on 4 (560
+    workgroups) and in pieces (18 and 40): one key, chunks around 32 and the 16 x 32 of a round, several rounds, a
+    padding row."""
     torch.manual_seed(71)
     lens = [1, 31, 32, 33, 511, 513, 1025, 700, 0] + [5 + 13 * i for i in range(rows - 9)]
     bs, width = 16, 70
@@ -922,6 +923,28 @@ def test_window_decode_many_waves(gpu, dt, H, G, rows, kw):
     args = (0.09, kw.pop("window"), kw.pop("keep"))
     want = ops.window_attention(q, kc, vc, pos, m, *args, gate, **kw)
     got = ops.window_attention(q.to(gpu), kc.to(gpu), vc.to(gpu), pos.to(gpu), _to(m, gpu), *args, gate.to(gpu), **kw)
+    assert (got[8] == 0).all()
+    ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
+    keep = torch.arange(rows) != 8
+    torch.testing.assert_close(got.cpu().float()[keep], want.float()[keep], rtol=1.01 * ulp, atol=2e-4)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,rows", [(16, 66), (20, 40), (16, 520)])
+@pytest.mark.parametrize("kw", [dict(window=0, keep=0), dict(window=300, keep=5, sink=0.3)])
+def test_window_decode_latent_many_rows(gpu, dt, H, rows, kw):
+    """Latent decode rows of steps that are not split: 66 and 80 workgroups of 8 waves (20 heads take two), 520 of 4;
+    one key, chunks around 32 and the 8 x 32 of a round, several rounds, a padding row."""
+    torch.manual_seed(72)
+    lens = [1, 31, 32, 33, 255, 257, 513, 1000, 0] + [5 + 13 * i % 700 for i in range(rows - 9)]
+    bs, nb, width = 16, 300, 63
+    tables = torch.randint(0, nb, (rows, width), dtype=torch.int32)
+    kc, q, gate = torch.randn(nb, 1, bs, 256).to(dt), torch.randn(rows, H, 256).to(dt), torch.rand(rows, H)
+    m, pos, kw = _meta([], [], lens, tables), torch.tensor(lens) - 1, dict(kw)
+    args = (0.06, kw.pop("window"), kw.pop("keep"))
+    want = ops.window_attention(q, kc, kc[..., :192], pos, m, *args, gate, **kw)
+    kg = kc.to(gpu)
+    got = ops.window_attention(q.to(gpu), kg, kg[..., :192], pos.to(gpu), _to(m, gpu), *args, gate.to(gpu), **kw)
     assert (got[8] == 0).all()
     ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
     keep = torch.arange(rows) != 8
@@ -1083,3 +1106,51 @@ def test_chunkwise_scans_keep_what_is_not_finite_to_later_rows(gpu, op, dt, wher
     else:
         hit[slot, heads, :, slice(c, c + 1) if where == "v" else slice(0, V)] = True
     assert not S[hit].isfinite().any() and torch.equal(S[~hit], S_w[~hit])
+
+
+@pytest.mark.parametrize("op,lens,before", [("mlstm", [45, 700, 400], [0, 7, 0]), ("mlstm", [780, 33], [0, 5]),
+                                            ("ssd", [45, 300, 33], [3, 0, 7]), ("ssd", [700, 420], [0, 5])])
+@pytest.mark.parametrize("where,val", [("v", float("nan")), ("v", float("-inf")), ("k", float("nan")), ("gate", float("nan"))])
+@pytest.mark.parametrize("at", [(0, 20), (0, 44), (1, 0), (1, 29), (0, 333), (0, 698), (1, 128), (1, 299), (1, 399)])
+def test_own_walks_keep_what_is_not_finite_to_later_rows(gpu, op, lens, before, where, val, at):
+    """As the test of the general walk above, in the walks that bf16 mLSTM rows (256 key channels, two workgroups per
+    head) and heads that share B and C take: whole sequences and segments (of 128 rows), the first, a middle and
+    the last one; two groups of four heads, of which one shows what the other keeps."""
+    seq, tok = at
+    if tok >= lens[seq]:
+        pytest.skip("no such row")
+    torch.manual_seed(93)
+    m, T, n = _chunk_step(lens, before, [])
+    m.state_slots = torch.tensor([n - 1, *range(n - 1)], dtype=torch.int32)
+    mg = _to(m, gpu)
+    if op == "mlstm":
+        H, G, d, V = 2, 2, 256, 272
+        x, g = torch.randn(T, 2 * H * d + 2 * H * V).bfloat16(), torch.cat([torch.randn(T, H), -torch.rand(T, H)], dim=1)
+        st, koff, voff = [torch.randn(n, H, d, V), torch.randn(n, H, d), torch.rand(n, H)], H * d, 2 * H * d
+        run = lambda x, g, s: ops.mlstm_scan(x, g, s, mg, H, d, V)   # noqa: E731
+    else:
+        H, G, d, V = 8, 2, 128, 40
+        x, g, st, koff, voff = torch.randn(T, H * V + 2 * G * d), torch.randn(T, H).bfloat16(), [torch.randn(n, H, d, V)], H * V, 0
+        a, b = torch.full((H,), -1.0).to(gpu), torch.zeros(H).to(gpu)
+        run = lambda x, g, s: ops.ssd_scan(x, g, a, b, b, s[0], mg, H, V, d, G)   # noqa: E731
+
+    def both():
+        s = [y.to(gpu) for y in st]
+        return run(x.to(gpu), g.to(gpu), s).cpu().view(T, H, V), s[0].cpu()
+    want, S_w = both()
+    assert want.isfinite().all() and S_w.isfinite().all()
+    t, end, h, c, grp = sum(lens[:seq]) + tok, sum(lens[:seq + 1]), H - 1, V - 3, G - 1
+    if where == "v":
+        x[t, voff + h * V + c] = val
+    elif where == "k":
+        x[t, koff + grp * d + 100] = val
+    else:
+        g[t, h] = val
+    got, S = both()
+    heads = slice(grp * (H // G), H) if where == "k" else slice(h, h + 1)
+    cols = slice(c, c + 1) if where == "v" else slice(0, V)
+    hit, hit_S = torch.zeros(T, H, V, dtype=torch.bool), torch.zeros(n, H, d, V, dtype=torch.bool)
+    hit[t:end, heads, cols] = True
+    hit_S[int(m.state_slots[seq]), heads, 100 if where == "k" else slice(0, d), cols] = True
+    assert not got[hit].isfinite().any() and torch.equal(got[~hit], want[~hit])
+    assert not S[hit_S].isfinite().any() and torch.equal(S[~hit_S], S_w[~hit_S])
