@@ -72,6 +72,31 @@ __device__ __forceinline__ void mm3_add(const bf16x8 (&a)[N][3], const bf16x8 (&
     }
 }
 
+// the same for two row tiles times two column tiles
+__device__ __forceinline__ void mm3(const bf16x8 (&a)[2][3], const bf16x8 (&b)[2][3], f32x4 (&c)[2][2]) {
+  constexpr int PA[6] = {0, 1, 2, 0, 1, 0}, PB[6] = {2, 1, 0, 1, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        c[i][j] = mfma16x16x32(a[i][PA[k]], b[j][PB[k]], k ? c[i][j] : f32x4{0.f, 0.f, 0.f, 0.f});
+}
+// hi + lo += a b
+__device__ __forceinline__ void mm3_add(const bf16x8 (&a)[2][3], const bf16x8 (&b)[2][3], f32x4 (&hi)[2][2], f32x4 (&lo)[2][2]) {
+  constexpr int PA[6] = {0, 1, 2, 0, 1, 0}, PB[6] = {2, 1, 0, 1, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        f32x4& c = k == 5 ? hi[i][j] : lo[i][j];
+        c = mfma16x16x32(a[i][PA[k]], b[j][PB[k]], c);
+      }
+}
+
 // Order of the instructions up to here from the last sched_barrier: N times one MFMA and V vector instructions, which
 // run beside it, an LDS read after every R-th and a memory instruction after every M-th (0: where they fall; in a
 // burst they would hold up the wave).  An MFMA of 16 x 16 x 32 takes 8 cycles of issue and 16 of the matrix core, a vector
@@ -186,16 +211,16 @@ __device__ __forceinline__ SegItem seg_item(int item, const int* qsl, int P, int
   return r;
 }
 
-// chunks of L tokens of the sequences before `seq`
-template <int L>
-__device__ __forceinline__ int chunks_before(int seq, const int* qsl) {
+// pieces of `rows` tokens (a sequence has one at least) of the sequences before `seq`: segments, or chunks
+__device__ __forceinline__ int pieces_before(int seq, const int* qsl, int rows) {
   const int lane = threadIdx.x & 63;
   int n = 0;
-  for (int p = lane; p < seq; p += 64) n += max(1, (qsl[p + 1] - qsl[p] + L - 1) / L);
+  for (int p = lane; p < seq; p += 64) n += max(1, (qsl[p + 1] - qsl[p] + rows - 1) / rows);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
   return n;
 }
+template <int L> __device__ __forceinline__ int chunks_before(int seq, const int* qsl) { return pieces_before(seq, qsl, L); }
 
 // column c of a k index that MFMAs read permuted, so that accumulators are operands as they lie:
 // the 4-column pieces of every 32 go in the order 0 4 1 5 2 6 3 7

@@ -590,10 +590,7 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
   const int colc = colok ? col : a.dv - 1;
   const int len = a.qsl[seq + 1] - a.qsl[seq], pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
   if (len <= 0 || slot < 0 || slot >= a.num_slots || pos0 < 0) return;
-  int first = 0;                             // segments of the sequences before this one
-  for (int p = lane; p < seq; p += 64) first += max(1, (a.qsl[p + 1] - a.qsl[p] + a.seg - 1) / a.seg);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) first += __shfl_xor(first, o, 64);
+  const int first = pieces_before(seq, a.qsl, a.seg);
   const int count = (len + a.seg - 1) / a.seg, w = a.dv + D;
   const float* Ss = a.S + ((int64_t)slot * a.H + h) * D * a.dv;
   f32x4 S[DT];
@@ -661,9 +658,7 @@ DeltaWork delta_chunk_plan(int P, int Tp, int H, int G, int V) {
   w.floats = (int64_t)chunks * L * (3 * H + 2 * G);
   const int want = (device_cus() + wgs - 1) / wgs;      // items for one workgroup per CU
   if (P * 3 > want) return w;
-  int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
-  seg = (seg + L - 1) / L * L;
-  if (seg < 8 * L) seg = 8 * L;
+  const int seg = segment_rows(P, Tp, want, L, 8);    // one round
   if (Tp / P < 3 * seg) return w;
   w.seg = seg;
   w.items = Tp / seg + P;

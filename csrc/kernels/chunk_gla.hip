@@ -414,10 +414,7 @@ __global__ __launch_bounds__(256) void gla_chain_kernel(const GlaArgs a) {
   const int seq = blockIdx.z, h = blockIdx.y, lane = threadIdx.x & 63;
   const int len = a.qsl[seq + 1] - a.qsl[seq], pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
   if (len <= a.seg || slot < 0 || slot >= a.num_slots || pos0 < 0) return;
-  int first = 0;                             // segments of the sequences before this one
-  for (int p = lane; p < seq; p += 64) first += max(1, (a.qsl[p + 1] - a.qsl[p] + a.seg - 1) / a.seg);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) first += __shfl_xor(first, o, 64);
+  const int first = pieces_before(seq, a.qsl, a.seg);
   const int count = (len + a.seg - 1) / a.seg, per = a.seg / L, sh = D * a.dv;
   const int chunk0 = chunks_before<L>(seq, a.qsl);
   const int at = blockIdx.x * 256 + threadIdx.x;
@@ -456,9 +453,7 @@ int plan(int P, int Tp, int H, int V, int* items) {
   *items = P;
   const int wgs = H * ((V + 127) / 128), want = (device_cus() + wgs - 1) / wgs;
   if (P * 2 > want) return 0;
-  int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
-  seg = (seg + L - 1) / L * L;
-  if (seg < 4 * L) seg = 4 * L;
+  const int seg = segment_rows(P, Tp, want, L, 4);    // one round
   if (Tp / P < 2 * seg) return 0;
   *items = Tp / seg + P;
   return seg;

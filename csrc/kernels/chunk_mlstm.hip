@@ -59,11 +59,6 @@ __device__ __forceinline__ int sw(int t) { return (t & 3) << 1 | (t >> 2 & 1) | 
 // likewise the 8 units of P's rows
 __device__ __forceinline__ int p_at(int t, int u) { return t * L + (u ^ (t >> 1 & 7)) * 8; }
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-// column (lane & 15) of four rows: lanes 4 r .. 4 r + 3 of every 16 address row r, 4 elements each
-__device__ __forceinline__ u32x2 ld_tr4(const bf16* p) {
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
-}
 __device__ __forceinline__ bf16x8 ld_tr8(const bf16* p0, const bf16* p1) {
   const u32x2 a = ld_tr4(p0), b = ld_tr4(p1);
   return __builtin_bit_cast(bf16x8, u32x4{a[0], a[1], b[0], b[1]});
@@ -691,10 +686,7 @@ __global__ __launch_bounds__(256) void mlstm_chain_kernel(const MlstmArgs a, int
   const int seq = blockIdx.z, h = blockIdx.y, lane = threadIdx.x & 63;
   const int len = a.qsl[seq + 1] - a.qsl[seq], pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
   if (len <= a.seg || slot < 0 || slot >= a.num_slots || pos0 < 0) return;
-  int first = 0;                             // segments of the sequences before this one
-  for (int p = lane; p < seq; p += 64) first += max(1, (a.qsl[p + 1] - a.qsl[p] + a.seg - 1) / a.seg);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) first += __shfl_xor(first, o, 64);
+  const int first = pieces_before(seq, a.qsl, a.seg);
   const int count = (len + a.seg - 1) / a.seg;
   const int64_t sh = (int64_t)D * a.dv, step = (int64_t)a.H * (sh + D);
   const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;   // (a multiple of 4 elements each)

@@ -27,4 +27,12 @@ inline bool chunk_rows_pay(long P, long Tp, long alone) {
   return P > 0 && Tp >= (rows < alone ? rows : alone) * P;
 }
 
+// Tokens per segment, whole chunks of L and `least` of them at least, so that P sequences of Tp rows come to at most
+// `want` segments
+inline int segment_rows(int P, int Tp, int want, int L, int least) {
+  const int seg = (Tp + want - P - 1) / (want - P);       // Tp / seg + P <= want
+  const int rows = (seg + L - 1) / L * L;
+  return rows < least * L ? least * L : rows;
+}
+
 }  // namespace kgc

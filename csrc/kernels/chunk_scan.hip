@@ -703,9 +703,7 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L, int least, int shorte
   // and the pieces are long enough to pay for computing every contribution twice
   const int want = (device_cus() + wgs - 1) / wgs;
   if (P * 2 > want) return p;
-  int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
-  seg = (seg + L - 1) / L * L;
-  if (seg < least * L) seg = least * L;
+  const int seg = segment_rows(P, Tp, want, L, least);    // one round
   if (Tp / P < 2 * seg || Tp / P < shortest * L) return p;
   p.seg = seg;
   p.items = Tp / seg + P;

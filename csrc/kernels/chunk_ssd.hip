@@ -185,32 +185,6 @@ __global__ __launch_bounds__(NT) void ssd_prep_kernel(const SsdArgs a) {
   }
 }
 
-// Two row tiles a times two column tiles b, three parts each: four sums side by side, since an MFMA waits for
-// the one whose sum it continues.  The corrections first, then the main products on top of them.
-__device__ __forceinline__ void mm3(const bf16x8 (&a)[2][3], const bf16x8 (&b)[2][3], f32x4 (&c)[2][2]) {
-  constexpr int PA[6] = {0, 1, 2, 0, 1, 0}, PB[6] = {2, 1, 0, 1, 0, 0};
-#pragma unroll
-  for (int k = 0; k < 6; ++k)
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        c[i][j] = mfma16x16x32(a[i][PA[k]], b[j][PB[k]], k ? c[i][j] : f32x4{0.f, 0.f, 0.f, 0.f});
-}
-// hi + lo += a b
-__device__ __forceinline__ void mm3_add(const bf16x8 (&a)[2][3], const bf16x8 (&b)[2][3], f32x4 (&hi)[2][2], f32x4 (&lo)[2][2]) {
-  constexpr int PA[6] = {0, 1, 2, 0, 1, 0}, PB[6] = {2, 1, 0, 1, 0, 0};
-#pragma unroll
-  for (int k = 0; k < 6; ++k)
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        f32x4& c = k == 5 ? hi[i][j] : lo[i][j];
-        c = mfma16x16x32(a[i][PA[k]], b[j][PB[k]], c);
-      }
-}
-
 // 1024 bytes from each wave's 64 lanes to LDS
 __device__ __forceinline__ void dma16(const void* src, void* dst) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
@@ -293,7 +267,6 @@ __global__ __launch_bounds__(NT, 2) void ssd_walk_kernel(const SsdArgs a) {
   const float skip = a.dskip[h];
   int rs = (int)a.stride, ro = (int)os;
   auto image = [&](int ci) { return a.img + ((int64_t)ci * a.G + grp) * IMG; };
-  auto record = [&](int ci) -> const TokenRec& { return a.rec[(int64_t)ci * a.H + h]; };
   // one of the six pieces that a wave brings of the parts of C or B^T
   auto dma = [&](const char* src, bf16* dst, int i) {
     dma16(src + lane * 16 + (wave * 6 + i) * 1024, reinterpret_cast<char*>(dst) + (wave * 6 + i) * 1024);
@@ -583,10 +556,7 @@ __global__ __launch_bounds__(NT) void ssd_chain_kernel(const SsdArgs a) {
   const int seq = blockIdx.z, h = blockIdx.y, lane = threadIdx.x & 63;
   const int len = a.qsl[seq + 1] - a.qsl[seq], pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
   if (len <= a.seg || slot < 0 || slot >= a.num_slots || pos0 < 0) return;
-  int first = 0;                             // segments of the sequences before this one
-  for (int p = lane; p < seq; p += 64) first += max(1, (a.qsl[p + 1] - a.qsl[p] + a.seg - 1) / a.seg);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) first += __shfl_xor(first, o, 64);
+  const int first = pieces_before(seq, a.qsl, a.seg);
   const int count = (len + a.seg - 1) / a.seg, sh = D * a.dv;
   const int64_t step = (int64_t)a.H * sh;
   const int at = (blockIdx.x * NT + threadIdx.x) * 4;     // (128 rows: a multiple of 4 elements)
@@ -634,9 +604,7 @@ SsdWork ssd_shared_plan(int P, int Tp, int H, int V, int G) {
   w.bytes = chunks * G * IMG + chunks * H * (int64_t)sizeof(TokenRec);
   const int cus = device_cus(), wpi = walk_wgs(H, V, G), want = (2 * cus + wpi - 1) / wpi;   // items for two workgroups per CU
   if (P * 2 > want) return w;
-  int seg = (Tp + want - P - 1) / (want - P);   // at most Tp / seg + P <= want segments: one round
-  seg = (seg + L - 1) / L * L;
-  if (seg < 4 * L) seg = 4 * L;
+  const int seg = segment_rows(P, Tp, want, L, 4);    // one round
   const int rows = Tp / P;
   const int64_t wgs = (int64_t)P * ((rows + seg - 1) / seg) * wpi;
   if (rows < 3 * seg && (wgs > cus || rows <= 2 * seg + (2 * wgs > cus ? 2 * L : 0))) return w;

@@ -39,12 +39,4 @@ __device__ __forceinline__ float elem_gate(const WindowExtra& ex, int64_t t, int
   return gate_sigmoid(to_f(static_cast<const T*>(ex.egate)[t * ex.egs + c]));
 }
 
-// column (lane & 15) of four rows of 16-bit elements in LDS: lanes 4 r .. 4 r + 3 of every 16 address
-// row r, 4 elements each
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2 ld_tr4(const void* p) {
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                       (__attribute__((address_space(3))) s16x4*)p));
-}
-
 }  // namespace kgc
