@@ -15,8 +15,9 @@
 //     R = V - gamma K S_0,  U = W R,  O = gamma Q S_0 + P U,  S = gamma_L S_0 + K^T U.
 // Accumulators are B operands as they lie (mfma_perm), so R, U and S never pass through LDS.
 //
-// Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each, six products of parts,
-// the corrections summed apart; exponents are differences of running sums kept in double.
+// Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each, six products of parts.  The corrections
+// of K S_0 and Q S_0 have sums of their own; those of W R, P U and K^T U are summed first and the main products on top
+// of them.  Exponents are differences of running sums kept in double.
 //
 // Few long sequences are cut into segments: a chunk walk is linear in its state, so a first pass
 // walks every segment from zero (with its values) and from the identity (without), a second chains
@@ -639,8 +640,8 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
 
 // Chunkwise for 128 key channels where the rows pay (chunk_rows.h; a chunk's workspace is 200 KB for 16
 // heads, which few rows per sequence would multiply, too).  16 x 1000 tokens of 16 heads with 128 x 128
-// states: 1328 us token by token, 261 us chunkwise (45 us for W and P); 2 x 8192: 7.5 ms and 0.73 ms.  Per wave and
-// chunk the walk issues 670 vector instructions and 168 MFMAs in 13700 cycles: 8100 of two waves' issue, 6100 of
+// states: 1328 us token by token, 259 to 269 us chunkwise (a quarter of it W and P); 2 x 8192: 7.5 ms and 0.70
+// ms.  Per wave and chunk the walk issues 700 vector instructions and 168 MFMAs in 13700 cycles: 8100 of two waves' issue, 6100 of
 // the LDS that 95 reads of 1 KB per wave keep busy, the rest the barriers and the chain R -> U.  (Products, systems and
 // update each by itself, sums of two MFMAs added afterwards: 1000 vector instructions, 293 us in all; W and P read
 // by every wave from memory: 276.)

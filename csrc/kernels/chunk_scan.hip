@@ -712,7 +712,7 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L, int least, int shorte
 
 // Chunkwise from 16 rows per sequence on, heads of 128 or 256 key channels in 16 bits (fp32 rows in
 // three parts do not fit LDS).  32 x 512 tokens, 4 heads of 256 x 512: 1957 us token by token, 222 us
-// chunkwise here and 131 in chunk_mlstm.hip, and nearer to float64 (3.5e-7 and 2.9e-7 against 5.0e-7).
+// chunkwise here and 128 to 136 in chunk_mlstm.hip, and nearer to float64 (3.5e-7 and 3.0e-7 against 5.0e-7).
 bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, int H, int d, int dv) {
   if (!((dtype == DT_BF16 || dtype == DT_F16) && P > 0 && Tp >= 16 * P && (d == 128 || d == 256) &&
         stride % 8 == 0 && (reinterpret_cast<uintptr_t>(qkvg) & 15) == 0 && dv >= 16 &&

@@ -15,10 +15,15 @@
 // instruction 4, so both fill only where a wave's own vector work (splitting S) stands between its MFMAs: the
 // regions below say in which order.  Per wave and chunk 226 MFMAs and 950 vector instructions, 81 % of the cycles at two
 // waves per SIMD (before the order was given: the same work in 1.5 times the time).  2 x 8192 tokens, 32 heads of
-// 128 x 64, us: images 22, contributions 58, states 11, walk 142 (chunk_scan.hip: 130 and 255).
+// 128 x 64, us: 220 in all (chunk_scan.hip 357); kernel by kernel in a trace, whose clocks are not warm, images 23,
+// contributions 60, states 11, walk 145 (130 and 255 there).
 //
-// Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each (24 bits), six products of parts,
-// the corrections summed apart; exponents are differences of running sums kept in double.
+// Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each (24 bits), six products of parts.  The
+// corrections of C S_0 and of C . B have sums of their own; those of P X and of the update are summed first and the main
+// products on top of them.  Exponents are differences of running sums kept in double.
+//
+// Workspace: 52 KB per chunk and group, 1 KB per chunk and head, and 4 D V bytes per segment and head: 76 MB for 2 x 8192
+// tokens with one group (27, 17 and 32; chunk_scan.hip 16), 268 MB with eight.
 //
 // Few long sequences are cut into segments: one walk makes every segment's contribution from a zero state
 // (B^T only), a small launch puts the states together in which the segments start, and the second walk has them all.

@@ -1,4 +1,4 @@
-// Shared by the windowed attention kernels (attention_window.hip, window_prefill.hip).
+// Shared by the windowed attention kernels (attention_window.hip, window_prefill.hip, window_split.hip).
 #pragma once
 #include "common.h"
 #include "launch.h"

@@ -20,10 +20,10 @@
 // What bounds it: instruction issue.  MFMAs of 32 x 32 x 16 leave six vector instructions' time beside each (two
 // of 16 x 16 x 32, the same work: four), so the next keys' weights, the maximum and the next tile's addresses stand
 // between them in the order given below.  8 x 2048 rows, window 1024: per tile and wave 48 MFMAs and 380 vector
-// instructions, 4000 cycles of two waves' issue of the 5800 that a tile takes; the rest is the barrier, and 3.5
-// rounds of workgroups that take 4.  197 us in MFMAs of 16 x 16 x 32, 178 so; 32 x 512 rows 92 -> 77, latent rows
-// 130 -> 114, capped and causal 288 -> 254.  (A ring of four tiles filled by LDS-DMA three tiles ahead: 249 us where
-// this took 229.)
+// instructions, in bf16 70 more where the maximum moves, 4000 cycles of two waves' issue of the 5800 that a tile
+// takes; the rest is the barrier, and 3.5 rounds of workgroups that take 4.  bf16, in MFMAs of 16 x 16 x 32 -> so, us:
+// 197 -> 179 to 184, 32 x 512 rows 90 -> 76, latent rows 124 -> 110 to 116, capped and causal with a gate 290 -> 261.
+// (A ring of four tiles filled by LDS-DMA three tiles ahead: 249 us where this took 229.)
 #include "device.h"
 #include "chunk.h"
 #include "window.h"
@@ -466,8 +466,8 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
                                int window, int keep_first, const float* gate, const WindowExtra& ex,
                                hipStream_t s) {
   // Four heads on one staged tile against one head per workgroup (bf16, 16 heads on 4 key/value heads): window
-  // 1024 with 8 x 2048 rows 355 -> 184 us, causal and capped 577 -> 260, 48 rows after 3000 83 -> 53; latent rows
-  // (one key/value head), 32 x 512 rows 380 -> 113 us; 8 x 64 rows 11.0 -> 10.2, latent 12.8 -> 12.4.  The maximum
+  // 1024 with 8 x 2048 rows 355 -> 182 us, causal and capped 577 -> 261, 48 rows after 3000 83 -> 54; latent rows
+  // (one key/value head), 32 x 512 rows 380 -> 116 us; 8 x 64 rows 11.0 -> 10.2, latent 12.8 -> 12.4.  The maximum
   // is taken before the scale, which has to be positive for that.
   if (n_work <= 0 || !(scale > 0.f) || H / G % HW != 0 || ex.pool > 0 || ex.vtab != nullptr ||
       blk_rows % BM != 0)

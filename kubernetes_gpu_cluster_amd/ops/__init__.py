@@ -775,7 +775,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                           int(block_size), v_table, interleaved,
                           meta.slot_mapping if pool > 0 else None, chunked,
                           float("-inf") if sink is None else float(sink),
-                          int(getattr(meta, "decode_max_ctx", 0)))
+                          getattr(meta, "decode_max_ctx", 0))
     return out
 
 

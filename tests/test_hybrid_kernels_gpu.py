@@ -1108,17 +1108,16 @@ def test_chunkwise_scans_keep_what_is_not_finite_to_later_rows(gpu, op, dt, wher
     assert not S[hit].isfinite().any() and torch.equal(S[~hit], S_w[~hit])
 
 
-@pytest.mark.parametrize("op,lens,before", [("mlstm", [45, 700, 400], [0, 7, 0]), ("mlstm", [780, 33], [0, 5]),
-                                            ("ssd", [45, 300, 33], [3, 0, 7]), ("ssd", [700, 420], [0, 5])])
 @pytest.mark.parametrize("where,val", [("v", float("nan")), ("v", float("-inf")), ("k", float("nan")), ("gate", float("nan"))])
-@pytest.mark.parametrize("at", [(0, 20), (0, 44), (1, 0), (1, 29), (0, 333), (0, 698), (1, 128), (1, 299), (1, 399)])
+@pytest.mark.parametrize("op,lens,before,at", [
+    (op, lens, before, at) for op, lens, before in (("mlstm", [45, 700, 400], [0, 7, 0]), ("mlstm", [780, 33], [0, 5]),
+                                                    ("ssd", [45, 300, 33], [3, 0, 7]), ("ssd", [700, 420], [0, 5]))
+    for at in ((0, 20), (0, 44), (0, 333), (0, 698), (1, 0), (1, 29), (1, 128), (1, 299), (1, 399)) if at[1] < lens[at[0]]])
 def test_own_walks_keep_what_is_not_finite_to_later_rows(gpu, op, lens, before, where, val, at):
     """As the test of the general walk above, in the walks that bf16 mLSTM rows (256 key channels, two workgroups per
     head) and heads that share B and C take: whole sequences and segments (of 128 rows), the first, a middle and
     the last one; two groups of four heads, of which one shows what the other keeps."""
     seq, tok = at
-    if tok >= lens[seq]:
-        pytest.skip("no such row")
     torch.manual_seed(93)
     m, T, n = _chunk_step(lens, before, [])
     m.state_slots = torch.tensor([n - 1, *range(n - 1)], dtype=torch.int32)
