@@ -78,12 +78,15 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   constexpr bool SAME = !ALIAS && DK == DV;           // a thread's key and value units: the same rows
   static_assert(BN * DK / 8 % NT == 0 && BN * DV / 8 % NT == 0, "whole units per thread");
   constexpr float LOG2E = 1.44269504088896340736f;
-  // The maximum that weights refer to moves when a score passes it by more than this.  f16: weights up to 2^8 and
-  // few rescalings of the sums.  bf16: always, since a pair of bf16 holds 17 bits of a weight, and all of the
-  // largest one where that is 1: of 8 x 1024 rows 0.221 % of the results are not the exact ones' rounding so,
-  // 0.239 % where the maximum stays 2^8 behind, which would be faster (8 x 2048 176 us, so 184; capped 255, 262; latent
-  // 32 x 512 104, 109).  f16, whose sums' own rounding counts: 0.165 % and 0.149 %.
-  constexpr float FAR = __is_same(T, f16) ? 8.f : 0.f;
+  // The maximum that weights refer to moves when a score passes it by more than FAR.  f16: weights up to 2^8 and few
+  // rescalings of the sums.  bf16: always, since a pair of bf16 holds 17 bits of a weight, and all of the largest one
+  // where that is 1: of 8 x 1024 rows 0.221 % of the results are not the exact ones' rounding so, 0.239 % where the maximum
+  // stays 2^8 behind.  (f16, whose sums' own rounding counts: 0.165 % and 0.149 %.)  The sums then move in most tiles, so
+  // they are scaled beside the first products of P V, whether they have to be or not: 4 x 300 rows after 2000 57.2 us where
+  // the maximum stays behind, 59.2 with the scaling in a branch before the weights, 57.5 so; 32 x 512 76.0, 77.7, 76.6; 8 x
+  // 2048, where the clock gives way, 184, 189, 187; latent 4 x 2000 after 500 165, 174, 173.
+  constexpr float FAR = 8.f;
+  constexpr bool EXACT = __is_same(T, bf16);
   extern __shared__ __align__(16) char smem[];
   T* Kb = reinterpret_cast<T*>(smem);                 // [2][BN][KST]
   T* Vb = ALIAS ? Kb : Kb + 2 * BN * KST;             // [2][BN][VST]
@@ -315,8 +318,16 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
         const uint32_t x = both[0], y = both[1];
         mx = fmaxf(__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)) * fl;
       }
-      if (__any(mx > m + FAR)) {
-        const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+      float alpha = 1.f;
+      if constexpr (EXACT) {
+        const float mn = fmaxf(m, mx);
+        alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+        m = mn;
+        l *= alpha;
+        o[0] *= alpha;
+      } else if (__any(mx > m + FAR)) {
+        const float mn = fmaxf(m, mx);
+        alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
         m = mn;
         l *= alpha;
 #pragma unroll
@@ -366,14 +377,17 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
           else if (n + 1 < 2 * NB * DT) load_v(n + 1);
           o[t] = mfma32x32x16(vf[n & 1], pl[j], o[t]);
           o[t] = mfma32x32x16(vf[n & 1], ph[j], o[t]);
+          if (EXACT && j == 0 && t + 1 < DT) o[t + 1] *= alpha;
         }
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
           __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+          if (EXACT && j == 0) __builtin_amdgcn_sched_group_barrier(0x002, NB == 2 ? 12 : 8, 0);
+          else __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+          if (EXACT && j == 0) __builtin_amdgcn_sched_group_barrier(0x002, NB == 2 ? 12 : 8, 0);
+          else __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
