@@ -1255,7 +1255,8 @@ void residual_group_norm(Tensor out, Tensor x, std::optional<Tensor> y, Tensor w
 }
 
 void depth_mix_norm(Tensor out, Tensor x, Tensor hist, Tensor y, Tensor coef, Tensor w,
-                    int64_t layer, int64_t groups, double eps) {
+                    int64_t layer, int64_t groups, double eps, std::optional<Tensor> sums, int64_t slot,
+                    int64_t first, at::TensorList ahead) {
   check_f32(x, "x");
   check_f32(hist, "hist");
   check_f32(coef, "coef");
@@ -1270,10 +1271,31 @@ void depth_mix_norm(Tensor out, Tensor x, Tensor hist, Tensor y, Tensor coef, Te
               y.device() == x.device(), "kgc.depth_mix_norm: out / y");
   TORCH_CHECK(groups >= 1 && groups <= 64 && W % groups == 0 && w.numel() == W,
               "kgc.depth_mix_norm: groups / weight");
+  const int64_t n = (int64_t)ahead.size();
+  kgc::DepthAhead m{};
+  m.n = (int)n;
+  if (slot >= 0 || n > 0) {
+    TORCH_CHECK(sums.has_value(), "kgc.depth_mix_norm: sums");
+    check_f32(*sums, "sums");
+    TORCH_CHECK(sums->dim() == 3 && sums->device() == x.device() && sums->size(1) >= rows && sums->size(2) == W &&
+                (slot < 0 || n == 0) && slot < sums->size(0) && n <= kgc::DEPTH_AHEAD && n <= sums->size(0),
+                "kgc.depth_mix_norm: sums [slots, cap, W], read or begun");
+  }
+  if (slot >= 0) {
+    TORCH_CHECK(first >= 0 && first <= layer + 1, "kgc.depth_mix_norm: results in the sum");
+    m.from = sums->data_ptr<float>() + slot * sums->stride(0);
+    m.first = (int)first;
+  }
+  for (int64_t i = 0; i < n; ++i) {
+    check_f32(ahead[i], "ahead");
+    TORCH_CHECK(ahead[i].device() == x.device() && ahead[i].numel() >= layer + 2, "kgc.depth_mix_norm: ahead");
+    m.to[i] = sums->data_ptr<float>() + i * sums->stride(0);
+    m.coef[i] = ahead[i].data_ptr<float>();
+  }
   kgc::launch_depth_mix_norm(dt_code(out), out.data_ptr(), x.data_ptr<float>(),
                              hist.data_ptr<float>(), y.data_ptr(), coef.data_ptr<float>(),
                              w.data_ptr<float>(), (int)layer, hist.stride(0), (int)rows, (int)W,
-                             (int)groups, (float)eps, stream());
+                             (int)groups, (float)eps, m, stream());
 }
 
 void head_norm_gate(Tensor out, Tensor o, Tensor gt, Tensor w, int64_t H, double eps) {
@@ -2678,7 +2700,7 @@ TORCH_LIBRARY(kgc, m) {
         "Tensor? shared, Tensor? gate) -> ()");
   m.def("residual_group_norm(Tensor(a!) out, Tensor(b!) x, Tensor? y, Tensor w, int groups, float eps) -> ()");
   m.def("depth_mix_norm(Tensor(a!) out, Tensor(b!) x, Tensor(c!) hist, Tensor y, Tensor coef, Tensor w, "
-        "int layer, int groups, float eps) -> ()");
+        "int layer, int groups, float eps, Tensor(d!)? sums, int slot, int first, Tensor[] ahead) -> ()");
   m.def("head_norm_gate(Tensor(a!) out, Tensor o, Tensor g, Tensor w, int H, float eps) -> ()");
   m.def("xielu(Tensor(a!) out, Tensor z, Tensor ab) -> ()");
   m.def("gate_proj(Tensor(a!) out, Tensor h, Tensor w, Tensor? bias, int kind_a, int kind_b, int split, "

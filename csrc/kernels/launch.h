@@ -255,9 +255,18 @@ void ar_err_copy_async(void* sig, uint32_t* host_dst, hipStream_t s);
 // fp32 residual stream x [rows, W]; `dtype` is the activation type of out / y / h / w
 void launch_residual_group_norm(int dtype, void* out, float* x, const void* y, const float* w,
                                 int rows, int W, int groups, float eps, hipStream_t s);
+// depth averages beyond the layer's own: its sum goes on from `from` [rows, W] (results before `first`; null
+// and 0: from nothing), and the sums of the n following layers over results 0 .. layer + 1 go to `to`
+constexpr int DEPTH_AHEAD = 3;
+struct DepthAhead {
+  const float* from;
+  float* to[DEPTH_AHEAD];
+  const float* coef[DEPTH_AHEAD];
+  int first, n;
+};
 void launch_depth_mix_norm(int dtype, void* out, float* x, float* hist, const void* y,
                            const float* coef, const float* w, int layer, int64_t hist_stride,
-                           int rows, int W, int groups, float eps, hipStream_t s);
+                           int rows, int W, int groups, float eps, const DepthAhead& m, hipStream_t s);
 void launch_head_norm_gate(int dtype, void* out, const float* o, const void* g, int64_t g_stride,
                            const float* w, int rows, int H, int dv, float eps, hipStream_t s);
 void launch_xielu(int dtype, void* out, const void* z, const float* ab, int64_t n, hipStream_t s);

@@ -96,6 +96,8 @@ class DilavikForCausalLM(nn.Module):
         self.lm_head = ParallelLMHead(cfg.vocab_size, cfg.hidden_size, dtype, device)
         self.hist = None            # [L + 1, Tcap, W] fp32: X_0 .. X_L of the step's rows
         self.stream = None          # [Tcap, W] fp32: the residual stream
+        self.sums = None            # [slots, Tcap, W] fp32: depth averages begun by an earlier layer
+        self.mix_plan = ops.depth_mix_plan(cfg.num_layers)
 
     # ------------------------------------------------------------------ engine hooks
     @property
@@ -125,6 +127,7 @@ class DilavikForCausalLM(nn.Module):
         L, W = len(self.layers), self.cfg.hidden_size
         self.hist = torch.zeros(L + 1, max_tokens, W, dtype=torch.float32, device=device)
         self.stream = torch.zeros(max_tokens, W, dtype=torch.float32, device=device)
+        self.sums = torch.zeros(max(n for _, n in self.mix_plan), max_tokens, W, dtype=torch.float32, device=device)
 
     @torch.no_grad()
     def init_random(self, seed: int = 0, std: float = 0.02) -> None:
@@ -169,7 +172,9 @@ class DilavikForCausalLM(nn.Module):
                 h = ops.group_rms_norm(x, layer.norm2, G, eps, dt, add=y)
                 y = layer.mlp(h)
             nxt = self.layers[i + 1].norm1 if i + 1 < len(self.layers) else self.final_norm
-            h = ops.depth_mix_norm(x, self.hist, i, y, layer.dwa, nxt, G, eps, dt)
+            take, n = self.mix_plan[i]
+            h = ops.depth_mix_norm(x, self.hist, i, y, layer.dwa, nxt, G, eps, dt, self.sums, take,
+                                   [l.dwa for l in self.layers[i + 1: i + 1 + n]])
             if taps is not None:
                 taps.append(x.clone())
         return h

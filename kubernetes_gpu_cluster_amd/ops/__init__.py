@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import math
 import os
-from typing import Optional
+from typing import Optional, Sequence
 
 import torch
 
@@ -649,20 +649,44 @@ def group_rms_norm(x: torch.Tensor, w: torch.Tensor, groups: int, eps: float,
 
 def depth_mix_norm(x: torch.Tensor, hist: torch.Tensor, layer: int, y: torch.Tensor,
                    coef: torch.Tensor, w: torch.Tensor, groups: int, eps: float,
-                   out_dtype: torch.dtype) -> torch.Tensor:
+                   out_dtype: torch.dtype, sums: Optional[torch.Tensor] = None,
+                   take: Optional[tuple] = None, ahead: Sequence[torch.Tensor] = ()) -> torch.Tensor:
     """End of layer ``layer`` of a depth-averaged decoder, in one pass over the rows:
     hist[layer + 1, :T] = x + y (the layer's result); x = sum_j coef[j] * hist[j, :T] over
     j <= layer + 1 (in place: what the next layer reads); returns grouped RMSNorm(x) * w
     (the next layer's first norm, or the model's final one).  hist [L + 1, Tcap, W] and x
-    are fp32; coef fp32 [layer + 2]."""
+    are fp32; coef fp32 [layer + 2].
+    Long stacks read the old results less often: ``ahead``, the weights of up to three
+    following layers, also leaves sums[i, :T] = sum_j ahead[i][j] hist[j, :T] over
+    j <= layer + 1 (sums fp32 [slots, Tcap, W]); ``take`` = (slot, n) starts this layer's sum
+    from such a sum over the first n results.  ``depth_mix_plan`` says which layers do what."""
     T = x.shape[0]
     if not _gpu(x):
         hist[layer + 1, :T] = x + y.float()
-        x.copy_(ref.depth_mix(hist, layer + 2, coef, T))
+        x.copy_(ref.depth_mix(hist, layer + 2, coef, T, *((sums[take[0]], take[1]) if take else ())))
+        for i, c in enumerate(ahead):
+            sums[i, :T] = ref.depth_mix(hist, layer + 2, c, T)
         return ref.group_rms_norm(x, w, groups, eps, out_dtype)
     out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    _k().depth_mix_norm(out, x, hist, y, coef, w, layer, groups, eps)
+    slot, first = take or (-1, 0)
+    _k().depth_mix_norm(out, x, hist, y, coef, w, layer, groups, eps, sums, slot, first, list(ahead))
     return out
+
+
+def depth_mix_plan(layers: int, most: int = 3) -> list:
+    """Per layer of a depth-averaged stack, (take, how many layers ahead) of ``depth_mix_norm``
+    with the fewest rows read and written: a group of k layers from layer i reads i + 1
+    results, writes and reads k - 1 sums, and reads the results of its own layers."""
+    best = [(0, [])]                      # for the last n layers: rows, group sizes
+    for n in range(1, layers + 1):
+        i = layers - n
+        best.append(min((i + 1 + 2 * (k - 1) + (k - 1) * (k - 2) // 2 + best[n - k][0], [k] + best[n - k][1])
+                        for k in range(1, min(most + 1, n) + 1)))
+    plan, i = [], 0
+    for k in best[layers][1]:
+        plan += [(None, k - 1)] + [((a - 1, i + 2), 0) for a in range(1, k)]
+        i += k
+    return plan
 
 
 def xielu(z: torch.Tensor, ab: torch.Tensor) -> torch.Tensor:

@@ -373,9 +373,12 @@ def group_rms_norm(x: torch.Tensor, w: torch.Tensor, groups: int, eps: float,
     return (xg.view(T, W) * w.float()).to(out_dtype)
 
 
-def depth_mix(hist: torch.Tensor, n: int, coef: torch.Tensor, T: int) -> torch.Tensor:
-    """sum_j coef[j] * hist[j, :T] over the first n layer results (fp32)."""
-    return torch.einsum("j,jtw->tw", coef[:n].float(), hist[:n, :T].float())
+def depth_mix(hist: torch.Tensor, n: int, coef: torch.Tensor, T: int,
+              begun: Optional[torch.Tensor] = None, first: int = 0) -> torch.Tensor:
+    """sum_j coef[j] * hist[j, :T] over the first n layer results (fp32); ``begun``: the sum
+    over the first ``first`` of them."""
+    s = torch.einsum("j,jtw->tw", coef[first:n].float(), hist[first:n, :T].float())
+    return s if begun is None else begun[:T] + s
 
 
 def xielu(z: torch.Tensor, ab: torch.Tensor) -> torch.Tensor:

@@ -53,6 +53,51 @@ def test_depth_mix_norm(gpu, dt):
     torch.testing.assert_close(got.cpu().float(), want.float(), **_tol(dt))
 
 
+@pytest.mark.parametrize("W,G", [(192, 3), (512, 2), (2044, 1), (2048, 1), (4352, 1), (8192, 4)])
+@pytest.mark.parametrize("layers", [3, 7, 12])
+def test_depth_mix_sums_begun_ahead(gpu, W, G, layers):
+    """The same rows, results and normed rows to the bit, whichever layer began a sum."""
+    torch.manual_seed(layers)
+    T, cap, dt = 5, 9, torch.bfloat16
+    ys = [torch.randn(T, W).to(dt).to(gpu) for _ in range(layers)]
+    dwa = [torch.randn(i + 2).to(gpu) for i in range(layers)]
+    w = (torch.rand(W) + 0.5).to(gpu)
+    start = torch.randn(T, W).to(gpu)
+    out = []
+    for plan in ([(None, 0)] * layers, ops.depth_mix_plan(layers)):
+        hist, x, rows = torch.full((layers + 1, cap, W), 7.0, device=gpu), start.clone(), []
+        sums = torch.full((3, cap, W), 7.0, device=gpu)
+        hist[0, :T] = start
+        for i, (take, n) in enumerate(plan):
+            h = ops.depth_mix_norm(x, hist, i, ys[i], dwa[i], w, G, 1e-5, dt, sums, take, dwa[i + 1: i + 1 + n])
+            rows += [h, x.clone()]
+        assert (hist[:, T:] == 7).all() and (sums[:, T:] == 7).all()
+        out.append(rows + [hist])
+    assert any(n for _, n in plan)
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    # and the sums themselves, from fp32 on the CPU
+    hc, sc, xc = hist.cpu(), torch.zeros(3, cap, W), start.cpu()
+    for i, (take, n) in enumerate(plan):
+        h = ops.depth_mix_norm(xc, hc, i, ys[i].cpu(), dwa[i].cpu(), w.cpu(), G, 1e-5, dt, sc, take,
+                               [c.cpu() for c in dwa[i + 1: i + 1 + n]])
+        bound = 2.0 ** -22 * (i + 2) * sum(c.abs() * r.abs() for c, r in zip(dwa[i].cpu(), hc[:, :T]))
+        assert ((out[1][2 * i + 1].cpu() - xc).abs() <= bound + 2.0 ** -20).all()
+        xc = out[1][2 * i + 1].cpu().clone()
+
+
+def test_depth_mix_refuses_sums_that_do_not_fit(gpu):
+    W, T, dt = 256, 3, torch.bfloat16
+    x, hist, w = torch.zeros(T, W, device=gpu), torch.zeros(4, T, W, device=gpu), torch.ones(W, device=gpu)
+    y, c, sums = torch.zeros(T, W, dtype=dt, device=gpu), torch.ones(5, device=gpu), torch.zeros(1, T, W, device=gpu)
+    call = lambda *a: ops.depth_mix_norm(x, hist, 1, y, c[:3], w, 1, 1e-5, dt, *a)   # noqa: E731
+    call(sums, (0, 2))
+    for bad in ((sums, (1, 2)), (sums, (0, 3)), (sums, (0, 2), [c]), (sums, None, [c, c]), (sums, None, [c[:2]]),
+                (sums[:, :2], None, [c]), (sums[..., :128], None, [c]), (sums.double(), (0, 2))):
+        with pytest.raises(RuntimeError):
+            call(*bad)
+
+
 @pytest.mark.parametrize("dt", DT)
 def test_xielu_gate_proj_head_norm(gpu, dt):
     torch.manual_seed(2)
