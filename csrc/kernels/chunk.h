@@ -97,6 +97,16 @@ __device__ __forceinline__ void mm3_add(const bf16x8 (&a)[2][3], const bf16x8 (&
       }
 }
 
+// a barrier that leaves the newest N memory operations on their way (a fence would wait for all)
+template <int N> __device__ __forceinline__ void meet() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 0x70);   // vmcnt(N) lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // Order of the instructions up to here from the last sched_barrier: N times one MFMA and V vector instructions, which
 // run beside it, an LDS read after every R-th and a memory instruction after every M-th (0: where they fall; in a
 // burst they would hold up the wave).  An MFMA of 16 x 16 x 32 takes 8 cycles of issue and 16 of the matrix core, a vector

@@ -8,7 +8,7 @@
 //     O   = diag(gamma) Q S_0 + P U,                    P_ts = e^(b_t - b_s) q_t . k_s         (s <= t)
 //     S_L = gamma_L S_0 + sum_s e^(b_L - b_s) k_s u_s^T
 // W = (I + A)^-1 diag(beta) and P depend on no state: a first launch computes them for all chunks at
-// once (a lane per column of the triangular inverse), as bf16 parts in the order the walk's MFMAs
+// once (the inverses by blocks of 16 rows), as bf16 parts in the order the walk's MFMAs
 // read them.  The walk then has no serial step finer than a chunk: a workgroup of 8 waves owns 128
 // value columns of a head, a wave 16 of them with their S in accumulators, and everything between
 // two stagings of k and q concerns one wave's columns only:
@@ -53,7 +53,7 @@ struct DeltaArgs {
   bf16* wp;                                  // [chunks][H][W, P][3][L][L], columns permuted
   // per token of a chunk, zero past the sequence's end:
   float* gam;                                // [chunks][H][L]: gamma_t
-  double* kw;                                // [chunks][H][L]: e^(b_L - b_t) times rk
+  f32x2* kw;                                 // [chunks][H][L]: e^(b_L - b_t) times rk, the rounding and what it leaves
   float *rk, *rq;                            // [chunks][G][L]: what makes k and q unit (q: d^-1/2 too)
   int seg;                                   // tokens per segment (0: sequences are not cut)
   float* seg_state;                          // [items][H][D][dv + D]: dS | M of a segment
@@ -85,11 +85,14 @@ __device__ __forceinline__ void wave_lds() {
 __device__ __forceinline__ int wp_unit(int t, int u) { return t * (L / 8) + (u ^ ((t >> 2) & 3)); }
 
 // ---- W, P, the gates and the norms of every chunk: one wave per (chunk, q / k group) -----------
+// Dots, P and A stay in the layout of the MFMAs that made them, [s][t] with t the lane's: a lane's elements of a row are
+// the units that the walk reads.  (I + A)^-1 by blocks of 16, a lane per column of each diagonal block of two
+// heads: T21 = -T22 A21 T11 in fp32 MFMAs.
 __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
-  __shared__ float KK[L][L + 1], QK[L][L + 1];           // [t][s]: dots of unit vectors, s <= t
-  __shared__ __align__(16) float X[2][L][L + 4];  // P, A, then W of two heads at a time
-  __shared__ double bs[2][L];
-  __shared__ float be[2][L], rks[L];
+  constexpr int XR = 20, XB = 16 * XR + 16;  // floats of a row of a block, of a block: the four on banks of their own
+  __shared__ __align__(16) float X[4 * XB];  // [head][block]: A, then its inverse
+  __shared__ __align__(16) double bs[2][L];
+  __shared__ __align__(16) float be[2][L];
   const SegItem it = seg_item(blockIdx.x, a.qsl, a.P, L);
   if (it.seq < 0) return;
   const int g = blockIdx.y, lane = threadIdx.x, lr = lane & 15, lg = lane >> 4;
@@ -102,8 +105,7 @@ __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
   const float* kb = qb + (int64_t)a.G * D;
   const int rs = (int)a.stride, hpg = a.H / a.G;
 
-  const int hf = lane >> 5;                  // this lane: column (and token) s of head h0 + hf
-  int s = lane & 31;
+  const int hf = lane >> 5, s = lane & 31;   // gates: this lane's token of head h0 + hf
   const int64_t row = (t0 + min(s, nl - 1)) * a.bas;
   auto head = [&](int h0) { return g * hpg + min(h0 + hf, hpg - 1); };
   float gx = ld_ba(a, row + head(0)), gz = ld_ba(a, row + a.H + head(0));   // land during the dots
@@ -114,15 +116,28 @@ __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
 #pragma unroll
   for (int i = 0; i < 3; ++i) dk[i] = dkl[i] = dq[i] = dql[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   double n2[2][2] = {{0.0, 0.0}, {0.0, 0.0}};             // [k, q][tile]
+  const int at[2] = {min(lr, nl - 1) * rs + lg * 8, min(16 + lr, nl - 1) * rs + lg * 8};
+  f32x4 in[2][2][2][2];                      // 32 columns of k and q, the next 32
+  auto fetch = [&](int j) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          in[j & 1][w][ti][i] = *reinterpret_cast<const f32x4*>((w ? qb : kb) + at[ti] + j * 32 + i * 4);
+  };
+  fetch(0);
 #pragma unroll
   for (int j = 0; j < KD; ++j) {
+    if (j + 1 < KD) fetch(j + 1);
+    __builtin_amdgcn_sched_barrier(0);
     bf16x8 f[2][2][3];
 #pragma unroll
     for (int w = 0; w < 2; ++w)
 #pragma unroll
       for (int ti = 0; ti < LT; ++ti) {
-        const float* p = (w ? qb : kb) + min(ti * 16 + lr, nl - 1) * rs + j * 32 + lg * 8;
-        const f32x4 x0 = *reinterpret_cast<const f32x4*>(p), x1 = *reinterpret_cast<const f32x4*>(p + 4);
+        const f32x4 x0 = in[j & 1][w][ti][0], x1 = in[j & 1][w][ti][1];
         const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
 #pragma unroll
         for (int i = 0; i < 8; ++i) n2[w][ti] = __builtin_fma((double)x[i], (double)x[i], n2[w][ti]);
@@ -134,6 +149,7 @@ __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
       mm<true, 3, 3>(f[0][si], f[0][ti], dk[tile], dkl[tile]);
       mm<true, 3, 3>(f[0][si], f[1][ti], dq[tile], dql[tile]);
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
   float rn[2][2];
 #pragma unroll
@@ -145,99 +161,162 @@ __global__ __launch_bounds__(64, 2) void delta_prep_kernel(const DeltaArgs a) {
       n += __shfl_xor(n, 32, 64);
       rn[w][ti] = (float)(1.0 / sqrt((n + 1e-6) * (w ? D : 1)));
       const int t = ti * 16 + lr;
-      if (lg == 0) {
-        (w ? a.rq : a.rk)[((int64_t)blockIdx.x * a.G + g) * L + t] = t < nl ? rn[w][ti] : 0.f;
-        if (w == 0) rks[t] = rn[w][ti];
-      }
+      if (lg == 0) (w ? a.rq : a.rk)[((int64_t)blockIdx.x * a.G + g) * L + t] = t < nl ? rn[w][ti] : 0.f;
     }
+  float kk[3][4], qk[3][4];                  // dots of unit vectors
 #pragma unroll
   for (int tile = 0; tile < 3; ++tile) {
-    const int ti = tile > 0, si = tile > 1, t = ti * 16 + lr;
+    const int ti = tile > 0, si = tile > 1;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int c = si * 16 + lg * 4 + r;
       const float f = __shfl(rn[0][si], lg * 4 + r, 64);
-      KK[t][c] = (dk[tile][r] + dkl[tile][r]) * (f * rn[0][ti]);
-      QK[t][c] = (dq[tile][r] + dql[tile][r]) * (f * rn[1][ti]);
+      kk[tile][r] = (dk[tile][r] + dkl[tile][r]) * (f * rn[0][ti]);
+      qk[tile][r] = (dq[tile][r] + dql[tile][r]) * (f * rn[1][ti]);
     }
   }
-  wave_lds();
+  const float r0 = __shfl(rn[0][0], s & 15, 64), r1 = __shfl(rn[0][1], s & 15, 64), rks = s < 16 ? r0 : r1;
 
   for (int h0 = 0; h0 < hpg; h0 += 2) {
-    const bool on = h0 + hf < hpg;
-    const int h = head(h0);
     const bool ok = s < nl;
-    const float x = gx;
-    const double z = (double)gz + (double)gb;
-    double f = -exp((double)ga) * (z > 40.0 ? z : log1p(exp(z)));
-    if (h0 + 2 < hpg) {
-      gx = ld_ba(a, row + head(h0 + 2));
-      gz = ld_ba(a, row + a.H + head(h0 + 2));
-      gb = a.dt_bias[head(h0 + 2)];
-      ga = a.a_log[head(h0 + 2)];
-    }
-    // a decay of e^-1e6 is zero; a finite floor keeps the differences of running sums defined
-    const double b = half_scan(!ok ? 0.0 : f < -1e6 ? -1e6 : f);
-    const uint64_t bb = __builtin_bit_cast(uint64_t, b);
-    const uint32_t bl = __shfl((int)(uint32_t)bb, 31 + 32 * hf, 64), bh = __shfl((int)(bb >> 32), 31 + 32 * hf, 64);
-    const double bL = __builtin_bit_cast(double, (uint64_t)bh << 32 | bl);
-    const float beta = ok ? 1.f / (1.f + expf(-x)) : 0.f;
-    bs[hf][s] = b;
-    be[hf][s] = beta;
-    if (on) {
-      a.gam[((int64_t)blockIdx.x * a.H + h) * L + s] = ok ? (float)exp(b) : 0.f;
-      a.kw[((int64_t)blockIdx.x * a.H + h) * L + s] = ok ? exp(bL - b) * rks[s] : 0.0;
+    {
+      const int h = head(h0);
+      const float x = gx;
+      const double z = (double)gz + (double)gb;
+      double f = -exp((double)ga) * (z > 40.0 ? z : log1p(exp(z)));
+      if (h0 + 2 < hpg) {
+        gx = ld_ba(a, row + head(h0 + 2));
+        gz = ld_ba(a, row + a.H + head(h0 + 2));
+        gb = a.dt_bias[head(h0 + 2)];
+        ga = a.a_log[head(h0 + 2)];
+      }
+      // a decay of e^-1e6 is zero; a finite floor keeps the differences of running sums defined
+      const double b = half_scan(!ok ? 0.0 : f < -1e6 ? -1e6 : f);
+      const uint64_t bb = __builtin_bit_cast(uint64_t, b);
+      const uint32_t bl = __shfl((int)(uint32_t)bb, 31 + 32 * hf, 64), bh = __shfl((int)(bb >> 32), 31 + 32 * hf, 64);
+      const double bL = __builtin_bit_cast(double, (uint64_t)bh << 32 | bl);
+      bs[hf][s] = b;
+      be[hf][s] = ok ? 1.f / (1.f + expf(-x)) : 0.f;
+      if (h0 + hf < hpg) {
+        a.gam[((int64_t)blockIdx.x * a.H + h) * L + s] = ok ? (float)exp(b) : 0.f;
+        const double w = ok ? exp(bL - b) * rks : 0.0;    // as a sum of two floats
+        const float wh = (float)w;
+        a.kw[((int64_t)blockIdx.x * a.H + h) * L + s] = f32x2{wh, (float)(w - wh)};
+      }
     }
     wave_lds();
-    // a matrix in X as three parts, eight (permuted) columns per store
-    auto put = [&](int mat) {
-      for (int u = lane; u < 2 * L * 4; u += 64) {
-        const int oct = u & 3, t = (u >> 2) & 31, hh = u >> 7;
-        if (h0 + hh >= hpg) continue;
-        const float* src = X[hh][t] + oct * 4;                      // pieces oct and oct + 4 of the row
-        const f32x4 p0 = *reinterpret_cast<const f32x4*>(src), p1 = *reinterpret_cast<const f32x4*>(src + 16);
-        const float y[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
-        bf16x8 o[3];
-        split8<3>(y, o);
-        bf16* dst = a.wp + (((int64_t)blockIdx.x * a.H + g * hpg + h0 + hh) * 2 + mat) * MAT + wp_unit(t, oct) * 8;
+    // rows of a matrix as three parts, eight (permuted) columns to a store: those of tile (ti, 0), then of (ti, 1)
+    auto put = [&](int hh, int mat, int ti, const float (&y)[8]) {
+      bf16x8 o[3];
+      split8<3>(y, o);
+      bf16* dst = a.wp + (((int64_t)blockIdx.x * a.H + g * hpg + h0 + hh) * 2 + mat) * MAT + wp_unit(ti * 16 + lr, lg) * 8;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(dst + i * L * L) = o[i];
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(dst + i * L * L) = o[i];
+    };
+    float a21[2][4];
+    int bad[2] = {L, L};                     // the first token whose row of A or write strength is not finite
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      const double tb[2] = {bs[hh][lr], bs[hh][16 + lr]};
+      const float bt[2] = {be[hh][lr], be[hh][16 + lr]};
+      float A[3][4], P[3][4], z = bt[0] + bt[1];
+#pragma unroll
+      for (int tile = 0; tile < 3; ++tile) {
+        const int ti = tile > 0, si = tile > 1;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int d = tile == 1 ? 16 : lr - (4 * lg + r);   // t - s
+          float e = exp_d(tb[ti] - bs[hh][si * 16 + 4 * lg + r]);
+          asm volatile("" : "+v"(e));        // (no branches)
+          P[tile][r] = d >= 0 ? e * qk[tile][r] : 0.f;
+          A[tile][r] = d > 0 ? bt[ti] * e * kk[tile][r] : 0.f;
+          z += A[tile][r];
+        }
+      }
+      if (h0 + hh < hpg) {
+        put(hh, 1, 0, {P[0][0], P[0][1], P[0][2], P[0][3], 0.f, 0.f, 0.f, 0.f});
+        put(hh, 1, 1, {P[1][0], P[1][1], P[1][2], P[1][3], P[2][0], P[2][1], P[2][2], P[2][3]});
+      }
+      // Products of blocks would carry what is not finite to the rows before it: such rows of A are left out,
+      // and those of W written as NaN from the first one on.
+      if (__any(!(fabsf(z) < INFINITY))) {
+        auto odd = [](float x) { return !(fabsf(x) < INFINITY); };
+        bool b0 = odd(bt[0]), b1 = odd(bt[1]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          b0 |= odd(A[0][r]);
+          b1 |= odd(A[1][r]) || odd(A[2][r]);
+        }
+        int f = b0 ? lr : b1 ? 16 + lr : L;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) f = min(f, __shfl_xor(f, o, 64));
+        bad[hh] = f;
+#pragma unroll
+        for (int tile = 0; tile < 3; ++tile)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if ((tile > 0) * 16 + lr >= f) A[tile][r] = 0.f;
+      }
+      *reinterpret_cast<f32x4*>(X + 2 * hh * XB + lr * XR + 4 * lg) = f32x4{A[0][0], A[0][1], A[0][2], A[0][3]};
+      *reinterpret_cast<f32x4*>(X + (2 * hh + 1) * XB + lr * XR + 4 * lg) = f32x4{A[2][0], A[2][1], A[2][2], A[2][3]};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a21[hh][r] = A[1][r];
+    }
+    wave_lds();
+    {                                        // column lr of the inverse of block lg, from the top
+      float* B = X + lg * XB;
+      float T[16];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        float x[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < t; j += 4) {
+          const f32x4 r = *reinterpret_cast<const f32x4*>(B + t * XR + j);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (j + i < t) x[i] += r[i] * T[j + i];
+        }
+        const float y = -((x[0] + x[1]) + (x[2] + x[3]));
+        T[t] = t == lr ? 1.f : t < lr ? 0.f : y;
       }
       wave_lds();
-    };
-    asm volatile("" : "+v"(s));               // masks are made where they are used, not kept
-    float e[L];
 #pragma unroll
-    for (int t = 0; t < L; ++t) {
-      e[t] = t >= s ? exp_d(bs[hf][t] - b) : 0.f;
-      X[hf][t][s] = t >= s ? e[t] * QK[t][s] : 0.f;
+      for (int t = 0; t < 16; ++t) B[t * XR + lr] = T[t];
     }
     wave_lds();
-    put(1);
-    asm volatile("" : "+v"(s));
 #pragma unroll
-    for (int t = 0; t < L; ++t) X[hf][t][s] = t > s ? be[hf][t] * e[t] * KK[t][s] : 0.f;
-    wave_lds();
-    asm volatile("" : "+v"(s));
-    // column s of (I + A)^-1, from the top; rows of A are read by all lanes of a half together
-    float T[L];
+    for (int hh = 0; hh < 2; ++hh) {
+      const float *B0 = X + 2 * hh * XB, *B1 = B0 + XB;
+      const f32x4 t11 = *reinterpret_cast<const f32x4*>(B0 + lr * XR + 4 * lg);
+      const f32x4 t22 = *reinterpret_cast<const f32x4*>(B1 + lr * XR + 4 * lg);
+      f32x4 m = {0.f, 0.f, 0.f, 0.f}, t21 = m;
 #pragma unroll
-    for (int t = 0; t < L; ++t) {
-      float x[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int r = 0; r < 4; ++r) m = __builtin_amdgcn_mfma_f32_16x16x4f32(a21[hh][r], B0[(4 * lg + r) * XR + lr], m, 0, 0, 0);
 #pragma unroll
-      for (int j = 0; j < t; j += 4) {
-        const f32x4 r = *reinterpret_cast<const f32x4*>(&X[hf][t][j]);
+      for (int r = 0; r < 4; ++r) t21 = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], t22[r], t21, 0, 0, 0);
+      const f32x4 c0 = *reinterpret_cast<const f32x4*>(&be[hh][4 * lg]), c1 = *reinterpret_cast<const f32x4*>(&be[hh][16 + 4 * lg]);
+      float w0[8], w1[8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (j + i < t) x[i] += r[i] * T[j + i];
+      for (int r = 0; r < 4; ++r) {
+        const bool in = 4 * lg + r <= lr;
+        w0[r] = in ? t11[r] * c0[r] : 0.f;
+        w0[4 + r] = 0.f;
+        w1[r] = -t21[r] * c0[r];
+        w1[4 + r] = in ? t22[r] * c1[r] : 0.f;
       }
-      T[t] = t == s ? 1.f : t < s ? 0.f : -((x[0] + x[1]) + (x[2] + x[3]));
-    }
-    wave_lds();
+      if (bad[hh] < L)
 #pragma unroll
-    for (int t = 0; t < L; ++t) X[hf][t][s] = t < s ? 0.f : T[t] * beta;   // (beta may be NaN)
-    wave_lds();
-    put(0);
+        for (int r = 0; r < 4; ++r) {
+          const bool in = 4 * lg + r <= lr;
+          if (lr >= bad[hh] && in) w0[r] = NAN;
+          if (16 + lr >= bad[hh]) w1[r] = NAN;
+          if (16 + lr >= bad[hh] && in) w1[4 + r] = NAN;
+        }
+      if (h0 + hh < hpg) {
+        put(hh, 0, 0, w0);
+        put(hh, 0, 1, w1);
+      }
+    }
+    wave_lds();                              // (the next heads write where these were read)
   }
 }
 
@@ -298,36 +377,43 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
   const float* vb = a.qkv + 2 * (int64_t)a.G * D + (int64_t)h * a.dv;
   const int vo = ident ? 0 : colc;
   int rs = (int)a.stride, ro = (int)os;
+  // (a base in vector registers would make every store of an output a loop over its values)
+  const uint64_t ob64 = reinterpret_cast<uint64_t>(a.out + start * os + (int64_t)h * a.dv);
+  char* const ob = reinterpret_cast<char*>((uint64_t)(uint32_t)uniform((int)(ob64 >> 32)) << 32 | (uint32_t)uniform((int)ob64));
 
   // Staging: a thread takes 8 columns of one row of q and k, and 8 tokens of one column of k, in
   // both cases the pieces 4 a .. and 16 + 4 a .. of 32: adjacent in the permuted order, one store.
-  // Rows past the sequence's end read its last (their factors are zero).
+  // Rows past the sequence's end: through descriptors that end with the chunk's last row, zeros.
   f32x4 rqv[2], rkv[2], rt[2];
-  double kw[8];
+  f32x2 kw[8];
   float nk = 0.f, nq = 0.f;
   const int ut = tid / 16, uc = (tid % 16 / 4) * 32 + (tid % 4) * 4, up_ = (tid % 16) * 8;
   const int ta = tid / D * 4, tc = tid % D;
+  auto rows_of = [&](const float* p, int c0, int w) {
+    const float* r = p + (int64_t)(start + c0) * a.stride;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(r), 0, ((min(L, len - c0) - 1) * rs + w) * 4, 0x00027000);
+  };
+  auto ld16 = [&](__amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0)); };
+  auto ld4 = [&](__amdgpu_buffer_rsrc_t r, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0)); };
   auto fetch_rows = [&](int c0, int ci) {
-    const int nl = min(L, len - c0);
-    const float* kr = kb + (int64_t)(start + c0) * a.stride;
-    const float* qr = qb + (int64_t)(start + c0) * a.stride;
-    const int at = __mul24(min(ut, nl - 1), rs) + uc;
-    rkv[0] = *reinterpret_cast<const f32x4*>(kr + at);
-    rkv[1] = *reinterpret_cast<const f32x4*>(kr + at + 16);
+    const uint32_t at = (__mul24(ut, rs) + uc) * 4;
+    const auto kr = rows_of(kb, c0, D);
+    rkv[0] = ld16(kr, at);
+    rkv[1] = ld16(kr, at + 64);
     nk = a.rk[((int64_t)ci * a.G + g) * L + ut];
     if (MODE != 1) {
-      rqv[0] = *reinterpret_cast<const f32x4*>(qr + at);
-      rqv[1] = *reinterpret_cast<const f32x4*>(qr + at + 16);
+      const auto qr = rows_of(qb, c0, D);
+      rqv[0] = ld16(qr, at);
+      rqv[1] = ld16(qr, at + 64);
       nq = a.rq[((int64_t)ci * a.G + g) * L + ut];
     }
   };
   auto fetch_cols = [&](int c0, int ci) {
-    const int nl = min(L, len - c0);
-    const float* kr = kb + (int64_t)(start + c0) * a.stride;
+    const auto kr = rows_of(kb, c0, D);
+    const uint32_t at = (__mul24(ta, rs) + tc) * 4;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      rt[i >> 2][i & 3] = kr[__mul24(min(ta + (i >> 2) * 16 + (i & 3), nl - 1), rs) + tc];
-    const double* w = a.kw + ((int64_t)ci * a.H + h) * L + ta;
+    for (int i = 0; i < 8; ++i) rt[i >> 2][i & 3] = ld4(kr, at + ((i >> 2) * 16 + (i & 3)) * rs * 4);
+    const f32x2* w = a.kw + ((int64_t)ci * a.H + h) * L + ta;
 #pragma unroll
     for (int i = 0; i < 8; ++i) kw[i] = w[(i >> 2) * 16 + (i & 3)];
   };
@@ -350,7 +436,7 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
     // k^T times the weight of its token in the update, tokens permuted: U is the B operand as it lies
     float x[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = (float)(rt[i >> 2][i & 3] * kw[i]);
+    for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf(rt[i >> 2][i & 3], kw[i][0], rt[i >> 2][i & 3] * kw[i][1]);
     bf16x8 p[3];
     split8<3>(x, p);
 #pragma unroll
@@ -366,14 +452,15 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
   // this lane's v and gammas (rows 4 lg + r of each tile)
   auto fetch_own = [&](Own& w, int c0, int ci) {
     const int nl = min(L, len - c0);
-    const float* vc = vb + (int64_t)(start + c0) * a.stride;
+    const auto vr = rows_of(vb, c0, a.dv);
+    const uint32_t at = (__mul24(lg * 4, rs) + vo) * 4;
     const float* gc = a.gam + ((int64_t)ci * a.H + h) * L;
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti) {
       w.gm[ti] = *reinterpret_cast<const f32x4*>(gc + ti * 16 + lg * 4);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        w.v[ti][r] = vc[__mul24(min(ti * 16 + lg * 4 + r, nl - 1), rs) + vo];
+        w.v[ti][r] = ld4(vr, at + (ti * 16 + r) * rs * 4);
     }
     w.gL = gc[nl - 1];
   };
@@ -391,13 +478,14 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
       for (int i = 0; i < 3; ++i)
         f[ti][i] = *reinterpret_cast<const bf16x8*>(m + i * L * L + wp_unit(ti * 16 + lr, lg) * 8);
   };
-  auto arrived = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
   // Staged rows are parked while the last chunk's update runs, columns beside the products with S: k^T is not
   // read before the barrier between the two.  (The last chunk, which has none to stage, is a copy of its own: a branch
   // would end the regions in which vector instructions and MFMAs are interleaved, and staging the same again took steps
   // of short prompts 3 to 8 % longer: 100 x 20 95.7 us, so 89.5, 400 x 16 345 and 307.)
   Own next;
+  bf16x8 sp[2][3];                           // parts of 32 rows of S; the first ones of the next chunk
+  split_s(sp[0], 0);
   dma(chunk0, 0, Ws);
   fetch_rows(0, chunk0);
   fetch_cols(0, chunk0);
@@ -407,9 +495,7 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
     constexpr bool LAST = decltype(last)::value;
     const int nl = LAST ? len - c0 : L, cn = c0 + L, cin = ci + 1;
     asm volatile("" : "+s"(rs), "+s"(ro));   // row offsets are computed per chunk, not kept
-    arrived();
-    __syncthreads();
-    const int64_t t0 = start + c0;
+    meet<MODE == 1 ? 0 : 8>();               // (the last chunk's outputs may still be on their way)
     const Own own = next;
     if (MODE != 1) dma(ci, 1, Ps);
     f32x4 r[LT], rl[LT], o[LT], ol[LT];
@@ -417,7 +503,7 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
     for (int ti = 0; ti < LT; ++ti) r[ti] = rl[ti] = o[ti] = ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
     // products with S in steps of 32 of its rows, k's and q's in turn: the next step's operands are read, and the
     // next parts of S made, beside the MFMAs
-    bf16x8 sp[2][3], f[2][LT][3];
+    bf16x8 f[2][LT][3];
     auto load_rows = [&](bf16x8 (&x)[LT][3], const bf16* m, int j) {
 #pragma unroll
       for (int ti = 0; ti < LT; ++ti)
@@ -426,14 +512,26 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
           x[ti][i] = *reinterpret_cast<const bf16x8*>(m + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
     };
     load_rows(f[0], Ks, 0);
-    split_s(sp[0], 0);
     __builtin_amdgcn_sched_barrier(0);
+    bf16x8 rp[3];
+    auto make_r = [&]() {                    // (rows past the end: W is zero there)
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int ti = i >> 2, e = i & 3;
+        x[i] = __builtin_fmaf(-own.gm[ti][e], r[ti][e] + rl[ti][e], ident ? 0.f : own.v[ti][e]);
+      }
+      if (LAST)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = (i >> 2) * 16 + lg * 4 + (i & 3) >= nl ? 0.f : x[i];
+      split8<3>(x, rp);
+    };
 #pragma unroll
     for (int j = 0; j < KD; ++j) {
       const int k = MODE != 1 ? 0 : j & 1;
       if (MODE != 1) load_rows(f[1], Qs, j);
       else if (j + 1 < KD) load_rows(f[k ^ 1], Ks, j + 1);
-      if (j + 1 < KD) split_s(sp[(j + 1) & 1], j + 1);
+      if (MODE == 1 && j + 1 < KD) split_s(sp[(j + 1) & 1], j + 1);
       if (!LAST && j == 0) fetch_rows(cn, cin);       // of the next chunk
       if (!LAST && j == 1) fetch_own(next, cn, cin);
       mm3_add<LT>(f[k], sp[j & 1], r, rl);
@@ -443,7 +541,8 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
       if (MODE != 1) {
         if (j + 1 < KD) load_rows(f[0], Ks, j + 1);
         else load_wp(Ws, f[0]);
-        if (j == KD - 2) park_cols();
+        if (j + 1 < KD) split_s(sp[(j + 1) & 1], j + 1);
+        else make_r();
         mm3_add<LT>(f[1], sp[j & 1], o, ol);
         interleave<12, 4, 2>();
         __builtin_amdgcn_sched_barrier(0);
@@ -451,27 +550,19 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
     }
     if (MODE == 1) {
       load_wp(Ws, f[0]);
-      park_cols();
+      make_r();
     }
     bf16x8 (&fw)[LT][3] = f[0];
-    // R, U = W R (rows past the end: W is zero there)
+    // U = W R
     bf16x8 up[3];
     int bad = L;                             // first token whose value is not finite
     {
       float x[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int ti = i >> 2, e = i & 3;
-        x[i] = __builtin_fmaf(-own.gm[ti][e], r[ti][e] + rl[ti][e], ident ? 0.f : own.v[ti][e]);
-      }
-      if (nl < L)
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if ((i >> 2) * 16 + lg * 4 + (i & 3) >= nl) x[i] = 0.f;
-      bf16x8 rp[3];
-      split8<3>(x, rp);
       f32x4 u[LT];
       mm3<LT>(fw, rp, u);
+      park_cols();
+      interleave<12, 6>();
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] = u[i >> 2][i & 3];
       // A row of R or W that is not finite reaches all rows of U, or all from its own on: the last one
@@ -492,10 +583,11 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
         bad = min(bad, take_nonfinite(x, L, tok));
       }
       split8<3>(x, up);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) asm volatile("" : "+v"(up[i]));   // before the barrier
     }
     const bool some_bad = __builtin_amdgcn_readfirstlane(__any(bad < L));
-    arrived();
-    __syncthreads();                         // k, q and W were read, k^T and P are there
+    meet<0>();                               // k, q and W were read, k^T and P are there
     if (!LAST) dma(cin, 0, Ws);
     auto load_cols = [&](bf16x8 (&x)[LT][3], int dt) {
 #pragma unroll
@@ -533,17 +625,26 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
     update(2);
     interleave<MODE != 1 ? 36 : 24, 3, 3, LAST ? 0 : 2>();
     __builtin_amdgcn_sched_barrier(0);
-    if (MODE != 1) {
-      if (some_bad)
+    if (some_bad) {                          // (before the last rows' update, which they pass through)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          asm volatile("" : "+v"(S[dt][e]));    // a branch, not selects in every chunk
+          if (bad < L) S[dt][e] = NAN;
+        }
+      if (MODE != 1)
 #pragma unroll
         for (int ti = 0; ti < LT; ++ti)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            asm volatile("" : "+v"(o[ti][e]));  // a branch, not selects in every chunk
+            asm volatile("" : "+v"(o[ti][e]));
             if (ti * 16 + lg * 4 + e >= bad) o[ti][e] = NAN;
           }
+    }
+    if (MODE != 1) {
       // through a descriptor that ends with the chunk's last value: writes past it do nothing
-      const auto od = __builtin_amdgcn_make_buffer_rsrc(a.out + t0 * os + (int64_t)h * a.dv, 0, ((nl - 1) * ro + a.dv) * 4, 0x00027000);
+      const auto od = __builtin_amdgcn_make_buffer_rsrc(ob + (int64_t)c0 * os * 4, 0, ((nl - 1) * ro + a.dv) * 4, 0x00027000);
       const uint32_t at = colok ? (uint32_t)(__mul24(lg * 4, ro) + col) * 4 : 1u << 30;
 #pragma unroll
       for (int ti = 0; ti < LT; ++ti)
@@ -554,18 +655,12 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
         }
       if (!LAST) park_rows(1, 2);
     }
+    if (!LAST) split_s(sp[0], 0);
     update(4);
     update(6);
-    interleave<24, 4, 2>();
+    if (MODE == 1 || LAST) interleave<24, 4, 2>();
+    else interleave<24, 6, 2, 3>();
     __builtin_amdgcn_sched_barrier(0);
-    if (some_bad)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          asm volatile("" : "+v"(S[dt][e]));
-          if (bad < L) S[dt][e] = NAN;
-        }
   };
   int c0 = 0, ci = chunk0;
   for (; c0 + L < len; c0 += L, ++ci) chunk(std::false_type(), c0, ci);
@@ -640,11 +735,14 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
 
 // Chunkwise for 128 key channels where the rows pay (chunk_rows.h; a chunk's workspace is 200 KB for 16
 // heads, which few rows per sequence would multiply, too).  16 x 1000 tokens of 16 heads with 128 x 128
-// states: 1328 us token by token, 259 to 269 us chunkwise (a quarter of it W and P); 2 x 8192: 7.5 ms and 0.70
-// ms.  Per wave and chunk the walk issues 700 vector instructions and 168 MFMAs in 13700 cycles: 8100 of two waves' issue, 6100 of
-// the LDS that 95 reads of 1 KB per wave keep busy, the rest the barriers and the chain R -> U.  (Products, systems and
-// update each by itself, sums of two MFMAs added afterwards: 1000 vector instructions, 293 us in all; W and P read
-// by every wave from memory: 276.)
+// states: 1328 us token by token, 245 us chunkwise, 55 of it W and P, whose bytes (k and q in, W and P out: 210 MB) take
+// 42; 2 x 8192: 7.5 ms and 0.68 ms.  Per wave and chunk the walk issues some 750 vector instructions and 168 MFMAs in 11000
+// cycles: 9000 of two waves' issue, 6100 of the LDS that 95 reads of 1 KB per wave keep busy, the rest the barriers and
+// the chain R -> U.  What the walk's issue was spent on before (281 us, on the same card): outputs stored in loops over the
+// values of a descriptor that was not scalar; weights of k^T in double; 64-bit addresses of every staged element; vector work
+// behind the products instead of between them.  And the first launch's (72 us): columns of the inverse of 32 rows, dots
+// through LDS.  (Products, systems and update each by itself, sums of two MFMAs added afterwards: 1000 vector instructions,
+// 293 us in all; W and P read by every wave from memory: 276.)
 bool delta_chunk_ok(const float* qkv, int P, int Tp, int H, int G, int d, int V) {
   return chunk_rows_pay(P, Tp, 48) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(qkv) & 15) == 0 &&
@@ -679,7 +777,7 @@ void launch_delta_chunk(int dtype, float* out, const float* qkv, const void* ba,
   a.P = P; a.H = H; a.G = G; a.dv = V; a.num_slots = num_slots;
   a.wp = (bf16*)wp;
   const int64_t rows = (int64_t)(Tp / L + P) * L;
-  a.kw = reinterpret_cast<double*>(ws);
+  a.kw = reinterpret_cast<f32x2*>(ws);
   a.gam = ws + 2 * rows * H;
   a.rk = a.gam + rows * H;
   a.rq = a.rk + rows * G;

@@ -78,16 +78,6 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t src, int at, void* 
   __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, at, 0, 0, 0);
 }
 
-// a barrier that leaves the newest N memory operations on their way (a fence would wait for all)
-template <int N> __device__ __forceinline__ void meet() {
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 0x70);   // vmcnt(N) lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 // what the waves share beside the rows
 template <int D, int MODE> struct __align__(16) WalkLds {
   bf16 Ps[MODE == 1 ? 512 : 3 * L * L];      // parts of the weighted scores

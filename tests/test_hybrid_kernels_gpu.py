@@ -1153,6 +1153,33 @@ def test_chunkwise_scans_keep_what_is_not_finite_to_later_rows(gpu, op, dt, wher
     assert not S[hit].isfinite().any() and torch.equal(S[~hit], S_w[~hit])
 
 
+@pytest.mark.parametrize("gate", ["strength", "decay"])
+@pytest.mark.parametrize("tok", [0, 1, 15, 16, 17, 31, 32, 62])
+def test_delta_systems_keep_gates_that_are_not_finite_to_later_rows(gpu, gate, tok):
+    """The triangular systems go by blocks of 16 tokens, two heads at a time: a write strength or decay that is NaN
+    in either block, of the middle one of three heads that share a key."""
+    torch.manual_seed(97)
+    H, G, d, V, lens = 6, 2, 128, 24, [63, 64]
+    m, T, n = _chunk_step(lens, [0, 5], [])
+    x, g, S0 = torch.randn(T, 2 * G * d + H * V), torch.randn(T, 2 * H), torch.randn(n, H, d, V)
+    x[:, G * d: 2 * G * d] += 2 * torch.randn(G * d)
+    a, b, mg = torch.full((H,), -1.0).to(gpu), torch.zeros(H).to(gpu), _to(m, gpu)
+
+    def both():
+        S = S0.to(gpu)
+        return ops.gated_delta_scan(x.to(gpu), g.to(gpu), a, b, S, mg, H, G, d, V).cpu().view(T, H, V), S.cpu()
+    want, S_w = both()
+    assert want.isfinite().all() and S_w.isfinite().all()
+    h, t = 4, lens[0] + tok
+    g[t, h + (H if gate == "decay" else 0)] = float("nan")
+    got, S = both()
+    hit, hit_S = torch.zeros(T, H, V, dtype=torch.bool), torch.zeros(n, H, d, V, dtype=torch.bool)
+    hit[t:, h] = True
+    hit_S[int(m.state_slots[1]), h] = True
+    assert not got[hit].isfinite().any() and torch.equal(got[~hit], want[~hit])
+    assert not S[hit_S].isfinite().any() and torch.equal(S[~hit_S], S_w[~hit_S])
+
+
 @pytest.mark.parametrize("where,val", [("v", float("nan")), ("v", float("-inf")), ("k", float("nan")), ("gate", float("nan"))])
 @pytest.mark.parametrize("op,lens,before,at", [
     (op, lens, before, at) for op, lens, before in (("mlstm", [45, 700, 400], [0, 7, 0]), ("mlstm", [780, 33], [0, 5]),
