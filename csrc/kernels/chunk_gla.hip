@@ -5,8 +5,8 @@
 // S_0 the state before it (products channel by channel):
 //     O   = (Q p) S_0 + A V,     A_ts = sum_c q_tc k_sc alpha_(s+1)c .. alpha_tc  (s <= t)
 //     S_L = diag(p_L) S_0 + (K r)^T V
-// Q p, K r, p_L and A depend on no state: a first launch computes them for all chunks at once, A by
-// running products from every s upwards (no quotient of products, so no decay is too small).  The walk
+// Q p, K r, p_L and A depend on no state: a first launch computes them for all chunks at once, A from products
+// of decays alone (no quotient of products, so no decay is too small).  The walk
 // then has no serial step finer than a chunk: a workgroup of 8 waves owns 128 value columns of a head,
 // a wave 16 of them with their S in accumulators.
 //
@@ -16,11 +16,13 @@
 // Few long sequences are cut into segments: one walk makes every segment's contribution from a zero state, a
 // small launch puts the states together in which the segments start, and the second walk has them all.
 //
-// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 259 us, 110 of them the first
-// launch (its LDS let two workgroups share a CU, and scalar LDS reads and shuffles held those up: 250; 148 MB
-// written) and 145 the walk (splitting S beside the MFMAs, operands a step ahead: 190 without, and reading those
-// 148 MB); 2 x 8192 410 (one walk per sequence: 1562), 1 x 4000 127 (659); token by token 1340 and 8140.  From
-// float64, relative norm: outputs 7.3e-7, states 1.04e-6.
+// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 214 us, 65 of them the first launch and 145 the
+// walk (splitting S beside the MFMAs, operands a step ahead: 190 without, and reading the 148 MB of the first).  The
+// first launch was 110 to 119 with A by vector instructions from running products and the decays by expf and log1pf:
+// it is bound by issue (1650 instructions a wave, of them 480 for the decays, 200 for products in double)
+// and by the 148 MB.  2 x 8192 351 (411; one walk per sequence: 1562), 1 x 4000 107 (127; 659), 4 x 60 21 (31); token by
+// token 1340 and 8140.  From float64, relative norm, 4 x 700 tokens: outputs 2.1e-7, states 2.3e-7 (9.1e-7 and
+// 1.3e-6 with expf, whose argument's rounding is the same for all of a sequence's decays).
 #include <type_traits>
 #include "chunk.h"
 #include "chunk_rows.h"
@@ -55,155 +57,278 @@ struct GlaArgs {
   float* seg_state;                          // [items][H][D][dv]: contribution, then state a segment starts from
 };
 
-// sum over eight neighbouring lanes, without the LDS
-__device__ __forceinline__ float sum8(float x) {
+// sum over the sixteen lanes of a row, without the LDS
+__device__ __forceinline__ float sum16(float x) {
   auto other = [](float y, auto ctrl) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), decltype(ctrl)::value, 0xf, 0xf, true));
   };
-  x += other(x, std::integral_constant<int, 0xb1>());     // lanes 1 0 3 2
-  x += other(x, std::integral_constant<int, 0x4e>());     // lanes 2 3 0 1
-  return x + other(x, std::integral_constant<int, 0x141>());   // the eight in reverse
+  x += other(x, std::integral_constant<int, 0x128>());    // rotated by 8, 4, 2, 1
+  x += other(x, std::integral_constant<int, 0x124>());
+  x += other(x, std::integral_constant<int, 0x122>());
+  return x + other(x, std::integral_constant<int, 0x121>());
 }
 
-// q p, k r, p_L and A of every chunk: one workgroup per (chunk, head)
-template <typename T>
-__global__ __launch_bounds__(256) void gla_prep_kernel(const GlaArgs a) {
-  // 49 KB, so that three workgroups share a CU: the bottleneck's rows lie where the decays come, A where k was
-  __shared__ __align__(16) float qs[L][D], ks[L][D], al[L][D];
-  __shared__ double half[D];
-  static_assert(RMAX <= D && L + 4 <= D, "");
-  float (&lw)[L][D] = al;
-  float (*X)[L + 4] = reinterpret_cast<float (*)[L + 4]>(&ks[0][0]);
+// sigmoid(x)^(1 / tau) = e^g, g = (min(x, 0) - log(1 + y)) / tau, y = e^-|x|.  The logarithm is 2 atanh(s), s =
+// y / (2 + y) <= 1/3, by its series to s^17 (what is left is 2^-29 of it), s with the division's remainder.
+// e^g = 2^n e^f, |f| <= log(2) / 2, by its series to f^7 (left: 2^-27): rounded once where n is 0, as a sequence's
+// errors add up with its decays'.
+__device__ __forceinline__ float decay(float x, float inv_tau) {
+  const float y = __builtin_amdgcn_exp2f(-1.44269504f * fabsf(x)), rc = __builtin_amdgcn_rcpf(2.f + y);
+  float s = y * rc;
+  s = __builtin_fmaf(__builtin_fmaf(-s, y, __builtin_fmaf(-2.f, s, y)), rc, s);
+  const float z = s * s;
+  float t = 2.f / 17.f;
+  t = __builtin_fmaf(t, z, 2.f / 15.f);
+  t = __builtin_fmaf(t, z, 2.f / 13.f);
+  t = __builtin_fmaf(t, z, 2.f / 11.f);
+  t = __builtin_fmaf(t, z, 2.f / 9.f);
+  t = __builtin_fmaf(t, z, 2.f / 7.f);
+  t = __builtin_fmaf(t, z, 2.f / 5.f);
+  t = __builtin_fmaf(t, z, 2.f / 3.f);
+  t = __builtin_fmaf(t * z, s, 2.f * s);
+  float g = (fminf(x, 0.f) - t) * inv_tau;
+  g = g < -150.f ? -150.f : g;               // (0 in 32 bits; NaN stays)
+  const float n = __builtin_rintf(1.44269504f * g);
+  const float f = __builtin_fmaf(n, 1.90465432e-9f, __builtin_fmaf(n, -0.693147182f, g));
+  float e = 1.f / 5040.f;
+  e = __builtin_fmaf(e, f, 1.f / 720.f);
+  e = __builtin_fmaf(e, f, 1.f / 120.f);
+  e = __builtin_fmaf(e, f, 1.f / 24.f);
+  e = __builtin_fmaf(e, f, 1.f / 6.f);
+  e = __builtin_fmaf(e, f, 0.5f);
+  e = __builtin_fmaf(e * f, f, f);
+  return __builtin_amdgcn_ldexpf(1.f + e, (int)n);
+}
+
+// q p, k r, p_L and A of every chunk: one workgroup per (chunk, head), a wave has 32 channels and each of its lanes
+// two of them for eight tokens, 8 lg on; no wave waits for another before the end.  The
+// decays come out of the matrix cores in that form.  A by halves: for a block of 2 n tokens, those t of its second half with
+// those s of its first are (q_t decays from the middle to t) . (k_s decays after s to the middle), so a tile of 16 x 16
+// has all blocks of one size, in fp32 MFMAs, with what lies between two blocks left out (n = 16, 8, 4, 2); the
+// rest, s = t and t - 1 in pairs, is summed over lanes.  VEC: rows of pairs, and fours of the decays' rank.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void gla_prep_kernel(const GlaArgs a) {
+  __shared__ __align__(16) float Z[4][L][36];          // a wave's rows of q and of k, then its part of A
   const SegItem it = seg_item(blockIdx.x, a.qsl, a.P, L);
   if (it.seq < 0) return;
-  const int h = blockIdx.y, tid = threadIdx.x;
+  const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c0 = it.idx * L, len = a.qsl[it.seq + 1] - a.qsl[it.seq], nl = min(L, len - c0);
   const int slot = a.slots[it.seq];
   if (nl <= 0 || slot < 0 || slot >= a.num_slots || a.seq_lens[it.seq] < len) return;
   const int64_t t0 = a.qsl[it.seq] + c0, at = (int64_t)blockIdx.x * a.H + h;
-  const T* proj = reinterpret_cast<const T*>(a.proj) + t0 * a.ps;
+  const int ch = wave * 32 + 2 * lr;
+  const T* proj = reinterpret_cast<const T*>(a.proj) + t0 * a.ps + h * D;
   const T* low = reinterpret_cast<const T*>(a.low) + t0 * a.ls;
-  for (int e = tid; e < nl * a.R; e += 256) {
-    const int t = e / a.R, j = e - t * a.R;
-    lw[t][j] = to_f(low[t * a.ls + j]);
+  typedef T T2 __attribute__((ext_vector_type(2)));
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  // the decays' arguments: token rows 8 (m >> 2) + (m & 3) (+ 4), columns this lane's channels
+  f32x4 x[2][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int tm = 8 * (lr >> 2) + (lr & 3);
+  T2 qv[8], kv[8];
+  const T* qr = proj + min(8 * lg, nl - 1) * a.ps + ch;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {              // (rows past the end: the last one again)
+    if (i > 0) qr += 8 * lg + i < nl ? a.ps : 0;
+    const T* kr = qr + (int64_t)a.H * D;
+    if constexpr (VEC) {
+      qv[i] = *reinterpret_cast<const T2*>(qr);
+      kv[i] = *reinterpret_cast<const T2*>(kr);
+    } else {
+      qv[i] = T2{qr[0], qr[1]};
+      kv[i] = T2{kr[0], kr[1]};
+    }
+  }
+  for (int j0 = 0; j0 < a.R; j0 += 16) {
+    f32x4 lv[2], wv[2];
+    const int j = j0 + 4 * lg;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const T* lp = low + min(tm + 4 * n, nl - 1) * a.ls;
+      const float* wp = a.a2 + (int64_t)h * D * a.R + (ch + n) * a.R;
+      if constexpr (VEC) {
+        const int jj = min(j, a.R - 4);
+        const T4 u = *reinterpret_cast<const T4*>(lp + jj);
+        wv[n] = *reinterpret_cast<const f32x4*>(wp + jj);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lv[n][i] = to_f(u[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          lv[n][i] = to_f(lp[min(j + i, a.R - 1)]);
+          wv[n][i] = wp[min(j + i, a.R - 1)];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        lv[n][i] = j + i < a.R ? lv[n][i] : 0.f;
+        wv[n][i] = j + i < a.R ? wv[n][i] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) x[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(lv[n][i], wv[m][i], x[n][m], 0, 0, 0);
   }
   const float scale = 1.f / sqrtf((float)D);
-  constexpr int V = 16 / sizeof(T);          // elements of 16 bytes
-  if (a.ps % V == 0 && reinterpret_cast<uintptr_t>(a.proj) % 16 == 0) {
-    typedef T TV __attribute__((ext_vector_type(V)));
-    for (int e = tid * V; e < L * D; e += 256 * V) {
-      const int t = e / D, c = e % D;
-      const T* row = proj + min(t, nl - 1) * a.ps + h * D + c;
-      const TV q = *reinterpret_cast<const TV*>(row), k = *reinterpret_cast<const TV*>(row + (int64_t)a.H * D);
+  float q[8][2], k[8][2], al[8][2], u[8][2], w[8][2];
 #pragma unroll
-      for (int i = 0; i < V; ++i) {
-        qs[t][c + i] = t < nl ? to_f(q[i]) * scale : 0.f;
-        ks[t][c + i] = t < nl ? to_f(k[i]) : 0.f;
-      }
+  for (int m = 0; m < 2; ++m) {
+    const float bias = a.a2b[h * D + ch + m];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float f = decay(x[i >> 2][m][i & 3] + bias, a.inv_tau);
+      al[i][m] = 8 * lg + i < nl ? f : 1.f;
+      q[i][m] = 8 * lg + i < nl ? to_f(qv[i][m]) * scale : 0.f;
+      k[i][m] = 8 * lg + i < nl ? to_f(kv[i][m]) : 0.f;
     }
-  } else for (int e = tid; e < L * D; e += 256) {
-    const int t = e / D, c = e % D;
-    const T* row = proj + t * a.ps + h * D + c;
-    qs[t][c] = t < nl ? to_f(row[0]) * scale : 0.f;
-    ks[t][c] = t < nl ? to_f(row[(int64_t)a.H * D]) : 0.f;
+  }
+  // products of the decays before and after these tokens, in double; mid: of the eight between them and the chunk's middle
+  double p[2], r[2];
+  float mid[2], whole[2];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    double f = al[0][m];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) f *= al[i][m];
+    const double next = __shfl_xor(f, 16, 64), pair = f * next, far = __shfl_xor(pair, 32, 64);
+    const double both = next * far;
+    p[m] = lg == 0 ? 1.0 : lg == 1 ? next : lg == 2 ? far : both;
+    r[m] = lg == 3 ? 1.0 : lg == 2 ? next : lg == 1 ? far : both;
+    mid[m] = lg == 0 || lg == 3 ? (float)next : 1.f;
+    whole[m] = (float)(pair * far);
+  }
+  float *qo = a.qp + at * L * D, *ko = a.kr + at * L * D;
+  const int to = 8 * lg * D + ch;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    f32x2 o;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      p[m] *= al[i][m];
+      o[m] = (float)(q[i][m] * p[m]);
+    }
+    *reinterpret_cast<f32x2*>(qo + to + i * D) = o;
+  }
+#pragma unroll
+  for (int i = 7; i >= 0; --i) {
+    f32x2 o;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      o[m] = (float)(k[i][m] * r[m]);
+      r[m] *= al[i][m];
+    }
+    *reinterpret_cast<f32x2*>(ko + to + i * D) = o;
+  }
+  if (lg == 0) *reinterpret_cast<f32x2*>(a.pl + at * D + ch) = f32x2{whole[0], whole[1]};
+  // q times the decays from 8 lg on, k times those up to 8 lg + 8
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    float f = 1.f, b = 1.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      f *= al[i][m];
+      u[i][m] = q[i][m] * f;
+      w[7 - i][m] = k[7 - i][m] * b;
+      b *= al[7 - i][m];
+    }
+  }
+  float (*z)[36] = Z[wave];
+  auto settle = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto put = [&](int row, float v0, float v1) { *reinterpret_cast<f32x2*>(&z[row][2 * lr]) = f32x2{v0, v1}; };
+  auto tile = [&]() {                        // rows of q in z[0 ..], rows of k in z[16 ..]
+    settle();
+    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+    f32x4 qz[2], kz[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      qz[i] = *reinterpret_cast<const f32x4*>(&z[lr][8 * lg + 4 * i]);
+      kz[i] = *reinterpret_cast<const f32x4*>(&z[16 + lr][8 * lg + 4 * i]);
+    }
+    settle();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) d = __builtin_amdgcn_mfma_f32_16x16x4f32(qz[i >> 2][i & 3], kz[i >> 2][i & 3], d, 0, 0, 0);
+    return d;
+  };
+  f32x4 d[4];
+  {
+    const bool second = lg >= 2;
+    const int row = (second ? 0 : 16) + 8 * (lg & 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) put(row + i, (second ? u[i][0] : w[i][0]) * mid[0], (second ? u[i][1] : w[i][1]) * mid[1]);
+    d[0] = tile();
+  }
+  {
+    const bool second = lg & 1;
+    const int row = (second ? 0 : 16) + 8 * (lg >> 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) put(row + i, second ? u[i][0] : w[i][0], second ? u[i][1] : w[i][1]);
+    d[1] = tile();
+  }
+  {
+    float f[2] = {1.f, 1.f}, b[2] = {1.f, 1.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) f[m] *= al[4 + i][m];
+      put(4 * lg + i, q[4 + i][0] * f[0], q[4 + i][1] * f[1]);
+      put(16 + 4 * lg + 3 - i, k[3 - i][0] * b[0], k[3 - i][1] * b[1]);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) b[m] *= al[3 - i][m];
+    }
+    d[2] = tile();
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int i = 4 * e, row = 4 * lg + 2 * e;
+    put(row, q[i + 2][0] * al[i + 2][0], q[i + 2][1] * al[i + 2][1]);
+    put(row + 1, q[i + 3][0] * (al[i + 2][0] * al[i + 3][0]), q[i + 3][1] * (al[i + 2][1] * al[i + 3][1]));
+    put(16 + row, k[i][0] * al[i + 1][0], k[i][1] * al[i + 1][1]);
+    put(16 + row + 1, k[i + 1][0], k[i + 1][1]);
+  }
+  d[3] = tile();
+  float same[8], last[4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) same[i] = sum16(q[i][0] * k[i][0] + q[i][1] * k[i][1]);
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    last[e] = sum16(q[2 * e + 1][0] * (k[2 * e][0] * al[2 * e + 1][0]) + q[2 * e + 1][1] * (k[2 * e][1] * al[2 * e + 1][1]));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {              // tile row 4 lg + i, column lr
+    const int row = 4 * lg + i;
+    z[16 + row][lr] = d[0][i];
+    if (row >> 3 == lr >> 3) z[row + (row & 8) + 8][lr + (lr & 8)] = d[1][i];
+    if (row >> 2 == lr >> 2) z[2 * row - (row & 3) + 4][2 * lr - (lr & 3)] = d[2][i];
+    if (row >> 1 == lr >> 1) z[2 * row - (row & 1) + 2][2 * lr - (lr & 1)] = d[3][i];
+  }
+  if (lr == 0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) z[8 * lg + i][8 * lg + i] = same[i];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) z[8 * lg + 2 * e + 1][8 * lg + 2 * e] = last[e];
   }
   __syncthreads();
-  // thread (channel, half of the tokens): decays, their products up to and after each token
-  const int c = tid % D, hf = tid / D, b = hf * (L / 2);
-  {
-    float acc[L / 2];
+  {                                          // four (permuted) columns per store
+    const int t = tid >> 3, oct = (tid & 7) >> 1, s = (tid & 1) * 16 + oct * 4;
+    f32x4 v[4];
 #pragma unroll
-    for (int i = 0; i < L / 2; ++i) acc[i] = 0.f;
-    const float* ar = a.a2 + ((int64_t)h * D + c) * a.R;
-    int j = 0;
-    if (a.R % 4 == 0)                        // four at a time: a quarter of the LDS reads
-      for (; j < a.R; j += 4) {
-        f32x4 w;
+    for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const f32x4*>(&Z[i][t][s]);
+    float y[4];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) w[n] = ar[j + n];
-#pragma unroll
-        for (int i = 0; i < L / 2; ++i) {
-          const f32x4 x = *reinterpret_cast<const f32x4*>(&lw[min(b + i, nl - 1)][j]);
-#pragma unroll
-          for (int n = 0; n < 4; ++n) acc[i] += w[n] * x[n];
-        }
-      }
-    for (; j < a.R; ++j) {
-      const float w = ar[j];
-#pragma unroll
-      for (int i = 0; i < L / 2; ++i) acc[i] += w * lw[min(b + i, nl - 1)][j];
-    }
-    const float bias = a.a2b[h * D + c];
-    double p = 1.0;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < L / 2; ++i) {
-      const float x = acc[i] + bias;
-      acc[i] = b + i < nl ? expf((fminf(x, 0.f) - log1pf(expf(-fabsf(x)))) * a.inv_tau) : 1.f;
-      al[b + i][c] = acc[i];
-      p *= acc[i];
-    }
-    if (hf == 0) half[c] = p;
-    __syncthreads();
-    const double first = half[c];            // the first half's product
-    __syncthreads();
-    if (hf == 1) half[c] = p;
-    __syncthreads();
-    const double second = half[c];
-    float* qo = a.qp + at * L * D + c;
-    float* ko = a.kr + at * L * D + c;
-    p = hf ? first : 1.0;
-#pragma unroll
-    for (int i = 0; i < L / 2; ++i) {
-      p *= acc[i];
-      qo[(b + i) * D] = (float)(qs[b + i][c] * p);
-    }
-    double r = hf ? 1.0 : second;
-#pragma unroll
-    for (int i = L / 2 - 1; i >= 0; --i) {
-      ko[(b + i) * D] = (float)(ks[b + i][c] * r);
-      r *= acc[i];
-    }
-    if (hf == 0) a.pl[at * D + c] = (float)(first * second);
-  }
-  // A: thread (column s, channels 32 i + 4 g ..) carries k_s times the decays since s; eight threads read 128
-  // bytes next to each other, and a wave begins at its first column
-  {
-    const int s = tid >> 3, g = (tid & 7) * 4;
-    float w[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) w[i] = ks[s][(i >> 2) * 32 + g + (i & 3)];
-    const int s0 = __builtin_amdgcn_readfirstlane(s & ~7);
-    __syncthreads();
-    for (int t = 0; t < s0; ++t)
-      if ((tid & 7) == 0) X[t][s] = 0.f;
-    for (int t = s0; t < L; ++t) {
-      float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-      for (int i = 0; i < 16; i += 4) {
-        const f32x4 d = *reinterpret_cast<const f32x4*>(&al[t][i * 8 + g]);
-        const f32x4 q = *reinterpret_cast<const f32x4*>(&qs[t][i * 8 + g]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          w[i + e] = t > s ? w[i + e] * d[e] : w[i + e];
-          (e & 1 ? a1 : a0) += w[i + e] * q[e];
-        }
-      }
-      const float x = sum8(a0 + a1);
-      if ((tid & 7) == 0) X[t][s] = t >= s ? x : 0.f;
-    }
-  }
-  __syncthreads();
-  if (tid < L * 4) {                         // eight (permuted) columns per store
-    const int t = tid >> 2, oct = tid & 3;
-    const f32x4 x0 = *reinterpret_cast<const f32x4*>(&X[t][oct * 4]);
-    const f32x4 x1 = *reinterpret_cast<const f32x4*>(&X[t][oct * 4 + 16]);
-    const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-    bf16x8 p[3];
-    split8<3>(x, p);
+    for (int e = 0; e < 4; ++e) y[e] = s + e <= t ? (v[0][e] + v[1][e]) + (v[2][e] + v[3][e]) : 0.f;
+    uint32_t y0[3], y1[3];
+    split2<3>(y[0], y[1], y0);
+    split2<3>(y[2], y[3], y1);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-      *reinterpret_cast<bf16x8*>(a.am + at * MAT + i * L * L + t * L + oct * 8) = p[i];
+      *reinterpret_cast<u32x2*>(a.am + at * MAT + i * L * L + t * L + (tid & 7) * 4) = u32x2{y0[i], y1[i]};
   }
 }
 
@@ -436,7 +561,13 @@ __global__ __launch_bounds__(256) void gla_chain_kernel(const GlaArgs a) {
 
 template <typename T>
 void run(const GlaArgs& a, int chunks, hipStream_t s) {
-  gla_prep_kernel<T><<<dim3(chunks, a.H), 256, 0, s>>>(a);
+  auto pairs = [](const void* p, int64_t stride, int n) {
+    return stride % n == 0 && reinterpret_cast<uintptr_t>(p) % (n * sizeof(T)) == 0;
+  };
+  if (a.R % 4 == 0 && pairs(a.proj, a.ps, 2) && pairs(a.low, a.ls, 4) && reinterpret_cast<uintptr_t>(a.a2) % 16 == 0)
+    gla_prep_kernel<T, true><<<dim3(chunks, a.H), 256, 0, s>>>(a);
+  else
+    gla_prep_kernel<T, false><<<dim3(chunks, a.H), 256, 0, s>>>(a);
   const int y = a.H * ((a.dv + 127) / 128);
   if (a.seg <= 0) {
     gla_walk_kernel<T, 0><<<dim3(a.P, y), NT, 0, s>>>(a);

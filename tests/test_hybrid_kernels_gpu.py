@@ -1076,6 +1076,65 @@ def test_gla_scan_chunkwise(gpu, dt, H, V, R, lens, before, D_ctx):
             assert _whole(got, want) and _whole(st, S)
 
 
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("R", [4, 20, 128])
+def test_gla_rows_off_their_alignment(gpu, dt, R):
+    """Ranks of a part of, one and several sixteens: rows read in pairs and fours, and the same values in rows of an
+    odd stride, from an odd address or with the projection off its 16 bytes, one by one: the same bits.  Units as
+    below, and the R + 1 terms of a decay's argument."""
+    torch.manual_seed(83)
+    H, d, V, tau = 2, 128, 48, 4.0
+    m, T, n = _chunk_step([33, 64, 47], [3, 0, 0], [])
+    W = 2 * H * d + H * V
+    x, low = (torch.randn(T, W) * 0.7).to(dt), (torch.randn(T, R) * 0.7).to(dt)
+    a2, bias, S0 = torch.randn(H * d, R) * 0.3 * (16 / max(R, 16)) ** 0.5, torch.randn(H * d) + 3.0, torch.randn(n, H, d, V)
+    z = low.double() @ a2.double().T + bias.double()
+    decay = torch.exp(torch.nn.functional.logsigmoid(z) / tau).view(T, H, d)
+    q, k, v = x.double().split([H * d, H * d, H * V], 1)
+    want, unit, S, SA = _matrix64(m, S0, q.view(T, H, d) * d ** -0.5, k.view(T, H, d), v.reshape(T, H, V), decay)
+
+    def run(x, low, a2):
+        st = S0.to(gpu)
+        return ops.gla_scan(x, low, a2, bias.to(gpu), st, _to(m, gpu), H, d, V, tau), st
+    def wider(t, off):                       # rows of an odd stride, `off` elements into them
+        w = torch.zeros(t.shape[0], t.shape[1] + 8 + (t.shape[1] + 1) % 2, dtype=t.dtype)
+        w[:, off:off + t.shape[1]] = t
+        return w.to(gpu)[:, off:off + t.shape[1]]
+    a2o = torch.zeros(a2.numel() + 1)
+    a2o[1:] = a2.flatten()
+    a2o = a2o.to(gpu)[1:].view_as(a2)
+    x, low, a2 = x.to(gpu), low.to(gpu), a2.to(gpu)
+    got, st = run(x, low, a2)
+    assert ((got.cpu() - want).abs() <= (d + 64 + R) * unit + 1e-30).all()
+    assert ((st.cpu() - S).abs() <= (128 + R) * SA + 1e-30).all()
+    for args in ((wider(x, 0), low, a2), (wider(x, 3), low, a2), (x, wider(low, 1), a2), (x, low, a2o)):
+        other, st2 = run(*args)
+        assert torch.equal(other, got) and torch.equal(st2, st)
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("tau", [16.0, 0.5])
+def test_gla_prompt_decays(gpu, dt, tau):
+    """One token's decay per channel, arguments from -60 to 100, seen as what it leaves of a state of ones: the others'
+    are 1 and the keys 0.  With g the exponent, in units of 2^-24: half of one for the result, 1 for
+    its series, and 4 |g| for the logarithm, the difference and the product of which g is rounded."""
+    H, d, V, T = 1, 128, 16, 40
+    m, _, n = _chunk_step([T], [3], [])
+    a2 = torch.zeros(H * d, 4)
+    a2[:, 0] = torch.cat([torch.linspace(-60, 100, 64), torch.linspace(-3, 3, 64)])
+    a2[:, 1] = 100.0
+    x, low = torch.zeros(T, 2 * H * d + H * V, dtype=dt), torch.zeros(T, 4, dtype=dt)
+    low[:, 1] = 1.0
+    low[17] = torch.tensor([1.0, 0, 0, 0])
+    st = torch.ones(n, H, d, V).to(gpu)
+    ops.gla_scan(x.to(gpu), low.to(gpu), a2.to(gpu), torch.zeros(H * d).to(gpu), st, _to(m, gpu), H, d, V, tau)
+    g = torch.nn.functional.logsigmoid(a2[:, 0].double()) / tau
+    want = g.exp()
+    got = st[0, 0].cpu().double()
+    assert torch.equal(got, got[:, :1].expand_as(got))
+    assert ((got[:, 0] - want).abs() <= (2 + 4 * g.abs()) * want * 2.0 ** -24 + 2.0 ** -149).all()
+
+
 @pytest.mark.parametrize("dt,R", [(torch.bfloat16, 16), (torch.float16, 7), (torch.float32, 4)])
 def test_gla_scan_long_segments(gpu, dt, R):
     """Segments of seven chunks, the last one short, beside a sequence that is not cut, on two workgroups per
