@@ -59,16 +59,17 @@ __device__ __forceinline__ void mm3(const bf16x8 (&a)[N][3], const bf16x8 (&b)[3
 #pragma unroll
     for (int i = 0; i < N; ++i) c[i] = mfma16x16x32(a[i][PA[k]], b[PB[k]], k ? c[i] : f32x4{0.f, 0.f, 0.f, 0.f});
 }
-// hi + lo += a b
-template <int N>
-__device__ __forceinline__ void mm3_add(const bf16x8 (&a)[N][3], const bf16x8 (&b)[3], f32x4 (&hi)[N], f32x4 (&lo)[N]) {
+// hi + lo += a b, the columns in NB parts (one sum for both: the corrections first)
+template <int N, int NB>
+__device__ __forceinline__ void mm3_add(const bf16x8 (&a)[N][3], const bf16x8 (&b)[NB], f32x4 (&hi)[N], f32x4 (&lo)[N]) {
   constexpr int PA[6] = {0, 1, 2, 0, 1, 0}, PB[6] = {2, 1, 0, 1, 0, 0};
 #pragma unroll
   for (int k = 0; k < 6; ++k)
 #pragma unroll
     for (int i = 0; i < N; ++i) {
+      if (PB[k] >= NB) continue;
       f32x4& c = k == 5 ? hi[i] : lo[i];
-      c = mfma16x16x32(a[i][PA[k]], b[PB[k]], c);
+      c = mfma16x16x32(a[i][PA[k]], b[PB[k] < NB ? PB[k] : 0], c);
     }
 }
 
@@ -158,8 +159,8 @@ __device__ __forceinline__ double lane63(double x) {
 // that share lane & 15; PAIR: of the two that share lane & 31).  Such values become zero; returned is the column's first such token, from
 // which on its outputs and its state have to be made NaN (`none`: every value is finite).  A sum that
 // overflows only costs the closer look.
-template <bool PAIR = false, int N, typename V, typename F>
-__device__ __forceinline__ int take_nonfinite(V (&v)[N], int none, F tok) {
+// what is not finite if a value is not, or the values' sum
+template <int N, typename V> __device__ __forceinline__ float nonfinite_sum(const V (&v)[N]) {
   float z = 0.f;
   if constexpr (sizeof(V) == 2) {            // products with zeros, two at a time
     typedef V V2 __attribute__((ext_vector_type(2)));
@@ -172,6 +173,11 @@ __device__ __forceinline__ int take_nonfinite(V (&v)[N], int none, F tok) {
 #pragma unroll
     for (int i = 0; i < N; ++i) z += (float)v[i];
   }
+  return z;
+}
+template <bool PAIR = false, int N, typename V, typename F>
+__device__ __forceinline__ int take_nonfinite(V (&v)[N], int none, F tok) {
+  const float z = nonfinite_sum(v);
   int first = none;
   if (__any(!(fabsf(z) < INFINITY))) {
 #pragma unroll

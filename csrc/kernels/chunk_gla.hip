@@ -10,17 +10,20 @@
 // then has no serial step finer than a chunk: a workgroup of 8 waves owns 128 value columns of a head,
 // a wave 16 of them with their S in accumulators.
 //
-// Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each, six products of parts, the
-// corrections summed apart; products p and r are kept in double.
+// Precision: fp32 operands enter the bf16 MFMAs as three bf16 parts each, six products of parts (16-bit values
+// in as many parts as they have: three products in bf16, five in f16), the corrections of the outputs summed apart;
+// products p and r are kept in double.
 //
 // Few long sequences are cut into segments: one walk makes every segment's contribution from a zero state, a
 // small launch puts the states together in which the segments start, and the second walk has them all.
 //
-// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 214 us, 65 of them the first launch and 145 the
-// walk (splitting S beside the MFMAs, operands a step ahead: 190 without, and reading the 148 MB of the first).  The
-// first launch was 110 to 119 with A by vector instructions from running products and the decays by expf and log1pf:
-// it is bound by issue (1650 instructions a wave, of them 480 for the decays, 200 for products in double)
-// and by the 148 MB.  2 x 8192 351 (411; one walk per sequence: 1562), 1 x 4000 107 (127; 659), 4 x 60 21 (31); token by
+// Measured (8 heads, 256 value columns, rank 16): 32 x 512 tokens 181 us, 65 of them the first launch and 125 (in a
+// trace) the walk.  The first launch was 110 to 119 with A by vector instructions from running products and the decays by
+// expf and log1pf: it is bound by issue (1650 instructions a wave, of them 480 for the decays, 200 for products in
+// double) and by 148 MB written.  The walk was 158 with values in three parts, a barrier on either side of the operands'
+// writing that waited for memory, p_L from memory: it is bound by issue, per wave and chunk 420 vector
+// instructions (40 % of them split S), 78 MFMAs, 80 others; from the same addresses and without writing outputs it
+// takes 15 us less.  2 x 8192 283 (411; one walk per sequence: 1562), 1 x 4000 96 (127; 659), 4 x 60 20 (31); token by
 // token 1340 and 8140.  From float64, relative norm, 4 x 700 tokens: outputs 2.1e-7, states 2.3e-7 (9.1e-7 and
 // 1.3e-6 with expf, whose argument's rounding is the same for all of a sequence's decays).
 #include <type_traits>
@@ -335,7 +338,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void gla_prep_kernel(c
 // MODE 0: whole sequences; 1: segments from zero (states only); 2: segments from the states that they start in
 template <typename T, int MODE>
 __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
-  __shared__ __align__(16) bf16 Qs[MODE == 1 ? 8 : 3 * L * DP], KT[3 * D * LP];
+  // twice: (k r)^T, q p (parts), A, p_L
+  constexpr int QS = 3 * D * LP * 2, AS = QS + (MODE == 1 ? 0 : 3 * L * DP * 2), PS = AS + (MODE == 1 ? 0 : NT * 16), HALF = PS + NT * 4;
+  __shared__ __align__(16) char sm[2 * HALF];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
   const int nct = (a.dv + 127) / 128;
   int seq = blockIdx.x, seg_idx = 0, seg_count = 1, item = 0;
@@ -365,6 +370,8 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
       for (int t = lg; t < len; t += 4) a.out[(start + t) * os + (int64_t)h * a.dv + col] = 0.f;
     return;
   }
+  // parts of a value, products of two row tiles with them
+  constexpr int NV = sizeof(T) == 4 ? 3 : __is_same(T, bf16) ? 1 : 2, NM = NV == 1 ? 6 : NV == 2 ? 10 : 12;
   f32x4 S[DT];
   float* Ss = a.S + ((int64_t)slot * a.H + h) * D * a.dv;
   float* mine = a.seg_state + ((int64_t)item * a.H + h) * D * a.dv;
@@ -376,156 +383,250 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
     for (int r = 0; r < 4; ++r) S[i][r] = zero ? 0.f : from[(i * 16 + 4 * lg + r) * a.dv + colc];
   const T* vb = reinterpret_cast<const T*>(a.proj) + 2 * (int64_t)a.H * D + (int64_t)h * a.dv + colc;
   // Staging: a thread takes 8 columns of one row of q p, and 8 tokens of one column of k r, in both
-  // cases the pieces 4 i .. and 16 + 4 i .. of 32: adjacent in the permuted order, one store.
+  // cases the pieces 4 i .. and 16 + 4 i .. of 32: adjacent in the permuted order, one store.  A and p_L as they are
+  // (threads past the end of A: its last piece again; four copies of p_L).
   f32x4 rq[2], rt[2];
-  const int ut = tid / 16, uc = (tid % 16 / 4) * 32 + (tid % 4) * 4, up_ = (tid % 16) * 8;
+  u32x4 ra;
+  float rp;
+  const int ut = tid / 16, uc = (tid % 16 / 4) * 32 + (tid % 4) * 4;
   const int ta = tid / D * 4, tc = tid % D;
-  const int chunk0 = chunks_before<L>(seq, a.qsl) + (MODE != 0 ? seg_idx * (a.seg / L) : 0);
-  auto fetch = [&](int ci) {
-    const int64_t at = ((int64_t)ci * a.H + h) * L * D;
+  const int qat = ut * D + uc, kat = ta * D + tc, aat = min(tid, MAT / 8 - 1) * 8;
+  const int chunk0 = __builtin_amdgcn_readfirstlane(chunks_before<L>(seq, a.qsl)) + (MODE != 0 ? seg_idx * (a.seg / L) : 0);
+  auto fetch_q = [&](int ci) {
+    const int64_t at = (int64_t)ci * a.H + h;
+    const float* qp = a.qp + at * L * D;
     if (MODE != 1) {
-      rq[0] = *reinterpret_cast<const f32x4*>(a.qp + at + ut * D + uc);
-      rq[1] = *reinterpret_cast<const f32x4*>(a.qp + at + ut * D + uc + 16);
-    }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) rt[i >> 2][i & 3] = a.kr[at + (ta + (i >> 2) * 16 + (i & 3)) * D + tc];
+      for (int i = 0; i < 2; ++i) rq[i] = *reinterpret_cast<const f32x4*>(qp + qat + 16 * i);
+      ra = *reinterpret_cast<const u32x4*>(a.am + at * MAT + aat);
+    }
+    rp = (a.pl + at * D)[tc];
   };
-  auto park = [&]() {
+  auto fetch_k = [&](int ci) {
+    const float *k0 = a.kr + ((int64_t)ci * a.H + h) * L * D, *k1 = k0 + 16 * D;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      rt[0][i] = k0[kat + i * D];
+      rt[1][i] = k1[kat + i * D];
+    }
+  };
+  bf16x8 pq[3], pk[3];
+  auto split_f = [&](const f32x4 (&x)[2], bf16x8 (&p)[3]) {
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = x[i >> 2][i & 3];
+    split8<3>(y, p);
+  };
+  auto park_q = [&](char* m) {
+    if (MODE != 1) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(m + QS + (i * L * DP + ut * DP + (tid % 16) * 8) * 2) = pq[i];
+    }
+  };
+  auto park_k = [&](char* m) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(m + ((i * D + tc) * LP + ta * 2) * 2) = pk[i];
+    if (MODE != 1) *reinterpret_cast<u32x4*>(m + AS + tid * 16) = ra;
+    reinterpret_cast<float*>(m + PS)[tid] = rp;
+  };
+  bf16x8 sp[2][3];                           // parts of 32 rows of S; the first ones of the next chunk
+  auto split_s = [&](int j) {
     float x[8];
-    bf16x8 p[3];
-    if (MODE != 1) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = rq[i >> 2][i & 3];
-      split8<3>(x, p);
-#pragma unroll
-      for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(Qs + i * L * DP + ut * DP + up_) = p[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = rt[i >> 2][i & 3];
-    split8<3>(x, p);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(KT + (i * D + tc) * LP + ta * 2) = p[i];
+    for (int i = 0; i < 8; ++i) x[i] = S[2 * j + (i >> 2)][i & 3];
+    split8<3>(x, sp[j & 1]);
   };
-  fetch(chunk0);
-  for (int c0 = 0, ci = chunk0; c0 < len; c0 += L, ++ci) {
-    const int nl = min(L, len - c0);
-    park();
-    __syncthreads();
-    const int64_t t0 = start + c0, at = (int64_t)ci * a.H + h;
-    // this lane's v (tokens 4 lg + r of each tile), its fragments of A, the channels' decays
-    T v[LT][4];
-#pragma unroll
-    for (int ti = 0; ti < LT; ++ti)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[ti][r] = vb[(t0 + min(ti * 16 + lg * 4 + r, nl - 1)) * a.ps];
-    bf16x8 fp[LT][3];
-    if (MODE != 1)
+  fetch_q(chunk0);
+  fetch_k(chunk0);
+  if (MODE != 1) {
+    split_s(0);
+    split_f(rq, pq);
+  }
+  split_f(rt, pk);
+  park_q(sm);
+  park_k(sm);
+  const T* vrow = vb + (int64_t)(start + 4 * lg) * a.ps;
+  char* ob = reinterpret_cast<char*>(a.out + start * os);
+  const uint32_t oat = colok ? (4 * lg * (int)os + h * a.dv + col) * 4 : 1u << 30;
+  bf16x8 fa[2][2][3];                        // two row tiles of an operand, a step ahead
+  auto load_q = [&](const char* m, int j) {
 #pragma unroll
     for (int ti = 0; ti < LT; ++ti)
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        fp[ti][i] = *reinterpret_cast<const bf16x8*>(a.am + at * MAT + i * L * L + (ti * 16 + lr) * L + lg * 8);
+        fa[j & 1][ti][i] = *reinterpret_cast<const bf16x8*>(m + QS + (i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8) * 2);
+  };
+  // MODE 1: a chunk is over before memory answers, so its loads are those of the one after the next
+  T v[LT][4];                                // this lane's v, tokens 4 lg + r of each tile
+  auto ask_v = [&](int c0) {                 // (rows past the end: the last one again)
+    const int nl = min(L, len - c0);
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti) {
+      const T* row = vb + (int64_t)(start + c0 + min(ti * 16 + lg * 4, nl - 1)) * a.ps;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (r > 0) row += ti * 16 + lg * 4 + r < nl ? a.ps : 0;
+        v[ti][r] = *row;
+      }
+    }
+  };
+  const int chunk1 = chunk0 + (len - 1) / L; // the last one
+  if (MODE == 1) {
+    ask_v(0);
+    fetch_q(min(chunk0 + 1, chunk1));
+    fetch_k(min(chunk0 + 1, chunk1));
+  }
+  meet<63>();
+  if (MODE != 1) load_q(sm, 0);
+  // A chunk: the next one is asked for beside the products with S and put into the other half of the LDS beside the
+  // state's update.  One barrier a chunk, which waits for no memory, before the update's last step: by then every wave has
+  // read what this half holds, and the next chunk's first operands come beside that step.  (The last chunk
+  // is a copy without these.)
+  auto chunk = [&](auto last, int c0, int ci, int half) {
+    constexpr bool LAST = decltype(last)::value;
+    const int nl = LAST ? len - c0 : L;
+    const char* m = sm + half * HALF;
+    char* mn = sm + (HALF - half * HALF);
+    if (MODE != 1)
+#pragma unroll
+    for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (LAST) v[ti][r] = vb[(int64_t)(start + c0 + min(ti * 16 + lg * 4 + r, nl - 1)) * a.ps];
+        else v[ti][r] = vrow[(int64_t)(ti * 16 + r) * a.ps];
+      }
+    vrow += (int64_t)L * a.ps;
     f32x4 o[LT], ol[LT];
-    bf16x8 fa[2][2][3];                      // two row tiles, a step ahead
+    bf16x8 fp[LT][3], vp[NV];
+    T x[8];
+    float z;
+    auto tok = [&](int i) { return (i >> 2) * 16 + lg * 4 + (i & 3); };
+    auto parts = [&]() {
+      if constexpr (NV == 1) {
+        vp[0] = bf16x8{x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]};
+      } else {
+        float y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = to_f(x[i]);
+        split8<NV>(y, vp);
+      }
+    };
+    auto split_v = [&]() {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = !LAST || tok(i) < nl ? v[i >> 2][i & 3] : (T)0.f;
+      z = nonfinite_sum(x);
+      parts();
+    };
+    __builtin_amdgcn_sched_barrier(0);
     if (MODE != 1) {
 #pragma unroll
       for (int ti = 0; ti < LT; ++ti) o[ti] = ol[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
-      bf16x8 sp[2][3];                       // parts of 32 rows of S, likewise
-      auto load_q = [&](int j) {
-#pragma unroll
-        for (int ti = 0; ti < LT; ++ti)
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-            fa[j & 1][ti][i] = *reinterpret_cast<const bf16x8*>(Qs + i * L * DP + (ti * 16 + lr) * DP + j * 32 + lg * 8);
-      };
-      auto split_s = [&](int j) {
-        float x[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = S[2 * j + (i >> 2)][i & 3];
-        split8<3>(x, sp[j & 1]);
-      };
-      load_q(0);
-      split_s(0);
-      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < KD; ++j) {
         if (j + 1 < KD) {
-          load_q(j + 1);
+          load_q(m, j + 1);
           split_s(j + 1);
+        } else {
+#pragma unroll
+          for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+              fp[ti][i] = *reinterpret_cast<const bf16x8*>(m + AS + (i * L * L + (ti * 16 + lr) * L + lg * 8) * 2);
+          split_v();
         }
-        f32x4 main[LT];                      // (rounded into its sum once per step)
-#pragma unroll
-        for (int ti = 0; ti < LT; ++ti) main[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
-        mm3_add(fa[j & 1], sp[j & 1], main, ol);
-#pragma unroll
-        for (int ti = 0; ti < LT; ++ti) o[ti] += main[ti];
-        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
-        interleave<12, 4>();
+        if (!LAST && j == 0) fetch_q(ci + 1);
+        if (!LAST && j == 1) fetch_k(ci + 1);
+        mm3_add(fa[j & 1], sp[j & 1], o, ol);
+        if (!LAST && j < 2) interleave<12, 4, 2, 1>();
+        else if (j + 1 < KD) interleave<12, 4, 2>();
+        else interleave<12, NV == 1 ? 2 : 6, 2>();
         __builtin_amdgcn_sched_barrier(0);
       }
+    } else {
+      split_v();
     }
-    fetch(c0 + L < len ? ci + 1 : ci);       // (the last one again at the end: no branch)
-    bf16x8 vp[3];
-    int bad;
-    {
-      float x[8];
-      auto tok = [&](int i) { return (i >> 2) * 16 + lg * 4 + (i & 3); };
+    float badf = 0.f;                        // what a column's state adds up from
+    if (__builtin_amdgcn_readfirstlane(__any(!(fabsf(z) < INFINITY)))) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = tok(i) < nl ? to_f(v[i >> 2][i & 3]) : 0.f;
-      bad = take_nonfinite(x, L, tok);
-      split8<3>(x, vp);
+      for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(vp[i]));   // a branch, not selects in every chunk
+      const int bad = take_nonfinite(x, L, tok);
+      parts();
+      badf = bad < L ? NAN : 0.f;
+      if (MODE != 1)
+#pragma unroll
+        for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (ti * 16 + lg * 4 + e >= bad) ol[ti][e] = NAN;
     }
-    const bool some_bad = __any(bad < L);
-    float* oc = a.out + t0 * os + (int64_t)h * a.dv + col;
-    if (MODE != 1)
-#pragma unroll
-    for (int ti = 0; ti < LT; ++ti) {
-      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
-      mm<true, 3, 3>(fp[ti], vp, hi, lo);
-      if (some_bad)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) hi[e] = ti * 16 + lg * 4 + e >= bad ? NAN : hi[e];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = ti * 16 + lg * 4 + e;
-        if (colok && t < nl) oc[t * os] = (o[ti][e] + hi[e]) + (ol[ti][e] + lo[e]);
-      }
-    }
-    f32x4 u[2][2], lo[2][2], pl[2][2];       // products of two row tiles, their corrections and decays
+    f32x4 u[2][2], pl[2][2];                 // products of two row tiles, their decays
     auto load_k = [&](int q) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-          fa[q & 1][t][i] = *reinterpret_cast<const bf16x8*>(KT + (i * D + (2 * q + t) * 16 + lr) * LP + lg * 8);
-        pl[q & 1][t] = *reinterpret_cast<const f32x4*>(a.pl + at * D + (2 * q + t) * 16 + 4 * lg);
+          fa[q & 1][t][i] = *reinterpret_cast<const bf16x8*>(m + ((i * D + (2 * q + t) * 16 + lr) * LP + lg * 8) * 2);
+        pl[q & 1][t] = *reinterpret_cast<const f32x4*>(m + PS + ((2 * q + t) * 16 + 4 * lg) * 4);
       }
     };
     auto add = [&](int q) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) S[2 * q + t][e] = __builtin_fmaf(S[2 * q + t][e], pl[q & 1][t][e], u[q & 1][t][e] + lo[q & 1][t][e]);
+        for (int e = 0; e < 4; ++e) S[2 * q + t][e] = __builtin_fmaf(S[2 * q + t][e], pl[q & 1][t][e], u[q & 1][t][e]);
     };
     load_k(0);
+    if (MODE != 1) {
+      mm3_add(fp, vp, o, ol);
+      if (!LAST) split_f(rq, pq);
+      interleave<NM, 48 / NM, 1>();
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < DT / 2; ++q) {
+      if (!LAST && q == 3) {
+        meet<63>();
+        if (MODE != 1) load_q(mn, 0);
+      }
 #pragma unroll
-      for (int t = 0; t < 2; ++t) u[q & 1][t] = lo[q & 1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-      mm3_add(fa[q & 1], vp, u[q & 1], lo[q & 1]);
+      for (int t = 0; t < 2; ++t) u[q & 1][t] = f32x4{badf, badf, badf, badf};
+      mm3_add(fa[q & 1], vp, u[q & 1], u[q & 1]);
       if (q > 0) add(q - 1);
       if (q + 1 < DT / 2) load_k(q + 1);
+      if (q == 0 && MODE != 1) {
+        // through a descriptor that ends with the chunk's last row: writes past it do nothing
+        const auto od = __builtin_amdgcn_make_buffer_rsrc(ob + (int64_t)c0 * os * 4, 0, nl * (int)os * 4, 0x00027000);
+#pragma unroll
+        for (int ti = 0; ti < LT; ++ti)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float y = o[ti][e] + ol[ti][e];
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), od, oat + (ti * 16 + e) * (int)os * 4, 0, 0);
+          }
+      }
+      if (!LAST) {
+        if (q == 0) split_f(rt, pk);
+        if (q == 1) {
+          park_q(mn);
+          park_k(mn);
+        }
+        if (q == 2 && MODE == 1) {
+          ask_v(c0 + L);
+          fetch_q(min(ci + 2, chunk1));
+          fetch_k(min(ci + 2, chunk1));
+        }
+        if (q == 3 && MODE != 1) split_s(0);
+      }
+      if (q == 0 && MODE != 1) interleave<NM, 72 / NM, 1, 1>();
+      else if (q == 3) interleave<NM, 60 / NM, 1>();
+      else interleave<NM, 4, 1>();
       __builtin_amdgcn_sched_barrier(0);
     }
     add(DT / 2 - 1);
-    if (some_bad)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S[dt][e] = bad < L ? NAN : S[dt][e];
-    __syncthreads();
-  }
+  };
+  int c0 = 0, ci = chunk0, half = 0;
+  for (; c0 + L < len; c0 += L, ++ci, half ^= 1) chunk(std::false_type{}, c0, ci, half);
+  chunk(std::true_type{}, c0, ci, half);
   float* dst = MODE == 1 ? mine : Ss;
   if (colok && (MODE != 2 || seg_idx + 1 == seg_count))
 #pragma unroll
