@@ -694,8 +694,7 @@ int plan(int P, int Tp, int H, int V, int* items) {
 }  // namespace
 
 bool gla_chunk_ok(int P, int Tp, int H, int d, int V, int R) {
-  // 1 x 48 tokens 46 -> 35 us, 64 x 48 218 -> 120, 4 x 60 63 -> 42; fewer rows: chunk_rows.h
-  return chunk_rows_pay(P, Tp, 32) && d == D && V >= 16 && R <= RMAX &&
+  return chunk_rows_pay(P, Tp, {11, 7, 4, 3}) && d == D && V >= 16 && R <= RMAX &&
          chunk_fits(0, (long)H * V, (long)H * ((V + 127) / 128));   // (row offsets have 64 bits)
 }
 // floats of workspace

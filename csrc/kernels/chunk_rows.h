@@ -11,20 +11,22 @@ inline bool chunk_fits(long stride, long cols, long blocks) {
   return stride < (1 << 22) && cols < 1000000 && blocks <= 65535;
 }
 
-// P sequences of Tp rows together; `alone`: rows from which one sequence by itself pays.  Token by token
-// a step costs its longest sequence and, once the chip is full, its rows; chunkwise it costs its chunks,
-// one at least per sequence, full or not.  Token by token -> chunkwise in us, 16 heads of 128 x 128 (delta
-// rule) and 8 of 128 x 256 (GLA):
-//                        delta           GLA
-//   1 x 24, 32, 44       22.5 -> 27.6, 27.7 -> 27.9, 36.8 -> 33.6;  26.5 -> 31.2, 31.8 -> 31.7, 43.1 -> 36.2
-//   4 x 24, 40           22.8 -> 28.5, 35.2 -> 37.7;  28.2 -> 32.7, 42.8 -> 39.8
-//   8 x 16, 24           23.8 -> 30.5, 35.4 -> 33.1;  25.7 -> 34.5, 37.2 -> 36.5
-//   32 x 12, 16          43.1 -> 47.7, 51.9 -> 48.0;  48.7 -> 50.7, 56.1 -> 52.8
-//   512 x 7, 128 x 12    386 -> 449, 152 -> 133;      509 -> 550, 173 -> 153
-//   1024 x 1             473 -> 880;                  639 -> 1044
-inline bool chunk_rows_pay(long P, long Tp, long alone) {
-  const long rows = Tp >= 1024 ? 12 : Tp >= 512 ? 16 : Tp >= 192 ? 24 : alone;
-  return P > 0 && Tp >= (rows < alone ? rows : alone) * P;
+// Rows per sequence from which P sequences of Tp rows together pay chunkwise: `rows` for fewer than 8 sequences, than 32,
+// than 128, and more.  Token by token a step costs its longest sequence and, once the chip is full, its rows;
+// chunkwise it costs its chunks, one at least per sequence, full or not.  From 1024 rows on 12 in any case: below, so
+// short rows would start more chunks than the engine's memory profile has.  Token by token -> chunkwise in
+// us, 16 heads of 128 x 128 (delta rule) and 8 of 128 x 256 (GLA), the shortest sequence three quarters of the longest:
+//                          delta                                      GLA
+//   1 x 16, 20, 24         16.0 -> 20.0, 19.8 -> 20.0, 22.5 -> 19.9;  17.9 -> 13.9, 24.0 -> 14.0, 26.6 -> 13.9
+//   1 x 8, 12              10.3 -> 19.9, 13.1 -> 19.9;                12.4 -> 13.9, 15.2 -> 13.9
+//   4 x 12, 16, 24         13.5 -> 20.8, 16.6 -> 20.8, 22.8 -> 20.7;  16.8 -> 15.4, 20.3 -> 15.4, 28.8 -> 15.3
+//   8 x 8, 12, 16          15.0 -> 21.6, 19.4 -> 21.7, 23.4 -> 21.8;  18.9 -> 16.1, 22.2 -> 16.0, 25.7 -> 16.2
+//   16 x 6, 8, 16          14.8 -> 23.7, 16.9 -> 24.1, 25.2 -> 24.2;  18.3 -> 18.4, 20.4 -> 18.7, 28.4 -> 18.8
+//   32 x 4, 8, 12          21.1 -> 35.7, 30.6 -> 35.5, 38.8 -> 35.3;  31.0 -> 30.2, 38.3 -> 30.0, 44.9 -> 29.6
+//   128 x 4, 8, 12         54.9 -> 89.2, 81.5 -> 86.8, 112 -> 88.7;   89.3 -> 69.0, 109 -> 66.4, 135 -> 68.4
+//   300 x 3, 512 x 7, 12   -, 329 -> 341, 471 -> 355;                 191 -> 173, 415 -> 294, 522 -> 303
+inline bool chunk_rows_pay(long P, long Tp, const int (&rows)[4]) {
+  return P > 0 && Tp >= P * (Tp >= 1024 ? 12 : rows[P < 8 ? 0 : P < 32 ? 1 : P < 128 ? 2 : 3]);
 }
 
 // Tokens per segment, whole chunks of L and `least` of them at least, so that P sequences of Tp rows come to at most

@@ -436,6 +436,21 @@ def test_memory_profile_covers_many_short_prompts():
     assert steps(4096, 100, 256, [()])[1] == [16] * 256 and steps(2048, 8192, 1, [()]) == [[2048]]
 
 
+def test_memory_profile_covers_small_steps_of_short_prompts():
+    """Steps of fewer than 1024 rows go chunkwise from three rows of each prompt on (the delta rule from ten): profiled
+    where that is more prompts than the large steps have."""
+    from types import SimpleNamespace
+
+    from kubernetes_gpu_cluster_amd.engine.model_runner import ModelRunner
+    steps = lambda budget, seqs, layout=((),): ModelRunner._profile_steps(SimpleNamespace(   # noqa: E731
+        token_budget=budget, max_model_len=8192, max_num_seqs=seqs, state_layout=list(layout)))
+    assert steps(2048, 1024) == [[2048], [12] * 170, [16] * 128, [25] * 81, [3] * 341]
+    assert steps(1024, 256) == [[1024], [12] * 85, [16] * 64, [25] * 40, [3] * 256, [10] * 102]
+    assert steps(1024, 60) == [[1024], [17] * 60, [25] * 40] and steps(200, 256)[-2:] == [[4] * 50, [10] * 20]
+    assert steps(2048, 1024, ()) == [[2048]]
+    assert steps(4096, 1024)[-1] == [25] * 163       # (4096 / 12 = 341 prompts already)
+
+
 def test_memory_profile_covers_images_of_chunks():
     """Where slots are many, twelve rows of each are too few for the Mamba-2 scan's images of chunks: the steps with
     the most started chunks among those that make them are profiled, too."""

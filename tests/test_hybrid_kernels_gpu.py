@@ -1239,6 +1239,41 @@ def test_delta_systems_keep_gates_that_are_not_finite_to_later_rows(gpu, gate, t
     assert not S[hit_S].isfinite().any() and torch.equal(S[~hit_S], S_w[~hit_S])
 
 
+@pytest.mark.parametrize("op,P,rows", [("delta", 1, 21), ("delta", 7, 21), ("delta", 8, 14), ("delta", 32, 10), ("delta", 90, 12),
+                                       ("gla", 1, 11), ("gla", 7, 11), ("gla", 8, 7), ("gla", 32, 4), ("gla", 128, 3),
+                                       ("gla", 341, 3), ("gla", 90, 12)])
+def test_short_prompts_on_both_sides_of_the_chunkwise_rule(gpu, op, P, rows):
+    """The fewest rows that go chunkwise (from 1024 rows on twelve of each sequence), seen by their workspace, and a row
+    less, which goes token by token: float64 within the bounds of the tests above."""
+    torch.manual_seed(98)
+    d, V, H = 128, 32, 2
+    for less in (0, 1):
+        m, T, n = _chunk_step([rows] * (P - 1) + [rows - less], [0] * P, [])
+        m.state_slots = torch.arange(n, dtype=torch.int32)
+        x, S = torch.randn(T, 2 * H * d + H * V), torch.randn(n, H, d, V) * 0.3
+        q, k, v = x.double().split([H * d, H * d, H * V], 1)
+        q, k, v, S_g, mg = q.view(T, H, d), k.view(T, H, d), v.reshape(T, H, V), S.to(gpu), _to(m, gpu)
+        if op == "delta":
+            g, a, b = torch.randn(T, 2 * H), torch.zeros(H), torch.full((H,), -2.0)
+            unit = lambda y: y * torch.rsqrt(y.pow(2).sum(-1, keepdim=True) + 1e-6)   # noqa: E731
+            decay = torch.exp(-torch.nn.functional.softplus(g[:, H:].double() - 2.0))[..., None]
+            terms, f, fs = (unit(q) * d ** -0.5, unit(k), v, decay, torch.sigmoid(g[:, :H].double())), 32, 32
+            args = (x.to(gpu), g.to(gpu), a.to(gpu), b.to(gpu), S_g, mg, H, H, d, V)
+        else:
+            g, a, b = torch.randn(T, 4), torch.randn(H * d, 4) * 0.3, torch.randn(H * d) + 3.0
+            decay = torch.exp(torch.nn.functional.logsigmoid(g.double() @ a.double().T + b.double()) / 4.0).view(T, H, d)
+            terms, f, fs = (q * d ** -0.5, k, v, decay), d + 64, 128
+            args = (x.to(gpu), g.to(gpu), a.to(gpu), b.to(gpu), S_g, mg, H, d, V, 4.0)
+        want, unit, S_w, S_u = _matrix64(m, S, *terms)
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_stats()["requested_bytes.all.allocated"]
+        got = (ops.gated_delta_scan if op == "delta" else ops.gla_scan)(*args)
+        asked = torch.cuda.memory_stats()["requested_bytes.all.allocated"] - before
+        assert (asked > 2 * got.numel() * got.element_size()) == (less == 0)
+        assert ((got.double().cpu() - want).abs() <= f * unit + 1e-30).all()
+        assert ((S_g.double().cpu() - S_w).abs() <= fs * S_u + 1e-30).all()
+
+
 @pytest.mark.parametrize("where,val", [("v", float("nan")), ("v", float("-inf")), ("k", float("nan")), ("gate", float("nan"))])
 @pytest.mark.parametrize("op,lens,before,at", [
     (op, lens, before, at) for op, lens, before in (("mlstm", [45, 700, 400], [0, 7, 0]), ("mlstm", [780, 33], [0, 5]),
