@@ -60,6 +60,14 @@ _enabled = os.environ.get("KGC_SKINNY_GEMM", "1") != "0"
 # "tail" (o / down -> residual add + RMSNorm), "sum" (any linear whose consumer adds rows or
 # K-slices itself: hyper-connected streams; also tried at M <= SKINNY_MAX_M, as "plain" is for
 # the shapes a model names).  S > 1: fp32 K-slices summed by the consumer.
+# "silu", "tail" and "qkv", whose consumers take slices, are tried from DG_MIN_M rows on: below,
+# the skinny kernels with the norms inside them have no launch to spare.  A skinny grid has a
+# workgroup per 16 or 32 columns whatever K, a K9m grid 128 or 64 columns of a slice of K: with 2048
+# columns and K 5504 172 to 256 workgroups, each with a deep pipeline, instead of 128 whose
+# loads wait for their MFMAs.  2048-wide layer, 32 rows, each with its consumer, us: qkv 8.2 ->
+# 6.2, o 10.4 -> 7.9, gate_up 19.0 -> 15.2, down 21.4 -> 11.3; 64 rows 12.4 -> 6.3, 14.7 -> 8.9,
+# 26.6 -> 17.0, 32.7 -> 12.3; 16 rows 6.6 -> 5.8, 8.8 -> 7.6, 15.0 -> 14.7, 17.2 -> 10.8.
+DG_MIN_M = 17
 DG_MAX_M = 512
 _plan_dg: dict[tuple[int, int, int, str], tuple[int, int]] = {}
 _dg_enabled = os.environ.get("KGC_DGEMM", "1") != "0"
@@ -554,7 +562,7 @@ def dgemm_plan_has_m(M: int, kind: str) -> bool:
 
 
 def tail_plan_has_m(M: int) -> bool:
-    """A fused projection-tail plan at this M: K9m split-K (M > 64) or SK_ACC_NORM."""
+    """A fused projection-tail plan at this M: K9m split-K (M >= DG_MIN_M) or SK_ACC_NORM."""
     return dgemm_plan_has_m(M, "tail") or any(k[0] == M for k in _plan_accnorm)
 
 
@@ -647,7 +655,7 @@ def tune_skinny(weights: Iterable[torch.Tensor], ms: Iterable[int], margin: floa
     norm-free layer's epilogues at M <= 16 (tail -> SK_ACC_SS, norm -> SK_RSCALE, silu ->
     SK_RSCALE_SILU) for ``rs_plan``.  ``sum_shapes``: (N, K) whose consumer sums K-slices
     (``linear_slices``), timed with ``sum_consumer(M)`` -> fn(y); ``stream_shapes``: (N, K) for
-    which K9m is also tried at M <= SKINNY_MAX_M."""
+    which K9m is also tried at M < DG_MIN_M, and as a plain projection at M <= SKINNY_MAX_M."""
     if not _enabled:
         return {}
     by_shape: dict[tuple[int, int], list[torch.Tensor]] = {}
@@ -704,7 +712,8 @@ def tune_skinny(weights: Iterable[torch.Tensor], ms: Iterable[int], margin: floa
             qd = (qkv_dims or {}).get((N, K))
             kind = ("sum" if (N, K) in sum_shapes else "silu" if (N, K) in silu_shapes else
                     "tail" if (N, K) in tail_shapes else "qkv" if qd else "plain")
-            lo = 0 if kind == "sum" or (N, K) in stream_shapes else SKINNY_MAX_M
+            lo = (0 if kind == "sum" or (N, K) in stream_shapes else
+                  SKINNY_MAX_M if kind == "plain" else DG_MIN_M - 1)
             _tune_dgemm(ws, N, K, [m for m in ms if lo < m <= DG_MAX_M], margin,
                         reps, res, kind, qd, sum_consumer)
     log.info("GEMM tuning: %d shapes in %.1f s", len(res), time.time() - t0)
@@ -731,7 +740,9 @@ def _dg_candidates(M: int, N: int, K: int, kind: str, packed: bool):
     from . import _k
     # 11-14: packed 64 / 80 / 112-wide column tiles (gemm_decode.hip kCfg) for the narrow
     # shards of a TP = 8 rank
-    cfgs = ([5, 7, 10, 2, 14, 3] if M <= SKINNY_MAX_M or (kind == "sum" and M <= 128) else
+    few = M <= SKINNY_MAX_M and kind in ("silu", "tail", "qkv")
+    cfgs = ([5, 10, 2, 14, 3, 9] if few else
+            [5, 7, 10, 2, 14, 3] if M <= SKINNY_MAX_M or (kind == "sum" and M <= 128) else
             [5, 7, 2, 14, 11] if M <= 128 else [6, 8, 4, 0, 10, 11, 12, 13, 14])
     out = []
     for c in range(_k().dgemm_num_cfgs()):
@@ -753,6 +764,8 @@ def _dg_candidates(M: int, N: int, K: int, kind: str, packed: bool):
         for S in splits:
             if S > K // 64 or (S > 1 and tiles * S > _DG_MAX_GRID):
                 continue
+            if few and tiles * S < 128:
+                continue            # (half of the CUs would idle: never the fastest)
             if S == 1 and kind == "silu" and not (epis >> 2) & 1:
                 continue
             out.append((c, S))
@@ -809,6 +822,12 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
 
         def lib():
             for w in ws:
+                if M <= SKINNY_MAX_M and kind == "silu":
+                    linear_silu(x, w)
+                    continue
+                if M <= SKINNY_MAX_M and kind == "tail":
+                    linear_add_rms(x, w, res_t, gamma, 1e-6)
+                    continue
                 y = linear(x, w) if M <= SKINNY_MAX_M else F.linear(x, w)
                 if kind == "silu":
                     silu_mul(y, act)
@@ -816,7 +835,9 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
                     fused_add_rms_norm(y, res_t, gamma, 1e-6)
                 elif kind in ("qkv", "sum"):
                     consume(y)
-        lib_t = _time(lib, reps)
+        # (a few rows' kernels are over before the next is launched eagerly: see _time_graphed)
+        first = _time_graphed if M <= SKINNY_MAX_M and kind in ("silu", "tail", "qkv") else _time
+        lib_t = first(lib, reps)
         best_t, best_cfg = float("inf"), None
         timed = []                  # (t, (cfg, S), run) of every candidate
         for cfg, S in _dg_candidates(M, N, K, kind, packed):
@@ -845,7 +866,7 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
                             _k().splitk_add_rms_norm(red, buf, res_t, gamma, 1e-6)
                         else:
                             _k().splitk_reduce(red, buf)
-            t = _time(run, reps)
+            t = first(run, reps)
             timed.append((t, (cfg, S), run))
         # refine: the few fastest candidates and the library re-timed in interleaved
         # rounds, median of each -- one short pass ranked near-ties by clock noise (the
@@ -876,6 +897,10 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
             _plan_dg[(M, N, K, kind)] = chosen
             if kind == "plain":
                 _plan.pop((M, N, K), None)
+            elif kind == "silu":    # (the skinny kernels' own plans are asked first)
+                _plan_silu.pop((M, N, K), None)
+            elif kind == "tail":
+                _plan_accnorm.pop((M, N, K), None)
         res[(M, N, K, kind)] = (chosen, lib_t * 1e3 / n, best_t * 1e3 / n, best_cfg)
         log.info("gemm M=%d N=%d K=%d %s: hipBLASLt %.1f us, K9m %s %.1f us -> %s", M, N, K,
                  kind, lib_t * 1e3 / n, best_cfg, best_t * 1e3 / n,

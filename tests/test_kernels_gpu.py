@@ -1216,6 +1216,70 @@ def test_linear_uses_tuned_plan(gpu):
 
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+@pytest.mark.parametrize("plan", [(3, 8), (14, 8), (5, 6), (10, 3), (9, 2), (2, 1)])
+def test_dgemm_plans_of_few_rows(gpu, M, plan):
+    """Rows below one row tile of K9m with what consumes them -- the residual add and norm, the SiLU pairs, slices for the
+    attention -- against fp32.  Rounding to bf16 is half of 2^-7, 2^-8 at most, of what is rounded: once for the
+    SiLU's product; for the residual the projection and the sum; the norm's row of that and its own.  1e-4 for sums of
+    K terms in fp32."""
+    from kubernetes_gpu_cluster_amd.ops import gemm
+    torch.manual_seed(M)
+    N, K = 1536, 1024
+    x, w = torch.randn(M, K, dtype=torch.bfloat16, device=gpu), torch.randn(N, K, dtype=torch.bfloat16, device=gpu) * 0.03
+    res, gamma = torch.randn(M, N, dtype=torch.bfloat16, device=gpu), torch.rand(N, dtype=torch.bfloat16, device=gpu) + 0.5
+    y = x.float().cpu() @ w.float().cpu().t()
+    gemm.pack_decode_weights([w], [w])
+    try:
+        for kind in ("silu", "tail", "qkv"):
+            gemm._plan_dg[(M, N, K, kind)] = plan
+        exp = torch.nn.functional.silu(y[:, : N // 2]) * y[:, N // 2:]
+        if plan[1] > 1 or (torch.ops.kgc.dgemm_cfg_epis(plan[0]) >> 2) & 1:
+            torch.testing.assert_close(gemm.linear_silu(x, w).float().cpu(), exp, atol=1e-4, rtol=2.0 ** -8)
+        e = 2.0 ** -8
+        want = res.float().cpu() + y
+        r = res.clone()
+        out, r2 = gemm.linear_add_rms(x, w, r, gamma, 1e-5)
+        assert ((r2.float().cpu() - want).abs() <= e * (y.abs() + (1 + e) * want.abs()) + 1e-4).all()
+        f = torch.rsqrt(want.pow(2).mean(1, keepdim=True) + 1e-5) * gamma.float().cpu()
+        # (the mean square of a row's errors is far below a rounding of its norm)
+        assert ((out.float().cpu() - want * f).abs() <= (e * (y.abs() + 2 * want.abs()) + 1e-4) * f * (1 + e) + e * (want * f).abs()).all()
+        q = gemm.linear_qkv(x, w)
+        assert q.shape == ((plan[1], M, N) if plan[1] > 1 else (M, N))
+        torch.testing.assert_close(q.float().cpu().sum(0) if plan[1] > 1 else q.float().cpu(), y, atol=1e-4,
+                                   rtol=1e-5 if plan[1] > 1 else 2.0 ** -8)
+    finally:
+        gemm.clear_plan()
+        gemm._packed.clear()
+
+
+def test_tuned_plans_of_few_rows(gpu):
+    """From 17 rows on a chosen K9m plan takes the place of the skinny epilogues that would be asked first; below,
+    and for projections without a consumer of slices, nothing is tried."""
+    from kubernetes_gpu_cluster_amd.ops import gemm
+    torch.manual_seed(6)
+    ws = [torch.randn(1024, 4096, dtype=torch.bfloat16, device=gpu) * 0.02 for _ in range(3)]
+    try:
+        for shapes in (dict(tail_shapes={(1024, 4096)}), dict(silu_shapes={(1024, 4096)})):
+            kind = "tail" if "tail_shapes" in shapes else "silu"
+            res = gemm.tune_skinny(ws, [8, 16, 32], **shapes)
+            assert {k for k in res if len(k) == 4} == {(32, 1024, 4096, kind)}
+            if (32, 1024, 4096, kind) in gemm._plan_dg:
+                assert (32, 1024, 4096) not in (gemm._plan_accnorm if kind == "tail" else gemm._plan_silu)
+            x = torch.randn(32, 4096, dtype=torch.bfloat16, device=gpu)
+            y = x.float() @ ws[0].float().t()
+            if kind == "silu":
+                torch.testing.assert_close(gemm.linear_silu(x, ws[0]).float(),
+                                           torch.nn.functional.silu(y[:, :512]) * y[:, 512:], atol=2e-2, rtol=2e-2)
+            else:
+                _, r = gemm.linear_add_rms(x, ws[0], torch.zeros(32, 1024, dtype=x.dtype, device=gpu),
+                                           torch.ones(1024, dtype=x.dtype, device=gpu), 1e-6)
+                torch.testing.assert_close(r.float(), y, atol=2e-2, rtol=2e-2)
+            gemm.clear_plan()
+    finally:
+        gemm.clear_plan()
+
+
 @pytest.mark.parametrize("M,N,K,plan", [(256, 2048, 4096, (8, 1)), (80, 1536, 2048, (5, 1)),
                                          (144, 1024, 1024, (0, 2)), (96, 2048, 2048, (2, 1)),
                                          (256, 2048, 4096, (4, 2)), (256, 7168, 1024, (6, 5)),
