@@ -11,22 +11,36 @@ inline bool chunk_fits(long stride, long cols, long blocks) {
   return stride < (1 << 22) && cols < 1000000 && blocks <= 65535;
 }
 
-// Rows per sequence from which P sequences of Tp rows together pay chunkwise: `rows` for fewer than 8 sequences, than 32,
-// than 128, and more.  Token by token a step costs its longest sequence and, once the chip is full, its rows;
-// chunkwise it costs its chunks, one at least per sequence, full or not.  From 1024 rows on 12 in any case: below, so
-// short rows would start more chunks than the engine's memory profile has.  Token by token -> chunkwise in
-// us, 16 heads of 128 x 128 (delta rule) and 8 of 128 x 256 (GLA), the shortest sequence three quarters of the longest:
-//                          delta                                      GLA
-//   1 x 16, 20, 24         16.0 -> 20.0, 19.8 -> 20.0, 22.5 -> 19.9;  17.9 -> 13.9, 24.0 -> 14.0, 26.6 -> 13.9
-//   1 x 8, 12              10.3 -> 19.9, 13.1 -> 19.9;                12.4 -> 13.9, 15.2 -> 13.9
-//   4 x 12, 16, 24         13.5 -> 20.8, 16.6 -> 20.8, 22.8 -> 20.7;  16.8 -> 15.4, 20.3 -> 15.4, 28.8 -> 15.3
-//   8 x 8, 12, 16          15.0 -> 21.6, 19.4 -> 21.7, 23.4 -> 21.8;  18.9 -> 16.1, 22.2 -> 16.0, 25.7 -> 16.2
-//   16 x 6, 8, 16          14.8 -> 23.7, 16.9 -> 24.1, 25.2 -> 24.2;  18.3 -> 18.4, 20.4 -> 18.7, 28.4 -> 18.8
-//   32 x 4, 8, 12          21.1 -> 35.7, 30.6 -> 35.5, 38.8 -> 35.3;  31.0 -> 30.2, 38.3 -> 30.0, 44.9 -> 29.6
-//   128 x 4, 8, 12         54.9 -> 89.2, 81.5 -> 86.8, 112 -> 88.7;   89.3 -> 69.0, 109 -> 66.4, 135 -> 68.4
-//   300 x 3, 512 x 7, 12   -, 329 -> 341, 471 -> 355;                 191 -> 173, 415 -> 294, 522 -> 303
-inline bool chunk_rows_pay(long P, long Tp, const int (&rows)[4]) {
-  return P > 0 && Tp >= P * (Tp >= 1024 ? 12 : rows[P < 8 ? 0 : P < 32 ? 1 : P < 128 ? 2 : 3]);
+// Whether prompt rows pay chunkwise, by what both ways take in us: token by token the states' way in and out and every
+// row, by P H ceil(V / 64) units of 64 columns; chunkwise a chunk of each sequence whatever its rows, by P H ceil(V / 128)
+// workgroups of the walk, of which a CU holds one, and P H of what goes before it.
+//     t0 + tu units (+ t1 from 192 units on) + rows max(r0, ru units)   against   max(c0 + s0 wgs, c1 + cw wgs) + cp P H
+// The constants are fitted to 3 to 12 rows of 1 to 512 sequences, rows the mean, which is less than the longest: what is
+// chosen by them was 0 to 60 % faster in 5 shapes of heads each, what is not up to 12 % slower than it could be.
+// Measured, token by token -> chunkwise:
+//                     1 x 8, 12, 24          8 x 8, 16        32 x 4, 6, 12            128 x 4, 8
+//   GLA  8 x 256      12.4, 15.2, 26.6 -> 13.9   18.9, 25.7 -> 16.1   31.0, 34.7, 44.9 -> 30   89, 109 -> 69
+//        2 x 128      11 rows 14.6 -> 13.2   12.4 -> 14.1     5 rows 12.0 -> 14.9      16.6 -> 21.8
+//        4 x 64, 512  14.4, 14.6 -> 12.9, 13.8   12.4, 19.1 -> 13.9, 15.4   5 rows 11.9, 33.6 -> 15.2, 24.9   17, 89 -> 32, 64
+//   delta 16 x 128    10.2, 12.8, 22.6 -> 19.9   15.0, 23.3 -> 21.7   21, 27, 38.7 -> 35       55, 81 -> 88
+//        4 x 128, 32 x 128   22 rows 25.2, 21.2 -> 19.8   15.7, 25.6 -> 20.2, 24.3   12 rows 20, 63 -> 21.7, 53
+//   mLSTM 4 of 256 x 512     25.2, 31.2 -> 19.0   27.1 -> 21.4   42, 49, 70 -> 42.6   151, 209 -> 139
+//        8 of 128 x 128      17.3, 21.5 -> 12.5   6 rows 16.0 -> 13.2   16.5, 18.8 -> 15.9   41, 55 -> 47
+//        16 of 128 x 64      15.3, 19.7 -> 12.3   6 rows 13.9 -> 13.1   14.5, 16.7 -> 24   39, 53 -> 79
+struct ChunkCost { double t0, tu, t1, r0, ru, c0, s0, c1, cw, cp; int least; };
+inline bool chunk_pays(const ChunkCost& k, long P, long Tp, long H, long V, double scale = 1.0) {
+  if (P <= 0 || Tp < k.least * P) return false;
+  const double units = (double)P * H * ((V + 63) / 64), wgs = (double)P * H * ((V + 127) / 128), rows = (double)Tp / P;
+  const double slope = k.ru * units > k.r0 ? k.ru * units : k.r0, a = k.c0 + k.s0 * wgs, b = k.c1 + k.cw * wgs;
+  return k.t0 + k.tu * units + (units > 192 ? k.t1 : 0) + rows * slope > scale * ((a > b ? a : b) + k.cp * P * H);
+}
+
+// The same for the scans that prepare chunks in a workspace: by the rows alone from `alone` rows of one
+// sequence on, 24 in steps of 192, 16 in steps of 512 and 12 in steps of 1024, and by the costs in steps of fewer than
+// 1024 rows (in larger ones short rows would start more chunks than the engine's memory profile has).
+inline bool chunk_rows_pay(const ChunkCost& k, long P, long Tp, long H, long V, long alone) {
+  const long rows = Tp >= 1024 ? 12 : Tp >= 512 ? 16 : Tp >= 192 ? 24 : alone;
+  return P > 0 && (Tp >= (rows < alone ? rows : alone) * P || (Tp < 1024 && chunk_pays(k, P, Tp, H, V)));
 }
 
 // Tokens per segment, whole chunks of L and `least` of them at least, so that P sequences of Tp rows come to at most

@@ -245,7 +245,7 @@ class ModelRunner:
         """Prompt steps with the largest activations: the token budget in prompts as long as
         they get, and for recurrent layers in as many as there are slots, too -- the chunkwise
         scans keep a workspace per started chunk of every sequence, from 12 rows of each on (in
-        steps of fewer than 1024 rows three, and the delta rule ten; csrc/kernels/chunk_rows.h), and the Mamba-2 scan images of the
+        steps of fewer than 1024 rows three, and the delta rule eight; csrc/kernels/chunk_rows.h), and the Mamba-2 scan images of the
         chunks' keys, from 16 rows of each on with few groups and 25 with many
         (csrc/kernels/chunk_ssd.hip)."""
         long, remaining = [], self.token_budget
@@ -258,7 +258,7 @@ class ModelRunner:
             [min(self.token_budget // n, self.max_model_len)] * n
             for n in dict.fromkeys(counts) if n > len(long)]
         small = min(self.token_budget, 1023)
-        for rows in (3 if small >= 384 else 4, 10):
+        for rows in (3, 8):
             n = min(self.max_num_seqs, small // rows)
             if self.state_layout and n > max(len(long), *counts):
                 steps.append([min(small // n, self.max_model_len)] * n)

@@ -437,7 +437,7 @@ def test_memory_profile_covers_many_short_prompts():
 
 
 def test_memory_profile_covers_small_steps_of_short_prompts():
-    """Steps of fewer than 1024 rows go chunkwise from three rows of each prompt on (the delta rule from ten): profiled
+    """Steps of fewer than 1024 rows go chunkwise from three rows of each prompt on (the delta rule from eight): profiled
     where that is more prompts than the large steps have."""
     from types import SimpleNamespace
 
@@ -445,8 +445,8 @@ def test_memory_profile_covers_small_steps_of_short_prompts():
     steps = lambda budget, seqs, layout=((),): ModelRunner._profile_steps(SimpleNamespace(   # noqa: E731
         token_budget=budget, max_model_len=8192, max_num_seqs=seqs, state_layout=list(layout)))
     assert steps(2048, 1024) == [[2048], [12] * 170, [16] * 128, [25] * 81, [3] * 341]
-    assert steps(1024, 256) == [[1024], [12] * 85, [16] * 64, [25] * 40, [3] * 256, [10] * 102]
-    assert steps(1024, 60) == [[1024], [17] * 60, [25] * 40] and steps(200, 256)[-2:] == [[4] * 50, [10] * 20]
+    assert steps(1024, 256) == [[1024], [12] * 85, [16] * 64, [25] * 40, [3] * 256, [8] * 127]
+    assert steps(1024, 60) == [[1024], [17] * 60, [25] * 40] and steps(200, 256)[-2:] == [[3] * 66, [8] * 25]
     assert steps(2048, 1024, ()) == [[2048]]
     assert steps(4096, 1024)[-1] == [25] * 163       # (4096 / 12 = 341 prompts already)
 
