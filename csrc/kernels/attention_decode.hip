@@ -44,14 +44,13 @@ constexpr int DEC_MAX_Z = 1024;  // z-slices the reduce kernel merges (host-chec
 // K1w runs where the grid has at least this many (seq, kv-head) pairs; smaller batches
 // take the 4-wave kernel (B = 1: 9.3 vs 12.3 us at ctx 640; ops/__init__.py mirrors it)
 constexpr int DEC_WAVE_MIN_PAIRS = 64;
-// ... and from this many pairs up a z-slice holds at least DEC_LONG_MIN_CHUNKS chunks
-// (ops/__init__.py also aims such grids at ~4 waves per CU instead of 8): with the KV
+// ... and the more pairs, the more chunks a z-slice holds at least (decode_min_chunks; from this many pairs up
+// ops/__init__.py also aims at ~4 waves per CU instead of 8): with the KV
 // streamed from HBM (tools/attn_bench.py cycles copies past the Infinity Cache), fewer,
 // longer slices won at every many-pairs shape measured -- B = 256 nq 8 / nkv 1 ctx 640:
 // 23.2 us at 2 slices of 10 chunks vs 26.9 at 7 of 3; B = 128 nq 32 / nkv 8: 65.0 vs
 // 68.8 us at one slice; B = 32 ctx 2300: 61.9 vs 66.5 (profiles/attn_decode_r5.jsonl)
 constexpr int DEC_LONG_PAIRS = 256;
-constexpr int DEC_LONG_MIN_CHUNKS = 10;
 
 // K1w: 32-token chunks per z-slice (>= min_per, at least 2: the pipeline depth); slices
 // past the context are empty and the reduce stops at decode_used_slices.  min_per is a
@@ -60,6 +59,9 @@ constexpr int DEC_LONG_MIN_CHUNKS = 10;
 // 2-3 chunks, each paying the q prologue and a partial write for little streaming.
 __host__ __device__ __forceinline__ int decode_slice_chunks(int nchunk, int Z, int min_per) {
   const int per = (nchunk + Z - 1) / Z;
+  // where the least length makes two slices, the second one short, shorter ones are as fast or faster
+  if (min_per == 4 && nchunk <= 8) min_per = 2;
+  if (min_per == 16 && nchunk > 16 && nchunk <= 24) min_per = 10;
   return per < min_per ? min_per : per;
 }
 __host__ __device__ __forceinline__ int decode_used_slices(int nchunk, int Z, int min_per) {
@@ -1019,14 +1021,19 @@ bool decode_use_wave(int B, int nkv) {
   return decode_wave_enabled() && (int64_t)B * nkv >= decode_wave_min_pairs();
 }
 
-// K1w's minimum 32-token chunks per z-slice for a launch of B x nkv pairs: from
-// DEC_LONG_PAIRS pairs up the chip is filled by the pairs themselves, so a context of up to
-// DEC_LONG_MIN_CHUNKS chunks stays one slice (no partials, no merge); below it slices of 2
-// (KGC_DECODE_MIN_CHUNKS overrides for every launch).
-static int decode_min_chunks(int B, int nkv) {
+// K1w's minimum 32-token chunks per z-slice for a launch of B x nkv pairs: the pairs fill the chip the more the more there
+// are, and a slice costs its q, its partial rows and their merge, so a context of up to that many chunks stays one
+// (a row much longer than the others still has all Z).  With the KV from HBM, Z for 8192 tokens, us, with 2 chunks (10
+// from 256 pairs on) -> now: 64 pairs x 300, 1000, 2000 tokens 10.5 -> 9.9, 14.6 -> 13.1, 22.9 -> 19.7; 128 x 128, 512,
+// 1000 9.5 -> 8.9, 14.6 -> 14.0, 22.0 -> 19.4; 192 x 1000 29.3 -> 25.5; 256 x 512 19.4 -> 18.8; 512 x 512, 1000 32.8 -> 31.1,
+// 55.7 -> 52.4.  (As many slices of one length would cost two divisions, 0.3 us.)  fp8 chunks take twice the instructions, and are as they were: 64 x 512 11.6, 12.8
+// in fours.  (KGC_DECODE_MIN_CHUNKS overrides for every launch).
+static int decode_min_chunks(int B, int nkv, bool kv_fp8) {
   const char* e = getenv("KGC_DECODE_MIN_CHUNKS");
   if (e) return atoi(e) < 2 ? 2 : atoi(e);
-  return (int64_t)B * nkv >= DEC_LONG_PAIRS ? DEC_LONG_MIN_CHUNKS : 2;
+  const int64_t pairs = (int64_t)B * nkv;
+  if (kv_fp8) return pairs >= DEC_LONG_PAIRS ? 10 : 2;
+  return pairs >= 2 * DEC_LONG_PAIRS ? 32 : pairs >= DEC_LONG_PAIRS ? 16 : pairs >= DEC_LONG_PAIRS / 2 ? 8 : 4;
 }
 
 template <typename T, int D, bool KV8, bool FUSE>
@@ -1041,7 +1048,7 @@ static void decode_dispatch(void* out, const void* q, const void* kc, const void
   // have written exactly the rows that plan names -- a single-slice row directly (nused ==
   // 1), the others as partials (tests/test_kernels_gpu.py
   // ::test_paged_decode_single_slice_rows_many_pairs)
-  const int min_per = decode_min_chunks(B, nkv);
+  const int min_per = decode_min_chunks(B, nkv, KV8);
   if (wave) {
     paged_decode_wave_kernel<T, D, KV8, FUSE><<<dim3(B, nkv, Z), 64, 0, s>>>(
         (T*)out, (const T*)q, kc, vc, bt, bt_stride, ctx, ml, es, tmp, nq, nkv, bs_log2,

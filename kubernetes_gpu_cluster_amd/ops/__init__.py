@@ -225,20 +225,31 @@ def _decode_z_cap(ws, B: int, nq: int) -> int:
 def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int = 0) -> int:
     """z-slices of the decode grid: enough waves to fill 256 CUs, bounded by the
     context (K1w: two 32-token chunks per wave; 4-wave kernel: 64-token partitions) and by
-    the 1024 slices the reduce kernel merges.  Z == 1 (large batches) lets the kernel
-    write its output directly."""
+    the 1024 slices the reduce kernel merges.  Z == 1 (large batches, short contexts) lets the kernel
+    write its output directly: the merge is 1.7 us, a chunk more per wave 0.55 (fp8 1.0), so up to 4 chunks (10 where
+    DECODE_LONG_PAIRS pairs fill the CUs) stay whole -- with the KV from HBM 64, 128, 256 pairs x 128 tokens 9.0 -> 7.0,
+    9.3 -> 7.2, 9.8 -> 8.1 us (fp8 10.0 -> 9.6, 10.6 -> 10.0, 11.8 -> 10.3), 256, 512 x 300 14.4 -> 12.7, 21.2 -> 19.5.
+    Fewer pairs than K1w takes leave CUs idle: 16 slices of two chunks or more (8 from 17 pairs on) and one per four
+    chunks up to 32, 8 pairs x 200, 512, 1000, 4000 tokens 9.5 -> 8.5, 14.7 -> 9.3, 15.1 -> 9.6, 15.5 -> 11.8, 32 pairs
+    12.0 -> 9.6, 15.2 -> 10.1, 15.5 -> 11.1, 22.9 -> 20.2."""
     pairs = max(1, batch * num_kv_heads)
     if decode_uses_wave(batch, num_kv_heads):
         chunks = max(1, math.ceil(max_ctx / DECODE_CHUNK))
+        if not target_waves and chunks <= (10 if pairs >= DECODE_LONG_PAIRS else 4):
+            return 1
         # from DECODE_LONG_PAIRS pairs up: ~4 waves per CU of longer slices (the kernel
-        # also keeps those slices >= 10 chunks, attention_decode.hip DEC_LONG_MIN_CHUNKS)
+        # also keeps those slices >= 16 chunks, attention_decode.hip decode_min_chunks)
         tgt = target_waves or (DECODE_LONG_TARGET_WAVES if pairs >= DECODE_LONG_PAIRS
                                else DECODE_TARGET_WAVES)
         want = math.ceil(tgt / pairs)
         return max(1, min(want, math.ceil(chunks / 2), 1024))
     parts = max(1, math.ceil(max_ctx / DECODE_PARTITION))
     want = math.ceil((target_waves or 4096) / (pairs * 4))
-    return max(1, min(want, math.ceil(parts / 4), 1024))
+    z = max(1, min(want, math.ceil(parts / 4), 1024))
+    chunks = math.ceil(max_ctx / DECODE_CHUNK)
+    if target_waves or chunks < 6:
+        return z
+    return max(z, min(math.ceil(chunks / 2), 16 if pairs <= 16 else 8), min(math.ceil(chunks / 4), 32))
 
 
 def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,

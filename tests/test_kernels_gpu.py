@@ -230,6 +230,32 @@ def test_paged_decode_rope(gpu, monkeypatch, kern, dt, d, nq, nkv, qk_norm, S, f
         torch.testing.assert_close(out.cpu().float(), exp.float(), **tol)
 
 
+@pytest.mark.parametrize("B,nkv", [(64, 1), (72, 2), (64, 4), (64, 8), (5, 2), (3, 8)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_paged_decode_slices_of_ragged_contexts(gpu, monkeypatch, B, nkv, fp8):
+    """Contexts at the edges of a slice's least length (2, 4, 8, 16, 32 chunks of 32 by the number of pairs, others in fp8)
+    and of the chunks, empty ones, some in one slice and some in all, at the grid of a short context, of the longest
+    one and of 8192 tokens (which the tables do not have): as the reference."""
+    for v in ("KGC_DECODE_WAVE_MIN_PAIRS", "KGC_DECODE_MIN_CHUNKS"):
+        monkeypatch.delenv(v, raising=False)
+    torch.manual_seed(22)
+    nq, d, bs = 4 * nkv, 128, 32
+    edges = [32 * c + o for c in (1, 2, 4, 5, 8, 9, 10, 16, 17, 24, 32, 33) for o in (0, 1)] + [1, 31, 0, 1300]
+    ctx = torch.tensor([edges[(7 * i + 3) % len(edges)] for i in range(B)])
+    ctx[0] = 1300
+    kc, vc, bt = _fill_random_cache(B, [max(int(c), 1) for c in ctx], nkv, bs, d, torch.bfloat16, gpu)
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    q = torch.randn(B, nq, d, dtype=torch.bfloat16, device=gpu)
+    cl = ctx.to(torch.int32).to(gpu)
+    exp = ref.paged_attention_decode(q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(), cl.cpu(), d ** -0.5)
+    for z in sorted({ops.decode_grid_z(B, nkv, c) for c in (100, 1300, 8192)}):
+        out = torch.full_like(q, float("nan"))
+        out = ops.paged_attention_decode(q, kc, vc, bt, cl, d ** -0.5, grid_z=z, out=out)
+        torch.testing.assert_close(out.cpu().float(), exp.float(), **_tol(torch.bfloat16))
+        assert torch.all(out[ctx.to(gpu) == 0] == 0)
+
+
 def test_paged_decode_single_slice_rows_many_pairs(gpu, monkeypatch):
     """at >= DECODE_LONG_PAIRS (seq, kv-head) pairs K1w keeps contexts of up to
     10 chunks in ONE slice, written directly (nused == 1), while longer contexts in the same
