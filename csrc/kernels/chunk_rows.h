@@ -16,7 +16,7 @@ inline bool chunk_fits(long stride, long cols, long blocks) {
 // workgroups of the walk, of which a CU holds one, and P H of what goes before it.
 //     t0 + tu units (+ t1 from 192 units on) + rows max(r0, ru units)   against   max(c0 + s0 wgs, c1 + cw wgs) + cp P H
 // The constants are fitted to 3 to 12 rows of 1 to 512 sequences, rows the mean, which is less than the longest: what is
-// chosen by them was 0 to 60 % faster in 5 shapes of heads each, what is not up to 12 % slower than it could be.
+// chosen by them was 0 to 60 % faster in 5 shapes of heads each, what is not up to 15 % slower than it could be.
 // Measured, token by token -> chunkwise:
 //                     1 x 8, 12, 24          8 x 8, 16        32 x 4, 6, 12            128 x 4, 8
 //   GLA  8 x 256      12.4, 15.2, 26.6 -> 13.9   18.9, 25.7 -> 16.1   31.0, 34.7, 44.9 -> 30   89, 109 -> 69
