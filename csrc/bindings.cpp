@@ -573,7 +573,7 @@ void moe_dgemm(Tensor C, Tensor A, Tensor Wp, Tensor sorted_ids, Tensor block_ex
   }
   if (rows == 0) return;
   kgc::launch_moe_dgemm(dt_code(Wp), (int)mode, C.data_ptr(), A.data_ptr(), Wp.data_ptr(),
-                        (int)rows, (int)N, (int)K, A.stride(0), (int)S, ss, (int)bm, (int)bn,
+                        (int)rows, (int)N, (int)K, (int)Wp.size(0), A.stride(0), (int)S, ss, (int)bm, (int)bn,
                         sorted_ids.data_ptr<int>(), block_expert.data_ptr<int>(),
                         meta.data_ptr<int>(), (int)npairs, (int)topk, stream());
 }

@@ -150,7 +150,7 @@ __global__ __launch_bounds__(DG_THREADS + LDW * 64, 1) void dgemm_kernel(
   // (WN = 4: a 2 x 4 wave grid, the 96-row K14m blocks: 48 rows x 32 columns per wave)
   const int wm = (wave & 7) / WN, wn = wave % WN;
   int z, j, mb, nb;
-  if (xmap) {
+  if (MOE == 0 && xmap) {
     // XCD-paired row blocks (host: S | 8, (N / BN) % (8 / S) == 0): workgroups L and L + 8
     // -- one XCD under round-robin placement (speed only, never correctness) -- take the
     // row blocks of the SAME weight columns and K-slice, so the second read of each weight
@@ -163,8 +163,13 @@ __global__ __launch_bounds__(DG_THREADS + LDW * 64, 1) void dgemm_kernel(
   } else {
     z = blockIdx.x % S;
     j = blockIdx.x / S;
-    mb = j % MB;
-    nb = j / MB;
+    if (MOE != 0 && xmap) {                        // column tiles fastest (moe_dgemm_t)
+      mb = j / (N / BN);
+      nb = j - mb * (N / BN);
+    } else {
+      mb = j % MB;
+      nb = j / MB;
+    }
   }
   const int m0 = mb * BM;
   if constexpr (MOE != 0) {
@@ -636,9 +641,18 @@ int dg_cfg_epis(int cfg) {
 
 template <typename T, int BM, int BN, int MOE>
 void moe_dgemm_t(int epi, void* C, const void* A, const void* Wp, int max_rows, int N, int K,
-                 int64_t lda, int S, int64_t ss, const DgAux& aux, hipStream_t s) {
+                 int64_t lda, int S, int64_t ss, int E, const DgAux& aux, hipStream_t s) {
   // 1-D grid, row blocks fastest: a column tile's blocks (one expert each) are dispatched
-  // together, so each XCD's L2 holds the activation rows of the experts it is dealt.
+  // together, so each XCD's L2 holds the activation rows of the experts it is dealt -- or column tiles fastest
+  // (xmap), each block's over all XCDs:
+  //   few pairs (SPARSE), most blocks without rows: with 8 or 16 blocks to a column tile the ones that have rows were
+  //     all on one XCD each.  8 experts of 4096 x 14336, top 2, 1 and 2 rows 266 -> 128 us, 318 -> 238; 16 of 4096 x 6400
+  //     1, 4 rows 213 -> 81, 281 -> 200; few experts of 64-row blocks: 4 of 2048 x 8192 1, 32 rows 60 -> 58, 97 -> 80;
+  //   the down projection of small blocks that all have rows (its K slices already go over the XCDs, its blocks then
+  //     did not): 8 experts 8 to 64 rows 540 -> 485, 16 experts 32 to 256 rows 505 -> 440 (gate_up so: 2 % slower);
+  //   gate_up of 128-row blocks, a multiple of 8, in many column tiles: 8 experts 512, 1024 rows 851 -> 753, 1475 -> 1388
+  //     (28 tiles to a block: 224 -> 236; more blocks to an expert would each stream its weights).
+  // Between, as before: 8 experts 4 to 6 rows 364 -> 378, 128 to 384 rows 509 -> 525 and more; 64 experts 8 rows 115 -> 130.
   // BM = 96 (a decode step's ~64 +- 3 sd pairs per expert in ONE block, a third fewer
   // padding rows than 128): 2 x 4 MFMA waves and 4 loader waves (12 A pieces per step).
   // BN = 256 (2 x 4 waves of 64 columns): a block's gathered rows are re-read by half as
@@ -648,10 +662,13 @@ void moe_dgemm_t(int epi, void* C, const void* A, const void* Wp, int max_rows, 
   constexpr int LDW = (BM == 96 || (BN == 256 && BM == 128)) ? 4 : 0;
   const int MB = max_rows / BM;
   const dim3 grid((unsigned)(MB * (N / BN) * S));
+  const bool sparse = aux.npairs < (E < 16 ? E : 16) || (E <= 4 && BM == 64);
+  const int xmap = sparse || (MOE == 1 ? BM == 128 && MB % 8 == 0 && MB <= 3 * E && N / BN >= 48
+                                       : BM == 64 && aux.npairs >= 2 * E);
 #define MOE_LAUNCH(EP)                                                                      \
   dgemm_kernel<T, BM, BN, EP, true, ABL_NONE, LDW, WN, MOE>                                 \
       <<<grid, DG_THREADS + LDW * 64, 0, s>>>(C, (const T*)A, (const T*)Wp, max_rows, N, K, \
-                                              lda, S, MB, ss, 0, partial_wt(), aux)
+                                              lda, S, MB, ss, xmap, partial_wt(), aux)
   if constexpr (MOE == 1) {
     MOE_LAUNCH(EPI_SILU);
   } else {
@@ -664,7 +681,7 @@ void moe_dgemm_t(int epi, void* C, const void* A, const void* Wp, int max_rows, 
 }  // namespace
 
 void launch_moe_dgemm(int dtype, int mode, void* C, const void* A, const void* Wp, int max_rows,
-                      int N, int K, int64_t lda, int S, int64_t slice_stride, int bm, int bn,
+                      int N, int K, int E, int64_t lda, int S, int64_t slice_stride, int bm, int bn,
                       const int* sorted_ids, const int* block_expert, const int* meta,
                       int npairs, int topk, hipStream_t s) {
   DgAux aux{};
@@ -676,8 +693,8 @@ void launch_moe_dgemm(int dtype, int mode, void* C, const void* A, const void* W
   aux.wexp = (int64_t)N * K;                     // one expert's packed weight, elements
   const int epi = mode == 1 ? EPI_SILU : S > 1 ? EPI_PARTIAL : EPI_OUT;
 #define MOE_BN(TT, BMM, MODE)                                                               \
-  if (bn == 256) moe_dgemm_t<TT, BMM, 256, MODE>(epi, C, A, Wp, max_rows, N, K, lda, S, slice_stride, aux, s); \
-  else moe_dgemm_t<TT, BMM, 128, MODE>(epi, C, A, Wp, max_rows, N, K, lda, S, slice_stride, aux, s);
+  if (bn == 256) moe_dgemm_t<TT, BMM, 256, MODE>(epi, C, A, Wp, max_rows, N, K, lda, S, slice_stride, E, aux, s); \
+  else moe_dgemm_t<TT, BMM, 128, MODE>(epi, C, A, Wp, max_rows, N, K, lda, S, slice_stride, E, aux, s);
 #define MOE_BM(TT, MODE)                                                                    \
   if (bm == 64) { MOE_BN(TT, 64, MODE) }                                                    \
   else if (bm == 96) { MOE_BN(TT, 96, MODE) }                                               \

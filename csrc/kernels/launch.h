@@ -153,7 +153,7 @@ struct DgAux {
 // bm = 64 | 96 | 128 row blocks (moe_align's), bn = 128 | 256 column tiles, max_rows = rows
 // of sorted_ids.
 void launch_moe_dgemm(int dtype, int mode, void* C, const void* A, const void* Wp, int max_rows,
-                      int N, int K, int64_t lda, int S, int64_t slice_stride, int bm, int bn,
+                      int N, int K, int E, int64_t lda, int S, int64_t slice_stride, int bm, int bn,
                       const int* sorted_ids, const int* block_expert, const int* meta,
                       int npairs, int topk, hipStream_t s);
 int dgemm_num_cfgs();

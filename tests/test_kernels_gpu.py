@@ -864,6 +864,25 @@ def test_fused_moe_packed_k14m(gpu, monkeypatch, T, bm, S, bn):
     torch.testing.assert_close(out.cpu().float(), exp.float(), **_tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("E,topk,H,I", [(4, 1, 512, 512), (8, 2, 512, 512), (16, 2, 256, 512), (20, 8, 256, 256)])
+@pytest.mark.parametrize("T", [1, 2, 3, 7, 8, 17, 40, 90])
+def test_fused_moe_packed_column_order(gpu, E, topk, H, I, T):
+    """Both orders of the grid by the pairs and the experts (at the edges of the rule: fewer pairs than experts or than
+    16, twice as many), and blocks without rows, vs the fp32 reference."""
+    x, w13, w2, tw, tid = _moe_case(torch.bfloat16, T, E, topk, H, I, gpu, seed=T + E)
+    out = ops.fused_moe(x, w13, w2, tw, tid, w13p=ops.moe_pack(w13, True), w2p=ops.moe_pack(w2, False))
+    exp = ref.moe_mlp_local(x.cpu(), w13.cpu(), w2.cpu(), tw.cpu(), tid.cpu())
+    torch.testing.assert_close(out.cpu().float(), exp.float(), **_tol(torch.bfloat16))
+
+
+def test_fused_moe_packed_column_order_of_large_blocks(gpu):
+    """128-row blocks, 16 of them, in 48 column tiles: gate_up goes by column tiles, the down projection by blocks."""
+    x, w13, w2, tw, tid = _moe_case(torch.bfloat16, 512, 8, 2, 128, 6144, gpu, seed=3)
+    out = ops.fused_moe(x, w13, w2, tw, tid, w13p=ops.moe_pack(w13, True), w2p=ops.moe_pack(w2, False))
+    exp = ref.moe_mlp_local(x.cpu(), w13.cpu(), w2.cpu(), tw.cpu(), tid.cpu())
+    torch.testing.assert_close(out.cpu().float(), exp.float(), **_tol(torch.bfloat16))
+
+
 def test_fused_moe_packed_graph_capture(gpu):
     """K14m captures into a hipGraph (row counts stay on the device) and replays with new
     routes: the decode graphs' form of the Mixtral block."""
