@@ -35,12 +35,16 @@ inline bool chunk_pays(const ChunkCost& k, long P, long Tp, long H, long V, doub
   return k.t0 + k.tu * units + (units > 192 ? k.t1 : 0) + rows * slope > scale * ((a > b ? a : b) + k.cp * P * H);
 }
 
-// The same for the scans that prepare chunks in a workspace: by the rows alone from `alone` rows of one
-// sequence on, 24 in steps of 192, 16 in steps of 512 and 12 in steps of 1024, and by the costs in steps of fewer than
+// By the rows alone, P sequences of Tp rows together: from `alone` rows of one sequence on, 24 in steps of 192, 16 in steps
+// of 512 and 12 in steps of 1024.
+inline bool chunk_rows_pay(long P, long Tp, long alone) {
+  const long rows = Tp >= 1024 ? 12 : Tp >= 512 ? 16 : Tp >= 192 ? 24 : alone;
+  return P > 0 && Tp >= (rows < alone ? rows : alone) * P;
+}
+// The same for the scans that prepare chunks in a workspace: by the rows, and by the costs in steps of fewer than
 // 1024 rows (in larger ones short rows would start more chunks than the engine's memory profile has).
 inline bool chunk_rows_pay(const ChunkCost& k, long P, long Tp, long H, long V, long alone) {
-  const long rows = Tp >= 1024 ? 12 : Tp >= 512 ? 16 : Tp >= 192 ? 24 : alone;
-  return P > 0 && (Tp >= (rows < alone ? rows : alone) * P || (Tp < 1024 && chunk_pays(k, P, Tp, H, V)));
+  return chunk_rows_pay(P, Tp, alone) || (Tp < 1024 && chunk_pays(k, P, Tp, H, V));
 }
 
 // Tokens per segment, whole chunks of L and `least` of them at least, so that P sequences of Tp rows come to at most

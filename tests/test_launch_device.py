@@ -3,6 +3,8 @@ device (csrc/kernels/device.h), and which prompt rows go chunkwise (csrc/kernels
 import os
 import subprocess
 
+import pytest
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 RUNTIME = """
 #pragma once
@@ -85,6 +87,33 @@ def test_devices_are_asked_one_by_one(tmp_path):
 def test_short_rows_stay_token_by_token(tmp_path):
     """Hundreds of chunks of one to eight rows used to go chunkwise from 1024 rows on."""
     _run(tmp_path, RULE)
+
+
+@pytest.mark.parametrize("cost, H, V, alone", [("4.0, 0.0062, 0.0, 0.85, 0.0021, 20.6, 0.0, 16.5, 0.037, 0.0, 8", 16, 128, 48),
+                                               ("6.1, 0.0148, 2.0, 0.72, 0.0014, 13.6, 0.0247, 0.0, 0.0, 0.0147, 3", 8, 256, 32)],
+                         ids=["delta", "gla"])
+def test_costs_only_add_to_steps_below_1024_rows(tmp_path, cost, H, V, alone):
+    """The memory profile has the chunks of the rule by rows from 1024 rows on, and of `least` rows each below."""
+    _run(tmp_path, """
+#include "chunk_rows.h"
+using kgc::chunk_rows_pay;
+#define CHECK(x) if (!(x)) return __LINE__
+int main() {
+  constexpr kgc::ChunkCost cost{%s};
+  const long H = %d, V = %d, alone = %d;
+  CHECK(!chunk_rows_pay(cost, 0, 0, H, V, alone));
+  bool more = false;
+  for (long P = 1; P <= 1024; ++P)
+    for (long Tp = P; Tp <= 64 * P; ++Tp) {
+      const bool rows = chunk_rows_pay(P, Tp, alone), both = chunk_rows_pay(cost, P, Tp, H, V, alone);
+      CHECK(both || !rows);
+      CHECK(both == rows || (Tp < 1024 && Tp >= cost.least * P));
+      more = more || both != rows;
+    }
+  CHECK(more);
+  return 0;
+}
+""" % (cost, H, V, alone))
 
 
 def test_chunk_offsets_fit_their_types(tmp_path):
