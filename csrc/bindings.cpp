@@ -7,6 +7,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include "kernels/chunk_rows.h"
 #include "kernels/launch.h"
 
 namespace {
@@ -1891,6 +1892,12 @@ void gla_scan(Tensor out, Tensor proj, Tensor low, Tensor a2, Tensor a2_bias, Te
                        (int)V, (int)R, (float)tau, (int)S.size(0), stream());
 }
 
+// (sequences, rows) of the small steps with the largest workspaces of the delta rule and of GLA (chunk_rows.h)
+std::vector<int64_t> scan_most_chunks(int64_t H, int64_t V, int64_t seqs, int64_t rows, int64_t len) {
+  const kgc::ChunkStep a = kgc::delta_most_chunks(H, V, seqs, rows, len), b = kgc::gla_most_chunks(H, V, seqs, rows, len);
+  return {a.P, a.Tp, b.P, b.Tp};
+}
+
 void selective_scan(Tensor out, Tensor x, Tensor dt, Tensor bc, Tensor At, Tensor dt_bias,
                     Tensor dskip, Tensor z, Tensor S, std::optional<Tensor> qsl,
                     std::optional<Tensor> seq_lens, std::optional<Tensor> ctx_lens, Tensor slots,
@@ -2656,6 +2663,7 @@ TORCH_LIBRARY(kgc, m) {
   m.def("gla_scan(Tensor(a!) out, Tensor proj, Tensor low, Tensor a2, Tensor a2_bias, Tensor(b!) S, "
         "Tensor? qsl, Tensor? seq_lens, Tensor? ctx_lens, Tensor slots, int P, int D, int Tp, int H, "
         "int d, int V, float tau) -> ()");
+  m.def("scan_most_chunks(int H, int V, int seqs, int rows, int len) -> int[]", &scan_most_chunks);
   m.def("selective_scan(Tensor(a!) out, Tensor x, Tensor dt, Tensor bc, Tensor At, Tensor dt_bias, "
         "Tensor dskip, Tensor z, Tensor(b!) S, Tensor? qsl, Tensor? seq_lens, Tensor? ctx_lens, "
         "Tensor slots, int P, int D, int Tp, float out_scale) -> ()");

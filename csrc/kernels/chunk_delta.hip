@@ -744,8 +744,7 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
 // through LDS.  (Products, systems and update each by itself, sums of two MFMAs added afterwards: 1000 vector instructions,
 // 293 us in all; W and P read by every wave from memory: 276.)
 bool delta_chunk_ok(const float* qkv, int P, int Tp, int H, int G, int d, int V) {
-  constexpr ChunkCost COST{4.0, 0.0062, 0.0, 0.85, 0.0021, 20.6, 0.0, 16.5, 0.037, 0.0, 8};
-  return chunk_rows_pay(COST, P, Tp, H, V, 48) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
+  return delta_rows_pay(P, Tp, H, V) && d == D && V >= 16 && ((int64_t)H * V) % 4 == 0 &&
          (reinterpret_cast<uintptr_t>(qkv) & 15) == 0 &&
          chunk_fits(2L * G * D + (long)H * V, (long)H * V, (long)H * ((V + 127) / 128 + 1));
 }

@@ -694,8 +694,7 @@ int plan(int P, int Tp, int H, int V, int* items) {
 }  // namespace
 
 bool gla_chunk_ok(int P, int Tp, int H, int d, int V, int R) {
-  constexpr ChunkCost COST{6.1, 0.0148, 2.0, 0.72, 0.0014, 13.6, 0.0247, 0.0, 0.0, 0.0147, 3};
-  return chunk_rows_pay(COST, P, Tp, H, V, 32) && d == D && V >= 16 && R <= RMAX &&
+  return gla_rows_pay(P, Tp, H, V) && d == D && V >= 16 && R <= RMAX &&
          chunk_fits(0, (long)H * V, (long)H * ((V + 127) / 128));   // (row offsets have 64 bits)
 }
 // floats of workspace

@@ -42,9 +42,42 @@ inline bool chunk_rows_pay(long P, long Tp, long alone) {
   return P > 0 && Tp >= (rows < alone ? rows : alone) * P;
 }
 // The same for the scans that prepare chunks in a workspace: by the rows, and by the costs in steps of fewer than
-// 1024 rows (in larger ones short rows would start more chunks than the engine's memory profile has).
+// 1024 rows (in larger ones short rows would start far more chunks than any other step, and the engine would set memory
+// aside for their workspace).
 inline bool chunk_rows_pay(const ChunkCost& k, long P, long Tp, long H, long V, long alone) {
   return chunk_rows_pay(P, Tp, alone) || (Tp < 1024 && chunk_pays(k, P, Tp, H, V));
+}
+
+// The delta rule's and GLA's, the costs as above.
+inline bool delta_rows_pay(long P, long Tp, long H, long V) {
+  constexpr ChunkCost COST{4.0, 0.0062, 0.0, 0.85, 0.0021, 20.6, 0.0, 16.5, 0.037, 0.0, 8};
+  return chunk_rows_pay(COST, P, Tp, H, V, 48);
+}
+inline bool gla_rows_pay(long P, long Tp, long H, long V) {
+  constexpr ChunkCost COST{6.1, 0.0148, 2.0, 0.72, 0.0014, 13.6, 0.0247, 0.0, 0.0, 0.0147, 3};
+  return chunk_rows_pay(COST, P, Tp, H, V, 32);
+}
+
+// Among steps of fewer than 1024 rows, at most `seqs` sequences of at most `len` rows and `rows` together, the one that
+// goes chunkwise by `pay`(P, Tp) and has the largest workspace, of Tp / 32 + P chunks (P = 0: none does).  The costs
+// say so neither at the fewest rows per sequence that they allow nor at the most sequences, so it is searched for.
+struct ChunkStep { long P, Tp; };
+template <typename F> inline ChunkStep most_chunks(F pay, long seqs, long rows, long len) {
+  ChunkStep best{0, 0};
+  if (rows > 1023) rows = 1023;
+  for (long P = 1; P <= seqs && P <= rows; ++P)
+    for (long Tp = rows < P * len ? rows : P * len; Tp >= P && Tp / 32 + P > best.Tp / 32 + best.P; --Tp)
+      if (pay(P, Tp)) {
+        best = {P, Tp};
+        break;
+      }
+  return best;
+}
+inline ChunkStep delta_most_chunks(long H, long V, long seqs, long rows, long len) {
+  return most_chunks([=](long P, long Tp) { return delta_rows_pay(P, Tp, H, V); }, seqs, rows, len);
+}
+inline ChunkStep gla_most_chunks(long H, long V, long seqs, long rows, long len) {
+  return most_chunks([=](long P, long Tp) { return gla_rows_pay(P, Tp, H, V); }, seqs, rows, len);
 }
 
 // Tokens per segment, whole chunks of L and `least` of them at least, so that P sequences of Tp rows come to at most

@@ -245,9 +245,9 @@ class ModelRunner:
         """Prompt steps with the largest activations: the token budget in prompts as long as
         they get, and for recurrent layers in as many as there are slots, too -- the chunkwise
         scans keep a workspace per started chunk of every sequence, from 12 rows of each on (in
-        steps of fewer than 1024 rows three, and the delta rule eight; csrc/kernels/chunk_rows.h), and the Mamba-2 scan images of the
-        chunks' keys, from 16 rows of each on with few groups and 25 with many
-        (csrc/kernels/chunk_ssd.hip)."""
+        steps of fewer than 1024 rows where their rule says so, for the model's own heads:
+        ``ops.scan_most_chunks``), and the Mamba-2 scan images of the chunks' keys, from 16 rows
+        of each on with few groups and 25 with many (csrc/kernels/chunk_ssd.hip)."""
         long, remaining = [], self.token_budget
         while remaining > 0:
             long.append(min(remaining, self.max_model_len))
@@ -262,6 +262,12 @@ class ModelRunner:
             n = min(self.max_num_seqs, small // rows)
             if self.state_layout and n > max(len(long), *counts):
                 steps.append([min(small // n, self.max_model_len)] * n)
+        covered = self.token_budget // 32 + counts[0] if self.token_budget >= 1024 else 0
+        for H, V in sorted({(s[0], s[2]) for shapes in self.state_layout for s in shapes
+                            if len(s) == 3 and s[1] == 128}):
+            steps += [s for s in ops.scan_most_chunks(H, V, self.max_num_seqs, self.token_budget,
+                                                      self.max_model_len)
+                      if sum(s) // 32 + len(s) > covered and s not in steps]
         return steps
 
     def release(self) -> None:

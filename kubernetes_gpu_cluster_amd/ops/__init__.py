@@ -1164,6 +1164,14 @@ def gla_scan(proj: torch.Tensor, low: torch.Tensor, a2: torch.Tensor, a2_bias: t
     return out
 
 
+def scan_most_chunks(H: int, V: int, seqs: int, rows: int, length: int) -> list:
+    """Per scan that prepares chunks in a workspace (delta rule, GLA; H heads of 128 x V), the prompt
+    lengths of the step with the largest one among steps of fewer than 1024 rows: at most
+    ``seqs`` prompts of at most ``length`` rows, ``rows`` together."""
+    r = _k().scan_most_chunks(H, V, seqs, rows, length)
+    return [[t // n + (i < t % n) for i in range(n)] for n, t in zip(r[::2], r[1::2]) if n]
+
+
 def selective_scan(x: torch.Tensor, dt: torch.Tensor, bc: torch.Tensor, At: torch.Tensor,
                    dt_bias: torch.Tensor, dskip: torch.Tensor, z: torch.Tensor,
                    state: torch.Tensor, meta, out_scale: float, out: torch.Tensor) -> torch.Tensor:

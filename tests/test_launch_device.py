@@ -89,31 +89,71 @@ def test_short_rows_stay_token_by_token(tmp_path):
     _run(tmp_path, RULE)
 
 
-@pytest.mark.parametrize("cost, H, V, alone", [("4.0, 0.0062, 0.0, 0.85, 0.0021, 20.6, 0.0, 16.5, 0.037, 0.0, 8", 16, 128, 48),
-                                               ("6.1, 0.0148, 2.0, 0.72, 0.0014, 13.6, 0.0247, 0.0, 0.0, 0.0147, 3", 8, 256, 32)],
-                         ids=["delta", "gla"])
-def test_costs_only_add_to_steps_below_1024_rows(tmp_path, cost, H, V, alone):
-    """The memory profile has the chunks of the rule by rows from 1024 rows on, and of `least` rows each below."""
+@pytest.mark.parametrize("op, H, V, alone, least", [("delta", 16, 128, 48, 8), ("gla", 8, 256, 32, 3)])
+def test_costs_only_add_to_steps_below_1024_rows(tmp_path, op, H, V, alone, least):
+    """The costs take no step back that the rows send chunkwise, and add none from 1024 rows on nor of fewer than `least`
+    rows per sequence."""
     _run(tmp_path, """
 #include "chunk_rows.h"
-using kgc::chunk_rows_pay;
+using kgc::chunk_rows_pay, kgc::%s_rows_pay;
 #define CHECK(x) if (!(x)) return __LINE__
 int main() {
-  constexpr kgc::ChunkCost cost{%s};
-  const long H = %d, V = %d, alone = %d;
-  CHECK(!chunk_rows_pay(cost, 0, 0, H, V, alone));
+  const long H = %d, V = %d, alone = %d, least = %d;
+  CHECK(!%s_rows_pay(0, 0, H, V));
   bool more = false;
   for (long P = 1; P <= 1024; ++P)
     for (long Tp = P; Tp <= 64 * P; ++Tp) {
-      const bool rows = chunk_rows_pay(P, Tp, alone), both = chunk_rows_pay(cost, P, Tp, H, V, alone);
+      const bool rows = chunk_rows_pay(P, Tp, alone), both = %s_rows_pay(P, Tp, H, V);
       CHECK(both || !rows);
-      CHECK(both == rows || (Tp < 1024 && Tp >= cost.least * P));
+      CHECK(both == rows || (Tp < 1024 && Tp >= least * P));
       more = more || both != rows;
     }
   CHECK(more);
   return 0;
 }
-""" % (cost, H, V, alone))
+""" % (op, H, V, alone, least, op, op))
+
+
+def test_memory_profile_has_the_chunks_of_every_small_step(tmp_path):
+    """No step of fewer than 1024 rows that goes chunkwise starts more chunks than the ones that the memory profile
+    runs and that go chunkwise, too, by the rules of the kernels, for any heads, budget and number of slots: the profile had
+    prompts of three and of eight rows, where the costs often say token by token."""
+    from types import SimpleNamespace
+
+    from kubernetes_gpu_cluster_amd.engine.model_runner import ModelRunner
+    cases = []
+    for H, V in ((2, 128), (4, 512), (8, 256), (16, 128), (16, 256), (32, 128), (32, 64), (64, 128)):
+        for budget in (100, 512, 1024, 2048, 16384):
+            for seqs, longest in ((16, 8192), (100, 8192), (512, 8192), (1024, 8192), (300, 60)):
+                steps = ModelRunner._profile_steps(SimpleNamespace(
+                    token_budget=budget, max_model_len=longest, max_num_seqs=seqs, state_layout=[((4, 64), (H, 128, V))]))
+                assert all(sum(s) <= budget and len(s) <= seqs and max(s) <= longest and min(s) > 0 for s in steps)
+                cases.append("{%d, %d, %d, %d, %d, {%s}}" % (H, V, budget, seqs, longest, ", ".join(
+                    "{%d, %d}" % (len(s), sum(s)) for s in steps)))
+    _run(tmp_path, """
+#include <cstdio>
+#include <vector>
+#include "chunk_rows.h"
+struct Case { long H, V, budget, seqs, longest; std::vector<kgc::ChunkStep> steps; };
+int main() {
+  const std::vector<Case> cases = {%s};
+  int missed = 0;
+  for (const Case& c : cases)
+    for (auto pay : {kgc::delta_rows_pay, kgc::gla_rows_pay}) {
+      long have = 0, most = 0;
+      for (auto s : c.steps)
+        if (pay(s.P, s.Tp, c.H, c.V) && s.Tp / 32 + s.P > have) have = s.Tp / 32 + s.P;
+      for (long P = 1; P <= c.seqs; ++P)
+        for (long Tp = P; Tp <= c.budget && Tp <= P * c.longest && Tp < 1024; ++Tp)
+          if (Tp / 32 + P > most && pay(P, Tp, c.H, c.V)) most = Tp / 32 + P;
+      if (have >= most) continue;
+      ++missed;
+      printf("%%s %%ld x %%ld, budget %%ld, %%ld slots: %%ld chunks profiled, %%ld possible\\n",
+             pay == kgc::gla_rows_pay ? "gla" : "delta", c.H, c.V, c.budget, c.seqs, have, most);
+    }
+  return missed ? 1 : 0;
+}
+""" % ", ".join(cases))
 
 
 def test_chunk_offsets_fit_their_types(tmp_path):
