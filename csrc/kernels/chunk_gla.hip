@@ -378,9 +378,16 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
   const bool own = MODE == 2 && seg_count > 1, zero = MODE == 1 || (pos0 == 0 && !own);
   const float* from = own ? mine : Ss;
 #pragma unroll
-  for (int i = 0; i < DT; ++i)
+  for (int i = 0; i < DT; ++i) S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // (one branch: as a choice per element they became 32, each of which waited for the load before it; 8 x 256, rows that go
+  // on from a state: 128 x 16 131 -> 88 us, 256 x 24 389 -> 200)
+  if (__builtin_amdgcn_readfirstlane(!zero)) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[i][r] = zero ? 0.f : from[(i * 16 + 4 * lg + r) * a.dv + colc];
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[i][r] = from[(i * 16 + 4 * lg + r) * a.dv + colc];
+    __builtin_amdgcn_sched_barrier(0);
+  }
   const T* vb = reinterpret_cast<const T*>(a.proj) + 2 * (int64_t)a.H * D + (int64_t)h * a.dv + colc;
   // Staging: a thread takes 8 columns of one row of q p, and 8 tokens of one column of k r, in both
   // cases the pieces 4 i .. and 16 + 4 i .. of 32: adjacent in the permuted order, one store.  A and p_L as they are
