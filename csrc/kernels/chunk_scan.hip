@@ -710,15 +710,16 @@ static ChunkWork chunk_plan(int P, int Tp, int wgs, int L, int least, int shorte
   return p;
 }
 
-// Chunkwise from 16 rows per sequence on or where the costs say so (chunk_mlstm.hip's kernel, which takes the larger steps
-// of bf16 rows, costs 0.7 of this file's), heads of 128 or 256 key channels in 16 bits (fp32 rows in
+// Chunkwise from 16 rows per sequence on or where the costs say so (of bf16 rows by a tenth: without, 4 rows were up to 12 %
+// slower, 4 of 256 x 512 16 x 4 27.4 -> 30.7; chunk_mlstm.hip's kernel, which takes their larger steps, costs 0.7 of
+// this file's), heads of 128 or 256 key channels in 16 bits (fp32 rows in
 // three parts do not fit LDS).  32 x 512 tokens, 4 heads of 256 x 512: 1957 us token by token, 222 us
 // chunkwise here and 128 to 136 in chunk_mlstm.hip, and nearer to float64 (3.5e-7 and 3.0e-7 against 5.0e-7).
 bool mlstm_chunk_ok(int dtype, int64_t stride, const void* qkvg, int P, int Tp, int H, int d, int dv) {
   constexpr ChunkCost COST[2] = {{10.0, 0.0085, 0.0, 0.92, 0.0022, 13.5, 0.014, 10.8, 0.04, 0.0, 2},
                                  {12.5, 0.0185, 0.0, 1.45, 0.0034, 20.0, 0.029, 10.8, 0.068, 0.0, 2}};
   if (!((dtype == DT_BF16 || dtype == DT_F16) && P > 0 && (d == 128 || d == 256) &&
-        (Tp >= 16 * P || chunk_pays(COST[d / 256], P, Tp, H, dv, dtype == DT_BF16 && dv > 128 && Tp >= 1024 ? 0.7 : 1.0)) &&
+        (Tp >= 16 * P || chunk_pays(COST[d / 256], P, Tp, H, dv, dtype != DT_BF16 ? 1.0 : dv > 128 && Tp >= 1024 ? 0.7 : 1.1)) &&
         stride % 8 == 0 && (reinterpret_cast<uintptr_t>(qkvg) & 15) == 0 && dv >= 16 &&
         chunk_fits(stride, (long)H * dv, (long)H * ((dv + 127) / 128))))
     return false;

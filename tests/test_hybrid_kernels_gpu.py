@@ -1247,7 +1247,7 @@ def test_delta_systems_keep_gates_that_are_not_finite_to_later_rows(gpu, gate, t
     assert not S[hit_S].isfinite().any() and torch.equal(S[~hit_S], S_w[~hit_S])
 
 
-@pytest.mark.parametrize("op,P,V,Tp", [("delta", 1, 32, 20), ("delta", 8, 512, 149), ("delta", 8, 32, 156), ("delta", 90, 32, 1080),
+@pytest.mark.parametrize("op,P,V,Tp", [("delta", 1, 32, 21), ("delta", 8, 512, 158), ("delta", 8, 32, 164), ("delta", 90, 32, 1080),
                                        ("gla", 1, 32, 11), ("gla", 8, 512, 83), ("gla", 100, 512, 300), ("gla", 90, 32, 1080)])
 def test_short_prompts_on_both_sides_of_the_chunkwise_rule(gpu, op, P, V, Tp):
     """The fewest rows that go chunkwise -- by the costs, and by the rows in steps of 1024 -- seen by their workspace, and
