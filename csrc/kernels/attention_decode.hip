@@ -32,6 +32,7 @@
 // with every wave building its own q in registers (4 dependent slice round trips
 // each): 149 vs 137 us for rope_kv + decode at B = 256, S = 4.
 #include "common.h"
+#include "decode_slices.h"
 #include "launch.h"
 #include <cstdlib>
 #include <type_traits>
@@ -44,31 +45,12 @@ constexpr int DEC_MAX_Z = 1024;  // z-slices the reduce kernel merges (host-chec
 // K1w runs where the grid has at least this many (seq, kv-head) pairs; smaller batches
 // take the 4-wave kernel (B = 1: 9.3 vs 12.3 us at ctx 640; ops/__init__.py mirrors it)
 constexpr int DEC_WAVE_MIN_PAIRS = 64;
-// ... and the more pairs, the more chunks a z-slice holds at least (decode_min_chunks; from this many pairs up
+// ... and the more pairs, the more chunks a z-slice holds at least (decode_slices.h; from DEC_LONG_PAIRS up
 // ops/__init__.py also aims at ~4 waves per CU instead of 8): with the KV
 // streamed from HBM (tools/attn_bench.py cycles copies past the Infinity Cache), fewer,
 // longer slices won at every many-pairs shape measured -- B = 256 nq 8 / nkv 1 ctx 640:
 // 23.2 us at 2 slices of 10 chunks vs 26.9 at 7 of 3; B = 128 nq 32 / nkv 8: 65.0 vs
 // 68.8 us at one slice; B = 32 ctx 2300: 61.9 vs 66.5 (profiles/attn_decode_r5.jsonl)
-constexpr int DEC_LONG_PAIRS = 256;
-
-// K1w: 32-token chunks per z-slice (>= min_per, at least 2: the pipeline depth); slices
-// past the context are empty and the reduce stops at decode_used_slices.  min_per is a
-// per-launch host choice (decode_min_chunks): the graph's Z is sized for max_model_len,
-// so at short contexts many-pairs grids would otherwise cut each context into slices of
-// 2-3 chunks, each paying the q prologue and a partial write for little streaming.
-__host__ __device__ __forceinline__ int decode_slice_chunks(int nchunk, int Z, int min_per) {
-  const int per = (nchunk + Z - 1) / Z;
-  // where the least length makes two slices, the second one short, shorter ones are as fast or faster
-  if (min_per == 4 && nchunk <= 8) min_per = 2;
-  if (min_per == 16 && nchunk > 16 && nchunk <= 24) min_per = 10;
-  return per < min_per ? min_per : per;
-}
-__host__ __device__ __forceinline__ int decode_used_slices(int nchunk, int Z, int min_per) {
-  const int per = decode_slice_chunks(nchunk, Z, min_per);
-  const int n = (nchunk + per - 1) / per;
-  return n < Z ? n : Z;
-}
 
 // max of x over lanes l and l ^ 16 / l ^ 32: the gfx950 permlane swaps hand each lane its
 // partner's value in the second register (VALU, no LDS round trip)
@@ -557,7 +539,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_wave_kernel(
     const void* __restrict__ vc_, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ ctx_lens, float* __restrict__ max_logits,
     float* __restrict__ exp_sums, float* __restrict__ tmp_out, int nq, int nkv, int bs_log2,
-    float scale_log2, float v_scale, int num_blocks, DecodeRope rp, int min_per) {
+    float scale_log2, float v_scale, int num_blocks, DecodeRope rp, DecodeLeast least) {
   typedef typename Vec8<T>::type V8;
   typedef std::conditional_t<KV8, uint8_t, T> C;
   const C* __restrict__ kc = reinterpret_cast<const C*>(kc_);
@@ -587,6 +569,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_wave_kernel(
   // non-empty slices come first and the reduce merges only those (a graph captured with
   // Z sized for max_model_len meets short contexts: most slices are then empty)
   const int nchunk = (ctx + 31) >> 5;
+  const int min_per = decode_min_chunks(least, nchunk);
   const int per = decode_slice_chunks(nchunk, Z, min_per);
   const int nused = decode_used_slices(nchunk, Z, min_per);
   const int c0 = min(nchunk, z * per);
@@ -852,7 +835,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_wave_kernel(
   l_run += __shfl_xor(l_run, 16, 64);
   l_run += __shfl_xor(l_run, 32, 64);
   const int64_t row = (int64_t)b * nq + h * G + r16;
-  // one slice covers the whole context (Z == 1, or min_per >= the context's chunks): the
+  // one slice covers the whole context (Z == 1, or its least length does): the
   // normalised output directly -- the reduce skips such a row
   if (Z == 1 || nused == 1) {
     if (z > 0) return;
@@ -893,7 +876,8 @@ template <typename T, int D, bool WAVE>
 __global__ __launch_bounds__(64) void paged_decode_reduce_kernel(
     T* __restrict__ out, const float* __restrict__ max_logits,
     const float* __restrict__ exp_sums, const float* __restrict__ tmp_out,
-    const int* __restrict__ ctx_lens, int nq, int Zg, int Zmax, int ctx_cap, int min_per) {
+    const int* __restrict__ ctx_lens, int nq, int Zg, int Zmax, int ctx_cap,
+    DecodeLeast least) {
   // The slice statistics are read in parallel (lane z), the weights staged in LDS,
   // and the partial rows loaded 8 slices at a time: the previous per-slice loop was a
   // chain of dependent L2 round trips (~7 us per call at B = 1; decode + reduce for
@@ -904,7 +888,8 @@ __global__ __launch_bounds__(64) void paged_decode_reduce_kernel(
   // as it clamps it (ctx_cap = bt_stride << bs_log2), so a ctx_len past the table never
   // makes this merge read slices that kernel did not write this step
   const int ctx = min(max(ctx_lens[b], 0), ctx_cap);
-  const int Z = WAVE ? decode_used_slices((ctx + 31) >> 5, Zg, min_per) : Zg;
+  const int nchunk = (ctx + 31) >> 5;
+  const int Z = WAVE ? decode_used_slices(nchunk, Zg, decode_min_chunks(least, nchunk)) : Zg;
   if (WAVE && Z == 1 && ctx > 0) return;     // the decode kernel wrote this row itself
   T* orow = out + ((int64_t)b * nq + hq) * D;
   constexpr int EPT = D / 64;
@@ -1021,19 +1006,10 @@ bool decode_use_wave(int B, int nkv) {
   return decode_wave_enabled() && (int64_t)B * nkv >= decode_wave_min_pairs();
 }
 
-// K1w's minimum 32-token chunks per z-slice for a launch of B x nkv pairs: the pairs fill the chip the more the more there
-// are, and a slice costs its q, its partial rows and their merge, so a context of up to that many chunks stays one
-// (a row much longer than the others still has all Z).  With the KV from HBM, Z for 8192 tokens, us, with 2 chunks (10
-// from 256 pairs on) -> now: 64 pairs x 300, 1000, 2000 tokens 10.5 -> 9.9, 14.6 -> 13.1, 22.9 -> 19.7; 128 x 128, 512,
-// 1000 9.5 -> 8.9, 14.6 -> 14.0, 22.0 -> 19.4; 192 x 1000 29.3 -> 25.5; 256 x 512 19.4 -> 18.8; 512 x 512, 1000 32.8 -> 31.1,
-// 55.7 -> 52.4.  (As many slices of one length would cost two divisions, 0.3 us.)  fp8 chunks take twice the instructions, and are as they were: 64 x 512 11.6, 12.8
-// in fours.  (KGC_DECODE_MIN_CHUNKS overrides for every launch).
-static int decode_min_chunks(int B, int nkv, bool kv_fp8) {
+// (KGC_DECODE_MIN_CHUNKS overrides the least length for every launch)
+static DecodeLeast decode_least_chunks(int B, int nkv, bool kv_fp8) {
   const char* e = getenv("KGC_DECODE_MIN_CHUNKS");
-  if (e) return atoi(e) < 2 ? 2 : atoi(e);
-  const int64_t pairs = (int64_t)B * nkv;
-  if (kv_fp8) return pairs >= DEC_LONG_PAIRS ? 10 : 2;
-  return pairs >= 2 * DEC_LONG_PAIRS ? 32 : pairs >= DEC_LONG_PAIRS ? 16 : pairs >= DEC_LONG_PAIRS / 2 ? 8 : 4;
+  return decode_least((int64_t)B * nkv, kv_fp8, e ? atoi(e) < 2 ? 2 : atoi(e) : 0);
 }
 
 template <typename T, int D, bool KV8, bool FUSE>
@@ -1043,16 +1019,16 @@ static void decode_dispatch(void* out, const void* q, const void* kc, const void
                             float scale_log2, float v_scale, int num_blocks,
                             const DecodeRope& rp, hipStream_t s) {
   const bool wave = decode_use_wave(B, nkv);
-  // ONE min_per value feeds both launches below: the decode kernel and its merge derive the
+  // ONE least length feeds both launches below: the decode kernel and its merge derive the
   // same slice plan from it (decode_used_slices), and the merge trusts the decode kernel to
   // have written exactly the rows that plan names -- a single-slice row directly (nused ==
   // 1), the others as partials (tests/test_kernels_gpu.py
   // ::test_paged_decode_single_slice_rows_many_pairs)
-  const int min_per = decode_min_chunks(B, nkv, KV8);
+  const DecodeLeast least = decode_least_chunks(B, nkv, KV8);
   if (wave) {
     paged_decode_wave_kernel<T, D, KV8, FUSE><<<dim3(B, nkv, Z), 64, 0, s>>>(
         (T*)out, (const T*)q, kc, vc, bt, bt_stride, ctx, ml, es, tmp, nq, nkv, bs_log2,
-        scale_log2, v_scale, num_blocks, rp, min_per);
+        scale_log2, v_scale, num_blocks, rp, least);
   } else {
     paged_decode_kernel<T, D, true, KV8, 4, 1, FUSE><<<dim3(B, nkv, Z), 256, 0, s>>>(
         (T*)out, (const T*)q, kc, vc, bt, bt_stride, ctx, ml, es, tmp, nq, nkv, bs_log2, Z,
@@ -1063,12 +1039,12 @@ static void decode_dispatch(void* out, const void* q, const void* kc, const void
     paged_decode_reduce_kernel<T, D, true><<<dim3(B, nq), 64, 0, s>>>((T*)out, ml, es, tmp, ctx,
                                                                       nq, Z, Z,
                                                                       bt_stride << bs_log2,
-                                                                      min_per);
+                                                                      least);
   else
     paged_decode_reduce_kernel<T, D, false><<<dim3(B, nq), 64, 0, s>>>((T*)out, ml, es, tmp,
                                                                        ctx, nq, Z, Z,
                                                                        bt_stride << bs_log2,
-                                                                       min_per);
+                                                                       least);
 }
 
 template <bool FUSE>

@@ -1,5 +1,6 @@
 """Host rules of the kernels' launchers, compiled against a fake runtime: what they ask of and set on a
-device (csrc/kernels/device.h), and which prompt rows go chunkwise (csrc/kernels/chunk_rows.h)."""
+device (csrc/kernels/device.h), which prompt rows go chunkwise (csrc/kernels/chunk_rows.h), and how decode contexts are cut
+into slices (csrc/kernels/decode_slices.h, ops.decode_grid_z)."""
 import os
 import subprocess
 
@@ -172,6 +173,37 @@ int main() {
     if (chunk_fits(x, 16, 1)) CHECK(63 * x + 256 <= INT32_MAX && x < (1 << 23));
     if (chunk_fits(16, x, 1)) CHECK(255 * x + x <= INT32_MAX && 63 * x <= INT32_MAX && (x + 15) / 16 <= 65535);
   }
+  return 0;
+}
+""")
+
+
+DECODE = """
+#define __host__
+#define __device__
+#define __forceinline__ inline
+#include "decode_slices.h"
+using namespace kgc;
+#define CHECK(x) if (!(x)) return __LINE__
+"""
+
+
+def test_decode_slices_cover_the_context_and_keep_a_fixed_length(tmp_path):
+    """Every chunk is in one of the slices that the merge reads, whatever the pairs, type and grid; a length set from
+    outside holds for every context (4 and 16 were taken for the rule's own and changed)."""
+    _run(tmp_path, DECODE + """
+int main() {
+  for (int fixed : {0, 1, 2, 3, 4, 8, 10, 16, 32})
+    for (int64_t pairs : {64, 127, 128, 255, 256, 511, 512, 4096})
+      for (bool fp8 : {false, true})
+        for (int n = 0; n <= 300; ++n) {
+          const int least = decode_min_chunks(decode_least(pairs, fp8, fixed), n);
+          CHECK(least >= 2 && (fixed == 0 || least == (fixed < 2 ? 2 : fixed)));
+          for (int Z : {1, 2, 3, 4, 7, 16, 32, 150}) {
+            const int per = decode_slice_chunks(n, Z, least), used = decode_used_slices(n, Z, least);
+            CHECK(per >= least && used <= Z && used * per >= n && (used == 0 ? n == 0 : (used - 1) * per < n));
+          }
+        }
   return 0;
 }
 """)
