@@ -182,6 +182,7 @@ DECODE = """
 #define __host__
 #define __device__
 #define __forceinline__ inline
+#include <initializer_list>
 #include "decode_slices.h"
 using namespace kgc;
 #define CHECK(x) if (!(x)) return __LINE__
