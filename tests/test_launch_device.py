@@ -208,3 +208,21 @@ int main() {
   return 0;
 }
 """)
+
+
+def test_decode_slices_of_a_row_much_longer_than_the_others(tmp_path):
+    """Such a row is over last, so its slices are no longer than the grid asks for or an eighth of the row, up to 8
+    chunks; from 256 pairs on 10 chunks, and from 512 on 16 where that is the whole row.  (One row of 500 tokens was two
+    slices with 192 pairs and one with 384, and the step 17 to 27 % slower than in slices of 2 and 10 chunks.)"""
+    _run(tmp_path, DECODE + """
+int main() {
+  for (int64_t pairs : {64, 127, 128, 192, 255, 256, 384, 511, 512, 768, 4096})
+    for (int n = 1; n <= 300; ++n)
+      for (int Z : {2, 3, 4, 9, 11, 16, 32, 150}) {
+        const int ask = (n + Z - 1) / Z, eighth = (n + 7) / 8;
+        const int most = pairs >= 512 && n <= 16 ? 16 : pairs >= 256 ? 10 : eighth < 2 ? 2 : eighth < 8 ? eighth : 8;
+        CHECK(decode_slice_chunks(n, Z, decode_min_chunks(decode_least(pairs, false, 0), n)) <= (ask > most ? ask : most));
+      }
+  return 0;
+}
+""")
