@@ -197,9 +197,9 @@ def decode_uses_wave(batch: int, num_kv_heads: int) -> bool:
 def decode_max_z(max_blocks: int, block_size: int) -> int:
     """The largest Z either kernel picks for this context capacity."""
     ctx = max_blocks * block_size
-    wave = math.ceil(math.ceil(ctx / DECODE_CHUNK) / 2)     # >= 2 chunks per K1w slice
+    wave = math.ceil(math.ceil(ctx / DECODE_CHUNK) / 2)     # >= 2 chunks per slice
     four = math.ceil(math.ceil(ctx / DECODE_PARTITION) / 4)
-    return max(1, min(1024, max(wave if decode_wave_kernel() else 1, four)))
+    return max(1, min(1024, max(wave if decode_wave_kernel() else min(wave, 32), four)))
 
 
 def decode_partials(batch: int, num_heads: int, head_dim: int, max_blocks: int,
@@ -238,7 +238,7 @@ def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int
         if not target_waves and chunks <= (10 if pairs >= DECODE_LONG_PAIRS else 4):
             return 1
         # from DECODE_LONG_PAIRS pairs up: ~4 waves per CU of longer slices (the kernel
-        # also keeps those slices >= 16 chunks, attention_decode.hip decode_min_chunks)
+        # also keeps those slices longer, csrc/kernels/decode_slices.h)
         tgt = target_waves or (DECODE_LONG_TARGET_WAVES if pairs >= DECODE_LONG_PAIRS
                                else DECODE_TARGET_WAVES)
         want = math.ceil(tgt / pairs)
@@ -247,7 +247,7 @@ def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int
     want = math.ceil((target_waves or 4096) / (pairs * 4))
     z = max(1, min(want, math.ceil(parts / 4), 1024))
     chunks = math.ceil(max_ctx / DECODE_CHUNK)
-    if target_waves or chunks < 6:
+    if target_waves or chunks < 6 or pairs >= DECODE_WAVE_MIN_PAIRS:
         return z
     return max(z, min(math.ceil(chunks / 2), 16 if pairs <= 16 else 8), min(math.ceil(chunks / 4), 32))
 

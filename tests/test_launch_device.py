@@ -226,3 +226,24 @@ int main() {
   return 0;
 }
 """)
+
+
+@pytest.mark.parametrize("wave,lim", [("1", None), ("0", None), ("1", "512")])
+def test_decode_grids_fit_what_is_set_aside_for_them(monkeypatch, wave, lim):
+    """Many slices are for steps of few (row, kv head) pairs: larger ones on the 4-wave kernel (K1w off, or from more pairs
+    on) keep a slice per 256 tokens as long as that fills the CUs, and every grid fits the partial rows."""
+    from kubernetes_gpu_cluster_amd import ops
+    monkeypatch.setenv("KGC_DECODE_WAVE", wave)
+    monkeypatch.delenv("KGC_DECODE_WAVE_MIN_PAIRS", raising=False)
+    if lim:
+        monkeypatch.setenv("KGC_DECODE_WAVE_MIN_PAIRS", lim)
+    if wave == "0":
+        assert [ops.decode_grid_z(256, 8, c) for c in (640, 8192)] == [1, 1] and ops.decode_grid_z(8, 8, 640) == 3
+    for nkv in (1, 2, 8, 32):
+        for B in (1, 2, 3, 5, 7, 8, 20, 63, 64, 300, 1024):
+            for ctx in (32, 96, 160, 192, 544, 1000, 4000, 8192, 131072):
+                z, pairs = ops.decode_grid_z(B, nkv, ctx), B * nkv
+                assert 1 <= z <= ops.decode_max_z(-(-ctx // 32), 32)
+                assert B * z <= ops.decode_partials(B, 1, 64, -(-ctx // 32), 32, "cpu")[0].numel()
+                if not ops.decode_uses_wave(B, nkv):
+                    assert (z == 1 or pairs * 4 * z <= 2 * 4096) and (pairs < 64 or z <= -(-4096 // (4 * pairs)))
