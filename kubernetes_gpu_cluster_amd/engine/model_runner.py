@@ -859,7 +859,7 @@ class ModelRunner:
         torch.cuda.synchronize()
         self.graph_pool = torch.cuda.graph_pool_handle()
         for B, bound in [(B, b) for B in sorted(self.buckets, reverse=True) for b in (*self._short_bounds(B), 0)]:
-            z = ops.decode_grid_z(B, nkv, self.max_model_len)
+            z = ops.decode_grid_z(B, nkv, self.max_model_len, capacity=True)
             meta = self._meta(B, 0, 0, B, 0, bound or self.max_model_len, z=z)
 
             def step_body(B=B, meta=meta):

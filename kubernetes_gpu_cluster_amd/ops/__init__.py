@@ -222,7 +222,8 @@ def _decode_z_cap(ws, B: int, nq: int) -> int:
     return max(1, min(1024, ws[0].numel() // max(1, B * nq)))
 
 
-def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int = 0) -> int:
+def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int = 0,
+                  capacity: bool = False) -> int:
     """z-slices of the decode grid: enough waves to fill 256 CUs, bounded by the
     context (K1w: two 32-token chunks per wave; 4-wave kernel: 64-token partitions) and by
     the 1024 slices the reduce kernel merges.  Z == 1 (large batches, short contexts) lets the kernel
@@ -231,7 +232,10 @@ def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int
     9.3 -> 7.2, 9.8 -> 8.1 us (fp8 10.0 -> 9.6, 10.6 -> 10.0, 11.8 -> 10.3), 256, 512 x 300 14.4 -> 12.7, 21.2 -> 19.5.
     Fewer pairs than K1w takes leave CUs idle: 16 slices of two chunks or more (8 from 17 pairs on) and one per four
     chunks up to 32, 8 pairs x 200, 512, 1000, 4000 tokens 9.5 -> 8.5, 14.7 -> 9.3, 15.1 -> 9.6, 15.5 -> 11.8, 32 pairs
-    12.0 -> 9.6, 15.2 -> 10.1, 15.5 -> 11.1, 22.9 -> 20.2."""
+    12.0 -> 9.6, 15.2 -> 10.1, 15.5 -> 11.1, 22.9 -> 20.2.
+    ``capacity``: max_ctx is what the rows may come to (a captured graph).  Empty slices cost too, so that the 4-wave
+    kernel has no more there than are as fast for short rows: 56 pairs, 32 slices instead of the 19 of 8192 tokens, 40, 500
+    tokens 11.9 -> 13.5, 15.0 -> 17.5; 8 instead of 3 of 544 8.8 -> 9.5, 15.5 -> 12.5 (4: 8.8, 11.7)."""
     pairs = max(1, batch * num_kv_heads)
     if decode_uses_wave(batch, num_kv_heads):
         chunks = max(1, math.ceil(max_ctx / DECODE_CHUNK))
@@ -249,6 +253,8 @@ def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int
     chunks = math.ceil(max_ctx / DECODE_CHUNK)
     if target_waves or chunks < 6 or pairs >= DECODE_WAVE_MIN_PAIRS:
         return z
+    if capacity:
+        return max(z, min(math.ceil(chunks / 2), 16 if pairs <= 16 else 8 if pairs <= 32 else 4))
     return max(z, min(math.ceil(chunks / 2), 16 if pairs <= 16 else 8), min(math.ceil(chunks / 4), 32))
 
 

@@ -247,3 +247,17 @@ def test_decode_grids_fit_what_is_set_aside_for_them(monkeypatch, wave, lim):
                 assert B * z <= ops.decode_partials(B, 1, 64, -(-ctx // 32), 32, "cpu")[0].numel()
                 if not ops.decode_uses_wave(B, nkv):
                     assert (z == 1 or pairs * 4 * z <= 2 * 4096) and (pairs < 64 or z <= -(-4096 // (4 * pairs)))
+
+
+def test_decode_graphs_have_few_empty_slices():
+    """A graph's grid is for any context up to its capacity, and an empty slice costs what a short row does not get back:
+    no more slices than one per 256 tokens of capacity, or 16, 8, 4 by the number of pairs; a step that knows its
+    longest row has as many as help that row."""
+    from kubernetes_gpu_cluster_amd import ops
+    for pairs in range(1, 64):
+        few = 16 if pairs <= 16 else 8 if pairs <= 32 else 4
+        for ctx in (32, 160, 192, 300, 544, 1000, 2048, 4096, 8192, 131072):
+            z, own = ops.decode_grid_z(pairs, 1, ctx, capacity=True), ops.decode_grid_z(pairs, 1, ctx)
+            assert z <= max(few, min(-(-1024 // pairs), -(-ctx // 256))) and z <= own
+    assert [ops.decode_grid_z(7, 8, c, capacity=True) for c in (544, 2048, 8192)] == [4, 8, 19]
+    assert [ops.decode_grid_z(4, 8, c, capacity=True) for c in (544, 2048, 8192)] == [8, 8, 32]
