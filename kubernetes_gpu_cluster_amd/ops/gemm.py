@@ -772,6 +772,17 @@ def _dg_candidates(M: int, N: int, K: int, kind: str, packed: bool):
     return out
 
 
+def _choose_dg(M: int, N: int, K: int, kind: str, plan: tuple[int, int]) -> None:
+    """K9m at this (M, N, K): the skinny kernels' own plans, which are asked first, are dropped."""
+    _plan_dg[(M, N, K, kind)] = plan
+    if kind == "plain":
+        _plan.pop((M, N, K), None)
+    elif kind == "silu":
+        _plan_silu.pop((M, N, K), None)
+    elif kind == "tail":
+        _plan_accnorm.pop((M, N, K), None)
+
+
 def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
                 kind: str, qkv_dims=None, sum_consumer=None) -> None:
     """hipBLASLt (at M <= SKINNY_MAX_M: what ``linear`` runs) vs the K9m candidates at each M in ``ms``, over all weights of the shape
@@ -790,7 +801,7 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
             fixed = _dg_table[key]
             if fixed is None or packed or not _dg_info(fixed[0])[2]:
                 if fixed is not None:
-                    _plan_dg[key] = fixed
+                    _choose_dg(*key, fixed)
                 res[key] = (fixed, float("nan"), float("nan"), fixed)
                 continue
         dev, dt = ws[0].device, ws[0].dtype
@@ -894,13 +905,7 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
         n = len(ws)
         chosen = best_cfg if best_t < lib_t * margin else None
         if chosen is not None:
-            _plan_dg[(M, N, K, kind)] = chosen
-            if kind == "plain":
-                _plan.pop((M, N, K), None)
-            elif kind == "silu":    # (the skinny kernels' own plans are asked first)
-                _plan_silu.pop((M, N, K), None)
-            elif kind == "tail":
-                _plan_accnorm.pop((M, N, K), None)
+            _choose_dg(M, N, K, kind, chosen)
         res[(M, N, K, kind)] = (chosen, lib_t * 1e3 / n, best_t * 1e3 / n, best_cfg)
         log.info("gemm M=%d N=%d K=%d %s: hipBLASLt %.1f us, K9m %s %.1f us -> %s", M, N, K,
                  kind, lib_t * 1e3 / n, best_cfg, best_t * 1e3 / n,
