@@ -1298,19 +1298,31 @@ def test_dgemm_plans_of_few_rows(gpu, M, plan):
         gemm._packed.clear()
 
 
-def test_tuned_plans_of_few_rows(gpu):
-    """From 17 rows on a chosen K9m plan takes the place of the skinny epilogues that would be asked first; below,
-    and for projections without a consumer of slices, nothing is tried."""
+def test_tuned_plans_of_few_rows(gpu, monkeypatch):
+    """From 17 rows on a chosen K9m plan takes the place of the skinny SiLU plan that would be asked first, and runs; below,
+    and for projections without a consumer of slices, nothing is tried.  (With so wide a margin K9m is always chosen.)"""
     from kubernetes_gpu_cluster_amd.ops import gemm
     torch.manual_seed(6)
+    monkeypatch.setenv("KGC_SKINNY_ACC_NORM", "0")
     ws = [torch.randn(1024, 4096, dtype=torch.bfloat16, device=gpu) * 0.02 for _ in range(3)]
+    ran, dgemm, tune = [], gemm.dgemm, gemm._tune_dgemm
+
+    def tune_dgemm(ws, N, K, ms, *a):
+        for m in ms if a[3] == "silu" else ():
+            gemm._plan_silu[m, N, K] = (2, 2, 4, False)      # whatever the timing said
+        tune(ws, N, K, ms, *a)
+    monkeypatch.setattr(gemm, "dgemm", lambda *a, **k: ran.append(a[2:4]) or dgemm(*a, **k))
+    monkeypatch.setattr(gemm, "_tune_dgemm", tune_dgemm)
     try:
-        for shapes in (dict(tail_shapes={(1024, 4096)}), dict(silu_shapes={(1024, 4096)})):
-            kind = "tail" if "tail_shapes" in shapes else "silu"
-            res = gemm.tune_skinny(ws, [8, 16, 32], **shapes)
-            assert {k for k in res if len(k) == 4} == {(32, 1024, 4096, kind)}
-            if (32, 1024, 4096, kind) in gemm._plan_dg:
-                assert (32, 1024, 4096) not in (gemm._plan_accnorm if kind == "tail" else gemm._plan_silu)
+        for shapes in (dict(tail_shapes={(1024, 4096)}), dict(silu_shapes={(1024, 4096)}), {}):
+            kind = next((k[:4] for k in shapes), "plain")
+            res = gemm.tune_skinny(ws, [8, 16, 32], margin=1e9, **shapes)
+            if kind == "plain":
+                assert not gemm.dgemm_plan() and all(len(k) == 3 for k in res)
+                continue
+            assert {k for k in res if len(k) == 4} == {(32, 1024, 4096, kind)} == set(gemm.dgemm_plan())
+            assert (32, 1024, 4096) not in gemm._plan_silu
+            del ran[:]
             x = torch.randn(32, 4096, dtype=torch.bfloat16, device=gpu)
             y = x.float() @ ws[0].float().t()
             if kind == "silu":
@@ -1320,6 +1332,7 @@ def test_tuned_plans_of_few_rows(gpu):
                 _, r = gemm.linear_add_rms(x, ws[0], torch.zeros(32, 1024, dtype=x.dtype, device=gpu),
                                            torch.ones(1024, dtype=x.dtype, device=gpu), 1e-6)
                 torch.testing.assert_close(r.float(), y, atol=2e-2, rtol=2e-2)
+            assert ran == [gemm.dgemm_plan()[32, 1024, 4096, kind]]
             gemm.clear_plan()
     finally:
         gemm.clear_plan()
