@@ -1255,7 +1255,7 @@ void residual_group_norm(Tensor out, Tensor x, std::optional<Tensor> y, Tensor w
                                   (float)eps, stream());
 }
 
-void depth_mix_norm(Tensor out, Tensor x, Tensor hist, Tensor y, Tensor coef, Tensor w,
+void depth_mix_sums(Tensor out, Tensor x, Tensor hist, Tensor y, Tensor coef, Tensor w,
                     int64_t layer, int64_t groups, double eps, std::optional<Tensor> sums, int64_t slot,
                     int64_t first, at::TensorList ahead) {
   check_f32(x, "x");
@@ -1297,6 +1297,11 @@ void depth_mix_norm(Tensor out, Tensor x, Tensor hist, Tensor y, Tensor coef, Te
                              hist.data_ptr<float>(), y.data_ptr(), coef.data_ptr<float>(),
                              w.data_ptr<float>(), (int)layer, hist.stride(0), (int)rows, (int)W,
                              (int)groups, (float)eps, m, stream());
+}
+
+void depth_mix_norm(Tensor out, Tensor x, Tensor hist, Tensor y, Tensor coef, Tensor w,
+                    int64_t layer, int64_t groups, double eps) {
+  depth_mix_sums(out, x, hist, y, coef, w, layer, groups, eps, std::nullopt, -1, 0, {});
 }
 
 void head_norm_gate(Tensor out, Tensor o, Tensor gt, Tensor w, int64_t H, double eps) {
@@ -2708,6 +2713,8 @@ TORCH_LIBRARY(kgc, m) {
         "Tensor? shared, Tensor? gate) -> ()");
   m.def("residual_group_norm(Tensor(a!) out, Tensor(b!) x, Tensor? y, Tensor w, int groups, float eps) -> ()");
   m.def("depth_mix_norm(Tensor(a!) out, Tensor(b!) x, Tensor(c!) hist, Tensor y, Tensor coef, Tensor w, "
+        "int layer, int groups, float eps) -> ()");
+  m.def("depth_mix_sums(Tensor(a!) out, Tensor(b!) x, Tensor(c!) hist, Tensor y, Tensor coef, Tensor w, "
         "int layer, int groups, float eps, Tensor(d!)? sums, int slot, int first, Tensor[] ahead) -> ()");
   m.def("head_norm_gate(Tensor(a!) out, Tensor o, Tensor g, Tensor w, int H, float eps) -> ()");
   m.def("xielu(Tensor(a!) out, Tensor z, Tensor ab) -> ()");
@@ -2850,6 +2857,7 @@ TORCH_LIBRARY_IMPL(kgc, CUDA, m) {
   m.impl("moe_route_softmax_all", &moe_route_softmax_all);
   m.impl("residual_group_norm", &residual_group_norm);
   m.impl("depth_mix_norm", &depth_mix_norm);
+  m.impl("depth_mix_sums", &depth_mix_sums);
   m.impl("head_norm_gate", &head_norm_gate);
   m.impl("xielu", &xielu);
   m.impl("gate_proj", &gate_proj);

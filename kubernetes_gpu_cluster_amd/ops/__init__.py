@@ -686,7 +686,7 @@ def depth_mix_norm(x: torch.Tensor, hist: torch.Tensor, layer: int, y: torch.Ten
         return ref.group_rms_norm(x, w, groups, eps, out_dtype)
     out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
     slot, first = take or (-1, 0)
-    _k().depth_mix_norm(out, x, hist, y, coef, w, layer, groups, eps, sums, slot, first, list(ahead))
+    _k().depth_mix_sums(out, x, hist, y, coef, w, layer, groups, eps, sums, slot, first, list(ahead))
     return out
 
 

@@ -86,6 +86,18 @@ def test_depth_mix_sums_begun_ahead(gpu, W, G, layers):
         xc = out[1][2 * i + 1].cpu().clone()
 
 
+def test_depth_mix_registered_op(gpu):
+    """The registered op without sums of following layers takes the arguments that it always took."""
+    torch.manual_seed(5)
+    W, T, dt = 256, 3, torch.bfloat16
+    start, hist, y = torch.randn(T, W).to(gpu), torch.randn(4, T, W).to(gpu), torch.randn(T, W).to(dt).to(gpu)
+    c, w, x, out = torch.randn(3).to(gpu), torch.rand(W).to(gpu), start.clone(), torch.empty(T, W, dtype=dt, device=gpu)
+    h, r = hist.clone(), start.clone()
+    torch.ops.kgc.depth_mix_norm(out, x, hist, y, c, w, 1, 1, 1e-5)
+    assert torch.equal(out, ops.depth_mix_norm(r, h, 1, y, c, w, 1, 1e-5, dt))
+    assert torch.equal(x, r) and torch.equal(hist, h) and not torch.equal(x, start)
+
+
 def test_depth_mix_refuses_sums_that_do_not_fit(gpu):
     W, T, dt = 256, 3, torch.bfloat16
     x, hist, w = torch.zeros(T, W, device=gpu), torch.zeros(4, T, W, device=gpu), torch.ones(W, device=gpu)
