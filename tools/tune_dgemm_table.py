@@ -2,7 +2,7 @@
 own start-up tuner (``tune_skinny`` -> ``_tune_dgemm``, every candidate timed with its
 consumer over every layer's copy of the weight) run with many more interleaved refinement
 rounds, on random weights of the model's decode-GEMM shapes, at the decode-graph buckets
-K9m serves (M = 65 .. max).  Writes profiles/tunableop/k9m_<model>_tp1_gfx950.json.
+K9m serves (M = 17 .. max).  Writes profiles/tunableop/k9m_<model>_tp1_gfx950.json.
 
     python tools/tune_dgemm_table.py --model llama-3-8b [--max-bs 256] [--rounds 15]
 """
@@ -42,7 +42,7 @@ def main():
              and (mcfg.tie_embeddings or "embed" not in n)]
     gemm.pack_decode_weights(plain, silu)
     ms = ([int(m) for m in a.ms.split(",")] if a.ms else
-          [m for m in graph_buckets(a.max_bs) if gemm.SKINNY_MAX_M < m <= gemm.DG_MAX_M])
+          [m for m in graph_buckets(a.max_bs) if gemm.DG_MIN_M <= m <= gemm.DG_MAX_M])
     t0 = time.time()
     res = gemm.tune_skinny(plain + silu, ms,
                            silu_shapes=model.silu_shapes(), tail_shapes=model.tail_shapes(),
