@@ -732,6 +732,7 @@ _DG_MAX_GRID = 264
 # this many interleaved rounds, the median decides
 _DG_REFINE = int(os.environ.get("KGC_DGEMM_REFINE", "3"))
 _DG_REFINE_ROUNDS = int(os.environ.get("KGC_DGEMM_REFINE_ROUNDS", "5"))
+_DG_RANK_BYTES = 512 << 20
 
 
 def _dg_candidates(M: int, N: int, K: int, kind: str, packed: bool):
@@ -846,9 +847,12 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
                     fused_add_rms_norm(y, res_t, gamma, 1e-6)
                 elif kind in ("qkv", "sum"):
                     consume(y)
-        # (a few rows' kernels are over before the next is launched eagerly: see _time_graphed)
-        first = _time_graphed if M <= SKINNY_MAX_M and kind in ("silu", "tail", "qkv") else _time
-        lib_t = first(lib, reps)
+        # A few rows' kernels are over before the next is launched eagerly (see _time_graphed).  They are ranked on as many
+        # weights as do not fit the Infinity Cache, and the library is timed in the rounds below only: the
+        # 16 choices of Llama-3-8B at 24 to 64 rows took 2.7 s of start-up on all 32 layers' weights.
+        few = M <= SKINNY_MAX_M and kind in ("silu", "tail", "qkv")
+        some = min(len(ws), -(-_DG_RANK_BYTES // (N * K * ws[0].element_size()))) if few else len(ws)
+        lib_t = float("nan") if few else _time(lib, reps)
         best_t, best_cfg = float("inf"), None
         timed = []                  # (t, (cfg, S), run) of every candidate
         for cfg, S in _dg_candidates(M, N, K, kind, packed):
@@ -859,8 +863,8 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
                                device=x.device))
             red = torch.empty(M, N // 2 if kind == "silu" else N, dtype=x.dtype, device=x.device)
 
-            def run(cfg=cfg, S=S, wl=wl, buf=buf, red=red, il=il):
-                for w in wl:
+            def run(cfg=cfg, S=S, wl=wl, buf=buf, red=red, il=il, n=len(ws)):
+                for w in wl[:n]:
                     if S == 1:
                         _k().dgemm(buf, x, w, cfg, 2 if kind == "silu" else 1)
                         if kind == "tail":
@@ -877,7 +881,7 @@ def _tune_dgemm(ws, N: int, K: int, ms, margin: float, reps: int, res: dict,
                             _k().splitk_add_rms_norm(red, buf, res_t, gamma, 1e-6)
                         else:
                             _k().splitk_reduce(red, buf)
-            t = first(run, reps)
+            t = _time_graphed(lambda: run(n=some), reps) if few else _time(run, reps)
             timed.append((t, (cfg, S), run))
         # refine: the few fastest candidates and the library re-timed in interleaved
         # rounds, median of each -- one short pass ranked near-ties by clock noise (the
