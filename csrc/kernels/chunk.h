@@ -154,11 +154,6 @@ __device__ __forceinline__ double lane63(double x) {
   return __builtin_bit_cast(double, hi << 32 | lo);
 }
 
-// The products over a chunk multiply a token's value by the masked zeros of the rows before it, which a
-// value that is not finite would reach.  v[i]: token tok(i) of the lane's column (one of the four lanes
-// that share lane & 15; PAIR: of the two that share lane & 31).  Such values become zero; returned is the column's first such token, from
-// which on its outputs and its state have to be made NaN (`none`: every value is finite).  A sum that
-// overflows only costs the closer look.
 // what is not finite if a value is not, or the values' sum
 template <int N, typename V> __device__ __forceinline__ float nonfinite_sum(const V (&v)[N]) {
   float z = 0.f;
@@ -175,6 +170,11 @@ template <int N, typename V> __device__ __forceinline__ float nonfinite_sum(cons
   }
   return z;
 }
+// The products over a chunk multiply a token's value by the masked zeros of the rows before it, which a
+// value that is not finite would reach.  v[i]: token tok(i) of the lane's column (one of the four lanes
+// that share lane & 15; PAIR: of the two that share lane & 31).  Such values become zero; returned is the column's first such token, from
+// which on its outputs and its state have to be made NaN (`none`: every value is finite).  A sum that
+// overflows only costs the closer look.
 template <bool PAIR = false, int N, typename V, typename F>
 __device__ __forceinline__ int take_nonfinite(V (&v)[N], int none, F tok) {
   const float z = nonfinite_sum(v);

@@ -53,7 +53,8 @@ struct DeltaArgs {
   bf16* wp;                                  // [chunks][H][W, P][3][L][L], columns permuted
   // per token of a chunk, zero past the sequence's end:
   float* gam;                                // [chunks][H][L]: gamma_t
-  f32x2* kw;                                 // [chunks][H][L]: e^(b_L - b_t) times rk, the rounding and what it leaves
+  f32x2* kw;                                 // [chunks][H][L]: e^(b_L - b_t) times rk, the rounding and what it leaves (48
+                                             // bits; weights below 2^-126 have fewer)
   float *rk, *rq;                            // [chunks][G][L]: what makes k and q unit (q: d^-1/2 too)
   int seg;                                   // tokens per segment (0: sequences are not cut)
   float* seg_state;                          // [items][H][D][dv + D]: dS | M of a segment
@@ -736,9 +737,10 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
 // Chunkwise for 128 key channels where the rows pay (chunk_rows.h; a chunk's workspace is 200 KB for 16
 // heads, which few rows per sequence would multiply, too).  16 x 1000 tokens of 16 heads with 128 x 128
 // states: 1328 us token by token, 245 us chunkwise, 55 of it W and P, whose bytes (k and q in, W and P out: 210 MB) take
-// 42; 2 x 8192: 7.5 ms and 0.68 ms.  Per wave and chunk the walk issues some 750 vector instructions and 168 MFMAs in 11000
-// cycles: 9000 of two waves' issue, 6100 of the LDS that 95 reads of 1 KB per wave keep busy, the rest the barriers and
-// the chain R -> U.  What the walk's issue was spent on before (281 us, on the same card): outputs stored in loops over the
+// 42; 2 x 8192: 7.5 ms and 0.68 ms.  Per wave and chunk the walk issues 580 vector instructions and 168 MFMAs in 11000
+// cycles: 7300 of two waves' issue (vector instructions in 52 % of the cycles, the matrix core in 47), 6100 of the LDS that 95
+// reads of 1 KB per wave keep busy, the rest the barriers and the chain R -> U.
+// What the walk's issue was spent on before (281 us, on the same card): outputs stored in loops over the
 // values of a descriptor that was not scalar; weights of k^T in double; 64-bit addresses of every staged element; vector work
 // behind the products instead of between them.  And the first launch's (72 us): columns of the inverse of 32 rows, dots
 // through LDS.  (Products, systems and update each by itself, sums of two MFMAs added afterwards: 1000 vector instructions,

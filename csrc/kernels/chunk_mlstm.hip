@@ -15,9 +15,10 @@
 //   P V, the update, the outputs; q of the next chunk arrives
 //   barrier (the outputs are still on their way)
 //
-// What bounds it: instruction issue, most of it the splitting of S, and at full load the clock that the power leaves.
-// Per wave and chunk 214 MFMAs of 32 cycles and 1600 vector instructions of 4, two waves per SIMD: 25500
-// cycles, 54 % of them the matrix core's, of 118 us at 1.87 GHz for 32 x 512 tokens, 4 heads of 256 x 512 (16 columns per
+// What bounds it: instruction issue, most of it the splitting of S, at the clock of full load (1.98 GHz where calls follow
+// each other, 2.4 for lighter kernels).  Per wave and chunk 214 MFMAs of 32 cycles and 1800 vector instructions of 4, two
+// waves per SIMD: the matrix core works in 49 % of the cycles, vector instructions are issued in 59 %; 126 to 132 us
+// for 32 x 512 tokens, 4 heads of 256 x 512 (16 columns per
 // wave: 222 us).  What it took: no spills (their reloads wait for every DMA before them; so lane numbers and places
 // are computed where they are used), the vector work and one memory instruction at a time between the MFMAs,
 // and barriers without the fence's wait for stores.

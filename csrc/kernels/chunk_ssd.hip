@@ -13,8 +13,8 @@
 //
 // What bounds it: instruction issue.  An MFMA takes 8 cycles of a SIMD's issue and 16 of its matrix core, a vector
 // instruction 4, so both fill only where a wave's own vector work (splitting S) stands between its MFMAs: the
-// regions below say in which order.  Per wave and chunk 226 MFMAs and 950 vector instructions, 81 % of the cycles at two
-// waves per SIMD (before the order was given: the same work in 1.5 times the time).  2 x 8192 tokens, 32 heads of
+// regions below say in which order.  Per wave and chunk 226 MFMAs and 950 vector instructions, in 44 and 58 % of the
+// cycles at two waves per SIMD (before the order was given: the same work in 1.5 times the time), 2.16 GHz in a loop of calls.  2 x 8192 tokens, 32 heads of
 // 128 x 64, us: 220 in all (chunk_scan.hip 357); kernel by kernel in a trace, whose clocks are not warm, images 23,
 // contributions 60, states 11, walk 145 (130 and 255 there).
 //

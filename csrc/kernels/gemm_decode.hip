@@ -1,4 +1,4 @@
-// K9m: mid-batch decode GEMM for gfx950 (M = 65..512 rows, the batch-256 decode step).
+// K9m: mid-batch decode GEMM for gfx950 (M = 17..512 rows, the batch-256 decode step).
 //
 //   C[M, N] = X[M, K] . W[N, K]^T      bf16 / f16 in, fp32 MFMA accumulation
 //
@@ -653,6 +653,8 @@ void moe_dgemm_t(int epi, void* C, const void* A, const void* Wp, int max_rows, 
   //   gate_up of 128-row blocks, a multiple of 8, in many column tiles: 8 experts 512, 1024 rows 851 -> 753, 1475 -> 1388
   //     (28 tiles to a block: 224 -> 236; more blocks to an expert would each stream its weights).
   // Between, as before: 8 experts 4 to 6 rows 364 -> 378, 128 to 384 rows 509 -> 525 and more; 64 experts 8 rows 115 -> 130.
+  // (gate_up of 128-row blocks that are no multiple of 8 is not pinned, and 4 to 8 % slower than by column tiles: 8 experts 520,
+  // 600, 760, 960 rows 817 -> 785, 1247 -> 1177, 1211 -> 1152, 1381 -> 1272.)
   // BM = 96 (a decode step's ~64 +- 3 sd pairs per expert in ONE block, a third fewer
   // padding rows than 128): 2 x 4 MFMA waves and 4 loader waves (12 A pieces per step).
   // BN = 256 (2 x 4 waves of 64 columns): a block's gathered rows are re-read by half as

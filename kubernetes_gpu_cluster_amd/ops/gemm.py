@@ -2,7 +2,7 @@
 GEMM (``csrc/kernels/gemm_skinny.hip``) for small-batch decode (M <= 64), or the K9m
 mid-batch decode GEMM (``csrc/kernels/gemm_decode.hip``: LDS-DMA ring, packed weight
 tiles, XCD-mapped split-K with the K-slice reduction fused into the consumer) for
-M = 65..512, where hipBLASLt leaves the long-K projections (the MLP down projection,
+M = 65..512 (from 17 rows on where a consumer takes its slices), where hipBLASLt leaves the long-K projections (the MLP down projection,
 K = 14336) at ~1.8 TB/s.
 
 Which one runs is a per-(M, N, K) decision made once at engine start by timing
