@@ -59,8 +59,8 @@ __global__ __launch_bounds__(NT) void residual_group_norm_kernel(
 }
 
 // hist [L + 1, Tcap, W]; layer result -> hist[layer + 1]; x = sum_j coef[j] hist[j], from sums m.from over
-// the results before m.first where an earlier layer began it; m.n later layers' sums are begun
-template <typename T>
+// the results before m.first where an earlier layer began it; A = m.n later layers' sums are begun
+template <typename T, int A>
 __global__ __launch_bounds__(NT) void depth_mix_norm_kernel(
     T* __restrict__ out, float* __restrict__ x, float* __restrict__ hist,
     const T* __restrict__ y, const float* __restrict__ coef, const float* __restrict__ w,
@@ -75,12 +75,16 @@ __global__ __launch_bounds__(NT) void depth_mix_norm_kernel(
   for (int c = threadIdx.x; c < W; c += NT) {
     const float r = xr[c] + to_f(yr[c]);
     hr[(int64_t)(layer + 1) * hist_stride + c] = r;
-    auto sum = [&](const float* cf, float acc, int j) {
-      for (; j <= layer; ++j) acc += cf[j] * hr[(int64_t)j * hist_stride + c];
-      return acc;
-    };
-    xr[c] = sum(coef, m.from != nullptr ? m.from[row * W + c] : 0.f, m.first) + own * r;
-    for (int a = 0; a < m.n; ++a) m.to[a][row * W + c] = sum(m.coef[a], 0.f, 0) + m.coef[a][layer + 1] * r;
+    float acc = A == 0 && m.from != nullptr ? m.from[row * W + c] : 0.f, ahead[A + 1] = {};
+    for (int j = A == 0 ? m.first : 0; j <= layer; ++j) {
+      const float h = hr[(int64_t)j * hist_stride + c];
+      acc += coef[j] * h;
+#pragma unroll
+      for (int a = 0; a < A; ++a) ahead[a] += m.coef[a][j] * h;
+    }
+    xr[c] = acc + own * r;
+#pragma unroll
+    for (int a = 0; a < A; ++a) m.to[a][row * W + c] = ahead[a] + m.coef[a][layer + 1] * r;
   }
   group_scales([&](int c) { return xr[c]; }, W, groups, eps, rs, scratch);
   const int gw = W / groups;
@@ -174,8 +178,9 @@ __global__ __launch_bounds__(NT) void residual_group_norm_vec_kernel(
 // The averages of A later layers are begun on the way (``m.to``), over the results that exist now: what is read
 // here is not read again by them.  A 12-layer stack so reads 26 rows of results and 7 of sums and writes 7
 // instead of reading 78, and every sum has the order it has without (14544 rows of 2048 through 12 layers: 2650
-// -> 1940 us).
-template <typename T, int V, int A>
+// -> 1940 us).  A sum that was begun (FROM) has an instance of its own: asked for in the loop that loads x and y, it made each of their
+// loads wait for the one before (16384 rows of 8192 through 2 layers, which begin none, 1167 -> 1282 us).
+template <typename T, int V, int A, bool FROM>
 __global__ __launch_bounds__(NT) void depth_mix_norm_vec_kernel(
     T* __restrict__ out, float* __restrict__ x, float* __restrict__ hist,
     const T* __restrict__ y, const float* __restrict__ coef, const float* __restrict__ w,
@@ -193,14 +198,14 @@ __global__ __launch_bounds__(NT) void depth_mix_norm_vec_kernel(
     r[k] = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
 #pragma unroll
     for (int i = 0; i <= A; ++i) acc[i][k] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (A == 0 && m.from != nullptr) acc[0][k] = ld4(m.from + row * W + c);
+    if (FROM) acc[0][k] = ld4(m.from + row * W + c);
   }
   auto add = [&](float4& s, float cj, const float4& h) {
     s = make_float4(s.x + cj * h.x, s.y + cj * h.y, s.z + cj * h.z, s.w + cj * h.w);
   };
   constexpr int U = V * A > 12 ? 2 : 4;   // rows of 8192 with sums ahead: a second wave per SIMD
 #pragma unroll U
-  for (int j = m.first; j <= layer; ++j) {
+  for (int j = FROM ? m.first : 0; j <= layer; ++j) {
 #pragma unroll
     for (int k = 0; k < V; ++k) {
       const int c = min(4 * (int)(threadIdx.x + NT * k), W - 4);
@@ -509,23 +514,30 @@ void launch_depth_mix_norm(int dtype, void* out, float* x, float* hist, const vo
              al16(hist) && al16(m.from);
   for (int i = 0; i < m.n; ++i) vec = vec && al16(m.to[i]);
   if (vec) {
-#define KGC_DMN_A(V, A)                                                                     \
-  KGC_DISPATCH_T(dtype, depth_mix_norm_vec_kernel<T, V, A><<<rows, NT, 0, s>>>(             \
+#define KGC_DMN_A(V, A, FROM)                                                               \
+  KGC_DISPATCH_T(dtype, depth_mix_norm_vec_kernel<T, V, A, FROM><<<rows, NT, 0, s>>>(       \
       (T*)out, x, hist, (const T*)y, coef, w, layer, hist_stride, W, gw, eps, m))
 #define KGC_DMN(V)                                                                          \
   do {                                                                                      \
-    if (m.n == 0) KGC_DMN_A(V, 0);                                                          \
-    else if (m.n == 1) KGC_DMN_A(V, 1);                                                     \
-    else if (m.n == 2) KGC_DMN_A(V, 2);                                                     \
-    else KGC_DMN_A(V, 3);                                                                   \
+    if (m.n == 1) KGC_DMN_A(V, 1, false);                                                   \
+    else if (m.n == 2) KGC_DMN_A(V, 2, false);                                              \
+    else if (m.n == 3) KGC_DMN_A(V, 3, false);                                              \
+    else if (m.from != nullptr) KGC_DMN_A(V, 0, true);                                      \
+    else KGC_DMN_A(V, 0, false);                                                            \
   } while (0)
     KGC_ROW_V(W, KGC_DMN);
 #undef KGC_DMN
 #undef KGC_DMN_A
     return;
   }
-  KGC_DISPATCH_T(dtype, depth_mix_norm_kernel<T><<<rows, NT, 0, s>>>(
-      (T*)out, x, hist, (const T*)y, coef, w, layer, hist_stride, W, groups, eps, m));
+#define KGC_DMN(A)                                                                          \
+  KGC_DISPATCH_T(dtype, depth_mix_norm_kernel<T, A><<<rows, NT, 0, s>>>(                    \
+      (T*)out, x, hist, (const T*)y, coef, w, layer, hist_stride, W, groups, eps, m))
+  if (m.n == 0) KGC_DMN(0);
+  else if (m.n == 1) KGC_DMN(1);
+  else if (m.n == 2) KGC_DMN(2);
+  else KGC_DMN(3);
+#undef KGC_DMN
 }
 
 void launch_head_norm_gate(int dtype, void* out, const float* o, const void* g, int64_t g_stride,
