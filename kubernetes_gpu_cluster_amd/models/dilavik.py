@@ -162,6 +162,7 @@ class DilavikForCausalLM(nn.Module):
         if self.hist is None or self.hist.shape[1] < T:
             self.prepare(cfg.max_position, max(T, 1), input_ids.device)
         G, eps, dt = cfg.norm_groups, cfg.rms_eps, self.dtype
+        sums = ops.depth_sums_pay(T, cfg.hidden_size)
         x = self.stream[:T]
         torch.mul(self.embed_tokens(input_ids), cfg.embed_scale, out=x)
         self.hist[0, :T].copy_(x)
@@ -172,7 +173,7 @@ class DilavikForCausalLM(nn.Module):
                 h = ops.group_rms_norm(x, layer.norm2, G, eps, dt, add=y)
                 y = layer.mlp(h)
             nxt = self.layers[i + 1].norm1 if i + 1 < len(self.layers) else self.final_norm
-            take, n = self.mix_plan[i]
+            take, n = self.mix_plan[i] if sums else (None, 0)
             h = ops.depth_mix_norm(x, self.hist, i, y, layer.dwa, nxt, G, eps, dt, self.sums, take,
                                    [l.dwa for l in self.layers[i + 1: i + 1 + n]])
             if taps is not None:

@@ -331,6 +331,36 @@ def test_layer_taps(models, device, dtype):
         assert np.abs(g - w).max() <= tol * np.abs(w).max()
 
 
+@pytest.mark.parametrize("device,dtype", DEVICES)
+def test_layers_with_and_without_sums_begun_ahead(models, monkeypatch, device, dtype):
+    """Few rows read all results in every layer, more follow the plan of begun sums: the same stream."""
+    from kubernetes_gpu_cluster_amd import ops
+    d, cfg, wts = models["mixed"]
+    eng = engine(models, "mixed", device, dtype)
+    model, mix = eng.executor.runner.model, ops.depth_mix_norm
+    toks, orig, runs, ahead = tokens_for(cfg, 19, 5), model.forward, [], []
+    monkeypatch.setattr(ops, "depth_mix_norm", lambda *a: ahead.append(bool(a[11])) or mix(*a))
+    model.forward = lambda *a, **k: orig(*a, taps=runs[-1], **k)
+    try:
+        for pay in (True, False):
+            monkeypatch.setattr(ops, "depth_sums_pay", lambda rows, W: pay)
+            runs.append([])
+            del ahead[:]
+            run_alone(TraceReplayer(eng), "t%d" % pay, toks, [len(toks)])
+            assert any(ahead) == pay and len(runs[-1]) == len(model.layers)
+    finally:
+        model.forward = orig
+    for a, b in zip(*runs):
+        torch.testing.assert_close(a, b, rtol=0 if device == "cuda" else 1e-5, atol=0 if device == "cuda" else 1e-5)
+
+
+def test_rows_that_begin_sums():
+    """Few rows of 1025 to 2048 columns do not (2048 columns, 24 layers, one row: 149 -> 167 us with them)."""
+    from kubernetes_gpu_cluster_amd import ops
+    assert [ops.depth_sums_pay(t, 2048) for t in (1, 64, 95, 96, 16384)] == [False, False, False, True, True]
+    assert [ops.depth_sums_pay(1, W) for W in (64, 1024, 1025, 2050, 4096)] == [True, True, False, True, True]
+
+
 # ---------------------------------------------------------------- generation entry points
 @pytest.mark.parametrize("device,dtype", DEVICES)
 def test_greedy_generation_through_scheduler(models, device, dtype):
