@@ -36,6 +36,7 @@
 // deploys, /root/reference/values-01-minimal-example2.yaml:6-7).
 #include "common.h"
 #include "launch.h"
+#include "moe_order.h"
 #include <cstdlib>
 
 namespace kgc {
@@ -642,19 +643,7 @@ int dg_cfg_epis(int cfg) {
 template <typename T, int BM, int BN, int MOE>
 void moe_dgemm_t(int epi, void* C, const void* A, const void* Wp, int max_rows, int N, int K,
                  int64_t lda, int S, int64_t ss, int E, const DgAux& aux, hipStream_t s) {
-  // 1-D grid, row blocks fastest: a column tile's blocks (one expert each) are dispatched
-  // together, so each XCD's L2 holds the activation rows of the experts it is dealt -- or column tiles fastest
-  // (xmap), each block's over all XCDs:
-  //   few pairs (SPARSE), most blocks without rows: with 8 or 16 blocks to a column tile the ones that have rows were
-  //     all on one XCD each.  8 experts of 4096 x 14336, top 2, 1 and 2 rows 266 -> 128 us, 318 -> 238; 16 of 4096 x 6400
-  //     1, 4 rows 213 -> 81, 281 -> 200; few experts of 64-row blocks: 4 of 2048 x 8192 1, 32 rows 60 -> 58, 97 -> 80;
-  //   the down projection of small blocks that all have rows (its K slices already go over the XCDs, its blocks then
-  //     did not): 8 experts 8 to 64 rows 540 -> 485, 16 experts 32 to 256 rows 505 -> 440 (gate_up so: 2 % slower);
-  //   gate_up of 128-row blocks, a multiple of 8, in many column tiles: 8 experts 512, 1024 rows 851 -> 753, 1475 -> 1388
-  //     (28 tiles to a block: 224 -> 236; more blocks to an expert would each stream its weights).
-  // Between, as before: 8 experts 4 to 6 rows 364 -> 378, 128 to 384 rows 509 -> 525 and more; 64 experts 8 rows 115 -> 130.
-  // (gate_up of 128-row blocks that are no multiple of 8 is not pinned, and 4 to 8 % slower than by column tiles: 8 experts 520,
-  // 600, 760, 960 rows 817 -> 785, 1247 -> 1177, 1211 -> 1152, 1381 -> 1272.)
+  // 1-D grid, row blocks fastest, or column tiles (xmap; moe_order.h).
   // BM = 96 (a decode step's ~64 +- 3 sd pairs per expert in ONE block, a third fewer
   // padding rows than 128): 2 x 4 MFMA waves and 4 loader waves (12 A pieces per step).
   // BN = 256 (2 x 4 waves of 64 columns): a block's gathered rows are re-read by half as
@@ -664,9 +653,7 @@ void moe_dgemm_t(int epi, void* C, const void* A, const void* Wp, int max_rows, 
   constexpr int LDW = (BM == 96 || (BN == 256 && BM == 128)) ? 4 : 0;
   const int MB = max_rows / BM;
   const dim3 grid((unsigned)(MB * (N / BN) * S));
-  const bool sparse = aux.npairs < (E < 16 ? E : 16) || (E <= 4 && BM == 64);
-  const int xmap = sparse || (MOE == 1 ? BM == 128 && MB % 8 == 0 && MB <= 3 * E && N / BN >= 48
-                                       : BM == 64 && aux.npairs >= 2 * E);
+  const int xmap = moe_columns_first(MOE == 1, E, BM, MB, N / BN, aux.npairs);
 #define MOE_LAUNCH(EP)                                                                      \
   dgemm_kernel<T, BM, BN, EP, true, ABL_NONE, LDW, WN, MOE>                                 \
       <<<grid, DG_THREADS + LDW * 64, 0, s>>>(C, (const T*)A, (const T*)Wp, max_rows, N, K, \
