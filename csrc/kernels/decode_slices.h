@@ -13,9 +13,10 @@ constexpr int DEC_LONG_PAIRS = 256;
 // max_model_len, so at short contexts many-pairs grids would otherwise cut each context into slices of 2-3 chunks, each paying
 // the q prologue and a partial write for little streaming.
 struct DecodeLeast {
-  int whole, lo, hi;                         // contexts of up to `whole` chunks (-1: none) are one slice; an eighth, from lo to hi
+  int whole, lo, hi;                         // contexts of up to `whole` chunks (-1: none) are one slice; from 24 chunks on an eighth, lo to hi
 };
-// Below 256 pairs a context has at most eight slices, up to slices of 8 chunks (2 chunks in any case -> now, KV from HBM, Z
+// Below 256 pairs a context of 24 chunks and more has at most eight slices, up to slices of 8 chunks (shorter ones gain
+// nothing: in threes 24 rows x 640 tokens 19.6 -> 20.4; 2 chunks in any case -> now, KV from HBM, Z
 // for 8192 tokens, 8 kv heads, us: 8, 16, 24 rows x 1000 tokens 15.3 -> 14.2, 22.9 -> 21.7, 32.4 -> 27.4, a quarter of 24
 // rows 1000 long and the others 100 27.0 -> 21.4); from 512 on one of 512 tokens is whole (10 chunks -> now: 64, 96 rows
 // x 512 33.7 -> 31.8, 48.1 -> 44.4).  Longer slices are faster yet where the contexts are alike (8 chunks from 128 pairs on,
@@ -30,7 +31,7 @@ inline DecodeLeast decode_least(int64_t pairs, bool kv_fp8, int fixed) {
   return {pairs >= 2 * DEC_LONG_PAIRS ? 16 : -1, 10, 10};
 }
 __host__ __device__ __forceinline__ int decode_min_chunks(const DecodeLeast& l, int nchunk) {
-  const int e = (nchunk + 7) >> 3, p = e < l.lo ? l.lo : e < l.hi ? e : l.hi;
+  const int e = nchunk < 24 ? 0 : (nchunk + 7) >> 3, p = e < l.lo ? l.lo : e < l.hi ? e : l.hi;
   return nchunk <= l.whole ? l.whole : p;
 }
 // slices past the context are empty and the merge stops at decode_used_slices

@@ -228,6 +228,20 @@ int main() {
 """)
 
 
+def test_decode_slices_of_middling_contexts(tmp_path):
+    """Contexts of fewer than 24 chunks are cut as short as the grid asks for (in threes 24 rows x 640 tokens 19.6 -> 20.4
+    us)."""
+    _run(tmp_path, DECODE + """
+int main() {
+  for (int64_t pairs : {64, 128, 192, 255}) {
+    for (int n = 1; n < 24; ++n) CHECK(decode_min_chunks(decode_least(pairs, false, 0), n) == 2);
+    CHECK(decode_min_chunks(decode_least(pairs, false, 0), 24) == 3 && decode_min_chunks(decode_least(pairs, false, 0), 32) == 4);
+  }
+  return 0;
+}
+""")
+
+
 @pytest.mark.parametrize("wave,lim", [("1", None), ("0", None), ("1", "512")])
 def test_decode_grids_fit_what_is_set_aside_for_them(monkeypatch, wave, lim):
     """Many slices are for steps of few (row, kv head) pairs: larger ones on the 4-wave kernel (K1w off, or from more pairs
