@@ -232,7 +232,8 @@ def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int
     9.3 -> 7.2, 9.8 -> 8.1 us (fp8 10.0 -> 9.6, 10.6 -> 10.0, 11.8 -> 10.3), 256, 512 x 300 14.4 -> 12.7, 21.2 -> 19.5.
     Fewer pairs than K1w takes leave CUs idle: 16 slices of two chunks or more (8 from 17 pairs on) and one per four
     chunks up to 32, 8 pairs x 200, 512, 1000, 4000 tokens 9.5 -> 8.5, 14.7 -> 9.3, 15.1 -> 9.6, 15.5 -> 11.8, 32 pairs
-    12.0 -> 9.6, 15.2 -> 10.1, 15.5 -> 11.1, 22.9 -> 20.2.
+    12.0 -> 9.6, 15.2 -> 10.1, 15.5 -> 11.1, 22.9 -> 20.2.  From 33 pairs on up to 16, and none for contexts of up to 256 tokens:
+    with them 56 pairs x 200, 3000 tokens 8.7 -> 9.2, 21.4 -> 22.5, 48 x 4000 22.6 -> 23.8 (fp8 20.2 -> 21.9).
     ``capacity``: max_ctx is what the rows may come to (a captured graph).  Empty slices cost too, so that the 4-wave
     kernel has no more there than are as fast for short rows: 56 pairs, 32 slices instead of the 19 of 8192 tokens, 40, 500
     tokens 11.9 -> 13.5, 15.0 -> 17.5; 8 instead of 3 of 544 8.8 -> 9.5, 15.5 -> 12.5 (4: 8.8, 11.7)."""
@@ -251,11 +252,11 @@ def decode_grid_z(batch: int, num_kv_heads: int, max_ctx: int, target_waves: int
     want = math.ceil((target_waves or 4096) / (pairs * 4))
     z = max(1, min(want, math.ceil(parts / 4), 1024))
     chunks = math.ceil(max_ctx / DECODE_CHUNK)
-    if target_waves or chunks < 6 or pairs >= DECODE_WAVE_MIN_PAIRS:
+    if target_waves or chunks < (6 if pairs <= 32 else 9) or pairs >= DECODE_WAVE_MIN_PAIRS:
         return z
     if capacity:
         return max(z, min(math.ceil(chunks / 2), 16 if pairs <= 16 else 8 if pairs <= 32 else 4))
-    return max(z, min(math.ceil(chunks / 2), 16 if pairs <= 16 else 8), min(math.ceil(chunks / 4), 32))
+    return max(z, min(math.ceil(chunks / 2), 16 if pairs <= 16 else 8), min(math.ceil(chunks / 4), 32 if pairs <= 32 else 16))
 
 
 def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,

@@ -242,6 +242,17 @@ int main() {
 """)
 
 
+def test_decode_grids_of_33_to_63_pairs(monkeypatch):
+    """On the 4-wave kernel at most 16 slices, and none more for up to 256 tokens (56 pairs x 200 8.7 -> 9.2 us)."""
+    from kubernetes_gpu_cluster_amd import ops
+    monkeypatch.setenv("KGC_DECODE_WAVE", "1")
+    monkeypatch.delenv("KGC_DECODE_WAVE_MIN_PAIRS", raising=False)
+    for B in (5, 6, 7):
+        assert [ops.decode_grid_z(B, 8, c) for c in (200, 256)] == [1, 1]
+        assert all(z <= max(16, -(-1024 // (8 * B))) for z in (ops.decode_grid_z(B, 8, c) for c in range(300, 8192, 100)))
+    assert ops.decode_grid_z(4, 8, 200) == 4 and ops.decode_grid_z(4, 8, 4000) == 32
+
+
 @pytest.mark.parametrize("wave,lim", [("1", None), ("0", None), ("1", "512")])
 def test_decode_grids_fit_what_is_set_aside_for_them(monkeypatch, wave, lim):
     """Many slices are for steps of few (row, kv head) pairs: larger ones on the 4-wave kernel (K1w off, or from more pairs
