@@ -233,7 +233,7 @@ def test_paged_decode_rope(gpu, monkeypatch, kern, dt, d, nq, nkv, qk_norm, S, f
 @pytest.mark.parametrize("B,nkv", [(64, 1), (72, 2), (64, 4), (64, 8), (5, 2), (3, 8)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_paged_decode_slices_of_ragged_contexts(gpu, monkeypatch, B, nkv, fp8):
-    """Contexts at the edges of a slice's least length (2 to 8 chunks of 32, 10 or 16 by the number of pairs) and of the
+    """Contexts at the edges of a slice's least length (2, 4 to 8 chunks of 32, 10 or 16 by the number of pairs) and of the
     chunks, empty ones, some in one slice and some in all, at the grid of a short context, of the longest one and of 8192
     tokens (which the tables do not have): as the reference."""
     for v in ("KGC_DECODE_WAVE_MIN_PAIRS", "KGC_DECODE_MIN_CHUNKS"):
