@@ -1330,6 +1330,45 @@ void xielu(Tensor out, Tensor z, Tensor ab) {
                     stream());
 }
 
+// shapes and alignment of prompt_silu / prompt_xielu (offsets within a tile and within w in 32 bits)
+bool prompt_gemm_fits(const Tensor& x, const Tensor& w, int64_t N) {
+  return x.dim() == 2 && w.dim() == 2 && x.size(0) >= 1 && x.size(0) <= (1 << 20) && w.size(1) == x.size(1) && w.is_contiguous() &&
+         x.stride(1) == 1 && x.stride(0) >= x.size(1) && x.stride(0) % 8 == 0 && x.stride(0) < (1 << 21) && x.size(1) % 128 == 0 &&
+         x.size(1) >= 128 && N >= 8 && N % 8 == 0 && N < (1 << 21) && w.numel() < (1ll << 30) &&
+         x.scalar_type() == w.scalar_type() && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) &&
+         x.device() == w.device() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
+}
+
+// whether prompt_silu (silu) or prompt_xielu takes the call and is the faster way
+bool prompt_gemm_pays(Tensor x, Tensor w, bool silu) {
+  if (!x.is_cuda() || w.dim() != 2 || (silu && w.size(0) % 2 != 0)) return false;
+  const int64_t N = silu ? w.size(0) / 2 : w.size(0);
+  if (!prompt_gemm_fits(x, w, N)) return false;
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  return kgc::prompt_gemm_pays(silu ? kgc::PROMPT_SILU : kgc::PROMPT_XIELU, (int)x.size(0), (int)N, (int)x.size(1));
+}
+
+void prompt_gemm(int act, Tensor out, Tensor x, Tensor w, const float* ab) {
+  check_gpu(x, "x");
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  TORCH_CHECK(w.dim() == 2 && (act != kgc::PROMPT_SILU || w.size(0) % 2 == 0), "kgc.prompt_gemm: w [N, K], SiLU: gate | up");
+  const int64_t N = act == kgc::PROMPT_SILU ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(prompt_gemm_fits(x, w, N), "kgc.prompt_gemm: x [M, K] and w of 16 bits, K in steps of 128, N of 8, 16-byte rows");
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == x.size(0) && out.size(1) == N && out.is_contiguous() &&
+              out.scalar_type() == x.scalar_type() && out.device() == x.device(), "kgc.prompt_gemm: out [M, N]");
+  kgc::launch_prompt_gemm(dt_code(x), act, out.data_ptr(), x.data_ptr(), w.data_ptr(), ab, (int)x.size(0), (int)N,
+                          (int)x.size(1), (int)x.stride(0), stream());
+}
+
+void prompt_silu(Tensor out, Tensor x, Tensor w) { prompt_gemm(kgc::PROMPT_SILU, out, x, w, nullptr); }
+
+void prompt_xielu(Tensor out, Tensor x, Tensor w, Tensor ab) {
+  check_f32(ab, "ab");
+  TORCH_CHECK(ab.numel() == 2 && ab.device() == x.device(), "kgc.prompt_xielu: ab [2]");
+  prompt_gemm(kgc::PROMPT_XIELU, out, x, w, ab.data_ptr<float>());
+}
+
 void gate_proj(Tensor out, Tensor h, Tensor w, std::optional<Tensor> bias, int64_t kind_a,
                int64_t kind_b, int64_t split, double cap) {
   check_gpu(h, "h");
@@ -2718,6 +2757,9 @@ TORCH_LIBRARY(kgc, m) {
         "int layer, int groups, float eps, Tensor(d!)? sums, int slot, int first, Tensor[] ahead) -> ()");
   m.def("head_norm_gate(Tensor(a!) out, Tensor o, Tensor g, Tensor w, int H, float eps) -> ()");
   m.def("xielu(Tensor(a!) out, Tensor z, Tensor ab) -> ()");
+  m.def("prompt_gemm_pays(Tensor x, Tensor w, bool silu) -> bool");
+  m.def("prompt_silu(Tensor(a!) out, Tensor x, Tensor w) -> ()");
+  m.def("prompt_xielu(Tensor(a!) out, Tensor x, Tensor w, Tensor ab) -> ()");
   m.def("gate_proj(Tensor(a!) out, Tensor h, Tensor w, Tensor? bias, int kind_a, int kind_b, int split, "
         "float cap) -> ()");
   m.def("rope_kv_store(Tensor qkv, Tensor positions, Tensor? table, Tensor(a!) q_out, Tensor(b!) k_cache, "
@@ -2860,6 +2902,9 @@ TORCH_LIBRARY_IMPL(kgc, CUDA, m) {
   m.impl("depth_mix_sums", &depth_mix_sums);
   m.impl("head_norm_gate", &head_norm_gate);
   m.impl("xielu", &xielu);
+  m.impl("prompt_gemm_pays", &prompt_gemm_pays);
+  m.impl("prompt_silu", &prompt_silu);
+  m.impl("prompt_xielu", &prompt_xielu);
   m.impl("gate_proj", &gate_proj);
   m.impl("rope_kv_store", &rope_kv_store);
   m.impl("window_attention", &window_attention);

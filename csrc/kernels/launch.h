@@ -269,6 +269,11 @@ void launch_depth_mix_norm(int dtype, void* out, float* x, float* hist, const vo
                            int rows, int W, int groups, float eps, const DepthAhead& m, hipStream_t s);
 void launch_head_norm_gate(int dtype, void* out, const float* o, const void* g, int64_t g_stride,
                            const float* w, int rows, int H, int dv, float eps, hipStream_t s);
+// act(x W^T): SILU with w = gate | up [2 N, K], XIELU with w [N, K]; K a multiple of 128, N of 8, rows of x in 16-byte units
+constexpr int PROMPT_SILU = 1, PROMPT_XIELU = 2;
+bool prompt_gemm_pays(int act, int M, int N, int K);
+void launch_prompt_gemm(int dtype, int act, void* out, const void* x, const void* w, const float* ab, int M, int N,
+                        int K, int ldx, hipStream_t s);
 void launch_xielu(int dtype, void* out, const void* z, const float* ab, int64_t n, hipStream_t s);
 void launch_gate_proj(int dtype, float* out, const void* h, const void* w, const float* bias,
                       int rows, int W, int N, int kind_a, int kind_b, int split, float cap,

@@ -11,7 +11,7 @@ the gates, the recurrence and the attention softmax stay in fp32.
 Kernel sequence per layer (ops/__init__.py, "hybrid decoders"):
   [depth_mix_norm of the previous layer -> h]  qkv GEMM -> gate_proj -> rope_kv_store ->
   window_attention (head gate in its epilogue) -> o GEMM -> group_rms_norm(add) -> up
-  GEMM -> xielu -> down GEMM -> depth_mix_norm
+  GEMM with xielu -> down GEMM -> depth_mix_norm
   mLSTM: qkvg GEMM -> gate_proj -> mlstm_scan -> head_norm_gate -> o GEMM -> depth_mix_norm
 One GPU per replica (TP = PP = 1).
 """
@@ -25,6 +25,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from ..ops.gemm import linear_xielu
 from ..parallel.layers import ParallelLMHead, ReplicatedLinear, VocabParallelEmbedding
 from ..parallel.state import get_state
 from .attention import ForwardContext, WindowedAttention
@@ -52,7 +53,7 @@ class XIELUMLP(nn.Module):
         self.act.data.copy_(torch.stack([sp[0], 0.5 + sp[1]]))
 
     def forward(self, h):
-        return self.down_proj(ops.xielu(self.up_proj(h), self.act))
+        return self.down_proj(linear_xielu(h, self.up_proj.weight, self.act))
 
 
 class DilavikLayer(nn.Module):

@@ -26,6 +26,7 @@ import torch.nn.functional as F
 log = logging.getLogger("kgc.gemm")
 
 SKINNY_MAX_M = 64
+PROMPT_MIN_M = SKINNY_MAX_M + 1    # fewer rows are the skinny plans' (csrc/kernels/gemm_prompt.hip, prompt_gemm_pays)
 # (mt, nt, nw, ntl) configurations the tuner tries; mt = 16-row batch tiles.
 _CONFIGS = [(mt, nt, nw, ntl) for mt in (1, 2, 4) for nt in (1, 2) for nw in (4, 8, 16)
             for ntl in (True, False)]
@@ -198,7 +199,8 @@ def _dg_plan(x: torch.Tensor, w: torch.Tensor, kind: str):
 def linear_silu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """silu_mul(linear(x, w, bias)) over a merged gate_up weight: where the plan runs K9m
     at this (M, N, K) the activation is the GEMM's epilogue (S = 1) or rides the split-K
-    reduction (``splitk_reduce_silu``), so the [M, 2I] gate_up output never exists."""
+    reduction (``splitk_reduce_silu``), so the [M, 2I] gate_up output never exists; nor
+    does it for prompt rows (csrc/kernels/gemm_prompt.hip)."""
     from . import _k, silu_mul
     if bias is None and x.is_cuda and x.dim() == 2 and x.stride(1) == 1 and _plan_silu:
         cfg = _plan_silu.get((x.shape[0], w.shape[0], w.shape[1]))
@@ -214,7 +216,29 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
             out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype, device=x.device)
             _k().splitk_reduce_silu(out, ws, _dg_info(cfg)[2])
             return out
+        if _prompt_pays(x, w, True):
+            out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype, device=x.device)
+            _k().prompt_silu(out, x, w)
+            return out
     return silu_mul(linear(x, w, bias))
+
+
+def _prompt_pays(x: torch.Tensor, w: torch.Tensor, silu: bool) -> bool:
+    """Whether a step's rows take the projection that has the activation in it (no plan of a
+    decode GEMM does, which come first)."""
+    from . import _k
+    return (x.is_cuda and x.dim() == 2 and x.shape[0] >= PROMPT_MIN_M and x.dtype in (torch.bfloat16, torch.float16)
+            and _k().prompt_gemm_pays(x, w, silu))
+
+
+def linear_xielu(x: torch.Tensor, w: torch.Tensor, ab: torch.Tensor) -> torch.Tensor:
+    """xielu(linear(x, w), ab); prompt rows in one launch (csrc/kernels/gemm_prompt.hip)."""
+    from . import _k, xielu
+    if _dg_plan(x, w, "plain") is None and _prompt_pays(x, w, False):
+        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        _k().prompt_xielu(out, x, w, ab)
+        return out
+    return xielu(linear(x, w), ab)
 
 
 def linear_qkv(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

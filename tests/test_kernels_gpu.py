@@ -1653,3 +1653,58 @@ def test_dg_table_fingerprint_guards_stale_tables(gpu, tmp_path, monkeypatch):
         assert gemm.load_dg_table("llama-3-8b") > 0
     finally:
         gemm.clear_plan()
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("act", ["silu", "xielu"])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 128),          # one quarter tile, one output unit, two steps
+                                   (129, 136, 384),      # a row and a unit past a quarter's edge
+                                   (300, 520, 256),
+                                   (1300, 4104, 128),    # halves in the last round
+                                   (3500, 5120, 384),   # whole rounds, then pieces
+                                   (2100, 7688, 256)])
+def test_prompt_gemm_matches_fp64(gpu, dt, act, M, N, K):
+    """The projection with its activation (gemm_prompt.hip) against float64.  Per element: the roundings of the result
+    and of the projection (2^-8 or 2^-11 of them, the latter times the activation's slope), and fp32 sums of K products
+    of unit variance in total, 4 sqrt(K) 2^-24, times slopes below 8 here."""
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, device=gpu).to(dt)[:, :K]           # a row stride of its own
+    w = (torch.randn(2 * N if act == "silu" else N, K, device=gpu) * K ** -0.5).to(dt)
+    z = x.double() @ w.double().t()
+    out = torch.full((M, N), float("nan"), dtype=dt, device=gpu)
+    if act == "silu":
+        g, s = z[:, :N], torch.sigmoid(z[:, :N])
+        want = g * s * z[:, N:]
+        slope = (s * (1 + g * (1 - s)) * g * z[:, N:]).abs() + want.abs()
+        ops._k().prompt_silu(out, x, w)
+    else:
+        ab = torch.tensor([0.7, 1.1], device=gpu)
+        a, b = ab.double()
+        want = torch.where(z > 0, a * z * z + z / 2, b * (torch.expm1(z) - z) + z / 2)
+        slope = (torch.where(z > 0, 2 * a * z, b * torch.expm1(z)) + 0.5).abs() * z.abs()
+        ops._k().prompt_xielu(out, x, w, ab)
+    u = 2.0 ** (-8 if dt == torch.bfloat16 else -11)
+    worst = ((out.double() - want).abs() - 1.02 * u * (want.abs() + slope)).max()
+    assert worst <= 8 * 4 * K ** 0.5 * 2.0 ** -24, float(worst)
+
+
+def test_prompt_gemm_routes(gpu):
+    """linear_silu and linear_xielu take it where it pays and its operands fit, and only there."""
+    from kubernetes_gpu_cluster_amd.ops import gemm
+    w = torch.randn(4096, 2048, device=gpu).to(torch.bfloat16) * 2048 ** -0.5
+    ab = torch.tensor([0.7, 1.1], device=gpu)
+    x = torch.randn(4096, 2048, device=gpu).to(torch.bfloat16)
+    out = torch.empty(4096, 2048, dtype=x.dtype, device=gpu)
+    ops._k().prompt_silu(out, x, w)
+    assert torch.equal(gemm.linear_silu(x, w), out)
+    out = torch.empty(4096, 4096, dtype=x.dtype, device=gpu)
+    ops._k().prompt_xielu(out, x, w, ab)
+    assert torch.equal(gemm.linear_xielu(x, w, ab), out)
+    pays = ops._k().prompt_gemm_pays
+    assert pays(x, w, True) and not pays(x[:, :2000], w[:, :2000].contiguous(), True)      # K in steps of 128
+    assert not pays(x.float(), w.float(), True) and not pays(x, w[:4090], True)            # N in steps of 8
+    flat = torch.randn(512 * 2048 + 1, device=gpu).to(torch.bfloat16)[1:].view(512, 2048)  # rows off 16 bytes
+    assert not pays(flat, w, True)
+    for y, v in ((x[:, :2000], w[:, :2000].contiguous()), (x.float(), w.float()), (flat, w)):
+        want = ops.silu_mul(torch.nn.functional.linear(y, v))
+        torch.testing.assert_close(gemm.linear_silu(y, v).float(), want.float(), atol=3e-2, rtol=2e-2)
