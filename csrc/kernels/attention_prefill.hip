@@ -37,10 +37,20 @@ __device__ __forceinline__ int kswz(int k) { return (k & 3) | (((k >> 3) & 3) <<
 __device__ __forceinline__ float max_rows(float x) {
   const uint32_t u = __builtin_bit_cast(uint32_t, x);
   const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  x = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  x = __builtin_elementwise_maximum(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
   const uint32_t w = __builtin_bit_cast(uint32_t, x);
   const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+  return __builtin_elementwise_maximum(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
+// a barrier that leaves the newest N memory operations on their way
+template <int N> __device__ __forceinline__ void pf_meet() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 0x70);   // vmcnt(N) lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 // cos / sin of one row's dims as pf_load_q uses them, loaded ahead of the rotation
@@ -106,6 +116,55 @@ __device__ __forceinline__ void pf_load_q(const T* qrow, const float* __restrict
 // P.V is complete, and O, l and m move together (no P at the old scale is pending).
 constexpr float PF_RESCALE_THR = 8.f;
 
+// keys behind a row's own position
+__device__ __forceinline__ void pf_mask(f32x4 (&s)[2][4], const int (&qpos)[2], int key0, int qd) {
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (key0 + (j >> 1) * 32 + 8 * qd + 4 * (j & 1) + i > qpos[qt]) s[qt][j][i] = -INFINITY;
+}
+
+// Lazy online softmax of a tile's scores (query = lane & 15: lane-local statistics): p = 2^(c s - m).  The maximum is the
+// one that hands on a NaN, whose row is NaN either way: v_max first quiets every score that an MFMA has made.
+template <typename T, int D>
+__device__ __forceinline__ void pf_softmax(const f32x4 (&s)[2][4], typename Vec8<T>::type (&pf)[2][2], f32x4 (&o)[2][D / 16],
+                                           float (&m)[2], float (&l)[2], float c) {
+  constexpr int DT = D / 16;
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) {
+    float tmax = s[qt][0][0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) tmax = __builtin_elementwise_maximum(tmax, s[qt][i >> 2][i & 3]);
+    tmax = max_rows(tmax);
+    tmax *= c;                              // -inf stays -inf (a fully masked row)
+    if (__any(tmax > m[qt] + PF_RESCALE_THR)) {
+      const float mn = __builtin_elementwise_maximum(m[qt], tmax);
+      const float alpha = __builtin_amdgcn_exp2f(m[qt] - mn);   // 0 on the first tile
+      m[qt] = mn;
+      l[qt] *= alpha;
+#pragma unroll
+      for (int t = 0; t < DT; ++t) o[qt][t] *= alpha;
+    }
+    const float nm = -m[qt];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      Pack8<T> pk;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float pa = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qt][2 * kk][i], c, nm));
+        const float pb = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qt][2 * kk + 1][i], c, nm));
+        l[qt] += pa + pb;
+        pk.h[i] = from_f<T>(pa);
+        pk.h[4 + i] = from_f<T>(pb);
+      }
+      pf[qt][kk] = pk.v;
+    }
+  }
+}
+
 // One 64-key tile for a wave's 32 query rows (two 16-row q-tiles), shared by both
 // kernels.  K / V are the staged LDS images; key0 = the tile's first key.  Scores stay
 // raw through the max (scale_log2 > 0 commutes with max) and enter the exponent as
@@ -140,46 +199,9 @@ __device__ __forceinline__ void pf_wave_tile(const T* __restrict__ K, const T* _
     s[0][j] = a0;
     s[1][j] = a1;
   }
-  // ---- causal mask + lazy online softmax (query = lane&15: lane-local stats)
   V8 pf[2][2];
-#pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    if constexpr (MASK) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (key0 + (j >> 1) * 32 + 8 * qd + 4 * (j & 1) + i > qpos[qt]) s[qt][j][i] = -INFINITY;
-    }
-    float tmax = fmaxf(fmaxf(s[qt][0][0], s[qt][0][1]), fmaxf(s[qt][0][2], s[qt][0][3]));
-#pragma unroll
-    for (int j = 1; j < 4; ++j)
-      tmax = fmaxf(tmax, fmaxf(fmaxf(s[qt][j][0], s[qt][j][1]), fmaxf(s[qt][j][2], s[qt][j][3])));
-    tmax = max_rows(tmax);
-    tmax *= c;                              // -inf stays -inf (a fully masked row)
-    if (__any(tmax > m[qt] + PF_RESCALE_THR)) {
-      const float mn = fmaxf(m[qt], tmax);
-      const float alpha = __builtin_amdgcn_exp2f(m[qt] - mn);   // 0 on the first tile
-      m[qt] = mn;
-      l[qt] *= alpha;
-#pragma unroll
-      for (int t = 0; t < DT; ++t) o[qt][t] *= alpha;
-    }
-    const float nm = -m[qt];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      Pack8<T> pk;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float pa = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qt][2 * kk][i], c, nm));
-        const float pb = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qt][2 * kk + 1][i], c, nm));
-        l[qt] += pa + pb;
-        pk.h[i] = from_f<T>(pa);
-        pk.h[4 + i] = from_f<T>(pb);
-      }
-      pf[qt][kk] = pk.v;
-    }
-  }
+  if constexpr (MASK) pf_mask(s, qpos, key0, qd);
+  pf_softmax<T, D>(s, pf, o, m, l, c);
   // ---- O^T += V^T . P^T
 #pragma unroll
   for (int t = 0; t < DT; ++t) {
@@ -544,7 +566,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_gqa_kernel(
   }
 }
 
-// Persistent GQA variant: ONE workgroup per CU walks the work list (items = (128-row work
+// Persistent GQA variant (fp8 caches, pages of fewer than 32 keys): ONE workgroup per CU walks the work list (items = (128-row work
 // item, kv-head group, QB-row sub-block), heaviest first, dealt round-robin), with the K / V
 // tile stream running ACROSS items: the last tile of an item loads the next item's first
 // tile into the free LDS buffer, so a new item starts with its tile already staged.
@@ -819,8 +841,8 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
       const int row = 4 * i + rl, qi = done.qbase + wrow + row;
       const u32x4 v = *reinterpret_cast<const u32x4*>(rows + row * D + cl * 8);
       if (qi < done.qlen)
-        *reinterpret_cast<u32x4*>(out + ((int64_t)(done.q0 + qi) * nq + done.hg0 + whead) * D +
-                                  ((cl ^ (row & 15)) * 8)) = v;
+        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out + ((int64_t)(done.q0 + qi) * nq + done.hg0 + whead) * D +
+                                  ((cl ^ (row & 15)) * 8)));
     }
     if (!has_next) break;
     // the next item's first tile is already staged in LDS buffer `buf`
@@ -830,13 +852,294 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
   }
 }
 
+// The walk for 16-bit caches with pages of 32 keys or more: as prefill_attn_gqa_persist_kernel, by workgroups of 4 waves
+// (4 heads x 32 queries) of which two share a CU, so that one computes while the other is between two items or waits.
+// K and V tiles come by DMA into two buffers each, in the order in which the MFMAs read them: unit c of key k at
+// c ^ f(k), V^T in groups of 8 keys as the cache has them; one barrier per tile.  A tile is asked for while the one before
+// it computes, its pages a tile before that, the next item's q in registers.  What only items need is read again from the
+// arguments: there are no scalar registers left for it.  Neighbouring items are the kv heads of the same rows, so that with
+// 8 of them an XCD sees one in all rounds.
+//
+// What bounds it: latency.  Of a tile's 5500 cycles (two waves per SIMD) 2050 are the matrix core's and 1900 vector
+// instructions'; a fifth is the barrier (four waves, each beside another workgroup's), and at 32 x 512 rows the rotation
+// of q and the output rows are another fifth and the slowest workgroup takes a quarter longer than the mean.  K / V write
+// included, the 8-wave walk -> here, us: 32 x 512 188.7 -> 174.9, 64 x 256 151.8 -> 143.6, 8 x 2048 398 -> 344, 4 x 4096 732 ->
+// 622, 20 x 300 80.6 -> 68.7, 8 x 500 after 3000 285 -> 243.  Items dealt over all XCDs: 8 x 2048 362; K by DMA a tile ahead and
+// V within its tile: 373; operands read six steps ahead in the source: 377; indices drawn from a counter: 499.
+struct WalkArgs {
+  const void *q, *kc, *vc;
+  void* out;
+  const float* cos_sin;
+  const int *block_tables, *qsl, *seq_lens, *work_seq, *work_mblk;
+  int64_t q_stride;
+  int bt_stride, nq, nkv, bs_log2, num_blocks, cs_rows, n_items;
+  float scale_log2, v_scale;
+};
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArgs) {
+  static_assert(D == 128 && PF_BN == 64 && sizeof(T) == 2, "rows and groups per DMA");
+  typedef typename Vec8<T>::type V8;
+  typedef __attribute__((address_space(3))) void* LdsPtr;
+  typedef const __attribute__((address_space(4))) WalkArgs* ArgPtr;
+  typedef const __attribute__((address_space(4))) int* ScalarPtr;
+  constexpr int GH = 4, QB = 32, ZS = PF_BM / QB, KS = D / 32, DT = D / 16, RB = D * 2;   // RB: bytes of a row
+  // (objects of their own: the compiler lets an LDS read follow every DMA into the object that it reads)
+  __shared__ __attribute__((aligned(16))) T K0[PF_BN * D], K1[PF_BN * D], V0[PF_BN * D], V1[PF_BN * D], all_rows[4 * 16 * D];
+  auto args = [] {                           // not kept: see above
+    ArgPtr p = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+  };
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r16 = lane & 15, qd = lane >> 4;
+  T* rows = all_rows + wave * 16 * D;        // where 16 output rows meet, to be stored 256 bytes at a time
+  // (lane and wave behind an opaque move: what depends on them alone is not kept over the tile loop)
+  auto opaque = [](int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+  };
+  auto uopaque = [](int x) {
+    asm volatile("" : "+s"(x));
+    return x;
+  };
+
+  // row0, nrow: rows of q; pos0: the first one's position; L: keys; k, v: the kv head's place in page 0
+  struct Item {
+    int row0, nrow, pos0, head, L, n_tiles;
+    const int* bt;
+    const char *k, *v;
+  };
+  auto decode = [&](int idx, Item& I) -> bool {
+    const ArgPtr a = args();
+    const int nkv = a->nkv, G = a->nq / nkv, Y = nkv * (G / GH), bs_log2 = a->bs_log2;
+    const int w = idx / (Y * ZS), r = idx - w * (Y * ZS), z = r / Y, y = r - z * Y, h = y / (G / GH);
+    const int seq = ((ScalarPtr)a->work_seq)[w], mb = ((ScalarPtr)a->work_mblk)[w];
+    const int q0 = ((ScalarPtr)a->qsl)[seq], qlen = ((ScalarPtr)a->qsl)[seq + 1] - q0;
+    int L_in = ((ScalarPtr)a->seq_lens)[seq];
+    const int cap = a->bt_stride << bs_log2;
+    KGC_DCHECK_RANGE(L_in, 0, cap + 1, "prefill seq_len");
+    I.L = min(L_in, cap);
+    const int ctx0 = I.L - qlen, qbase = mb * PF_BM + (ZS - 1 - z) * QB;
+    if (qlen <= 0 || ctx0 < 0 || qbase >= qlen) return false;
+    I.row0 = q0 + qbase;
+    I.nrow = min(qlen - qbase, QB);
+    I.pos0 = ctx0 + qbase;
+    I.head = h * G + (y % (G / GH)) * GH;
+    I.n_tiles = (I.pos0 + I.nrow - 1) / PF_BN + 1;
+    I.bt = a->block_tables + (int64_t)seq * a->bt_stride;
+    const int64_t at = (int64_t)h * ((int64_t)RB << bs_log2);
+    I.k = static_cast<const char*>(a->kc) + at;
+    I.v = static_cast<const char*>(a->vc) + at;
+    return true;
+  };
+  // rounds of items, alternating direction (as the 8-wave walk's)
+  const int G_ = gridDim.x, b_ = blockIdx.x, n_items = args()->n_items;
+  const int turn = G_ % 8 == 0 ? (G_ - 8 - (b_ & ~7)) | (b_ & 7) : G_ - 1 - b_;
+  auto next_valid = [&](int r, Item& I) -> int {
+    while (r * G_ < n_items) {
+      const int idx = r * G_ + ((r & 1) ? turn : b_);
+      if (idx < n_items && decode(idx, I)) break;
+      ++r;
+    }
+    return r;
+  };
+  const int bs_log2 = args()->bs_log2, bsm = (1 << bs_log2) - 1;
+  const uint32_t page_bytes = (uint32_t)args()->nkv * ((uint32_t)RB << bs_log2);
+  // The two pages (or halves of one) of a tile, in even and odd lanes: a scalar load would make every LDS read
+  // that is waited for beside it wait for it.
+  auto page_ids = [&](const int* bt, int L, int kt) {
+    int i = min(kt * PF_BN + 32 * (opaque(lane) & 1), L - 1) >> bs_log2;
+    KGC_DCHECK_RANGE(i, 0, args()->bt_stride, "block-table column");
+    int v = bt[i];
+    KGC_DCHECK_RANGE(v, 0, args()->num_blocks, "block id");
+    return v;
+  };
+  // (buffer loads: behind a flat one every wait is one for everything)
+  auto dma = [&](__amdgpu_buffer_rsrc_t src, T* dst, int at) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (LdsPtr)dst, 16, at, 0, 0, 0);
+  };
+  // DMA u of a wave: keys 16 u + 4 wave .. + 3 of the tile, and half of the group of 8 keys that holds them
+  auto ask_k = [&](const char* k, int L, int kt, const uint64_t (&at)[2], T* K, int u) {
+    const int w = uopaque(wave), key = min(kt * PF_BN + 16 * u + 4 * w + qd, L - 1);
+    const int c = r16 ^ (qd | ((2 * u + (w >> 1)) & 3) << 2);
+    const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(k + at[u >> 1]), 0, RB << bs_log2, 0x00027000);
+    dma(src, K + (16 * u + 4 * w) * D, (key & bsm) * RB + c * 16);
+  };
+  auto ask_v = [&](const char* v, int L, int kt, const uint64_t (&at)[2], T* V, int u) {
+    const int w = uopaque(wave), g = 2 * u + (w >> 1), key = min(kt * PF_BN + 8 * g, L - 1) & ~7;
+    const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(v + at[u >> 1]), 0, RB << bs_log2, 0x00027000);
+    dma(src, V + g * 8 * D + (w & 1) * 4 * D, (key & bsm) * RB + (w & 1) * 1024 + lane * 16);
+  };
+  // the wave's 32 rows of q as they are; rows past the last: zeros
+  Pack8<T> qn[2][KS];
+  auto ask_q = [&](const Item& I) {
+    const ArgPtr a = args();
+    const int ln = opaque(lane), rs = (int)a->q_stride * 2;
+    const auto src = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(static_cast<const char*>(a->q) + ((int64_t)I.row0 * a->q_stride + (int64_t)(I.head + wave) * D) * 2), 0,
+        (I.nrow - 1) * rs + RB, 0x00027000);
+    const int at = (ln & 15) * rs + (ln >> 4) * 16;
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        qn[qt][s].u = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, at + qt * 16 * rs + s * 64, 0, 0));
+  };
+  V8 qf[2][KS];
+  int qpos[2];
+  auto take_q = [&](const Item& I) {
+    const ArgPtr a = args();
+    const float* cos_sin = a->cos_sin;
+    const int ln = opaque(lane), r16 = ln & 15, qd = ln >> 4;
+    PfRot<D> rot[2];
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      qpos[qt] = I.pos0 + min(qt * 16 + r16, I.nrow - 1);
+      if (cos_sin != nullptr) pf_issue_rot<D>(cos_sin + (int64_t)min(qpos[qt], a->cs_rows - 1) * D, qd, rot[qt]);
+    }
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      if (cos_sin != nullptr) pf_rotate<T, D>(rot[qt], qn[qt]);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) qf[qt][s] = qn[qt][s].v;
+    }
+  };
+
+  Item cur, nxt;
+  int it = next_valid(0, cur);
+  if (it * G_ >= n_items) return;            // uniform: the whole workgroup leaves
+  uint64_t at[2];                            // of the tile that computes next
+  int id = page_ids(cur.bt, cur.L, 0), page[2];       // pages of the one behind it
+  auto pages = [&] {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) page[p] = __builtin_amdgcn_readlane(id, p);
+  };
+  auto places = [&] {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) at[p] = (uint64_t)(uint32_t)page[p] * page_bytes;
+  };
+  pages();
+  places();
+  ask_q(cur);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    ask_k(cur.k, cur.L, 0, at, K0, u);
+    ask_v(cur.v, cur.L, 0, at, V0, u);
+  }
+  int nit = next_valid(it + 1, nxt);
+  bool has_next = nit * G_ < n_items;
+  if (!has_next) nxt = cur;
+  id = cur.n_tiles > 1 ? page_ids(cur.bt, cur.L, 1) : page_ids(nxt.bt, nxt.L, 0);
+  pages();
+  take_q(cur);
+  f32x4 o[2][DT];
+  float m[2], l[2];
+  auto fresh = [&] {
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      m[qt] = -INFINITY, l[qt] = 0.f;
+#pragma unroll
+      for (int t = 0; t < DT; ++t) o[qt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  fresh();
+  const float c = args()->scale_log2;
+  int kt = 0;
+  // One tile, in K and V (or on its way there); the one behind it goes to Kn and Vn.  True after the last tile of the last item.
+  auto tile = [&](const T* K, const T* V, T* Kn, T* Vn) -> bool {
+    const bool last = kt + 1 == cur.n_tiles;
+    // it is here (the output rows stored behind it need not be there), and everyone is done with the one before it
+    if (kt == 0) pf_meet<8>();
+    else pf_meet<0>();
+    places();
+    if (kt == 0) ask_q(nxt);
+    const bool own = kt + 2 < cur.n_tiles;
+    id = page_ids(own ? cur.bt : nxt.bt, own ? cur.L : nxt.L, own ? kt + 2 : last ? min(1, nxt.n_tiles - 1) : 0);
+    // (behind the last item its rows again)
+    const char *nk = last ? nxt.k : cur.k, *nv = last ? nxt.v : cur.v;
+    const int nL = last ? nxt.L : cur.L, nkt = last ? 0 : kt + 1;
+    f32x4 s[2][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const T* krow = K + ((j >> 1) * 32 + 8 * (r16 >> 2) + (r16 & 3) + 4 * (j & 1)) * D;
+      f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const V8 f = *reinterpret_cast<const V8*>(krow + (((4 * ks + qd) ^ r16) * 8));
+        a0 = mfma16x16x32(f, qf[0][ks], a0);
+        a1 = mfma16x16x32(f, qf[1][ks], a1);
+      }
+      s[0][j] = a0;
+      s[1][j] = a1;
+      ask_k(nk, nL, nkt, at, Kn, j);         // (one DMA at a time: a burst holds the wave up)
+    }
+    V8 pf[2][2];
+    if ((kt + 1) * PF_BN - 1 > cur.pos0) pf_mask(s, qpos, kt * PF_BN, qd);
+    pf_softmax<T, D>(s, pf, o, m, l, c);
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const V8 f = *reinterpret_cast<const V8*>(V + (4 * kk + qd) * 8 * D + (16 * t + r16) * 8);
+        o[0][t] = mfma16x16x32(f, pf[0][kk], o[0][t]);
+        o[1][t] = mfma16x16x32(f, pf[1][kk], o[1][t]);
+      }
+      if (t & 1) ask_v(nv, nL, nkt, at, Vn, t >> 1);
+    }
+    pages();                                 // (older than the tile's DMAs)
+    ++kt;
+    if (!last) return false;
+    // ---- the item's rows, and the next one's q
+    take_q(nxt);
+    const int ln = opaque(lane), r16 = ln & 15, qd = ln >> 4;
+    const ArgPtr a = args();
+    const int os = a->nq * RB;
+    const auto od = __builtin_amdgcn_make_buffer_rsrc(
+        static_cast<char*>(a->out) + (int64_t)cur.row0 * os + (int64_t)(cur.head + wave) * RB, 0, (cur.nrow - 1) * os + RB, 0x00027000);
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      float tot = l[qt];
+      tot += __shfl_xor(tot, 16, 64);
+      tot += __shfl_xor(tot, 32, 64);
+      const float inv = a->v_scale / tot;
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        Pack4<T> pk;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pk.h[i] = from_f<T>(o[qt][t][i] * inv);
+        *reinterpret_cast<u32x2*>(rows + r16 * D + (((2 * t + (qd >> 1)) ^ r16) * 8) + 4 * (qd & 1)) = pk.u;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {          // rows past the last are not written
+        const u32x4 v = *reinterpret_cast<const u32x4*>(rows + (4 * i + qd) * D + r16 * 8);
+        __builtin_amdgcn_raw_buffer_store_b128(v, od, (qt * 16 + 4 * i + qd) * os + ((r16 ^ qd) * 16 ^ i * 64), 0, 2);
+      }
+    }
+    if (!has_next) return true;
+    cur = nxt;
+    it = nit;
+    nit = next_valid(it + 1, nxt);
+    has_next = nit * G_ < n_items;
+    if (!has_next) nxt = cur;
+    if (cur.n_tiles == 1) {                  // (the pages behind it were taken to be its own)
+      id = page_ids(nxt.bt, nxt.L, 0);
+      pages();
+    }
+    fresh();
+    kt = 0;
+    return false;
+  };
+  while (!tile(K0, V0, K1, V1) && !tile(K1, V1, K0, V0)) {}
+  __builtin_amdgcn_s_waitcnt(0x0f70);        // DMAs end before the LDS is another's
+}
+
 // KGC_PREFILL_GQA=0: the one-head-per-workgroup kernel everywhere (A/B and tests)
 static int prefill_gqa_enabled() {
   const char* e = getenv("KGC_PREFILL_GQA");
   return e ? atoi(e) : 1;
 }
 
-// KGC_PREFILL_PERSIST=0: the one-shot GQA grid everywhere, =1: the persistent walk (A/B, tests)
+// KGC_PREFILL_PERSIST=0: the one-shot GQA grid everywhere, =1: the persistent walks (A/B, tests)
 static int prefill_persist_mode() {
   const char* e = getenv("KGC_PREFILL_PERSIST");
   return e ? atoi(e) : -1;
@@ -852,12 +1155,28 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
   const int G = nq / nkv;
   const int64_t n_items = (int64_t)n_work * nkv * (G / GH) * (PF_BM / (256 / GH));
   const int n_cu = device_cus();
-  // The walk pays with more items than CUs (32 x 512 rows, 32 heads: 162 us against 185); with one item
+  const int mode = prefill_persist_mode();
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const bool dma = aligned(q) && q_stride % 8 == 0;    // 16-byte DMAs
+  if constexpr (!KV8) {
+    // Few rows on short tables are one tile each, for which the walk has nothing to overlap (2 x 64 rows 17.2 us, the one-shot
+    // grid 16.2; 16 x 60 27.2 and 27.5); all else is faster so: one-shot grid -> walk, K / V write included, us: 512 rows
+    // 32.5 -> 27.5, 1000 51.9 -> 39.1, 2000 after 2000 164 -> 128, 8 x 100 after 3000 127 -> 98, 4 x 300 30.4 -> 27.8.
+    const int64_t n = (int64_t)n_work * nkv * (G / 4) * (PF_BM / 32);
+    const bool pays = n > 2 * n_cu || ((int64_t)bt_stride << bs_log2) > 128;
+    if (dma && aligned(kc) && aligned(vc) && aligned(out) && bs_log2 >= 5 && (mode < 0 ? pays : mode != 0) &&
+        n < ((int64_t)1 << 30) && q_stride < (1 << 24) && (int64_t)nq * D < (1 << 24) &&
+        ((int64_t)nkv * D << bs_log2) < ((int64_t)1 << 31)) {       // offsets inside an item and a page in 32 bits
+      const WalkArgs a{q, kc, vc, out, cos_sin, bt, qsl, sl, ws, wm, q_stride, bt_stride, nq, nkv, bs_log2, num_blocks,
+                       cs_rows, (int)n, scale_log2, v_scale};
+      prefill_attn_walk_kernel<T, D><<<(int)std::min<int64_t>(n, 2 * n_cu), 256, 0, s>>>(a);
+      return;
+    }
+  }
+  // The 8-wave walk pays with more items than CUs (32 x 512 rows, 32 heads: 162 us against 185); with one item
   // per CU or less, twice as many workgroups of half the rows do (8 x 100 rows after 3000: 119 against
   // 128, 512 rows alone 26 against 28, 2000 after 2000 159 against 161).
-  const int mode = prefill_persist_mode();
-  const bool dma = reinterpret_cast<uintptr_t>(q) % 16 == 0 && q_stride % 8 == 0;    // 16-byte DMAs
-  // one workgroup per CU: launch_bounds(512, 1), 128 KB of LDS (K / V tiles, the waves' q / output rows)
+  // One workgroup per CU: launch_bounds(512, 1), 128 KB of LDS (K / V tiles, the waves' q / output rows).
   const auto walk = &prefill_attn_gqa_persist_kernel<T, D, KV8, GH>;
   if (dma && (mode < 0 ? n_items > n_cu : mode != 0) && n_items < ((int64_t)1 << 30)) {
     walk<<<(int)std::min<int64_t>(n_items, n_cu), 512, 0, s>>>(

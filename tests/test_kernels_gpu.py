@@ -1708,3 +1708,48 @@ def test_prompt_gemm_routes(gpu):
     for y, v in ((x[:, :2000], w[:, :2000].contiguous()), (x.float(), w.float()), (flat, w)):
         want = ops.silu_mul(torch.nn.functional.linear(y, v))
         torch.testing.assert_close(gemm.linear_silu(y, v).float(), want.float(), atol=3e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("nq,nkv,bs", [(32, 8, 32), (8, 1, 64), (12, 3, 128)])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("shape", ["short_many", "mixed_chunked", "one_item"])
+def test_prefill_walk_of_large_pages(gpu, monkeypatch, dt, nq, nkv, bs, rope, shape):
+    """The walk of 4-wave workgroups (16-bit caches, pages of 32 keys or more) against the one-shot grid, whose tiles
+    and sums it has: bit for bit, by itself and from a captured graph.  Items of one tile before and after long ones,
+    lengths around tiles, pages and blocks, empty sub-blocks, q rows with a stride of their own."""
+    torch.manual_seed(31 + nq + bs)
+    d = 128
+    if shape == "short_many":
+        seq_lens = [200, 64, 65, 63, 1, 129, 300, 32, 33, 500] * 9
+        query_lens = [L - L // 3 if i % 4 == 0 else L for i, L in enumerate(seq_lens)]
+    elif shape == "mixed_chunked":
+        seq_lens, query_lens = [5, 130, 300, 64, 700, 1030, 17], [5, 130, 100, 1, 257, 1030, 3]
+    else:
+        seq_lens, query_lens = [40], [40]
+    kc, vc, bt = _fill_random_cache(len(seq_lens), seq_lens, nkv, bs, d, dt, gpu)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)   # noqa: E731
+    qsl, sl = i32([0] + query_lens).cumsum(0).int(), i32(seq_lens)
+    ws, wm = map(i32, ops.prefill_work_list(query_lens, seq_lens))
+    qkv = torch.randn(sum(query_lens), (nq + 2 * nkv) * d + 64, dtype=dt, device=gpu)[:, :-64]
+    cs = ref.rope_cos_sin_cache(d, 1100, 500000.0).to(gpu)
+
+    def run():
+        if rope:
+            return ops.prefill_attention_rope(qkv, cs, kc, vc, bt, qsl, sl, d ** -0.5, nq, d, ws, wm)
+        q = qkv[:, : nq * d].contiguous().view(-1, nq, d)
+        return ops.prefill_attention(q, kc, vc, bt, qsl, sl, d ** -0.5, ws, wm)
+    outs = []
+    for persist in ("0", "1"):
+        monkeypatch.setenv("KGC_PREFILL_PERSIST", persist)
+        outs.append(run().clone())
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and bool(torch.isfinite(outs[1]).all())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = run()
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, outs[0])
