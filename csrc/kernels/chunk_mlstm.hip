@@ -561,11 +561,12 @@ __global__ __launch_bounds__(NT) void mlstm_walk_kernel(const MlstmArgs a) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) S[0][j] *= decay;
     }
+    // (past the caches, which whole lines of results would fill: 32 x 512 tokens 131 -> 127.6 us, 1 x 4000 102.4 -> 101)
     auto put_o = [&](int i, int g, const f32x4& f) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float y = o[i][g * 4 + r] * f[r];
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), od, oat + (i * 32 + g * 8 + r) * ro * 4, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), od, oat + (i * 32 + g * 8 + r) * ro * 4, 0, 2);
       }
     };
     // ---- n <- decay n + sum_t w_t k_t: 32 rows per wave, the weights' parts as columns ------------
