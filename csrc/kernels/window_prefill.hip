@@ -24,6 +24,13 @@
 // takes; the rest is the barrier, and 3.5 rounds of workgroups that take 4.  bf16, in MFMAs of 16 x 16 x 32 -> so, us:
 // 197 -> 179 to 184, 32 x 512 rows 90 -> 76, latent rows 124 -> 110 to 116, capped and causal with a gate 290 -> 261.
 // (A ring of four tiles filled by LDS-DMA three tiles ahead: 249 us where this took 229.)
+//
+// That is ROWS64, one workgroup to a CU.  A step that does not fill the chip with them, or fills it just beyond a round, is
+// bound by one workgroup's chain of tiles, 4 us each; two forms shorten it.  ROWS32: 4 waves own 32 rows, two workgroups
+// to a CU (3 us for a tile where a workgroup has the CU for itself).  ROWS32X2: 8 waves own 32 rows, and of the tiles each
+// 4 waves take every other one; their sums meet at the end.  Both copy tiles by DMA into unpadded buffers, without the
+// registers and the instructions that eight units per thread would take (by registers: capped ones spill, latent rows
+// at 32 rows 142 us where DMA takes 115).  Figures: at the rule below.
 #include "device.h"
 #include "chunk.h"
 #include "window.h"
@@ -34,7 +41,8 @@ namespace kgc {
 
 namespace {
 
-constexpr int BM = 64, BN = 64, HW = 4, NT = 512;     // rows, keys per tile, heads per workgroup
+enum { ROWS64, ROWS32, ROWS32X2 };                    // forms: see above
+constexpr int BN = 64, HW = 4;                        // keys per tile, heads per workgroup
 
 // two weights as value + remainder
 template <typename T>
@@ -64,8 +72,8 @@ __device__ __forceinline__ float tanh_far(float y) {
 
 // KS: dk / 16; DT: dv / 32; NB: blocks of 32 keys per softmax step (fewer: fewer registers); ALIAS: values
 // are the first dv columns of the key rows
-template <typename T, int KS, int DT, int NB, bool ALIAS, bool CAP>
-__global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
+template <typename T, int KS, int DT, int NB, bool ALIAS, bool CAP, int FORM>
+__global__ __launch_bounds__(FORM == ROWS32 ? 256 : 512, 2) void window_prefill_gqa_kernel(
     T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k_cache,
     const T* __restrict__ v_cache, const int* __restrict__ qsl, const int* __restrict__ seq_lens,
     const int* __restrict__ pbt, int bt_stride, const int* __restrict__ work_seq,
@@ -73,7 +81,12 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
     int num_blocks, float scale, int window, int keep_first, const float* __restrict__ gate,
     WindowExtra ex) {
   typedef typename Vec8<T>::type V8;
-  constexpr int DK = KS * 16, DV = DT * 32, KST = DK + 8, VST = ALIAS ? KST : DV + 8;
+  typedef __attribute__((address_space(3))) void* LdsPtr;
+  constexpr bool DMA = FORM != ROWS64;
+  constexpr int BM = DMA ? 32 : 64, NT = 512, GR = FORM == ROWS32X2 ? 2 : 1;   // GR: groups of 4 waves by DMA
+  constexpr int DK = KS * 16, DV = DT * 32, KST = DMA ? DK : DK + 8, VST = ALIAS ? KST : DMA ? DV : DV + 8;
+  constexpr int RPD = 512 / DK, NKD = BN / 4 / RPD, NVD = ALIAS ? 0 : NKD, LR = BN + RPD;   // rows per DMA, DMAs per wave and tile
+  static_assert(!DMA || ((RPD == 4 && (ALIAS || DK == DV)) || (RPD == 2 && ALIAS)), "rows of a DMA");
   constexpr int NKU = BN * DK / 8 / NT, NVU = ALIAS ? 0 : BN * DV / 8 / NT;
   constexpr bool SAME = !ALIAS && DK == DV;           // a thread's key and value units: the same rows
   static_assert(BN * DK / 8 % NT == 0 && BN * DV / 8 % NT == 0, "whole units per thread");
@@ -88,22 +101,25 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   constexpr float FAR = 8.f;
   constexpr bool EXACT = __is_same(T, bf16);
   extern __shared__ __align__(16) char smem[];
+  // (objects of their own: the compiler lets an LDS read follow every DMA into the object that it reads)
+  __shared__ __align__(16) T K0[DMA ? GR * LR * DK : 8], K1[DMA ? GR * LR * DK : 8],
+      V0[DMA && NVD ? GR * LR * DV : 8], V1[DMA && NVD ? GR * LR * DV : 8];
   T* Kb = reinterpret_cast<T*>(smem);                 // [2][BN][KST]
   T* Vb = ALIAS ? Kb : Kb + 2 * BN * KST;             // [2][BN][VST]
   // head groups run fastest: workgroups are dealt round-robin over the XCDs, so every XCD sees all
   // row blocks of its heads
-  const int item = blockIdx.y / (blk_rows / BM), sub = blockIdx.y % (blk_rows / BM);
+  const int hg = blockIdx.x, item = blockIdx.y / (blk_rows / BM), sub = blockIdx.y % (blk_rows / BM);
   const int seq = work_seq[item];
   const int q0 = qsl[seq], qlen = qsl[seq + 1] - q0, ctx0 = seq_lens[seq] - qlen;
   const int r0 = work_blk[item] * blk_rows + sub * BM;
   if (r0 >= qlen || ctx0 < 0) return;
   const int rows = min(BM, qlen - r0);
   const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, col = lane & 31, hh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = blockIdx.x * HW / (H / G);
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wave = GR == 2 ? wv & 3 : wv, group = GR == 2 ? wv >> 2 : 0;
+  const int g = hg * HW / (H / G);
   // a lane's column: a row of one of the wave's two heads (which is swapped from one row group to the next,
   // so that the waves write, and read the gates of, all four heads at a time: 1 %)
-  const int head = (int)blockIdx.x * HW + 2 * (wave & 1) + ((col >> 4) ^ (wave >> 1 & 1));
+  const int head = hg * HW + 2 * (wave & 1) + ((col >> 4) ^ (wave >> 1 & 1));
   const int* bt = pbt + (int64_t)seq * bt_stride;
   const int wr = r0 + 16 * (wave >> 1);               // the wave's first row
   const int myrow = wr + r16, qpos = ctx0 + myrow;
@@ -120,8 +136,9 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[t][i] = 0.f;
-  float m = ex.sink * LOG2E, l = hh == 0 && ex.sink > -INFINITY ? 1.f : 0.f;
-  const int p_min = ctx0 + r0, p_max = ctx0 + r0 + rows - 1;
+  float m = group == 0 ? ex.sink * LOG2E : -INFINITY, l = group == 0 && hh == 0 && ex.sink > -INFINITY ? 1.f : 0.f;
+  // (tiles start where those of 64 rows do, so that both forms have the same results)
+  const int p_min = ctx0 + (r0 & ~63), p_max = ctx0 + r0 + rows - 1;
   const int lo_min = first_visible(p_min, window, ex.chunked);
   const int ns = window > 0 ? min(keep_first, lo_min) : 0;
   const int nsink = (ns + BN - 1) / BN, ntile = nsink + (p_max - lo_min + BN) / BN;
@@ -138,8 +155,8 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   int pgk[NKU], ink[NKU], pgv[NVU > 0 ? NVU : 1], inv_[NVU > 0 ? NVU : 1];
   u32x4 rk[NKU], rv[NVU > 0 ? NVU : 1];
   // (whatever the page size, without a branch: it would end the region that the loads are placed in)
-  auto page = [&](int u, int per, int kb, int hi, int& pg, int& in) {
-    const uint32_t key = min(kb + u / per, hi - 1);
+  auto page = [&](uint32_t key, int hi, int& pg, int& in) {
+    key = min(key, (uint32_t)hi - 1);
     uint32_t at = __umulhi(key, bs_inv), r = key - at * bs;        // bs_inv = (2^32 - 1) / bs: at most one too few
     if (r >= (uint32_t)bs) {
       ++at;
@@ -151,10 +168,10 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
   auto pages = [&](int t) {
     const int kb = first_key(t), hi = end_key(t, kb);
 #pragma unroll
-    for (int i = 0; i < NKU; ++i) page(tid + NT * i, DK / 8, kb, hi, pgk[i], ink[i]);
+    for (int i = 0; i < NKU; ++i) page(kb + (tid + NT * i) / (DK / 8), hi, pgk[i], ink[i]);
     if constexpr (!SAME)
 #pragma unroll
-      for (int i = 0; i < NVU; ++i) page(tid + NT * i, DV / 8, kb, hi, pgv[i], inv_[i]);
+      for (int i = 0; i < NVU; ++i) page(kb + (tid + NT * i) / (DV / 8), hi, pgv[i], inv_[i]);
   };
   // element offset of a key's row, page by page (products of 32 bits each: a multiply-add)
   const uint32_t kpage = (uint32_t)G * bs * krs, vpage = (uint32_t)G * bs * vrs;
@@ -189,33 +206,95 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
     }
   };
 
+  // ---- tiles by DMA, RPD rows at a time that lie in one page: a tile's rows from the one before its first key whose
+  // position is a multiple of RPD.  The unit c of 16 bytes of row k lies at c ^ f(k), f(k) = (k & 3) << 2 | (k >> 2 & 3): neither
+  // the reads of 16 rows at one unit nor the transposing ones of 4 rows at four units meet in a bank.  Rows past the last
+  // key are zeros (as are their weights).  Of the i-th RPD rows lane i keeps the place, from the head's first page
+  // on, and the bytes that there are (0 past the last tile).
+  int idn = 0, inn = 0, left = 0, bytes = 0;          // n: page and row in it, of the tile after the next
+  uint32_t off0 = 0, off1 = 0;
+  const int rb = krs * (int)sizeof(T);                // (values, if they are others, at the same places of theirs)
+  auto page_ids = [&](int t) {
+    const int kb = first_key(t), hi = end_key(t, kb), key = (kb & -RPD) + RPD * lane;
+    left = t < ntile ? min(hi - key, RPD) : 0;
+    page(key, hi, idn, inn);
+  };
+  auto take_pages = [&] {
+    const uint64_t at = (uint64_t)((uint32_t)idn < (uint32_t)num_blocks ? idn : 0) * kpage + (uint64_t)(uint32_t)inn * (uint32_t)krs;
+    off0 = (uint32_t)(at << 1);
+    off1 = (uint32_t)(at >> 31);
+    bytes = max(left, 0) * rb;
+  };
+  auto dma = [&](__amdgpu_buffer_rsrc_t src, T* dst, int off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (LdsPtr)dst, 16, off, 0, 0, 0);
+  };
+  const char *kg = reinterpret_cast<const char*>(k_cache + (int64_t)g * bs * krs), *vg = reinterpret_cast<const char*>(v_cache + (int64_t)g * bs * krs);
+  const int rr = lane / (64 / RPD), row0 = RPD * wave + rr, lane_at = rr * rb + ((lane % (64 / RPD)) ^ ((row0 & 3) << 2 | (row0 >> 2 & 3))) * 16;
+  // DMA u of the tile that take_pages() was last called for (rows 4 RPD u further: the unit's bit 1 turned over
+  // where that is an odd multiple of 8)
+  auto ask = [&](const char* from, T* dst, int u) {
+    const int n = 4 * u + wave;
+    const uint64_t at = (uint64_t)__builtin_amdgcn_readlane(off1, n) << 32 | (uint32_t)__builtin_amdgcn_readlane(off0, n);
+    const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(from + at), 0, __builtin_amdgcn_readlane(bytes, n), 0x00027000);
+    dma(src, dst + RPD * n * DK, RPD == 2 ? lane_at ^ (u & 1) * 32 : lane_at);
+  };
+  auto ask_k = [&](T* K, int u) { ask(kg, K, u); };
+  auto ask_v = [&](T* V, int u) { ask(vg, V, u); };
+  // where the operands lie: 8 elements of S^T's key row and depth 16 d, 4 of V^T's key row + .. and column 32 t .., from the
+  // lane's place in bytes (by DMA its unit's bits are turned over)
+  auto k_at = [&](const T* Kt, int ka, int row, int d) {
+    const char* at = reinterpret_cast<const char*>(Kt + row * KST);
+    if constexpr (!DMA) return at + ka + 32 * d;
+    else return at + (ka ^ (d & 7) * 32) + (d >> 3) * 256;
+  };
+  auto v_at = [&](const T* Vt, int va, int row, int half, int t) {
+    const char* at = reinterpret_cast<const char*>(Vt + (row + 8 * half) * VST);
+    if constexpr (!DMA) return reinterpret_cast<const T*>(at + va + 64 * t);
+    else return reinterpret_cast<const T*>(at + (va ^ ((t & 3) * 64 + half * 32)) + (t >> 2) * 256);
+  };
+
   const float sl = CAP ? scale / ex.softcap : scale * LOG2E;
   const float fl = CAP ? ex.softcap * LOG2E : sl;  // what is left to multiply (> 0: see the launcher)
-  pages(0);
-  fetch();
-  pages(min(1, ntile - 1));
-  park(0);
-  __syncthreads();
-  for (int tile = 0; tile < ntile; ++tile) {
-    const int buf = tile & 1;
+  // One tile, in Kt and Vt (by DMA: or on its way there; the one behind it goes to Kn and Vn)
+  auto compute = [&](int tile, const T* Kt, const T* Vt, T* Kn, T* Vn) {
     // in flight while this tile is computed (the last one again at the end); where a tile is one step, the
     // addresses are made beside the products of S
     const auto next = [&] {
-      fetch();
-      pages(min(tile + 2, ntile - 1));
+      if constexpr (!DMA) {
+        fetch();
+        pages(min(tile + 2, ntile - 1));
+      }
     };
-    if (NB != 2 && tile + 1 < ntile) next();
+    if (!DMA && NB != 2 && tile + 1 < ntile) next();
     const bool sink = tile < nsink;
     const int kb = first_key(tile), hi = end_key(tile, kb);
-    const T* Kt = Kb + buf * BN * KST;
-    const T* Vt = Vb + buf * BN * VST;
+#pragma unroll
     for (int st = 0; st < BN / 32 / NB; ++st) {
       const int k0 = kb + st * 32 * NB, k1 = k0 + 32 * NB;         // this step's keys
       // nothing of them is visible to the wave's rows (kept first tokens can sit in a main tile
       // when the earliest window starts before them)
       if (!live || k0 > wp_hi || k0 >= hi || (!sink && min(hi, k1) <= w_lo && k0 >= keep_first)) {
         if (NB == 2) next();
+        if constexpr (DMA)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            ask_k(Kn, st * 4 + u);
+            if (NVD) ask_v(Vn, u);
+          }
         continue;
+      }
+      int ka, va;
+      if constexpr (DMA) {
+        const int off = kb & (RPD - 1), kr = col + off, vr = 4 * hh + (r16 >> 2) + off;
+        ka = (kr * DK + (hh ^ ((kr & 3) << 2 | (kr >> 2 & 3))) * 8) * 2;
+        va = (vr * VST + ((2 * (col >> 4) + (r16 >> 1 & 1)) ^ ((vr & 3) << 2 | (vr >> 2 & 3))) * 8 + 4 * (r16 & 1)) * 2;
+        if (KS == 16) {                      // for want of registers: not kept over the tiles
+          asm volatile("" : "+v"(ka));
+          asm volatile("" : "+v"(va));
+        }
+      } else {
+        ka = (col * KST + 8 * hh) * 2;
+        va = ((4 * hh + (r16 >> 2)) * VST + 16 * (col >> 4) + 4 * (r16 & 3)) * 2;
       }
       f32x16 s[NB];
       float mx = -INFINITY;
@@ -225,11 +304,10 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
         // S^T, four products at a time and the operands of the next four on their way; beside the first ones the next
         // tile's addresses and loads (operands read just in time: 8 x 2048 189.3 -> 187.5 us, 1 x 8192 130 -> 126)
         V8 kf[2][4];
-        const T* krow = Kt + (st * NB * 32 + col) * KST + 8 * hh;
         auto load_k = [&](int g) {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            kf[g & 1][i] = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(krow + (g * 4 / KS) * 32 * KST + 16 * (g * 4 % KS + i)));
+            kf[g & 1][i] = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(k_at(Kt, ka, 32 * (st * NB + g * 4 / KS), g * 4 % KS + i)));
         };
         static_assert(KS % 4 == 0, "");
         load_k(0);
@@ -249,35 +327,38 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[0][i]);
           __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-          interleave<4, 8, 0, 1>();
+          if constexpr (DMA) ask_k(Kn, g);
+          interleave<4, 8, 0, DMA ? 4 : 1>();
           __builtin_amdgcn_sched_barrier(0);
         }
       } else
 #pragma unroll
       for (int b = 0; b < NB; ++b) {         // S^T; beside a block's products the maximum of the one before it
-        const T* krow = Kt + ((st * NB + b) * 32 + col) * KST + 8 * hh;
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[b][i] = 0.f;
 #pragma unroll
         for (int d = 0; d < KS; ++d)
-          s[b] = mfma32x32x16(__builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(krow + 16 * d)), qf[d], s[b]);
+          s[b] = mfma32x32x16(__builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(k_at(Kt, ka, 32 * (st * NB + b), d))), qf[d], s[b]);
+        if constexpr (DMA)
+#pragma unroll
+          for (int u = 0; u < 4 / NB; ++u) ask_k(Kn, st * 4 + b * (4 / NB) + u);
         if (!CAP && b > 0)
 #pragma unroll
           for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[b - 1][i]);
         // (whole loops under each uniform test: a branch per element costs more than its work)
         if constexpr (CAP) {                 // tanh(score / cap); scores beyond 5/8 of the cap are rare
-          constexpr int GR = NB == 1 ? 4 : 16;            // at a time: registers
+          constexpr int CG = NB == 1 ? 4 : 16;            // at a time: registers
 #pragma unroll
-          for (int i0 = 0; i0 < 16; i0 += GR) {
+          for (int i0 = 0; i0 < 16; i0 += CG) {
             float far = 0.f;
 #pragma unroll
-            for (int i = i0; i < i0 + GR; ++i) {
+            for (int i = i0; i < i0 + CG; ++i) {
               s[b][i] *= sl;
               far = fmaxf(far, fabsf(s[b][i]));
             }
             if (__any(far > 0.625f)) {
 #pragma unroll
-              for (int i = i0; i < i0 + GR; ++i) {
+              for (int i = i0; i < i0 + CG; ++i) {
                 const float y = s[b][i], near = tanh_near(y);
                 float t = tanh_far(y);
                 asm("" : "+v"(t));           // (no branch per element)
@@ -286,7 +367,7 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
               }
             } else {
 #pragma unroll
-              for (int i = i0; i < i0 + GR; ++i) s[b][i] = tanh_near(s[b][i]);
+              for (int i = i0; i < i0 + CG; ++i) s[b][i] = tanh_near(s[b][i]);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
@@ -359,8 +440,8 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
       constexpr bool AHEAD = NB == 2;
       V8 vf[2];
       auto load_v = [&](int n) {             // 16 keys n / DT, columns n % DT
-        const T* vrow = Vt + ((st * NB * 32) + 16 * (n / DT) + 4 * hh + (r16 >> 2)) * VST + 16 * (col >> 4) + 4 * (r16 & 3) + 32 * (n % DT);
-        const u32x2 a = ld_tr4(vrow), b = ld_tr4(vrow + 8 * VST);
+        const int row = 32 * NB * st + 16 * (n / DT);
+        const u32x2 a = ld_tr4(v_at(Vt, va, row, 0, n % DT)), b = ld_tr4(v_at(Vt, va, row, 1, n % DT));
         vf[n & 1] = __builtin_bit_cast(V8, (u32x4{a[0], a[1], b[0], b[1]}));
       };
       if (AHEAD) {
@@ -370,6 +451,7 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
 #pragma unroll
       for (int j = 0; j < 2 * NB; ++j) {
         if (j + 1 < 2 * NB) weigh(j + 1);
+        if constexpr (DMA && NVD > 0) ask_v(Vn, j);
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
           const int n = j * DT + t;
@@ -392,9 +474,81 @@ __global__ __launch_bounds__(NT) void window_prefill_gqa_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (tile + 1 < ntile) {
-      park(buf ^ 1);
-      __syncthreads();                       // the next tile is there; this one was read
+  };
+  if constexpr (DMA) {
+    auto rest = [&](int t, T* K, T* V) {     // the last rows of a tile that starts between two multiples of RPD
+      if (wave == 0 && (first_key(t) & (RPD - 1)) != 0) {
+        ask_k(K, NKD);
+        if (NVD) ask_v(V, NKD);
+      }
+    };
+    T *Ka = K0 + group * LR * DK, *Kz = K1 + group * LR * DK, *Va = ALIAS ? Ka : V0 + group * LR * DV, *Vz = ALIAS ? Kz : V1 + group * LR * DV;
+    page_ids(group);
+    take_pages();
+    page_ids(group + GR);
+#pragma unroll
+    for (int u = 0; u < NKD; ++u) {
+      ask_k(Ka, u);
+      if (NVD) ask_v(Va, u);
+    }
+    rest(group, Ka, Va);
+    take_pages();
+    auto step = [&](int t, const T* K, const T* V, T* Kn, T* Vn) {
+      meet<0>();                             // it is here, and everyone is done with the one before it
+      page_ids(t + 2 * GR);
+      rest(t + GR, Kn, Vn);
+      if (GR == 1 || t < ntile) compute(t, K, V, Kn, Vn);
+      take_pages();                          // (older than the tile's DMAs)
+    };
+    for (int t = 0; t < ntile; t += 2 * GR) {
+      step(t + group, Ka, Va, Kz, Vz);
+      if (t + GR < ntile) step(t + GR + group, Kz, Vz, Ka, Va);
+    }
+    if constexpr (GR == 1) {
+      __builtin_amdgcn_s_waitcnt(0x0f70);    // DMAs end before the LDS is another's
+    } else {                                 // the second group's sums join the first one's
+      constexpr int N0 = DT == 4 ? 2 : 4;    // column blocks in K0; then K1
+      static_assert(GR * LR * DK * sizeof(T) >= N0 * 16384 && GR * LR * DK * sizeof(T) >= (DT - N0) * 16384 + 2048, "");
+      auto sums = [&](int t, int k) {
+        return reinterpret_cast<f32x4*>(t < N0 ? K0 : K1) + ((t < N0 ? t : t - N0) * 4 + k) * 256 + (tid & 255);
+      };
+      float2* const ml = reinterpret_cast<float2*>(reinterpret_cast<char*>(K1) + (DT - N0) * 16384) + (tid & 255);
+      meet<0>();
+      if (group == 1) {
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) *sums(t, k) = f32x4{o[t][4 * k], o[t][4 * k + 1], o[t][4 * k + 2], o[t][4 * k + 3]};
+        *ml = make_float2(m, l);
+      }
+      meet<0>();
+      if (group == 1) return;
+      const float2 other = *ml;
+      const float mn = fmaxf(m, other.x), ref = mn == -INFINITY ? 0.f : mn;
+      const float a0 = __builtin_amdgcn_exp2f(m - ref), a1 = __builtin_amdgcn_exp2f(other.x - ref);
+      l = l * a0 + other.y * a1;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const f32x4 x = *sums(t, k);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[t][4 * k + i] = o[t][4 * k + i] * a0 + x[i] * a1;
+        }
+    }
+  } else {
+    pages(0);
+    fetch();
+    pages(min(1, ntile - 1));
+    park(0);
+    __syncthreads();
+    for (int t = 0; t < ntile; ++t) {
+      const int buf = t & 1;
+      compute(t, Kb + buf * BN * KST, Vb + buf * BN * VST, nullptr, nullptr);
+      if (t + 1 < ntile) {
+        park(buf ^ 1);
+        __syncthreads();                     // the next tile is there; this one was read
+      }
     }
   }
   l += __shfl_xor(l, 32, 64);
@@ -454,14 +608,39 @@ bool run(T* out, const T* q, const T* kc, const T* vc, const int* qsl, const int
          int bt_stride, const int* work_seq, const int* work_blk, int n_work, int blk_rows, int H, int G,
          int krs, int vrs, int bs, int num_blocks, float scale, int window, int keep_first, const float* gate,
          const WindowExtra& ex, hipStream_t s) {
-  constexpr size_t lds = sizeof(T) * 2 * BN * (KS * 16 + 8 + (ALIAS ? 0 : DT * 32 + 8));
-  const auto kernel = &window_prefill_gqa_kernel<T, KS, DT, NB, ALIAS, CAP>;
-  static OncePerDevice once;
-  if (!allow_lds(once, kernel, lds)) return false;
-  kernel<<<dim3(H / HW, n_work * (blk_rows / BM)), NT, lds, s>>>(
-      out, q, kc, vc, qsl, seq_lens, pbt, bt_stride, work_seq, work_blk, blk_rows, H, G, krs, vrs, bs, 0xffffffffu / (uint32_t)bs,
-      num_blocks, scale, window, keep_first, gate, ex);
-  return true;
+  const int64_t wgs = (int64_t)(H / HW) * n_work * (blk_rows / 32);
+  int64_t span = (int64_t)bt_stride * bs;
+  if (window > 0) span = std::min<int64_t>(span, (int64_t)window + keep_first + 64);
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  // 16-byte units of rows of one page per DMA, keys and values at the same places
+  const bool dma = bs % (512 / (KS * 16)) == 0 && aligned(kc) && aligned(vc) && krs % 8 == 0 && krs == vrs && krs < 1 << 20 &&
+                   n_work <= 65535 / (blk_rows / 32);
+  auto go = [&](auto form) {
+    constexpr int F = decltype(form)::value;
+    const auto kernel = &window_prefill_gqa_kernel<T, KS, DT, NB, ALIAS, CAP, F>;
+    constexpr size_t lds = F != ROWS64 ? 0 : sizeof(T) * 2 * BN * (KS * 16 + 8 + (ALIAS ? 0 : DT * 32 + 8));
+    static OncePerDevice once;
+    if (lds > 0 && !allow_lds(once, kernel, lds)) return false;
+    kernel<<<dim3(H / HW, n_work * (blk_rows / (F == ROWS64 ? 64 : 32))), F == ROWS32 ? 256 : 512, lds, s>>>(
+        out, q, kc, vc, qsl, seq_lens, pbt, bt_stride, work_seq, work_blk, blk_rows, H, G, krs, vrs, bs, 0xffffffffu / (uint32_t)bs,
+        num_blocks, scale, window, keep_first, gate, ex);
+    return true;
+  };
+  // In bf16, ROWS64 -> here, us.  With no more workgroups of 32 rows than CUs two groups for each, but where the tables hold
+  // three tiles at most: 16 heads on 4, window 1024, 1 x 512 rows 26.6 -> 18.9, 1 x 2048 55.3 -> 38.0, 4 x 300 after 2000 57.8
+  // -> 37.3, 1 x 60 after 3000 57.5 -> 36.1, causal and capped 1 x 100 after 4000 229 -> 137, latent rows 2 x 1000 77.3 -> 49.1;
+  // 2 x 150 12.5 -> 13.1 (32 rows, one group: 12.4), latent 4 x 64 12.1 -> 13.1 (10.0).  Where 64 rows each leave at most half
+  // of the CUs a workgroup in the last round: 1 x 5000 100 -> 86.6, 6 x 1000 54.4 -> 49.2, 12 x 300 22.9 -> 20.5, 40 x 100 after
+  // 300 46.3 -> 44.3; where it is fuller, two workgroups to a CU are no faster than one of twice the rows: 32 x 512 81 -> 82, 20 x
+  // 300 after 1500 108 -> 112, 2 x 2000 in chunks of 1024 after 500 49 -> 64.  Contexts beyond 4096 leave the last round to
+  // the longest rows: capped 1 x 6000 after 1000 369 -> 402.  Latent rows beyond one round in any case: 4 x 2048 155 -> 142,
+  // 24 x 400 64 -> 61, 8 x 2048 260 -> 254, 60 x 200 70 -> 67 (within one: 1 x 4096 86 -> 89, 30 x 100 17.5 -> 18.8).
+  const int64_t n_cu = device_cus(), last = wgs / 2 % n_cu;
+  const bool spare = wgs / 2 > n_cu && (KS == 16 || (last > 0 && 2 * last <= n_cu && span <= 4096));
+  const int form = !dma ? ROWS64 : wgs <= n_cu ? span > 192 ? ROWS32X2 : ROWS32 : spare ? ROWS32 : ROWS64;
+  if (form == ROWS32X2) return go(std::integral_constant<int, ROWS32X2>());
+  if (form == ROWS32) return go(std::integral_constant<int, ROWS32>());
+  return go(std::integral_constant<int, ROWS64>());
 }
 
 template <typename T, bool CAP, typename... A>
@@ -484,7 +663,7 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
   // (one key/value head), 32 x 512 rows 380 -> 116 us; 8 x 64 rows 11.0 -> 10.2, latent 12.8 -> 12.4.  The maximum
   // is taken before the scale, which has to be positive for that.
   if (n_work <= 0 || !(scale > 0.f) || H / G % HW != 0 || ex.pool > 0 || ex.vtab != nullptr ||
-      blk_rows % BM != 0)
+      blk_rows % 64 != 0)
     return false;
   if ((int64_t)G * bs * std::max(krs, vrs) >= (int64_t)1 << 32) return false;   // pages are 32-bit factors of the offsets
   const bool alias = kc == vc && krs == vrs;

@@ -648,6 +648,58 @@ def test_window_attention_shared_tiles(gpu, dt, H, G, latent, bs, kw):
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("latent", [False, True])
+@pytest.mark.parametrize("n,bs,kw", [
+    (9, 4, dict(window=200, keep=70)), (9, 32, dict(window=0, keep=0, softcap=20.0)),      # every other tile each
+    (9, 6, dict(window=256, keep=0, chunked=True, sink=0.4)),
+    (4, 32, dict(window=60, keep=3)),                                                     # 32 rows, few tiles
+    (130, 2, dict(window=90, keep=66)), (130, 16, dict(window=0, keep=0))])               # 32 rows, two workgroups to a CU
+def test_window_attention_forms(gpu, dt, latent, n, bs, kw):
+    """Prompt rows where workgroups own 32 rows, two groups of waves share the tiles or one has them all: windows
+    that begin between the rows that are copied together, tiles of kept tokens, odd and even numbers of tiles,
+    one row to 70, tables that end inside a tile (what lay in LDS there before is not finite).  Calls that
+    only differ in pages of a row less have the same bits where no two groups share the tiles; the bound is
+    the shared tiles'."""
+    torch.manual_seed(41)
+    H, dk, dv = 4, *((256, 192) if latent else (128, 128))
+    P_q = [1 + (i * 23) % (70 if n < 100 else 7) for i in range(n)]
+    old = [(i * 61) % (600 if n == 9 else 130) for i in range(n)]
+    P_sl, T = [a + b for a, b in zip(P_q, old)], sum(P_q)
+    pos = torch.cat([torch.arange(o, o + a) for a, o in zip(P_q, old)])
+    q, kw = torch.randn(T, H, dk).to(dt), dict(kw)
+    args = (0.08, kw.pop("window"), kw.pop("keep"))
+    keys = [torch.randn(s, dk).to(dt) for s in P_sl]
+    vals = [k[:, :dv] if latent else torch.randn(k.shape[0], dv).to(dt) for k in keys]
+
+    def pack(bs, dev):
+        width = max(P_sl) // bs + 1
+        tables = torch.randperm(n * width).view(n, width)
+        kc = torch.zeros(n * width, 1, bs, dk, dtype=dt)
+        vc = torch.zeros(n * width, 1, bs, dv, dtype=dt)
+        for t, k, v in zip(tables, keys, vals):
+            j = torch.arange(k.shape[0])
+            kc[t[j // bs], 0, j % bs] = k
+            vc[t[j // bs], 0, j % bs] = v
+        kc = kc.to(dev)
+        return kc, kc[..., :dv] if latent else vc.to(dev), _to(_meta(P_q, P_sl, [], tables.int()), dev)
+
+    def run(bs, dev):
+        kc, vc, m = pack(bs, dev)
+        return ops.window_attention(q.to(dev), kc, vc, pos.to(dev), m, *args, None, **kw)
+
+    want = run(bs, "cpu")
+    kc, vc, m = pack(bs, gpu)
+    for c in (kc, vc):                       # every CU's LDS
+        c.fill_(float("nan"))
+    ops.window_attention(q.to(gpu), kc, vc, pos.to(gpu), m, *args, None, **kw)
+    got = run(bs, gpu)
+    ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
+    torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
+    if n != 9:
+        assert torch.equal(got, run(bs - 1, gpu))
+
+
 def _rounded_once(got, want, unit, eps):
     """got (16 bits) within half a unit in its last place of want (float64), and eps of ``unit`` for the arithmetic."""
     bits, low = (7, -126) if got.dtype == torch.bfloat16 else (10, -14)
