@@ -230,6 +230,25 @@ def test_paged_decode_rope(gpu, monkeypatch, kern, dt, d, nq, nkv, qk_norm, S, f
         torch.testing.assert_close(out.cpu().float(), exp.float(), **tol)
 
 
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("d,fp8", [(128, False), (128, True), (64, False)])
+def test_paged_decode_long_tables(gpu, dt, d, fp8):
+    """Tables that may hold more K and V than the last-level cache (their tail names one page; V is then read past the
+    caches): the bits of the same call with tables of the contexts' own width, in one slice and in three."""
+    torch.manual_seed(23)
+    nkv, bs, ctx = 8, 32, [1, 31, 32, 33, 64, 200, 500, 0] * 4
+    kc, vc, bt = _fill_random_cache(len(ctx), [max(c, 1) for c in ctx], nkv, bs, d, dt, gpu)
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    q, cl = torch.randn(len(ctx), 4 * nkv, d, dtype=dt, device=gpu), torch.tensor(ctx, dtype=torch.int32, device=gpu)
+    wide = torch.cat([bt, bt[:, :1].expand(-1, 300)], 1).contiguous()
+    per = len(ctx) * nkv * bs * 2 * d * kc.element_size()
+    assert per * bt.shape[1] < 128 << 20 < per * wide.shape[1]
+    for z in (1, 3):
+        want = ops.paged_attention_decode(q, kc, vc, bt, cl, d ** -0.5, grid_z=z)
+        assert torch.equal(ops.paged_attention_decode(q, kc, vc, wide, cl, d ** -0.5, grid_z=z), want)
+
+
 @pytest.mark.parametrize("B,nkv", [(64, 1), (72, 2), (64, 4), (64, 8), (5, 2), (3, 8)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_paged_decode_slices_of_ragged_contexts(gpu, monkeypatch, B, nkv, fp8):
