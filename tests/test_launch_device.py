@@ -315,3 +315,15 @@ int main() {
   return 0;
 }
 """)
+
+
+@pytest.mark.parametrize("E,N,K,rows,want", [
+    (8, 4096, 14336, 1, 8), (8, 4096, 14336, 6, 2),                   # few pairs: near one workgroup per CU, as ever
+    (8, 4096, 14336, 8, 4), (8, 4096, 14336, 256, 4), (8, 4096, 14336, 700, 2), (8, 4096, 14336, 2048, 1),
+    (16, 4096, 6400, 8, 1), (16, 4096, 6400, 512, 2),
+    (8, 4096, 3584, 256, 1), (32, 2048, 1408, 64, 1), (1, 256, 1 << 20, 64, 16)])
+def test_expert_down_projection_slices(E, N, K, rows, want):
+    """K-slices of the experts' down projection (top 2, column tiles of 256): up to two rounds of workgroups
+    where every expert has rows and a slice keeps 48 steps."""
+    S = ops.moe_dgemm_splitk(2 * rows, E, N, K, ops.moe_k14m_bm(2 * rows, E), 256)
+    assert S == want and 1 <= S <= 16 and K // 64 // S >= 8
