@@ -322,8 +322,10 @@ int main() {
     (8, 4096, 14336, 8, 4), (8, 4096, 14336, 256, 4), (8, 4096, 14336, 700, 2), (8, 4096, 14336, 2048, 1),
     (16, 4096, 6400, 8, 1), (16, 4096, 6400, 512, 2),
     (8, 4096, 3584, 256, 1), (32, 2048, 1408, 64, 1), (1, 256, 1 << 20, 64, 16)])
-def test_expert_down_projection_slices(E, N, K, rows, want):
+def test_expert_down_projection_slices(monkeypatch, E, N, K, rows, want):
     """K-slices of the experts' down projection (top 2, column tiles of 256): up to two rounds of workgroups
     where every expert has rows and a slice keeps 48 steps."""
+    from kubernetes_gpu_cluster_amd import ops
+    monkeypatch.delenv("KGC_MOE_SPLITK", raising=False)
     S = ops.moe_dgemm_splitk(2 * rows, E, N, K, ops.moe_k14m_bm(2 * rows, E), 256)
     assert S == want and 1 <= S <= 16 and K // 64 // S >= 8
