@@ -635,9 +635,14 @@ bool run(T* out, const T* q, const T* kc, const T* vc, const int* qsl, const int
   // 300 after 1500 108 -> 112, 2 x 2000 in chunks of 1024 after 500 49 -> 64.  Contexts beyond 4096 leave the last round to
   // the longest rows: capped 1 x 6000 after 1000 369 -> 402.  Latent rows beyond one round in any case: 4 x 2048 155 -> 142,
   // 24 x 400 64 -> 61, 8 x 2048 260 -> 254, 60 x 200 70 -> 67 (within one: 1 x 4096 86 -> 89, 30 x 100 17.5 -> 18.8).
+  // Without a window a prompt's rows have one tile to as many as its length, and the longest rows' chain lasts past the
+  // others: two groups up to two rounds (capped 1 x 3000 175 -> 113, 2 x 1500 92 -> 59, 2 x 2048 114 -> 88, 4 x 1000 67.5 -> 55; rows
+  // alike gain little, 2 x 2048 after 2000 225 -> 213, 8 x 500 after 2000 160 -> 160, or lose on shorter tables, 10 x 256 after
+  // 500 54 -> 56; windowed 1 x 3000 61 -> 65).
   const int64_t n_cu = device_cus(), last = wgs / 2 % n_cu;
+  const bool pairs = wgs <= n_cu ? span > 192 : wgs <= 2 * n_cu && window <= 0 && span >= 1000;
   const bool spare = wgs / 2 > n_cu && (KS == 16 || (last > 0 && 2 * last <= n_cu && span <= 4096));
-  const int form = !dma ? ROWS64 : wgs <= n_cu ? span > 192 ? ROWS32X2 : ROWS32 : spare ? ROWS32 : ROWS64;
+  const int form = !dma ? ROWS64 : pairs ? ROWS32X2 : wgs <= n_cu || spare ? ROWS32 : ROWS64;
   if (form == ROWS32X2) return go(std::integral_constant<int, ROWS32X2>());
   if (form == ROWS32) return go(std::integral_constant<int, ROWS32>());
   return go(std::integral_constant<int, ROWS64>());
