@@ -875,8 +875,10 @@ struct WalkArgs {
   int bt_stride, nq, nkv, bs_log2, num_blocks, cs_rows, n_items;
   float scale_log2, v_scale;
 };
-template <typename T, int D>
-__global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArgs) {
+// GR = 2: the tiles of one item per workgroup, every other one for each of two groups of 4 waves, whose sums meet at the
+// end (the rule: at the launch).
+template <typename T, int D, int GR>
+__global__ __launch_bounds__(256 * GR, 2) void prefill_attn_walk_kernel(const WalkArgs) {
   static_assert(D == 128 && PF_BN == 64 && sizeof(T) == 2, "rows and groups per DMA");
   typedef typename Vec8<T>::type V8;
   typedef __attribute__((address_space(3))) void* LdsPtr;
@@ -884,13 +886,15 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArg
   typedef const __attribute__((address_space(4))) int* ScalarPtr;
   constexpr int GH = 4, QB = 32, ZS = PF_BM / QB, KS = D / 32, DT = D / 16, RB = D * 2;   // RB: bytes of a row
   // (objects of their own: the compiler lets an LDS read follow every DMA into the object that it reads)
-  __shared__ __attribute__((aligned(16))) T K0[PF_BN * D], K1[PF_BN * D], V0[PF_BN * D], V1[PF_BN * D], all_rows[4 * 16 * D];
+  constexpr int TE = PF_BN * D;              // elements of a tile
+  __shared__ __attribute__((aligned(16))) T K0[GR * TE], K1[GR * TE], V0[GR * TE], V1[GR * TE], all_rows[4 * 16 * D];
   auto args = [] {                           // not kept: see above
     ArgPtr p = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(p));
     return p;
   };
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wave = GR == 2 ? wv & 3 : wv, group = GR == 2 ? wv >> 2 : 0;
   const int r16 = lane & 15, qd = lane >> 4;
   T* rows = all_rows + wave * 16 * D;        // where 16 output rows meet, to be stored 256 bytes at a time
   // (lane and wave behind an opaque move: what depends on them alone is not kept over the tile loop)
@@ -1009,7 +1013,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArg
   int it = next_valid(0, cur);
   if (it * G_ >= n_items) return;            // uniform: the whole workgroup leaves
   uint64_t at[2];                            // of the tile that computes next
-  int id = page_ids(cur.bt, cur.L, 0), page[2];       // pages of the one behind it
+  int id = page_ids(cur.bt, cur.L, group), page[2];       // pages of the one behind it
   auto pages = [&] {
 #pragma unroll
     for (int p = 0; p < 2; ++p) page[p] = __builtin_amdgcn_readlane(id, p);
@@ -1023,13 +1027,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArg
   ask_q(cur);
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    ask_k(cur.k, cur.L, 0, at, K0, u);
-    ask_v(cur.v, cur.L, 0, at, V0, u);
+    ask_k(cur.k, cur.L, group, at, K0 + group * TE, u);
+    ask_v(cur.v, cur.L, group, at, V0 + group * TE, u);
   }
   int nit = next_valid(it + 1, nxt);
   bool has_next = nit * G_ < n_items;
   if (!has_next) nxt = cur;
-  id = cur.n_tiles > 1 ? page_ids(cur.bt, cur.L, 1) : page_ids(nxt.bt, nxt.L, 0);
+  id = GR == 2 || cur.n_tiles > 1 ? page_ids(cur.bt, cur.L, group + GR) : page_ids(nxt.bt, nxt.L, 0);
   pages();
   take_q(cur);
   f32x4 o[2][DT];
@@ -1037,27 +1041,28 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArg
   auto fresh = [&] {
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
-      m[qt] = -INFINITY, l[qt] = 0.f;
+      m[qt] = group == 0 ? -INFINITY : -1e30f, l[qt] = 0.f;     // (the second group's rows may see none of its keys)
 #pragma unroll
       for (int t = 0; t < DT; ++t) o[qt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
   };
   fresh();
   const float c = args()->scale_log2;
-  int kt = 0;
+  int kt = group;
   // One tile, in K and V (or on its way there); the one behind it goes to Kn and Vn.  True after the last tile of the last item.
   auto tile = [&](const T* K, const T* V, T* Kn, T* Vn) -> bool {
-    const bool last = kt + 1 == cur.n_tiles;
+    const bool last = GR == 1 && kt + 1 == cur.n_tiles;
     // it is here (the output rows stored behind it need not be there), and everyone is done with the one before it
-    if (kt == 0) pf_meet<8>();
+    if (GR == 1 && kt == 0) pf_meet<8>();
     else pf_meet<0>();
+    if (GR == 1 || kt < cur.n_tiles) {
     places();
-    if (kt == 0) ask_q(nxt);
-    const bool own = kt + 2 < cur.n_tiles;
-    id = page_ids(own ? cur.bt : nxt.bt, own ? cur.L : nxt.L, own ? kt + 2 : last ? min(1, nxt.n_tiles - 1) : 0);
+    if (GR == 1 && kt == 0) ask_q(nxt);
+    const bool own = GR == 2 || kt + 2 < cur.n_tiles;
+    id = page_ids(own ? cur.bt : nxt.bt, own ? cur.L : nxt.L, own ? kt + 2 * GR : last ? min(1, nxt.n_tiles - 1) : 0);
     // (behind the last item its rows again)
     const char *nk = last ? nxt.k : cur.k, *nv = last ? nxt.v : cur.v;
-    const int nL = last ? nxt.L : cur.L, nkt = last ? 0 : kt + 1;
+    const int nL = last ? nxt.L : cur.L, nkt = last ? 0 : kt + GR;
     f32x4 s[2][4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1087,10 +1092,37 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArg
       if (t & 1) ask_v(nv, nL, nkt, at, Vn, t >> 1);
     }
     pages();                                 // (older than the tile's DMAs)
-    ++kt;
-    if (!last) return false;
+    }
+    kt += GR;
+    if (GR == 1 ? !last : kt - group < cur.n_tiles) return false;
+    if constexpr (GR == 2) {                 // the second group's sums join the first one's, by way of its own tiles
+      f32x4* const in[4] = {reinterpret_cast<f32x4*>(K0 + TE), reinterpret_cast<f32x4*>(K1 + TE), reinterpret_cast<f32x4*>(V0 + TE),
+                            reinterpret_cast<f32x4*>(V1 + TE)};
+      f32x4* const ml = reinterpret_cast<f32x4*>(rows) + lane;
+      const int to = wave * 64 + lane;
+      static_assert(DT == 8 && TE * sizeof(T) == 4 * 256 * sizeof(f32x4), "four sums of a lane per tile");
+      pf_meet<0>();
+      if (group == 1) {
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+          for (int t = 0; t < DT; ++t) in[2 * qt + (t >> 2)][(t & 3) * 256 + to] = o[qt][t];
+        *ml = f32x4{m[0], l[0], m[1], l[1]};
+      }
+      pf_meet<0>();
+      if (group == 1) return true;
+      const f32x4 other = *ml;
+#pragma unroll
+      for (int qt = 0; qt < 2; ++qt) {
+        const float mn = __builtin_elementwise_maximum(m[qt], other[2 * qt]);
+        const float a0 = __builtin_amdgcn_exp2f(m[qt] - mn), a1 = __builtin_amdgcn_exp2f(other[2 * qt] - mn);
+        l[qt] = l[qt] * a0 + other[2 * qt + 1] * a1;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[qt][t] = o[qt][t] * a0 + in[2 * qt + (t >> 2)][(t & 3) * 256 + to] * a1;
+      }
+    }
     // ---- the item's rows, and the next one's q
-    take_q(nxt);
+    if (GR == 1) take_q(nxt);
     const int ln = opaque(lane), r16 = ln & 15, qd = ln >> 4;
     const ArgPtr a = args();
     const int os = a->nq * RB;
@@ -1115,7 +1147,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArg
         __builtin_amdgcn_raw_buffer_store_b128(v, od, (qt * 16 + 4 * i + qd) * os + ((r16 ^ qd) * 16 ^ i * 64), 0, 2);
       }
     }
-    if (!has_next) return true;
+    if (GR == 2 || !has_next) return true;
     cur = nxt;
     it = nit;
     nit = next_valid(it + 1, nxt);
@@ -1129,7 +1161,12 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_walk_kernel(const WalkArg
     kt = 0;
     return false;
   };
-  while (!tile(K0, V0, K1, V1) && !tile(K1, V1, K0, V0)) {}
+  if constexpr (GR == 1) {
+    while (!tile(K0, V0, K1, V1) && !tile(K1, V1, K0, V0)) {}
+  } else {
+    T *const Ka = K0 + group * TE, *const Kb = K1 + group * TE, *const Va = V0 + group * TE, *const Vb = V1 + group * TE;
+    while (!tile(Ka, Va, Kb, Vb) && !tile(Kb, Vb, Ka, Va)) {}
+  }
   __builtin_amdgcn_s_waitcnt(0x0f70);        // DMAs end before the LDS is another's
 }
 
@@ -1148,7 +1185,7 @@ static int prefill_persist_mode() {
 template <typename T, int D, bool KV8, int GH>
 static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const void* vc,
                                  const int* bt, int bt_stride, const int* qsl, const int* sl,
-                                 const int* ws, const int* wm, int n_work, int nq, int nkv,
+                                 const int* ws, const int* wm, int n_work, int n_seq, int nq, int nkv,
                                  int bs_log2, float scale_log2, float v_scale, int num_blocks,
                                  int64_t q_stride, const float* cos_sin, int cs_rows, hipStream_t s) {
   constexpr size_t lds = 2 * 2 * PF_BN * D * sizeof(T);
@@ -1169,7 +1206,12 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
         ((int64_t)nkv * D << bs_log2) < ((int64_t)1 << 31)) {       // offsets inside an item and a page in 32 bits
       const WalkArgs a{q, kc, vc, out, cos_sin, bt, qsl, sl, ws, wm, q_stride, bt_stride, nq, nkv, bs_log2, num_blocks,
                        cs_rows, (int)n, scale_log2, v_scale};
-      prefill_attn_walk_kernel<T, D><<<(int)std::min<int64_t>(n, 2 * n_cu), 256, 0, s>>>(a);
+      // Two groups of waves per item where there is at most one item per CU, or one prompt's are two: its last rows' chain of
+      // tiles outlasts the others.  us, one group -> two: 512 rows 27.8 -> 24.8, 1000 39.2 -> 33.0, 300 after 3000 85 -> 62, 4 x 200
+      // after 1000 43.4 -> 36.9, 1500 52.6 -> 44.0, 2000 65.0 -> 58.3, 2000 after 2000 125 -> 116; other prompts beyond one item per CU 6 x 256
+      // 28.3 -> 33.9, 4 x 500 after 1000 64.7 -> 65.8, 12 x 100 after 1000 56 -> 60; 16 x 128 28.9 -> 34.7, 4096 160 -> 170.
+      if (mode < 0 && n <= (n_seq == 1 ? 2 : 1) * n_cu) prefill_attn_walk_kernel<T, D, 2><<<(int)n, 512, 0, s>>>(a);
+      else prefill_attn_walk_kernel<T, D, 1><<<(int)std::min<int64_t>(n, 2 * n_cu), 256, 0, s>>>(a);
       return;
     }
   }
@@ -1192,17 +1234,17 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
 template <typename T, int D, bool KV8>
 static void prefill_dispatch(const void* q, void* out, const void* kc, const void* vc,
                              const int* bt, int bt_stride, const int* qsl, const int* sl,
-                             const int* ws, const int* wm, int n_work, int nq, int nkv,
+                             const int* ws, const int* wm, int n_work, int n_seq, int nq, int nkv,
                              int bs_log2, float scale_log2, float v_scale, int num_blocks,
                              int64_t q_stride, const float* cos_sin, int cs_rows, hipStream_t s) {
   const int G = nkv > 0 ? nq / nkv : 1;
   if constexpr (D == 128) if (prefill_gqa_enabled() && nq % nkv == 0 && (G == 4 || G % 8 == 0)) {
     if (G == 4)
-      prefill_gqa_dispatch<T, D, KV8, 4>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work,
+      prefill_gqa_dispatch<T, D, KV8, 4>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, n_seq,
                                          nq, nkv, bs_log2, scale_log2, v_scale, num_blocks,
                                          q_stride, cos_sin, cs_rows, s);
     else
-      prefill_gqa_dispatch<T, D, KV8, 8>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work,
+      prefill_gqa_dispatch<T, D, KV8, 8>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, n_seq,
                                          nq, nkv, bs_log2, scale_log2, v_scale, num_blocks,
                                          q_stride, cos_sin, cs_rows, s);
     return;
@@ -1216,7 +1258,7 @@ static void prefill_dispatch(const void* q, void* out, const void* kc, const voi
 void launch_prefill_attention(int dtype, const void* q, void* out, const void* k_cache,
                               const void* v_cache, const int* block_tables, int bt_stride,
                               const int* query_start_loc, const int* seq_lens,
-                              const int* work_seq, const int* work_mblk, int n_work, int nq,
+                              const int* work_seq, const int* work_mblk, int n_work, int n_seq, int nq,
                               int nkv, int D, int bs_log2, float scale, bool kv_fp8,
                               float k_scale, float v_scale, int num_blocks, int64_t q_stride,
                               const float* cos_sin, int cs_rows, hipStream_t s) {
@@ -1224,8 +1266,8 @@ void launch_prefill_attention(int dtype, const void* q, void* out, const void* k
   const float sl2 = scale * k_scale * 1.4426950408889634f;
 #define KGC_PF(TT, DD, K8)                                                                 \
   prefill_dispatch<TT, DD, K8>(q, out, k_cache, v_cache, block_tables, bt_stride,          \
-                               query_start_loc, seq_lens, work_seq, work_mblk, n_work, nq, \
-                               nkv, bs_log2, sl2, v_scale, num_blocks, q_stride, cos_sin, cs_rows, s)
+                               query_start_loc, seq_lens, work_seq, work_mblk, n_work, n_seq, \
+                               nq, nkv, bs_log2, sl2, v_scale, num_blocks, q_stride, cos_sin, cs_rows, s)
 #define KGC_PF_D(TT, K8) \
   if (D == 128) KGC_PF(TT, 128, K8); else KGC_PF(TT, 64, K8)
   if (dtype == DT_BF16) {

@@ -62,7 +62,7 @@ void launch_paged_decode_rope(int dtype, const DecodeRope& rp, void* out, void* 
 void launch_prefill_attention(int dtype, const void* q, void* out, const void* k_cache,
                               const void* v_cache, const int* block_tables, int bt_stride,
                               const int* query_start_loc, const int* seq_lens,
-                              const int* work_seq, const int* work_mblk, int n_work, int nq,
+                              const int* work_seq, const int* work_mblk, int n_work, int n_seq, int nq,
                               int nkv, int D, int bs_log2, float scale, bool kv_fp8,
                               float k_scale, float v_scale, int num_blocks, int64_t q_stride,
                               const float* cos_sin, int cs_rows, hipStream_t s);

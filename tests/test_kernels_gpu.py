@@ -1730,6 +1730,30 @@ def test_prompt_gemm_routes(gpu):
 
 
 @pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("nq,nkv,bs", [(32, 8, 32), (8, 1, 64)])
+@pytest.mark.parametrize("query_lens,seq_lens", [
+    ([129], [129]), ([1], [200]), ([64, 65], [64, 65]), ([33, 100, 1, 32], [161, 1000, 65, 800]), ([1100], [1100]), ([3000], [3000])])
+def test_prefill_walk_two_groups(gpu, monkeypatch, dt, nq, nkv, bs, query_lens, seq_lens):
+    """Few items, or one prompt's: two groups of waves take every other tile (the second none, one masked for some rows,
+    as many, one less).  Against one group: a weight's rounding is half a unit, 2^-9 (f16 2^-12) of it, on both sides, so
+    results differ by twice that of the weighted mean of |v|, by no more than max |v|, and by their own rounding."""
+    torch.manual_seed(37 + nq)
+    monkeypatch.delenv("KGC_PREFILL_PERSIST", raising=False)
+    d = 128
+    kc, vc, bt = _fill_random_cache(len(seq_lens), seq_lens, nkv, bs, d, dt, gpu)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)   # noqa: E731
+    qsl, sl = i32([0] + query_lens).cumsum(0).int(), i32(seq_lens)
+    ws, wm = map(i32, ops.prefill_work_list(query_lens, seq_lens))
+    q = torch.randn(sum(query_lens), nq, d, dtype=dt, device=gpu)
+    run = lambda: ops.prefill_attention(q, kc, vc, bt, qsl, sl, d ** -0.5, ws, wm)   # noqa: E731
+    two, again = run(), run()
+    monkeypatch.setenv("KGC_PREFILL_PERSIST", "1")
+    one, unit = run(), 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    assert torch.equal(two, again)
+    torch.testing.assert_close(two.float(), one.float(), atol=unit * float(vc.abs().max()), rtol=2 * unit)
+
+
+@pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("nq,nkv,bs", [(32, 8, 32), (8, 1, 64), (12, 3, 128)])
 @pytest.mark.parametrize("rope", [False, True])
 @pytest.mark.parametrize("shape", ["short_many", "mixed_chunked", "one_item"])
