@@ -22,6 +22,7 @@
 // Few long sequences are cut into segments: a chunk walk is linear in its state, so a first pass
 // walks every segment from zero (with its values) and from the identity (without), a second chains
 // S <- M_j S + dS_j over the segments, and the third walks all segments from their own states.
+#include <algorithm>
 #include <type_traits>
 #include "chunk.h"
 #include "chunk_rows.h"
@@ -679,9 +680,16 @@ __global__ __launch_bounds__(NT) void delta_walk_kernel(const DeltaArgs a) {
   }
 }
 
-// ---- S_in of every segment: S <- M_j S + dS_j, a wave per 16 columns of one (sequence, head) ----
-__global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
-  const int lane = threadIdx.x, lr = lane & 15, lg = lane >> 4;
+// ---- S_in of every segment: S <- M_j S + dS_j.  A workgroup owns 16 columns of one (sequence, head), each of its 8 waves 16
+// rows: the parts of S pass through LDS, the next segment's rows of M are on their way meanwhile.  (One wave for the 16
+// columns, M read when it is needed, bound by that chain: 24 us a segment; 1 x 2000 tokens of 16 heads 267 -> 107 us, 1 x 8192
+// 616 -> 300.)
+__global__ __launch_bounds__(NT) void delta_chain_kernel(const DeltaArgs a) {
+  static_assert(NW == DT, "a wave per 16 rows");
+  typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
+  __shared__ __align__(16) uint32_t sx[2][KD][3][64][4];
+  const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int seq = blockIdx.x, h = blockIdx.y, col = blockIdx.z * 16 + lr;
   const bool colok = col < a.dv;
   const int colc = colok ? col : a.dv - 1;
@@ -690,45 +698,54 @@ __global__ __launch_bounds__(64) void delta_chain_kernel(const DeltaArgs a) {
   const int first = pieces_before(seq, a.qsl, a.seg);
   const int count = (len + a.seg - 1) / a.seg, w = a.dv + D;
   const float* Ss = a.S + ((int64_t)slot * a.H + h) * D * a.dv;
-  f32x4 S[DT];
+  f32x4 S;
 #pragma unroll
-  for (int i = 0; i < DT; ++i)
+  for (int e = 0; e < 4; ++e) S[e] = pos0 == 0 ? 0.f : Ss[(wave * 16 + 4 * lg + e) * a.dv + colc];
+  F4 m[KD][2];                               // row wave * 16 + lr of M, columns in the permuted order
+  f32x4 d;
+  auto fetch = [&](int j) {
+    const float* st = a.seg_state + ((int64_t)(first + j) * a.H + h) * D * w;
+    const float* row = st + (wave * 16 + lr) * w + a.dv + lg * 4;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) S[i][e] = pos0 == 0 ? 0.f : Ss[(i * 16 + 4 * lg + e) * a.dv + colc];
-  for (int j = 0; j < count; ++j) {
-    const int64_t ih = (int64_t)(first + j) * a.H + h;
-    float* dst = a.seg_in + ih * D * a.dv;
+    for (int k = 0; k < KD; ++k)
 #pragma unroll
-    for (int i = 0; i < DT; ++i)
+      for (int i = 0; i < 2; ++i) m[k][i] = *reinterpret_cast<const F4*>(row + k * 32 + i * 16);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (colok) dst[(i * 16 + 4 * lg + e) * a.dv + col] = S[i][e];
+    for (int e = 0; e < 4; ++e) d[e] = st[(wave * 16 + 4 * lg + e) * w + colc];
+  };
+  if (count > 1) fetch(0);
+  for (int j = 0;; ++j) {
+    float* dst = a.seg_in + ((int64_t)(first + j) * a.H + h) * D * a.dv;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (colok) dst[(wave * 16 + 4 * lg + e) * a.dv + col] = S[e];
     if (j + 1 == count) break;
-    const float* st = a.seg_state + ih * D * w;
-    bf16x8 sp[KD][3];
+    uint32_t p0[3], p1[3];
+    split2<3>(S[0], S[1], p0);
+    split2<3>(S[2], S[3], p1);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(&sx[j & 1][wave >> 1][p][lane][2 * (wave & 1)]) = u32x2{p0[p], p1[p]};
+    bf16x8 fa[KD][3];
 #pragma unroll
     for (int k = 0; k < KD; ++k) {
       float x[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = S[2 * k + (i >> 2)][i & 3];
-      split8<3>(x, sp[k]);
+      for (int i = 0; i < 8; ++i) x[i] = m[k][i >> 2][i & 3];
+      split8<3>(x, fa[k]);
+    }
+    const f32x4 dc = d;
+    if (j + 2 < count) fetch(j + 1);
+    meet<63>();                              // (the parts are there; loads and stores stay on their way)
+    f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
+#pragma unroll
+    for (int k = 0; k < KD; ++k) {
+      bf16x8 sp[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) sp[p] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&sx[j & 1][k][p][lane][0]));
+      mm<true, 3, 3>(fa[k], sp, hi, lo);
     }
 #pragma unroll
-    for (int i = 0; i < DT; ++i) {
-      f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = hi;
-#pragma unroll
-      for (int k = 0; k < KD; ++k) {         // row i * 16 + lr of M, columns in the permuted order
-        const float* m = st + (i * 16 + lr) * w + a.dv + k * 32 + lg * 4;
-        float x[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = m[(e >> 2) * 16 + (e & 3)];
-        bf16x8 fa[3];
-        split8<3>(x, fa);
-        mm<true, 3, 3>(fa, sp[k], hi, lo);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) S[i][e] = hi[e] + lo[e] + st[(i * 16 + 4 * lg + e) * w + colc];
-    }
+    for (int e = 0; e < 4; ++e) S[e] = hi[e] + lo[e] + dc[e];
   }
 }
 
@@ -759,7 +776,13 @@ DeltaWork delta_chunk_plan(int P, int Tp, int H, int G, int V) {
   w.floats = (int64_t)chunks * L * (3 * H + 2 * G);
   const int want = (device_cus() + wgs - 1) / wgs;      // items for one workgroup per CU
   if (P * 3 > want) return w;
-  const int seg = segment_rows(P, Tp, want, L, 8);    // one round
+  // One round of the third pass, whose segments have 8 chunks at least; where that leaves more than a round of the first
+  // one (the identity's workgroups beside the values'), shorter ones that fill it.  us, 8 chunks -> so, 16 heads: 1 x 400 tokens
+  // 76 (whole) -> 62, 500 90 (whole) -> 66, 700 117 (whole) -> 72, 1000 106 -> 86, 2 x 500 91 (whole) -> 78; 1 x 2000 in 13 segments instead
+  // of 8 114 -> 126.
+  int seg = segment_rows(P, Tp, want, L, 8);
+  const int first = device_cus() / (wgs + H);
+  if (first > 0) seg = std::min(seg, segment_rows(P, Tp, first + P, L, 3));
   if (Tp / P < 3 * seg) return w;
   w.seg = seg;
   w.items = Tp / seg + P;
@@ -792,7 +815,7 @@ void launch_delta_chunk(int dtype, float* out, const float* qkv, const void* ba,
     delta_walk_kernel<0><<<dim3(P, H * nct), NT, 0, s>>>(a);
   } else {
     delta_walk_kernel<1><<<dim3(work.items, H * (nct + 1)), NT, 0, s>>>(a);
-    delta_chain_kernel<<<dim3(P, H, (V + 15) / 16), 64, 0, s>>>(a);
+    delta_chain_kernel<<<dim3(P, H, (V + 15) / 16), NT, 0, s>>>(a);
     delta_walk_kernel<2><<<dim3(work.items, H * nct), NT, 0, s>>>(a);
   }
 }

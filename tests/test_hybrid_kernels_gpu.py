@@ -547,6 +547,14 @@ def test_gated_delta_scan_chunkwise(gpu, dt, H, G, V, lens, before, D_ctx):
     assert _whole(got, want) and _whole(S_g, S_w)
 
 
+@pytest.mark.parametrize("H,G,V,lens,before", [
+    (16, 8, 128, [400], [0]), (2, 1, 130, [289, 520], [0, 31]), (8, 8, 22, [96 * 4], [5]), (4, 2, 128, [1, 700], [0, 0])])
+def test_gated_delta_scan_short_segments(gpu, H, G, V, lens, before):
+    """Few sequences in segments of three chunks: one that ends with a segment, one that is shorter than a segment,
+    columns that are no multiple of 4, 16 or 128, states that enter."""
+    test_gated_delta_scan_chunkwise(gpu, torch.bfloat16, H, G, V, lens, before, [])
+
+
 @pytest.mark.parametrize("path", ["fast", "simple"])
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,G,dk,dv,window,keep", [(4, 2, 96, 64, 70, 5), (4, 1, 128, 128, 150, 3),
