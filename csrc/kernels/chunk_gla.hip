@@ -642,29 +642,51 @@ __global__ __launch_bounds__(NT) void gla_walk_kernel(const GlaArgs a) {
       for (int r = 0; r < 4; ++r) dst[(i * 16 + 4 * lg + r) * a.dv + col] = S[i][r];
 }
 
-// ---- the states in which segments start, in place of the contributions: one element per thread ------------
+// ---- the states in which segments start, in place of the contributions: W elements of a row per thread (4 where rows
+// are multiples of it).  What bounds it is memory's latency, so four segments' loads go out before the first of
+// them is stored, and a row's decays are read by fewer threads.  Calls of 8 heads of 128 x 256, us: 1 x 1000 tokens 53.2 -> 49.0,
+// 1 x 2000 70.6 -> 60.5, 4 x 600 71.0 -> 64.2, 1 x 8192 153.5 -> 145.5.
+template <int W>
 __global__ __launch_bounds__(256) void gla_chain_kernel(const GlaArgs a) {
+  typedef float FW __attribute__((ext_vector_type(W)));
   const int seq = blockIdx.z, h = blockIdx.y, lane = threadIdx.x & 63;
   const int len = a.qsl[seq + 1] - a.qsl[seq], pos0 = a.seq_lens[seq] - len, slot = a.slots[seq];
   if (len <= a.seg || slot < 0 || slot >= a.num_slots || pos0 < 0) return;
   const int first = pieces_before(seq, a.qsl, a.seg);
   const int count = (len + a.seg - 1) / a.seg, per = a.seg / L, sh = D * a.dv;
   const int chunk0 = chunks_before<L>(seq, a.qsl);
-  const int at = blockIdx.x * 256 + threadIdx.x;
+  const int at = (blockIdx.x * 256 + threadIdx.x) * W;
   if (at >= sh) return;
   const int64_t step = (int64_t)a.H * sh;
   const float* pl = a.pl + ((int64_t)chunk0 * a.H + h) * D + at / a.dv;
   float* p = a.seg_state + ((int64_t)first * a.H + h) * sh + at;
-  float S = pos0 == 0 ? 0.f : a.S[((int64_t)slot * a.H + h) * sh + at];
-  for (int j = 0; j < count - 1; ++j) {
-    const float c = p[j * step];
-    double f = 1.0;                          // the segment's decay
-#pragma unroll 8
-    for (int k = 0; k < per; ++k) f *= pl[(int64_t)(j * per + k) * a.H * D];
-    p[j * step] = S;
-    S = __builtin_fmaf((float)f, S, c);
+  FW S = {};
+  if (pos0 != 0) S = *reinterpret_cast<const FW*>(a.S + ((int64_t)slot * a.H + h) * sh + at);
+  constexpr int U = 4;
+  for (int j0 = 0; j0 < count - 1; j0 += U) {
+    FW c[U];
+    double f[U];                             // the segments' decays
+    const float* g[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = min(j0 + u, count - 2);
+      c[u] = *reinterpret_cast<const FW*>(p + j * step);
+      g[u] = pl + (int64_t)j * per * a.H * D;
+      f[u] = 1.0;
+    }
+#pragma unroll 4
+    for (int k = 0; k < per; ++k)
+#pragma unroll
+      for (int u = 0; u < U; ++u) f[u] *= g[u][(int64_t)k * a.H * D];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (j0 + u >= count - 1) break;
+      *reinterpret_cast<FW*>(p + (j0 + u) * step) = S;
+#pragma unroll
+      for (int r = 0; r < W; ++r) S[r] = __builtin_fmaf((float)f[u], S[r], c[u][r]);
+    }
   }
-  p[(count - 1) * step] = S;
+  *reinterpret_cast<FW*>(p + (count - 1) * step) = S;
 }
 
 template <typename T>
@@ -681,7 +703,10 @@ void run(const GlaArgs& a, int chunks, hipStream_t s) {
     gla_walk_kernel<T, 0><<<dim3(a.P, y), NT, 0, s>>>(a);
   } else {
     gla_walk_kernel<T, 1><<<dim3(a.items, y), NT, 0, s>>>(a);
-    gla_chain_kernel<<<dim3((D * a.dv + 255) / 256, a.H, a.P), 256, 0, s>>>(a);
+    if (a.dv % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.S) | reinterpret_cast<uintptr_t>(a.seg_state)) & 15) == 0)
+      gla_chain_kernel<4><<<dim3((D * a.dv / 4 + 255) / 256, a.H, a.P), 256, 0, s>>>(a);
+    else
+      gla_chain_kernel<1><<<dim3((D * a.dv + 255) / 256, a.H, a.P), 256, 0, s>>>(a);
     gla_walk_kernel<T, 2><<<dim3(a.items, y), NT, 0, s>>>(a);
   }
 }

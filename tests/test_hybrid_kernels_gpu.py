@@ -1156,6 +1156,14 @@ def test_gla_scan_chunkwise(gpu, dt, H, V, R, lens, before, D_ctx):
             assert _whole(got, want) and _whole(st, S)
 
 
+@pytest.mark.parametrize("V", [30, 32])
+@pytest.mark.parametrize("lens,before", [([2100], [7]), ([700, 330], [0, 40])])
+def test_gla_scan_segments_of_odd_rows(gpu, V, lens, before):
+    """Few sequences in segments, more and fewer than four of them: state rows of a multiple of 4 elements, which the
+    chain over the segments takes at a time, and of none."""
+    test_gla_scan_chunkwise(gpu, torch.bfloat16, 2, V, 5, lens, before, [])
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("R", [4, 20, 128])
 def test_gla_rows_off_their_alignment(gpu, dt, R):
