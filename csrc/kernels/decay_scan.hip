@@ -198,7 +198,7 @@ __global__ __launch_bounds__(NT) void gla_scan_kernel(
 // flight while the decays are computed (the scan above reads 64 bytes of a row).  V a multiple of 4.
 // Bound by the state's bytes: 64 rows of 8 heads [128, 256], 134 MB, 42 us by the scan, 25 here (5.4 TB/s; a
 // large copy reaches 4.8); 8 rows 11.5 -> 10.
-template <typename T, int RI>
+template <typename T, int RI, bool ONCE>
 __global__ __launch_bounds__(NT) void gla_decode_kernel(
     float* __restrict__ out, const T* __restrict__ proj, int64_t ps, const T* __restrict__ low,
     int64_t ls, const float* __restrict__ a2, const float* __restrict__ a2b, float* __restrict__ S,
@@ -223,7 +223,10 @@ __global__ __launch_bounds__(NT) void gla_decode_kernel(
   for (int i = 0; i < RI; ++i) {
     const int r = rg + 16 * i;
     Sr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (pos != 0 && r < d && colok) Sr[i] = *reinterpret_cast<const float4*>(Sp + (int64_t)r * V);
+    if (pos != 0 && r < d && colok) {
+      const f32x4* at = reinterpret_cast<const f32x4*>(Sp + (int64_t)r * V);
+      Sr[i] = __builtin_bit_cast(float4, ONCE ? __builtin_nontemporal_load(at) : *at);
+    }
   }
   const T* row = proj + t * ps;
   float v[4];
@@ -254,7 +257,11 @@ __global__ __launch_bounds__(NT) void gla_decode_kernel(
     const float kv = kqa[0][r], qv = kqa[1][r], av = kqa[2][r];
     Sr[i] = make_float4(av * Sr[i].x + kv * v[0], av * Sr[i].y + kv * v[1], av * Sr[i].z + kv * v[2],
                         av * Sr[i].w + kv * v[3]);
-    if (r < d && colok) *reinterpret_cast<float4*>(Sp + (int64_t)r * V) = Sr[i];
+    if (r < d && colok) {
+      f32x4* at = reinterpret_cast<f32x4*>(Sp + (int64_t)r * V);
+      if (ONCE) __builtin_nontemporal_store(__builtin_bit_cast(f32x4, Sr[i]), at);
+      else *at = __builtin_bit_cast(f32x4, Sr[i]);
+    }
     y[0] += Sr[i].x * qv;
     y[1] += Sr[i].y * qv;
     y[2] += Sr[i].z * qv;
@@ -413,14 +420,24 @@ void launch_gla_scan(int dtype, float* out, const void* proj, int64_t ps, const 
   if (P == 0 && V % 4 == 0 && reinterpret_cast<uintptr_t>(S) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(out) % 16 == 0) {
     const dim3 grid(D, H, (V + 63) / 64);
-#define KGC_GLA_D(RI)                                                                        \
-  KGC_DS_DISPATCH_T(dtype, gla_decode_kernel<T, RI><<<grid, NT, 0, s>>>(                     \
+    // States of 128 MB and more are read and written past the caches (whole lines, once a step; the last-level cache has 256
+    // MB): 128 rows of 8 heads of 128 x 256 64.3 -> 53.4 us, 256 119 -> 107.  Smaller ones may still lie there from the
+    // step before: 64 rows on three sets of states in turn 25.8 -> 28.2 (on twelve, from memory, 35.1 -> 28.4).
+    const bool once = (int64_t)D * H * d * V * (int64_t)sizeof(float) >= (int64_t)128 << 20;
+#define KGC_GLA_ROWS(RI, ONCE)                                                               \
+  KGC_DS_DISPATCH_T(dtype, gla_decode_kernel<T, RI, ONCE><<<grid, NT, 0, s>>>(               \
       out, (const T*)proj, ps, (const T*)low, ls, a2, a2b, S, ctx_lens, slots, Tp, H, d, V,  \
       R, 1.f / tau, num_slots))
+#define KGC_GLA_D(RI)                                                                        \
+  do {                                                                                       \
+    if (once) KGC_GLA_ROWS(RI, true);                                                        \
+    else KGC_GLA_ROWS(RI, false);                                                            \
+  } while (0)
     if (d <= 64) KGC_GLA_D(4);
     else if (d <= 128) KGC_GLA_D(8);
     else KGC_GLA_D(16);
 #undef KGC_GLA_D
+#undef KGC_GLA_ROWS
     return;
   }
   bool narrow = scan_narrow(P + D, H, V);

@@ -223,7 +223,7 @@ __global__ __launch_bounds__(NT) void causal_conv_kernel(
 // ---- Mamba-2 recurrence ---------------------------------------------------------------------
 // xbc fp32 [T, H V + 2 G N] = x | B | C; dt [T, H] (row stride dts) raw step sizes.
 // RPT: rows of S per lane (N <= row groups * RPT); LOGC: log2 of the columns per wave.
-template <typename T, int RPT, int LOGC>
+template <typename T, int RPT, int LOGC, bool ONCE>
 __global__ __launch_bounds__(NT) void ssd_scan_kernel(
     float* __restrict__ out, const float* __restrict__ xbc, const T* __restrict__ dt,
     int64_t dts, const float* __restrict__ a_log, const float* __restrict__ dt_bias,
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(NT) void ssd_scan_kernel(
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int r = NRG * i + rg;
-    Sr[i] = (!fresh && r < N && colok) ? Sp[(int64_t)r * V + col] : 0.f;
+    Sr[i] = (!fresh && r < N && colok) ? ONCE ? __builtin_nontemporal_load(Sp + (int64_t)r * V + col) : Sp[(int64_t)r * V + col] : 0.f;
   }
   const float A = expf(a_log[h]), dtb = dt_bias[h], Dh = dskip[h];
   for (int t0 = 0; t0 < q.len; t0 += TB) {
@@ -316,7 +316,10 @@ __global__ __launch_bounds__(NT) void ssd_scan_kernel(
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int r = NRG * i + rg;
-    if (r < N && colok) Sp[(int64_t)r * V + col] = Sr[i];
+    if (r < N && colok) {
+      if (ONCE) __builtin_nontemporal_store(Sr[i], Sp + (int64_t)r * V + col);
+      else Sp[(int64_t)r * V + col] = Sr[i];
+    }
   }
 }
 
@@ -325,7 +328,7 @@ __global__ __launch_bounds__(NT) void ssd_scan_kernel(
 // pre-activations.  With the token's S_0 = the state before it:
 //   S^T k = g S_0^T k,  o = S_new^T q = g S_0^T q + (k . q) u,  S_new = g S_0 + k u^T
 // so both sums over rows are taken over S_0 in one pass.
-template <typename T, int RPT, int LOGC>
+template <typename T, int RPT, int LOGC, bool ONCE>
 __global__ __launch_bounds__(NT) void gated_delta_scan_kernel(
     float* __restrict__ out, const float* __restrict__ qkv, const T* __restrict__ ba,
     int64_t bas, const float* __restrict__ a_log, const float* __restrict__ dt_bias,
@@ -359,7 +362,7 @@ __global__ __launch_bounds__(NT) void gated_delta_scan_kernel(
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int r = NRG * i + rg;
-    Sr[i] = (!fresh && r < d && colok) ? Sp[(int64_t)r * V + col] : 0.f;
+    Sr[i] = (!fresh && r < d && colok) ? ONCE ? __builtin_nontemporal_load(Sp + (int64_t)r * V + col) : Sp[(int64_t)r * V + col] : 0.f;
   }
   const float A = expf(a_log[h]), dtb = dt_bias[h], qscale = 1.f / sqrtf((float)d);
   for (int t0 = 0; t0 < q.len; t0 += TB) {
@@ -435,7 +438,10 @@ __global__ __launch_bounds__(NT) void gated_delta_scan_kernel(
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int r = NRG * i + rg;
-    if (r < d && colok) Sp[(int64_t)r * V + col] = Sr[i];
+    if (r < d && colok) {
+      if (ONCE) __builtin_nontemporal_store(Sr[i], Sp + (int64_t)r * V + col);
+      else Sp[(int64_t)r * V + col] = Sr[i];
+    }
   }
 }
 
@@ -547,6 +553,14 @@ static int pow2_at_least(int n, int lo) {
   return p;
 }
 
+// States of 128 MB and more are read and written past the caches where a workgroup takes whole lines (64 columns): once
+// a step, and the last-level cache has 256 MB.  Decode rows, us: 32 heads of 128 x 64, 128 rows 63.3 -> 57.2, 256 113.4 -> 110.4;
+// the delta rule's 16 of 128 x 128, 128 rows 70.9 -> 62.1, 256 127.0 -> 119.6.  (64 rows of either may still lie there from the
+// step before; of the GLA's, which lose by it: decay_scan.hip.)
+static bool states_once(int seqs, int H, int d, int V) {
+  return (int64_t)seqs * H * d * V * (int64_t)sizeof(float) >= (int64_t)128 << 20;
+}
+
 void launch_ssd_scan(int dtype, float* out, const float* xbc, const void* dt, int64_t dts,
                      const float* a_log, const float* dt_bias, const float* dskip, float* S,
                      const int* qsl, const int* seq_lens, const int* ctx_lens, const int* slots,
@@ -556,22 +570,29 @@ void launch_ssd_scan(int dtype, float* out, const float* xbc, const void* dt, in
   const bool narrow = scan_narrow(P + D, H, V);
   const int ct = narrow ? 16 : 64, rp = pow2_at_least(N, narrow ? 64 : 16);
   const dim3 grid(P + D, H, (V + ct - 1) / ct);
-#define KGC_SSD_W(R, L)                                                                      \
-  KGC_PM_DISPATCH_T(dtype, ssd_scan_kernel<T, R, L><<<grid, NT, scan_lds(rp, ct, 2), s>>>(   \
+  const bool once = states_once(P + D, H, N, V);
+#define KGC_SSD_W(R, L, ONCE)                                                                      \
+  KGC_PM_DISPATCH_T(dtype, ssd_scan_kernel<T, R, L, ONCE><<<grid, NT, scan_lds(rp, ct, 2), s>>>(   \
       out, xbc, (const T*)dt, dts, a_log, dt_bias, dskip, S, qsl, seq_lens, ctx_lens, slots, P, \
       Tp, H, V, N, G, num_slots))
+#define KGC_SSD_W_WIDE(R)                                                                     \
+  do {                                                                                       \
+    if (once) KGC_SSD_W(R, 4, true);                                                          \
+    else KGC_SSD_W(R, 4, false);                                                              \
+  } while (0)
   // rows per lane = padded rows / row groups (4 wide, 16 narrow); at least 4
   if (!narrow) {
-    if (rp <= 16) KGC_SSD_W(4, 4);
-    else if (rp == 32) KGC_SSD_W(8, 4);
-    else if (rp == 64) KGC_SSD_W(16, 4);
-    else if (rp == 128) KGC_SSD_W(32, 4);
-    else KGC_SSD_W(64, 4);
+    if (rp <= 16) KGC_SSD_W_WIDE(4);
+    else if (rp == 32) KGC_SSD_W_WIDE(8);
+    else if (rp == 64) KGC_SSD_W_WIDE(16);
+    else if (rp == 128) KGC_SSD_W_WIDE(32);
+    else KGC_SSD_W_WIDE(64);
   } else {
-    if (rp <= 64) KGC_SSD_W(4, 2);
-    else if (rp == 128) KGC_SSD_W(8, 2);
-    else KGC_SSD_W(16, 2);
+    if (rp <= 64) KGC_SSD_W(4, 2, false);
+    else if (rp == 128) KGC_SSD_W(8, 2, false);
+    else KGC_SSD_W(16, 2, false);
   }
+#undef KGC_SSD_W_WIDE
 #undef KGC_SSD_W
 }
 
@@ -584,21 +605,28 @@ void launch_gated_delta_scan(int dtype, float* out, const float* qkv, const void
   const bool narrow = scan_narrow(P + D, H, V);
   const int ct = narrow ? 16 : 64, rp = pow2_at_least(d, narrow ? 64 : 16);
   const dim3 grid(P + D, H, (V + ct - 1) / ct);
-#define KGC_GD_W(R, L)                                                                       \
-  KGC_PM_DISPATCH_T(dtype, gated_delta_scan_kernel<T, R, L><<<grid, NT, scan_lds(rp, ct, 3), s>>>( \
+  const bool once = states_once(P + D, H, d, V);
+#define KGC_GD_W(R, L, ONCE)                                                                       \
+  KGC_PM_DISPATCH_T(dtype, gated_delta_scan_kernel<T, R, L, ONCE><<<grid, NT, scan_lds(rp, ct, 3), s>>>( \
       out, qkv, (const T*)ba, bas, a_log, dt_bias, S, qsl, seq_lens, ctx_lens, slots, P, Tp, H, \
       G, d, V, num_slots))
+#define KGC_GD_W_WIDE(R)                                                                     \
+  do {                                                                                       \
+    if (once) KGC_GD_W(R, 4, true);                                                          \
+    else KGC_GD_W(R, 4, false);                                                              \
+  } while (0)
   if (!narrow) {
-    if (rp <= 16) KGC_GD_W(4, 4);
-    else if (rp == 32) KGC_GD_W(8, 4);
-    else if (rp == 64) KGC_GD_W(16, 4);
-    else if (rp == 128) KGC_GD_W(32, 4);
-    else KGC_GD_W(64, 4);
+    if (rp <= 16) KGC_GD_W_WIDE(4);
+    else if (rp == 32) KGC_GD_W_WIDE(8);
+    else if (rp == 64) KGC_GD_W_WIDE(16);
+    else if (rp == 128) KGC_GD_W_WIDE(32);
+    else KGC_GD_W_WIDE(64);
   } else {
-    if (rp <= 64) KGC_GD_W(4, 2);
-    else if (rp == 128) KGC_GD_W(8, 2);
-    else KGC_GD_W(16, 2);
+    if (rp <= 64) KGC_GD_W(4, 2, false);
+    else if (rp == 128) KGC_GD_W(8, 2, false);
+    else KGC_GD_W(16, 2, false);
   }
+#undef KGC_GD_W_WIDE
 #undef KGC_GD_W
 }
 

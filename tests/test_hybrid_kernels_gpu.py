@@ -936,6 +936,36 @@ def test_gla_decode_rows(gpu, dt, H, d, V, R):
     assert (got.cpu()[2] == 0).all() and (st.cpu()[2] == terms[0][2]).all()
 
 
+@pytest.mark.parametrize("op", ["gla", "ssd", "delta"])
+def test_decode_states_beyond_the_caches(gpu, op):
+    """Decode rows whose states are 128 MB and more, which are read and written past the caches: the bits of the
+    same rows in two steps of half as many, of a fresh row and of a padding row too."""
+    torch.manual_seed(43)
+    n, H, d, V, R = 130, *dict(gla=(8, 128, 256, 16), ssd=(32, 128, 64, 0), delta=(16, 128, 128, 0))[op]
+    S = torch.randn(n, H, d, V, device=gpu)
+    assert S.numel() * 4 >= 128 << 20 > S[:n // 2].numel() * 4
+    rnd = lambda *s: torch.randn(*s, device=gpu)   # noqa: E731
+    ctx, slots = [2 + i for i in range(n)], [(i * 7) % n for i in range(n)]
+    ctx[3], slots[70] = 1, -1
+    if op == "gla":
+        x, y, a2, b = rnd(n, 2 * H * d + H * V).bfloat16(), rnd(n, R).bfloat16(), rnd(H * d, R), rnd(H * d)
+        run = lambda r, s, m: ops.gla_scan(x[r], y[r], a2, b, s, m, H, d, V, 16.0)   # noqa: E731
+    elif op == "ssd":
+        x, y, p = rnd(n, H * V + 2 * d), rnd(n, H).bfloat16(), [rnd(H) - 2 for _ in range(3)]
+        run = lambda r, s, m: ops.ssd_scan(x[r], y[r], *p, s, m, H, V, d, 1)   # noqa: E731
+    else:
+        x, y, p = rnd(n, H * d + H * V), rnd(n, 2 * H).bfloat16(), [rnd(H) - 2 for _ in range(2)]
+        run = lambda r, s, m: ops.gated_delta_scan(x[r], y[r], *p, s, m, H, H // 2, d, V)   # noqa: E731
+
+    def step(r, s):
+        t = torch.zeros(len(ctx[r]), 1, dtype=torch.int32)
+        return run(r, s, _to(_meta([], [], ctx[r], t, slots=slots[r]), gpu))
+    once, twice = S.clone(), S.clone()
+    got = step(slice(0, n), once)
+    want = torch.cat([step(slice(0, n // 2), twice), step(slice(n // 2, n), twice)])
+    assert torch.equal(got, want) and torch.equal(once, twice) and not torch.equal(once, S)
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,W,N", [(64, 128, 1), (65, 1024, 17), (79, 1152, 8), (1000, 2048, 16), (64, 2304, 33),
                                       (100, 4096, 5), (8200, 256, 8)])
