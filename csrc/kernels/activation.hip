@@ -3,6 +3,7 @@
 // per thread on a 2-D grid (memory-bound; no index division).
 #include <algorithm>
 
+#include "activation.h"
 #include "common.h"
 #include "launch.h"
 
@@ -21,10 +22,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(T* __restrict__ out, int6
   g.u = *reinterpret_cast<const u32x4*>(xr + c * 8);
   u.u = *reinterpret_cast<const u32x4*>(xr + I + c * 8);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float gf = to_f(g.h[j]);
-    o.h[j] = from_f<T>(gf / (1.f + __expf(-gf)) * to_f(u.h[j]));
-  }
+  for (int j = 0; j < 8; ++j) o.h[j] = from_f<T>(silu_mul_of(to_f(g.h[j]), to_f(u.h[j])));
   *reinterpret_cast<u32x4*>(out + r * os + c * 8) = o.u;
 }
 

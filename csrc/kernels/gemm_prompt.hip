@@ -12,12 +12,15 @@
 // during the last steps and its outputs' conversion.  The MFMAs are written with their accumulators tied: left to the
 // compiler, 256 of 256 accumulators in flight are copied around (half the rate).
 //
-// What bounds it: the power limit at long K (8192^3 plain products 1.58 PFLOP/s at 1.79 GHz, matrix cores busy 84 % of
-// the cycles; the library 1.60), the outputs' conversion besides at K = 2048.  Library and activation launch -> here, us:
-// 14336 x 2048 -> 2 x 5504 SILU 580 -> 451, 14336 x 2048 -> 8256 XIELU 466 to 553 -> 413, 16384 x 4096 -> 2 x 14336 SILU
-// 2803 -> 2550.  A last round of few tiles goes over the CUs in pieces (plan_of).
+// What bounds it: the power limit at long K (8192^3 plain products 1.58 PFLOP/s at 1.79 GHz, the library 1.60), the
+// outputs' conversion besides at K = 2048, beside which the matrix cores idle (one wave per SIMD): of 419 us of XIELU about 70.
+// Library and activation launch -> here, us: 14336 x 2048 -> 2 x 5504 SILU 566 -> 459, 14336 x 2048 -> 8256 XIELU 467 -> 419,
+// 16384 x 4096 -> 2 x 14336 SILU 2746 -> 2540.  (The activations are those of their own launches, to the bit; a quotient by
+// v_rcp and a series of two terms took 442 and 398 us and were less exact.)  A last round of few tiles goes over the CUs in
+// pieces (plan_of).
 #include <type_traits>
 
+#include "activation.h"
 #include "common.h"
 #include "device.h"
 #include "launch.h"
@@ -61,18 +64,6 @@ template <int N> __device__ __forceinline__ void meet() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-}
-
-__device__ __forceinline__ float silu_gate(float g, float u) {
-  return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * -1.44269504088896340736f)) * u;
-}
-// e^z - 1 - z: below -1/32 as it is written (off by 1e-7 where the result is 0.016 at least), from there on z^2 (1/2 + z/6),
-// whose next term is z^2 / 12 of it
-__device__ __forceinline__ float xielu_of(float z, float a, float b) {
-  const float q = z * z;
-  const float t = __builtin_amdgcn_exp2f(z * 1.44269504088896340736f) - (1.f + z);
-  const float e = z > -0.03125f ? q * __builtin_fmaf(z, 1.f / 6.f, 0.5f) : t;
-  return __builtin_fmaf(z > 0.f ? a : b, z > 0.f ? q : e, 0.5f * z);
 }
 
 // Walks over tiles (or pieces) of 2 MT x 2 NT 16-row tiles, MT x NT per wave: numbers first, first + step, .. < count.
@@ -228,9 +219,9 @@ __device__ __forceinline__ void walk(const PromptArgs& g, T* x0, T* x1, T* w0, T
         Pack8<T> o;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          // (of the projection as rounded to T: a row's result does not depend on which way its step took)
+          // (of the projection as rounded to T, as a launch of the activation reads it)
           const float z = to_f(from_f<T>(acc[2 * p + (e >> 2)][j][e & 3]));
-          if constexpr (SILU) o.h[e] = from_f<T>(silu_gate(z, to_f(from_f<T>(acc[NT / 2 + 2 * p + (e >> 2)][j][e & 3]))));
+          if constexpr (SILU) o.h[e] = from_f<T>(silu_mul_of(z, to_f(from_f<T>(acc[NT / 2 + 2 * p + (e >> 2)][j][e & 3]))));
           else o.h[e] = from_f<T>(xielu_of(z, pa, pb));
         }
         *reinterpret_cast<u32x4*>(rows + rr * CW + (((p * 4 + qd) ^ (rr & (U - 1))) * 8)) = o.u;
@@ -292,12 +283,13 @@ Plan plan_of(int act, int M, int N) {
 // SILU and 0.7, from 1024 rows on, for XIELU, whose outputs' conversion takes an eighth of a tile's time and whose activation
 // launch moves less.  Below, one round of quarters at K <= 2048 pays from 65 rows on: the library takes 26 us for any.  us,
 // library and activation -> here:
-//   SILU  K 2048 -> 2 x 5504, 512 rows 36 -> 29, 1024 60 -> 49, 2048 94 -> 78, 2700 137 -> 98, 6000 311 -> 203;  -> 2 x 2752, 256
-//         27 -> 20, 512 27 -> 20, 1024 37 -> 28, 3072 86 -> 64, 14336 372 -> 235
-//         K 4096 -> 2 x 14336, 64 52 -> 74, 320 82 -> 93, 512 106 -> 103, 768 171 -> 158, 2700 585 -> 447, 16384 2803 -> 2550;
-//         -> 2 x 3584, 512 40 -> 35, 768 51 -> 52, 2700 246 -> 124
-//   XIELU K 2048 -> 8256, 256 28 -> 23, 512 33 -> 34, 1024 53 -> 58, 1536 70 -> 60, 4096 154 -> 134, 14336 466 -> 413
-//         K 4096 -> 21504, 512 92 -> 105, 1024 174 -> 171, 2048 293 -> 295, 4096 596 -> 539, 8192 1231 -> 1046
+//   SILU  K 2048 -> 2 x 5504, 256 rows 29 -> 20, 512 36 -> 29, 1024 58 -> 49, 2048 94 -> 78, 2700 134 -> 96, 6000 299 -> 202,
+//         14336 566 -> 459;  -> 2 x 2752, 256 29 -> 20, 1024 37 -> 29, 3072 84 -> 66, 14336 357 -> 237
+//         K 4096 -> 2 x 14336, 320 75 -> 82, 512 105 -> 91, 768 170 -> 139, 2700 577 -> 432, 16384 2746 -> 2540;
+//         -> 2 x 3584, 512 40 -> 36, 768 50 -> 51, 2700 250 -> 123
+//   XIELU K 2048 -> 8256, 256 29 -> 23, 512 34 -> 35, 1024 53 -> 58, 1536 70 -> 60, 2048 93 -> 78, 3000 113 -> 113, 4096 150 -> 135,
+//         8192 319 -> 250, 14336 467 -> 419
+//         K 4096 -> 21504, 512 88 -> 100, 1024 174 -> 155, 2048 296 -> 287, 4096 586 -> 529, 8192 1219 -> 1030
 bool prompt_gemm_pays(int act, int M, int N, int K) {
   const Plan p = plan_of(act, M, N);
   const int cus = device_cus(), rest = p.tm * p.tn - p.whole;

@@ -13,6 +13,7 @@
 // One workgroup per row.  Rows of any width are walked twice (sum of squares, then scale), the second
 // walk re-reading what the same thread wrote in the first; where vectors fit, the row stays in
 // registers.
+#include "activation.h"
 #include "common.h"
 #include "launch.h"
 
@@ -295,8 +296,7 @@ __global__ __launch_bounds__(NT) void xielu_kernel(T* __restrict__ out, const T*
   }
 }
 
-// eight 16-bit elements per thread and step.  exp(v) - 1 - v without cancellation: the series
-// v^2 (1/2 + v/6 + .. + v^6/40320) from -1/2 up, where its next term is 5e-8 of it, else 2^(v log2 e).
+// eight 16-bit elements per thread and step
 template <typename T>
 __global__ __launch_bounds__(NT) void xielu_vec_kernel(T* __restrict__ out, const T* __restrict__ z,
                                                        const float* __restrict__ ab, int64_t n8) {
@@ -305,18 +305,7 @@ __global__ __launch_bounds__(NT) void xielu_vec_kernel(T* __restrict__ out, cons
     Pack8<T> v, o;
     v.u = reinterpret_cast<const u32x4*>(z)[i];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float x = to_f(v.h[j]);
-      float p = 1.f / 40320.f;
-      p = p * x + 1.f / 5040.f;
-      p = p * x + 1.f / 720.f;
-      p = p * x + 1.f / 120.f;
-      p = p * x + 1.f / 24.f;
-      p = p * x + 1.f / 6.f;
-      p = p * x + 0.5f;
-      const float e = x > -0.5f ? x * x * p : (__builtin_amdgcn_exp2f(x * 1.44269504088896340736f) - 1.f) - x;
-      o.h[j] = from_f<T>(x > 0.f ? a * x * x + 0.5f * x : b * e + 0.5f * x);
-    }
+    for (int j = 0; j < 8; ++j) o.h[j] = from_f<T>(xielu_of(to_f(v.h[j]), a, b));
     reinterpret_cast<u32x4*>(out)[i] = o.u;
   }
 }

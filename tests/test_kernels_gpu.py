@@ -1707,6 +1707,28 @@ def test_prompt_gemm_matches_fp64(gpu, dt, act, M, N, K):
     assert worst <= 8 * 4 * K ** 0.5 * 2.0 ** -24, float(worst)
 
 
+@pytest.mark.parametrize("dt", DT)
+def test_prompt_gemm_activations_are_the_launches(gpu, dt):
+    """Projections that are exactly every 16-bit number (K's first column alone): the bits of the activation's own
+    launch, whose series and quotient hold for small and for large ones, infinities and NaN."""
+    every = torch.arange(-2 ** 15, 2 ** 15, dtype=torch.int32).to(torch.int16).view(dt)
+    every = every[(every == 0) | ~(every.float().abs() < torch.finfo(dt).tiny)]     # (products need not keep subnormals)
+    z = every[: every.numel() // 8 * 8].to(gpu)
+    N, K = z.numel(), 128
+    w = torch.zeros(2 * N, K, dtype=dt, device=gpu)
+    w[:N, 0], w[N:, 0] = z, torch.randn(N, device=gpu).to(dt)
+    x = torch.zeros(3, K, dtype=dt, device=gpu)
+    x[:, 0] = 1
+    out = torch.empty(3, N, dtype=dt, device=gpu)
+    same = dict(rtol=0, atol=0, equal_nan=True)
+    for b in (0.6, 1.1, 4.0):
+        ab = torch.tensor([0.7, b], device=gpu)
+        ops._k().prompt_xielu(out, x, w[:N], ab)
+        torch.testing.assert_close(out, ops.xielu(z.expand(3, N).contiguous(), ab), **same)
+    ops._k().prompt_silu(out, x, w)
+    torch.testing.assert_close(out, ops.silu_mul(w[:, 0].expand(3, 2 * N).contiguous()), **same)
+
+
 def test_prompt_gemm_routes(gpu):
     """linear_silu and linear_xielu take it where it pays and its operands fit, and only there."""
     from kubernetes_gpu_cluster_amd.ops import gemm
