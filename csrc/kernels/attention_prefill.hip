@@ -1041,7 +1041,8 @@ __global__ __launch_bounds__(256 * GR, 2) void prefill_attn_walk_kernel(const Wa
   auto fresh = [&] {
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
-      m[qt] = group == 0 ? -INFINITY : -1e30f, l[qt] = 0.f;     // (the second group's rows may see none of its keys)
+      // (rows may see none of the second group's keys: no score is below a maximum of the least number, and its sum is 0)
+      m[qt] = group == 0 ? -INFINITY : -__FLT_MAX__, l[qt] = 0.f;
 #pragma unroll
       for (int t = 0; t < DT; ++t) o[qt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }

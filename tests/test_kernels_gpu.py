@@ -1751,6 +1751,22 @@ def test_prompt_gemm_routes(gpu):
         torch.testing.assert_close(gemm.linear_silu(y, v).float(), want.float(), atol=3e-2, rtol=2e-2)
 
 
+def _causal_fp64(q, kc, vc, bt, qsl, seq_lens, scale):
+    """Per row and head: the float64 result, and the weighted mean of |v|."""
+    nq, nkv = q.shape[1], kc.shape[1]
+    want = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+    mean = torch.empty_like(want)
+    for i, L in enumerate(seq_lens):
+        a, b = int(qsl[i]), int(qsl[i + 1])
+        k, v = (x.double() for x in ref._gather_kv(kc, vc, bt[i], L, 1.0, 1.0))
+        late = torch.arange(L, device=q.device) > torch.arange(L - (b - a), L, device=q.device)[:, None]
+        for h in range(nq):
+            g = h // (nq // nkv)
+            p = ((q[a:b, h].double() @ k[:, g].t()) * scale).masked_fill(late, float("-inf")).softmax(-1)
+            want[a:b, h], mean[a:b, h] = p @ v[:, g], p @ v[:, g].abs()
+    return want, mean
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("nq,nkv,bs", [(32, 8, 32), (8, 1, 64)])
 @pytest.mark.parametrize("query_lens,seq_lens", [
@@ -1773,6 +1789,28 @@ def test_prefill_walk_two_groups(gpu, monkeypatch, dt, nq, nkv, bs, query_lens, 
     one, unit = run(), 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
     assert torch.equal(two, again)
     torch.testing.assert_close(two.float(), one.float(), atol=unit * float(vc.abs().max()), rtol=2 * unit)
+
+
+@pytest.mark.parametrize("query_lens,seq_lens", [([129], [129]), ([33, 100, 1, 32], [161, 1000, 65, 800]), ([1100], [1100])])
+def test_prefill_walk_two_groups_low_scores(gpu, monkeypatch, query_lens, seq_lens):
+    """Scores that are all below -1e30 (exactly -k 2^100, k of 1 to 1.75; a scale of ln 2 leaves them as exponents of 2):
+    the mean of the values whose key is the least, as with one group, also where the second group has none."""
+    torch.manual_seed(38)
+    nq, nkv, bs, d, dt = 8, 2, 32, 128, torch.bfloat16
+    kc, vc, bt = _fill_random_cache(len(seq_lens), seq_lens, nkv, bs, d, dt, gpu)
+    kc.zero_()
+    kc[..., 0] = (torch.randint(4, 8, kc.shape[:-1], device=gpu) * 2.0 ** 48).to(dt)
+    q = torch.zeros(sum(query_lens), nq, d, dtype=dt, device=gpu)
+    q[..., 0] = -2.0 ** 50
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)   # noqa: E731
+    qsl, sl = i32([0] + query_lens).cumsum(0).int(), i32(seq_lens)
+    ws, wm = map(i32, ops.prefill_work_list(query_lens, seq_lens))
+    scale = 1 / 1.4426950408889634
+    want, mean = _causal_fp64(q, kc, vc, bt, qsl, seq_lens, scale)
+    for mode in (None, "1"):
+        monkeypatch.setenv("KGC_PREFILL_PERSIST", mode) if mode else monkeypatch.delenv("KGC_PREFILL_PERSIST", raising=False)
+        got = ops.prefill_attention(q, kc, vc, bt, qsl, sl, scale, ws, wm).double()
+        assert bool(((got - want).abs() <= 1.02 * 2.0 ** -8 * want.abs() + 2.0 ** -13 * mean).all())
 
 
 @pytest.mark.parametrize("dt", DT)
