@@ -533,9 +533,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
 // kernel runs with Zmax = Z).
 // (A four-deep variant -- four named chunk buffers at one wave per SIMD -- measured slower
 // at every shape, e.g. 21.5 vs 17.5 us at B = 256, nq 8 / nkv 1, one slice: removed.)
-// ONCE: V's lines, which nothing reads again, leave the caches alone (an instruction reads whole ones; K's take two each: as
-// these they come a tenth slower).  The rule: at the launch.
-template <typename T, int D, bool KV8, bool FUSE, bool ONCE>
+template <typename T, int D, bool KV8, bool FUSE>
 __global__ __launch_bounds__(64, 2) void paged_decode_wave_kernel(
     T* __restrict__ out, const T* __restrict__ q, const void* __restrict__ kc_,
     const void* __restrict__ vc_, const int* __restrict__ block_tables, int bt_stride,
@@ -549,11 +547,6 @@ __global__ __launch_bounds__(64, 2) void paged_decode_wave_kernel(
   auto ldf = [](const C* p) -> u32x4 {
     if constexpr (KV8) return fp8x8_widen<T>(*reinterpret_cast<const u32x2*>(p));
     else return *reinterpret_cast<const u32x4*>(p);
-  };
-  auto ldv = [&](const C* p) -> u32x4 {
-    if constexpr (!ONCE) return ldf(p);
-    else if constexpr (KV8) return fp8x8_widen<T>(__builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p)));
-    else return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
   };
   constexpr int KS = D / 32, DT = D / 16;
   __shared__ __attribute__((aligned(16))) T lds_q[FUSE ? 16 : 1][FUSE ? D + 8 : 8];
@@ -603,15 +596,16 @@ __global__ __launch_bounds__(64, 2) void paged_decode_wave_kernel(
     const C* kb = kbase + blk_of(tb) * blk_stride + (int64_t)(tb & bsm) * D + 8 * qd;
     if (dok) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int s2 = 0; s2 < KS; ++s2) f.k[j][s2].u = ldf((j ? kb : ka) + 32 * s2);
+      for (int s2 = 0; s2 < KS; ++s2) {
+        f.k[0][s2].u = ldf(ka + 32 * s2);
+        f.k[1][s2].u = ldf(kb + 32 * s2);
+      }
     }
     const int t0 = min(base + 8 * qd, end - 1) & ~7;
     const C* va = vbase + blk_of(t0) * blk_stride + ((t0 & bsm) >> 3) * (D * 8) + r16 * 8;
     if (dov) {
 #pragma unroll
-      for (int t = 0; t < DT; ++t) f.v[t].u = ldv(va + 16 * t * 8);
+      for (int t = 0; t < DT; ++t) f.v[t].u = ldf(va + 16 * t * 8);
     }
   };
   auto issue = [&](Frag& f, int ci) { issue_part(f, ci, true, true); };
@@ -1032,16 +1026,9 @@ static void decode_dispatch(void* out, const void* q, const void* kc, const void
   // ::test_paged_decode_single_slice_rows_many_pairs)
   const DecodeLeast least = decode_least_chunks(B, nkv, KV8);
   if (wave) {
-    // V read past the caches where K and V of as many tokens as the tables hold are more than half of the last-level
-    // cache (256 MB); less of it may still lie there, and is then faster by plain loads.  Calls on three sets of pages in turn,
-    // 8 kv heads, us: 256 x 640 116.5 -> 109.5, 256 x 200 44.0 -> 38.9, 64 x 600 34.7 -> 30.0, 64 x 4000 171 -> 155, 128 x 4000
-    // 323 -> 293, fp8 128 x 640 38.2 -> 33.3, 16 x 4000 35.8 -> 33.0; below the line 32 x 600 18.0 -> 18.6, 4 x 4000 17.3 -> 18.5
-    // (on 12 sets, from memory, 21.3 -> 20.0 and 20.0 -> 19.4).
-    auto kernel = &paged_decode_wave_kernel<T, D, KV8, FUSE, false>;
-    const int64_t held = (int64_t)bt_stride << bs_log2;
-    if ((int64_t)B * nkv * held * (2 * D * (KV8 ? 1 : 2)) > (int64_t)128 << 20) kernel = &paged_decode_wave_kernel<T, D, KV8, FUSE, true>;
-    kernel<<<dim3(B, nkv, Z), 64, 0, s>>>((T*)out, (const T*)q, kc, vc, bt, bt_stride, ctx, ml, es, tmp, nq, nkv, bs_log2,
-                                          scale_log2, v_scale, num_blocks, rp, least);
+    paged_decode_wave_kernel<T, D, KV8, FUSE><<<dim3(B, nkv, Z), 64, 0, s>>>(
+        (T*)out, (const T*)q, kc, vc, bt, bt_stride, ctx, ml, es, tmp, nq, nkv, bs_log2,
+        scale_log2, v_scale, num_blocks, rp, least);
   } else {
     paged_decode_kernel<T, D, true, KV8, 4, 1, FUSE><<<dim3(B, nkv, Z), 256, 0, s>>>(
         (T*)out, (const T*)q, kc, vc, bt, bt_stride, ctx, ml, es, tmp, nq, nkv, bs_log2, Z,

@@ -233,8 +233,8 @@ def test_paged_decode_rope(gpu, monkeypatch, kern, dt, d, nq, nkv, qk_norm, S, f
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("d,fp8", [(128, False), (128, True), (64, False)])
 def test_paged_decode_long_tables(gpu, dt, d, fp8):
-    """Tables that may hold more K and V than the last-level cache (their tail names one page; V is then read past the
-    caches): the bits of the same call with tables of the contexts' own width, in one slice and in three."""
+    """Tables as wide as a service's longest request (their tail names one page): the bits of the same call with tables of the
+    contexts' own width, in one slice and in three."""
     torch.manual_seed(23)
     nkv, bs, ctx = 8, 32, [1, 31, 32, 33, 64, 200, 500, 0] * 4
     kc, vc, bt = _fill_random_cache(len(ctx), [max(c, 1) for c in ctx], nkv, bs, d, dt, gpu)
