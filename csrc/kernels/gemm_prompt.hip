@@ -279,25 +279,32 @@ Plan plan_of(int act, int M, int N) {
 }  // namespace
 
 // Whether it is faster than the library's projection and a launch of the activation, which fill small or odd numbers of tiles
-// better.  Of the rounds' time (quarters and halves as above) the useful part of the tiles must be half, from 512 rows on, for
-// SILU and 0.7, from 1024 rows on, for XIELU, whose outputs' conversion takes an eighth of a tile's time and whose activation
-// launch moves less.  Below, one round of quarters at K <= 2048 pays from 65 rows on: the library takes 26 us for any.  us,
-// library and activation -> here:
+// better: by the useful part of the time of the rounds (quarters and halves as above).  From 512 rows on for SILU and 1024 for
+// XIELU, whose outputs' conversion takes a sixth of a tile's time at K = 2048 and whose activation launch moves less.
+// K <= 2048, where the library takes 26 us at least: one round of quarters from 65 rows on; else half (a single round of tiles
+// 0.54), XIELU 0.7, and not below K = 2048, where the conversion takes as long as the products.  Longer K: 0.77.  Over 19 shapes
+// of 1024 to 8192 columns and 80 to 16384 rows with weights from memory, what the rule takes is 1.23 times as fast in the
+// geometric mean, 0.976 at worst; half of the rounds' time for all K took as many shapes again at 0.79 to 1.05.
+// us, library and activation -> here:
 //   SILU  K 2048 -> 2 x 5504, 256 rows 29 -> 20, 512 36 -> 29, 1024 58 -> 49, 2048 94 -> 78, 2700 134 -> 96, 6000 299 -> 202,
 //         14336 566 -> 459;  -> 2 x 2752, 256 29 -> 20, 1024 37 -> 29, 3072 84 -> 66, 14336 357 -> 237
-//         K 4096 -> 2 x 14336, 320 75 -> 82, 512 105 -> 91, 768 170 -> 139, 2700 577 -> 432, 16384 2746 -> 2540;
-//         -> 2 x 3584, 512 40 -> 36, 768 50 -> 51, 2700 250 -> 123
-//   XIELU K 2048 -> 8256, 256 29 -> 23, 512 34 -> 35, 1024 53 -> 58, 1536 70 -> 60, 2048 93 -> 78, 3000 113 -> 113, 4096 150 -> 135,
-//         8192 319 -> 250, 14336 467 -> 419
-//         K 4096 -> 21504, 512 88 -> 100, 1024 174 -> 155, 2048 296 -> 287, 4096 586 -> 529, 8192 1219 -> 1030
+//         K 4096 -> 2 x 14336, 512 105 -> 91, 768 170 -> 139, 2700 577 -> 432, 16384 2746 -> 2540; not 320 75 -> 82, 640 145 -> 156;
+//         -> 2 x 5504, 3072 315 -> 206, 16384 1206 -> 995; not 768 79 -> 93;  -> 2 x 3584, 2700 250 -> 123; not 1280 83 -> 94
+//         K 8192 -> 2 x 7168, 1024 217 -> 180, 5120 950 -> 827; not 512 119 -> 132, 640 141 -> 171
+//   XIELU K 2048 -> 8256, 256 29 -> 23, 1536 70 -> 60, 2048 93 -> 78, 3000 113 -> 113, 4096 150 -> 135, 8192 319 -> 250, 14336 467 ->
+//         419; not 512 34 -> 35, 1024 53 -> 58
+//         K 4096 -> 21504, 2560 472 -> 361, 4096 586 -> 529, 8192 1219 -> 1030; not 512 88 -> 100, 1152 184 -> 198
 bool prompt_gemm_pays(int act, int M, int N, int K) {
   const Plan p = plan_of(act, M, N);
   const int cus = device_cus(), rest = p.tm * p.tn - p.whole;
-  if (M > 64 && p.whole == 0 && p.pieces == 4 && K <= 2048) return true;
-  if (M < (act == PROMPT_SILU ? 512 : 1024)) return false;
+  const bool silu = act == PROMPT_SILU, pieces = p.whole == 0;
+  if (M > 64 && pieces && p.pieces == 4 && K <= 2048) return true;
+  if (M < (silu ? 512 : 1024)) return false;
   const double rounds = (p.whole + cus - 1) / cus + (rest == 0 ? 0. : p.pieces == 4 ? 0.43 : 0.62);
-  const double useful = (double)M * N / (BT * (act == PROMPT_SILU ? BT / 2 : BT)) / cus;
-  return useful >= rounds * (act == PROMPT_SILU ? 0.5 : 0.7);
+  const double useful = (double)M * N / (BT * (silu ? BT / 2 : BT)) / cus;
+  if (K > 2048) return useful >= rounds * 0.77;
+  if (silu) return useful >= rounds * (rounds == 1. ? 0.54 : 0.5);
+  return (K == 2048 || pieces) && useful >= rounds * 0.7;
 }
 
 void launch_prompt_gemm(int dtype, int act, void* out, const void* x, const void* w, const float* ab, int M, int N,

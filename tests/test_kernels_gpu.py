@@ -1751,6 +1751,22 @@ def test_prompt_gemm_routes(gpu):
         torch.testing.assert_close(gemm.linear_silu(y, v).float(), want.float(), atol=3e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("silu,K,N,M,want", [
+    (True, 2048, 2752, 80, True), (True, 2048, 5504, 1024, True), (True, 2048, 5504, 800, False), (True, 2048, 5504, 576, False),
+    (True, 4096, 14336, 2700, True), (True, 4096, 5504, 768, False), (True, 4096, 7168, 640, False), (True, 4096, 3584, 1280, False),
+    (True, 8192, 7168, 1024, True), (True, 8192, 3584, 768, False), (True, 8192, 3584, 3584, False),
+    (False, 2048, 8256, 256, True), (False, 2048, 8256, 14336, True), (False, 2048, 8256, 1024, False),
+    (False, 4096, 21504, 2560, True), (False, 4096, 21504, 1152, False), (False, 1024, 4096, 1024, True), (False, 1024, 4096, 3072, False)])
+def test_prompt_gemm_rule(gpu, silu, K, N, M, want):
+    """The projection with its activation is taken where its tiles fill the CUs, and left to the library where that was
+    measured to be faster (gemm_prompt.hip has the times)."""
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("lines for 256 CUs")
+    x = torch.empty(M, K, dtype=torch.bfloat16, device=gpu)
+    w = torch.empty(2 * N if silu else N, K, dtype=torch.bfloat16, device=gpu)
+    assert ops._k().prompt_gemm_pays(x, w, silu) == want
+
+
 def _causal_fp64(q, kc, vc, bt, qsl, seq_lens, scale):
     """Per row and head: the float64 result, and the weighted mean of |v|."""
     nq, nkv = q.shape[1], kc.shape[1]
