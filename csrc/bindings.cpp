@@ -285,7 +285,7 @@ void paged_decode_rope(Tensor out, Tensor qkv, Tensor positions, Tensor cos_sin,
 
 void prefill_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables,
                        Tensor query_start_loc, Tensor seq_lens, Tensor work_seq,
-                       Tensor work_mblk, double scale, double k_scale, double v_scale) {
+                       Tensor work_mblk, double scale, double k_scale, double v_scale, int64_t max_len) {
   check_gpu(q, "q");
   c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
   TORCH_CHECK(q.dim() == 3 && q.is_contiguous(), "q [T, nq, d] contiguous");
@@ -305,7 +305,7 @@ void prefill_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Ten
                                 v_cache.data_ptr(), block_tables.data_ptr<int>(),
                                 (int)block_tables.stride(0), query_start_loc.data_ptr<int>(),
                                 seq_lens.data_ptr<int>(), work_seq.data_ptr<int>(),
-                                work_mblk.data_ptr<int>(), (int)work_seq.numel(), (int)P, (int)nq,
+                                work_mblk.data_ptr<int>(), (int)work_seq.numel(), (int)P, max_len, (int)nq,
                                 (int)k_cache.size(1), (int)d,
                                 log2_exact(k_cache.size(2), "block_size"), (float)scale,
                                 k_cache.scalar_type() == at::kFloat8_e4m3fn, (float)k_scale,
@@ -318,7 +318,7 @@ void prefill_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Ten
 void prefill_attention_rope(Tensor out, Tensor qkv, Tensor cos_sin, Tensor k_cache,
                             Tensor v_cache, Tensor block_tables, Tensor query_start_loc,
                             Tensor seq_lens, Tensor work_seq, Tensor work_mblk, int64_t nq,
-                            double scale, double k_scale, double v_scale) {
+                            double scale, double k_scale, double v_scale, int64_t max_len) {
   check_gpu(qkv, "qkv");
   c10::hip::HIPGuardMasqueradingAsCUDA g(qkv.device());
   TORCH_CHECK(out.dim() == 3 && out.is_contiguous() && out.size(1) == nq &&
@@ -346,7 +346,7 @@ void prefill_attention_rope(Tensor out, Tensor qkv, Tensor cos_sin, Tensor k_cac
                                 v_cache.data_ptr(), block_tables.data_ptr<int>(),
                                 (int)block_tables.stride(0), query_start_loc.data_ptr<int>(),
                                 seq_lens.data_ptr<int>(), work_seq.data_ptr<int>(),
-                                work_mblk.data_ptr<int>(), (int)work_seq.numel(), (int)P, (int)nq,
+                                work_mblk.data_ptr<int>(), (int)work_seq.numel(), (int)P, max_len, (int)nq,
                                 (int)nkv, (int)d, log2_exact(k_cache.size(2), "block_size"),
                                 (float)scale, k_cache.scalar_type() == at::kFloat8_e4m3fn,
                                 (float)k_scale, (float)v_scale, (int)k_cache.size(0),
@@ -1470,7 +1470,7 @@ void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
                       std::optional<Tensor> gate, bool fast, double softcap, double out_scale,
                       std::optional<Tensor> elem_gate, int64_t pool, int64_t block_size,
                       std::optional<Tensor> v_table, bool interleaved,
-                      std::optional<Tensor> slots, bool chunked, double sink, int64_t max_ctx) {
+                      std::optional<Tensor> slots, bool chunked, double sink, int64_t max_ctx, int64_t max_len) {
   check_gpu(q, "q");
   c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
   TORCH_CHECK(q.dim() == 3 && q.is_contiguous() && act_dtype(q), "kgc.window_attention: q [T, H, dk]");
@@ -1590,7 +1590,7 @@ void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
                                     work_seq->data_ptr<int>(), work_blk->data_ptr<int>(), (int)nw,
                                     kgc::prefill_block_m(), (int)H, (int)G, (int)dk, (int)dv,
                                     (int)krs, (int)vrs, bs, nb, (float)scale, (int)window, (int)keep_first, gp, ex,
-                                    stream());
+                                    {(int)P, Tp, max_len}, stream());
     rest &= ~1;
   }
   if (fast && aligned && D > 0 &&
@@ -2768,7 +2768,7 @@ TORCH_LIBRARY(kgc, m) {
         "Tensor? seq_lens, Tensor? pbt, Tensor? ctx_lens, Tensor? dbt, Tensor? work_seq, Tensor? work_blk, "
         "int P, int D, int Tp, float scale, int window, int keep_first, Tensor? gate, bool fast, "
         "float softcap, float out_scale, Tensor? elem_gate, int pool, int block_size, "
-        "Tensor? v_table, bool interleaved, Tensor? slots, bool chunked, float sink, int max_ctx=0) -> ()");
+        "Tensor? v_table, bool interleaved, Tensor? slots, bool chunked, float sink, int max_ctx=0, int max_len=0) -> ()");
   m.def("mlstm_scan(Tensor(a!) out, Tensor qkvg, Tensor gates, Tensor(b!) S, Tensor(c!) n, Tensor(d!) m, "
         "Tensor? qsl, Tensor? seq_lens, Tensor? ctx_lens, Tensor slots, int P, int D, int Tp, int H, int d, "
         "int dv) -> ()");
@@ -2791,11 +2791,11 @@ TORCH_LIBRARY(kgc, m) {
         "Tensor? row_scale=None) -> ()");
   m.def("prefill_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, "
         "Tensor block_tables, Tensor query_start_loc, Tensor seq_lens, Tensor work_seq, "
-        "Tensor work_mblk, float scale, float k_scale=1.0, float v_scale=1.0) -> ()");
+        "Tensor work_mblk, float scale, float k_scale=1.0, float v_scale=1.0, int max_len=0) -> ()");
   m.def("prefill_attention_rope(Tensor(a!) out, Tensor qkv, Tensor cos_sin, Tensor k_cache, "
         "Tensor v_cache, Tensor block_tables, Tensor query_start_loc, Tensor seq_lens, "
         "Tensor work_seq, Tensor work_mblk, int nq, float scale, float k_scale=1.0, "
-        "float v_scale=1.0) -> ()");
+        "float v_scale=1.0, int max_len=0) -> ()");
   m.def("sample(Tensor(a!) out, Tensor logits, Tensor temperature, Tensor top_k, Tensor top_p, "
         "Tensor seeds, bool thresholds=True) -> ()");
   m.def("sample_vp(Tensor(a!) packed, Tensor logits, int V, Tensor temperature, Tensor seeds, "

@@ -1096,7 +1096,9 @@ __global__ __launch_bounds__(256 * GR, 2) void prefill_attn_walk_kernel(const Wa
     }
     kt += GR;
     if (GR == 1 ? !last : kt - group < cur.n_tiles) return false;
-    if constexpr (GR == 2) {                 // the second group's sums join the first one's, by way of its own tiles
+    if (GR == 2 && cur.n_tiles == 1) {       // the second group has none
+      if (group == 1) return true;
+    } else if constexpr (GR == 2) {          // the second group's sums join the first one's, by way of its own tiles
       f32x4* const in[4] = {reinterpret_cast<f32x4*>(K0 + TE), reinterpret_cast<f32x4*>(K1 + TE), reinterpret_cast<f32x4*>(V0 + TE),
                             reinterpret_cast<f32x4*>(V1 + TE)};
       f32x4* const ml = reinterpret_cast<f32x4*>(rows) + lane;
@@ -1186,7 +1188,7 @@ static int prefill_persist_mode() {
 template <typename T, int D, bool KV8, int GH>
 static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const void* vc,
                                  const int* bt, int bt_stride, const int* qsl, const int* sl,
-                                 const int* ws, const int* wm, int n_work, int n_seq, int nq, int nkv,
+                                 const int* ws, const int* wm, int n_work, int n_seq, int64_t max_len, int nq, int nkv,
                                  int bs_log2, float scale_log2, float v_scale, int num_blocks,
                                  int64_t q_stride, const float* cos_sin, int cs_rows, hipStream_t s) {
   constexpr size_t lds = 2 * 2 * PF_BN * D * sizeof(T);
@@ -1197,11 +1199,12 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool dma = aligned(q) && q_stride % 8 == 0;    // 16-byte DMAs
   if constexpr (!KV8) {
-    // Few rows on short tables are one tile each, for which the walk has nothing to overlap (2 x 64 rows 17.2 us, the one-shot
-    // grid 16.2; 16 x 60 27.2 and 27.5); all else is faster so: one-shot grid -> walk, K / V write included, us: 512 rows
-    // 32.5 -> 27.5, 1000 51.9 -> 39.1, 2000 after 2000 164 -> 128, 8 x 100 after 3000 127 -> 98, 4 x 300 30.4 -> 27.8.
+    // Few rows of short sequences are one tile each, for which the walk has nothing to overlap (K / V write included, one-shot grid
+    // -> walk, us: 2 x 64 rows 14.5 -> 15.6, 1 x 30 16.3 -> 17.2, 8 x 128 20.2 -> 20.1); all else is faster so: 512 rows 31.1 -> 23.2, 1000
+    // 51.9 -> 39.1, 2000 after 2000 164 -> 128, 8 x 100 after 3000 127 -> 98, 4 x 300 30.1 -> 27.5.
     const int64_t n = (int64_t)n_work * nkv * (G / 4) * (PF_BM / 32);
-    const bool pays = n > 2 * n_cu || ((int64_t)bt_stride << bs_log2) > 128;
+    const int64_t table = (int64_t)bt_stride << bs_log2, length = max_len > 0 ? std::min(max_len, table) : table;
+    const bool pays = n > 2 * n_cu || length > 128;
     if (dma && aligned(kc) && aligned(vc) && aligned(out) && bs_log2 >= 5 && (mode < 0 ? pays : mode != 0) &&
         n < ((int64_t)1 << 30) && q_stride < (1 << 24) && (int64_t)nq * D < (1 << 24) &&
         ((int64_t)nkv * D << bs_log2) < ((int64_t)1 << 31)) {       // offsets inside an item and a page in 32 bits
@@ -1235,17 +1238,17 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
 template <typename T, int D, bool KV8>
 static void prefill_dispatch(const void* q, void* out, const void* kc, const void* vc,
                              const int* bt, int bt_stride, const int* qsl, const int* sl,
-                             const int* ws, const int* wm, int n_work, int n_seq, int nq, int nkv,
+                             const int* ws, const int* wm, int n_work, int n_seq, int64_t max_len, int nq, int nkv,
                              int bs_log2, float scale_log2, float v_scale, int num_blocks,
                              int64_t q_stride, const float* cos_sin, int cs_rows, hipStream_t s) {
   const int G = nkv > 0 ? nq / nkv : 1;
   if constexpr (D == 128) if (prefill_gqa_enabled() && nq % nkv == 0 && (G == 4 || G % 8 == 0)) {
     if (G == 4)
-      prefill_gqa_dispatch<T, D, KV8, 4>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, n_seq,
+      prefill_gqa_dispatch<T, D, KV8, 4>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, n_seq, max_len,
                                          nq, nkv, bs_log2, scale_log2, v_scale, num_blocks,
                                          q_stride, cos_sin, cs_rows, s);
     else
-      prefill_gqa_dispatch<T, D, KV8, 8>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, n_seq,
+      prefill_gqa_dispatch<T, D, KV8, 8>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, n_seq, max_len,
                                          nq, nkv, bs_log2, scale_log2, v_scale, num_blocks,
                                          q_stride, cos_sin, cs_rows, s);
     return;
@@ -1259,7 +1262,7 @@ static void prefill_dispatch(const void* q, void* out, const void* kc, const voi
 void launch_prefill_attention(int dtype, const void* q, void* out, const void* k_cache,
                               const void* v_cache, const int* block_tables, int bt_stride,
                               const int* query_start_loc, const int* seq_lens,
-                              const int* work_seq, const int* work_mblk, int n_work, int n_seq, int nq,
+                              const int* work_seq, const int* work_mblk, int n_work, int n_seq, int64_t max_len, int nq,
                               int nkv, int D, int bs_log2, float scale, bool kv_fp8,
                               float k_scale, float v_scale, int num_blocks, int64_t q_stride,
                               const float* cos_sin, int cs_rows, hipStream_t s) {
@@ -1267,7 +1270,7 @@ void launch_prefill_attention(int dtype, const void* q, void* out, const void* k
   const float sl2 = scale * k_scale * 1.4426950408889634f;
 #define KGC_PF(TT, DD, K8)                                                                 \
   prefill_dispatch<TT, DD, K8>(q, out, k_cache, v_cache, block_tables, bt_stride,          \
-                               query_start_loc, seq_lens, work_seq, work_mblk, n_work, n_seq, \
+                               query_start_loc, seq_lens, work_seq, work_mblk, n_work, n_seq, max_len, \
                                nq, nkv, bs_log2, sl2, v_scale, num_blocks, q_stride, cos_sin, cs_rows, s)
 #define KGC_PF_D(TT, K8) \
   if (D == 128) KGC_PF(TT, 128, K8); else KGC_PF(TT, 64, K8)

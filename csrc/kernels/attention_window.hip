@@ -1786,11 +1786,11 @@ void launch_window_prefill_mfma(int dtype, void* out, const void* q, const void*
                                 const int* pbt, int bt_stride, const int* work_seq,
                                 const int* work_blk, int n_work, int blk_rows, int H, int G,
                                 int dk, int dv, int krs, int vrs, int bs, int num_blocks, float scale, int window,
-                                int keep_first, const float* gate, WindowExtra ex, hipStream_t s) {
+                                int keep_first, const float* gate, WindowExtra ex, const PromptShape& ps, hipStream_t s) {
   if (n_work <= 0) return;
   if (launch_window_prefill_gqa(dtype, out, q, k_cache, v_cache, qsl, seq_lens, pbt, bt_stride, work_seq,
                                 work_blk, n_work, blk_rows, H, G, dk, dv, krs, vrs, bs, num_blocks, scale,
-                                window, keep_first, gate, ex, s))
+                                window, keep_first, gate, ex, ps, s))
     return;
   if (dtype == DT_BF16)
     prefill_dispatch<bf16>((bf16*)out, (const bf16*)q, (const bf16*)k_cache,

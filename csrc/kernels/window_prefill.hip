@@ -506,6 +506,9 @@ __global__ __launch_bounds__(FORM == ROWS32 ? 256 : 512, 2) void window_prefill_
     }
     if constexpr (GR == 1) {
       __builtin_amdgcn_s_waitcnt(0x0f70);    // DMAs end before the LDS is another's
+    } else if (ntile == 1) {                 // the second group has none
+      __builtin_amdgcn_s_waitcnt(0x0f70);
+      if (group == 1) return;
     } else {                                 // the second group's sums join the first one's
       constexpr int N0 = DT == 4 ? 2 : 4;    // column blocks in K0; then K1
       static_assert(GR * LR * DK * sizeof(T) >= N0 * 16384 && GR * LR * DK * sizeof(T) >= (DT - N0) * 16384 + 2048, "");
@@ -607,9 +610,10 @@ template <typename T, int KS, int DT, int NB, bool ALIAS, bool CAP>
 bool run(T* out, const T* q, const T* kc, const T* vc, const int* qsl, const int* seq_lens, const int* pbt,
          int bt_stride, const int* work_seq, const int* work_blk, int n_work, int blk_rows, int H, int G,
          int krs, int vrs, int bs, int num_blocks, float scale, int window, int keep_first, const float* gate,
-         const WindowExtra& ex, hipStream_t s) {
+         const WindowExtra& ex, const PromptShape& ps, hipStream_t s) {
   const int64_t wgs = (int64_t)(H / HW) * n_work * (blk_rows / 32);
   int64_t span = (int64_t)bt_stride * bs;
+  if (ps.max_len > 0) span = std::min(span, ps.max_len);
   if (window > 0) span = std::min<int64_t>(span, (int64_t)window + keep_first + 64);
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   // 16-byte units of rows of one page per DMA, keys and values at the same places
@@ -626,23 +630,33 @@ bool run(T* out, const T* q, const T* kc, const T* vc, const int* qsl, const int
         num_blocks, scale, window, keep_first, gate, ex);
     return true;
   };
-  // In bf16, ROWS64 -> here, us.  With no more workgroups of 32 rows than CUs two groups for each, but where the tables hold
-  // three tiles at most: 16 heads on 4, window 1024, 1 x 512 rows 26.6 -> 18.9, 1 x 2048 55.3 -> 38.0, 4 x 300 after 2000 57.8
-  // -> 37.3, 1 x 60 after 3000 57.5 -> 36.1, causal and capped 1 x 100 after 4000 229 -> 137, latent rows 2 x 1000 77.3 -> 49.1;
-  // 2 x 150 12.5 -> 13.1 (32 rows, one group: 12.4), latent 4 x 64 12.1 -> 13.1 (10.0).  Where 64 rows each leave at most half
-  // of the CUs a workgroup in the last round: 1 x 5000 100 -> 86.6, 6 x 1000 54.4 -> 49.2, 12 x 300 22.9 -> 20.5, 40 x 100 after
-  // 300 46.3 -> 44.3; where it is fuller, two workgroups to a CU are no faster than one of twice the rows: 32 x 512 81 -> 82, 20 x
-  // 300 after 1500 108 -> 112, 2 x 2000 in chunks of 1024 after 500 49 -> 64.  Contexts beyond 4096 leave the last round to
-  // the longest rows: capped 1 x 6000 after 1000 369 -> 402.  Latent rows beyond one round in any case: 4 x 2048 155 -> 142,
-  // 24 x 400 64 -> 61, 8 x 2048 260 -> 254, 60 x 200 70 -> 67 (within one: 1 x 4096 86 -> 89, 30 x 100 17.5 -> 18.8).
+  // In bf16, ROWS64 -> here, us (16 heads on 4 unless it says latent).
+  // With no more workgroups of 32 rows than CUs two groups for each: window 1024, 1 x 512 rows 26.6 -> 18.9, 1 x 2048 55.3 -> 38.0,
+  // 4 x 300 after 2000 57.8 -> 37.3, 1 x 60 after 3000 57.5 -> 36.1, causal and capped 1 x 100 after 4000 229 -> 137, latent 2 x 1000
+  // 77.3 -> 49.1.  Three tiles at most: one group (4 x 64 8.9 -> 7.5, two groups 9.4; 2 x 100 10.8 -> 9.4; latent 4 x 64 12.2 -> 9.7, 13.0);
+  // ROWS64 itself where a prompt ends in a block of at most 35 rows, the waves of the others being idle there (1 x 30
+  // 7.0, 7.3 by one group; 20 after 160 11.2, 11.9; 2 x 150 11.4, 12.1).
   // Without a window a prompt's rows have one tile to as many as its length, and the longest rows' chain lasts past the
-  // others: two groups up to two rounds (capped 1 x 3000 175 -> 113, 2 x 1500 92 -> 59, 2 x 2048 114 -> 88, 4 x 1000 67.5 -> 55; rows
-  // alike gain little, 2 x 2048 after 2000 225 -> 213, 8 x 500 after 2000 160 -> 160, or lose on shorter tables, 10 x 256 after
-  // 500 54 -> 56; windowed 1 x 3000 61 -> 65).
-  const int64_t n_cu = device_cus(), last = wgs / 2 % n_cu;
-  const bool pairs = wgs <= n_cu ? span > 192 : wgs <= 2 * n_cu && window <= 0 && span >= 1000;
-  const bool spare = wgs / 2 > n_cu && (KS == 16 || (last > 0 && 2 * last <= n_cu && span <= 4096));
-  const int form = !dma ? ROWS64 : pairs ? ROWS32X2 : wgs <= n_cu || spare ? ROWS32 : ROWS64;
+  // others: two groups up to two rounds for prompts of 500 rows and more (capped 1 x 3000 175 -> 113, 2 x 1500 92 -> 59, 2 x 2048 114 ->
+  // 88, 4 x 1000 67.5 -> 55; 8 x 500 after 2000 161 -> 161), of which fewer lose: 16 x 140 13.8 -> 21.8, 10 x 256 19.0 -> 20.4, 31 x 106
+  // after 3583 221 -> 243; windowed 1 x 3000 61 -> 65.
+  // Beyond, one group where 64 rows each are no more than 11/8 of a round, of windowed prompts or ones of up to 128 rows: window
+  // 1024, 1 x 5000 103 -> 90, 12 x 300 23.4 -> 22.0, 7 x 546 after 1500 107 -> 91 (2 x 2500 69.2 -> 70.6), causal 40 x 100 24.4 -> 22.4, 36 x
+  // 128 32.1 -> 23.2, 40 x 60 after 2000 208 -> 189.  Where the last round is fuller two workgroups to a CU are no faster than one
+  // of twice the rows (24 x 300 38.0 -> 41, 6 x 1000 capped 66.4 -> 67.5), and of longer causal prompts as many lose as gain: 5 x 1000
+  // 56.6 -> 52, 3 x 2134 104 -> 94, but 2 x 2500 111 -> 117, 5 x 1000 after 1000 124 -> 131, capped 17 x 181 21.8 -> 23.6, 1 x 6000 after
+  // 1000 369 -> 402.
+  // Latent rows beyond one round: 32 x 250 50.7 -> 48.4, 5 x 1000 83 -> 73, 4 x 2048 155 -> 142, 8 x 2048 260 -> 254, 80 x 64 48 -> 36 (16 x
+  // 380 46.1 -> 47.2, 12 x 512 54.2 -> 55); but causal 1 x 8000 613 -> 641.  Within one: 1 x 4096 86 -> 89, 30 x 100 17.5 -> 18.8.
+  const int64_t n_cu = device_cus(), mean = ps.rows / std::max(1, ps.seqs);
+  // blocks of 64 rows that have rows: of the last 128 of a prompt the second 64 have none where those rows are 64 at most
+  const double tail = 128. - ((double)n_work * blk_rows - (double)ps.rows) / std::max(1, ps.seqs);
+  const int64_t full = (H / HW) * (int64_t)(n_work * (blk_rows / 64) - ps.seqs * std::min(1., std::max(0., 0.5 + (64 - tail) / 16)));
+  const bool pairs = wgs <= n_cu ? span > 192 : wgs <= 2 * n_cu && window <= 0 && mean >= 500;
+  const bool ends = KS == 16 || mean > 192 || (mean - 1) % 64 >= 35;
+  const bool spare = wgs / 2 > n_cu && (KS == 16 ? window > 0 || mean <= 6000 || full > 2 * n_cu
+                                                 : ends && 8 * full <= 11 * n_cu && span <= 4096 && (window > 0 || mean <= 128));
+  const int form = !dma ? ROWS64 : pairs ? ROWS32X2 : (wgs <= n_cu && ends) || spare ? ROWS32 : ROWS64;
   if (form == ROWS32X2) return go(std::integral_constant<int, ROWS32X2>());
   if (form == ROWS32) return go(std::integral_constant<int, ROWS32>());
   return go(std::integral_constant<int, ROWS64>());
@@ -662,7 +676,7 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
                                const int* work_seq, const int* work_blk, int n_work, int blk_rows, int H,
                                int G, int dk, int dv, int krs, int vrs, int bs, int num_blocks, float scale,
                                int window, int keep_first, const float* gate, const WindowExtra& ex,
-                               hipStream_t s) {
+                               const PromptShape& ps, hipStream_t s) {
   // Four heads on one staged tile against one head per workgroup (bf16, 16 heads on 4 key/value heads): window
   // 1024 with 8 x 2048 rows 355 -> 182 us, causal and capped 577 -> 261, 48 rows after 3000 83 -> 54; latent rows
   // (one key/value head), 32 x 512 rows 380 -> 116 us; 8 x 64 rows 11.0 -> 10.2, latent 12.8 -> 12.4.  The maximum
@@ -676,7 +690,7 @@ bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* 
     typedef std::remove_pointer_t<decltype(o)> T;
     return dispatch<T, decltype(cap)::value>(dk, dv, alias, o, (const T*)q, (const T*)kc, (const T*)vc, qsl, seq_lens,
                                              pbt, bt_stride, work_seq, work_blk, n_work, blk_rows, H, G, krs, vrs,
-                                             bs, num_blocks, scale, window, keep_first, gate, ex, s);
+                                             bs, num_blocks, scale, window, keep_first, gate, ex, ps, s);
   };
   const bool capped = ex.softcap > 0.f;
   if (dtype == DT_BF16) return capped ? go(std::true_type(), (bf16*)out) : go(std::false_type(), (bf16*)out);

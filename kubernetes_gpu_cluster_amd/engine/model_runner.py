@@ -501,6 +501,7 @@ class ModelRunner:
             m.prefill_seq_lens = d32[L.sl:L.sl + P]
             m.work_seq = d32[L.ws:L.ws + W]
             m.work_mblk = d32[L.wm:L.wm + W]
+            m.prefill_max_len = int(self.h32.numpy()[L.sl:L.sl + P].max())   # (this rank's host copy)
         if D:
             m.decode_block_tables = d32[L.dbt:L.dbt + D * mb].view(D, mb)
             m.decode_ctx_lens = d32[L.ctx:L.ctx + D]
@@ -570,6 +571,7 @@ class ModelRunner:
             mh.query_start_loc, mh.prefill_seq_lens = v[0], v[1]
             mh.prefill_block_tables = v[2].view(np_, mb)
             mh.work_seq, mh.work_mblk = v[3], v[4]
+            mh.prefill_max_len = int((sa, sb)[h].max(initial=0))
             metas.append(mh)
         return a, metas[0], metas[1]
 

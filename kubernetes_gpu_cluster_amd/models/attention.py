@@ -30,6 +30,7 @@ class AttnMetadata:
     prefill_seq_lens: Optional[torch.Tensor] = None       # [P] int32 (context incl. chunk)
     work_seq: Optional[torch.Tensor] = None
     work_mblk: Optional[torch.Tensor] = None
+    prefill_max_len: int = 0                              # no prefill sequence is longer (0: not known)
     # decode part
     decode_block_tables: Optional[torch.Tensor] = None    # [D, max_blocks] int32
     decode_ctx_lens: Optional[torch.Tensor] = None        # [D] int32
@@ -73,7 +74,8 @@ class PagedAttention(nn.Module):
         if tp:
             o = ops.prefill_attention(q[:tp], kc, vc, m.prefill_block_tables, m.query_start_loc,
                                       m.prefill_seq_lens, self.scale, m.work_seq, m.work_mblk,
-                                      out=out[:tp], k_scale=ctx.k_scale, v_scale=ctx.v_scale)
+                                      out=out[:tp], k_scale=ctx.k_scale, v_scale=ctx.v_scale,
+                                      max_len=m.prefill_max_len)
             if o.data_ptr() != out.data_ptr():
                 out[:tp].copy_(o)
         if m.num_decodes:

@@ -132,7 +132,7 @@ class LlamaAttention(nn.Module):
             o = ops.prefill_attention_rope(
                 qkv, ctx.cos_sin, kc, vc, m.prefill_block_tables, m.query_start_loc,
                 m.prefill_seq_lens, self.attn.scale, self.nq, self.cfg.head_dim, m.work_seq,
-                m.work_mblk, k_scale=ctx.k_scale, v_scale=ctx.v_scale)
+                m.work_mblk, k_scale=ctx.k_scale, v_scale=ctx.v_scale, max_len=m.prefill_max_len)
             return o.view(o.shape[0], self.nq * self.cfg.head_dim)
         q = ops.rope_kv_write(qkv, positions, ctx.cos_sin, kc, vc, ctx.attn.slot_mapping,
                               self.nq, self.nkv, self.cfg.head_dim,

@@ -338,20 +338,22 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                       seq_lens: torch.Tensor, scale: float, work_seq: torch.Tensor = None,
                       work_mblk: torch.Tensor = None,
                       out: Optional[torch.Tensor] = None, k_scale: float = 1.0,
-                      v_scale: float = 1.0) -> torch.Tensor:
+                      v_scale: float = 1.0, max_len: int = 0) -> torch.Tensor:
+    """``max_len``: no sequence is longer (0: not known; the tables' width is taken for it).  It
+    chooses between kernels, and limits nothing."""
     if not _gpu(q):
         return ref.prefill_attention(q, k_cache, v_cache, block_tables, query_start_loc,
                                      seq_lens, scale, k_scale, v_scale)
     if work_seq is None:
-        qsl = query_start_loc.tolist()
-        ws, wm = prefill_work_list([qsl[i + 1] - qsl[i] for i in range(len(qsl) - 1)],
-                                   seq_lens.tolist())
+        qsl, lens = query_start_loc.tolist(), seq_lens.tolist()
+        ws, wm = prefill_work_list([qsl[i + 1] - qsl[i] for i in range(len(qsl) - 1)], lens)
+        max_len = max(lens, default=0)
         work_seq = torch.tensor(ws, dtype=torch.int32, device=q.device)
         work_mblk = torch.tensor(wm, dtype=torch.int32, device=q.device)
     if out is None:
         out = torch.empty_like(q)
     _k().prefill_attention(out, q, k_cache, v_cache, block_tables, query_start_loc, seq_lens,
-                           work_seq, work_mblk, scale, k_scale, v_scale)
+                           work_seq, work_mblk, scale, k_scale, v_scale, max_len)
     return out
 
 
@@ -361,22 +363,23 @@ def prefill_attention_rope(qkv: torch.Tensor, cos_sin: torch.Tensor, k_cache: to
                            num_heads: int, head_dim: int, work_seq: Optional[torch.Tensor] = None,
                            work_mblk: Optional[torch.Tensor] = None,
                            out: Optional[torch.Tensor] = None,
-                           k_scale: float = 1.0, v_scale: float = 1.0) -> torch.Tensor:
+                           k_scale: float = 1.0, v_scale: float = 1.0,
+                           max_len: int = 0) -> torch.Tensor:
     """K2 on a prefill-only step whose q is still the unrotated QKV projection row: NeoX
     RoPE (position = context start + row, as the engine numbers tokens) is applied as the
     kernel loads q, so q is never written or re-read (k / v: ``kv_write_rope``)."""
     T = qkv.shape[0]
     if work_seq is None:
-        qsl = query_start_loc.tolist()
-        ws, wm = prefill_work_list([qsl[i + 1] - qsl[i] for i in range(len(qsl) - 1)],
-                                   seq_lens.tolist())
+        qsl, lens = query_start_loc.tolist(), seq_lens.tolist()
+        ws, wm = prefill_work_list([qsl[i + 1] - qsl[i] for i in range(len(qsl) - 1)], lens)
+        max_len = max(lens, default=0)
         work_seq = torch.tensor(ws, dtype=torch.int32, device=qkv.device)
         work_mblk = torch.tensor(wm, dtype=torch.int32, device=qkv.device)
     if out is None:
         out = torch.empty(T, num_heads, head_dim, dtype=qkv.dtype, device=qkv.device)
     _k().prefill_attention_rope(out, qkv, cos_sin, k_cache, v_cache, block_tables,
                                 query_start_loc, seq_lens, work_seq, work_mblk, num_heads, scale,
-                                k_scale, v_scale)
+                                k_scale, v_scale, max_len)
     return out
 
 
@@ -822,10 +825,11 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if out is None:
         out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
     ws, wb = getattr(meta, "work_seq", None), getattr(meta, "work_mblk", None)
+    max_len = getattr(meta, "prefill_max_len", 0)
     if meta.num_prefills and ws is None:
-        qsl = meta.query_start_loc.tolist()
-        a, b = prefill_work_list([qsl[i + 1] - qsl[i] for i in range(meta.num_prefills)],
-                                 meta.prefill_seq_lens.tolist())
+        qsl, lens = meta.query_start_loc.tolist(), meta.prefill_seq_lens.tolist()
+        a, b = prefill_work_list([qsl[i + 1] - qsl[i] for i in range(meta.num_prefills)], lens)
+        max_len = max(lens)
         ws = torch.tensor(a, dtype=torch.int32, device=q.device)
         wb = torch.tensor(b, dtype=torch.int32, device=q.device)
     _k().window_attention(out, q, k_cache, v_cache, meta.query_start_loc,
@@ -837,7 +841,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                           int(block_size), v_table, interleaved,
                           meta.slot_mapping if pool > 0 else None, chunked,
                           float("-inf") if sink is None else float(sink),
-                          getattr(meta, "decode_max_ctx", 0))
+                          getattr(meta, "decode_max_ctx", 0), max_len)
     return out
 
 

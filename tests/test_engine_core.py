@@ -419,6 +419,36 @@ def test_step_plan_header_carries_the_tp_overlap_split():
     assert q.split == 1 and q.vp == 1 and q.T == 40
 
 
+@pytest.mark.parametrize("split", [False, True])
+def test_prefill_meta_names_its_longest_sequence(monkeypatch, split):
+    """The attention kernels are chosen by the longest sequence of a step, not by the tables' width (max_model_len): the
+    step's metadata has it, and so has each half of a step that is split to overlap its all-reduces."""
+    import torch
+
+    from kubernetes_gpu_cluster_amd.engine.model_runner import ModelRunner
+    from kubernetes_gpu_cluster_amd.models import build_model
+    from kubernetes_gpu_cluster_amd.models.configs import PRESETS
+    from kubernetes_gpu_cluster_amd.parallel.state import ParallelState, set_state
+    set_state(ParallelState())
+    cfg = PRESETS["tiny-llama"]
+    model = build_model(cfg, torch.float32, torch.device("cpu"))
+    runner = ModelRunner(model, cfg, torch.float32, torch.device("cpu"), 16, 256, 4, 128, True)
+    runner.init_kv_cache(48)
+    monkeypatch.setattr(runner, "_overlap_ok", lambda Tp: split)
+    bm = BlockManager(48, 16, 4, runner.max_blocks)
+    seqs = [_seq(str(i), n) for i, n in enumerate((7, 60, 11))]
+    for sq in seqs:
+        bm.allocate(sq, len(sq.prompt_token_ids))
+    seqs[1].num_computed = 40                      # 20 of its rows after 40
+    chunks = [(sq, len(sq.prompt_token_ids) - sq.num_computed) for sq in seqs]
+    plan, _ = runner.build_plan(chunks, [], bm.table)
+    runner._upload(plan)
+    m = runner._meta(plan.T, plan.Tp, plan.P, plan.D, plan.W, plan.max_ctx, split=plan.split)
+    metas = [m] + (list(m.split[1:]) if split else [])
+    assert plan.split == int(split) and m.prefill_max_len == 60 and m.prefill_block_tables.shape[1] * 16 == 256
+    assert [x.prefill_max_len for x in metas] == [int(x.prefill_seq_lens.max()) for x in metas]
+
+
 def test_memory_profile_covers_many_short_prompts():
     """The step that sizes the KV pool: the longest prompts, and for recurrent layers (whose
     chunkwise scans keep a workspace per sequence and started chunk) as many prompts as there

@@ -2,6 +2,7 @@
 (``ops.reference``), op by op, in bf16 and fp32, on sizes that are not multiples of the
 wave (odd head sizes, several norm groups, chunks that continue a slot's state)."""
 import math
+import re
 import types
 
 import pytest
@@ -654,6 +655,42 @@ def test_window_attention_shared_tiles(gpu, dt, H, G, latent, bs, kw):
                                0.08, args[1], args[2], gate.to(gpu), elem_gate=eg.to(gpu), out_scale=1.3, **kw)
     ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
+
+
+def _window_forms(f):
+    """Forms of the shared-tile prompt kernel (0: 64 rows, 1: 32 rows, 2: 32 rows and two groups of waves) in a call."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        f()
+        torch.cuda.synchronize()
+    keys = [e.key for e in prof.key_averages() if "window_prefill_gqa_kernel" in e.key]
+    return [int(re.search(r"(?:ELi|, )(\d)(?:EE|>)", k).group(1)) for k in keys]
+
+
+@pytest.mark.parametrize("latent", [False, True])
+@pytest.mark.parametrize("n,L,old,window,form", [
+    (1, 30, 0, 0, (0, 1)), (4, 64, 0, 0, (1, 1)), (2, 150, 0, 1024, (0, 1)), (1, 20, 300, 0, (2, 2)),       # up to one round of 32 rows
+    (16, 140, 0, 0, (0, 0)), (5, 700, 0, 0, (2, 2)), (4, 700, 0, 1024, (0, 0)),                            # up to two
+    (40, 100, 0, 0, (1, 1)), (24, 300, 0, 1024, (0, 1)), (10, 512, 0, 0, (0, 1)), (12, 300, 0, 1024, (1, 1))])
+def test_window_attention_forms_by_length(gpu, latent, n, L, old, window, form):
+    """Tables as wide as a service's longest request take no other form than tables of the sequences' own width where
+    the step's longest sequence is named; form: of heads with keys and values of their own, of latent rows."""
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("forms for 256 CUs")
+    bs, H, G, dk, dv = 32, 16, *((1, 256, 192) if latent else (4, 128, 128))
+    width = -(-(L + old) // bs)
+    kc = torch.zeros(n * width, G, bs, dk, dtype=torch.bfloat16, device=gpu)
+    vc = kc[..., :dv] if latent else torch.zeros_like(kc)
+    tables = torch.arange(n * width, dtype=torch.int32).view(n, width)
+    wide = torch.cat([tables, tables[:, :1].expand(-1, 256)], 1).contiguous()
+    q = torch.zeros(n * L, H, dk, dtype=torch.bfloat16, device=gpu)
+    pos = torch.arange(old, old + L, device=gpu).repeat(n)
+
+    def run(t, longest):
+        m = _to(_meta([L] * n, [L + old] * n, [], t), gpu)
+        m.prefill_max_len = longest
+        m.work_seq, m.work_mblk = (torch.tensor(x, dtype=torch.int32, device=gpu) for x in ops.prefill_work_list([L] * n, [L + old] * n))
+        return _window_forms(lambda: ops.window_attention(q, kc, vc, pos, m, 0.08, window, 0))
+    assert run(tables, 0) == run(wide, L + old) == [form[latent]]
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])

@@ -1807,6 +1807,31 @@ def test_prefill_walk_two_groups(gpu, monkeypatch, dt, nq, nkv, bs, query_lens, 
     torch.testing.assert_close(two.float(), one.float(), atol=unit * float(vc.abs().max()), rtol=2 * unit)
 
 
+@pytest.mark.parametrize("n,L,walk", [(2, 64, False), (1, 30, False), (1, 129, True), (1, 512, True)])
+def test_prefill_walk_by_length(gpu, monkeypatch, n, L, walk):
+    """Tables as wide as a service's longest request take no other kernel than tables of the sequences' own width where
+    the step's longest sequence is named, or its work list is made here."""
+    monkeypatch.delenv("KGC_PREFILL_PERSIST", raising=False)
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("lines for 256 CUs")
+    nq, nkv, bs, d = 32, 8, 32, 128
+    kc, vc, bt = _fill_random_cache(n, [L] * n, nkv, bs, d, torch.bfloat16, gpu)
+    bt = bt[:, : -(-L // bs)].contiguous()
+    wide = torch.cat([bt, bt[:, :1].expand(-1, 256)], 1).contiguous()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)   # noqa: E731
+    qsl, sl = i32([0] + [L] * n).cumsum(0).int(), i32([L] * n)
+    ws, wm = map(i32, ops.prefill_work_list([L] * n, [L] * n))
+    q = torch.randn(n * L, nq, d, dtype=torch.bfloat16, device=gpu)
+
+    def walks(*a, **kw):
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+            ops.prefill_attention(q, kc, vc, *a, **kw)
+            torch.cuda.synchronize()
+        return any("prefill_attn_walk_kernel" in e.key for e in prof.key_averages())
+    scale = d ** -0.5
+    assert [walks(bt, qsl, sl, scale, ws, wm), walks(wide, qsl, sl, scale, ws, wm, max_len=L), walks(wide, qsl, sl, scale)] == [walk] * 3
+
+
 @pytest.mark.parametrize("query_lens,seq_lens", [([129], [129]), ([33, 100, 1, 32], [161, 1000, 65, 800]), ([1100], [1100])])
 def test_prefill_walk_two_groups_low_scores(gpu, monkeypatch, query_lens, seq_lens):
     """Scores that are all below -1e30 (exactly -k 2^100, k of 1 to 1.75; a scale of ln 2 leaves them as exponents of 2):
