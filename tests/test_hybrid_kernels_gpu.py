@@ -695,20 +695,21 @@ def test_window_attention_forms_by_length(gpu, latent, n, L, old, window, form):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("latent", [False, True])
-@pytest.mark.parametrize("n,bs,kw", [
-    (9, 4, dict(window=200, keep=70)), (9, 32, dict(window=0, keep=0, softcap=20.0)),      # every other tile each
-    (9, 6, dict(window=256, keep=0, chunked=True, sink=0.4)),
-    (4, 32, dict(window=60, keep=3)),                                                     # 32 rows, few tiles
-    (130, 2, dict(window=90, keep=66)), (130, 16, dict(window=0, keep=0))])               # 32 rows, two workgroups to a CU
-def test_window_attention_forms(gpu, dt, latent, n, bs, kw):
+@pytest.mark.parametrize("n,bs,kw,forms", [
+    (9, 4, dict(window=200, keep=70), (2, 2)), (9, 32, dict(window=0, keep=0, softcap=20.0), (2, 2)),      # every other tile each
+    (9, 12, dict(window=256, keep=0, chunked=True, sink=0.4), (2, 2)),
+    (4, 32, dict(window=60, keep=3), (0, 1)), (4, 32, dict(window=60, keep=3, rows=60), (1, 1)),           # 32 rows, few tiles
+    (130, 4, dict(window=90, keep=66, rows=60), (1, 1)), (130, 20, dict(window=0, keep=0), (0, 1))])       # two workgroups to a CU
+def test_window_attention_forms(gpu, dt, latent, n, bs, kw, forms):
     """Prompt rows where workgroups own 32 rows, two groups of waves share the tiles or one has them all: windows
     that begin between the rows that are copied together, tiles of kept tokens, odd and even numbers of tiles,
-    one row to 70, tables that end inside a tile (what lay in LDS there before is not finite).  Calls that
-    only differ in pages of a row less have the same bits where no two groups share the tiles; the bound is
-    the shared tiles'."""
+    one row to 70, tables that end inside a tile (what lay in LDS there before is not finite).  Calls in
+    pages of a row less, which are of 64 rows for want of whole copies, have the same bits where no two groups share
+    the tiles; the bound is the shared tiles'."""
     torch.manual_seed(41)
     H, dk, dv = 4, *((256, 192) if latent else (128, 128))
-    P_q = [1 + (i * 23) % (70 if n < 100 else 7) for i in range(n)]
+    q_rows, kw = kw.get("rows"), {k: v for k, v in kw.items() if k != "rows"}
+    P_q = [q_rows + i % 3 if q_rows else 1 + (i * 23) % (70 if n < 100 else 7) for i in range(n)]
     old = [(i * 61) % (600 if n == 9 else 130) for i in range(n)]
     P_sl, T = [a + b for a, b in zip(P_q, old)], sum(P_q)
     pos = torch.cat([torch.arange(o, o + a) for a, o in zip(P_q, old)])
@@ -741,7 +742,10 @@ def test_window_attention_forms(gpu, dt, latent, n, bs, kw):
     got = run(bs, gpu)
     ulp = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -10       # neighbours where rounding differs
     torch.testing.assert_close(got.cpu().float(), want.float(), rtol=1.01 * ulp, atol=2e-4)
+    if torch.cuda.get_device_properties(gpu).multi_processor_count == 256:
+        assert _window_forms(lambda: run(bs, gpu)) == [forms[latent]]
     if n != 9:
+        assert _window_forms(lambda: run(bs - 1, gpu)) == [0]
         assert torch.equal(got, run(bs - 1, gpu))
 
 
