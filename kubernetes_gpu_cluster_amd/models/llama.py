@@ -350,7 +350,7 @@ class LlamaForCausalLM(nn.Module):
             for i in (0, 1):
                 pend[i].wait()
                 xi, res[i] = ops.fused_add_rms_norm(h[i], res[i], ln2.weight, ln2.eps)
-                d = gemm.linear(gemm.linear_silu(xi, gu.weight, gu.bias),
+                d = gemm.linear(gemm.linear_silu(xi, gu.weight, gu.bias, cus_shared=True),
                                 layer.mlp.down_proj.weight)
                 h[i], pend[i] = d, comm.tp_all_reduce_async(d)
             prev = layer

@@ -196,11 +196,17 @@ def _dg_plan(x: torch.Tensor, w: torch.Tensor, kind: str):
     return p
 
 
-def linear_silu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+def linear_silu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                cus_shared: bool = False) -> torch.Tensor:
     """silu_mul(linear(x, w, bias)) over a merged gate_up weight: where the plan runs K9m
     at this (M, N, K) the activation is the GEMM's epilogue (S = 1) or rides the split-K
     reduction (``splitk_reduce_silu``), so the [M, 2I] gate_up output never exists; nor
-    does it for prompt rows (csrc/kernels/gemm_prompt.hip)."""
+    does it for prompt rows (csrc/kernels/gemm_prompt.hip).
+
+    ``cus_shared``: another stream's kernel (a collective) holds some of the CUs meanwhile.  Prompt rows
+    then stay with the library: the kernel for them deals its tiles to one workgroup per CU, and those whose
+    CU is held run after the others.  With 16 CUs held, 4096 -> 2 x 3584, 8192 rows: library 366 us, that
+    kernel 574 (350 with all CUs for itself); 8192 -> 2 x 3584, 1024 rows 114, 175 (119)."""
     from . import _k, silu_mul
     if bias is None and x.is_cuda and x.dim() == 2 and x.stride(1) == 1 and _plan_silu:
         cfg = _plan_silu.get((x.shape[0], w.shape[0], w.shape[1]))
@@ -216,7 +222,7 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
             out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype, device=x.device)
             _k().splitk_reduce_silu(out, ws, _dg_info(cfg)[2])
             return out
-        if _prompt_pays(x, w, True):
+        if not cus_shared and _prompt_pays(x, w, True):
             out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype, device=x.device)
             _k().prompt_silu(out, x, w)
             return out

@@ -18,6 +18,34 @@ def test_linear_silu_fallback_matches_layer_math():
     torch.testing.assert_close(gemm.linear_silu(x, w), exp, atol=1e-5, rtol=1e-5)
 
 
+def test_projection_beside_a_collective_stays_with_the_library(monkeypatch):
+    """A prefill step in two halves runs one half's feed-forward while the other's all-reduce holds CUs: the kernel
+    that deals the projection's tiles to all CUs in advance is not asked for there, and is elsewhere."""
+    from types import SimpleNamespace
+
+    from kubernetes_gpu_cluster_amd.models import configs
+    from kubernetes_gpu_cluster_amd.models import llama
+    asked, shared = [], []
+    monkeypatch.setattr(gemm, "_prompt_pays", lambda x, w, silu: asked.append(silu))
+    x, w = torch.randn(70, 64), torch.randn(96, 64) * 0.1
+    same = gemm.linear_silu(x, w, cus_shared=True)
+    assert not asked and torch.equal(gemm.linear_silu(x, w), same) and asked == [True]
+
+    cfg = configs.PRESETS["tiny-llama"]
+    m = llama.LlamaForCausalLM(cfg, torch.float32, torch.device("cpu"))
+    for p in m.parameters():
+        torch.nn.init.normal_(p, std=0.02)
+    real = gemm.linear_silu
+    monkeypatch.setattr(gemm, "linear_silu", lambda *a, cus_shared=False: shared.append(cus_shared) or real(*a, cus_shared=cus_shared))
+    monkeypatch.setattr(llama.comm, "tp_all_reduce_async", lambda t: SimpleNamespace(wait=lambda: None))
+    monkeypatch.setattr(llama.LlamaAttention, "attend", lambda self, pos, qkv, ctx, *a: qkv[:, : self.nq * cfg.head_dim])
+    halves = (10, SimpleNamespace(), SimpleNamespace())
+    ctx = llama.ForwardContext(SimpleNamespace(split=halves), [])
+    with torch.inference_mode():
+        m._forward_tp_overlap(torch.arange(20), torch.randn(20, cfg.hidden_size), ctx)
+    assert shared == [True] * 2 * cfg.num_layers and asked == [True]
+
+
 def test_linear_add_rms_fallback_matches_layer_math():
     torch.manual_seed(1)
     x = torch.randn(7, 32)
