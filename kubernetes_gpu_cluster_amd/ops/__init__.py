@@ -562,12 +562,14 @@ def moe_dgemm_splitk(npairs: int, E: int, N: int, K: int, bm: int, bn: int = 128
     times N/bn column tiles times S near one workgroup per CU, each slice >= 8 K-steps
     (KGC_MOE_SPLITK overrides, as for the register-staged kernel).
 
-    Where every expert has rows, and by the blocks that they then take, up to two rounds of workgroups with slices
-    of 48 steps or more: one for half of the CUs reads 4.5 TB/s, and a round's end leaves CUs idle for less long.  Top 2,
-    weights from memory, us a call: 8 experts of 4096 x 14336, 8, 64, 128, 256, 512, 700 rows 442 -> 435, 484 -> 470, 508 -> 464,
-    512 -> 476, 865 -> 793, 1230 -> 1113; 16 of 4096 x 6400, 64, 512 rows 441 -> 437, 523 -> 474.  Shorter slices cost what they
-    save: 8 of 4096 x 3584, 256, 512 rows 140 -> 148, 247 -> 272, 8 of 2048 x 5504, 64 rows 110 -> 118; and so do more rounds: 8 of
-    4096 x 14336, 256 rows in 8 slices 495."""
+    Where every expert has rows, and by the blocks that they then take, slices that make two full rounds of workgroups
+    on 256 CUs, of 48 steps or more: one for half of the CUs reads 4.5 TB/s, and a round's end leaves CUs idle for less long.  Top
+    2, weights from memory, us a call: 8 experts of 4096 x 14336, 8, 64, 128, 256, 512, 700 rows 443 -> 434, 485 -> 475, 508 -> 465,
+    509 -> 476, 863 -> 803, 1235 -> 1123; 4 of them, 300 rows 615 -> 547; 16 of 4096 x 6400, 17, 64, 512 rows 342 -> 346, 415 -> 412,
+    519 -> 472.  One round, or one and a half, costs more than it saves: 8 of 4096 x 7168 in 2 slices (256 workgroups), 256, 300
+    rows 263 -> 279, 284 -> 313; 8 of 6144 x 16384 in 2 (384), 8, 64, 400 rows 694 -> 739, 837 -> 857, 952 -> 1038; and so do more
+    rounds or shorter slices: 8 of 4096 x 14336, 256 rows in 8 slices 495, 8 of 5120 x 14336 in 4 (640), 400 rows 689 -> 721, 8 of
+    4096 x 3584, 512 rows 247 -> 272."""
     if os.environ.get("KGC_MOE_SPLITK") is not None:
         return max(1, int(os.environ["KGC_MOE_SPLITK"]))
     blocks = min((npairs + bm - 1) // bm + E, max(1, npairs))
@@ -578,8 +580,7 @@ def moe_dgemm_splitk(npairs: int, E: int, N: int, K: int, bm: int, bn: int = 128
     mean = npairs / max(1, E)
     if mean >= 2:
         wgs = E * math.ceil((mean + mean ** 0.5) / bm) * (N // bn)
-        while S < 16 and wgs * S * 2 <= 640 and K // 64 // (2 * S) >= 48:
-            S *= 2
+        S = max([S] + [n for n in (2, 4, 8, 16) if 448 <= wgs * n <= 512 and K // 64 // n >= 48])
     return S
 
 

@@ -321,9 +321,11 @@ int main() {
     (8, 4096, 14336, 1, 8), (8, 4096, 14336, 6, 2),                   # few pairs: near one workgroup per CU, as ever
     (8, 4096, 14336, 8, 4), (8, 4096, 14336, 256, 4), (8, 4096, 14336, 700, 2), (8, 4096, 14336, 2048, 1),
     (16, 4096, 6400, 8, 1), (16, 4096, 6400, 512, 2),
-    (8, 4096, 3584, 256, 1), (32, 2048, 1408, 64, 1), (1, 256, 1 << 20, 64, 16)])
+    (8, 4096, 3584, 256, 1), (32, 2048, 1408, 64, 1), (1, 256, 1 << 20, 64, 16),
+    (4, 4096, 14336, 300, 4), (4, 4096, 14336, 100, 2), (8, 6144, 16384, 64, 1),      # less than two rounds, and more: as ever
+    (8, 4096, 7168, 256, 1), (8, 5120, 14336, 64, 1), (8, 2048, 8192, 1000, 1)])
 def test_expert_down_projection_slices(monkeypatch, E, N, K, rows, want):
-    """K-slices of the experts' down projection (top 2, column tiles of 256): up to two rounds of workgroups
+    """K-slices of the experts' down projection (top 2, column tiles of 256): two full rounds of workgroups
     where every expert has rows and a slice keeps 48 steps."""
     from kubernetes_gpu_cluster_amd import ops
     monkeypatch.delenv("KGC_MOE_SPLITK", raising=False)
