@@ -305,7 +305,7 @@ void prefill_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Ten
                                 v_cache.data_ptr(), block_tables.data_ptr<int>(),
                                 (int)block_tables.stride(0), query_start_loc.data_ptr<int>(),
                                 seq_lens.data_ptr<int>(), work_seq.data_ptr<int>(),
-                                work_mblk.data_ptr<int>(), (int)work_seq.numel(), (int)P, max_len, (int)nq,
+                                work_mblk.data_ptr<int>(), (int)work_seq.numel(), {(int)P, out.size(0), max_len}, (int)nq,
                                 (int)k_cache.size(1), (int)d,
                                 log2_exact(k_cache.size(2), "block_size"), (float)scale,
                                 k_cache.scalar_type() == at::kFloat8_e4m3fn, (float)k_scale,
@@ -346,7 +346,7 @@ void prefill_attention_rope(Tensor out, Tensor qkv, Tensor cos_sin, Tensor k_cac
                                 v_cache.data_ptr(), block_tables.data_ptr<int>(),
                                 (int)block_tables.stride(0), query_start_loc.data_ptr<int>(),
                                 seq_lens.data_ptr<int>(), work_seq.data_ptr<int>(),
-                                work_mblk.data_ptr<int>(), (int)work_seq.numel(), (int)P, max_len, (int)nq,
+                                work_mblk.data_ptr<int>(), (int)work_seq.numel(), {(int)P, out.size(0), max_len}, (int)nq,
                                 (int)nkv, (int)d, log2_exact(k_cache.size(2), "block_size"),
                                 (float)scale, k_cache.scalar_type() == at::kFloat8_e4m3fn,
                                 (float)k_scale, (float)v_scale, (int)k_cache.size(0),

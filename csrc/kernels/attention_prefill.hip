@@ -22,6 +22,7 @@
 #include "common.h"
 #include "device.h"
 #include "launch.h"
+#include "prefill_items.h"
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -857,8 +858,7 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
 // K and V tiles come by DMA into two buffers each, in the order in which the MFMAs read them: unit c of key k at
 // c ^ f(k), V^T in groups of 8 keys as the cache has them; one barrier per tile.  A tile is asked for while the one before
 // it computes, its pages a tile before that, the next item's q in registers.  What only items need is read again from the
-// arguments: there are no scalar registers left for it.  Neighbouring items are the kv heads of the same rows, so that with
-// 8 of them an XCD sees one in all rounds.
+// arguments: there are no scalar registers left for it.  The order of the items: prefill_items.h.
 //
 // What bounds it: latency.  Of a tile's 5500 cycles (two waves per SIMD) 2050 are the matrix core's and 1900 vector
 // instructions'; a fifth is the barrier (four waves, each beside another workgroup's), and at 32 x 512 rows the rotation
@@ -879,12 +879,12 @@ struct WalkArgs {
 // end (the rule: at the launch).
 template <typename T, int D, int GR>
 __global__ __launch_bounds__(256 * GR, 2) void prefill_attn_walk_kernel(const WalkArgs) {
-  static_assert(D == 128 && PF_BN == 64 && sizeof(T) == 2, "rows and groups per DMA");
+  static_assert(D == 128 && PF_BN == 64 && sizeof(T) == 2 && PF_BM == 32 * WALK_BLOCKS, "rows and groups per DMA");
   typedef typename Vec8<T>::type V8;
   typedef __attribute__((address_space(3))) void* LdsPtr;
   typedef const __attribute__((address_space(4))) WalkArgs* ArgPtr;
   typedef const __attribute__((address_space(4))) int* ScalarPtr;
-  constexpr int GH = 4, QB = 32, ZS = PF_BM / QB, KS = D / 32, DT = D / 16, RB = D * 2;   // RB: bytes of a row
+  constexpr int GH = 4, QB = 32, KS = D / 32, DT = D / 16, RB = D * 2;   // RB: bytes of a row
   // (objects of their own: the compiler lets an LDS read follow every DMA into the object that it reads)
   constexpr int TE = PF_BN * D;              // elements of a tile
   __shared__ __attribute__((aligned(16))) T K0[GR * TE], K1[GR * TE], V0[GR * TE], V1[GR * TE], all_rows[4 * 16 * D];
@@ -916,14 +916,16 @@ __global__ __launch_bounds__(256 * GR, 2) void prefill_attn_walk_kernel(const Wa
   auto decode = [&](int idx, Item& I) -> bool {
     const ArgPtr a = args();
     const int nkv = a->nkv, G = a->nq / nkv, Y = nkv * (G / GH), bs_log2 = a->bs_log2;
-    const int w = idx / (Y * ZS), r = idx - w * (Y * ZS), z = r / Y, y = r - z * Y, h = y / (G / GH);
+    int w, z, y;
+    walk_item(idx, Y, w, z, y);
+    const int h = y / (G / GH);
     const int seq = ((ScalarPtr)a->work_seq)[w], mb = ((ScalarPtr)a->work_mblk)[w];
     const int q0 = ((ScalarPtr)a->qsl)[seq], qlen = ((ScalarPtr)a->qsl)[seq + 1] - q0;
     int L_in = ((ScalarPtr)a->seq_lens)[seq];
     const int cap = a->bt_stride << bs_log2;
     KGC_DCHECK_RANGE(L_in, 0, cap + 1, "prefill seq_len");
     I.L = min(L_in, cap);
-    const int ctx0 = I.L - qlen, qbase = mb * PF_BM + (ZS - 1 - z) * QB;
+    const int ctx0 = I.L - qlen, qbase = mb * PF_BM + z * QB;
     if (qlen <= 0 || ctx0 < 0 || qbase >= qlen) return false;
     I.row0 = q0 + qbase;
     I.nrow = min(qlen - qbase, QB);
@@ -936,12 +938,11 @@ __global__ __launch_bounds__(256 * GR, 2) void prefill_attn_walk_kernel(const Wa
     I.v = static_cast<const char*>(a->vc) + at;
     return true;
   };
-  // rounds of items, alternating direction (as the 8-wave walk's)
   const int G_ = gridDim.x, b_ = blockIdx.x, n_items = args()->n_items;
-  const int turn = G_ % 8 == 0 ? (G_ - 8 - (b_ & ~7)) | (b_ & 7) : G_ - 1 - b_;
+  const bool by_xcd = args()->nq / GH % 8 == 0;
   auto next_valid = [&](int r, Item& I) -> int {
     while (r * G_ < n_items) {
-      const int idx = r * G_ + ((r & 1) ? turn : b_);
+      const int idx = walk_index(r, b_, G_, by_xcd);
       if (idx < n_items && decode(idx, I)) break;
       ++r;
     }
@@ -1188,7 +1189,7 @@ static int prefill_persist_mode() {
 template <typename T, int D, bool KV8, int GH>
 static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const void* vc,
                                  const int* bt, int bt_stride, const int* qsl, const int* sl,
-                                 const int* ws, const int* wm, int n_work, int n_seq, int64_t max_len, int nq, int nkv,
+                                 const int* ws, const int* wm, int n_work, const PromptShape& ps, int nq, int nkv,
                                  int bs_log2, float scale_log2, float v_scale, int num_blocks,
                                  int64_t q_stride, const float* cos_sin, int cs_rows, hipStream_t s) {
   constexpr size_t lds = 2 * 2 * PF_BN * D * sizeof(T);
@@ -1200,11 +1201,12 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
   const bool dma = aligned(q) && q_stride % 8 == 0;    // 16-byte DMAs
   if constexpr (!KV8) {
     // Few rows of short sequences are one tile each, for which the walk has nothing to overlap (K / V write included, one-shot grid
-    // -> walk, us: 2 x 64 rows 14.5 -> 15.6, 1 x 30 16.3 -> 17.2, 8 x 128 20.2 -> 20.1); all else is faster so: 512 rows 31.1 -> 23.2, 1000
-    // 51.9 -> 39.1, 2000 after 2000 164 -> 128, 8 x 100 after 3000 127 -> 98, 4 x 300 30.1 -> 27.5.
+    // -> walk, us: 2 x 64 rows 14.5 -> 15.6, 1 x 30 16.3 -> 17.2, 8 x 128 20.2 -> 20.1; of many, those of up to 48 rows below 5
+    // items per CU: attention alone 20 x 32 9.1 -> 9.8, 32 x 40 10.1 -> 10.7, 48 x 40 16.9 -> 15.9); all else is faster so: 512 rows
+    // 31.1 -> 23.2, 1000 51.9 -> 39.1, 2000 after 2000 164 -> 128, 8 x 100 after 3000 127 -> 98, 4 x 300 30.1 -> 27.5.
     const int64_t n = (int64_t)n_work * nkv * (G / 4) * (PF_BM / 32);
-    const int64_t table = (int64_t)bt_stride << bs_log2, length = max_len > 0 ? std::min(max_len, table) : table;
-    const bool pays = n > 2 * n_cu || length > 128;
+    const int64_t table = (int64_t)bt_stride << bs_log2, length = ps.max_len > 0 ? std::min(ps.max_len, table) : table;
+    const bool pays = length > 128 || (n > 2 * n_cu && (n > 5 * n_cu || ps.rows > (int64_t)48 * ps.seqs));
     if (dma && aligned(kc) && aligned(vc) && aligned(out) && bs_log2 >= 5 && (mode < 0 ? pays : mode != 0) &&
         n < ((int64_t)1 << 30) && q_stride < (1 << 24) && (int64_t)nq * D < (1 << 24) &&
         ((int64_t)nkv * D << bs_log2) < ((int64_t)1 << 31)) {       // offsets inside an item and a page in 32 bits
@@ -1214,7 +1216,7 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
       // tiles outlasts the others.  us, one group -> two: 512 rows 27.8 -> 24.8, 1000 39.2 -> 33.0, 300 after 3000 85 -> 62, 4 x 200
       // after 1000 43.4 -> 36.9, 1500 52.6 -> 44.0, 2000 65.0 -> 58.3, 2000 after 2000 125 -> 116; other prompts beyond one item per CU 6 x 256
       // 28.3 -> 33.9, 4 x 500 after 1000 64.7 -> 65.8, 12 x 100 after 1000 56 -> 60; 16 x 128 28.9 -> 34.7, 4096 160 -> 170.
-      if (mode < 0 && n <= (n_seq == 1 ? 2 : 1) * n_cu) prefill_attn_walk_kernel<T, D, 2><<<(int)n, 512, 0, s>>>(a);
+      if (mode < 0 && n <= (ps.seqs == 1 ? 2 : 1) * n_cu) prefill_attn_walk_kernel<T, D, 2><<<(int)n, 512, 0, s>>>(a);
       else prefill_attn_walk_kernel<T, D, 1><<<(int)std::min<int64_t>(n, 2 * n_cu), 256, 0, s>>>(a);
       return;
     }
@@ -1238,17 +1240,17 @@ static void prefill_gqa_dispatch(const void* q, void* out, const void* kc, const
 template <typename T, int D, bool KV8>
 static void prefill_dispatch(const void* q, void* out, const void* kc, const void* vc,
                              const int* bt, int bt_stride, const int* qsl, const int* sl,
-                             const int* ws, const int* wm, int n_work, int n_seq, int64_t max_len, int nq, int nkv,
+                             const int* ws, const int* wm, int n_work, const PromptShape& ps, int nq, int nkv,
                              int bs_log2, float scale_log2, float v_scale, int num_blocks,
                              int64_t q_stride, const float* cos_sin, int cs_rows, hipStream_t s) {
   const int G = nkv > 0 ? nq / nkv : 1;
   if constexpr (D == 128) if (prefill_gqa_enabled() && nq % nkv == 0 && (G == 4 || G % 8 == 0)) {
     if (G == 4)
-      prefill_gqa_dispatch<T, D, KV8, 4>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, n_seq, max_len,
+      prefill_gqa_dispatch<T, D, KV8, 4>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, ps,
                                          nq, nkv, bs_log2, scale_log2, v_scale, num_blocks,
                                          q_stride, cos_sin, cs_rows, s);
     else
-      prefill_gqa_dispatch<T, D, KV8, 8>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, n_seq, max_len,
+      prefill_gqa_dispatch<T, D, KV8, 8>(q, out, kc, vc, bt, bt_stride, qsl, sl, ws, wm, n_work, ps,
                                          nq, nkv, bs_log2, scale_log2, v_scale, num_blocks,
                                          q_stride, cos_sin, cs_rows, s);
     return;
@@ -1262,7 +1264,7 @@ static void prefill_dispatch(const void* q, void* out, const void* kc, const voi
 void launch_prefill_attention(int dtype, const void* q, void* out, const void* k_cache,
                               const void* v_cache, const int* block_tables, int bt_stride,
                               const int* query_start_loc, const int* seq_lens,
-                              const int* work_seq, const int* work_mblk, int n_work, int n_seq, int64_t max_len, int nq,
+                              const int* work_seq, const int* work_mblk, int n_work, const PromptShape& ps, int nq,
                               int nkv, int D, int bs_log2, float scale, bool kv_fp8,
                               float k_scale, float v_scale, int num_blocks, int64_t q_stride,
                               const float* cos_sin, int cs_rows, hipStream_t s) {
@@ -1270,7 +1272,7 @@ void launch_prefill_attention(int dtype, const void* q, void* out, const void* k
   const float sl2 = scale * k_scale * 1.4426950408889634f;
 #define KGC_PF(TT, DD, K8)                                                                 \
   prefill_dispatch<TT, DD, K8>(q, out, k_cache, v_cache, block_tables, bt_stride,          \
-                               query_start_loc, seq_lens, work_seq, work_mblk, n_work, n_seq, max_len, \
+                               query_start_loc, seq_lens, work_seq, work_mblk, n_work, ps, \
                                nq, nkv, bs_log2, sl2, v_scale, num_blocks, q_stride, cos_sin, cs_rows, s)
 #define KGC_PF_D(TT, K8) \
   if (D == 128) KGC_PF(TT, 128, K8); else KGC_PF(TT, 64, K8)

@@ -59,11 +59,15 @@ void launch_paged_decode_rope(int dtype, const DecodeRope& rp, void* out, void* 
                               float* tmp_out, int B, int nq, int nkv, int D, int bs_log2,
                               int Z, float scale, bool kv_fp8, float k_scale, float v_scale,
                               int num_blocks, hipStream_t s);
-// (max_len: no sequence is longer, 0 where that is not known)
+// what the host knows of a step's prompts: sequences, their rows, and a length that none exceeds (0: not known)
+struct PromptShape {
+  int seqs;
+  int64_t rows, max_len;
+};
 void launch_prefill_attention(int dtype, const void* q, void* out, const void* k_cache,
                               const void* v_cache, const int* block_tables, int bt_stride,
                               const int* query_start_loc, const int* seq_lens,
-                              const int* work_seq, const int* work_mblk, int n_work, int n_seq, int64_t max_len, int nq,
+                              const int* work_seq, const int* work_mblk, int n_work, const PromptShape& ps, int nq,
                               int nkv, int D, int bs_log2, float scale, bool kv_fp8,
                               float k_scale, float v_scale, int num_blocks, int64_t q_stride,
                               const float* cos_sin, int cs_rows, hipStream_t s);
@@ -356,11 +360,6 @@ void launch_window_split(int dtype, void* out, const void* q, const void* k_cach
                          int keep_first, const float* gate, const WindowExtra& ex, int Z, float* work,
                          hipStream_t s);
 bool window_prefill_mfma_ok(int dtype, int dk, int dv);
-// what the host knows of a step's prompts: sequences, their rows, and a length that none exceeds (0: not known)
-struct PromptShape {
-  int seqs;
-  int64_t rows, max_len;
-};
 // false: not its shape
 bool launch_window_prefill_gqa(int dtype, void* out, const void* q, const void* kc, const void* vc,
                                const int* qsl, const int* seq_lens, const int* pbt, int bt_stride,

@@ -289,6 +289,57 @@ def test_decode_graphs_have_few_empty_slices():
     assert [ops.decode_grid_z(4, 8, c, capacity=True) for c in (544, 2048, 8192)] == [8, 8, 32]
 
 
+def test_order_of_the_prompts_items(tmp_path):
+    """The paged prompts' walk has every block of every work item and head group once; and where only the first blocks
+    of the work items have rows (short prompts), every XCD has its share of them, and so has a workgroup in two rounds."""
+    _run(tmp_path, """
+#include <algorithm>
+#include <cstdlib>
+#include <initializer_list>
+#include <set>
+#include <tuple>
+#include <vector>
+#define __host__
+#define __device__
+#include "prefill_items.h"
+#define CHECK(x) if (!(x)) return __LINE__
+int main() {
+  for (int groups : {1, 2, 3, 4, 6, 8, 16})
+    for (int works : {1, 7, 100, 256})
+      for (int grid : {96, 200, 512}) {
+        const int n = works * groups * kgc::WALK_BLOCKS;
+        std::set<std::tuple<int, int, int>> seen;
+        for (int r = 0; r * grid < n; ++r)
+          for (int b = 0; b < grid; ++b) {
+            const int i = kgc::walk_index(r, b, grid, groups % 8 == 0);
+            if (i >= n) continue;
+            int w, block, g;
+            kgc::walk_item(i, groups, w, block, g);
+            CHECK(w >= 0 && w < works && block >= 0 && block < kgc::WALK_BLOCKS && g >= 0 && g < groups);
+            seen.insert(std::make_tuple(w, block, g));
+          }
+        CHECK((int)seen.size() == n);
+      }
+  for (int groups : {1, 2, 4, 8})
+    for (int blocks : {1, 2, 3}) {
+      const int grid = 512, works = 2 * grid / (groups * kgc::WALK_BLOCKS);       // two rounds
+      std::vector<int> of_wg(grid), of_xcd(8);
+      for (int r = 0; r < 2; ++r)
+        for (int b = 0; b < grid; ++b) {
+          int w, block, g;
+          kgc::walk_item(kgc::walk_index(r, b, grid, groups % 8 == 0), groups, w, block, g);
+          const bool rows = block < blocks;
+          of_wg[b] += rows, of_xcd[b & 7] += rows;
+        }
+      for (int x : of_xcd) CHECK(x == works * groups * blocks / 8);
+      const auto most = std::max_element(of_wg.begin(), of_wg.end());
+      CHECK(*most <= (blocks + 1) / 2);
+    }
+  return 0;
+}
+""")
+
+
 def test_order_of_the_experts_blocks(tmp_path):
     """Column tiles first where that was measured faster.  The down projection of more than 16 experts (33.3 -> 38.4 us) and
     gate_up of few experts in more than one round of workgroups (123 -> 137) went so, too."""
