@@ -420,9 +420,11 @@ void launch_gla_scan(int dtype, float* out, const void* proj, int64_t ps, const 
   if (P == 0 && V % 4 == 0 && reinterpret_cast<uintptr_t>(S) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(out) % 16 == 0) {
     const dim3 grid(D, H, (V + 63) / 64);
-    // States of 128 MB and more are read and written past the caches (whole lines, once a step; the last-level cache has 256
-    // MB): 128 rows of 8 heads of 128 x 256 64.3 -> 53.4 us, 256 119 -> 107.  Smaller ones may still lie there from the
-    // step before: 64 rows on three sets of states in turn 25.8 -> 28.2 (on twelve, from memory, 35.1 -> 28.4).
+    // States of 128 MB and more are read and written past the caches: whole lines, once a step, and a model's other layers
+    // pass through the last-level cache (256 MB) before the next one.  8 heads of 128 x 256, us: 128 rows on three sets of
+    // states in turn 64.3 -> 53.4, 256 119 -> 107 (128 on one set alone, half of which stays in that cache, 46 -> 53).  Below,
+    // what is right depends on what else the caller's step reads, which is not known here: 64 rows on three sets of states
+    // (201 MB, which fit) 25.8 -> 28.2, on twelve, as between a model's steps, 35.1 -> 28.4.  They keep plain loads.
     const bool once = (int64_t)D * H * d * V * (int64_t)sizeof(float) >= (int64_t)128 << 20;
 #define KGC_GLA_ROWS(RI, ONCE)                                                               \
   KGC_DS_DISPATCH_T(dtype, gla_decode_kernel<T, RI, ONCE><<<grid, NT, 0, s>>>(               \

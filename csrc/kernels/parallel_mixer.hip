@@ -554,9 +554,10 @@ static int pow2_at_least(int n, int lo) {
 }
 
 // States of 128 MB and more are read and written past the caches where a workgroup takes whole lines (64 columns): once
-// a step, and the last-level cache has 256 MB.  Decode rows, us: 32 heads of 128 x 64, 128 rows 63.3 -> 57.2, 256 113.4 -> 110.4;
-// the delta rule's 16 of 128 x 128, 128 rows 70.9 -> 62.1, 256 127.0 -> 119.6.  (64 rows of either may still lie there from the
-// step before; of the GLA's, which lose by it: decay_scan.hip.)
+// a step, and a model's other layers pass through the last-level cache (256 MB) before the next one.  Decode rows on three
+// sets of states in turn, us: 32 heads of 128 x 64, 128 rows 63.3 -> 57.2, 256 113.4 -> 110.4; the delta rule's 16 of 128 x 128,
+// 128 rows 70.9 -> 62.1, 256 127.0 -> 119.6.  On one set alone, part of which stays in that cache, 128 rows lose: 47 -> 57 and
+// 56 -> 61.  Smaller states keep plain loads, as in decay_scan.hip, where both sides of that are.
 static bool states_once(int seqs, int H, int d, int V) {
   return (int64_t)seqs * H * d * V * (int64_t)sizeof(float) >= (int64_t)128 << 20;
 }
