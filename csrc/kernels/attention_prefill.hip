@@ -863,9 +863,9 @@ __global__ __launch_bounds__(512, 1) void prefill_attn_gqa_persist_kernel(
 // What bounds it: latency.  At 32 x 512 rows vector instructions issue in 47 % of a SIMD's busy cycles and its matrix core
 // works in 24 % (4 x 4096: 54 and 41 %), at 2.4 GHz; LDS reads take 16 %, without conflicts.  The rest is waits.  Per
 // MFMA, 32 x 512 takes 1.9 times as long as 4 x 4096: the ends of items (q's rows and rotation, the output rows) and unequal
-// workgroups.  K / V write included, the 8-wave walk -> here, us: 32 x 512 188.7 -> 174.9, 64 x 256 151.8 -> 143.6, 8 x 2048 398 -> 344, 4 x 4096 732 ->
-// 622, 20 x 300 80.6 -> 68.7, 8 x 500 after 3000 285 -> 243.  Items dealt over all XCDs: 8 x 2048 362; K by DMA a tile ahead and
-// V within its tile: 373; operands read six steps ahead in the source: 377; indices drawn from a counter: 499.
+// workgroups.  K / V write included, the 8-wave walk -> here, us: 32 x 512 187.1 -> 171.6, 64 x 256 152 -> 144, 8 x 2048 401 ->
+// 341, 4 x 4096 726 -> 609, 20 x 300 79.3 -> 68.0, 8 x 500 after 3000 285 -> 243.  (Then 344:) items dealt over all XCDs, 8 x 2048
+// 362; K by DMA a tile ahead and V within its tile: 373; operands read six steps ahead in the source: 377; indices drawn from a counter: 499.
 struct WalkArgs {
   const void *q, *kc, *vc;
   void* out;
